@@ -18,7 +18,7 @@ _module = None
 
 def build(reference_root: str = "/root/reference") -> bool:
     """Run the reference recipe if the reference tree is present."""
-    if not os.path.isdir(reference_root):
+    if not os.path.isdir(os.path.join(reference_root, "fast_rnnt", "csrc")):
         return False
     subprocess.check_call(["make", "-C", _HERE, "-s", "ref", f"REF={reference_root}"])
     return True
