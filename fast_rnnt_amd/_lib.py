@@ -60,6 +60,14 @@ _SIGNATURES = {
     "frnnt_lattice_logprobs_fwd_bf16": ([_P] * 9 + [_I] * 8 + [_P], _I),
     "frnnt_lattice_logprobs_bwd_f16": ([_P] * 8 + [_I] * 8 + [_P], _I),
     "frnnt_lattice_logprobs_bwd_bf16": ([_P] * 8 + [_I] * 8 + [_P], _I),
+    "frnnt_lattice_loss_fwd_f32": ([_P] * 14 + [_I] * 7 + [_D, _I, _I, _P, _P], _I),
+    "frnnt_lattice_loss_bwd_f32": ([_P] * 6 + [_I, _D] + [_P] * 3 + [_I] * 7 + [_P], _I),
+    "frnnt_lattice_loss_fwd_f64": ([_P] * 14 + [_I] * 7 + [_D, _I, _I, _P, _P], _I),
+    "frnnt_lattice_loss_bwd_f64": ([_P] * 6 + [_I, _D] + [_P] * 3 + [_I] * 7 + [_P], _I),
+    "frnnt_lattice_loss_fwd_f16": ([_P] * 14 + [_I] * 7 + [_D, _I, _I, _P, _P], _I),
+    "frnnt_lattice_loss_bwd_f16": ([_P] * 6 + [_I, _D] + [_P] * 3 + [_I] * 7 + [_P], _I),
+    "frnnt_lattice_loss_fwd_bf16": ([_P] * 14 + [_I] * 7 + [_D, _I, _I, _P, _P], _I),
+    "frnnt_lattice_loss_bwd_bf16": ([_P] * 6 + [_I, _D] + [_P] * 3 + [_I] * 7 + [_P], _I),
     "frnnt_prune_ranges_f32": ([_P] * 4 + [_I] * 5 + [_P], _I),
     "frnnt_prune_ranges_f64": ([_P] * 4 + [_I] * 5 + [_P], _I),
     "frnnt_prune_gather_f32": ([_P] * 3 + [_I] * 5 + [_P], _I),

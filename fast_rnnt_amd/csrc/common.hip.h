@@ -90,6 +90,16 @@ struct AccOf<Narrow<IO>> {
   typedef float type;
 };
 
+// The largest of three, as the one instruction it is.  fmaxf() costs a canonicalising
+// v_max_f32 per operand on top (the compiler quiets signalling NaNs first), which tripled the
+// instruction count of the row maxima in the GEMM loops; v_max3_f32 itself ignores quiet NaNs
+// like fmaxf and quiets signalling ones.
+__device__ __forceinline__ float max3_raw(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // log(exp(a) + exp(b)) with the reference's handling of non-finite operands
 // (fast_rnnt/csrc/mutual_information.h:36-65): the larger operand is returned
 // untouched when the difference is not a finite number.

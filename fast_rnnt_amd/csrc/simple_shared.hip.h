@@ -55,15 +55,6 @@ typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 // exp(x - m) as one fused multiply-add and one v_exp_f32: 2^(x log2(e) - m log2(e)),
 // with shift2 = -m log2(e) prepared per row; x = -inf gives 0.
 constexpr float kLog2e = 1.44269504088896341f;
-// The largest of three, as the one instruction it is.  fmaxf() costs a canonicalising
-// v_max_f32 per operand on top (the compiler quiets signalling NaNs first), which tripled the
-// instruction count of the row maxima in the GEMM loops; v_max3_f32 itself ignores quiet NaNs
-// like fmaxf and quiets signalling ones.
-__device__ __forceinline__ float max3_raw(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
 __device__ __forceinline__ float exp_shifted(float x, float shift2) {
   return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, shift2));
 }

@@ -643,6 +643,202 @@ LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols
                                        need_am));
 }
 
+// ---- rnnt_loss and rnnt_loss_pruned behind one autograd node ------------------------------
+// forward = frnnt_lattice_loss_fwd: px / py from the logits (rnnt_loss.py:343-449, :856-1024), the
+// recursion, its backward with a gradient of ones, the reduction; backward =
+// frnnt_lattice_loss_bwd.  Occupation gradients that were handed out are scaled in place first
+// (mutual_information.py:173-181); otherwise their scale is applied as they are read.
+inline int abi_lattice_loss_fwd(at::ScalarType type, const void *logits, const int64_t *sym,
+                                const int64_t *rng, const int64_t *bnd, float *px, float *py,
+                                float *norm, float *xr, float *yr, float *p, float *sc, float *gx,
+                                float *gy, float *loss, int B, int S, int T, int R, int C,
+                                int term, int kind, double delay, int red, int checks,
+                                int32_t *status, void *st) {
+  if (type == at::kFloat)
+    return frnnt_lattice_loss_fwd_f32(static_cast<const float *>(logits), sym, rng, bnd, px, py,
+                                      norm, xr, yr, p, sc, gx, gy, loss, B, S, T, R, C, term, kind,
+                                      delay, red, checks, status, st);
+  return (type == at::kHalf ? frnnt_lattice_loss_fwd_f16 : frnnt_lattice_loss_fwd_bf16)(
+      logits, sym, rng, bnd, px, py, norm, xr, yr, p, sc, gx, gy, loss, B, S, T, R, C, term, kind,
+      delay, red, checks, status, st);
+}
+inline int abi_lattice_loss_fwd(at::ScalarType, const void *logits, const int64_t *sym,
+                                const int64_t *rng, const int64_t *bnd, double *px, double *py,
+                                double *norm, double *xr, double *yr, double *p, double *sc,
+                                double *gx, double *gy, double *loss, int B, int S, int T, int R,
+                                int C, int term, int kind, double delay, int red, int checks,
+                                int32_t *status, void *st) {
+  return frnnt_lattice_loss_fwd_f64(static_cast<const double *>(logits), sym, rng, bnd, px, py,
+                                    norm, xr, yr, p, sc, gx, gy, loss, B, S, T, R, C, term, kind,
+                                    delay, red, checks, status, st);
+}
+inline int abi_lattice_loss_bwd(at::ScalarType type, const void *logits, const int64_t *sym,
+                                const int64_t *rng, const int64_t *bnd, const float *norm,
+                                const float *g, int gstride, double gscale, const float *gx,
+                                const float *gy, void *out, int B, int S, int T, int R, int C,
+                                int term, int kind, void *st) {
+  if (type == at::kFloat)
+    return frnnt_lattice_loss_bwd_f32(static_cast<const float *>(logits), sym, rng, bnd, norm, g,
+                                      gstride, gscale, gx, gy, static_cast<float *>(out), B, S, T,
+                                      R, C, term, kind, st);
+  return (type == at::kHalf ? frnnt_lattice_loss_bwd_f16 : frnnt_lattice_loss_bwd_bf16)(
+      logits, sym, rng, bnd, norm, g, gstride, gscale, gx, gy, out, B, S, T, R, C, term, kind, st);
+}
+inline int abi_lattice_loss_bwd(at::ScalarType, const void *logits, const int64_t *sym,
+                                const int64_t *rng, const int64_t *bnd, const double *norm,
+                                const double *g, int gstride, double gscale, const double *gx,
+                                const double *gy, void *out, int B, int S, int T, int R, int C,
+                                int term, int kind, void *st) {
+  return frnnt_lattice_loss_bwd_f64(static_cast<const double *>(logits), sym, rng, bnd, norm, g,
+                                    gstride, gscale, gx, gy, static_cast<double *>(out), B, S, T,
+                                    R, C, term, kind, st);
+}
+
+struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &logits, const Tensor &symbols,
+                               const std::optional<Tensor> &ranges,
+                               const std::optional<Tensor> &boundary, int64_t term, int64_t kind,
+                               double delay_penalty, bool want_grads, int64_t reduction,
+                               int64_t checks, bool need_grad) {
+    return logits.scalar_type() == at::kDouble
+               ? run<double>(ctx, logits, symbols, or_undefined(ranges), or_undefined(boundary),
+                             term, kind, delay_penalty, want_grads, reduction, checks, need_grad)
+               : run<float>(ctx, logits, symbols, or_undefined(ranges), or_undefined(boundary),
+                            term, kind, delay_penalty, want_grads, reduction, checks, need_grad);
+  }
+
+  template <typename R>
+  static variable_list run(AutogradContext *ctx, const Tensor &logits_, const Tensor &symbols,
+                           const Tensor &ranges, const Tensor &boundary, int64_t term,
+                           int64_t kind, double delay_penalty, bool want_grads, int64_t reduction,
+                           int64_t checks, bool need_grad) {
+    const Tensor logits = logits_.contiguous(), sym = symbols.contiguous();
+    const Tensor rng = ranges.defined() ? ranges.contiguous() : Tensor();
+    const Tensor bnd = boundary.defined() ? boundary.contiguous() : Tensor();
+    const int64_t B = logits.size(0), T = logits.size(1), K = logits.size(2), C = logits.size(3),
+                  S = sym.size(1);
+    const int64_t T1 = kind == 0 ? T + 1 : T;
+    ctx->set_materialize_grads(false);
+    DeviceGuard guard(logits.device());
+    const auto opts = logits.options().dtype(c10::CppTypeToScalarType<R>::value);
+    // internal buffers in one allocation: norm | px | py | xr | yr | p | scores
+    Carver carve;
+    const int64_t o_nr = carve.take(B * T * K), o_px = carve.take(B * S * T1),
+                  o_py = carve.take(B * (S + 1) * T), o_xr = carve.take(B * T * K),
+                  o_yr = carve.take(B * T * K), o_p = carve.take(B * (S + 1) * (T + 1)),
+                  o_sc = carve.take(B);
+    Tensor work = at::empty({carve.total}, opts);
+    R *w = work.data_ptr<R>();
+    Tensor gx, gy;
+    if (want_grads || need_grad) {
+      gx = at::empty({B, S, T1}, opts);
+      gy = at::empty({B, S + 1, T}, opts);
+    }
+    Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
+    check_rc(abi_lattice_loss_fwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
+                                  iptr(bnd), w + o_px, w + o_py, w + o_nr, w + o_xr, w + o_yr,
+                                  w + o_p, w + o_sc, ptr<R>(gx), ptr<R>(gy), ptr<R>(loss), (int)B,
+                                  (int)S, (int)T, (int)K, (int)C, (int)term, (int)kind,
+                                  delay_penalty > 0.0 ? delay_penalty : 0.0, (int)reduction,
+                                  (int)checks, status_for(logits, bnd), stream_of(logits)),
+             "frnnt_lattice_loss_fwd");
+    if (need_grad) {
+      // (absent tensors are not saved: saved tensors must be defined)
+      variable_list save{logits, sym, work, gx, gy};
+      if (rng.defined()) save.push_back(rng);
+      if (bnd.defined()) save.push_back(bnd);
+      ctx->save_for_backward(std::move(save));
+      ctx->saved_data["meta"] =
+          std::vector<int64_t>{term, kind, reduction, rng.defined(), bnd.defined(), want_grads};
+    }
+    // (undefined tensors cannot be outputs of an autograd node)
+    if (!want_grads) return {loss};
+    ctx->mark_non_differentiable({gx, gy});
+    return {loss, gx, gy};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    variable_list out(11);
+    const Tensor &g_loss = grads[0];
+    if (!g_loss.defined()) return out;
+    const auto saved = ctx->get_saved_variables();
+    out[0] = saved[0].scalar_type() == at::kDouble ? run_backward<double>(ctx, saved, g_loss)
+                                                   : run_backward<float>(ctx, saved, g_loss);
+    return out;
+  }
+
+  template <typename R>
+  static Tensor run_backward(AutogradContext *ctx, const variable_list &saved,
+                             const Tensor &g_loss) {
+    const Tensor &logits = saved[0], &sym = saved[1], &work = saved[2];
+    Tensor gx = saved[3], gy = saved[4];
+    const std::vector<int64_t> meta = ctx->saved_data["meta"].toIntVector();
+    const int64_t kind = meta[1], reduction = meta[2];
+    const Tensor rng = meta[3] ? saved[5] : Tensor();
+    const Tensor bnd = meta[4] ? saved[5 + meta[3]] : Tensor();
+    const int64_t B = logits.size(0), T = logits.size(1), K = logits.size(2), C = logits.size(3),
+                  S = sym.size(1);
+    DeviceGuard guard(logits.device());
+    const Tensor g = g_loss.contiguous();
+    const int stride = reduction == kRedNone ? 1 : 0;
+    const double scale = reduction == kRedMean ? -1.0 / (double)B : -1.0;
+    void *stream = stream_of(logits);
+    const bool handed_out = meta[5] != 0;
+    if (handed_out)
+      check_rc(abi_mi_scale_grads(ptr<R>(gx), ptr<R>(gy), ptr<R>(g), stride, scale, (int)B, (int)S,
+                                  (int)T, (int)(kind != 0), stream),
+               "frnnt_mi_scale_grads");
+    Tensor grad = at::empty(logits.sizes(), logits.options());
+    check_rc(abi_lattice_loss_bwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
+                                  iptr(bnd), work.data_ptr<R>(),
+                                  handed_out ? (const R *)nullptr : ptr<R>(g), stride, scale,
+                                  ptr<R>(gx), ptr<R>(gy), grad.data_ptr(), (int)B, (int)S, (int)T,
+                                  (int)K, (int)C, (int)meta[0], (int)kind, stream),
+             "frnnt_lattice_loss_bwd");
+    return grad;
+  }
+};
+
+LossResult lattice_loss(const Tensor &logits, const Tensor &symbols,
+                        const std::optional<Tensor> &ranges_,
+                        const std::optional<Tensor> &boundary_, int64_t termination_symbol,
+                        int64_t rnnt_type, double delay_penalty, bool return_grad,
+                        int64_t reduction, int64_t checks) {
+  const Tensor ranges = or_undefined(ranges_), boundary = or_undefined(boundary_);
+  TORCH_CHECK(logits.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): logits");
+  TORCH_CHECK(logits.scalar_type() == at::kFloat || logits.scalar_type() == at::kDouble ||
+                  logits.scalar_type() == at::kHalf || logits.scalar_type() == at::kBFloat16,
+              "fast_rnnt_amd supports float32, float64, float16 and bfloat16 logits, got ",
+              logits.scalar_type());
+  TORCH_CHECK(logits.dim() == 4 && symbols.dim() == 2 && symbols.size(0) == logits.size(0),
+              "logits must be [B][T][S+1 or s_range][C], symbols [B][S]");
+  const int64_t B = logits.size(0);
+  auto check_index = [&](const Tensor &t, const char *name) {
+    TORCH_CHECK(t.scalar_type() == at::kLong && t.device() == logits.device(), name,
+                " must be an int64 tensor on the device of the logits");
+  };
+  check_index(symbols, "symbols");
+  if (ranges.defined()) {
+    check_index(ranges, "ranges");
+    TORCH_CHECK(ranges.dim() == 3 && ranges.size(0) == B && ranges.size(1) == logits.size(1) &&
+                    ranges.size(2) == logits.size(2),
+                "ranges must have the first three sizes of the logits");
+  } else {
+    TORCH_CHECK(logits.size(2) == symbols.size(1) + 1, "logits must be [B][T][S+1][C]");
+  }
+  if (boundary.defined()) {
+    check_index(boundary, "boundary");
+    TORCH_CHECK(boundary.dim() == 2 && boundary.size(0) == B && boundary.size(1) == 4,
+                "boundary must have shape [B][4]");
+  }
+  TORCH_CHECK(rnnt_type >= 0 && rnnt_type <= 2, "rnnt_type must be 0, 1 or 2");
+  TORCH_CHECK(reduction >= 0 && reduction <= 2, "reduction must be 0 (none), 1 (mean) or 2 (sum)");
+  const bool need_grad = at::GradMode::is_enabled() && logits.requires_grad();
+  return as_result(LatticeLossFn::apply(logits, symbols, ranges_, boundary_, termination_symbol,
+                                        rnnt_type, delay_penalty, return_grad, reduction, checks,
+                                        need_grad));
+}
+
 void set_deferred_checks(bool on) { g_deferred = on; }
 bool deferred_checks() { return g_deferred; }
 
@@ -661,6 +857,10 @@ TORCH_LIBRARY(fast_rnnt_amd, m) {
       "simple_loss(Tensor lm, Tensor am, Tensor symbols, Tensor? boundary, int termination_symbol, "
       "int rnnt_type, float delay_penalty, bool return_grad, int reduction, int checks) -> "
       "(Tensor, Tensor?, Tensor?)");
+  m.def(
+      "lattice_loss(Tensor logits, Tensor symbols, Tensor? ranges, Tensor? boundary, "
+      "int termination_symbol, int rnnt_type, float delay_penalty, bool return_grad, "
+      "int reduction, int checks) -> (Tensor, Tensor?, Tensor?)");
 }
 // (PyTorch-ROCm keeps the dispatch key name CUDA for the MI355X)
 TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
@@ -668,12 +868,14 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
   m.impl("mutual_information_backward", &mutual_information_backward);
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
+  m.impl("lattice_loss", &lattice_loss);
 }
 // The loss ops carry their own autograd nodes: the same functions serve the Autograd key
 // (they call the C ABI themselves and never re-dispatch).
 TORCH_LIBRARY_IMPL(fast_rnnt_amd, Autograd, m) {
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
+  m.impl("lattice_loss", &lattice_loss);
 }
 
 PYBIND11_MODULE(_C, m) {
@@ -687,6 +889,10 @@ PYBIND11_MODULE(_C, m) {
   m.def("recursion_loss", &recursion_loss, py::arg("px"), py::arg("py"), py::arg("boundary"),
         py::arg("return_grad"), py::arg("reduction"), py::arg("checks") = 0);
   m.def("simple_loss", &simple_loss, py::arg("lm"), py::arg("am"), py::arg("symbols"),
+        py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
+        py::arg("delay_penalty"), py::arg("return_grad"), py::arg("reduction"),
+        py::arg("checks") = 0);
+  m.def("lattice_loss", &lattice_loss, py::arg("logits"), py::arg("symbols"), py::arg("ranges"),
         py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
         py::arg("delay_penalty"), py::arg("return_grad"), py::arg("reduction"),
         py::arg("checks") = 0);

@@ -297,10 +297,7 @@ class _LatticeLogprobs(torch.autograd.Function):
     frnnt_lattice_logprobs_fwd/bwd."""
 
     @staticmethod
-    def forward(ctx, logits, symbols, ranges, boundary, termination_symbol, rnnt_type,
-                window_only=False):
-        # window_only: the caller feeds (px, py) to the recursion with this same boundary,
-        # so cells outside each utterance's window may stay undefined and carry no gradient
+    def forward(ctx, logits, symbols, ranges, boundary, termination_symbol, rnnt_type):
         B, T, R, C = logits.shape
         S = symbols.shape[1]
         kind = _RNNT_TYPES[rnnt_type]
@@ -313,7 +310,6 @@ class _LatticeLogprobs(torch.autograd.Function):
         bnd_c = boundary.contiguous() if boundary is not None else None
         opts = dict(dtype=_lattice_dtype(logits.dtype), device=logits.device)
         T1 = T + 1 if kind == 0 else T
-        windowed = bool(window_only) and bnd_c is not None
         with torch.cuda.device(logits.device):
             px = torch.empty(B, S, T1, **opts)
             py = torch.empty(B, S + 1, T, **opts)
@@ -323,16 +319,16 @@ class _LatticeLogprobs(torch.autograd.Function):
             _lib.call("frnnt_lattice_logprobs_fwd_" + sfx, lg.data_ptr(), sym_c.data_ptr(),
                       _lib.ptr(rng_c), _lib.ptr(bnd_c), px.data_ptr(), py.data_ptr(),
                       norm.data_ptr(), xr.data_ptr(), yr.data_ptr(), B, S, T, R, C,
-                      int(termination_symbol), kind, int(windowed), _lib.stream_of(logits))
+                      int(termination_symbol), kind, 0, _lib.stream_of(logits))
         if ctx.needs_input_grad[0]:
             ctx.save_for_backward(lg, sym_c, rng_c, bnd_c, norm)
-            ctx.meta = (B, S, T, R, C, int(termination_symbol), kind, sfx, int(windowed))
+            ctx.meta = (B, S, T, R, C, int(termination_symbol), kind, sfx)
         return px, py
 
     @staticmethod
     def backward(ctx, gpx, gpy):
         lg, sym, rng, bnd, norm = ctx.saved_tensors
-        B, S, T, R, C, term, kind, sfx, windowed = ctx.meta
+        B, S, T, R, C, term, kind, sfx = ctx.meta
         opts = dict(dtype=norm.dtype, device=lg.device)
         T1 = T + 1 if kind == 0 else T
         with torch.cuda.device(lg.device):
@@ -341,25 +337,39 @@ class _LatticeLogprobs(torch.autograd.Function):
             grad = torch.empty_like(lg)
             _lib.call("frnnt_lattice_logprobs_bwd_" + sfx, lg.data_ptr(), sym.data_ptr(),
                       _lib.ptr(rng), _lib.ptr(bnd), norm.data_ptr(), gpx.data_ptr(),
-                      gpy.data_ptr(), grad.data_ptr(), B, S, T, R, C, term, kind, windowed,
+                      gpy.data_ptr(), grad.data_ptr(), B, S, T, R, C, term, kind, 0,
                       _lib.stream_of(lg))
-        return grad, None, None, None, None, None, None
+        return grad, None, None, None, None, None
 
 
-def _joint_logprobs(logits, symbols, termination_symbol, boundary, rnnt_type, window_only):
+def _check_joint(logits, symbols, boundary, rnnt_type, checks):
+    """The argument checks of rnnt_loss.py:395-410; ``checks`` != 0: the boundary rows are left
+    to the recursion's forward kernel (see :func:`_device_checks`)."""
     assert logits.ndim == 4, logits.ndim
     (B, T, S1, C) = logits.shape
     S = S1 - 1
     assert symbols.shape == (B, S), symbols.shape
     assert rnnt_type in ["regular", "modified", "constrained"], rnnt_type
-    # (window_only: the caller is a loss function, whose recursion tests the rows itself)
-    on_device = bool(window_only) and _device_checks(rnnt_type, boundary) != 0
-    validate_st_lengths(S, T, rnnt_type == "regular", boundary, on_device=on_device)
+    validate_st_lengths(S, T, rnnt_type == "regular", boundary, on_device=checks != 0)
     _check_tensors([("logits", logits)], [("symbols", symbols), ("boundary", boundary)])
-    if window_only and boundary is not None:
-        _assert_boundary(boundary, B, S, T, on_device=on_device)
-    return _LatticeLogprobs.apply(logits, symbols, None, boundary, termination_symbol, rnnt_type,
-                                  window_only)
+
+
+def _lattice_loss(logits, symbols, ranges, termination_symbol, boundary, rnnt_type, delay_penalty,
+                  reduction, return_grad, checks):
+    """What rnnt_loss and rnnt_loss_pruned do once their arguments are checked: one autograd node
+    of the operator module (px / py from the logits, the recursion, its backward with a gradient
+    of ones, the reduction)."""
+    if boundary is not None:
+        _assert_boundary(boundary, logits.shape[0], symbols.shape[1], logits.shape[1],
+                         on_device=checks != 0)
+    if reduction not in _REDUCTIONS:
+        # (the reference finds this out after the recursion has run: same exception)
+        raise ValueError(f"reduction should be ('none' | 'mean' | 'sum'), given {reduction}")
+    _lib.suffix(logits.dtype, narrow=True)
+    loss, px_grad, py_grad = _lib.ops().lattice_loss(
+        logits, symbols, ranges, boundary, int(termination_symbol), _RNNT_TYPES[rnnt_type],
+        float(delay_penalty), bool(return_grad), _REDUCTIONS[reduction], checks)
+    return (loss, (px_grad, py_grad)) if return_grad else loss
 
 
 def get_rnnt_logprobs_joint(
@@ -368,7 +378,8 @@ def get_rnnt_logprobs_joint(
 ) -> Tuple[Tensor, Tensor]:
     """(px, py) from the full joiner output ``logits`` of shape ``(B, T, S+1, C)``
     (fast_rnnt/python/fast_rnnt/rnnt_loss.py:343-449)."""
-    return _joint_logprobs(logits, symbols, termination_symbol, boundary, rnnt_type, False)
+    _check_joint(logits, symbols, boundary, rnnt_type, 0)
+    return _LatticeLogprobs.apply(logits, symbols, None, boundary, termination_symbol, rnnt_type)
 
 
 def rnnt_loss(
@@ -379,9 +390,10 @@ def rnnt_loss(
     """The unpruned RNN-T loss on joiner logits ``(B, T, S+1, C)`` (rnnt_loss.py:452-547).
     The logits of cells outside an utterance's boundary window are not read: the
     recursion never visits them and their gradient is exactly zero."""
-    px, py = _joint_logprobs(logits, symbols, termination_symbol, boundary, rnnt_type, True)
-    return _recursion_and_reduce(px, py, boundary, rnnt_type, delay_penalty, reduction,
-                                 return_grad)
+    checks = _device_checks(rnnt_type, boundary)
+    _check_joint(logits, symbols, boundary, rnnt_type, checks)
+    return _lattice_loss(logits, symbols, None, termination_symbol, boundary, rnnt_type,
+                         delay_penalty, reduction, return_grad, checks)
 
 
 def _monotonic_lower_bound(x: Tensor) -> Tensor:
@@ -580,21 +592,16 @@ def _roll_by_shifts(src: Tensor, shifts: torch.LongTensor):
     return torch.gather(src, 2, index)
 
 
-def _pruned_logprobs(logits, symbols, ranges, termination_symbol, boundary, rnnt_type,
-                     window_only):
+def _check_pruned(logits, symbols, ranges, boundary, rnnt_type, checks):
+    """The argument checks of rnnt_loss.py:916-938; ``checks`` as in :func:`_check_joint`."""
     assert logits.ndim == 4, logits.ndim
     (B, T, s_range, C) = logits.shape
     assert ranges.shape == (B, T, s_range), f"{ranges.shape} == ({B}, {T}, {s_range})"
     (B, S) = symbols.shape
     assert rnnt_type in ["regular", "modified", "constrained"], rnnt_type
-    on_device = bool(window_only) and _device_checks(rnnt_type, boundary) != 0
-    validate_st_lengths(S, T, rnnt_type == "regular", boundary, on_device=on_device)
+    validate_st_lengths(S, T, rnnt_type == "regular", boundary, on_device=checks != 0)
     _check_tensors([("logits", logits)],
                    [("symbols", symbols), ("ranges", ranges), ("boundary", boundary)])
-    if window_only and boundary is not None:
-        _assert_boundary(boundary, B, S, T, on_device=on_device)
-    return _LatticeLogprobs.apply(logits, symbols, ranges, boundary, termination_symbol,
-                                  rnnt_type, window_only)
 
 
 def get_rnnt_logprobs_pruned(
@@ -604,8 +611,8 @@ def get_rnnt_logprobs_pruned(
     """(px, py) from pruned joiner logits ``(B, T, s_range, C)`` and the
     ``ranges`` they were computed for (rnnt_loss.py:856-1024); lattice cells
     outside the kept range of their frame are -inf."""
-    return _pruned_logprobs(logits, symbols, ranges, termination_symbol, boundary, rnnt_type,
-                            False)
+    _check_pruned(logits, symbols, ranges, boundary, rnnt_type, 0)
+    return _LatticeLogprobs.apply(logits, symbols, ranges, boundary, termination_symbol, rnnt_type)
 
 
 def rnnt_loss_pruned(
@@ -615,10 +622,10 @@ def rnnt_loss_pruned(
 ) -> Tensor:
     """The pruned RNN-T loss on joiner logits ``(B, T, s_range, C)`` (rnnt_loss.py:1027-1132).
     As in :func:`rnnt_loss`, logits outside an utterance's boundary window are not read."""
-    px, py = _pruned_logprobs(logits, symbols, ranges, termination_symbol, boundary, rnnt_type,
-                              True)
-    return _recursion_and_reduce(px, py, boundary, rnnt_type, delay_penalty, reduction,
-                                 return_grad)
+    checks = _device_checks(rnnt_type, boundary)
+    _check_pruned(logits, symbols, ranges, boundary, rnnt_type, checks)
+    return _lattice_loss(logits, symbols, ranges, termination_symbol, boundary, rnnt_type,
+                         delay_penalty, reduction, return_grad, checks)
 
 
 class _SmoothedCombine(torch.autograd.Function):

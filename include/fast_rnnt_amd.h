@@ -418,6 +418,66 @@ int frnnt_lattice_logprobs_bwd_bf16(const void *logits, const int64_t *symbols,
                                     void *stream);
 
 /*
+ * A whole loss on joiner logits: rnnt_loss (ranges == NULL, R == S+1; rnnt_loss.py:452-547) and
+ * rnnt_loss_pruned (:1027-1132).  _fwd chains frnnt_lattice_logprobs_fwd (window_only when a
+ * boundary is given; delay_penalty > 0 is added to px as in rnnt_loss.py:309-324) and
+ * frnnt_mi_loss_fwd, with that function's px_grad / py_grad (both NULL: not wanted), loss,
+ * reduction, checks and status.  _bwd is frnnt_lattice_logprobs_bwd on occupation gradients that
+ * have NOT been scaled: utterance b's are taken times
+ * score_grad_scale * score_grad[b * score_grad_stride] (stride 0 or 1) as they are read;
+ * score_grad == NULL: as they are.  For 2-byte logits every other buffer is float32.
+ */
+int frnnt_lattice_loss_fwd_f32(const float *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, float *px, float *py, float *norm,
+                               float *xr, float *yr, float *p, float *scores, float *px_grad,
+                               float *py_grad, float *loss, int B, int S, int T, int R, int C,
+                               int termination_symbol, int rnnt_type, double delay_penalty,
+                               int reduction, int checks, int32_t *status, void *stream);
+int frnnt_lattice_loss_fwd_f64(const double *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, double *px, double *py, double *norm,
+                               double *xr, double *yr, double *p, double *scores, double *px_grad,
+                               double *py_grad, double *loss, int B, int S, int T, int R, int C,
+                               int termination_symbol, int rnnt_type, double delay_penalty,
+                               int reduction, int checks, int32_t *status, void *stream);
+int frnnt_lattice_loss_fwd_f16(const void *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, float *px, float *py, float *norm,
+                               float *xr, float *yr, float *p, float *scores, float *px_grad,
+                               float *py_grad, float *loss, int B, int S, int T, int R, int C,
+                               int termination_symbol, int rnnt_type, double delay_penalty,
+                               int reduction, int checks, int32_t *status, void *stream);
+int frnnt_lattice_loss_fwd_bf16(const void *logits, const int64_t *symbols, const int64_t *ranges,
+                                const int64_t *boundary, float *px, float *py, float *norm,
+                                float *xr, float *yr, float *p, float *scores, float *px_grad,
+                                float *py_grad, float *loss, int B, int S, int T, int R, int C,
+                                int termination_symbol, int rnnt_type, double delay_penalty,
+                                int reduction, int checks, int32_t *status, void *stream);
+int frnnt_lattice_loss_bwd_f32(const float *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, const float *norm, const float *score_grad,
+                               int score_grad_stride, double score_grad_scale,
+                               const float *px_grad, const float *py_grad, float *logits_grad,
+                               int B, int S, int T, int R, int C, int termination_symbol,
+                               int rnnt_type, void *stream);
+int frnnt_lattice_loss_bwd_f64(const double *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, const double *norm,
+                               const double *score_grad, int score_grad_stride,
+                               double score_grad_scale, const double *px_grad,
+                               const double *py_grad, double *logits_grad, int B, int S, int T,
+                               int R, int C, int termination_symbol, int rnnt_type, void *stream);
+int frnnt_lattice_loss_bwd_f16(const void *logits, const int64_t *symbols, const int64_t *ranges,
+                               const int64_t *boundary, const float *norm, const float *score_grad,
+                               int score_grad_stride, double score_grad_scale,
+                               const float *px_grad, const float *py_grad, void *logits_grad,
+                               int B, int S, int T, int R, int C, int termination_symbol,
+                               int rnnt_type, void *stream);
+int frnnt_lattice_loss_bwd_bf16(const void *logits, const int64_t *symbols, const int64_t *ranges,
+                                const int64_t *boundary, const float *norm,
+                                const float *score_grad, int score_grad_stride,
+                                double score_grad_scale, const float *px_grad,
+                                const float *py_grad, void *logits_grad, int B, int S, int T,
+                                int R, int C, int termination_symbol, int rnnt_type,
+                                void *stream);
+
+/*
  * Pruning bounds.  Replaces the device work of get_rnnt_prune_ranges
  * (rnnt_loss.py:726-777 with _adjust_pruning_lower_bound :584-632).  s_range is
  * the FINAL window size: the caller has already raised it to the regular

@@ -1,0 +1,50 @@
+"""The row kernels of the losses on logits (csrc/lattice_logprobs.hip) where their split of a row
+over lanes and 16-byte pieces can go wrong: vocabularies on either side of every split (a quarter,
+a half, a whole wave per row, 2 ... 20 pieces per lane, rows in chunks), rows that share a
+piece with their neighbours, logits that begin off a 16-byte boundary.  Oracle: the CPU
+restatement on the same values in float32."""
+import pytest
+import torch
+
+import fast_rnnt_amd
+from oracle import losses as O
+
+pytestmark = pytest.mark.gpu
+# gradients: 1e-4 absolute and one unit in the last place of the type
+ULP = {torch.float32: 1e-5, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}
+LENGTHS = [1, 3, 63, 64, 65, 125, 128, 131, 256, 257, 503, 1025, 2050, 2565, 3590, 5113, 5121,
+           10245]
+
+
+@pytest.mark.parametrize("C", LENGTHS)
+@pytest.mark.parametrize("dtype", list(ULP))
+def test_loss_on_logits_of_any_row_length(gpu_device, dtype, C):
+    B, S, T, R = 2, 4, 9, 3
+    g = torch.Generator().manual_seed(C)
+    symbols = torch.randint(0, C, (B, S), generator=g)
+    boundary = torch.tensor([[0, 0, S, T], [0, 1, S - 1, T - 2]])
+    begin = torch.clamp(torch.arange(T) * (S + 1 - R) // (T - 3), max=S + 1 - R)
+    ranges = (begin.reshape(1, T, 1) + torch.arange(R)).expand(B, T, R).contiguous()
+    for ranges_, K, shift, kind, handed_out in [(None, S + 1, 0, "regular", True),
+                                                (None, S + 1, 1, "constrained", False),
+                                                (ranges, R, 0, "modified", False),
+                                                (ranges, R, 3, "regular", False)]:
+        print(f"C={C} {dtype} K={K} shift={shift} {kind}", flush=True)
+        flat = (2 * torch.randn(shift + B * T * K * C, generator=g)).to(dtype)
+        cpu = flat[shift:].reshape(B, T, K, C).float().requires_grad_(True)
+        gpu = flat.to(gpu_device)[shift:].reshape(B, T, K, C).requires_grad_(True)
+        args = dict(boundary=boundary, rnnt_type=kind, delay_penalty=0.01, reduction="mean")
+        dev = dict(args, boundary=boundary.to(gpu_device), return_grad=handed_out)
+        if ranges_ is None:
+            want = O.loss_joint(cpu, symbols, 0, **args)
+            got = fast_rnnt_amd.rnnt_loss(gpu, symbols.to(gpu_device), 0, **dev)
+        else:
+            want = O.loss_pruned(cpu, symbols, ranges_, 0, **args)
+            got = fast_rnnt_amd.rnnt_loss_pruned(gpu, symbols.to(gpu_device),
+                                                 ranges_.to(gpu_device), 0, **dev)
+        got = got[0] if handed_out else got
+        assert abs(got.item() - want.item()) <= 1e-5 * max(1.0, abs(want.item()))
+        (3.0 * want).backward()
+        (3.0 * got).backward()
+        off = (gpu.grad.float().cpu() - cpu.grad).abs()
+        assert bool((off <= 1e-4 + ULP[dtype] * cpu.grad.abs()).all()), off.max().item()
