@@ -195,4 +195,17 @@ int mi_backward_and_loss(const double *px, const int64_t *boundary, const double
                          double *px_grad, double *py_grad, const double *scores, double *loss,
                          int B, int S, int T, int modified, int reduction, void *stream);
 
+// ((T_b - 1) / 2 - t) * delay_penalty, what rnnt_loss.py:309-324 adds to px, rounded as there.
+template <typename R>
+struct Delay {
+  R scale;  // 0: no penalty
+  __device__ __forceinline__ R at(R px, const int64_t *boundary, int b, int t, int T) const {
+    if (scale == 0) return px;
+    // (the reference's offsets are float32 when they come from the boundary's integers)
+    if (boundary)
+      return px + (R)(((float)(boundary[4 * b + 3] - 1) / 2 - (float)t) * (float)scale);
+    return px + ((R)(T - 1) / 2 - (R)t) * scale;
+  }
+};
+
 }  // namespace frnnt

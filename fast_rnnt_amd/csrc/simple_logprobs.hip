@@ -28,7 +28,6 @@
 namespace frnnt {
 namespace {
 
-
 // Which XCD works on which utterance in the gradient products.  Workgroup i runs on XCD
 // i % 8 and all tiles of an utterance stay on one XCD (one L2 holds its operands), so a launch of
 // many tiles lasts as long as its fullest XCD; with utterance b on XCD b % 8 that is left to
@@ -176,8 +175,8 @@ __global__ void __launch_bounds__(kGemmThreads)
     simple_fwd_kernel(const R *__restrict__ lm, const R *__restrict__ am,
                       const int64_t *__restrict__ symbols, const int64_t *__restrict__ boundary,
                       const R *__restrict__ lm_max, const R *__restrict__ am_max,
-                      R *__restrict__ px, R *__restrict__ py, R *__restrict__ norm_raw, int S,
-                      int T, int C, int term, int rnnt_type) {
+                      R *__restrict__ px, R *__restrict__ py, R *__restrict__ norm_raw,
+                      Delay<R> delay, int S, int T, int C, int term, int rnnt_type) {
   __shared__ R lds[4 * TileK<R>::value * kPitch];
   const int b = blockIdx.z;
   const int s_tile = blockIdx.y * kTileM, t_tile = blockIdx.x * kTileN;
@@ -213,7 +212,7 @@ __global__ void __launch_bounds__(kGemmThreads)
       else
         v = (amb[(long)t * C + sym] + lmb[(long)s * C + sym]) - norm;
       if (t == t_mask) v = Num<R>::neg_inf();
-      pxb[(long)s * T1 + t] = v;
+      pxb[(long)s * T1 + t] = delay.at(v, boundary, b, t, T);
     }
   });
   // the extra column of the regular lattice: nothing can be emitted after the last frame
@@ -223,32 +222,37 @@ __global__ void __launch_bounds__(kGemmThreads)
   }
 }
 
-// constrained lattice: px[b,s,t] += py[b,s+1,t]   (rnnt_loss.py:224-225)
+// constrained lattice: px[b,s,t] += py[b,s+1,t]   (rnnt_loss.py:224-225), then the delay penalty
 template <typename R>
 __global__ void __launch_bounds__(256)
-    add_next_row_kernel(R *__restrict__ px, const R *__restrict__ py, long total, int S, int T) {
+    add_next_row_kernel(R *__restrict__ px, const R *__restrict__ py,
+                        const int64_t *__restrict__ boundary, Delay<R> delay, long total, int S,
+                        int T) {
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= total) return;
   const long b = idx / ((long)S * T);
   const long rem = idx - b * (long)S * T;
   const int s = (int)(rem / T), t = (int)(rem - (long)s * T);
-  px[idx] += py[(b * (S + 1) + s + 1) * T + t];
+  px[idx] = delay.at(px[idx] + py[(b * (S + 1) + s + 1) * T + t], boundary, (int)b, t, T);
 }
 
 // ---- backward ------------------------------------------------------------------------
 // 256-thread workgroups.  The first ceil(B*(S+1)/4) of them give each wave one
-// lattice row (b, s): D[b,s,:] and the two row sums.  The remaining ones take 64
-// frames of one utterance each and form the column sums, the four waves splitting
-// the lattice rows.  Loads are issued in batches of four before anything is
-// stored, so a row costs one memory round trip, not one per 64 frames.  The last
-// workgroup ranks the utterances for the gradient products (rank_utterances).
+// lattice row (b, s): D[b,s,:] and the two row sums.  With `score_grad` the wave first scales
+// its row of the occupation gradients in place (scale_by_batch_kernel's work, for lattices whose
+// rows do not read each other's: one pass over them less).  Loads are issued in batches of
+// four before anything is stored, so a row costs one memory round trip, not one per 64 frames.
+// In double the next workgroups take 64 frames of one utterance each and form the column
+// sums, the four waves splitting the lattice rows (the float product forms those it needs).  The
+// last workgroup ranks the utterances for the gradient products (rank_utterances).
 template <typename R>
 __global__ void __launch_bounds__(256)
-    simple_bwd_prep_kernel(const R *__restrict__ gpx, const R *__restrict__ gpy,
+    simple_bwd_prep_kernel(R *__restrict__ gpx, R *__restrict__ gpy,
                            const R *__restrict__ norm_raw, const int64_t *__restrict__ boundary,
-                           const int64_t *__restrict__ window, R *__restrict__ dmat,
-                           R *__restrict__ row_x, R *__restrict__ row_y, R *__restrict__ col_y,
-                           int B, int S, int T, int ldd, int rnnt_type) {
+                           const int64_t *__restrict__ window, const R *__restrict__ score_grad,
+                           int stride, R scale, R *__restrict__ dmat, R *__restrict__ row_x,
+                           R *__restrict__ row_y, R *__restrict__ col_y, int B, int S, int T,
+                           int ldd, int rnnt_type) {
   __shared__ R partial[4][kWave];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
@@ -261,29 +265,39 @@ __global__ void __launch_bounds__(256)
     if (row >= n_rows) return;
     const int b = (int)(row / S1), s = (int)(row % S1);
     const int t_mask = (rnnt_type == kRegular && boundary) ? (int)boundary[4 * b + 3] : -1;
-    // outside the window nothing is read (the normalizers there may be undefined): D = 0
+    // outside the window nothing counts (the normalizers there may be undefined): D = 0
     const Limits lim = limits_of(window, b, S, T);
     const bool row_in = s >= lim.s_begin && s <= lim.s_end;
-    const R *gx_row = s < S ? gpx + ((long)b * S + s) * T1 : nullptr;
+    R *gx_row = s < S ? gpx + ((long)b * S + s) * T1 : nullptr;
     const R *gx_prev = (constrained && s >= 1) ? gpx + ((long)b * S + s - 1) * T1 : nullptr;
-    const R *gy_row = gpy + row * T;
+    R *gy_row = gpy + row * T;
     const R *nr_row = norm_raw + row * T;
     R *d_row = dmat + row * ldd;
+    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
     R sx = 0, sy = 0;
-    for (int t0 = 0; t0 < T; t0 += 4 * kWave) {
+    for (int t0 = 0; t0 < T1; t0 += 4 * kWave) {
       R gx[4], gy[4], nr[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = t0 + u * kWave + lane;
         const bool ok = t < T && row_in && t >= lim.t_begin && t < lim.t_end;
-        gx[u] = (ok && gx_row && t != t_mask) ? gx_row[t] : (R)0;
-        gy[u] = ok ? gy_row[t] : (R)0;
+        gx[u] = (gx_row && (score_grad ? t < T1 : ok)) ? gx_row[t] : (R)0;
+        gy[u] = (score_grad ? t < T : ok) ? gy_row[t] : (R)0;
         if (ok && gx_prev && t != t_mask) gy[u] += gx_prev[t];
         nr[u] = ok ? nr_row[t] : (R)0;
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = t0 + u * kWave + lane;
+        const bool ok = t < T && row_in && t >= lim.t_begin && t < lim.t_end;
+        if (score_grad) {
+          gx[u] *= g;
+          gy[u] *= g;
+          if (gx_row && t < T1) gx_row[t] = gx[u];
+          if (t < T) gy_row[t] = gy[u];
+        }
+        if (!ok || t == t_mask) gx[u] = (R)0;
+        if (!ok) gy[u] = (R)0;
         if (t < T) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
         sx += gx[u];
         sy += gy[u];
@@ -433,649 +447,622 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-
-// four consecutive floats at any element-aligned address (global memory takes
-// unaligned 16-byte accesses); `valid` (0..4) leading elements are read, the rest is 0
-__device__ __forceinline__ dgemm::floatx4 load4_guarded(const float *base, int off, int valid,
-                                                        float fill = 0.f) {
-  dgemm::floatx4 r = {fill, fill, fill, fill};
-  if (valid >= 4) {
-    const floatx4u t = *reinterpret_cast<const floatx4u *>(base + off);
-    r[0] = t[0], r[1] = t[1], r[2] = t[2], r[3] = t[3];
-  } else {
+// ---- float32 gradient products on the bfloat16 matrix cores ----------------------------------
+//   lm.grad[s,c] = exp(lm[s,c] - max[s]) * sum_t D[s,t] exp(am[t,c] - max[t]) + one-hots
+//   am.grad[t,c] = exp(am[t,c] - max[t]) * sum_s D[s,t] exp(lm[s,c] - max[s]) + one-hots
+// A workgroup of four waves takes kM rows (lattice rows of lm.grad, frames of am.grad) x kC
+// vocabulary entries, a wave kM / 2 x kC / 2 of them as 32 x 32 accumulators.  k (frames, lattice
+// rows) runs in chunks of 32: the 256 threads fetch a chunk of both operands, apply exp to
+// the one that needs it, split the values into bfloat16 parts (Split8) and write them to LDS as
+// [k-step][row or entry][part][16 k]; after a barrier every wave reads its operands from there.
+// Where an operand lies k-major in memory (am and lm always, D for am.grad) a thread takes eight
+// consecutive k of one column -- loads that are contiguous over the lanes -- and has its
+// 16-byte piece of the operand without any transposition.
+// Four workgroups share a compute unit (37 KB of LDS, 128 registers each): while one waits for
+// memory, at a barrier or for its epilogue the others convert or multiply; one alone takes 1 us per
+// chunk, a full compute unit 1.6 us for four.  What bounds them then: the VALU (about 26 cycles per
+// 64 operand elements for exp and split) beside 12 matrix cycles per k and 32 x 32 outputs.
+// Measured (both products): B 32, S 80, T 250, C 500: 29 us with the float32 matrix instruction,
+// 24 here; B 64, S 120, T 600, C 500: 119 and 79; B 16, S 120, T 400, C 5000: 202 and 134.
+constexpr int kProdThreads = 256;
+constexpr int kProdC = 64;         // vocabulary entries of a tile
+constexpr int kProdPerCu = 4;      // workgroups that share a compute unit
+constexpr long kMinWideTiles = 256;
+constexpr int kProdK = 32;       // k per chunk: two k-steps
+constexpr int kProdRowBytes = 96;
+template <int kM, int kC>
+struct ProdShape {
+  static constexpr int kRows = kM + kC;                         // rows of a k-step in LDS: m, then c
+  static constexpr int kStepBytes = kRows * kProdRowBytes;
+  static constexpr size_t kLdsBytes = 2 * kStepBytes;  // (holds the listed gx rows as well)
+  static constexpr int kMTiles = kM / 64, kCTiles = kC / 64;    // 32-row and -column tiles per wave
+  static constexpr int kMColumns = kM / 64, kColumns = kC / 64; // columns per thread of a k-major fetch
+};
+typedef int intx4 __attribute__((ext_vector_type(4)));
+// Byte offset of k-octet `octet` (0 .. 3) of row `row` within a chunk's LDS image; the parts lie 32
+// bytes apart.  Rows whose bit 3 is set have the halves of a part swapped: the 16-byte accesses of
+// 16 consecutive rows then fall on all 64 banks (rows are 24 words apart).
+template <int kM, int kC>
+__device__ __forceinline__ int octet_at(int row, int octet) {
+  return (octet >> 1) * ProdShape<kM, kC>::kStepBytes + row * kProdRowBytes +
+         16 * ((octet & 1) ^ ((row >> 3) & 1));
+}
+__device__ __forceinline__ void write_octet(char *to, const float (&e)[8]) {
+  uintx4 hi, mid, lo;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < valid) r[i] = base[off + i];
+  for (int q = 0; q < 4; ++q) {
+    unsigned h, m, l;
+    split_pair(e[2 * q], e[2 * q + 1], h, m, l);
+    hi[q] = h, mid[q] = m, lo[q] = l;
   }
-  return r;
+  *reinterpret_cast<uintx4 *>(to) = hi;
+  *reinterpret_cast<uintx4 *>(to + 32) = mid;
+  *reinterpret_cast<uintx4 *>(to + 64) = lo;
+}
+__device__ __forceinline__ Split8 read_octet(const char *at) {
+  Split8 o;
+  o.hi = *reinterpret_cast<const bf16x8 *>(at);
+  o.mid = *reinterpret_cast<const bf16x8 *>(at + 32);
+  o.lo = *reinterpret_cast<const bf16x8 *>(at + 64);
+  return o;
+}
+// eight k of one column of a k-major matrix (rows `ld` floats apart): `off` is the byte offset of
+// the column in row k0, rows from `k_end` on read as 0
+__device__ __forceinline__ void fetch_octet(float (&into)[8], __amdgpu_buffer_rsrc_t rs, int off,
+                                            int k0, int k_end, int ld) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    into[i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        rs, k0 + i < k_end ? off : kNowhere, (k0 + i) * ld * 4, 0));
+}
+// (the gradients that a product writes are FRNNT_F32, FRNNT_F16 or FRNNT_BF16)
+__device__ __forceinline__ int out_bytes(int type) { return type == FRNNT_F32 ? 4 : 2; }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t out_buffer(void *base, long first, int count,
+                                                             int type) {
+  const int size = out_bytes(type);
+  return __builtin_amdgcn_make_buffer_rsrc(static_cast<char *>(base) + first * size, 0, count * size,
+                                           0x00020000);
+}
+// f(store) with store(resource, there, element, uniform element, value) for the type
+template <typename F>
+__device__ __forceinline__ void with_store(int type, F f) {
+  if (type == FRNNT_F32)
+    f([](__amdgpu_buffer_rsrc_t rs, bool there, int at, int uniform, float x) {
+      put_float(rs, there, 4 * at, x, 4 * uniform);
+    });
+  else
+    f([type](__amdgpu_buffer_rsrc_t rs, bool there, int at, int uniform, float x) {
+      const uint16_t half = HalfIO::store(x), bf16 = (uint16_t)pack_bf16(x, 0.f);
+      __builtin_amdgcn_raw_buffer_store_b16((short)(type == FRNNT_F16 ? half : bf16), rs,
+                                            there ? 2 * at : kNowhere, 2 * uniform, 0);
+    });
+}
+// the products of a chunk: the first `m_tiles` of this wave's 32-row tiles
+template <int kM, int kC>
+__device__ __forceinline__ void multiply_chunk(const char *lds, int wave_m, int wave_n, int half,
+                                               int r32, int m_tiles,
+                                               dgemm::floatx16 (&acc)[ProdShape<kM, kC>::kMTiles]
+                                                                     [ProdShape<kM, kC>::kCTiles]) {
+  constexpr int kMTiles = ProdShape<kM, kC>::kMTiles;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    Split8 m_op[kMTiles];
+#pragma unroll
+    for (int j = 0; j < kMTiles; ++j)
+      m_op[j] = read_octet(lds + octet_at<kM, kC>(kM / 2 * wave_m + 32 * j + r32, 2 * g + half));
+#pragma unroll
+    for (int n = 0; n < ProdShape<kM, kC>::kCTiles; ++n) {
+      const Split8 c_op = read_octet(
+          lds + octet_at<kM, kC>(kM + (kC / 2) * wave_n + 32 * n + r32, 2 * g + half));
+#pragma unroll
+      for (int j = 0; j < kMTiles; ++j)
+        if (m_tiles > j) acc[j][n] = multiply_add(m_op[j], c_op, acc[j][n]);
+    }
+  }
 }
 
-// ---- fp32: MFMA kernels with LDS slabs / panels (xcd_grid.hip.h) --------------------
-
-// lm gradient:  lm.grad[s,c] = exp(lm[s,c] - max[s]) * sum_t D[s,t] exp(am[t,c] - max[t])
-// + [c = sym[s]] row_x[s] + [c = term] row_y[s].  Same scheme as the normalizer GEMM:
-// k runs over frames and is split between the waves of a workgroup; a wave turns its
-// 32-frame slabs -- D[96 rows][32 k], fetched as coalesced 16-byte pieces and
-// transposed through its own LDS region, and exp(am[32 k][32 c] - max) -- into MFMA
-// operands without waiting for any other wave; the partial sums meet once at the end.
-// A workgroup covers kS lattice rows x 32 vocabulary entries and takes the frames in slabs
-// of kK: 96 rows with 32 frames, or 128 rows with 16 (the form that pads S+1 less, as in
-// the normalizer kernel).
-constexpr int kLmC = 32;
-constexpr int kLmWaves = 4;
-constexpr int kLmThreads = kLmWaves * kWave;
-constexpr int kLmOutPitch = kLmC + 1;  // pitch of a wave's partial sums in LDS
-template <int kS, int kK>
-struct LmShape {
-  // (row pitch of the D slab: 16-byte aligned rows, as in PanelShape)
-  static constexpr int kPitch = kK + 4;
-  static constexpr int kSlab = kS * kPitch + kK * kLmC;  // floats per wave: D slab, then am slab
-  static constexpr int kSums = kS * kLmOutPitch;         // floats of a wave's partial sums
-  static constexpr size_t kLdsBytes =
-      (size_t)kLmWaves * (kSlab > kSums ? kSlab : kSums) * sizeof(float);
-  static constexpr int kItems = kS * kLmC / 4 / kLmThreads;  // 16-byte outputs per thread
-  static constexpr int kRowLanes = kK / 4;                   // lanes that share a row of the D slab
-  static constexpr int kRowsPerLoad = kWave / kRowLanes;
-  static_assert(kS % kRowsPerLoad == 0 && kK % 8 == 0 && kS % 32 == 0, "shape");
-};
-
-template <int kS, int kK>
-__device__ __forceinline__ void simple_bwd_lm_slab_body(
+template <int kM, int kC>
+__device__ __forceinline__ void simple_bwd_lm_body(
     int block_id, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const float *__restrict__ lm_max,
     const float *__restrict__ am_max, const float *__restrict__ dmat,
     const float *__restrict__ row_x, const float *__restrict__ row_y,
-    float *__restrict__ lm_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
-    int ldd, int term, int part_shift) {
-  using Shape = LmShape<kS, kK>;
-  constexpr int kLmS = kS, kLmK = kK, kLmPitch = Shape::kPitch, kLmSlab = Shape::kSlab;
-  constexpr int kLmItems = Shape::kItems;
+    void *__restrict__ lm_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
+    int ldd, int term, int part_shift, int out_type) {
+  using Shape = ProdShape<kM, kC>;
   using namespace dgemm;
-  extern __shared__ __align__(16) float lm_lds[];
+  extern __shared__ __align__(16) char prod_lds[];
+  __shared__ float row_mx[kM], row_rx[kM], row_ry[kM];
+  __shared__ int row_sym[kM];
   const int S1 = S + 1;
-  const int c_tiles = (C + kLmC - 1) / kLmC, s_tiles = (S1 + kLmS - 1) / kLmS;
+  const int c_tiles = (C + kC - 1) / kC, s_tiles = (S1 + kM - 1) / kM;
   int b, tile;
   Limits lim;
   if (!place_block(block_id, c_tiles, s_tiles, part_shift, B, row_x, window, S, T, b, tile, lim))
     return;
-  const int s_tile = (tile / c_tiles) * kLmS, c_tile = (tile % c_tiles) * kLmC;
+  const int s_tile = (tile / c_tiles) * kM, c_tile = (tile % c_tiles) * kC;
   const float *lmb = lm + (long)b * S1 * C;
   const float *amb = am + (long)b * T * C;
-  const float *lmx = lm_max + (long)b * S1;
   const float *amx = am_max + (long)b * T;
   const float *db = dmat + (long)b * S1 * ldd;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_m = wave >> 1, wave_n = wave & 1;
   const int half = lane >> 5, r32 = lane & 31;
   // With a window, D vanishes at frames >= t_end and on rows > s_end: the sum over frames
-  // stops at t_end (the row maxima of later frames may not even be defined) and 32-row
-  // tiles past s_end are left at 0.
+  // stops at t_end (the row maxima of later frames may not even be defined) and rows past s_end
+  // get exact zeros.
   const int t_lim = __builtin_amdgcn_readfirstlane(lim.t_end);
   const int s_lim = __builtin_amdgcn_readfirstlane(min(S1, lim.s_end + 1));
-
-  // what this lane fetches of every slab: D rows sub_a + kRowsA j at k-offset kq_a; am
-  // rows (frames) sub + 8 j at vocabulary offset kq
-  constexpr int kRowsA = Shape::kRowsPerLoad;
-  constexpr int kLoadsA = kLmS / kRowsA, kLoadsB = kLmK / 8;
-  const int sub = lane >> 3, kq = 4 * (lane & 7);
-  const int sub_a = lane / Shape::kRowLanes, kq_a = 4 * (lane % Shape::kRowLanes);
-  floatx4 sa[kLoadsA], sb[kLoadsB];
-  float shift2[kLoadsB];  // -(the frame's maximum) * log2(e)
-  // The loads go through buffer resources that cover D[b] and am[b]: one instruction
-  // each, no branch; a row past the last one lies past the resource and reads as 0.
-  // Frames at and past T (the last slab) must give products of 0: there D is replaced
-  // by 0 (the pad of a D row is not defined; am reads as 0 or holds the next utterance's
-  // frames, exp of which is finite).  Vocabulary columns at and past C belong to the next
-  // row: they only feed output columns that are never written.
-  typedef int intx4 __attribute__((ext_vector_type(4)));
+  // The loads go through buffer resources that cover D[b] and am[b]: one instruction each, no
+  // branch; a row past the last one lies past the resource and reads as 0.  Frames at and past
+  // t_lim must give products of 0: there D is replaced by 0 and am reads as 0, whose
+  // exponential is finite.  Vocabulary columns at and past C belong to the next row: they only
+  // feed output columns that are never written.
   const __amdgpu_buffer_rsrc_t d_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(db), 0, S1 * ldd * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t am_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(amb), 0, T * C * 4, 0x00020000);
-  const int d_off = ((s_tile + sub_a) * ldd + kq_a) * 4, am_off = (sub * C + c_tile + kq) * 4;  // bytes
-  auto as_floats = [](intx4 raw) {
-    return floatx4{__int_as_float(raw[0]), __int_as_float(raw[1]), __int_as_float(raw[2]),
-                   __int_as_float(raw[3])};
-  };
+  // D lies k-contiguous: eight lanes per row; a thread takes rows sub + 32 j at k-offset kq
+  const int sub = tid / 8, kq = 4 * (tid % 8);
+  const int d_off = ((s_tile + sub) * ldd + kq) * 4;
+  const int am_off = (c_tile + lane) * 4;
+  struct {
+    floatx4 d[kM / 32];
+    float a[Shape::kColumns][8], shift2[8];
+  } stage;
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < kLoadsA; ++j)
-      sa[j] = as_floats(__builtin_amdgcn_raw_buffer_load_b128(
-          d_rs, d_off, (kRowsA * j * ldd + k0) * 4, 0));  // (uniform part: scalar register)
-    if (k0 + kLmK > t_lim) {  // (wave-uniform) the slab that holds the last frame
+    for (int j = 0; j < kM / 32; ++j) {
+      const intx4 raw = __builtin_amdgcn_raw_buffer_load_b128(d_rs, d_off, (32 * j * ldd + k0) * 4, 0);
+      stage.d[j] = floatx4{__int_as_float(raw[0]), __int_as_float(raw[1]), __int_as_float(raw[2]),
+                        __int_as_float(raw[3])};
+    }
+    if (k0 + kProdK > t_lim) {  // (uniform) the chunk that holds the last frame
 #pragma unroll
-      for (int j = 0; j < kLoadsA; ++j)
+      for (int j = 0; j < kM / 32; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (k0 + kq_a + i >= t_lim) sa[j][i] = 0.f;
+          if (k0 + kq + i >= t_lim) stage.d[j][i] = 0.f;
     }
 #pragma unroll
-    for (int j = 0; j < kLoadsB; ++j) {
-      const int tr = k0 + sub + 8 * j;
-      sb[j] = as_floats(__builtin_amdgcn_raw_buffer_load_b128(
-          am_rs, am_off, (k0 + 8 * j) * C * 4, 0));
-      shift2[j] = tr < t_lim ? -amx[tr] * kLog2e : 0.f;
-      // a frame past the last one meets D = 0; its factor only has to be finite
-      if (tr >= t_lim) sb[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < Shape::kColumns; ++n)
+      fetch_octet(stage.a[n], am_rs, am_off + 256 * n, k0 + 8 * wave, t_lim, C);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = k0 + 8 * wave + i;
+      const float mx = amx[min(t, t_lim - 1)];
+      stage.shift2[i] = t < t_lim ? -mx * kLog2e : 0.f;
     }
   };
-  const int chunks = (t_lim + kLmK - 1) / kLmK;
-  int chunk = wave;
-  if (chunk < chunks) fetch(chunk * kLmK);
-
-  // epilogue inputs behind the first slab: this thread's pieces of lm (row item / 8,
-  // vocabulary entries 4 (item % 8) ..)
-  floatx4 lm_in[kLmItems];
-#pragma unroll
-  for (int j = 0; j < kLmItems; ++j) {
-    const int item = tid + kLmThreads * j;
-    const int sr = s_tile + item / 8, c = c_tile + 4 * (item % 8);
-    lm_in[j] = load4_guarded(lmb, sr * C + c, sr < S1 ? min(4, max(C - c, 0)) : 0);
+  if (t_lim > 0) fetch(0);
+  if (tid < kM) {
+    const int s = s_tile + tid, at = 4 * s;
+    const long first = (long)b * S1;
+    const float mx = get_float(buffer_of(lm_max + first, S1 * 4), s < s_lim, at);
+    const float rx = get_float(buffer_of(row_x + first, S1 * 4), s < S, at);
+    const float ry = get_float(buffer_of(row_y + first, S1 * 4), s < S1, at);
+    row_sym[tid] = get_symbol(symbols_of(symbols + (long)b * S, S), s < S, s, C);
+    row_mx[tid] = mx, row_rx[tid] = rx, row_ry[tid] = ry;
   }
-  // ... and its rows' maximum, symbol and row sums
-  float row_mx[kLmItems], row_rx[kLmItems], row_ry[kLmItems];
-  int row_sym[kLmItems];
+  const int m_tiles = min(Shape::kMTiles, (s_lim - s_tile - kM / 2 * wave_m + 31) / 32);  // (may be <= 0)
+  floatx16 acc[Shape::kMTiles][Shape::kCTiles];
 #pragma unroll
-  for (int j = 0; j < kLmItems; ++j) {
-    const int sr = s_tile + (tid + kLmThreads * j) / 8;
-    const bool ok = sr < S1;
-    row_mx[j] = ok ? lmx[sr] : 0.f;
-    row_sym[j] = sr < S ? (int)symbols[(long)b * S + sr] : -1;
-    row_rx[j] = ok ? row_x[(long)b * S1 + sr] : 0.f;
-    row_ry[j] = ok ? row_y[(long)b * S1 + sr] : 0.f;
-  }
-
-  const int live_tiles = min(kLmS / 32, (s_lim - s_tile + 31) / 32);  // 32-row tiles with rows that count
-  float *as = lm_lds + wave * kLmSlab;
-  float *bs = as + kLmS * kLmPitch;
-  floatx16 acc[kLmS / 32];
+  for (int j = 0; j < Shape::kMTiles; ++j)
 #pragma unroll
-  for (int j = 0; j < kLmS / 32; ++j)
+    for (int n = 0; n < Shape::kCTiles; ++n)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[j][v] = 0.f;
-  for (; chunk < chunks; chunk += kLmWaves) {
+      for (int v = 0; v < 16; ++v) acc[j][n][v] = 0.f;
+  auto consume = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < kLoadsA; ++j)
-      *reinterpret_cast<floatx4 *>(as + (sub_a + kRowsA * j) * kLmPitch + kq_a) = sa[j];
-#pragma unroll
-    for (int j = 0; j < kLoadsB; ++j) {
-      floatx4 e;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) e[i] = exp_shifted(sb[j][i], shift2[j]);
-      *reinterpret_cast<floatx4 *>(bs + (sub + 8 * j) * kLmC + kq) = e;
+    for (int j = 0; j < kM / 32; ++j) {
+      unsigned h0, h1, m0, m1, l0, l1;
+      split_pair(stage.d[j][0], stage.d[j][1], h0, m0, l0);
+      split_pair(stage.d[j][2], stage.d[j][3], h1, m1, l1);
+      char *to = prod_lds + octet_at<kM, kC>(sub + 32 * j, kq / 8) + 2 * (kq % 8);
+      *reinterpret_cast<uintx2 *>(to) = uintx2{h0, h1};
+      *reinterpret_cast<uintx2 *>(to + 32) = uintx2{m0, m1};
+      *reinterpret_cast<uintx2 *>(to + 64) = uintx2{l0, l1};
     }
-    if (chunk + kLmWaves < chunks) fetch((chunk + kLmWaves) * kLmK);
-    // MFMA i of the slab multiplies frames i (lanes 0..31) and i + kK / 2 (lanes 32..63) -- the
-    // order in which a slab's frames are summed is free -- so that a lane takes its D row's
-    // share of the slab with 16-byte reads
-    constexpr int kHalfK = kLmK / 2;
-    const float *ap = as + r32 * kLmPitch + kHalfK * half;
-    const float *bp = bs + kHalfK * half * kLmC + r32;
-    float bv[kHalfK];
 #pragma unroll
-    for (int i = 0; i < kHalfK; ++i) bv[i] = bp[i * kLmC];
+    for (int n = 0; n < Shape::kColumns; ++n) {
+      float e[8];
 #pragma unroll
-    for (int j = 0; j < kLmS / 32; ++j)
-      if (j < live_tiles) {
+      for (int i = 0; i < 8; ++i) e[i] = exp_shifted(stage.a[n][i], stage.shift2[i]);
+      write_octet(prod_lds + octet_at<kM, kC>(kM + lane + 64 * n, wave), e);
+    }
+    if (k0 + kProdK < t_lim) fetch(k0 + kProdK);
+    lds_barrier();
+    multiply_chunk<kM, kC>(prod_lds, wave_m, wave_n, half, r32, m_tiles, acc);
+    lds_barrier();  // the operands have been read
+  };
+  for (int k0 = 0; k0 < t_lim; k0 += kProdK) consume(k0);
+  if (t_lim <= 0) lds_barrier();
+
+  // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
+  // (the exponentials' arguments of all tiles are requested together)
+  const __amdgpu_buffer_rsrc_t lm_rs = buffer_of(lmb, S1 * C * 4);
+  const __amdgpu_buffer_rsrc_t out_rs = out_buffer(lm_grad, (long)b * S1 * C, S1 * C, out_type);
+  const int m0 = kM / 2 * wave_m + 4 * half, c0 = c_tile + (kC / 2) * wave_n + r32;
+  auto row_of = [&](int j, int v) { return m0 + 32 * j + 8 * (v / 4) + v % 4; };
+  const int first = (s_tile + m0) * C + c0;  // (element)
+  auto below = [&](int j, int v) { return (32 * j + 8 * (v / 4) + v % 4) * C; };  // (uniform)
+  float in[Shape::kMTiles][Shape::kCTiles][16];
 #pragma unroll
-        for (int i4 = 0; i4 < kHalfK / 4; ++i4) {
-          const floatx4 a = *reinterpret_cast<const floatx4 *>(ap + j * 32 * kLmPitch + 4 * i4);
+  for (int j = 0; j < Shape::kMTiles; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], bv[4 * i4 + i], acc[j], 0, 0, 0);
+    for (int n = 0; n < Shape::kCTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        in[j][n][v] = get_float(lm_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(j, v));
+  with_store(out_type, [&](auto store) {
+#pragma unroll
+    for (int j = 0; j < Shape::kMTiles; ++j)
+#pragma unroll
+      for (int n = 0; n < Shape::kCTiles; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = row_of(j, v), s = s_tile + m, c = c0 + 32 * n;
+          float g = __expf(in[j][n][v] - row_mx[m]) * acc[j][n][v];
+          if (c == row_sym[m]) g += row_rx[m];
+          if (c == term) g += row_ry[m];
+          store(out_rs, c < C, first + 32 * n, below(j, v), s < s_lim ? g : 0.f);
         }
-      }
-  }
-
-  // the partial sums meet: [wave][kS][33] in the slab space
-  __syncthreads();
-  float *part = lm_lds + wave * Shape::kSums;
-#pragma unroll
-  for (int j = 0; j < kLmS / 32; ++j)
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-      part[(32 * j + 8 * (v / 4) + 4 * half + (v % 4)) * kLmOutPitch + r32] = acc[j][v];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < kLmItems; ++j) {
-    const int item = tid + kLmThreads * j;
-    const int m = item / 8, n = 4 * (item % 8), sr = s_tile + m, c = c_tile + n;
-    if (sr >= S1 || c >= C) continue;
-    const float mx = row_mx[j], rx = row_rx[j], ry = row_ry[j];
-    const int sym = row_sym[j];
-    float g[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float sum = 0.f;
-#pragma unroll
-      for (int w = 0; w < kLmWaves; ++w)
-        sum += lm_lds[w * Shape::kSums + m * kLmOutPitch + n + i];
-      g[i] = __expf(lm_in[j][i] - mx) * sum;
-      if (c + i == sym) g[i] += rx;
-      if (c + i == term) g[i] += ry;
-    }
-    float *dst = lm_grad + ((long)b * S1 + sr) * C + c;
-    if (c + 4 <= C) {
-      *reinterpret_cast<floatx4u *>(dst) = floatx4u{g[0], g[1], g[2], g[3]};
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c + i < C) dst[i] = g[i];
-    }
-  }
+  });
 }
 
-// am gradient, LDS-panel form.  k runs over the S+1 lattice rows, which is short, so
-// a workgroup brings ALL of k (up to 128 rows per pass) for its 64 (frames) x 64
-// (vocabulary) tile into LDS: D[k][t] and exp(lm[k][c] - max[k]) are both contiguous
-// along the output dimension, so the panels arrive as coalesced 16-byte loads, and the
-// matrix cores read the dense product's operands from LDS only.  What bounds this kernel is the number of
-// vector-memory INSTRUCTIONS a compute unit can retire (an instruction costs about
-// the same whether it moves 4 or 16 bytes per lane), so every global access here is
-// 16 bytes wide and row-contiguous: the am tile comes in that way too, and the
-// result leaves through an LDS transpose as whole 256-byte row segments.
-// Every global load is in flight before the first one is consumed: a workgroup pays
-// one memory round trip.
-// The per-symbol term  sum_s [c = sym[b,s]] gx[b,s,t]  is a second product on the
-// matrix core, gx^T times a one-hot matrix made in registers from the symbols: it is
-// exact (products by 0 or 1) and has a fixed summation order; k-pairs none of whose
-// symbols falls into the wave's 32 vocabulary columns are skipped (wave-uniform).  With
-// a large vocabulary almost every pair is skipped, so gx has no panel: a wave reads the
-// few 128-byte row pieces it needs straight from memory, the first eight of them
-// requested before the dense product so that they arrive under it.
-constexpr int kAmT = 64;       // frames per workgroup
-constexpr int kAmC = 64;       // vocabulary entries per workgroup
-constexpr int kAmHotAhead = 8; // per-symbol pairs whose gx values are requested ahead
-constexpr int kAmOutPitch = 68;  // row pitch of the result tiles staged in LDS
-constexpr int kAmQ = kAmT / 4;   // 16-byte pieces per panel row (kAmT == kAmC)
-
-constexpr int kAmCap = 64;     // most lattice rows per pass
-// rows of k per pass: passes of equal (even) size, none above kAmCap
-int am_rows_per_pass(int S) {
-  const int passes = (S + 1 + kAmCap - 1) / kAmCap;
-  return std::min(kAmCap, ((S + 1 + passes - 1) / passes + 1) & ~1);
-}
-size_t am_panel_lds_bytes(int rows_cap) {
-  const size_t panels = (size_t)rows_cap * (kAmT + kAmC) * sizeof(float);
-  const size_t staging = (size_t)2 * kAmT * kAmOutPitch * sizeof(float);
-  return std::max(panels, staging) + (size_t)(2 * rows_cap + 2 * kAmT) * sizeof(float);
-}
-
-// kCap: most lattice rows a pass may hold (the launch's rows_cap is at most that); it sets
-// how many panel pieces a thread keeps in registers.
-template <int kCap>
-__device__ __forceinline__ void simple_bwd_am_panel_body(
+// The per-symbol term of am.grad,  sum_s [c = sym[b,s]] gx[b,s,t],  is a second product, gx^T times
+// a one-hot matrix made in registers from the symbols, on the float32 matrix instruction: it is
+// exact (products by 0 or 1) and has a fixed summation order.  The lattice rows whose symbol lies
+// in the workgroup's vocabulary range are listed in order; their gx rows go to LDS, some at a
+// time, and are multiplied two rows at a time onto the finished dense results.
+template <int kM, int kC>
+__device__ __forceinline__ void simple_bwd_am_body(
     int block_id, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const int64_t *__restrict__ boundary,
     const float *__restrict__ lm_max, const float *__restrict__ am_max,
     const float *__restrict__ dmat, const float *__restrict__ gpx,
-    const float *__restrict__ row_x, const float *__restrict__ col_y,
-    float *__restrict__ am_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
-    int ldd, int term, int rnnt_type, int rows_cap, int part_shift) {
+    const float *__restrict__ gpy, const float *__restrict__ row_x,
+    void *__restrict__ am_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
+    int ldd, int term, int rnnt_type, int part_shift, int out_type) {
+  using Shape = ProdShape<kM, kC>;
   using namespace dgemm;
-  extern __shared__ __align__(16) float am_lds[];
-  int *sym_s = reinterpret_cast<int *>(am_lds);   // [rows_cap] symbols of the pass (-1: none)
-  float *lmx_s = am_lds + rows_cap;               // [rows_cap] lm_max of the pass
-  float *shift_s = lmx_s + rows_cap;              // [kAmT] am_max of the tile's frames
-  float *extra_s = shift_s + kAmT;                // [kAmT] col_y of the tile's frames
-  float *As = extra_s + kAmT;                     // [rows_cap][kAmT]   D[k][t]
-  float *Bs = As + rows_cap * kAmT;               // [rows_cap][kAmC]   exp(lm[k][c] - max[k])
-  float *out_acc = As;                            // result tiles, after the last pass
-  float *out_hot = As + kAmT * kAmOutPitch;
+  extern __shared__ __align__(16) char prod_lds[];
+  __shared__ float frame_mx[kM], frame_y[4][kM];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
-  const int c_tiles = (C + kAmC - 1) / kAmC, t_tiles = (T + kAmT - 1) / kAmT;
+  const int c_tiles = (C + kC - 1) / kC, t_tiles = (T + kM - 1) / kM;
   int b, tile;
   Limits lim;
   if (!place_block(block_id, c_tiles, t_tiles, part_shift, B, row_x, window, S, T, b, tile, lim))
     return;
-  const int t_tile = (tile / c_tiles) * kAmT, c_tile = (tile % c_tiles) * kAmC;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t_tile = (tile / c_tiles) * kM, c_tile = (tile % c_tiles) * kC;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_m = wave >> 1, wave_n = wave & 1;
   const int half = lane >> 5, r32 = lane & 31;
-  const int wt = (wave >> 1) * 32, wc = (wave & 1) * 32;  // this wave's 32 x 32 sub-tile
   const float *lmb = lm + (long)b * S1 * C;
   const float *amb = am + (long)b * T * C;
+  const float *lmx = lm_max + (long)b * S1;
   const float *db = dmat + (long)b * S1 * ldd;
   const float *gxb = gpx + (long)b * S * T1;
-  // symbols are < C < 2^31: their low words (little endian) are enough to compare
-  const int *sym_lo = reinterpret_cast<const int *>(symbols + (long)b * S);
+  const __amdgpu_buffer_rsrc_t sym_rs = symbols_of(symbols + (long)b * S, S);
   const int t_mask = (rnnt_type == kRegular && boundary) ? (int)boundary[4 * b + 3] : -1;
-  const int c_lo = c_tile + wc;  // first vocabulary column of this wave
-  // a thread's 16-byte piece of a 64-wide row: row q_row + 16 * step, columns 4 * q_col ..
-  const int q_row = tid / kAmQ, q_col = 4 * (tid % kAmQ);
   // With a window, D vanishes on rows > s_end and at frames >= t_end, where the frames'
   // maxima may not even be defined: such frames get exact zeros, the sum over the lattice
-  // rows stops at s_end, and a tile without a frame below t_end only stores zeros.
-  const int t_lim = lim.t_end, k_lim = min(S1, lim.s_end + 1);
-  if (t_tile >= t_lim) {
+  // rows stops at s_end.
+  const int t_lim = __builtin_amdgcn_readfirstlane(lim.t_end);
+  const int k_lim = __builtin_amdgcn_readfirstlane(min(S1, lim.s_end + 1));
+  const bool live = t_tile < t_lim;
+  const __amdgpu_buffer_rsrc_t am_rs = buffer_of(amb, T * C * 4);
+  const __amdgpu_buffer_rsrc_t out_rs = out_buffer(am_grad, (long)b * T * C, T * C, out_type);
+  const int m0 = kM / 2 * wave_m + 4 * half, c_lo = c_tile + (kC / 2) * wave_n, c0 = c_lo + r32;
+  auto row_of = [&](int j, int v) { return m0 + 32 * j + 8 * (v / 4) + v % 4; };
+  const int first = (t_tile + m0) * C + c0;  // (element)
+  auto below = [&](int j, int v) { return (32 * j + 8 * (v / 4) + v % 4) * C; };  // (uniform)
+  floatx16 acc[Shape::kMTiles][Shape::kCTiles];
 #pragma unroll
-    for (int j = 0; j < kAmT / 16; ++j) {
-      const int t = t_tile + q_row + 16 * j, c = c_tile + q_col;
-      if (t >= T || c >= C) continue;
-      float *dst = am_grad + ((long)b * T + t) * C + c;
-      if (c + 4 <= C) {
-        *reinterpret_cast<floatx4u *>(dst) = floatx4u{0.f, 0.f, 0.f, 0.f};
-      } else {
-        for (int i = 0; i < 4; ++i)
-          if (c + i < C) dst[i] = 0.f;
+  for (int j = 0; j < Shape::kMTiles; ++j)
+#pragma unroll
+    for (int n = 0; n < Shape::kCTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[j][n][v] = 0.f;
+  if (live) {
+    // (resources as in the kernel above; frames at and past T of D's rows only feed outputs that
+    // are never written, lattice rows that do not count read as 0)
+    const __amdgpu_buffer_rsrc_t d_rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(db), 0, S1 * ldd * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t lm_rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(lmb), 0, S1 * C * 4, 0x00020000);
+    const int d_off = (t_tile + lane) * 4, lm_off = (c_tile + lane) * 4;
+    struct {
+      float d[Shape::kMColumns][8], l[Shape::kColumns][8], shift2[8];
+    } stage;
+    auto fetch = [&](int k0) {
+#pragma unroll
+      for (int n = 0; n < Shape::kMColumns; ++n)
+        fetch_octet(stage.d[n], d_rs, d_off + 256 * n, k0 + 8 * wave, k_lim, ldd);
+#pragma unroll
+      for (int n = 0; n < Shape::kColumns; ++n)
+        fetch_octet(stage.l[n], lm_rs, lm_off + 256 * n, k0 + 8 * wave, k_lim, C);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int k = k0 + 8 * wave + i;
+        const float mx = lmx[min(k, k_lim - 1)];
+        stage.shift2[i] = k < k_lim ? -mx * kLog2e : 0.f;
       }
-    }
-    return;
-  }
-
-  // epilogue inputs: per-frame terms through LDS (visible after the barriers of the
-  // first pass), and this thread's pieces of the am tile, rows q_row + 16 * j
-  if (tid < kAmT) {
-    const int t = t_tile + tid;
-    shift_s[tid] = t < t_lim ? am_max[(long)b * T + t] : 0.f;
-    extra_s[tid] = t < t_lim ? col_y[(long)b * T + t] : 0.f;
-  }
-  // The panel and tile loads go through buffer resources that cover D[b], lm[b] and
-  // am[b]: one instruction each, no branch, any alignment.  A row past the last one lies
-  // past the resource and reads as 0; a column past the end of a row belongs to the next
-  // row, and only feeds frames >= T or vocabulary entries >= C, which are never written.
-  typedef int intx4 __attribute__((ext_vector_type(4)));
-  // (rows that do not count lie past the resources: they read as 0 and move no data)
-  const __amdgpu_buffer_rsrc_t d_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(db), 0, k_lim * ldd * 4, 0x00020000);
-  const __amdgpu_buffer_rsrc_t lm_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(lmb), 0, k_lim * C * 4, 0x00020000);
-  const __amdgpu_buffer_rsrc_t am_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(amb), 0, T * C * 4, 0x00020000);
-  auto get4 = [](__amdgpu_buffer_rsrc_t rs, int byte_offset) {
-    const intx4 raw = __builtin_amdgcn_raw_buffer_load_b128(rs, byte_offset, 0, 0);
-    return floatx4{__int_as_float(raw[0]), __int_as_float(raw[1]), __int_as_float(raw[2]),
-                   __int_as_float(raw[3])};
-  };
-  floatx4 am_in[kAmT / 16];
-#pragma unroll
-  for (int j = 0; j < kAmT / 16; ++j)
-    am_in[j] = get4(am_rs, ((t_tile + q_row + 16 * j) * C + c_tile + q_col) * 4);
-
-  floatx16 acc, hot;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = hot[v] = 0.f;
-  constexpr int kSteps = kCap / 16;
-  constexpr int kNowhere = (int)0x80000000;  // an offset outside every resource: reads 0, moves nothing
-  floatx4 ra[kSteps], rb[kSteps];
-  // a pass's pieces of the two panels: rows k0 + q_row + 16 j of D and of lm, while they
-  // belong to the pass
-  auto request = [&](int k0) {
-    const int end = min(k0 + rows_cap, k_lim);
-#pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-      const int k = k0 + q_row + 16 * j;
-      ra[j] = get4(d_rs, k < end ? (k * ldd + t_tile + q_col) * 4 : kNowhere);
-      rb[j] = get4(lm_rs, k < end ? (k * C + c_tile + q_col) * 4 : kNowhere);
-    }
-  };
-  request(0);
-  for (int k0 = 0; k0 < k_lim; k0 += rows_cap) {
-    const int rows = min(rows_cap, k_lim - k0);
-    const int pairs = (rows + 1) / 2;
-    if (k0 > 0) __syncthreads();  // the previous pass's readers are done with the panels
-    for (int k = tid; k < 2 * pairs; k += 256) {
-      sym_s[k] = (k0 + k < S) ? sym_lo[2 * (k0 + k)] : -1;
-      lmx_s[k] = (k < rows) ? lm_max[(long)b * S1 + k0 + k] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-      const int k = q_row + 16 * j;
-      if (k >= 2 * pairs) continue;
-      *reinterpret_cast<floatx4 *>(As + k * kAmT + q_col) = ra[j];
-    }
-    __syncthreads();  // lmx_s and sym_s are visible
-    // per-symbol product: the pairs with a symbol among this wave's columns ...
-    bool in = false;
-    if (lane < pairs)
-      in = (unsigned)(sym_s[2 * lane] - c_lo) < 32u || (unsigned)(sym_s[2 * lane + 1] - c_lo) < 32u;
-    unsigned long long wanted = __ballot(in);
-    // ... and this lane's gx[k][t] of pair i (k = 2 i + half, t = the wave's frame r32):
-    // nothing for the masked frame, past T or past the last symbol
-    const int hot_t = t_tile + wt + r32;
-    const bool hot_ok = hot_t < T && hot_t != t_mask;
-    auto hot_value = [&](int i) {
-      const int k = k0 + 2 * i + half;
-      return (hot_ok && k < S) ? gxb[(long)k * T1 + hot_t] : 0.f;
     };
-    int ahead[kAmHotAhead];
-    float ahead_v[kAmHotAhead];
+    if (k_lim > 0) fetch(0);
+    if (tid < kM) {
+      const int t = t_tile + tid;
+      const float mx = get_float(buffer_of(am_max + (long)b * T, T * 4), t < t_lim, 4 * t);
+      frame_mx[tid] = mx;
+    }
+    const int m_tiles = min(Shape::kMTiles, (t_lim - t_tile - kM / 2 * wave_m + 31) / 32);  // (may be <= 0)
+    auto consume = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < kAmHotAhead; ++u) {
-      ahead[u] = -1;
-      ahead_v[u] = 0.f;
-      if (wanted) {
-        ahead[u] = __builtin_ctzll(wanted);
-        wanted &= wanted - 1;
-        ahead_v[u] = hot_value(ahead[u]);
+      for (int n = 0; n < Shape::kMColumns; ++n)
+        write_octet(prod_lds + octet_at<kM, kC>(lane + 64 * n, wave), stage.d[n]);
+#pragma unroll
+      for (int n = 0; n < Shape::kColumns; ++n) {
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = exp_shifted(stage.l[n][i], stage.shift2[i]);
+        write_octet(prod_lds + octet_at<kM, kC>(kM + lane + 64 * n, wave), e);
+      }
+      if (k0 + kProdK < k_lim) fetch(k0 + kProdK);
+      lds_barrier();
+      multiply_chunk<kM, kC>(prod_lds, wave_m, wave_n, half, r32, m_tiles, acc);
+      lds_barrier();  // the operands have been read
+    };
+    for (int k0 = 0; k0 < k_lim; k0 += kProdK) consume(k0);
+  }
+
+  // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
+  if (live) {
+    // the exponentials' arguments of all tiles are requested together
+    float in[Shape::kMTiles][Shape::kCTiles][16];
+#pragma unroll
+    for (int j = 0; j < Shape::kMTiles; ++j)
+#pragma unroll
+      for (int n = 0; n < Shape::kCTiles; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          in[j][n][v] = get_float(am_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(j, v));
+    // The termination symbol's term, sum_s gy[s,t], in the workgroups that hold its column: every
+    // wave sums a quarter of the lattice rows.
+    const __amdgpu_buffer_rsrc_t gx_rs = buffer_of(gxb, S * T1 * 4);
+    if ((unsigned)(term - c_tile) < (unsigned)kC) {  // (uniform)
+      const __amdgpu_buffer_rsrc_t gy_rs = buffer_of(gpy + (long)b * S1 * T, S1 * T * 4);
+      float sum[Shape::kMColumns] = {};
+      constexpr int kAhead = 8;
+      auto add_rows = [&](__amdgpu_buffer_rsrc_t rs, int rows, int pitch) {
+        for (int s0 = wave; s0 < rows; s0 += 4 * kAhead) {
+          float y[kAhead][Shape::kMColumns];
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int w = 0; w < Shape::kMColumns; ++w) {
+              const int s = s0 + 4 * u, t = t_tile + lane + 64 * w;
+              y[u][w] = get_float(rs, s < rows && t >= lim.t_begin && t < t_lim, 4 * t, s * pitch * 4);
+            }
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int w = 0; w < Shape::kMColumns; ++w) sum[w] += y[u][w];
+        }
+      };
+      add_rows(gy_rs, k_lim, T);
+      // (constrained: py[s + 1] also went into px[s])
+      if (rnnt_type == kConstrained) add_rows(gx_rs, min(k_lim, S), T1);
+#pragma unroll
+      for (int w = 0; w < Shape::kMColumns; ++w) frame_y[wave][lane + 64 * w] = sum[w];
+      lds_barrier();
+    }
+    constexpr int kHotPitch = kM + 4;
+    constexpr int kHotRows = kM == 128 ? 64 : 32;  // rows of the list in LDS at a time
+    static_assert(Shape::kLdsBytes >= kHotRows * (kHotPitch + 1) * 4, "room for the listed rows");
+    float *hot = reinterpret_cast<float *>(prod_lds);
+    int *hot_sym = reinterpret_cast<int *>(hot + kHotRows * kHotPitch);
+    const int s_count = min(k_lim, S);
+    auto multiply_hot = [&](int listed) {
+      lds_barrier();  // the listed rows are in LDS
+      for (int i = 0; i < listed; i += 2) {
+        const int row = i + half;
+        const int sym = row < listed ? hot_sym[row] : -1;
+        // (wave-uniform) does one of the two fall into this wave's columns
+        if (!__any((unsigned)(sym - c_lo) < (unsigned)(kC / 2))) continue;
+        float value[Shape::kMTiles];
+#pragma unroll
+        for (int j = 0; j < Shape::kMTiles; ++j)
+          value[j] = row < listed ? hot[row * kHotPitch + kM / 2 * wave_m + 32 * j + r32] : 0.f;
+#pragma unroll
+        for (int n = 0; n < Shape::kCTiles; ++n) {
+          const float one = sym == c0 + 32 * n ? 1.f : 0.f;
+          if (!__any(one != 0.f)) continue;
+#pragma unroll
+          for (int j = 0; j < Shape::kMTiles; ++j)
+            acc[j][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(value[j], one, acc[j][n], 0, 0, 0);
+        }
+      }
+      lds_barrier();  // ... and have been read
+    };
+    auto finish_dense = [&]() {
+#pragma unroll
+      for (int j = 0; j < Shape::kMTiles; ++j)
+#pragma unroll
+        for (int n = 0; n < Shape::kCTiles; ++n)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int m = row_of(j, v);
+            acc[j][n][v] *= __expf(in[j][n][v] - frame_mx[m]);
+            if (c0 + 32 * n == term)
+              acc[j][n][v] += (frame_y[0][m] + frame_y[1][m]) + (frame_y[2][m] + frame_y[3][m]);
+          }
+    };
+    int listed = 0;
+    bool dense_done = false;
+    for (int s0 = 0; s0 < s_count; s0 += kWave) {
+      const int sym = get_symbol(sym_rs, s0 + lane < s_count, s0 + lane, C);
+      unsigned long long hits = __ballot((unsigned)(sym - c_tile) < (unsigned)kC);
+      while (hits) {  // (uniform over the workgroup)
+        // the next sixteen rows of the list, four per wave: kM frames each (nothing for the masked
+        // frame and past T), requested together
+        int row[4];
+        const int old = listed;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          if (u % 4 == 0) row[u / 4] = -1;
+          const int at = hits ? __builtin_ctzll(hits) : -1;
+          if (u % 4 == wave) row[u / 4] = at;
+          listed += hits ? 1 : 0;
+          hits &= hits - 1;
+        }
+        float value[4][Shape::kMColumns];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int w = 0; w < Shape::kMColumns; ++w) {
+            const int t = t_tile + lane + 64 * w;
+            value[u][w] = get_float(gx_rs, row[u] >= 0 && t < T && t != t_mask,
+                                    ((s0 + row[u]) * T1 + t) * 4);
+          }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (row[u] < 0) continue;  // (wave-uniform)
+          const int slot = old + 4 * u + wave;
+#pragma unroll
+          for (int w = 0; w < Shape::kMColumns; ++w) hot[slot * kHotPitch + lane + 64 * w] = value[u][w];
+          const int its = __builtin_amdgcn_readlane(sym, row[u]);
+          if (lane == 0) hot_sym[slot] = its;
+        }
+        if (listed > kHotRows - 16) {
+          if (!dense_done) finish_dense();
+          dense_done = true;
+          multiply_hot(listed);
+          listed = 0;
+        }
       }
     }
-#pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-      const int k = q_row + 16 * j, c = c_tile + q_col;
-      if (k >= 2 * pairs) continue;
-      const float mx = lmx_s[k];
-      floatx4 e;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) e[i] = (k < rows && c + i < C) ? __expf(rb[j][i] - mx) : 0.f;
-      *reinterpret_cast<floatx4 *>(Bs + k * kAmC + q_col) = e;
-    }
-    // the next pass's panels are on their way while this one is multiplied
-    if (k0 + rows_cap < k_lim) request(k0 + rows_cap);
-    __syncthreads();
-    // dense product
-    const float *ap = As + half * kAmT + wt + r32;
-    const float *bp = Bs + half * kAmC + wc + r32;
-#pragma unroll 4
-    for (int i = 0; i < pairs; ++i)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[2 * i * kAmT], bp[2 * i * kAmC], acc, 0, 0, 0);
-    // per-symbol product
-#pragma unroll
-    for (int u = 0; u < kAmHotAhead; ++u) {
-      if (ahead[u] < 0) continue;
-      const float h = (sym_s[2 * ahead[u] + half] == c_lo + r32) ? 1.f : 0.f;
-      hot = __builtin_amdgcn_mfma_f32_32x32x2f32(ahead_v[u], h, hot, 0, 0, 0);
-    }
-    while (wanted) {
-      const int i = __builtin_ctzll(wanted);
-      wanted &= wanted - 1;
-      const float h = (sym_s[2 * i + half] == c_lo + r32) ? 1.f : 0.f;
-      hot = __builtin_amdgcn_mfma_f32_32x32x2f32(hot_value(i), h, hot, 0, 0, 0);
-    }
+    if (!dense_done) finish_dense();
+    if (listed > 0) multiply_hot(listed);
   }
-  // results through LDS, so that they leave as whole row segments
-  __syncthreads();
+  with_store(out_type, [&](auto store) {
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = wt + 8 * (v / 4) + 4 * half + (v % 4);
-    out_acc[row * kAmOutPitch + wc + r32] = acc[v];
-    out_hot[row * kAmOutPitch + wc + r32] = hot[v];
-  }
-  __syncthreads();
+    for (int j = 0; j < Shape::kMTiles; ++j)
 #pragma unroll
-  for (int j = 0; j < kAmT / 16; ++j) {
-    const int row = q_row + 16 * j, t = t_tile + row, c = c_tile + q_col;
-    if (t >= T || c >= C) continue;
-    const floatx4 sum = *reinterpret_cast<const floatx4 *>(out_acc + row * kAmOutPitch + q_col);
-    const floatx4 one = *reinterpret_cast<const floatx4 *>(out_hot + row * kAmOutPitch + q_col);
-    const float shift = shift_s[row], extra = extra_s[row];
-    floatx4 res;
+      for (int n = 0; n < Shape::kCTiles; ++n)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      res[i] = __expf(am_in[j][i] - shift) * sum[i] + one[i];
-      if (c + i == term) res[i] += extra;
-      if (t >= t_lim) res[i] = 0.f;
-    }
-    float *dst = am_grad + ((long)b * T + t) * C + c;
-    if (c + 4 <= C) {
-      *reinterpret_cast<floatx4u *>(dst) = floatx4u{res[0], res[1], res[2], res[3]};
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c + i < C) dst[i] = res[i];
-    }
-  }
+        for (int v = 0; v < 16; ++v) {
+          const int t = t_tile + row_of(j, v);
+          store(out_rs, c0 + 32 * n < C, first + 32 * n, below(j, v), t < t_lim ? acc[j][n][v] : 0.f);
+        }
+  });
 }
 
-// launchers: float goes to the slab / panel kernels, double to the LDS-tiled ones
-
+// launchers: float goes to the product kernels above, double to the LDS-tiled ones
 void launch_fwd_gemm(const float *lm, const float *am, const int64_t *symbols,
                      const int64_t *boundary, float *lm_max, float *am_max, float *px,
-                     float *py, float *norm_raw, const int64_t *window, int B, int S, int T,
-                     int C, int term, int rnnt_type, hipStream_t stream) {
-  launch_normalizer_f32(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw, window, B, S,
-                        T, C, term, rnnt_type, stream);
+                     float *py, float *norm_raw, const int64_t *window, float *workspace,
+                     double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
+                     hipStream_t stream) {
+  launch_normalizer_f32(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw, window,
+                        workspace, delay_penalty, B, S, T, C, term, rnnt_type, stream);
 }
 void launch_fwd_gemm(const double *lm, const double *am, const int64_t *symbols,
                      const int64_t *boundary, const double *lm_max, const double *am_max,
-                     double *px, double *py, double *norm_raw, const int64_t *, int B, int S,
-                     int T, int C, int term, int rnnt_type, hipStream_t stream) {
+                     double *px, double *py, double *norm_raw, const int64_t *, double *,
+                     double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
+                     hipStream_t stream) {
   // (the double kernels compute the whole lattice whether or not a window is given)
   const int t_tiles = T > 0 ? (T + kTileN - 1) / kTileN : 1;
   const dim3 grid(t_tiles, (S + 1 + kTileM - 1) / kTileM, B);
   hipLaunchKernelGGL(simple_fwd_kernel<double>, grid, dim3(kGemmThreads), 0, stream, lm, am,
-                     symbols, boundary, lm_max, am_max, px, py, norm_raw, S, T, C, term,
-                     rnnt_type);
-}
-template <int kS, int kK>
-__global__ void __launch_bounds__(kLmThreads, 2)
-    simple_bwd_lm_slab_kernel(const float *__restrict__ lm, const float *__restrict__ am,
-                              const int64_t *__restrict__ symbols,
-                              const float *__restrict__ lm_max,
-                              const float *__restrict__ am_max, const float *__restrict__ dmat,
-                              const float *__restrict__ row_x, const float *__restrict__ row_y,
-                              float *__restrict__ lm_grad, const int64_t *__restrict__ window,
-                              int B, int S, int T, int C, int ldd, int term, int part_shift) {
-  simple_bwd_lm_slab_body<kS, kK>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
-                                  row_y, lm_grad, window, B, S, T, C, ldd, term, part_shift);
-}
-template <int kCap, int kPerCu>
-__global__ void __launch_bounds__(256, kPerCu)
-    simple_bwd_am_panel_kernel(const float *__restrict__ lm, const float *__restrict__ am,
-                               const int64_t *__restrict__ symbols,
-                               const int64_t *__restrict__ boundary,
-                               const float *__restrict__ lm_max,
-                               const float *__restrict__ am_max, const float *__restrict__ dmat,
-                               const float *__restrict__ gpx, const float *__restrict__ row_x,
-                               const float *__restrict__ col_y, float *__restrict__ am_grad,
-                               const int64_t *__restrict__ window, int B, int S, int T, int C,
-                               int ldd, int term, int rnnt_type, int rows_cap, int part_shift) {
-  simple_bwd_am_panel_body<kCap>((int)blockIdx.x, lm, am, symbols, boundary, lm_max, am_max, dmat,
-                                 gpx, row_x, col_y, am_grad, window, B, S, T, C, ldd, term,
-                                 rnnt_type, rows_cap, part_shift);
+                     symbols, boundary, lm_max, am_max, px, py, norm_raw,
+                     Delay<double>{delay_penalty}, S, T, C, term, rnnt_type);
 }
 // Both gradient products in one launch: the first lm_blocks workgroups take tiles of
 // lm.grad, the rest tiles of am.grad.  The two only read what the prep kernel left, so
-// their workgroups share the chip.  The order matters: the am tiles are short and mostly
-// wait for memory, and fill the end of the launch better than the lm tiles do (c2 shape:
-// 30.4 us with the lm tiles first, 33.2 with the am tiles first, 36.9 with the two kinds
-// dealt out alternately).  lm_blocks is a multiple of 8, so a workgroup's XCD is the same
-// in both numberings.
-static_assert(kLmThreads == 256, "the two kinds of workgroup must have the same size");
-template <int kS, int kK>
-__global__ void __launch_bounds__(256, 2)
+// their workgroups share the chip.  lm_blocks is a multiple of 8, so a workgroup's XCD is the same
+// in both numberings.  (One after the other they take as long at the large sizes and 5 to 10 us
+// longer where either leaves the chip partly idle.)
+template <int kMl, int kMa>
+__global__ void __launch_bounds__(kProdThreads, kProdPerCu)
     simple_bwd_am_lm_kernel(const float *__restrict__ lm, const float *__restrict__ am,
                             const int64_t *__restrict__ symbols,
                             const int64_t *__restrict__ boundary,
                             const float *__restrict__ lm_max, const float *__restrict__ am_max,
                             const float *__restrict__ dmat, const float *__restrict__ gpx,
-                            const float *__restrict__ row_x, const float *__restrict__ row_y,
-                            const float *__restrict__ col_y, float *__restrict__ lm_grad,
-                            float *__restrict__ am_grad, const int64_t *__restrict__ window, int B,
-                            int S, int T, int C, int ldd, int term, int rnnt_type, int rows_cap,
-                            int lm_blocks, int lm_part_shift, int am_part_shift) {
+                            const float *__restrict__ gpy, const float *__restrict__ row_x,
+                            const float *__restrict__ row_y, void *__restrict__ lm_grad,
+                            void *__restrict__ am_grad, const int64_t *__restrict__ window, int B,
+                            int S, int T, int C, int ldd, int term, int rnnt_type,
+                            int lm_blocks, int part_shift, int out_type) {
   if ((int)blockIdx.x < lm_blocks)
-    simple_bwd_lm_slab_body<kS, kK>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
-                                    row_y, lm_grad, window, B, S, T, C, ldd, term, lm_part_shift);
+    simple_bwd_lm_body<kMl, kProdC>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
+                                    row_y, lm_grad, window, B, S, T, C, ldd, term, part_shift,
+                                    out_type);
   else
-    simple_bwd_am_panel_body<kAmCap>((int)blockIdx.x - lm_blocks, lm, am, symbols, boundary, lm_max,
-                                     am_max, dmat, gpx, row_x, col_y, am_grad, window, B, S, T, C,
-                                     ldd, term, rnnt_type, rows_cap, am_part_shift);
+    simple_bwd_am_body<kMa, kProdC>((int)blockIdx.x - lm_blocks, lm, am, symbols, boundary, lm_max,
+                                    am_max, dmat, gpx, gpy, row_x, am_grad, window, B, S, T, C,
+                                    ldd, term, rnnt_type, part_shift, out_type);
 }
-// lm.grad and am.grad together (float only)
-void launch_bwd_both(const float *lm, const float *am, const int64_t *symbols,
-                     const int64_t *boundary, const float *lm_max, const float *am_max,
-                     const float *dmat, const float *gpx, const float *row_x, const float *row_y,
-                     const float *col_y, float *lm_grad, float *am_grad, const int64_t *window,
-                     int B, int S, int T, int C, int ldd, int term, int rnnt_type,
-                     hipStream_t stream) {
-  const int S1 = S + 1;
-  const bool rows96 = (S1 + 95) / 96 * 96 < (S1 + 127) / 128 * 128;
-  const int rows = rows96 ? 96 : 128;
-  const int lm_c = (C + kLmC - 1) / kLmC, am_c = (C + kAmC - 1) / kAmC;
-  const int lm_shift = part_shift_for(B, lm_c), am_shift = part_shift_for(B, am_c);
-  const int rows_cap = am_rows_per_pass(S);
-  // (frames in slabs of 16 here also for the 96-row form: its LDS is then 50 KB, not 67,
-  // and three workgroups fit on a CU whichever product they work on: 33.4 us against 36.2)
-  const size_t lm_lds = rows96 ? LmShape<96, 16>::kLdsBytes : LmShape<128, 16>::kLdsBytes;
-  const size_t lds = std::max(lm_lds, am_panel_lds_bytes(rows_cap));
-  const unsigned am_blocks = placed_grid(am_c, (T + kAmT - 1) / kAmT, B, am_shift);
-  const unsigned lm_blocks = placed_grid(lm_c, (S1 + rows - 1) / rows, B, lm_shift);
-  auto kernel = rows96 ? simple_bwd_am_lm_kernel<96, 16> : simple_bwd_am_lm_kernel<128, 16>;
-  (void)allow_lds(reinterpret_cast<const void *>(kernel), lds);
-  hipLaunchKernelGGL(kernel, dim3(am_blocks + lm_blocks), dim3(256), lds, stream, lm, am, symbols,
-                     boundary, lm_max, am_max, dmat, gpx, row_x, row_y, col_y, lm_grad, am_grad,
-                     window, B, S, T, C, ldd, term, rnnt_type, rows_cap, (int)lm_blocks, lm_shift,
-                     am_shift);
+template <int kMl, int kMa>
+void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
+                  const int64_t *boundary, const float *lm_max, const float *am_max,
+                  const float *dmat, const float *gpx, const float *gpy, const float *row_x,
+                  const float *row_y, void *lm_grad, void *am_grad, const int64_t *window, int B,
+                  int S, int T, int C, int ldd, int term, int rnnt_type, int out_type,
+                  hipStream_t stream) {
+  constexpr size_t lds = ProdShape<(kMl > kMa ? kMl : kMa), kProdC>::kLdsBytes;
+  const int c_tiles = (C + kProdC - 1) / kProdC, shift = part_shift_for(B, c_tiles);
+  const unsigned am_blocks =
+      am_grad && T > 0 ? placed_grid(c_tiles, (T + kMa - 1) / kMa, B, shift) : 0;
+  const unsigned lm_blocks = lm_grad ? placed_grid(c_tiles, (S + kMl) / kMl, B, shift) : 0;
+  if (am_blocks + lm_blocks == 0) return;
+  hipLaunchKernelGGL((simple_bwd_am_lm_kernel<kMl, kMa>), dim3(am_blocks + lm_blocks),
+                     dim3(kProdThreads), lds, stream, lm, am, symbols, boundary, lm_max, am_max,
+                     dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad, window, B, S, T, C, ldd,
+                     term, rnnt_type, (int)lm_blocks, shift, out_type);
 }
-void launch_bwd_both(const double *, const double *, const int64_t *, const int64_t *,
-                     const double *, const double *, const double *, const double *,
-                     const double *, const double *, const double *, double *, double *,
-                     const int64_t *, int, int, int, int, int, int, int, hipStream_t) {}
-void launch_bwd_lm(const float *lm, const float *am, const int64_t *symbols, const float *lm_max,
-                   const float *am_max, const float *dmat, const float *row_x, const float *row_y,
-                   float *lm_grad, const int64_t *window, int B, int S, int T, int C, int ldd,
-                   int term, hipStream_t stream) {
-  // the row count per workgroup that leaves fewer padding rows; 128 on a tie
-  const int S1 = S + 1;
-  const bool rows96 = (S1 + 95) / 96 * 96 < (S1 + 127) / 128 * 128;
-  const int rows = rows96 ? 96 : 128;
-  const int c_tiles = (C + kLmC - 1) / kLmC, shift = part_shift_for(B, c_tiles);
-  auto kernel = rows96 ? simple_bwd_lm_slab_kernel<96, 32> : simple_bwd_lm_slab_kernel<128, 16>;
-  const size_t lds = rows96 ? LmShape<96, 32>::kLdsBytes : LmShape<128, 16>::kLdsBytes;
-  (void)allow_lds(reinterpret_cast<const void *>(kernel), lds);
-  hipLaunchKernelGGL(kernel, dim3(placed_grid(c_tiles, (S1 + rows - 1) / rows, B, shift)),
-                     dim3(kLmThreads), lds, stream, lm, am, symbols, lm_max, am_max, dmat, row_x,
-                     row_y, lm_grad, window, B, S, T, C, ldd, term, shift);
+// Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand along
+// the vocabulary half as
+// often as 64 (am.grad at B 16, T 400, C 5000: 92 against 97 us; lm.grad 60 against 65), which is
+// what counts once the chip is full; they lose where the padding of the last tile outweighs
+// that (up to 64 rows: 24 against 18 us at B 21, S 47, T 333, C 503) or where fewer of them than fill
+// the chip remain (B 3, S 250, T 1335, C 198: 71 against 55 us).
+bool wide_tile(long columns_of_tiles, int rows) {
+  const long wide = (rows + 127) / 128, narrow = (rows + 63) / 64;
+  return narrow > 1 && 14 * wide <= 8 * narrow && columns_of_tiles * wide >= kMinWideTiles;
 }
-void launch_bwd_lm(const double *lm, const double *am, const int64_t *symbols,
-                   const double *lm_max, const double *am_max, const double *dmat,
-                   const double *row_x, const double *row_y, double *lm_grad, const int64_t *, int B,
-                   int S, int T, int C, int ldd, int term, hipStream_t stream) {
-  const dim3 grid((C + kTileN - 1) / kTileN, (S + 1 + kTileM - 1) / kTileM, B);
-  hipLaunchKernelGGL(simple_bwd_lm_kernel<double>, grid, dim3(kGemmThreads), 0, stream, lm, am,
-                     symbols, lm_max, am_max, dmat, row_x, row_y, lm_grad, S, T, C, ldd, term);
+void launch_bwd(const float *lm, const float *am, const int64_t *symbols, const int64_t *boundary,
+                const float *lm_max, const float *am_max, const float *dmat, const float *gpx,
+                const float *gpy, const float *row_x, const float *row_y, const float *, void *lm_grad,
+                void *am_grad, const int64_t *window, int B, int S, int T, int C, int ldd, int term,
+                int rnnt_type, int out_type, hipStream_t stream) {
+  const long columns = (long)B * ((C + kProdC - 1) / kProdC);
+  const bool wide_l = wide_tile(columns, S + 1), wide_a = wide_tile(columns, T);
+  auto launch = wide_l ? wide_a ? launch_bwd_t<128, 128> : launch_bwd_t<128, 64>
+                       : wide_a ? launch_bwd_t<64, 128> : launch_bwd_t<64, 64>;
+  launch(lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad,
+         window, B, S, T, C, ldd, term, rnnt_type, out_type, stream);
 }
-void launch_bwd_am(const float *lm, const float *am, const int64_t *symbols,
-                   const int64_t *boundary, const float *lm_max, const float *am_max,
-                   const float *dmat, const float *gpx, const float *row_x, const float *col_y,
-                   float *am_grad, const int64_t *window, int B, int S, int T, int C, int ldd,
-                   int term, int rnnt_type, hipStream_t stream) {
-  const int c_tiles = (C + kAmC - 1) / kAmC, shift = part_shift_for(B, c_tiles);
-  // rows of k held in LDS per pass: all of them when they fit
-  // Rows of k held in LDS per pass: at most 64, in passes of equal size.  The workgroup's
-  // phases (panels in, exp, products, results out) do not overlap inside it, so the compute
-  // unit needs several of them; 64 rows of panels leave room for four (128 rows: two), and the
-  // next pass's panels are requested before the current one is multiplied (B = 16, S + 1 = 121,
-  // T = 400, C = 5000: 154 us with one pass of 122 rows, 138 with two of 64 as three workgroups
-  // per compute unit).
-  const int rows_cap = am_rows_per_pass(S);
-  const size_t lds = am_panel_lds_bytes(rows_cap);
-  // (the 16-byte accesses need no alignment)
-  auto kernel = simple_bwd_am_panel_kernel<kAmCap, 4>;
-  (void)allow_lds(reinterpret_cast<const void *>(kernel), lds);
-  hipLaunchKernelGGL(kernel, dim3(placed_grid(c_tiles, (T + kAmT - 1) / kAmT, B, shift)), dim3(256),
-                     lds, stream, lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, row_x, col_y,
-                     am_grad, window, B, S, T, C, ldd, term, rnnt_type, rows_cap, shift);
-}
-void launch_bwd_am(const double *lm, const double *am, const int64_t *symbols,
-                   const int64_t *boundary, const double *lm_max, const double *am_max,
-                   const double *dmat, const double *gpx, const double *, const double *col_y,
-                   double *am_grad, const int64_t *, int B, int S, int T, int C, int ldd, int term,
-                   int rnnt_type, hipStream_t stream) {
-  const dim3 grid((C + kTileN - 1) / kTileN, (T + kTileM - 1) / kTileM, B);
-  hipLaunchKernelGGL(simple_bwd_am_kernel<double>, grid, dim3(kGemmThreads), 0, stream, lm, am,
-                     lm_max, am_max, dmat, col_y, am_grad, S, T, C, ldd, term);
+void launch_bwd(const double *lm, const double *am, const int64_t *symbols,
+                const int64_t *boundary, const double *lm_max, const double *am_max,
+                const double *dmat, const double *gpx, const double *, const double *row_x,
+                const double *row_y, const double *col_y, void *lm_grad_, void *am_grad_,
+                const int64_t *, int B, int S, int T, int C, int ldd, int term, int rnnt_type, int,
+                hipStream_t stream) {
+  double *lm_grad = static_cast<double *>(lm_grad_), *am_grad = static_cast<double *>(am_grad_);
+  const unsigned c_tiles = (C + kTileN - 1) / kTileN;
+  if (lm_grad)
+    hipLaunchKernelGGL(simple_bwd_lm_kernel<double>, dim3(c_tiles, (S + 1 + kTileM - 1) / kTileM, B),
+                       dim3(kGemmThreads), 0, stream, lm, am, symbols, lm_max, am_max, dmat, row_x,
+                       row_y, lm_grad, S, T, C, ldd, term);
+  if (!am_grad || T <= 0) return;
+  hipLaunchKernelGGL(simple_bwd_am_kernel<double>, dim3(c_tiles, (T + kTileM - 1) / kTileM, B),
+                     dim3(kGemmThreads), 0, stream, lm, am, lm_max, am_max, dmat, col_y, am_grad, S,
+                     T, C, ldd, term);
   if (S > 0) {  // the double path keeps the separate per-symbol scatter
     const long n = (long)B * T;
     hipLaunchKernelGGL(simple_bwd_symbols_kernel<double>, dim3((unsigned)((n + 255) / 256)),
@@ -1085,9 +1072,20 @@ void launch_bwd_am(const double *lm, const double *am, const int64_t *symbols,
 }
 
 template <typename R>
+void launch_scale(R *px_grad, R *py_grad, const R *score_grad, int score_grad_stride,
+                  double score_grad_scale, int B, int S, int T, int modified, hipStream_t stream) {
+  const int per_x = S * (modified ? T : T + 1), per_y = (S + 1) * T;
+  const int x_blocks = (per_x + 1023) / 1024, y_blocks = (per_y + 1023) / 1024;
+  if (x_blocks + y_blocks > 0)
+    hipLaunchKernelGGL(scale_by_batch_kernel<R>, dim3(x_blocks + y_blocks, B), dim3(256), 0, stream,
+                       px_grad, py_grad, score_grad, score_grad_stride, (R)score_grad_scale, per_x,
+                       per_y, x_blocks);
+}
+
+template <typename R>
 int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary, R *px,
-             R *py, R *lm_max, R *am_max, R *norm_raw, int B, int S, int T, int C, int term,
-             int rnnt_type, int window_only, void *stream_) {
+             R *py, R *lm_max, R *am_max, R *norm_raw, R *workspace, double delay_penalty, int B,
+             int S, int T, int C, int term, int rnnt_type, int window_only, void *stream_) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_fwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2)
     return fail(FRNNT_EINVAL, "simple_logprobs_fwd: rnnt_type must be 0, 1 or 2");
@@ -1107,16 +1105,16 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   if (!std::is_same<R, float>::value)
     hipLaunchKernelGGL(row_max_kernel<R>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream,
                        lm, am, lm_max, am_max, n_lm, n_am, C);
-  {
-    // (the grid always has at least one column of tiles, so that the -inf column of
-    // an empty-frame regular lattice is still written)
-    launch_fwd_gemm(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw,
-                    window_only ? boundary : nullptr, B, S, T, C, term, rnnt_type, stream);
-    if (rnnt_type == kConstrained && S > 0 && T > 0) {
-      const long total = (long)B * S * T;
-      hipLaunchKernelGGL(add_next_row_kernel<R>, dim3((unsigned)((total + 255) / 256)), dim3(256),
-                         0, stream, px, py, total, S, T);
-    }
+  // (the grid always has at least one column of tiles, so that the -inf column of
+  // an empty-frame regular lattice is still written)
+  const bool constrained = rnnt_type == kConstrained;
+  launch_fwd_gemm(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw,
+                  window_only ? boundary : nullptr, workspace, constrained ? 0.0 : delay_penalty, B,
+                  S, T, C, term, rnnt_type, stream);
+  if (constrained && S > 0 && T > 0) {
+    const long total = (long)B * S * T;
+    hipLaunchKernelGGL(add_next_row_kernel<R>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       stream, px, py, boundary, Delay<R>{(R)delay_penalty}, total, S, T);
   }
   return check_launch("simple_logprobs_fwd");
 }
@@ -1125,14 +1123,15 @@ template <typename R>
 int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary,
              const R *lm_max, const R *am_max, const R *norm_raw, const R *score_grad,
              int score_grad_stride, double score_grad_scale, R *px_grad, R *py_grad, R *dmat,
-             R *row_x, R *row_y, R *col_y, R *lm_grad, R *am_grad, int B, int S, int T, int C,
-             int term, int rnnt_type, int window_only, void *stream_) {
+             R *row_x, R *row_y, R *col_y, void *lm_grad, void *am_grad, int B, int S, int T, int C,
+             int term, int rnnt_type, int window_only, int out_type, void *stream_) {
+  constexpr bool is_float = std::is_same<R, float>::value;
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_bwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2 || term < 0 || term >= C)
     return fail(FRNNT_EINVAL, "simple_logprobs_bwd: bad rnnt_type or termination symbol");
   if (B == 0) return FRNNT_OK;
   if (!lm || !am || (!symbols && S > 0) || !lm_max || !am_max || !norm_raw || !px_grad ||
-      !py_grad || !dmat || !row_x || !row_y || !col_y)
+      !py_grad || !dmat || !row_x || !row_y || (!is_float && !col_y))
     return fail(FRNNT_EINVAL, "simple_logprobs_bwd: null pointer");
   // (the float32 kernels address an utterance's lm / am / D rows by 32-bit byte offsets)
   if (std::is_same<R, float>::value &&
@@ -1140,38 +1139,27 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
        (long)(S + 1) * (T + 3) * 4 >= (1L << 31)))
     return fail(FRNNT_ELIMIT, "simple_logprobs_bwd: one utterance's lm, am or lattice exceeds 2 GiB");
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  if (score_grad) {
-    if (score_grad_stride != 0 && score_grad_stride != 1)
-      return fail(FRNNT_EINVAL, "simple_logprobs_bwd: score_grad_stride must be 0 or 1");
-    const int T1 = rnnt_type == kRegular ? T + 1 : T;
-    const int per_x = S * T1, per_y = (S + 1) * T;
-    const int x_blocks = (per_x + 1023) / 1024, y_blocks = (per_y + 1023) / 1024;
-    if (x_blocks + y_blocks > 0)
-      hipLaunchKernelGGL(scale_by_batch_kernel<R>, dim3(x_blocks + y_blocks, B), dim3(256), 0,
-                         stream, px_grad, py_grad, score_grad, score_grad_stride,
-                         (R)score_grad_scale, per_x, per_y, x_blocks);
+  if (score_grad && score_grad_stride != 0 && score_grad_stride != 1)
+    return fail(FRNNT_EINVAL, "simple_logprobs_bwd: score_grad_stride must be 0 or 1");
+  // The occupation gradients are scaled as they are read, except where other workgroups than
+  // the one that scales a row read it: the row above's in the constrained lattice, the
+  // columns in double.  (B 64, S 120, T 600: 20 us instead of 30 in two launches.)
+  const bool fused = is_float && rnnt_type != kConstrained;
+  if (score_grad && !fused) {
+    launch_scale(px_grad, py_grad, score_grad, score_grad_stride, score_grad_scale, B, S, T,
+                 rnnt_type != kRegular, stream);
+    score_grad = nullptr;
   }
   const int ldd = (T + 3) & ~3;  // leading dimension of dmat: 16-byte rows
   // (the double kernels ignore the window: they take the whole lattice as it is)
-  const int64_t *window = (window_only && std::is_same<R, float>::value) ? boundary : nullptr;
-  const long prep_blocks = ((long)B * (S + 1) + 3) / 4 + (long)B * ((T + kWave - 1) / kWave) + 1;
+  const int64_t *window = (window_only && is_float) ? boundary : nullptr;
+  const long prep_blocks = ((long)B * (S + 1) + 3) / 4 + 1 +
+                           (is_float ? 0 : (long)B * ((T + kWave - 1) / kWave));
   hipLaunchKernelGGL(simple_bwd_prep_kernel<R>, dim3((unsigned)prep_blocks), dim3(256), 0, stream,
-                     px_grad, py_grad, norm_raw, boundary, window, dmat, row_x, row_y, col_y, B, S, T,
-                     ldd, rnnt_type);
-  // (one launch for both products while they are short: at B (S+1) T C = 3.2e8 it saves
-  // about 1 us of 37; at 3.9e9 the common LDS and register budget costs 8 %)
-  if (std::is_same<R, float>::value && lm_grad && am_grad && T > 0 &&
-      (double)B * (S + 1) * T * C < 1e9) {
-    launch_bwd_both(lm, am, symbols, boundary, lm_max, am_max, dmat, px_grad, row_x, row_y, col_y,
-                    lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, stream);
-    return check_launch("simple_logprobs_bwd");
-  }
-  if (lm_grad)
-    launch_bwd_lm(lm, am, symbols, lm_max, am_max, dmat, row_x, row_y, lm_grad, window, B, S, T, C,
-                  ldd, term, stream);
-  if (am_grad && T > 0)
-    launch_bwd_am(lm, am, symbols, boundary, lm_max, am_max, dmat, px_grad, row_x, col_y, am_grad, window,
-                  B, S, T, C, ldd, term, rnnt_type, stream);
+                     px_grad, py_grad, norm_raw, boundary, window, score_grad, score_grad_stride,
+                     (R)score_grad_scale, dmat, row_x, row_y, col_y, B, S, T, ldd, rnnt_type);
+  launch_bwd(lm, am, symbols, boundary, lm_max, am_max, dmat, px_grad, py_grad, row_x, row_y, col_y,
+             lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type, stream);
   return check_launch("simple_logprobs_bwd");
 }
 
@@ -1186,13 +1174,8 @@ int scale_grads_impl(R *px_grad, R *py_grad, const R *score_grad, int score_grad
   if (B == 0) return FRNNT_OK;
   if (!px_grad || !py_grad || !score_grad)
     return fail(FRNNT_EINVAL, "mi_scale_grads: null pointer");
-  const int T1 = modified ? T : T + 1;
-  const int per_x = S * T1, per_y = (S + 1) * T;
-  const int x_blocks = (per_x + 1023) / 1024, y_blocks = (per_y + 1023) / 1024;
-  if (x_blocks + y_blocks > 0)
-    hipLaunchKernelGGL(scale_by_batch_kernel<R>, dim3(x_blocks + y_blocks, B), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), px_grad, py_grad, score_grad,
-                       score_grad_stride, (R)score_grad_scale, per_x, per_y, x_blocks);
+  launch_scale(px_grad, py_grad, score_grad, score_grad_stride, score_grad_scale, B, S, T, modified,
+               static_cast<hipStream_t>(stream));
   return check_launch("mi_scale_grads");
 }
 
@@ -1205,6 +1188,32 @@ int reduce_impl(const R *scores, R *loss, int B, int reduction, void *stream) {
   hipLaunchKernelGGL(loss_reduce_kernel<R>, dim3(1), dim3(kWave), 0,
                      static_cast<hipStream_t>(stream), scores, loss, B, reduction);
   return check_launch("loss_reduce");
+}
+
+// 2-byte inputs as float32: eight elements per thread, in 16-byte accesses where the input is
+// aligned to them (the output always is).
+template <typename IO>
+__global__ void __launch_bounds__(256)
+    widen_kernel(const uint16_t *__restrict__ lm, const uint16_t *__restrict__ am,
+                 float *__restrict__ lm_wide, float *__restrict__ am_wide, long n_lm, long n_am,
+                 unsigned lm_blocks) {
+  const bool is_lm = blockIdx.x < lm_blocks;
+  const uint16_t *from = is_lm ? lm : am;
+  float *to = is_lm ? lm_wide : am_wide;
+  const long n = is_lm ? n_lm : n_am;
+  const long first = (long)(is_lm ? blockIdx.x : blockIdx.x - lm_blocks) * 2048;
+  const long at = first + 8 * threadIdx.x;
+  if ((reinterpret_cast<uintptr_t>(from) & 15) == 0 && at + 8 <= n) {
+    const uintx4 raw = *reinterpret_cast<const uintx4 *>(from + at);
+    dgemm::floatx4 v[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = IO::load((uint16_t)(raw[i / 2] >> (16 * (i % 2))));
+    *reinterpret_cast<dgemm::floatx4 *>(to + at) = v[0];
+    *reinterpret_cast<dgemm::floatx4 *>(to + at + 4) = v[1];
+  } else {
+    for (int i = 0; i < 8; ++i)
+      if (at + i < n) to[at + i] = IO::load(from[at + i]);
+  }
 }
 
 // ---- scratch that the library owns: for callers that cannot allocate --------------------
@@ -1233,9 +1242,58 @@ float *own_scratch_address() {
 }
 
 }  // namespace
+
+int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
+                        const int64_t *boundary, float *px, float *py, float *lm_max,
+                        float *am_max, float *norm_raw, float *workspace, double delay_penalty,
+                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        void *stream) {
+  return fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, workspace,
+                         delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
+}
+int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
+                        const int64_t *boundary, double *px, double *py, double *lm_max,
+                        double *am_max, double *norm_raw, double *workspace, double delay_penalty,
+                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        void *stream) {
+  return fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, workspace,
+                          delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
+}
+void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
+                  long n_lm, long n_am, hipStream_t stream) {
+  const unsigned lm_blocks = (unsigned)((n_lm + 2047) / 2048), am_blocks = (unsigned)((n_am + 2047) / 2048);
+  if (lm_blocks + am_blocks == 0) return;
+  hipLaunchKernelGGL((dtype == FRNNT_F16 ? widen_kernel<HalfIO> : widen_kernel<Bf16IO>),
+                     dim3(lm_blocks + am_blocks), dim3(256), 0, stream,
+                     static_cast<const uint16_t *>(lm), static_cast<const uint16_t *>(am), lm_wide,
+                     am_wide, n_lm, n_am, lm_blocks);
+}
+
 }  // namespace frnnt
 
 extern "C" {
+
+int frnnt_additive_loss_bwd(int dtype, const void *lm, const void *am, const int64_t *symbols,
+                            const int64_t *boundary, const void *lm_max, const void *am_max,
+                            const void *norm_raw, const void *score_grad, int score_grad_stride,
+                            double score_grad_scale, void *px_grad, void *py_grad, void *dmat,
+                            void *row_x, void *row_y, void *col_y, void *lm_grad, void *am_grad,
+                            int B, int S, int T, int C, int termination_symbol, int rnnt_type,
+                            void *stream) {
+  if (dtype < FRNNT_F32 || dtype > FRNNT_BF16)
+    return frnnt::fail(FRNNT_EINVAL, "additive_loss_bwd: unknown dtype");
+  auto call = [&](auto r) {
+    using R = decltype(r);
+    auto in = [](const void *p) { return static_cast<const R *>(p); };
+    auto out = [](void *p) { return static_cast<R *>(p); };
+    return frnnt::bwd_impl<R>(in(lm), in(am), symbols, boundary, in(lm_max), in(am_max),
+                              in(norm_raw), in(score_grad), score_grad_stride, score_grad_scale,
+                              out(px_grad), out(py_grad), out(dmat), out(row_x), out(row_y),
+                              out(col_y), lm_grad, am_grad, B, S, T, C, termination_symbol,
+                              rnnt_type, boundary != nullptr, dtype, stream);
+  };
+  return dtype == FRNNT_F64 ? call(double()) : call(float());
+}
 
 int frnnt_simple_logprobs_bwd_noalloc_f32(const float *lm, const float *am, const int64_t *symbols,
                                           const int64_t *boundary, const float *lm_max,
@@ -1279,7 +1337,7 @@ int frnnt_simple_logprobs_bwd_noalloc_f32(const float *lm, const float *am, cons
   return frnnt::bwd_impl<float>(lm, am, symbols, boundary, lm_max, am_max, norm_raw, score_grad,
                                 score_grad_stride, score_grad_scale, px_grad, py_grad, dmat, row_x,
                                 row_y, col_y, lm_grad, am_grad, B, S, T, C, termination_symbol,
-                                rnnt_type, window_only, stream);
+                                rnnt_type, window_only, FRNNT_F32, stream);
 }
 
 int frnnt_simple_logprobs_fwd_f32(const float *lm, const float *am, const int64_t *symbols,
@@ -1287,16 +1345,18 @@ int frnnt_simple_logprobs_fwd_f32(const float *lm, const float *am, const int64_
                                   float *am_max, float *norm_raw, int B, int S, int T, int C,
                                   int termination_symbol, int rnnt_type, int window_only,
                                   void *stream) {
-  return frnnt::fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, B, S,
-                                T, C, termination_symbol, rnnt_type, window_only, stream);
+  return frnnt::fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
+                                nullptr, 0.0, B, S, T, C, termination_symbol, rnnt_type,
+                                window_only, stream);
 }
 int frnnt_simple_logprobs_fwd_f64(const double *lm, const double *am, const int64_t *symbols,
                                   const int64_t *boundary, double *px, double *py, double *lm_max,
                                   double *am_max, double *norm_raw, int B, int S, int T, int C,
                                   int termination_symbol, int rnnt_type, int window_only,
                                   void *stream) {
-  return frnnt::fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, B, S,
-                                 T, C, termination_symbol, rnnt_type, window_only, stream);
+  return frnnt::fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
+                                 nullptr, 0.0, B, S, T, C, termination_symbol, rnnt_type,
+                                 window_only, stream);
 }
 int frnnt_simple_logprobs_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
                                   const int64_t *boundary, const float *lm_max,
@@ -1310,7 +1370,7 @@ int frnnt_simple_logprobs_bwd_f32(const float *lm, const float *am, const int64_
   return frnnt::bwd_impl<float>(lm, am, symbols, boundary, lm_max, am_max, norm_raw, score_grad,
                                 score_grad_stride, score_grad_scale, px_grad, py_grad, dmat, row_x,
                                 row_y, col_y, lm_grad, am_grad, B, S, T, C, termination_symbol,
-                                rnnt_type, window_only, stream);
+                                rnnt_type, window_only, FRNNT_F32, stream);
 }
 int frnnt_simple_logprobs_bwd_f64(const double *lm, const double *am, const int64_t *symbols,
                                   const int64_t *boundary, const double *lm_max,
@@ -1324,7 +1384,7 @@ int frnnt_simple_logprobs_bwd_f64(const double *lm, const double *am, const int6
   return frnnt::bwd_impl<double>(lm, am, symbols, boundary, lm_max, am_max, norm_raw, score_grad,
                                  score_grad_stride, score_grad_scale, px_grad, py_grad, dmat,
                                  row_x, row_y, col_y, lm_grad, am_grad, B, S, T, C,
-                                 termination_symbol, rnnt_type, window_only, stream);
+                                 termination_symbol, rnnt_type, window_only, FRNNT_F32, stream);
 }
 
 int frnnt_mi_scale_grads_f32(float *px_grad, float *py_grad, const float *score_grad,

@@ -67,38 +67,6 @@ inline int abi_mi_backward(const double *px, const double *py, const int64_t *bn
   inline int abi_##NAME PARAMS_F { return frnnt_##NAME##_f32 ARGS; }     \
   inline int abi_##NAME PARAMS_D { return frnnt_##NAME##_f64 ARGS; }
 
-FRNNT_BOTH(simple_logprobs_fwd,
-           (const float *lm, const float *am, const int64_t *sym, const int64_t *bnd, float *px,
-            float *py, float *lmx, float *amx, float *nr, int B, int S, int T, int C, int term,
-            int kind, int window, void *st),
-           (const double *lm, const double *am, const int64_t *sym, const int64_t *bnd, double *px,
-            double *py, double *lmx, double *amx, double *nr, int B, int S, int T, int C, int term,
-            int kind, int window, void *st),
-           (lm, am, sym, bnd, px, py, lmx, amx, nr, B, S, T, C, term, kind, window, st))
-FRNNT_BOTH(simple_loss_fwd,
-           (const float *lm, const float *am, const int64_t *sym, const int64_t *bnd, float *px,
-            float *py, float *lmx, float *amx, float *nr, float *p, float *sc, float *gx,
-            float *gy, float *loss, int B, int S, int T, int C, int term, int kind, int red,
-            int checks, int32_t *status, void *st),
-           (const double *lm, const double *am, const int64_t *sym, const int64_t *bnd, double *px,
-            double *py, double *lmx, double *amx, double *nr, double *p, double *sc, double *gx,
-            double *gy, double *loss, int B, int S, int T, int C, int term, int kind, int red,
-            int checks, int32_t *status, void *st),
-           (lm, am, sym, bnd, px, py, lmx, amx, nr, p, sc, gx, gy, loss, B, S, T, C, term, kind,
-            red, checks, status, st))
-FRNNT_BOTH(simple_logprobs_bwd,
-           (const float *lm, const float *am, const int64_t *sym, const int64_t *bnd,
-            const float *lmx, const float *amx, const float *nr, const float *g, int gstride,
-            double gscale, float *gx, float *gy, float *dmat, float *rx, float *ry, float *cy,
-            float *lmg, float *amg, int B, int S, int T, int C, int term, int kind, int window,
-            void *st),
-           (const double *lm, const double *am, const int64_t *sym, const int64_t *bnd,
-            const double *lmx, const double *amx, const double *nr, const double *g, int gstride,
-            double gscale, double *gx, double *gy, double *dmat, double *rx, double *ry,
-            double *cy, double *lmg, double *amg, int B, int S, int T, int C, int term, int kind,
-            int window, void *st),
-           (lm, am, sym, bnd, lmx, amx, nr, g, gstride, gscale, gx, gy, dmat, rx, ry, cy, lmg, amg,
-            B, S, T, C, term, kind, window, st))
 FRNNT_BOTH(mi_loss_fwd,
            (const float *px, const float *py, const int64_t *bnd, float *p, float *sc, float *gx,
             float *gy, float *loss, int B, int S, int T, int modified, int red, int checks,
@@ -113,9 +81,6 @@ FRNNT_BOTH(mi_scale_grads,
            (double *gx, double *gy, const double *g, int gstride, double gscale, int B, int S,
             int T, int modified, void *st),
            (gx, gy, g, gstride, gscale, B, S, T, modified, st))
-FRNNT_BOTH(loss_reduce,
-           (const float *sc, float *loss, int B, int red, void *st),
-           (const double *sc, double *loss, int B, int red, void *st), (sc, loss, B, red, st))
 #undef FRNNT_BOTH
 
 void check_rc(int rc, const char *what) {
@@ -443,113 +408,72 @@ LossResult recursion_loss(const Tensor &px, const Tensor &py,
 }
 
 // ---- rnnt_loss_simple behind one autograd node -------------------------------------------
-// forward = frnnt_simple_loss_fwd: px / py (row maxima + MFMA contraction,
-// rnnt_loss.py:66-227), the recursion, its backward with a gradient of ones
+// forward = frnnt_additive_loss_fwd: px / py (row maxima + MFMA contraction, rnnt_loss.py:66-227,
+// the delay penalty :309-324), the recursion, its backward with a gradient of ones
 // (mutual_information.py:159-168), the reduction (rnnt_loss.py:326-340);
-// backward = frnnt_simple_logprobs_bwd: scales the occupation gradients in place by the
+// backward = frnnt_additive_loss_bwd: scales the occupation gradients in place by the
 // gradient of the scores (mutual_information.py:173-181) and pushes them through the two
-// gradient products to lm.grad and am.grad.
-void apply_delay_penalty(Tensor px, const Tensor &boundary, bool regular, double delay_penalty) {
-  // px += ((T_b - 1) / 2 - t) * delay_penalty, in the reference's operation order
-  // (rnnt_loss.py:309-324)
-  const int64_t B = px.size(0), T0 = px.size(2);
-  const int64_t T = regular ? T0 - 1 : T0;
-  Tensor offset;
-  if (boundary.defined())
-    offset = at::true_divide(boundary.select(1, 3) - 1, 2);
-  else
-    offset = at::scalar_tensor((double)(T - 1) / 2, px.options()).expand({B, 1, 1});
-  Tensor penalty = offset.reshape({B, 1, 1}) -
-                   at::arange(T0, px.options().dtype(at::kLong)).reshape({1, 1, T0});
-  penalty = penalty * delay_penalty;
-  px += penalty.to(px.scalar_type());
+// gradient products to lm.grad and am.grad.  float16 / bfloat16 inputs are widened by the first
+// kernel and their gradients written in their type; everything between is float32.
+int dtype_code(at::ScalarType t) {
+  return t == at::kFloat ? FRNNT_F32 : t == at::kDouble ? FRNNT_F64 : t == at::kHalf ? FRNNT_F16 : FRNNT_BF16;
 }
 
 struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
-  static variable_list forward(AutogradContext *ctx, const Tensor &lm, const Tensor &am,
+  static variable_list forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &am_,
                                const Tensor &symbols, const std::optional<Tensor> &boundary_,
                                int64_t term, int64_t kind, double delay_penalty, bool want_grads,
                                int64_t reduction, int64_t checks, bool need_lm, bool need_am) {
     const Tensor boundary = or_undefined(boundary_);
-    return am.scalar_type() == at::kFloat
-               ? run<float>(ctx, lm, am, symbols, boundary, term, kind, delay_penalty, want_grads,
-                            reduction, checks, need_lm, need_am)
-               : run<double>(ctx, lm, am, symbols, boundary, term, kind, delay_penalty,
-                             want_grads, reduction, checks, need_lm, need_am);
-  }
-
-  template <typename R>
-  static variable_list run(AutogradContext *ctx, const Tensor &lm_, const Tensor &am_,
-                           const Tensor &symbols, const Tensor &boundary, int64_t term,
-                           int64_t kind, double delay_penalty, bool want_grads, int64_t reduction,
-                           int64_t checks, bool need_lm, bool need_am) {
     const Tensor lm = lm_.contiguous(), am = am_.contiguous(), sym = symbols.contiguous();
     const Tensor bnd = boundary.defined() ? boundary.contiguous() : Tensor();
     const int64_t B = am.size(0), T = am.size(1), C = am.size(2), S = lm.size(1) - 1;
     const int64_t T1 = kind == 0 ? T + 1 : T;
     const bool need_grad = need_lm || need_am;
+    const int dtype = dtype_code(am.scalar_type());
+    const bool narrow = dtype >= FRNNT_F16;
     ctx->set_materialize_grads(false);
     DeviceGuard guard(am.device());
-    void *stream = stream_of(am);
-    const auto opts = am.options();
-    // internal buffers in one allocation: px | py | lm_max | am_max | norm_raw | p | scores
-    const int64_t n_px = B * S * T1, n_py = B * (S + 1) * T;
+    const auto opts = am.options().dtype(narrow ? at::kFloat : am.scalar_type());
+    const int64_t item = dtype == FRNNT_F64 ? 8 : 4;
+    // what the backward reads, in one allocation: lm_max | am_max | norm_raw | wide lm | wide am
+    const int64_t n_py = B * (S + 1) * T;
+    Carver keep;
+    const int64_t o_lmx = keep.take(B * (S + 1)), o_amx = keep.take(B * T),
+                  o_nr = keep.take(need_grad ? n_py : 0),
+                  o_lmw = keep.take(narrow ? B * (S + 1) * C : 0),
+                  o_amw = keep.take(narrow ? B * T * C : 0);
+    Tensor kept = at::empty({keep.total}, opts);
+    // what it does not: px | py | p | scores | workspace
+    const int64_t n_ws = frnnt_additive_loss_workspace(dtype, (int)B, (int)S, (int)T, (int)C);
     Carver carve;
-    const int64_t o_px = carve.take(n_px), o_py = carve.take(n_py),
-                  o_lmx = carve.take(B * (S + 1)), o_amx = carve.take(B * T),
-                  o_nr = carve.take(need_grad ? n_py : 0),
-                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B);
-    Tensor work = at::empty({carve.total}, opts);
-    R *w = work.data_ptr<R>();
+    const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(n_py),
+                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B),
+                  o_ws = carve.take(n_ws);
+    const Tensor work = at::empty({carve.total}, opts);
+    char *k = static_cast<char *>(kept.data_ptr()), *w = static_cast<char *>(work.data_ptr());
     Tensor gx, gy;
     if (want_grads || need_grad) {
       gx = at::empty({B, S, T1}, opts);
       gy = at::empty({B, S + 1, T}, opts);
     }
     Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
-    R *nr = need_grad ? w + o_nr : nullptr;
-    int32_t *status = status_for(am, bnd);
-    if (delay_penalty > 0.0) {
-      // the penalty is applied to px between the two stages (rnnt_loss.py:309-326)
-      check_rc(abi_simple_logprobs_fwd(ptr<R>(lm), ptr<R>(am), iptr(sym), iptr(bnd), w + o_px,
-                                       w + o_py, w + o_lmx, w + o_amx, nr, (int)B, (int)S, (int)T,
-                                       (int)C, (int)term, (int)kind, bnd.defined() ? 1 : 0,
-                                       stream),
-               "frnnt_simple_logprobs_fwd");
-      apply_delay_penalty(work.narrow(0, o_px, n_px).view({B, S, T1}), boundary, kind == 0,
-                          delay_penalty);
-      const int modified = kind != 0;
-      check_rc(abi_mi_forward(w + o_px, w + o_py, iptr(bnd), w + o_p, w + o_sc, (int)B, (int)S,
-                              (int)T, modified, (int)checks, status, stream),
-               "frnnt_mi_forward");
-      if (gx.defined())
-        check_rc(abi_mi_backward(w + o_px, w + o_py, iptr(bnd), w + o_p, (R *)nullptr, ptr<R>(gx),
-                                 ptr<R>(gy), (int)B, (int)S, (int)T, modified, 0, stream),
-                 "frnnt_mi_backward");
-      check_rc(abi_loss_reduce(w + o_sc, ptr<R>(loss), (int)B, (int)reduction, stream),
-               "frnnt_loss_reduce");
-    } else {
-      check_rc(abi_simple_loss_fwd(ptr<R>(lm), ptr<R>(am), iptr(sym), iptr(bnd), w + o_px,
-                                   w + o_py, w + o_lmx, w + o_amx, nr, w + o_p, w + o_sc,
-                                   ptr<R>(gx), ptr<R>(gy), ptr<R>(loss), (int)B, (int)S, (int)T,
-                                   (int)C, (int)term, (int)kind, (int)reduction, (int)checks,
-                                   status, stream),
-               "frnnt_simple_loss_fwd");
-    }
+    check_rc(frnnt_additive_loss_fwd(
+                 dtype, lm.data_ptr(), am.data_ptr(), iptr(sym), iptr(bnd),
+                 narrow ? k + o_lmw * item : nullptr, narrow ? k + o_amw * item : nullptr,
+                 w + o_px * item, w + o_py * item, k + o_lmx * item, k + o_amx * item,
+                 need_grad ? k + o_nr * item : nullptr, w + o_p * item, w + o_sc * item,
+                 gx.defined() ? gx.data_ptr() : nullptr, gy.defined() ? gy.data_ptr() : nullptr,
+                 loss.data_ptr(), n_ws ? w + o_ws * item : nullptr, (int)B, (int)S, (int)T, (int)C,
+                 (int)term, (int)kind, delay_penalty, (int)reduction, (int)checks,
+                 status_for(am, bnd), stream_of(am)),
+             "frnnt_additive_loss_fwd");
     if (need_grad) {
       // (an absent boundary is not saved: saved tensors must be defined)
-      if (bnd.defined())
-        ctx->save_for_backward({lm, am, sym, work, gx, gy, bnd});
-      else
-        ctx->save_for_backward({lm, am, sym, work, gx, gy});
-      ctx->saved_data["term"] = term;
-      ctx->saved_data["kind"] = kind;
-      ctx->saved_data["reduction"] = reduction;
-      ctx->saved_data["o_lmx"] = o_lmx;
-      ctx->saved_data["o_amx"] = o_amx;
-      ctx->saved_data["o_nr"] = o_nr;
-      ctx->saved_data["need_lm"] = need_lm;
-      ctx->saved_data["need_am"] = need_am;
+      variable_list save{lm, am, sym, kept, gx, gy};
+      if (bnd.defined()) save.push_back(bnd);
+      ctx->save_for_backward(std::move(save));
+      ctx->saved_data["meta"] = std::vector<int64_t>{term, kind, reduction, need_lm, need_am};
     }
     // (undefined tensors cannot be outputs of an autograd node)
     if (!gx.defined()) return {loss};
@@ -562,28 +486,22 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
     const Tensor &g_loss = grads[0];
     if (!g_loss.defined()) return out;
     const auto saved = ctx->get_saved_variables();
-    const Tensor &am = saved[1];
-    if (am.scalar_type() == at::kFloat)
-      run_backward<float>(ctx, saved, g_loss, out);
-    else
-      run_backward<double>(ctx, saved, g_loss, out);
-    return out;
-  }
-
-  template <typename R>
-  static void run_backward(AutogradContext *ctx, const variable_list &saved, const Tensor &g_loss,
-                           variable_list &out) {
-    const Tensor &lm = saved[0], &am = saved[1], &sym = saved[2], &work = saved[3];
+    const Tensor &lm = saved[0], &am = saved[1], &sym = saved[2], &kept = saved[3];
     Tensor gx = saved[4], gy = saved[5];
     const Tensor bnd = saved.size() > 6 ? saved[6] : Tensor();
-    const int64_t term = ctx->saved_data["term"].toInt(), kind = ctx->saved_data["kind"].toInt(),
-                  reduction = ctx->saved_data["reduction"].toInt(),
-                  o_lmx = ctx->saved_data["o_lmx"].toInt(),
-                  o_amx = ctx->saved_data["o_amx"].toInt(), o_nr = ctx->saved_data["o_nr"].toInt();
-    const bool need_lm = ctx->saved_data["need_lm"].toBool(),
-               need_am = ctx->saved_data["need_am"].toBool();
+    const std::vector<int64_t> meta = ctx->saved_data["meta"].toIntVector();
+    const int64_t reduction = meta[2];
     const int64_t B = am.size(0), T = am.size(1), C = am.size(2), S = lm.size(1) - 1;
+    const int dtype = dtype_code(am.scalar_type());
+    const bool narrow = dtype >= FRNNT_F16;
+    const int64_t item = dtype == FRNNT_F64 ? 8 : 4;
     DeviceGuard guard(am.device());
+    // (the forward's layout)
+    Carver keep;
+    const int64_t o_lmx = keep.take(B * (S + 1)), o_amx = keep.take(B * T),
+                  o_nr = keep.take(B * (S + 1) * T), o_lmw = keep.take(narrow ? B * (S + 1) * C : 0),
+                  o_amw = keep.take(narrow ? B * T * C : 0);
+    char *k = static_cast<char *>(kept.data_ptr());
     // d loss / d scores[b] = scale * g_loss[b * stride]
     const Tensor g = g_loss.contiguous();
     const int stride = reduction == kRedNone ? 1 : 0;
@@ -593,22 +511,21 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
     Carver carve;
     const int64_t o_d = carve.take(B * (S + 1) * ldd), o_rx = carve.take(B * (S + 1)),
                   o_ry = carve.take(B * (S + 1)), o_cy = carve.take(B * T);
-    Tensor scratch = at::empty({carve.total}, am.options());
-    R *s = scratch.data_ptr<R>();
-    R *w = work.data_ptr<R>();
-    Tensor lm_grad = need_lm ? at::empty(lm.sizes(), lm.options()) : Tensor();
-    Tensor am_grad = need_am ? at::empty(am.sizes(), am.options()) : Tensor();
+    const Tensor scratch = at::empty({carve.total}, kept.options());
+    char *s = static_cast<char *>(scratch.data_ptr());
+    if (meta[3]) out[0] = at::empty(lm.sizes(), lm.options());
+    if (meta[4]) out[1] = at::empty(am.sizes(), am.options());
     // gx / gy are scaled in place by the scores' gradient, exactly as the recursion's autograd
     // node does to the tensors it handed out
-    check_rc(abi_simple_logprobs_bwd(ptr<R>(lm), ptr<R>(am), iptr(sym), iptr(bnd), w + o_lmx,
-                                     w + o_amx, w + o_nr, ptr<R>(g), stride, scale, ptr<R>(gx),
-                                     ptr<R>(gy), s + o_d, s + o_rx, s + o_ry, s + o_cy,
-                                     ptr<R>(lm_grad), ptr<R>(am_grad), (int)B, (int)S, (int)T,
-                                     (int)C, (int)term, (int)kind, bnd.defined() ? 1 : 0,
-                                     stream_of(am)),
-             "frnnt_simple_logprobs_bwd");
-    out[0] = lm_grad;
-    out[1] = am_grad;
+    check_rc(frnnt_additive_loss_bwd(
+                 dtype, narrow ? k + o_lmw * item : lm.data_ptr(),
+                 narrow ? k + o_amw * item : am.data_ptr(), iptr(sym), iptr(bnd), k + o_lmx * item,
+                 k + o_amx * item, k + o_nr * item, g.data_ptr(), stride, scale, gx.data_ptr(),
+                 gy.data_ptr(), s + o_d * item, s + o_rx * item, s + o_ry * item, s + o_cy * item,
+                 meta[3] ? out[0].data_ptr() : nullptr, meta[4] ? out[1].data_ptr() : nullptr,
+                 (int)B, (int)S, (int)T, (int)C, (int)meta[0], (int)meta[1], stream_of(am)),
+             "frnnt_additive_loss_bwd");
+    return out;
   }
 };
 
@@ -617,7 +534,8 @@ LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols
                        int64_t rnnt_type, double delay_penalty, bool return_grad,
                        int64_t reduction, int64_t checks) {
   const Tensor boundary = or_undefined(boundary_);
-  require_float_gpu(am, "am");
+  if (am.scalar_type() != at::kHalf && am.scalar_type() != at::kBFloat16) require_float_gpu(am, "am");
+  TORCH_CHECK(am.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): am");
   TORCH_CHECK(lm.dim() == 3 && am.dim() == 3 && symbols.dim() == 2,
               "lm and am must be 3-dimensional, symbols 2-dimensional");
   const int64_t B = am.size(0), S = lm.size(1) - 1;

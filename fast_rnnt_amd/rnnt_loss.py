@@ -281,7 +281,7 @@ def rnnt_loss_simple(
         _assert_boundary(boundary, B, S, T, on_device=checks != 0)
     if reduction not in ("none", "mean", "sum"):
         raise ValueError(f"reduction should be ('none' | 'mean' | 'sum'), given {reduction}")
-    lm, am = _widen(lm, am)
+    _lib.suffix(am.dtype, narrow=True)
     # the whole device pipeline is one autograd node of the operator module: px / py (row
     # maxima + MFMA contraction), the recursion, its backward with a gradient of ones, the
     # reduction; its backward scales the occupation gradients in place and runs the two
