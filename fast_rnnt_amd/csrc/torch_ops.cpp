@@ -757,6 +757,161 @@ LossResult lattice_loss(const Tensor &logits, const Tensor &symbols,
                                         need_grad));
 }
 
+// ---- get_rnnt_prune_ranges and do_rnnt_pruning ---------------------------------------------
+// What get_rnnt_prune_ranges needs of the boundary rows (their copy on the host): the smallest
+// s_end, the smallest t_end - s_end, whether a t_end is 0, and the largest
+// trunc((s_end - 1) / t_end) + 2 (rnnt_loss.py:696-710).
+std::tuple<int64_t, int64_t, bool, int64_t> boundary_summary(const Tensor &rows) {
+  TORCH_CHECK(rows.device().is_cpu() && rows.scalar_type() == at::kLong && rows.dim() == 2 &&
+                  rows.size(1) == 4 && rows.is_contiguous() && rows.size(0) > 0,
+              "rows must be a contiguous int64 [B][4] tensor on the host");
+  const int64_t *r = rows.data_ptr<int64_t>();
+  int64_t least_s = r[2], least_slack = r[3] - r[2], most = INT64_MIN;
+  bool empty = false;
+  for (int64_t b = 0; b < rows.size(0); ++b, r += 4) {
+    least_s = std::min(least_s, r[2]);
+    least_slack = std::min(least_slack, r[3] - r[2]);
+    if (r[3] == 0) empty = true;
+    else most = std::max(most, (r[2] - 1) / r[3] + 2);
+  }
+  return {least_s, least_slack, empty, most};
+}
+
+Tensor prune_ranges(const Tensor &px_grad, const Tensor &py_grad, const Tensor &boundary,
+                    int64_t s_range) {
+  require_float_gpu(px_grad, "px_grad");
+  TORCH_CHECK(px_grad.dim() == 3 && py_grad.dim() == 3, "px_grad and py_grad must be 3-dimensional");
+  const int64_t B = px_grad.size(0), S = px_grad.size(1), T1 = px_grad.size(2), T = py_grad.size(2);
+  TORCH_CHECK((T1 == T || T1 == T + 1) && py_grad.size(0) == B && py_grad.size(1) == S + 1 &&
+                  py_grad.scalar_type() == px_grad.scalar_type() &&
+                  py_grad.device() == px_grad.device(),
+              "px_grad must be [B][S][T or T+1], py_grad [B][S+1][T] of the same type and device");
+  TORCH_CHECK(boundary.dim() == 2 && boundary.size(0) == B && boundary.size(1) == 4 &&
+                  boundary.scalar_type() == at::kLong && boundary.device() == px_grad.device(),
+              "boundary must be an int64 [B][4] tensor on the same device");
+  DeviceGuard guard(px_grad.device());
+  const Tensor gx = px_grad.contiguous(), gy = py_grad.contiguous(), bnd = boundary.contiguous();
+  Tensor ranges = at::empty({B, T, s_range}, bnd.options());
+  const int modified = T1 == T;
+  check_rc(gx.scalar_type() == at::kFloat
+               ? frnnt_prune_ranges_f32(ptr<float>(gx), ptr<float>(gy), iptr(bnd),
+                                        ranges.data_ptr<int64_t>(), (int)B, (int)S, (int)T,
+                                        modified, (int)s_range, stream_of(gx))
+               : frnnt_prune_ranges_f64(ptr<double>(gx), ptr<double>(gy), iptr(bnd),
+                                        ranges.data_ptr<int64_t>(), (int)B, (int)S, (int)T,
+                                        modified, (int)s_range, stream_of(gx)),
+           "frnnt_prune_ranges");
+  return ranges;
+}
+
+Tensor gather_rows(const Tensor &lm, const Tensor &rng) {
+  const int B = (int)rng.size(0), T = (int)rng.size(1), R = (int)rng.size(2),
+            S = (int)lm.size(1) - 1, C = (int)lm.size(2);
+  Tensor out = at::empty({B, T, R, C}, lm.options());
+  void *stream = stream_of(lm);
+  int rc;
+  switch (lm.scalar_type()) {
+    case at::kFloat:
+      rc = frnnt_prune_gather_f32(ptr<float>(lm), iptr(rng), ptr<float>(out), B, S, T, R, C, stream);
+      break;
+    case at::kDouble:
+      rc = frnnt_prune_gather_f64(ptr<double>(lm), iptr(rng), ptr<double>(out), B, S, T, R, C, stream);
+      break;
+    case at::kHalf:
+      rc = frnnt_prune_gather_f16(lm.data_ptr(), iptr(rng), out.data_ptr(), B, S, T, R, C, stream);
+      break;
+    default:
+      rc = frnnt_prune_gather_bf16(lm.data_ptr(), iptr(rng), out.data_ptr(), B, S, T, R, C, stream);
+  }
+  check_rc(rc, "frnnt_prune_gather");
+  return out;
+}
+
+// do_rnnt_pruning as one autograd node (rnnt_loss.py:780-818): am_pruned is a view of am, lm_pruned
+// a gathered copy; backward = frnnt_pruning_bwd, which reads a gradient that both share -- the
+// joiner that follows adds the two -- once.
+struct PruningFn : public torch::autograd::Function<PruningFn> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &am, const Tensor &lm_,
+                               const Tensor &ranges) {
+    DeviceGuard guard(lm_.device());
+    const Tensor lm = lm_.contiguous(), rng = ranges.contiguous();
+    const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2), C = lm.size(2);
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({rng});
+    ctx->saved_data["rows"] = lm.size(1);
+    return {am.unsqueeze(2).expand({B, T, R, C}), gather_rows(lm, rng)};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    variable_list out(3);
+    const Tensor rng = ctx->get_saved_variables()[0];
+    const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2),
+                  S1 = ctx->saved_data["rows"].toInt();
+    const Tensor &any = grads[0].defined() ? grads[0] : grads[1];
+    if (!any.defined()) return out;
+    const int64_t C = any.size(3);
+    DeviceGuard guard(any.device());
+    const Tensor ga = grads[0].defined() ? grads[0].contiguous() : Tensor();
+    // (one tensor stays one, also where a copy of it has to be made)
+    const Tensor gl = !grads[1].defined()                                ? Tensor()
+                      : ga.defined() && grads[1].is_same(grads[0]) ? ga
+                                                                         : grads[1].contiguous();
+    if (ga.defined()) out[0] = at::empty({B, T, C}, any.options());
+    if (gl.defined()) out[1] = at::empty({B, S1, C}, any.options());
+    auto at_ = [](const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
+    check_rc(frnnt_pruning_bwd(dtype_code(any.scalar_type()), at_(ga), at_(gl), iptr(rng),
+                               at_(out[0]), at_(out[1]), (int)B, (int)S1 - 1, (int)T, (int)R,
+                               (int)C, stream_of(any)),
+             "frnnt_pruning_bwd");
+    return out;
+  }
+};
+
+// lm alone
+struct GatherRowsFn : public torch::autograd::Function<GatherRowsFn> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &ranges) {
+    DeviceGuard guard(lm_.device());
+    const Tensor lm = lm_.contiguous(), rng = ranges.contiguous();
+    ctx->save_for_backward({rng});
+    ctx->saved_data["rows"] = lm.size(1);
+    return gather_rows(lm, rng);
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const Tensor rng = ctx->get_saved_variables()[0];
+    const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2), C = grads[0].size(3),
+                  S1 = ctx->saved_data["rows"].toInt();
+    DeviceGuard guard(grads[0].device());
+    const Tensor g = grads[0].contiguous();
+    Tensor lm_grad = at::empty({B, S1, C}, g.options());
+    check_rc(frnnt_pruning_bwd(dtype_code(g.scalar_type()), nullptr, g.data_ptr(), iptr(rng),
+                               nullptr, lm_grad.data_ptr(), (int)B, (int)S1 - 1, (int)T, (int)R,
+                               (int)C, stream_of(g)),
+             "frnnt_pruning_bwd");
+    return {lm_grad, Tensor()};
+  }
+};
+
+std::tuple<Tensor, Tensor> pruning(const Tensor &am, const Tensor &lm, const Tensor &ranges) {
+  TORCH_CHECK(lm.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): lm");
+  TORCH_CHECK(lm.scalar_type() == at::kFloat || lm.scalar_type() == at::kDouble ||
+                  lm.scalar_type() == at::kHalf || lm.scalar_type() == at::kBFloat16,
+              "fast_rnnt_amd supports float32, float64, float16 and bfloat16 tensors here, got ",
+              lm.scalar_type());
+  TORCH_CHECK(am.dim() == 3 && lm.dim() == 3 && ranges.dim() == 3 && am.size(0) == lm.size(0) &&
+                  ranges.size(0) == lm.size(0) && am.size(1) == ranges.size(1),
+              "am must be [B][T][C], lm [B][S+1][C], ranges [B][T][s_range]");
+  TORCH_CHECK(am.device() == lm.device() && ranges.device() == lm.device() &&
+                  am.scalar_type() == lm.scalar_type() && ranges.scalar_type() == at::kLong,
+              "am and lm must share a device and a type, ranges be int64 on that device");
+  const bool grad_mode = at::GradMode::is_enabled();
+  if (grad_mode && am.requires_grad() && lm.requires_grad() && am.size(2) == lm.size(2)) {
+    const variable_list out = PruningFn::apply(am, lm, ranges);
+    return {out[0], out[1]};
+  }
+  return {am.unsqueeze(2).expand({am.size(0), am.size(1), ranges.size(2), lm.size(2)}),
+          GatherRowsFn::apply(lm, ranges)};
+}
+
 void set_deferred_checks(bool on) { g_deferred = on; }
 bool deferred_checks() { return g_deferred; }
 
@@ -779,6 +934,8 @@ TORCH_LIBRARY(fast_rnnt_amd, m) {
       "lattice_loss(Tensor logits, Tensor symbols, Tensor? ranges, Tensor? boundary, "
       "int termination_symbol, int rnnt_type, float delay_penalty, bool return_grad, "
       "int reduction, int checks) -> (Tensor, Tensor?, Tensor?)");
+  m.def("prune_ranges(Tensor px_grad, Tensor py_grad, Tensor boundary, int s_range) -> Tensor");
+  m.def("pruning(Tensor am, Tensor lm, Tensor ranges) -> (Tensor, Tensor)");
 }
 // (PyTorch-ROCm keeps the dispatch key name CUDA for the MI355X)
 TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
@@ -787,6 +944,8 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
   m.impl("lattice_loss", &lattice_loss);
+  m.impl("prune_ranges", &prune_ranges);
+  m.impl("pruning", &pruning);
 }
 // The loss ops carry their own autograd nodes: the same functions serve the Autograd key
 // (they call the C ABI themselves and never re-dispatch).
@@ -794,6 +953,7 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, Autograd, m) {
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
   m.impl("lattice_loss", &lattice_loss);
+  m.impl("pruning", &pruning);
 }
 
 PYBIND11_MODULE(_C, m) {
@@ -814,6 +974,10 @@ PYBIND11_MODULE(_C, m) {
         py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
         py::arg("delay_penalty"), py::arg("return_grad"), py::arg("reduction"),
         py::arg("checks") = 0);
+  m.def("boundary_summary", &boundary_summary, py::arg("rows"));
+  m.def("prune_ranges", &prune_ranges, py::arg("px_grad"), py::arg("py_grad"), py::arg("boundary"),
+        py::arg("s_range"));
+  m.def("pruning", &pruning, py::arg("am"), py::arg("lm"), py::arg("ranges"));
   m.def("set_deferred_checks", &set_deferred_checks, py::arg("on"));
   m.def("deferred_checks", &deferred_checks);
   m.def("check_boundaries", &check_boundaries, py::arg("device"));

@@ -67,7 +67,7 @@ class MutualInformationRecursionFunction(torch.autograd.Function):
         return (px_grad, py_grad, None, None, None)
 
 
-_rows_cache = []  # [(weakref to the tensor, its version counter, rows)]
+_rows_cache = []  # [(weakref to the tensor, its version counter, rows, the rows as a host tensor)]
 
 
 def boundary_rows(boundary: Tensor, reread: bool = False):
@@ -77,16 +77,25 @@ def boundary_rows(boundary: Tensor, reread: bool = False):
     from the device only once.  Every in-place torch operation bumps the version
     counter; a writer that bypasses it (``.data``, a raw-pointer kernel) must pass
     ``reread=True`` once, or call :func:`forget_boundary_rows`."""
+    return _boundary_entry(boundary, reread)[2]
+
+
+def boundary_on_host(boundary: Tensor) -> Tensor:
+    """The host copy behind :func:`boundary_rows`, as a tensor."""
+    return _boundary_entry(boundary, False)[3]
+
+
+def _boundary_entry(boundary, reread):
     version = boundary._version
     if not reread:
-        for ref, ver, rows in _rows_cache:
-            if ref() is boundary and ver == version:
-                return rows
-    rows = boundary.tolist()
+        for entry in _rows_cache:
+            if entry[0]() is boundary and entry[1] == version:
+                return entry
+    host = boundary.detach().cpu().contiguous()
     _rows_cache[:] = [e for e in _rows_cache if e[0]() is not boundary and e[0]() is not None]
-    _rows_cache.insert(0, (weakref.ref(boundary), version, rows))
+    _rows_cache.insert(0, (weakref.ref(boundary), version, host.tolist(), host))
     del _rows_cache[8:]
-    return rows
+    return _rows_cache[0]
 
 
 def forget_boundary_rows() -> None:

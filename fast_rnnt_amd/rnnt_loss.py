@@ -20,8 +20,8 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .mutual_information import (_assert_boundary, boundary_rows,  # noqa: F401
-                                 mutual_information_recursion)
+from .mutual_information import (_assert_boundary, boundary_on_host,  # noqa: F401
+                                 boundary_rows, mutual_information_recursion)
 
 _RNNT_TYPES = {"regular": 0, "modified": 1, "constrained": 2}
 
@@ -430,26 +430,25 @@ def get_rnnt_prune_ranges(px_grad: Tensor, py_grad: Tensor, boundary: Tensor,
     assert T1 in [T, T + 1], T1
     assert py_grad.shape == (B, S + 1, T), py_grad.shape
     assert boundary.shape == (B, 4), boundary.shape
-    validate_st_lengths(S, T, is_regular, boundary)
+    # From the host copy of the boundary rows that an earlier call on the same tensor has
+    # usually left behind (no kernels and no wait for the device then): the assertions of
+    # validate_st_lengths, and the maximum over the batch of trunc((S_b - 1) / T_b) + 2
+    # (rnnt_loss.py:696-710).
+    s_range_min = None
+    if B > 0 and boundary.dtype == torch.int64:
+        least_s, least_slack, empty, s_range_min = _lib.ops().boundary_summary(
+            boundary_on_host(boundary))
+        assert least_s >= 1, boundary[:, 2]
+        assert is_regular or least_slack >= 0, \
+            f"Modified transducer requires T >= S, but got T={boundary[:, 3]} and S={boundary[:, 2]}"
+        if is_regular and empty:
+            raise RuntimeError("ZeroDivisionError")  # what the reference's integer division raises
     _check_tensors([("px_grad", px_grad), ("py_grad", py_grad)], [("boundary", boundary)])
-
-    if is_regular:
-        # max over the batch of trunc((S_b - 1) / T_b) + 2 (rnnt_loss.py:696-710), from the
-        # host copy of the boundary rows that the loss call before this one has usually left
-        # behind: no kernels and no wait for the device here
-        s_range_min = None
-        for _s_begin, _t_begin, s_end, t_end in boundary_rows(boundary):
-            if t_end == 0:
-                raise RuntimeError("ZeroDivisionError")  # what the reference's integer division raises
-            quotient = abs(s_end - 1) // abs(t_end)
-            if (s_end - 1 < 0) != (t_end < 0):
-                quotient = -quotient
-            s_range_min = quotient + 2 if s_range_min is None else max(s_range_min, quotient + 2)
-        if s_range_min is not None and s_range < s_range_min:
-            print(f"Warning: get_rnnt_prune_ranges - got s_range={s_range} "
-                  f"for boundaries S={boundary[:, 2]}, T={boundary[:, 3]}. "
-                  f"Adjusting to {s_range_min}")
-            s_range = s_range_min
+    if is_regular and s_range_min is not None and s_range < s_range_min:
+        print(f"Warning: get_rnnt_prune_ranges - got s_range={s_range} "
+              f"for boundaries S={boundary[:, 2]}, T={boundary[:, 3]}. "
+              f"Adjusting to {s_range_min}")
+        s_range = s_range_min
     if s_range > S:
         s_range = S + 1
     if is_regular:
@@ -461,44 +460,7 @@ def get_rnnt_prune_ranges(px_grad: Tensor, py_grad: Tensor, boundary: Tensor,
             "Pruning range for modified RNN-T should be equal to or greater than 1, "
             "or no valid paths could survive pruning.")
 
-    sfx = _lib.suffix(px_grad.dtype)
-    gx, gy = px_grad.detach().contiguous(), py_grad.detach().contiguous()
-    bnd = boundary.contiguous()
-    with torch.cuda.device(px_grad.device):
-        ranges = torch.empty(B, T, int(s_range), dtype=torch.int64, device=px_grad.device)
-        _lib.call("frnnt_prune_ranges_" + sfx, gx.data_ptr(), gy.data_ptr(), bnd.data_ptr(),
-                  ranges.data_ptr(), B, S, T, int(not is_regular), int(s_range),
-                  _lib.stream_of(px_grad))
-    return ranges
-
-
-class _PruneGather(torch.autograd.Function):
-    """lm_pruned[b,t,j,:] = lm[b, ranges[b,t,j], :]: frnnt_prune_gather / _bwd."""
-
-    @staticmethod
-    def forward(ctx, lm, ranges):
-        B, S1, C = lm.shape
-        _, T, R = ranges.shape
-        sfx = _lib.suffix(lm.dtype, narrow=True)
-        lm_c, rng_c = lm.contiguous(), ranges.contiguous()
-        with torch.cuda.device(lm.device):
-            out = torch.empty(B, T, R, C, dtype=lm.dtype, device=lm.device)
-            _lib.call("frnnt_prune_gather_" + sfx, lm_c.data_ptr(), rng_c.data_ptr(),
-                      out.data_ptr(), B, S1 - 1, T, R, C, _lib.stream_of(lm))
-        ctx.save_for_backward(rng_c)
-        ctx.meta = (B, S1, T, R, C, sfx)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        (rng,) = ctx.saved_tensors
-        B, S1, T, R, C, sfx = ctx.meta
-        grad = grad.contiguous()
-        with torch.cuda.device(grad.device):
-            lm_grad = torch.empty(B, S1, C, dtype=grad.dtype, device=grad.device)
-            _lib.call("frnnt_prune_gather_bwd_" + sfx, grad.data_ptr(), rng.data_ptr(),
-                      lm_grad.data_ptr(), B, S1 - 1, T, R, C, _lib.stream_of(grad))
-        return lm_grad, None
+    return _lib.ops().prune_ranges(px_grad.detach(), py_grad.detach(), boundary, int(s_range))
 
 
 def do_rnnt_pruning(am: Tensor, lm: Tensor, ranges: Tensor) -> Tuple[Tensor, Tensor]:
@@ -513,9 +475,7 @@ def do_rnnt_pruning(am: Tensor, lm: Tensor, ranges: Tensor) -> Tuple[Tensor, Ten
     (B, T, s_range) = ranges.shape
     (B, S1, C) = lm.shape
     _check_tensors([("am", am), ("lm", lm)], [("ranges", ranges)])
-    am_pruning = am.unsqueeze(2).expand((B, T, s_range, C))
-    lm_pruning = _PruneGather.apply(lm, ranges)
-    return am_pruning, lm_pruning
+    return _lib.ops().pruning(am, lm, ranges)
 
 
 _ACTIVATIONS = {None: 0, "none": 0, "tanh": 1}

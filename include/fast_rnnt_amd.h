@@ -561,6 +561,18 @@ int frnnt_prune_gather_bwd_bf16(const void *grad, const int64_t *ranges, void *l
                                 int S, int T, int R, int C, void *stream);
 
 /*
+ * Both adjoints of do_rnnt_pruning (rnnt_loss.py:780-818) at once, for elements of any type
+ * (FRNNT_F32 ...):
+ *   am_grad[b][t][:] = sum_j am_pruned_grad[b][t][j][:]
+ *   lm_grad[b][s][:] = sum over the (t, j) with ranges[b][t][j] = s of lm_pruned_grad[b][t][j][:]
+ * in a fixed order.  Either output may be NULL; the two gradients may be one tensor, whose
+ * entries are then read once.  2-byte elements are summed in float32.
+ */
+int frnnt_pruning_bwd(int dtype, const void *am_pruned_grad, const void *lm_pruned_grad,
+                      const int64_t *ranges, void *am_grad, void *lm_grad, int B, int S, int T,
+                      int R, int C, void *stream);
+
+/*
  * The joiner's input straight from the pruning bounds:
  *   out[b][t][j][:] = act(am[b][t][:] + lm[b][ranges[b][t][j]][:])
  * i.e. what a joiner of the usual form computes first from the two tensors of
