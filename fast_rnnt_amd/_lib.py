@@ -46,8 +46,7 @@ _SIGNATURES = {
     "frnnt_smoothed_logprobs_bwd_f64": ([_P] * 21 + [_I] * 6 + [_D, _D, _P], _I),
     "frnnt_simple_loss_fwd_f32": ([_P] * 14 + [_I] * 8 + [_P, _P], _I),
     "frnnt_simple_loss_fwd_f64": ([_P] * 14 + [_I] * 8 + [_P, _P], _I),
-    "frnnt_additive_loss_workspace": ([_I] * 5, ctypes.c_int64),
-    "frnnt_additive_loss_fwd": ([_I] + [_P] * 17 + [_I] * 6 + [_D, _I, _I, _P, _P], _I),
+    "frnnt_additive_loss_fwd": ([_I] + [_P] * 16 + [_I] * 6 + [_D, _I, _I, _P, _P], _I),
     "frnnt_additive_loss_bwd": ([_I] + [_P] * 8 + [_I, _D] + [_P] * 8 + [_I] * 6 + [_P], _I),
     "frnnt_mi_loss_fwd_f32": ([_P] * 8 + [_I] * 6 + [_P, _P], _I),
     "frnnt_mi_loss_fwd_f64": ([_P] * 8 + [_I] * 6 + [_P, _P], _I),

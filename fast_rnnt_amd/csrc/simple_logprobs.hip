@@ -475,6 +475,8 @@ struct ProdShape {
   static constexpr int kRows = kM + kC;                         // rows of a k-step in LDS: m, then c
   static constexpr int kStepBytes = kRows * kProdRowBytes;
   static constexpr size_t kLdsBytes = 2 * kStepBytes;  // (holds the listed gx rows as well)
+  // (four workgroups share 160 KB: with the bodies' own arrays, 6 floats per row)
+  static_assert(kLdsBytes + 6 * 4 * kM <= 40 << 10, "LDS per CU");
   static constexpr int kMTiles = kM / 64, kCTiles = kC / 64;    // 32-row and -column tiles per wave
   static constexpr int kMColumns = kM / 64, kColumns = kC / 64; // columns per thread of a k-major fetch
 };
@@ -728,7 +730,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
   using Shape = ProdShape<kM, kC>;
   using namespace dgemm;
   extern __shared__ __align__(16) char prod_lds[];
-  __shared__ float frame_mx[kM], frame_y[4][kM];
+  __shared__ float frame_mx[kM], frame_y[kM];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
   const int c_tiles = (C + kC - 1) / kC, t_tiles = (T + kM - 1) / kM;
@@ -834,6 +836,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
     const __amdgpu_buffer_rsrc_t gx_rs = buffer_of(gxb, S * T1 * 4);
     if ((unsigned)(term - c_tile) < (unsigned)kC) {  // (uniform)
       const __amdgpu_buffer_rsrc_t gy_rs = buffer_of(gpy + (long)b * S1 * T, S1 * T * 4);
+      float *part = reinterpret_cast<float *>(prod_lds);
       float sum[Shape::kMColumns] = {};
       constexpr int kAhead = 8;
       auto add_rows = [&](__amdgpu_buffer_rsrc_t rs, int rows, int pitch) {
@@ -856,7 +859,10 @@ __device__ __forceinline__ void simple_bwd_am_body(
       // (constrained: py[s + 1] also went into px[s])
       if (rnnt_type == kConstrained) add_rows(gx_rs, min(k_lim, S), T1);
 #pragma unroll
-      for (int w = 0; w < Shape::kMColumns; ++w) frame_y[wave][lane + 64 * w] = sum[w];
+      for (int w = 0; w < Shape::kMColumns; ++w) part[wave * kM + lane + 64 * w] = sum[w];
+      lds_barrier();
+      if (tid < kM)
+        frame_y[tid] = (part[tid] + part[kM + tid]) + (part[2 * kM + tid] + part[3 * kM + tid]);
       lds_barrier();
     }
     constexpr int kHotPitch = kM + 4;
@@ -897,7 +903,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
             const int m = row_of(j, v);
             acc[j][n][v] *= __expf(in[j][n][v] - frame_mx[m]);
             if (c0 + 32 * n == term)
-              acc[j][n][v] += (frame_y[0][m] + frame_y[1][m]) + (frame_y[2][m] + frame_y[3][m]);
+              acc[j][n][v] += frame_y[m];
           }
     };
     int listed = 0;
@@ -963,16 +969,14 @@ __device__ __forceinline__ void simple_bwd_am_body(
 // launchers: float goes to the product kernels above, double to the LDS-tiled ones
 void launch_fwd_gemm(const float *lm, const float *am, const int64_t *symbols,
                      const int64_t *boundary, float *lm_max, float *am_max, float *px,
-                     float *py, float *norm_raw, const int64_t *window, float *workspace,
-                     double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
+                     float *py, float *norm_raw, const int64_t *window, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
                      hipStream_t stream) {
   launch_normalizer_f32(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw, window,
-                        workspace, delay_penalty, B, S, T, C, term, rnnt_type, stream);
+                        delay_penalty, B, S, T, C, term, rnnt_type, stream);
 }
 void launch_fwd_gemm(const double *lm, const double *am, const int64_t *symbols,
                      const int64_t *boundary, const double *lm_max, const double *am_max,
-                     double *px, double *py, double *norm_raw, const int64_t *, double *,
-                     double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
+                     double *px, double *py, double *norm_raw, const int64_t *, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
                      hipStream_t stream) {
   // (the double kernels compute the whole lattice whether or not a window is given)
   const int t_tiles = T > 0 ? (T + kTileN - 1) / kTileN : 1;
@@ -1084,7 +1088,7 @@ void launch_scale(R *px_grad, R *py_grad, const R *score_grad, int score_grad_st
 
 template <typename R>
 int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary, R *px,
-             R *py, R *lm_max, R *am_max, R *norm_raw, R *workspace, double delay_penalty, int B,
+             R *py, R *lm_max, R *am_max, R *norm_raw, double delay_penalty, int B,
              int S, int T, int C, int term, int rnnt_type, int window_only, void *stream_) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_fwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2)
@@ -1109,7 +1113,7 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   // an empty-frame regular lattice is still written)
   const bool constrained = rnnt_type == kConstrained;
   launch_fwd_gemm(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw,
-                  window_only ? boundary : nullptr, workspace, constrained ? 0.0 : delay_penalty, B,
+                  window_only ? boundary : nullptr, constrained ? 0.0 : delay_penalty, B,
                   S, T, C, term, rnnt_type, stream);
   if (constrained && S > 0 && T > 0) {
     const long total = (long)B * S * T;
@@ -1245,18 +1249,16 @@ float *own_scratch_address() {
 
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
-                        float *am_max, float *norm_raw, float *workspace, double delay_penalty,
-                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream) {
-  return fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, workspace,
+  return fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
                          delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
 }
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
-                        double *am_max, double *norm_raw, double *workspace, double delay_penalty,
-                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        double *am_max, double *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream) {
-  return fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, workspace,
+  return fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
                           delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
 }
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
@@ -1346,7 +1348,7 @@ int frnnt_simple_logprobs_fwd_f32(const float *lm, const float *am, const int64_
                                   int termination_symbol, int rnnt_type, int window_only,
                                   void *stream) {
   return frnnt::fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                                nullptr, 0.0, B, S, T, C, termination_symbol, rnnt_type,
+                                0.0, B, S, T, C, termination_symbol, rnnt_type,
                                 window_only, stream);
 }
 int frnnt_simple_logprobs_fwd_f64(const double *lm, const double *am, const int64_t *symbols,
@@ -1355,7 +1357,7 @@ int frnnt_simple_logprobs_fwd_f64(const double *lm, const double *am, const int6
                                   int termination_symbol, int rnnt_type, int window_only,
                                   void *stream) {
   return frnnt::fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                                 nullptr, 0.0, B, S, T, C, termination_symbol, rnnt_type,
+                                 0.0, B, S, T, C, termination_symbol, rnnt_type,
                                  window_only, stream);
 }
 int frnnt_simple_logprobs_bwd_f32(const float *lm, const float *am, const int64_t *symbols,

@@ -35,7 +35,7 @@ template <typename R, typename Forward, typename Backward, typename Reduce>
 int simple_loss_fwd(Forward forward, Backward backward, Reduce reduce,
                     const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary,
                     R *px, R *py, R *lm_max, R *am_max, R *norm_raw, R *p, R *scores, R *px_grad,
-                    R *py_grad, R *loss, R *workspace, int B, int S, int T, int C, int term,
+                    R *py_grad, R *loss, int B, int S, int T, int C, int term,
                     int rnnt_type, double delay_penalty, int reduction, int checks,
                     int32_t *status, void *stream) {
   if ((px_grad == nullptr) != (py_grad == nullptr))
@@ -43,7 +43,7 @@ int simple_loss_fwd(Forward forward, Backward backward, Reduce reduce,
   // px / py only feed the recursion below, with the same boundary: what lies outside an
   // utterance's window need not be computed
   const int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                                     workspace, delay_penalty, B, S, T, C, term, rnnt_type,
+                                     delay_penalty, B, S, T, C, term, rnnt_type,
                                      boundary != nullptr, stream);
   if (rc != FRNNT_OK) return rc;
   return mi_loss_fwd<R>(forward, backward, reduce, px, py, boundary, p, scores, px_grad, py_grad,
@@ -83,7 +83,7 @@ int frnnt_simple_loss_fwd_f32(const float *lm, const float *am, const int64_t *s
   return frnnt::simple_loss_fwd<float>(frnnt_mi_forward_checked_f32,
                                        frnnt_mi_backward_f32, frnnt_loss_reduce_f32, lm, am,
                                        symbols, boundary, px, py, lm_max, am_max, norm_raw, p,
-                                       scores, px_grad, py_grad, loss, nullptr, B, S,
+                                       scores, px_grad, py_grad, loss, B, S,
                                        T, C, termination_symbol, rnnt_type, 0.0, reduction, checks,
                                        status, stream);
 }
@@ -96,20 +96,16 @@ int frnnt_simple_loss_fwd_f64(const double *lm, const double *am, const int64_t 
   return frnnt::simple_loss_fwd<double>(frnnt_mi_forward_checked_f64,
                                         frnnt_mi_backward_f64, frnnt_loss_reduce_f64, lm, am,
                                         symbols, boundary, px, py, lm_max, am_max, norm_raw, p,
-                                        scores, px_grad, py_grad, loss, nullptr, B, S,
+                                        scores, px_grad, py_grad, loss, B, S,
                                         T, C, termination_symbol, rnnt_type, 0.0, reduction, checks,
                                         status, stream);
 }
 
-int64_t frnnt_additive_loss_workspace(int dtype, int B, int S, int T, int C) {
-  if (dtype == FRNNT_F64 || B <= 0 || S < 0 || T <= 0 || C < 1) return 0;
-  return (int64_t)frnnt::normalizer_workspace_floats(B, S, T, C);
-}
 int frnnt_additive_loss_fwd(int dtype, const void *lm, const void *am, const int64_t *symbols,
                             const int64_t *boundary, void *lm_wide, void *am_wide, void *px,
                             void *py, void *lm_max, void *am_max, void *norm_raw, void *p,
                             void *scores, void *px_grad, void *py_grad, void *loss,
-                            void *workspace, int B, int S, int T, int C, int termination_symbol,
+                            int B, int S, int T, int C, int termination_symbol,
                             int rnnt_type, double delay_penalty, int reduction, int checks,
                             int32_t *status, void *stream) {
   using frnnt::fail;
@@ -130,7 +126,7 @@ int frnnt_additive_loss_fwd(int dtype, const void *lm, const void *am, const int
     return frnnt::simple_loss_fwd<R>(
         forward, backward, reduce, static_cast<const R *>(lm), static_cast<const R *>(am), symbols,
         boundary, out(px), out(py), out(lm_max), out(am_max), out(norm_raw), out(p), out(scores),
-        out(px_grad), out(py_grad), out(loss), out(workspace), B, S, T, C, termination_symbol,
+        out(px_grad), out(py_grad), out(loss), B, S, T, C, termination_symbol,
         rnnt_type, delay_penalty > 0.0 ? delay_penalty : 0.0, reduction, checks, status, stream);
   };
   if (dtype == FRNNT_F64)

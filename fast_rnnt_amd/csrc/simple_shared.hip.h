@@ -113,26 +113,20 @@ __device__ __forceinline__ void lds_barrier() {
 }  // namespace
 
 // The float32 normalizer product with px / py in its epilogue (simple_normalizer.hip).
-// `workspace`: normalizer_workspace_floats() floats, or NULL (the sum over the vocabulary is then
-// not cut into stretches).
 void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symbols,
                            const int64_t *boundary, float *lm_max, float *am_max, float *px,
-                           float *py, float *norm_raw, const int64_t *window, float *workspace,
+                           float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
                            int rnnt_type, hipStream_t stream);
-size_t normalizer_workspace_floats(int B, int S, int T, int C);
 
-// frnnt_simple_logprobs_fwd with a workspace (may be NULL) and the delay penalty
-// (simple_logprobs.hip).
+// frnnt_simple_logprobs_fwd with the delay penalty (simple_logprobs.hip).
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
-                        float *am_max, float *norm_raw, float *workspace, double delay_penalty,
-                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream);
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
-                        double *am_max, double *norm_raw, double *workspace, double delay_penalty,
-                        int B, int S, int T, int C, int term, int rnnt_type, int window_only,
+                        double *am_max, double *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream);
 // 2-byte lm and am (`dtype`: FRNNT_F16 or FRNNT_BF16) as float32, in one launch.
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,

@@ -444,12 +444,10 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
                   o_lmw = keep.take(narrow ? B * (S + 1) * C : 0),
                   o_amw = keep.take(narrow ? B * T * C : 0);
     Tensor kept = at::empty({keep.total}, opts);
-    // what it does not: px | py | p | scores | workspace
-    const int64_t n_ws = frnnt_additive_loss_workspace(dtype, (int)B, (int)S, (int)T, (int)C);
+    // what it does not: px | py | p | scores
     Carver carve;
     const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(n_py),
-                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B),
-                  o_ws = carve.take(n_ws);
+                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B);
     const Tensor work = at::empty({carve.total}, opts);
     char *k = static_cast<char *>(kept.data_ptr()), *w = static_cast<char *>(work.data_ptr());
     Tensor gx, gy;
@@ -464,7 +462,7 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
                  w + o_px * item, w + o_py * item, k + o_lmx * item, k + o_amx * item,
                  need_grad ? k + o_nr * item : nullptr, w + o_p * item, w + o_sc * item,
                  gx.defined() ? gx.data_ptr() : nullptr, gy.defined() ? gy.data_ptr() : nullptr,
-                 loss.data_ptr(), n_ws ? w + o_ws * item : nullptr, (int)B, (int)S, (int)T, (int)C,
+                 loss.data_ptr(), (int)B, (int)S, (int)T, (int)C,
                  (int)term, (int)kind, delay_penalty, (int)reduction, (int)checks,
                  status_for(am, bnd), stream_of(am)),
              "frnnt_additive_loss_fwd");

@@ -301,9 +301,6 @@ int frnnt_simple_loss_fwd_f64(const double *lm, const double *am, const int64_t 
  * float otherwise.  _fwd is frnnt_simple_loss_fwd, and
  *   lm_wide [B][S+1][C], am_wide [B][T][C]: out for 2-byte inputs, the inputs as float32 (the
  *     backward reads them); not used (NULL) for the other types
- *   workspace: frnnt_additive_loss_workspace() floats, or NULL: with it the contraction over a
- *     large vocabulary is cut into stretches where that fills the chip better (the sums then round
- *     a little differently); the function returns 0 where no workspace is of use
  *   delay_penalty > 0 is added to px as in rnnt_loss.py:309-324.
  * _bwd is frnnt_simple_logprobs_bwd with window_only set when a boundary is given: lm, am the
  * inputs (lm_wide, am_wide for 2-byte inputs), lm_grad, am_grad of the inputs' type `dtype`.
@@ -312,12 +309,11 @@ int frnnt_simple_loss_fwd_f64(const double *lm, const double *am, const int64_t 
 #define FRNNT_F64 1
 #define FRNNT_F16 2
 #define FRNNT_BF16 3
-int64_t frnnt_additive_loss_workspace(int dtype, int B, int S, int T, int C);
 int frnnt_additive_loss_fwd(int dtype, const void *lm, const void *am, const int64_t *symbols,
                             const int64_t *boundary, void *lm_wide, void *am_wide, void *px,
                             void *py, void *lm_max, void *am_max, void *norm_raw, void *p,
                             void *scores, void *px_grad, void *py_grad, void *loss,
-                            void *workspace, int B, int S, int T, int C, int termination_symbol,
+                            int B, int S, int T, int C, int termination_symbol,
                             int rnnt_type, double delay_penalty, int reduction, int checks,
                             int32_t *status, void *stream);
 int frnnt_additive_loss_bwd(int dtype, const void *lm, const void *am, const int64_t *symbols,

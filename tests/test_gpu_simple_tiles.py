@@ -1,6 +1,6 @@
-"""rnnt_loss_simple where the kernels' choice of tiles and of stretches of the vocabulary, and
+"""rnnt_loss_simple where the kernels' choice of tiles and
 their splits into chunks, can go wrong: sizes on either side of a tile of lattice rows, frames and
-vocabulary entries, sums over 1 ... 8 stretches, batches small and large, 2-byte inputs, long
+vocabulary entries, sums over few and many chunks, batches small and large, 2-byte inputs, long
 lists of equal symbols.  Oracle: the CPU restatement on the same values in float32."""
 import pytest
 import torch
