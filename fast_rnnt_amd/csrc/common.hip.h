@@ -185,9 +185,18 @@ __device__ __forceinline__ void reduce_scores(const R *__restrict__ scores, R *_
   if (lane == 0) loss[0] = reduction == 1 ? -(acc / (R)B) : -acc;
 }
 
-// The recursion's backward with a gradient of ones which, on its way, also reduces the
+// The recursion's forward for a caller that goes on to mi_backward_and_loss with `px_grad` (NULL: it
+// does not): what that kernel wants to find there is prepared along with what this one wants.
+// Host side, mi_recursion.hip.
+int mi_forward(const float *px, const float *py, const int64_t *boundary, float *p, float *scores,
+               int B, int S, int T, int modified, int checks, int32_t *status, float *px_grad,
+               void *stream);
+int mi_forward(const double *px, const double *py, const int64_t *boundary, double *p,
+               double *scores, int B, int S, int T, int modified, int checks, int32_t *status,
+               double *px_grad, void *stream);
+// The backward with a gradient of ones, after such a forward, which, on its way, also reduces the
 // forward's scores to the loss (a staging wave of the first workgroup does it once its
-// tiles are done): saves the launch of a reduction kernel.  Host side, mi_recursion.hip.
+// tiles are done): saves the launch of a reduction kernel.
 int mi_backward_and_loss(const float *px, const int64_t *boundary, const float *p, float *px_grad,
                          float *py_grad, const float *scores, float *loss, int B, int S, int T,
                          int modified, int reduction, void *stream);

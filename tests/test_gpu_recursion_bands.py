@@ -1,0 +1,46 @@
+"""The recursion where every band of 64 lattice rows has a workgroup of its own: two, three and four
+bands, sizes at the edges of bands and of 32-step tiles, windows that leave bands out, are empty or
+start inside the lattice.  The same utterances in a batch too large for that run with one workgroup
+each: the results must be the same bits.  Oracle: the CPU restatement in float32."""
+import pytest
+import torch
+
+from fast_rnnt_amd import _fast_rnnt
+from oracle import recursion as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("S,T", [(64, 1200), (100, 900), (127, 800), (128, 700), (129, 513), (191, 600),
+                                 (192, 320), (200, 257), (255, 288), (255, 300)])
+def test_bands_in_workgroups_of_their_own(gpu_device, S, T, modified):
+    g = torch.Generator().manual_seed(S + T)
+    rows = [[0, 0, S, T], [0, 0, S, T - 1], [0, 0, min(S, 63), T], [0, 0, 64, T], [1, 3, S, T],
+            [2, 1, S - 1, T - 31], [0, 0, S, 0], [5, 9, 5, T], [0, 5, S // 2, T - 7]]
+    n, T1 = len(rows), T if modified else T + 1
+    px = -1 + torch.randn(n, S, T1, generator=g)
+    py = -1 + torch.randn(n, S + 1, T, generator=g)
+    bnd = torch.tensor(rows)
+
+    def run(copies):
+        args = [x.to(gpu_device).repeat(copies, 1, 1) for x in (px, py)]
+        args.append(bnd.to(gpu_device).repeat(copies, 1))
+        p = torch.zeros(n * copies, S + 1, T + 1, device=gpu_device)
+        print(f"S={S} T={T} modified={modified} B={n * copies}", flush=True)
+        scores = _fast_rnnt.mutual_information_forward(*args, p)
+        seed = torch.ones(n * copies, device=gpu_device)
+        gx, gy = _fast_rnnt.mutual_information_backward(*args, p, seed)
+        return [x[-n:].cpu() for x in (scores, p, gx, gy, seed)]
+
+    got, whole = run(1), run(30)
+    for a, b in zip(got, whole):
+        assert torch.equal(a, b)
+    p_cpu = torch.zeros(n, S + 1, T + 1)
+    want = oracle.mi_forward(px, py, bnd, p_cpu)
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got[0]), finite)
+    assert bool(((got[0] - want).abs()[finite] <= 1e-5 * want.abs()[finite].clamp(min=1)).all())
+    gx, gy = oracle.mi_backward(px, py, bnd, p_cpu, torch.ones(n))
+    for a, b in ((got[2], gx), (got[3], gy)):
+        assert not torch.isnan(a).any() and bool((a - b).norm() <= 2e-3 * b.norm().clamp(min=1))
