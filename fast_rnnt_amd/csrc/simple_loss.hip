@@ -10,31 +10,27 @@ namespace {
 
 // The tail every loss function shares (e.g. rnnt_loss.py:326-340): the recursion, its
 // backward with a gradient of ones when the occupation gradients are wanted, the reduction.
-template <typename R, typename Backward, typename Reduce>
-int mi_loss_fwd(Backward backward, Reduce reduce, const R *px, const R *py,
+template <typename R, typename Reduce>
+int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
                 const int64_t *boundary, R *p, R *scores, R *px_grad, R *py_grad, R *loss, int B,
                 int S, int T, int modified, int reduction, int checks, int32_t *status,
                 void *stream) {
   if ((px_grad == nullptr) != (py_grad == nullptr))
     return fail(FRNNT_EINVAL, "mi_loss_fwd: px_grad and py_grad go together");
-  const bool with_loss = loss && B > 0;
-  int rc = mi_forward(px, py, boundary, p, scores, B, S, T, modified, checks, status,
-                      with_loss ? px_grad : nullptr, stream);
+  int rc = mi_forward(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad, stream);
   if (rc != FRNNT_OK) return rc;
   if (px_grad) {
     // with a loss to form, the backward kernel reduces the scores on its way
-    if (with_loss)
-      return mi_backward_and_loss(px, boundary, p, px_grad, py_grad, scores, loss, B, S, T,
-                                  modified, reduction, stream);
-    rc = backward(px, py, boundary, p, nullptr, px_grad, py_grad, B, S, T, modified, 0, stream);
-    if (rc != FRNNT_OK) return rc;
+    rc = mi_backward_and_loss(px, boundary, p, px_grad, py_grad, scores, loss, B, S, T, modified,
+                              reduction, stream);
+    if (rc != FRNNT_OK || B > 0) return rc;
   }
   if (loss) rc = reduce(scores, loss, B, reduction, stream);
   return rc;
 }
 
-template <typename R, typename Backward, typename Reduce>
-int simple_loss_fwd(Backward backward, Reduce reduce,
+template <typename R, typename Reduce>
+int simple_loss_fwd(Reduce reduce,
                     const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary,
                     R *px, R *py, R *lm_max, R *am_max, R *norm_raw, R *p, R *scores, R *px_grad,
                     R *py_grad, R *loss, int B, int S, int T, int C, int term,
@@ -48,7 +44,7 @@ int simple_loss_fwd(Backward backward, Reduce reduce,
                                      delay_penalty, B, S, T, C, term, rnnt_type,
                                      boundary != nullptr, stream);
   if (rc != FRNNT_OK) return rc;
-  return mi_loss_fwd<R>(backward, reduce, px, py, boundary, p, scores, px_grad, py_grad,
+  return mi_loss_fwd<R>(reduce, px, py, boundary, p, scores, px_grad, py_grad,
                         loss, B, S, T, rnnt_type != kRegular, reduction, checks, status, stream);
 }
 
@@ -61,8 +57,7 @@ int frnnt_mi_loss_fwd_f32(const float *px, const float *py, const int64_t *bound
                           float *scores, float *px_grad, float *py_grad, float *loss, int B, int S,
                           int T, int modified, int reduction, int checks, int32_t *status,
                           void *stream) {
-  return frnnt::mi_loss_fwd<float>(frnnt_mi_backward_f32,
-                                   frnnt_loss_reduce_f32, px, py, boundary, p, scores, px_grad,
+  return frnnt::mi_loss_fwd<float>(frnnt_loss_reduce_f32, px, py, boundary, p, scores, px_grad,
                                    py_grad, loss, B, S, T, modified, reduction, checks, status,
                                    stream);
 }
@@ -70,8 +65,7 @@ int frnnt_mi_loss_fwd_f64(const double *px, const double *py, const int64_t *bou
                           double *scores, double *px_grad, double *py_grad, double *loss, int B,
                           int S, int T, int modified, int reduction, int checks, int32_t *status,
                           void *stream) {
-  return frnnt::mi_loss_fwd<double>(frnnt_mi_backward_f64,
-                                    frnnt_loss_reduce_f64, px, py, boundary, p, scores, px_grad,
+  return frnnt::mi_loss_fwd<double>(frnnt_loss_reduce_f64, px, py, boundary, p, scores, px_grad,
                                     py_grad, loss, B, S, T, modified, reduction, checks, status,
                                     stream);
 }
@@ -82,7 +76,7 @@ int frnnt_simple_loss_fwd_f32(const float *lm, const float *am, const int64_t *s
                               float *px_grad, float *py_grad, float *loss, int B, int S, int T,
                               int C, int termination_symbol, int rnnt_type, int reduction,
                               int checks, int32_t *status, void *stream) {
-  return frnnt::simple_loss_fwd<float>(                                       frnnt_mi_backward_f32, frnnt_loss_reduce_f32, lm, am,
+  return frnnt::simple_loss_fwd<float>(                                       frnnt_loss_reduce_f32, lm, am,
                                        symbols, boundary, px, py, lm_max, am_max, norm_raw, p,
                                        scores, px_grad, py_grad, loss, B, S,
                                        T, C, termination_symbol, rnnt_type, 0.0, reduction, checks,
@@ -94,7 +88,7 @@ int frnnt_simple_loss_fwd_f64(const double *lm, const double *am, const int64_t 
                               double *px_grad, double *py_grad, double *loss, int B, int S, int T,
                               int C, int termination_symbol, int rnnt_type, int reduction,
                               int checks, int32_t *status, void *stream) {
-  return frnnt::simple_loss_fwd<double>(                                        frnnt_mi_backward_f64, frnnt_loss_reduce_f64, lm, am,
+  return frnnt::simple_loss_fwd<double>(                                        frnnt_loss_reduce_f64, lm, am,
                                         symbols, boundary, px, py, lm_max, am_max, norm_raw, p,
                                         scores, px_grad, py_grad, loss, B, S,
                                         T, C, termination_symbol, rnnt_type, 0.0, reduction, checks,
@@ -120,19 +114,18 @@ int frnnt_additive_loss_fwd(int dtype, const void *lm, const void *am, const int
     lm = lm_wide;
     am = am_wide;
   }
-  auto call = [&](auto r, auto backward, auto reduce) {
+  auto call = [&](auto r, auto reduce) {
     using R = decltype(r);
     auto out = [](void *q) { return static_cast<R *>(q); };
     return frnnt::simple_loss_fwd<R>(
-        backward, reduce, static_cast<const R *>(lm), static_cast<const R *>(am), symbols,
+        reduce, static_cast<const R *>(lm), static_cast<const R *>(am), symbols,
         boundary, out(px), out(py), out(lm_max), out(am_max), out(norm_raw), out(p), out(scores),
         out(px_grad), out(py_grad), out(loss), B, S, T, C, termination_symbol,
         rnnt_type, delay_penalty > 0.0 ? delay_penalty : 0.0, reduction, checks, status, stream);
   };
   if (dtype == FRNNT_F64)
-    return call(double(), frnnt_mi_backward_f64,
-                frnnt_loss_reduce_f64);
-  return call(float(), frnnt_mi_backward_f32, frnnt_loss_reduce_f32);
+    return call(double(), frnnt_loss_reduce_f64);
+  return call(float(), frnnt_loss_reduce_f32);
 }
 
 }  // extern "C"

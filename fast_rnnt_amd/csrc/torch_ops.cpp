@@ -369,6 +369,58 @@ struct RecursionLossFn : public torch::autograd::Function<RecursionLossFn> {
   }
 };
 
+// mutual_information_recursion (mutual_information.py:24-181) behind one autograd node: the scores,
+// the occupation gradients whenever they are handed out or a gradient may be wanted, and their
+// in-place scaling in the backward.  Unless they are handed out nobody else holds them by then, so
+// that px.grad and py.grad take them over without a copy.
+struct RecursionFn : public torch::autograd::Function<RecursionFn> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &px_, const Tensor &py_,
+                               const std::optional<Tensor> &boundary_, bool want_grads,
+                               bool need_grad) {
+    const Tensor boundary = or_undefined(boundary_);
+    const Tensor px = px_.contiguous(), py = py_.contiguous();
+    const Tensor bnd = boundary.defined() ? boundary.contiguous() : Tensor();
+    const int64_t B = px.size(0), S = px.size(1), T1 = px.size(2), T = py.size(2);
+    DeviceGuard guard(px.device());
+    const auto opts = px.options();
+    Tensor p = at::empty({B, S + 1, T + 1}, opts), scores = at::empty({B}, opts);
+    Tensor gx, gy;
+    if (want_grads || need_grad) {
+      gx = at::empty({B, S, T1}, opts);
+      gy = at::empty({B, S + 1, T}, opts);
+    }
+    auto run = [&](auto r) {
+      using R = decltype(r);
+      return abi_mi_loss_fwd(ptr<R>(px), ptr<R>(py), iptr(bnd), ptr<R>(p), ptr<R>(scores),
+                             ptr<R>(gx), ptr<R>(gy), (R *)nullptr, (int)B, (int)S, (int)T,
+                             (int)(T1 == T), 0, 0, status_for(px, bnd), stream_of(px));
+    };
+    check_rc(px.scalar_type() == at::kFloat ? run(float()) : run(double()), "frnnt_mi_loss_fwd");
+    if (need_grad) ctx->save_for_backward({gx, gy});
+    if (!want_grads) return {scores};
+    ctx->mark_non_differentiable({gx, gy});
+    return {scores, gx, gy};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &gx = saved[0], &gy = saved[1];
+    const int64_t B = gx.size(0), S = gx.size(1), T1 = gx.size(2), T = gy.size(2);
+    DeviceGuard guard(gx.device());
+    const Tensor g = grads[0].contiguous();
+    auto run = [&](auto r) {
+      using R = decltype(r);
+      return abi_mi_scale_grads(ptr<R>(gx), ptr<R>(gy), ptr<R>(g), 1, 1.0, (int)B, (int)S, (int)T,
+                                (int)(T1 == T), stream_of(gx));
+    };
+    check_rc(gx.scalar_type() == at::kFloat ? run(float()) : run(double()), "frnnt_mi_scale_grads");
+    // (a second backward through the node finds them changed, as it would after torch's own "*=")
+    gx.unsafeGetTensorImpl()->bump_version();
+    gy.unsafeGetTensorImpl()->bump_version();
+    return {gx, gy, Tensor(), Tensor(), Tensor()};
+  }
+};
+
 void require_float_gpu(const Tensor &t, const char *name) {
   TORCH_CHECK(t.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): ", name);
   TORCH_CHECK(t.scalar_type() == at::kFloat || t.scalar_type() == at::kDouble,
@@ -384,6 +436,24 @@ LossResult as_result(const variable_list &out) {
     gy = out[2];
   }
   return LossResult(out[0], gx, gy);
+}
+
+LossResult recursion(const Tensor &px, const Tensor &py, const std::optional<Tensor> &boundary_,
+                     bool return_grad) {
+  const Tensor boundary = or_undefined(boundary_);
+  require_float_gpu(px, "px");
+  TORCH_CHECK(px.dim() == 3 && py.dim() == 3, "px and py must be 3-dimensional");
+  const int64_t B = px.size(0), S = px.size(1), T1 = px.size(2), T = py.size(2);
+  TORCH_CHECK((T1 == T || T1 == T + 1) && py.size(0) == B && py.size(1) == S + 1,
+              "px must be [B][S][T or T+1], py [B][S+1][T]");
+  TORCH_CHECK(px.device() == py.device() && px.scalar_type() == py.scalar_type(),
+              "px and py must share one device and one dtype");
+  if (boundary.defined())
+    TORCH_CHECK(boundary.dim() == 2 && boundary.size(0) == B && boundary.size(1) == 4 &&
+                    boundary.scalar_type() == at::kLong && boundary.device() == px.device(),
+                "boundary must be an int64 [B][4] tensor on the same device");
+  const bool need_grad = at::GradMode::is_enabled() && (px.requires_grad() || py.requires_grad());
+  return as_result(RecursionFn::apply(px, py, boundary_, return_grad, need_grad));
 }
 
 LossResult recursion_loss(const Tensor &px, const Tensor &py,
@@ -922,6 +992,9 @@ TORCH_LIBRARY(fast_rnnt_amd, m) {
       "mutual_information_backward(Tensor px, Tensor py, Tensor? boundary, Tensor p, "
       "Tensor(a!) ans_grad) -> Tensor[]");
   m.def(
+      "recursion(Tensor px, Tensor py, Tensor? boundary, bool return_grad) -> "
+      "(Tensor, Tensor?, Tensor?)");
+  m.def(
       "recursion_loss(Tensor px, Tensor py, Tensor? boundary, bool return_grad, int reduction, "
       "int checks) -> (Tensor, Tensor?, Tensor?)");
   m.def(
@@ -939,6 +1012,7 @@ TORCH_LIBRARY(fast_rnnt_amd, m) {
 TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
   m.impl("mutual_information_forward", &mutual_information_forward);
   m.impl("mutual_information_backward", &mutual_information_backward);
+  m.impl("recursion", &recursion);
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
   m.impl("lattice_loss", &lattice_loss);
@@ -948,6 +1022,7 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
 // The loss ops carry their own autograd nodes: the same functions serve the Autograd key
 // (they call the C ABI themselves and never re-dispatch).
 TORCH_LIBRARY_IMPL(fast_rnnt_amd, Autograd, m) {
+  m.impl("recursion", &recursion);
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
   m.impl("lattice_loss", &lattice_loss);
@@ -962,6 +1037,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("mutual_information_backward", &mutual_information_backward, py::arg("px"),
         py::arg("py"), py::arg("boundary"), py::arg("p"), py::arg("ans_grad"));
   m.def("with_cuda", &with_cuda);
+  m.def("recursion", &recursion, py::arg("px"), py::arg("py"), py::arg("boundary"),
+        py::arg("return_grad"));
   m.def("recursion_loss", &recursion_loss, py::arg("px"), py::arg("py"), py::arg("boundary"),
         py::arg("return_grad"), py::arg("reduction"), py::arg("checks") = 0);
   m.def("simple_loss", &simple_loss, py::arg("lm"), py::arg("am"), py::arg("symbols"),

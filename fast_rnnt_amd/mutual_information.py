@@ -16,55 +16,12 @@ row (default ``[0, 0, S, T]``)::
 with out-of-window terms taken as -inf; the result is ``p[b, s_end, t_end]``.
 """
 import weakref
-from typing import List, Optional, Sequence, Tuple, Union
+from typing import Optional, Sequence, Tuple, Union
 
 import torch
 from torch import Tensor
 
 from . import _fast_rnnt, _lib
-
-
-class MutualInformationRecursionFunction(torch.autograd.Function):
-    """fast_rnnt/python/fast_rnnt/mutual_information.py:24-181.
-
-    ``forward`` runs the forward operator and, when gradients may be needed,
-    immediately the backward operator with a gradient of ones; ``backward`` then
-    only scales those stored occupation gradients (in place, which also changes
-    the tensors handed out through ``pxy_grads``).
-    """
-
-    @staticmethod
-    def forward(ctx, px: Tensor, py: Tensor, pxy_grads: List[Optional[Tensor]],
-                boundary: Optional[Tensor] = None, return_grad: bool = False) -> Tensor:
-        (B, S, T1) = px.shape
-        T = py.shape[-1]
-        assert T1 in [T, T + 1]
-        assert py.shape == (B, S + 1, T)
-        if boundary is not None:
-            assert boundary.shape == (B, 4)
-
-        p = torch.empty(B, S + 1, T + 1, device=px.device, dtype=px.dtype)
-        ans = _fast_rnnt.mutual_information_forward(px, py, boundary, p)
-
-        px_grad, py_grad = None, None
-        if return_grad or px.requires_grad or py.requires_grad:
-            ans_grad = torch.ones(B, device=px.device, dtype=px.dtype)
-            (px_grad, py_grad) = _fast_rnnt.mutual_information_backward(
-                px, py, boundary, p, ans_grad)
-            ctx.save_for_backward(px_grad, py_grad)
-        assert len(pxy_grads) == 2
-        pxy_grads[0] = px_grad
-        pxy_grads[1] = py_grad
-        return ans
-
-    @staticmethod
-    def backward(ctx, ans_grad: Tensor) -> Tuple[Tensor, Tensor, None, None, None]:
-        (px_grad, py_grad) = ctx.saved_tensors
-        (B,) = ans_grad.shape
-        ans_grad = ans_grad.reshape(B, 1, 1)
-        px_grad *= ans_grad
-        py_grad *= ans_grad
-        return (px_grad, py_grad, None, None, None)
 
 
 _rows_cache = []  # [(weakref to the tensor, its version counter, rows, the rows as a host tensor)]
@@ -163,10 +120,11 @@ def mutual_information_recursion(
     if boundary is not None:
         _assert_boundary(boundary, B, S, T, on_device=_lib.ops().deferred_checks())
 
-    px, py = px.contiguous(), py.contiguous()
-    pxy_grads = [None, None]
-    scores = MutualInformationRecursionFunction.apply(px, py, pxy_grads, boundary, return_grad)
-    px_grad, py_grad = pxy_grads
+    # one autograd node of the operator module (mutual_information.py:24-181): its forward runs
+    # the forward operator and, when gradients may be needed, immediately the backward operator
+    # with a gradient of ones; its backward only scales those stored occupation gradients (in
+    # place, which also changes the tensors handed out here)
+    scores, px_grad, py_grad = _lib.ops().recursion(px, py, boundary, bool(return_grad))
     return (scores, (px_grad, py_grad)) if return_grad else scores
 
 
