@@ -44,6 +44,9 @@ _SIGNATURES = {
     "frnnt_smoothed_logprobs_fwd_f64": ([_P] * 14 + [_I] * 6 + [_D, _D, _P], _I),
     "frnnt_smoothed_logprobs_bwd_f32": ([_P] * 21 + [_I] * 6 + [_D, _D, _P], _I),
     "frnnt_smoothed_logprobs_bwd_f64": ([_P] * 21 + [_I] * 6 + [_D, _D, _P], _I),
+    "frnnt_smoothed_loss_kept": ([_I] * 4, ctypes.c_int64),
+    "frnnt_smoothed_loss_fwd_f32": ([_P] * 15 + [_I] * 6 + [_D] * 3 + [_I, _I, _P, _P], _I),
+    "frnnt_smoothed_loss_bwd_f32": ([_P] * 6 + [_I, _D] + [_P] * 5 + [_I] * 6 + [_D, _D, _P], _I),
     "frnnt_simple_loss_fwd_f32": ([_P] * 14 + [_I] * 8 + [_P, _P], _I),
     "frnnt_simple_loss_fwd_f64": ([_P] * 14 + [_I] * 8 + [_P, _P], _I),
     "frnnt_additive_loss_fwd": ([_I] + [_P] * 16 + [_I] * 6 + [_D, _I, _I, _P, _P], _I),

@@ -240,7 +240,8 @@ __global__ void __launch_bounds__(256)
 // 256-thread workgroups.  The first ceil(B*(S+1)/4) of them give each wave one
 // lattice row (b, s): D[b,s,:] and the two row sums.  With `score_grad` the wave first scales
 // its row of the occupation gradients in place (scale_by_batch_kernel's work, for lattices whose
-// rows do not read each other's: one pass over them less).  Loads are issued in batches of
+// rows do not read each other's: one pass over them less).  `joint`: what they count for here
+// (1, less in the smoothed loss).  Loads are issued in batches of
 // four before anything is stored, so a row costs one memory round trip, not one per 64 frames.
 // In double the next workgroups take 64 frames of one utterance each and form the column
 // sums, the four waves splitting the lattice rows (the float product forms those it needs).  The
@@ -250,7 +251,7 @@ __global__ void __launch_bounds__(256)
     simple_bwd_prep_kernel(R *__restrict__ gpx, R *__restrict__ gpy,
                            const R *__restrict__ norm_raw, const int64_t *__restrict__ boundary,
                            const int64_t *__restrict__ window, const R *__restrict__ score_grad,
-                           int stride, R scale, R *__restrict__ dmat, R *__restrict__ row_x,
+                           int stride, R scale, R joint, R *__restrict__ dmat, R *__restrict__ row_x,
                            R *__restrict__ row_y, R *__restrict__ col_y, int B, int S, int T,
                            int ldd, int rnnt_type) {
   __shared__ R partial[4][kWave];
@@ -298,6 +299,8 @@ __global__ void __launch_bounds__(256)
         }
         if (!ok || t == t_mask) gx[u] = (R)0;
         if (!ok) gy[u] = (R)0;
+        gx[u] *= joint;
+        gy[u] *= joint;
         if (t < T) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
         sx += gx[u];
         sy += gy[u];
@@ -563,7 +566,7 @@ __device__ __forceinline__ void multiply_chunk(const char *lds, int wave_m, int 
   }
 }
 
-template <int kM, int kC>
+template <int kM, int kC, bool kSmooth>
 __device__ __forceinline__ void simple_bwd_lm_body(
     int block_id, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const float *__restrict__ lm_max,
@@ -708,7 +711,9 @@ __device__ __forceinline__ void simple_bwd_lm_body(
           float g = __expf(in[j][n][v] - row_mx[m]) * acc[j][n][v];
           if (c == row_sym[m]) g += row_rx[m];
           if (c == term) g += row_ry[m];
-          store(out_rs, c < C, first + 32 * n, below(j, v), s < s_lim ? g : 0.f);
+          if (!(s < s_lim)) g = 0.f;
+          if (kSmooth) g += get_float(out_rs, c < C, 4 * (first + 32 * n), 4 * below(j, v));
+          store(out_rs, c < C, first + 32 * n, below(j, v), g);
         }
   });
 }
@@ -718,7 +723,7 @@ __device__ __forceinline__ void simple_bwd_lm_body(
 // exact (products by 0 or 1) and has a fixed summation order.  The lattice rows whose symbol lies
 // in the workgroup's vocabulary range are listed in order; their gx rows go to LDS, some at a
 // time, and are multiplied two rows at a time onto the finished dense results.
-template <int kM, int kC>
+template <int kM, int kC, bool kSmooth>
 __device__ __forceinline__ void simple_bwd_am_body(
     int block_id, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const int64_t *__restrict__ boundary,
@@ -726,11 +731,11 @@ __device__ __forceinline__ void simple_bwd_am_body(
     const float *__restrict__ dmat, const float *__restrict__ gpx,
     const float *__restrict__ gpy, const float *__restrict__ row_x,
     void *__restrict__ am_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
-    int ldd, int term, int rnnt_type, int part_shift, int out_type) {
+    int ldd, int term, int rnnt_type, int part_shift, int out_type, const SmoothTerms &smooth) {
   using Shape = ProdShape<kM, kC>;
   using namespace dgemm;
   extern __shared__ __align__(16) char prod_lds[];
-  __shared__ float frame_mx[kM], frame_y[kM];
+  __shared__ float frame_mx[kM], frame_y[kM], frame_w[kSmooth ? kM : 1];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
   const int c_tiles = (C + kC - 1) / kC, t_tiles = (T + kM - 1) / kM;
@@ -799,6 +804,11 @@ __device__ __forceinline__ void simple_bwd_am_body(
       const int t = t_tile + tid;
       const float mx = get_float(buffer_of(am_max + (long)b * T, T * 4), t < t_lim, 4 * t);
       frame_mx[tid] = mx;
+      if (kSmooth) {
+        const float g = get_float(buffer_of(smooth.am_g + (long)b * T, T * 4), t < t_lim, 4 * t);
+        const float z = get_float(buffer_of(smooth.am_z + (long)b * T, T * 4), t < t_lim, 4 * t);
+        frame_w[tid] = t < t_lim ? -smooth.am_scale * g / z : 0.f;
+      }
     }
     const int m_tiles = min(Shape::kMTiles, (t_lim - t_tile - kM / 2 * wave_m + 31) / 32);  // (may be <= 0)
     auto consume = [&](int k0) {
@@ -862,7 +872,8 @@ __device__ __forceinline__ void simple_bwd_am_body(
       for (int w = 0; w < Shape::kMColumns; ++w) part[wave * kM + lane + 64 * w] = sum[w];
       lds_barrier();
       if (tid < kM)
-        frame_y[tid] = (part[tid] + part[kM + tid]) + (part[2 * kM + tid] + part[3 * kM + tid]);
+        frame_y[tid] = ((part[tid] + part[kM + tid]) + (part[2 * kM + tid] + part[3 * kM + tid])) *
+                       (kSmooth ? smooth.symbol_scale : 1.f);
       lds_barrier();
     }
     constexpr int kHotPitch = kM + 4;
@@ -884,7 +895,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
           value[j] = row < listed ? hot[row * kHotPitch + kM / 2 * wave_m + 32 * j + r32] : 0.f;
 #pragma unroll
         for (int n = 0; n < Shape::kCTiles; ++n) {
-          const float one = sym == c0 + 32 * n ? 1.f : 0.f;
+          const float one = sym == c0 + 32 * n ? (kSmooth ? smooth.symbol_scale : 1.f) : 0.f;
           if (!__any(one != 0.f)) continue;
 #pragma unroll
           for (int j = 0; j < Shape::kMTiles; ++j)
@@ -893,6 +904,11 @@ __device__ __forceinline__ void simple_bwd_am_body(
       }
       lds_barrier();  // ... and have been read
     };
+    float unigram[Shape::kCTiles];
+    if (kSmooth)
+#pragma unroll
+      for (int n = 0; n < Shape::kCTiles; ++n)
+        unigram[n] = get_float(buffer_of(smooth.unigram, C * 4), c0 + 32 * n < C, 4 * (c0 + 32 * n));
     auto finish_dense = [&]() {
 #pragma unroll
       for (int j = 0; j < Shape::kMTiles; ++j)
@@ -901,6 +917,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
             const int m = row_of(j, v);
+            if (kSmooth) acc[j][n][v] += frame_w[m] * unigram[n];
             acc[j][n][v] *= __expf(in[j][n][v] - frame_mx[m]);
             if (c0 + 32 * n == term)
               acc[j][n][v] += frame_y[m];
@@ -990,7 +1007,7 @@ void launch_fwd_gemm(const double *lm, const double *am, const int64_t *symbols,
 // their workgroups share the chip.  lm_blocks is a multiple of 8, so a workgroup's XCD is the same
 // in both numberings.  (One after the other they take as long at the large sizes and 5 to 10 us
 // longer where either leaves the chip partly idle.)
-template <int kMl, int kMa>
+template <int kMl, int kMa, bool kSmooth>
 __global__ void __launch_bounds__(kProdThreads, kProdPerCu)
     simple_bwd_am_lm_kernel(const float *__restrict__ lm, const float *__restrict__ am,
                             const int64_t *__restrict__ symbols,
@@ -1001,33 +1018,33 @@ __global__ void __launch_bounds__(kProdThreads, kProdPerCu)
                             const float *__restrict__ row_y, void *__restrict__ lm_grad,
                             void *__restrict__ am_grad, const int64_t *__restrict__ window, int B,
                             int S, int T, int C, int ldd, int term, int rnnt_type,
-                            int lm_blocks, int part_shift, int out_type) {
+                            int lm_blocks, int part_shift, int out_type, SmoothTerms smooth) {
   if ((int)blockIdx.x < lm_blocks)
-    simple_bwd_lm_body<kMl, kProdC>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
+    simple_bwd_lm_body<kMl, kProdC, kSmooth>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
                                     row_y, lm_grad, window, B, S, T, C, ldd, term, part_shift,
                                     out_type);
   else
-    simple_bwd_am_body<kMa, kProdC>((int)blockIdx.x - lm_blocks, lm, am, symbols, boundary, lm_max,
+    simple_bwd_am_body<kMa, kProdC, kSmooth>((int)blockIdx.x - lm_blocks, lm, am, symbols, boundary, lm_max,
                                     am_max, dmat, gpx, gpy, row_x, am_grad, window, B, S, T, C,
-                                    ldd, term, rnnt_type, part_shift, out_type);
+                                    ldd, term, rnnt_type, part_shift, out_type, smooth);
 }
-template <int kMl, int kMa>
+template <int kMl, int kMa, bool kSmooth>
 void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
                   const int64_t *boundary, const float *lm_max, const float *am_max,
                   const float *dmat, const float *gpx, const float *gpy, const float *row_x,
                   const float *row_y, void *lm_grad, void *am_grad, const int64_t *window, int B,
                   int S, int T, int C, int ldd, int term, int rnnt_type, int out_type,
-                  hipStream_t stream) {
+                  const SmoothTerms &smooth, hipStream_t stream) {
   constexpr size_t lds = ProdShape<(kMl > kMa ? kMl : kMa), kProdC>::kLdsBytes;
   const int c_tiles = (C + kProdC - 1) / kProdC, shift = part_shift_for(B, c_tiles);
   const unsigned am_blocks =
       am_grad && T > 0 ? placed_grid(c_tiles, (T + kMa - 1) / kMa, B, shift) : 0;
   const unsigned lm_blocks = lm_grad ? placed_grid(c_tiles, (S + kMl) / kMl, B, shift) : 0;
   if (am_blocks + lm_blocks == 0) return;
-  hipLaunchKernelGGL((simple_bwd_am_lm_kernel<kMl, kMa>), dim3(am_blocks + lm_blocks),
+  hipLaunchKernelGGL((simple_bwd_am_lm_kernel<kMl, kMa, kSmooth>), dim3(am_blocks + lm_blocks),
                      dim3(kProdThreads), lds, stream, lm, am, symbols, boundary, lm_max, am_max,
                      dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad, window, B, S, T, C, ldd,
-                     term, rnnt_type, (int)lm_blocks, shift, out_type);
+                     term, rnnt_type, (int)lm_blocks, shift, out_type, smooth);
 }
 // Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand along
 // the vocabulary half as
@@ -1039,24 +1056,40 @@ bool wide_tile(long columns_of_tiles, int rows) {
   const long wide = (rows + 127) / 128, narrow = (rows + 63) / 64;
   return narrow > 1 && 14 * wide <= 8 * narrow && columns_of_tiles * wide >= kMinWideTiles;
 }
+template <bool kSmooth>
+void launch_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
+                    const int64_t *boundary, const float *lm_max, const float *am_max,
+                    const float *dmat, const float *gpx, const float *gpy, const float *row_x,
+                    const float *row_y, void *lm_grad, void *am_grad, const int64_t *window, int B,
+                    int S, int T, int C, int ldd, int term, int rnnt_type, int out_type,
+                    const SmoothTerms &smooth, hipStream_t stream) {
+  const long columns = (long)B * ((C + kProdC - 1) / kProdC);
+  const bool wide_l = wide_tile(columns, S + 1), wide_a = wide_tile(columns, T);
+  auto launch = wide_l ? wide_a ? launch_bwd_t<128, 128, kSmooth> : launch_bwd_t<128, 64, kSmooth>
+                       : wide_a ? launch_bwd_t<64, 128, kSmooth> : launch_bwd_t<64, 64, kSmooth>;
+  launch(lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad,
+         window, B, S, T, C, ldd, term, rnnt_type, out_type, smooth, stream);
+}
 void launch_bwd(const float *lm, const float *am, const int64_t *symbols, const int64_t *boundary,
                 const float *lm_max, const float *am_max, const float *dmat, const float *gpx,
                 const float *gpy, const float *row_x, const float *row_y, const float *, void *lm_grad,
                 void *am_grad, const int64_t *window, int B, int S, int T, int C, int ldd, int term,
-                int rnnt_type, int out_type, hipStream_t stream) {
-  const long columns = (long)B * ((C + kProdC - 1) / kProdC);
-  const bool wide_l = wide_tile(columns, S + 1), wide_a = wide_tile(columns, T);
-  auto launch = wide_l ? wide_a ? launch_bwd_t<128, 128> : launch_bwd_t<128, 64>
-                       : wide_a ? launch_bwd_t<64, 128> : launch_bwd_t<64, 64>;
-  launch(lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad,
-         window, B, S, T, C, ldd, term, rnnt_type, out_type, stream);
+                int rnnt_type, int out_type, const SmoothTerms *smooth, hipStream_t stream) {
+  if (smooth)
+    launch_bwd_f32<true>(lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, gpy, row_x, row_y,
+                         lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type,
+                         *smooth, stream);
+  else
+    launch_bwd_f32<false>(lm, am, symbols, boundary, lm_max, am_max, dmat, gpx, gpy, row_x, row_y,
+                          lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type, {},
+                          stream);
 }
 void launch_bwd(const double *lm, const double *am, const int64_t *symbols,
                 const int64_t *boundary, const double *lm_max, const double *am_max,
                 const double *dmat, const double *gpx, const double *, const double *row_x,
                 const double *row_y, const double *col_y, void *lm_grad_, void *am_grad_,
                 const int64_t *, int B, int S, int T, int C, int ldd, int term, int rnnt_type, int,
-                hipStream_t stream) {
+                const SmoothTerms *, hipStream_t stream) {
   double *lm_grad = static_cast<double *>(lm_grad_), *am_grad = static_cast<double *>(am_grad_);
   const unsigned c_tiles = (C + kTileN - 1) / kTileN;
   if (lm_grad)
@@ -1128,7 +1161,8 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
              const R *lm_max, const R *am_max, const R *norm_raw, const R *score_grad,
              int score_grad_stride, double score_grad_scale, R *px_grad, R *py_grad, R *dmat,
              R *row_x, R *row_y, R *col_y, void *lm_grad, void *am_grad, int B, int S, int T, int C,
-             int term, int rnnt_type, int window_only, int out_type, void *stream_) {
+             int term, int rnnt_type, int window_only, int out_type, void *stream_,
+             const SmoothTerms *smooth = nullptr) {
   constexpr bool is_float = std::is_same<R, float>::value;
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_bwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2 || term < 0 || term >= C)
@@ -1161,9 +1195,10 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
                            (is_float ? 0 : (long)B * ((T + kWave - 1) / kWave));
   hipLaunchKernelGGL(simple_bwd_prep_kernel<R>, dim3((unsigned)prep_blocks), dim3(256), 0, stream,
                      px_grad, py_grad, norm_raw, boundary, window, score_grad, score_grad_stride,
-                     (R)score_grad_scale, dmat, row_x, row_y, col_y, B, S, T, ldd, rnnt_type);
+                     (R)score_grad_scale, smooth ? (R)smooth->joint : (R)1, dmat, row_x, row_y, col_y, B,
+                     S, T, ldd, rnnt_type);
   launch_bwd(lm, am, symbols, boundary, lm_max, am_max, dmat, px_grad, py_grad, row_x, row_y, col_y,
-             lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type, stream);
+             lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type, smooth, stream);
   return check_launch("simple_logprobs_bwd");
 }
 
@@ -1260,6 +1295,18 @@ int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbo
                         void *stream) {
   return fwd_impl<double>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
                           delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
+}
+int simple_logprobs_bwd_smoothed(const float *lm, const float *am, const int64_t *symbols,
+                                 const int64_t *boundary, const float *lm_max, const float *am_max,
+                                 const float *norm_raw, const float *score_grad,
+                                 int score_grad_stride, double score_grad_scale, float *px_grad,
+                                 float *py_grad, float *dmat, float *row_x, float *row_y,
+                                 const SmoothTerms &smooth, float *lm_grad, float *am_grad, int B,
+                                 int S, int T, int C, int term, int rnnt_type, void *stream) {
+  return bwd_impl<float>(lm, am, symbols, boundary, lm_max, am_max, norm_raw, score_grad,
+                         score_grad_stride, score_grad_scale, px_grad, py_grad, dmat, row_x, row_y,
+                         nullptr, lm_grad, am_grad, B, S, T, C, term, rnnt_type, boundary != nullptr,
+                         FRNNT_F32, stream, &smooth);
 }
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
                   long n_lm, long n_am, hipStream_t stream) {

@@ -128,6 +128,24 @@ int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbo
                         const int64_t *boundary, double *px, double *py, double *lm_max,
                         double *am_max, double *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream);
+// What the smoothed loss adds to the gradient products (smoothed_logprobs.hip): lm_grad already holds
+// its own part of lm's gradient, and
+//   am.grad[t,c] -= exp(am[t,c] - max[t]) * am_scale * am_g[t] / am_z[t] * unigram[c],
+// the per-symbol and termination terms of am are taken times symbol_scale, and everything that
+// belongs to the joint model times `joint`.
+struct SmoothTerms {
+  const float *am_g, *am_z, *unigram;
+  float am_scale, symbol_scale, joint;
+};
+// The backward of the joint model within the smoothed loss: simple_logprobs_bwd with these terms.
+// px_grad and py_grad are scaled in place by score_grad (may be NULL).
+int simple_logprobs_bwd_smoothed(const float *lm, const float *am, const int64_t *symbols,
+                                 const int64_t *boundary, const float *lm_max, const float *am_max,
+                                 const float *norm_raw, const float *score_grad,
+                                 int score_grad_stride, double score_grad_scale, float *px_grad,
+                                 float *py_grad, float *dmat, float *row_x, float *row_y,
+                                 const SmoothTerms &smooth, float *lm_grad, float *am_grad, int B,
+                                 int S, int T, int C, int term, int rnnt_type, void *stream);
 // 2-byte lm and am (`dtype`: FRNNT_F16 or FRNNT_BF16) as float32, in one launch.
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
                   long n_lm, long n_am, hipStream_t stream);

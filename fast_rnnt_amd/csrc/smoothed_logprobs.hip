@@ -21,7 +21,7 @@
 //           - a sum_{b,t} G[b,t] exp(am[b,t,c] - max) / Z[b,t]
 // with rx / ry the row sums of the incoming px / py gradients, cy / G the column sums of
 // gy / gx + gy, q = exp(am - max) U / Z the am-only posterior and Z = exp(An - max).
-#include "common.hip.h"
+#include "simple_shared.hip.h"
 
 namespace frnnt {
 namespace {
@@ -186,7 +186,8 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// one thread per px / py element, t fastest
+// one thread per px / py element, t fastest.  delay, ends: the delay penalty and the boundary rows
+// that it is counted from (the fused loss; rnnt_loss.py:1470-1479)
 template <typename R>
 __global__ void __launch_bounds__(256)
     smoothed_combine_kernel(const R *__restrict__ lm, const R *__restrict__ am,
@@ -196,7 +197,8 @@ __global__ void __launch_bounds__(256)
                             const R *__restrict__ lm_sum, const R *__restrict__ am_max,
                             const R *__restrict__ am_z, const R *__restrict__ unigram,
                             R *__restrict__ px, R *__restrict__ py, int B, int S, int T, int C,
-                            int term, int regular, R k_joint, R k_lm, R k_am) {
+                            int term, int regular, R k_joint, R k_lm, R k_am, Delay<R> delay,
+                            const int64_t *__restrict__ ends) {
   const int T1 = regular ? T + 1 : T;
   const int S1 = S + 1;
   const long n_px = (long)B * S * T1, n_py = (long)B * S1 * T;
@@ -221,7 +223,7 @@ __global__ void __launch_bounds__(256)
     // nothing can be emitted after an utterance's last frame (fix_for_boundary,
     // rnnt_loss.py:45-63, applied by the reference after the interpolation)
     if (boundary && regular && boundary[4 * b + 3] == t) v = Num<R>::neg_inf();
-    px[idx] = v;
+    px[idx] = delay.at(v, ends, b, t, T);
   } else if (idx < n_px + n_py) {
     const long j = idx - n_px;
     const int t = (int)(j % T);
@@ -258,7 +260,8 @@ __global__ void __launch_bounds__(256)
                                  const R *__restrict__ lm_sum, const R *__restrict__ am_max,
                                  const R *__restrict__ am_z, const R *__restrict__ unigram,
                                  R *__restrict__ px, R *__restrict__ py, int S, int T, int C,
-                                 int term, int regular, R k_joint, R k_lm, R k_am) {
+                                 int term, int regular, R k_joint, R k_lm, R k_am, Delay<R> delay,
+                                 const int64_t *__restrict__ ends) {
   extern __shared__ __align__(16) unsigned char combine_lds[];
   const int S1 = S + 1, T1 = regular ? T + 1 : T, pitch = S1 | 1;
   R *am_s = reinterpret_cast<R *>(combine_lds);  // [32][pitch]: am[t][sym[s]], column S: am[t][term]
@@ -310,7 +313,7 @@ __global__ void __launch_bounds__(256)
     // nothing can be emitted after an utterance's last frame (fix_for_boundary,
     // rnnt_loss.py:45-63, applied by the reference after the interpolation)
     if (t == t_mask) v = ninf;
-    pxb[(long)s * T1 + t] = v;
+    pxb[(long)s * T1 + t] = delay.at(v, ends, b, t, T);
   }
   const R *pyjb = pyj + (long)b * S1 * T;
   R *pyb = py + (long)b * S1 * T;
@@ -326,18 +329,20 @@ __global__ void __launch_bounds__(256)
 
 // Row sums rx, ry (one wave per lattice row; rx over all T1 columns) and column sums
 // cy = sum_s gy, G = sum_s (gx + gy) over the frames (64 frames per block, waves split
-// the rows); also the gradients of the joint inputs, k * (gx, gy).
+// the rows, eight of a wave's requested together); also the gradients of the joint inputs,
+// k * (gx, gy), where gxj and gyj are given.
 // t_masks (optional): per utterance the frame whose px the forward kernel set to -inf for
 // the regular lattice; like the reference's scatter_ there (rnnt_loss.py:45-63) that cuts
 // the gradient, whatever the recursion left in px_grad at those cells (1 when no path
-// exists at all, 0 otherwise).
+// exists at all, 0 otherwise).  score_grad (optional): gpx and gpy are taken times
+// scale * score_grad[b * stride].
 template <typename R>
 __global__ void __launch_bounds__(256)
     smoothed_bwd_sums_kernel(const R *__restrict__ gpx, const R *__restrict__ gpy,
-                             const int64_t *__restrict__ boundary,
-                             R *__restrict__ gxj, R *__restrict__ gyj, R *__restrict__ row_x,
-                             R *__restrict__ row_y, R *__restrict__ col_y, R *__restrict__ col_g,
-                             int B, int S, int T, int T1, R k_joint) {
+                             const int64_t *__restrict__ boundary, const R *__restrict__ score_grad,
+                             int stride, R scale, R *__restrict__ gxj, R *__restrict__ gyj,
+                             R *__restrict__ row_x, R *__restrict__ row_y, R *__restrict__ col_y,
+                             R *__restrict__ col_g, int B, int S, int T, int T1, R k_joint) {
   __shared__ R part[2][4][kWave];
   const int S1 = S + 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -348,19 +353,20 @@ __global__ void __launch_bounds__(256)
     if (row >= n_rows) return;
     const int b = (int)(row / S1), s = (int)(row % S1);
     const int t_mask = boundary ? (int)boundary[4 * b + 3] : -1;
+    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
     R sx = 0, sy = 0;
     if (s < S) {
       const long o = ((long)b * S + s) * T1;
       for (int t = lane; t < T1; t += kWave) {
-        const R v = t == t_mask ? (R)0 : gpx[o + t];
-        gxj[o + t] = v * k_joint;
+        const R v = t == t_mask ? (R)0 : gpx[o + t] * g;
+        if (gxj) gxj[o + t] = v * k_joint;
         sx += v;
       }
     }
     const long o = row * T;
     for (int t = lane; t < T; t += kWave) {
-      const R v = gpy[o + t];
-      gyj[o + t] = v * k_joint;
+      const R v = gpy[o + t] * g;
+      if (gyj) gyj[o + t] = v * k_joint;
       sy += v;
     }
     sx = wave_total(sx);
@@ -375,11 +381,22 @@ __global__ void __launch_bounds__(256)
     const int b = (int)(cb / tiles), t = (int)(cb % tiles) * kWave + lane;
     const bool ok = t < T;
     const bool masked = boundary && boundary[4 * b + 3] == t;
+    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
     R ax = 0, ay = 0;
-    for (int s = wave; s < S1; s += 4) {
-      if (ok) {
-        ay += gpy[((long)b * S1 + s) * T + t];
-        if (s < S && !masked) ax += gpx[((long)b * S + s) * T1 + t];
+    constexpr int kAhead = 8;
+    for (int s0 = wave; s0 < S1; s0 += 4 * kAhead) {
+      R x[kAhead], y[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int s = s0 + 4 * u, tc = ok ? t : 0;
+        y[u] = gpy[((long)b * S1 + min(s, S)) * T + tc];
+        x[u] = S > 0 ? gpx[((long)b * S + min(s, S - 1)) * T1 + tc] : (R)0;
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int s = s0 + 4 * u;
+        if (s < S1) ay += y[u] * g;
+        if (s < S && !masked) ax += x[u] * g;
       }
     }
     part[0][wave][lane] = ax;
@@ -611,7 +628,7 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
              const R *pxj, const R *pyj, R *px,
              R *py, R *lm_max, R *lm_sum, R *am_max, R *am_z, R *unigram, R *partial, int B, int S,
              int T, int C, int term, int regular, double lm_only_scale, double am_only_scale,
-             void *stream_) {
+             void *stream_, double delay_penalty = 0.0, const int64_t *ends = nullptr) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "smoothed_logprobs_fwd: bad size");
   if (term < 0 || term >= C)
     return fail(FRNNT_EINVAL, "smoothed_logprobs_fwd: termination symbol outside [0, C)");
@@ -644,11 +661,12 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
                        dim3((unsigned)((T1 + kCombineFrames - 1) / kCombineFrames), (unsigned)B),
                        dim3(256), tile_lds, stream, lm, am, symbols, boundary, pxj, pyj, lm_max,
                        lm_sum, am_max, am_z, unigram, px, py, S, T, C, term, regular, k_joint, k_lm,
-                       k_am);
+                       k_am, Delay<R>{(R)delay_penalty}, ends);
   else if (total > 0)
     hipLaunchKernelGGL(smoothed_combine_kernel<R>, dim3((unsigned)((total + 255) / 256)),
                        dim3(256), 0, stream, lm, am, symbols, boundary, pxj, pyj, lm_max, lm_sum, am_max,
-                       am_z, unigram, px, py, B, S, T, C, term, regular, k_joint, k_lm, k_am);
+                       am_z, unigram, px, py, B, S, T, C, term, regular, k_joint, k_lm, k_am,
+                       Delay<R>{(R)delay_penalty}, ends);
   return check_launch("smoothed_logprobs_fwd");
 }
 
@@ -675,8 +693,8 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   const int64_t *t_masks = regular ? boundary : nullptr;
   const long sums_blocks = (n_lm + 3) / 4 + (long)B * ((T + kWave - 1) / kWave);
   hipLaunchKernelGGL(smoothed_bwd_sums_kernel<R>, dim3((unsigned)sums_blocks), dim3(256), 0, stream,
-                     px_grad, py_grad, t_masks, pxj_grad, pyj_grad, row_x, row_y, col_y, col_g, B, S,
-                     T, T1, k_joint);
+                     px_grad, py_grad, t_masks, (const R *)nullptr, 0, (R)1, pxj_grad, pyj_grad, row_x,
+                     row_y, col_y, col_g, B, S, T, T1, k_joint);
   const int blocks = (int)((n_am + kRowsPerBlock - 1) / kRowsPerBlock);
   if (n_am > 0)
     hipLaunchKernelGGL(weighted_column_partial_kernel<R>, dim3(blocks), dim3(256), 0, stream, am,
@@ -705,6 +723,28 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
     }
   }
   return check_launch("smoothed_logprobs_bwd");
+}
+
+// ---- the whole loss in float32 -----------------------------------------------------------------
+// What its backward keeps: [S1 rows of lm] max (joint), max, sum; [T frames of am] max (joint), max,
+// z; unigram; the joint normalizers.
+struct Kept {
+  float *lm_max, *s_lm_max, *lm_sum, *am_max, *s_am_max, *am_z, *unigram, *norm_raw;
+  size_t floats;
+};
+Kept keep_of(float *base, long B, long S, long T, long C) {
+  size_t at = 0;
+  auto take = [&](size_t n) {
+    float *p = base + at;
+    at += (n + 3) & ~(size_t)3;
+    return p;
+  };
+  Kept k;
+  k.lm_max = take(B * (S + 1)), k.s_lm_max = take(B * (S + 1)), k.lm_sum = take(B * (S + 1));
+  k.am_max = take(B * T), k.s_am_max = take(B * T), k.am_z = take(B * T);
+  k.unigram = take(C), k.norm_raw = take(B * (S + 1) * T);
+  k.floats = at;
+  return k;
 }
 
 }  // namespace
@@ -762,6 +802,88 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
                                  py_grad, px_joint_grad, py_joint_grad, lm_grad, am_grad, row_x,
                                  row_y, col_y, col_g, g_unigram, partial, B, S, T, C,
                                  termination_symbol, regular, lm_only_scale, am_only_scale, stream);
+}
+
+int64_t frnnt_smoothed_loss_kept(int B, int S, int T, int C) {
+  return (int64_t)frnnt::keep_of(nullptr, B, S, T, C).floats;
+}
+int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t *symbols,
+                                const int64_t *boundary, float *px_joint, float *py_joint,
+                                float *px, float *py, float *kept, float *partial, float *p,
+                                float *scores, float *px_grad, float *py_grad, float *loss, int B,
+                                int S, int T, int C, int termination_symbol, int rnnt_type,
+                                double lm_only_scale, double am_only_scale, double delay_penalty,
+                                int reduction, int checks, int32_t *status, void *stream) {
+  using namespace frnnt;
+  if (rnnt_type != kRegular && rnnt_type != kModified)
+    return fail(FRNNT_EINVAL, "smoothed_loss_fwd: rnnt_type must be 0 or 1");
+  if (B > 0 && !kept) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: null pointer");
+  const int regular = rnnt_type == kRegular;
+  const Kept k = keep_of(kept, B, S, T, C);
+  int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px_joint, py_joint, k.lm_max, k.am_max,
+                               k.norm_raw, 0.0, B, S, T, C, termination_symbol, rnnt_type,
+                               boundary != nullptr, stream);
+  if (rc != FRNNT_OK) return rc;
+  rc = fwd_impl<float>(lm, am, symbols, boundary, px_joint, py_joint, px, py, k.s_lm_max, k.lm_sum,
+                       k.s_am_max, k.am_z, k.unigram, partial, B, S, T, C, termination_symbol,
+                       regular, lm_only_scale, am_only_scale, stream,
+                       delay_penalty > 0.0 ? delay_penalty : 0.0, boundary);
+  if (rc != FRNNT_OK) return rc;
+  return frnnt_mi_loss_fwd_f32(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, !regular,
+                               reduction, checks, status, stream);
+}
+int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
+                                const int64_t *boundary, const float *kept, const float *score_grad,
+                                int score_grad_stride, double score_grad_scale, float *px_grad,
+                                float *py_grad, float *scratch, float *lm_grad, float *am_grad,
+                                int B, int S, int T, int C, int termination_symbol, int rnnt_type,
+                                double lm_only_scale, double am_only_scale, void *stream_) {
+  using namespace frnnt;
+  if (B < 0 || S < 0 || T < 0 || C < 1 || termination_symbol < 0 || termination_symbol >= C ||
+      (rnnt_type != kRegular && rnnt_type != kModified) ||
+      (score_grad_stride != 0 && score_grad_stride != 1))
+    return fail(FRNNT_EINVAL, "smoothed_loss_bwd: bad size or type");
+  if (B == 0) return FRNNT_OK;
+  if (!lm || !am || (!symbols && S > 0) || !kept || !score_grad || !px_grad || !py_grad || !scratch ||
+      !lm_grad || !am_grad)
+    return fail(FRNNT_EINVAL, "smoothed_loss_bwd: null pointer");
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const Kept k = keep_of(const_cast<float *>(kept), B, S, T, C);
+  const bool regular = rnnt_type == kRegular;
+  const int T1 = regular ? T + 1 : T;
+  const long n_lm = (long)B * (S + 1), n_am = (long)B * T;
+  const float k_lm = (float)lm_only_scale, k_am = (float)am_only_scale;
+  const float k_joint = (float)(1.0 - lm_only_scale - am_only_scale);
+  // scratch: the sums of the unscaled gradients first, the joint model's buffers after them
+  size_t at = 0;
+  auto take = [&](size_t n) {
+    float *q = scratch + at;
+    at += (n + 3) & ~(size_t)3;
+    return q;
+  };
+  float *row_x = take(n_lm), *row_y = take(n_lm), *col_y = take(n_am), *col_g = take(n_am);
+  float *g_unigram = take(C), *partial = take((n_am + 15) / 16 * C);
+  float *dmat = take(n_lm * ((T + 3) & ~3)), *joint_x = take(n_lm), *joint_y = take(n_lm);
+  hipLaunchKernelGGL(smoothed_bwd_sums_kernel<float>,
+                     dim3((unsigned)((n_lm + 3) / 4 + (long)B * ((T + kWave - 1) / kWave))), dim3(256), 0,
+                     stream, px_grad, py_grad, regular ? boundary : nullptr, score_grad,
+                     score_grad_stride, (float)score_grad_scale, nullptr, nullptr, row_x, row_y,
+                     col_y, col_g, B, S, T, T1, k_joint);
+  const int blocks = (int)((n_am + kRowsPerBlock - 1) / kRowsPerBlock);
+  if (n_am > 0)
+    hipLaunchKernelGGL(weighted_column_partial_kernel<float>, dim3(blocks), dim3(256), 0, stream, am,
+                       k.s_am_max, col_g, k.am_z, partial, n_am, C);
+  hipLaunchKernelGGL(unigram_grad_kernel<float>, dim3((C + kColsPerBlock - 1) / kColsPerBlock),
+                     dim3(kUnigramThreads), 0, stream, partial, symbols, row_x, row_y, k.unigram,
+                     g_unigram, n_am > 0 ? blocks : 0, B, S, C, termination_symbol, k_am);
+  hipLaunchKernelGGL(smoothed_bwd_lm_kernel<float>, dim3((unsigned)((n_lm + 3) / 4)), dim3(256), 0,
+                     stream, lm, symbols, k.s_lm_max, k.lm_sum, row_x, row_y, g_unigram, lm_grad, n_lm,
+                     S, C, termination_symbol, k_lm, (float)(1.0 / (double)n_lm));
+  const SmoothTerms smooth{col_g, k.am_z, k.unigram, k_am, k_joint + k_am, k_joint};
+  return simple_logprobs_bwd_smoothed(lm, am, symbols, boundary, k.lm_max, k.am_max, k.norm_raw,
+                                      score_grad, score_grad_stride, score_grad_scale, px_grad,
+                                      py_grad, dmat, joint_x, joint_y, smooth, lm_grad, am_grad, B, S,
+                                      T, C, termination_symbol, rnnt_type, stream_);
 }
 
 }  // extern "C"

@@ -597,13 +597,8 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
   }
 };
 
-LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols,
-                       const std::optional<Tensor> &boundary_, int64_t termination_symbol,
-                       int64_t rnnt_type, double delay_penalty, bool return_grad,
-                       int64_t reduction, int64_t checks) {
-  const Tensor boundary = or_undefined(boundary_);
-  if (am.scalar_type() != at::kHalf && am.scalar_type() != at::kBFloat16) require_float_gpu(am, "am");
-  TORCH_CHECK(am.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): am");
+void check_additive(const Tensor &lm, const Tensor &am, const Tensor &symbols,
+                    const Tensor &boundary) {
   TORCH_CHECK(lm.dim() == 3 && am.dim() == 3 && symbols.dim() == 2,
               "lm and am must be 3-dimensional, symbols 2-dimensional");
   const int64_t B = am.size(0), S = lm.size(1) - 1;
@@ -620,6 +615,16 @@ LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols
     TORCH_CHECK(boundary.dim() == 2 && boundary.size(0) == B && boundary.size(1) == 4 &&
                     boundary.scalar_type() == at::kLong && boundary.device() == am.device(),
                 "boundary must be an int64 [B][4] tensor on the same device");
+}
+
+LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols,
+                       const std::optional<Tensor> &boundary_, int64_t termination_symbol,
+                       int64_t rnnt_type, double delay_penalty, bool return_grad,
+                       int64_t reduction, int64_t checks) {
+  const Tensor boundary = or_undefined(boundary_);
+  if (am.scalar_type() != at::kHalf && am.scalar_type() != at::kBFloat16) require_float_gpu(am, "am");
+  TORCH_CHECK(am.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): am");
+  check_additive(lm, am, symbols, boundary);
   TORCH_CHECK(rnnt_type >= 0 && rnnt_type <= 2, "rnnt_type must be 0, 1 or 2");
   TORCH_CHECK(reduction >= 0 && reduction <= 2, "reduction must be 0 (none), 1 (mean) or 2 (sum)");
   const bool grad_mode = at::GradMode::is_enabled();
@@ -627,6 +632,102 @@ LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols
   return as_result(SimpleLossFn::apply(lm, am, symbols, boundary_, termination_symbol, rnnt_type,
                                        delay_penalty, return_grad, reduction, checks, need_lm,
                                        need_am));
+}
+
+// ---- rnnt_loss_smoothed behind one autograd node (float32; regular and modified lattices) -----
+// forward = frnnt_smoothed_loss_fwd, backward = frnnt_smoothed_loss_bwd: the joint model's node
+// above with the lm-only and am-only models' terms folded into its kernels.
+struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &am_,
+                               const Tensor &symbols, const std::optional<Tensor> &boundary_,
+                               int64_t term, int64_t kind, double lm_scale, double am_scale,
+                               double delay_penalty, bool want_grads, int64_t reduction,
+                               int64_t checks, bool need_grad) {
+    const Tensor boundary = or_undefined(boundary_);
+    const Tensor lm = lm_.contiguous(), am = am_.contiguous(), sym = symbols.contiguous();
+    const Tensor bnd = boundary.defined() ? boundary.contiguous() : Tensor();
+    const int64_t B = am.size(0), T = am.size(1), C = am.size(2), S = lm.size(1) - 1;
+    const int64_t T1 = kind == 0 ? T + 1 : T;
+    ctx->set_materialize_grads(false);
+    DeviceGuard guard(am.device());
+    const auto opts = am.options();
+    Tensor kept = at::empty({frnnt_smoothed_loss_kept((int)B, (int)S, (int)T, (int)C)}, opts);
+    const int64_t n_px = B * S * T1, n_py = B * (S + 1) * T;
+    Carver carve;
+    const int64_t o_jx = carve.take(n_px), o_jy = carve.take(n_py), o_px = carve.take(n_px),
+                  o_py = carve.take(n_py), o_p = carve.take(B * (S + 1) * (T + 1)),
+                  o_sc = carve.take(B), o_part = carve.take((B * (S + 1) + 15) / 16 * C);
+    const Tensor work = at::empty({carve.total}, opts);
+    float *w = work.data_ptr<float>();
+    Tensor gx, gy;
+    if (want_grads || need_grad) {
+      gx = at::empty({B, S, T1}, opts);
+      gy = at::empty({B, S + 1, T}, opts);
+    }
+    Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
+    check_rc(frnnt_smoothed_loss_fwd_f32(
+                 ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), w + o_jx, w + o_jy, w + o_px,
+                 w + o_py, ptr<float>(kept), w + o_part, w + o_p, w + o_sc, ptr<float>(gx),
+                 ptr<float>(gy), ptr<float>(loss), (int)B, (int)S, (int)T, (int)C, (int)term,
+                 (int)kind, lm_scale, am_scale, delay_penalty, (int)reduction, (int)checks,
+                 status_for(am, bnd), stream_of(am)),
+             "frnnt_smoothed_loss_fwd");
+    if (need_grad) {
+      variable_list save{lm, am, sym, kept, gx, gy};
+      if (bnd.defined()) save.push_back(bnd);
+      ctx->save_for_backward(std::move(save));
+      ctx->saved_data["meta"] = std::vector<int64_t>{term, kind, reduction};
+      ctx->saved_data["scales"] = std::vector<double>{lm_scale, am_scale};
+    }
+    if (!gx.defined()) return {loss};
+    ctx->mark_non_differentiable({gx, gy});
+    return {loss, gx, gy};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    variable_list out(13);
+    const Tensor &g_loss = grads[0];
+    if (!g_loss.defined()) return out;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &lm = saved[0], &am = saved[1], &sym = saved[2], &kept = saved[3];
+    Tensor gx = saved[4], gy = saved[5];
+    const Tensor bnd = saved.size() > 6 ? saved[6] : Tensor();
+    const std::vector<int64_t> meta = ctx->saved_data["meta"].toIntVector();
+    const std::vector<double> scales = ctx->saved_data["scales"].toDoubleVector();
+    const int64_t reduction = meta[2];
+    const int64_t B = am.size(0), T = am.size(1), C = am.size(2), S = lm.size(1) - 1;
+    DeviceGuard guard(am.device());
+    const Tensor g = g_loss.contiguous();
+    const Tensor scratch =
+        at::empty({B * (S + 1) * (4 + (T + 3) / 4 * 4) + 2 * B * T + C + (B * T + 15) / 16 * C + 40},
+                  am.options());
+    out[0] = at::empty(lm.sizes(), lm.options());
+    out[1] = at::empty(am.sizes(), am.options());
+    check_rc(frnnt_smoothed_loss_bwd_f32(
+                 ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), ptr<float>(kept),
+                 ptr<float>(g), reduction == kRedNone ? 1 : 0,
+                 reduction == kRedMean ? -1.0 / (double)B : -1.0, ptr<float>(gx), ptr<float>(gy),
+                 ptr<float>(scratch), ptr<float>(out[0]), ptr<float>(out[1]), (int)B, (int)S, (int)T,
+                 (int)C, (int)meta[0], (int)meta[1], scales[0], scales[1], stream_of(am)),
+             "frnnt_smoothed_loss_bwd");
+    return out;
+  }
+};
+
+LossResult smoothed_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols,
+                         const std::optional<Tensor> &boundary_, int64_t termination_symbol,
+                         int64_t rnnt_type, double lm_only_scale, double am_only_scale,
+                         double delay_penalty, bool return_grad, int64_t reduction,
+                         int64_t checks) {
+  require_float_gpu(am, "am");
+  TORCH_CHECK(am.scalar_type() == at::kFloat, "smoothed_loss takes float32 tensors");
+  check_additive(lm, am, symbols, or_undefined(boundary_));
+  TORCH_CHECK(rnnt_type == 0 || rnnt_type == 1, "rnnt_type must be 0 or 1");
+  TORCH_CHECK(reduction >= 0 && reduction <= 2, "reduction must be 0 (none), 1 (mean) or 2 (sum)");
+  const bool need_grad = at::GradMode::is_enabled() && (lm.requires_grad() || am.requires_grad());
+  return as_result(SmoothedLossFn::apply(lm, am, symbols, boundary_, termination_symbol, rnnt_type,
+                                         lm_only_scale, am_only_scale, delay_penalty, return_grad,
+                                         reduction, checks, need_grad));
 }
 
 // ---- rnnt_loss and rnnt_loss_pruned behind one autograd node ------------------------------
@@ -1002,6 +1103,11 @@ TORCH_LIBRARY(fast_rnnt_amd, m) {
       "int rnnt_type, float delay_penalty, bool return_grad, int reduction, int checks) -> "
       "(Tensor, Tensor?, Tensor?)");
   m.def(
+      "smoothed_loss(Tensor lm, Tensor am, Tensor symbols, Tensor? boundary, "
+      "int termination_symbol, int rnnt_type, float lm_only_scale, float am_only_scale, "
+      "float delay_penalty, bool return_grad, int reduction, int checks) -> "
+      "(Tensor, Tensor?, Tensor?)");
+  m.def(
       "lattice_loss(Tensor logits, Tensor symbols, Tensor? ranges, Tensor? boundary, "
       "int termination_symbol, int rnnt_type, float delay_penalty, bool return_grad, "
       "int reduction, int checks) -> (Tensor, Tensor?, Tensor?)");
@@ -1015,6 +1121,7 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, CUDA, m) {
   m.impl("recursion", &recursion);
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
+  m.impl("smoothed_loss", &smoothed_loss);
   m.impl("lattice_loss", &lattice_loss);
   m.impl("prune_ranges", &prune_ranges);
   m.impl("pruning", &pruning);
@@ -1025,6 +1132,7 @@ TORCH_LIBRARY_IMPL(fast_rnnt_amd, Autograd, m) {
   m.impl("recursion", &recursion);
   m.impl("recursion_loss", &recursion_loss);
   m.impl("simple_loss", &simple_loss);
+  m.impl("smoothed_loss", &smoothed_loss);
   m.impl("lattice_loss", &lattice_loss);
   m.impl("pruning", &pruning);
 }
@@ -1045,6 +1153,10 @@ PYBIND11_MODULE(_C, m) {
         py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
         py::arg("delay_penalty"), py::arg("return_grad"), py::arg("reduction"),
         py::arg("checks") = 0);
+  m.def("smoothed_loss", &smoothed_loss, py::arg("lm"), py::arg("am"), py::arg("symbols"),
+        py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
+        py::arg("lm_only_scale"), py::arg("am_only_scale"), py::arg("delay_penalty"),
+        py::arg("return_grad"), py::arg("reduction"), py::arg("checks") = 0);
   m.def("lattice_loss", &lattice_loss, py::arg("logits"), py::arg("symbols"), py::arg("ranges"),
         py::arg("boundary"), py::arg("termination_symbol"), py::arg("rnnt_type"),
         py::arg("delay_penalty"), py::arg("return_grad"), py::arg("reduction"),

@@ -675,9 +675,8 @@ def get_rnnt_logprobs_smoothed(
                               am_only_scale, boundary, rnnt_type, False)
 
 
-def _smoothed_logprobs(lm, am, symbols, termination_symbol, lm_only_scale, am_only_scale,
-                       boundary, rnnt_type, from_loss):
-    # from_loss: the recursion that follows tests the boundary rows on the device
+def _check_smoothed(lm, am, symbols, boundary, rnnt_type, checks):
+    """The argument checks of get_rnnt_logprobs_smoothed; ``checks`` as in :func:`_check_joint`."""
     assert lm.ndim == 3, lm.ndim
     assert am.ndim == 3, am.ndim
     assert lm.shape[0] == am.shape[0], (lm.shape[0], am.shape[0])
@@ -686,9 +685,15 @@ def _smoothed_logprobs(lm, am, symbols, termination_symbol, lm_only_scale, am_on
     S = lm.shape[1] - 1
     assert symbols.shape == (B, S), symbols.shape
     assert rnnt_type in ["regular", "modified", "constrained"], rnnt_type
-    validate_st_lengths(S, T, rnnt_type == "regular", boundary,
-                        on_device=from_loss and _device_checks(rnnt_type, boundary) != 0)
+    validate_st_lengths(S, T, rnnt_type == "regular", boundary, on_device=checks != 0)
     _check_tensors([("am", am), ("lm", lm)], [("symbols", symbols), ("boundary", boundary)])
+
+
+def _smoothed_logprobs(lm, am, symbols, termination_symbol, lm_only_scale, am_only_scale,
+                       boundary, rnnt_type, from_loss):
+    # from_loss: the recursion that follows tests the boundary rows on the device
+    _check_smoothed(lm, am, symbols, boundary, rnnt_type,
+                    _device_checks(rnnt_type, boundary) if from_loss else 0)
 
     lm, am = _widen(lm, am)
     # joint part, without the boundary / constrained post-processing (applied last)
@@ -720,6 +725,23 @@ def rnnt_loss_smoothed(
     delay_penalty: float = 0.0, reduction: Optional[str] = "mean", return_grad: bool = False,
 ) -> Union[Tuple[Tensor, Tuple[Tensor, Tensor]], Tensor]:
     """rnnt_loss_simple with lm-only / am-only smoothing (rnnt_loss.py:1372-1494)."""
+    if rnnt_type != "constrained" and am.dtype in (torch.float32, *_NARROW):
+        # one autograd node of the operator module
+        checks = _device_checks(rnnt_type, boundary)
+        _check_smoothed(lm, am, symbols, boundary, rnnt_type, checks)
+        if reduction not in _REDUCTIONS:
+            # (the reference finds this out after the recursion has run: same exception)
+            raise ValueError(f"reduction should be ('none' | 'mean' | 'sum'), given {reduction}")
+        if boundary is not None:
+            _assert_boundary(boundary, am.shape[0], symbols.shape[1], am.shape[1],
+                             on_device=checks != 0)
+        lm, am = _widen(lm, am)
+        # (exact zeros would turn -inf * 0 into nan)
+        loss, px_grad, py_grad = _lib.ops().smoothed_loss(
+            lm, am, symbols, boundary, int(termination_symbol), _RNNT_TYPES[rnnt_type],
+            float(lm_only_scale) or 1.0e-20, float(am_only_scale) or 1.0e-20,
+            float(delay_penalty), bool(return_grad), _REDUCTIONS[reduction], checks)
+        return (loss, (px_grad, py_grad)) if return_grad else loss
     px, py = _smoothed_logprobs(lm, am, symbols, termination_symbol, lm_only_scale,
                                 am_only_scale, boundary, rnnt_type, True)
     return _recursion_and_reduce(px, py, boundary, rnnt_type, delay_penalty, reduction,

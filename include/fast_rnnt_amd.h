@@ -274,6 +274,35 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
                                     double am_only_scale, void *stream);
 
 /*
+ * rnnt_loss_smoothed (rnnt_loss.py:1372-1494) in float32 for the regular and the modified lattice
+ * (rnnt_type 0, 1): _fwd chains frnnt_simple_logprobs_fwd (window_only when a boundary is
+ * given), frnnt_smoothed_logprobs_fwd, the delay penalty and frnnt_mi_loss_fwd; _bwd scales px_grad
+ * and py_grad in place as frnnt_simple_logprobs_bwd does (score_grad is required) and forms the
+ * whole lm_grad and am_grad: the am-only model's terms inside the joint model's gradient
+ * product, the lm-only model's beneath it.
+ *   kept: frnnt_smoothed_loss_kept() floats, written by _fwd for _bwd
+ *   px_joint, py_joint, px, py, p, scores: as in those entry points, not needed afterwards
+ *   partial [ceil(B*(S+1)/16)][C]: scratch
+ *   scratch of _bwd: B (S+1) (4 + T rounded up to 4) + 2 B T + C + ceil(B*T/16) C floats, each
+ *     of its nine parts rounded up to 4 (40 more are enough for that)
+ */
+int64_t frnnt_smoothed_loss_kept(int B, int S, int T, int C);
+int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t *symbols,
+                                const int64_t *boundary, float *px_joint, float *py_joint,
+                                float *px, float *py, float *kept, float *partial, float *p,
+                                float *scores, float *px_grad, float *py_grad, float *loss, int B,
+                                int S, int T, int C, int termination_symbol, int rnnt_type,
+                                double lm_only_scale, double am_only_scale, double delay_penalty,
+                                int reduction, int checks, int32_t *status, void *stream);
+int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
+                                const int64_t *boundary, const float *kept,
+                                const float *score_grad, int score_grad_stride,
+                                double score_grad_scale, float *px_grad, float *py_grad,
+                                float *scratch, float *lm_grad, float *am_grad, int B, int S,
+                                int T, int C, int termination_symbol, int rnnt_type,
+                                double lm_only_scale, double am_only_scale, void *stream);
+
+/*
  * Forward pipeline of rnnt_loss_simple (rnnt_loss.py:230-340) in one call:
  * frnnt_simple_logprobs_fwd, frnnt_mi_forward, then -- when px_grad / py_grad are
  * given -- frnnt_mi_backward with a gradient of ones (what the recursion's autograd
