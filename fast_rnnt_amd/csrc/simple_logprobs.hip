@@ -237,6 +237,25 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---- backward ------------------------------------------------------------------------
+// `n` consecutive values of an array, one wave's row (its address is wave-uniform)
+template <typename R>
+struct Row {
+  R *base;
+  int n;
+  __device__ __forceinline__ Row(R *base_, int n_) : base(base_), n(n_) {}
+  __device__ __forceinline__ R get(bool there, int t) const { return there && t < n ? base[t] : (R)0; }
+  __device__ __forceinline__ void put(int t, R v) const {
+    if (t < n) base[t] = v;
+  }
+};
+template <>
+struct Row<float> {
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ Row(float *base, int n) : rs(buffer_of(base, 4 * n)) {}
+  __device__ __forceinline__ float get(bool there, int t) const { return get_float(rs, there, 4 * t); }
+  __device__ __forceinline__ void put(int t, float v) const { put_float(rs, true, 4 * t, v); }
+};
+
 // 256-thread workgroups.  The first ceil(B*(S+1)/4) of them give each wave one
 // lattice row (b, s): D[b,s,:] and the two row sums.  With `score_grad` the wave first scales
 // its row of the occupation gradients in place (scale_by_batch_kernel's work, for lattices whose
@@ -257,7 +276,8 @@ __global__ void __launch_bounds__(256)
   __shared__ R partial[4][kWave];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long n_rows = (long)B * S1;
   const long row_blocks = (n_rows + 3) / 4;
   const bool constrained = rnnt_type == kConstrained;
@@ -269,38 +289,39 @@ __global__ void __launch_bounds__(256)
     // outside the window nothing counts (the normalizers there may be undefined): D = 0
     const Limits lim = limits_of(window, b, S, T);
     const bool row_in = s >= lim.s_begin && s <= lim.s_end;
-    R *gx_row = s < S ? gpx + ((long)b * S + s) * T1 : nullptr;
-    const R *gx_prev = (constrained && s >= 1) ? gpx + ((long)b * S + s - 1) * T1 : nullptr;
-    R *gy_row = gpy + row * T;
-    const R *nr_row = norm_raw + row * T;
+    // (a float row is read and written through a buffer resource over it: no branch around a
+    // load, which would end in a wait for all of them; rows that do not exist are empty)
+    const Row<R> gx_row(gpx + ((long)b * S + min(s, S - 1)) * T1, s < S ? T1 : 0);
+    const Row<R> gx_prev(gpx + ((long)b * S + max(s - 1, 0)) * T1, constrained && s >= 1 ? T1 : 0);
+    const Row<R> gy_row(gpy + row * T, T), nr_row(const_cast<R *>(norm_raw) + row * T, T);
     R *d_row = dmat + row * ldd;
-    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
+    const bool scaled = score_grad != nullptr;
+    const R g = scaled ? scale * score_grad[(long)b * stride] : (R)1;
     R sx = 0, sy = 0;
     for (int t0 = 0; t0 < T1; t0 += 4 * kWave) {
-      R gx[4], gy[4], nr[4];
+      R gx[4], gy[4], above[4], nr[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = t0 + u * kWave + lane;
         const bool ok = t < T && row_in && t >= lim.t_begin && t < lim.t_end;
-        gx[u] = (gx_row && (score_grad ? t < T1 : ok)) ? gx_row[t] : (R)0;
-        gy[u] = (score_grad ? t < T : ok) ? gy_row[t] : (R)0;
-        if (ok && gx_prev && t != t_mask) gy[u] += gx_prev[t];
-        nr[u] = ok ? nr_row[t] : (R)0;
+        gx[u] = gx_row.get(scaled || ok, t);
+        gy[u] = gy_row.get(scaled || ok, t);
+        above[u] = constrained ? gx_prev.get(ok && t != t_mask, t) : (R)0;
+        nr[u] = nr_row.get(ok, t);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = t0 + u * kWave + lane;
         const bool ok = t < T && row_in && t >= lim.t_begin && t < lim.t_end;
-        if (score_grad) {
-          gx[u] *= g;
-          gy[u] *= g;
-          if (gx_row && t < T1) gx_row[t] = gx[u];
-          if (t < T) gy_row[t] = gy[u];
+        gy[u] += above[u];
+        gx[u] *= g;
+        gy[u] *= g;
+        if (scaled) {
+          gx_row.put(t, gx[u]);
+          gy_row.put(t, gy[u]);
         }
-        if (!ok || t == t_mask) gx[u] = (R)0;
-        if (!ok) gy[u] = (R)0;
-        gx[u] *= joint;
-        gy[u] *= joint;
+        gx[u] = ok && t != t_mask ? gx[u] * joint : (R)0;
+        gy[u] = ok ? gy[u] * joint : (R)0;
         if (t < T) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
         sx += gx[u];
         sy += gy[u];
@@ -1229,8 +1250,10 @@ int reduce_impl(const R *scores, R *loss, int B, int reduction, void *stream) {
   return check_launch("loss_reduce");
 }
 
-// 2-byte inputs as float32: eight elements per thread, in 16-byte accesses where the input is
-// aligned to them (the output always is).
+// 2-byte inputs as float32: a thread takes four groups of four elements, a workgroup's groups side by
+// side, in 8-byte loads where the input is aligned to them and 16-byte stores (the output always
+// is).  Bound by memory.
+constexpr int kWidenBlock = 4 * 4 * 256;  // elements
 template <typename IO>
 __global__ void __launch_bounds__(256)
     widen_kernel(const uint16_t *__restrict__ lm, const uint16_t *__restrict__ am,
@@ -1240,18 +1263,23 @@ __global__ void __launch_bounds__(256)
   const uint16_t *from = is_lm ? lm : am;
   float *to = is_lm ? lm_wide : am_wide;
   const long n = is_lm ? n_lm : n_am;
-  const long first = (long)(is_lm ? blockIdx.x : blockIdx.x - lm_blocks) * 2048;
-  const long at = first + 8 * threadIdx.x;
-  if ((reinterpret_cast<uintptr_t>(from) & 15) == 0 && at + 8 <= n) {
-    const uintx4 raw = *reinterpret_cast<const uintx4 *>(from + at);
-    dgemm::floatx4 v[2];
+  const long first = (long)(is_lm ? blockIdx.x : blockIdx.x - lm_blocks) * kWidenBlock;
+  const long at = first + 4 * threadIdx.x;
+  if ((reinterpret_cast<uintptr_t>(from) & 7) == 0 && first + kWidenBlock <= n) {
+    uintx2 raw[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = IO::load((uint16_t)(raw[i / 2] >> (16 * (i % 2))));
-    *reinterpret_cast<dgemm::floatx4 *>(to + at) = v[0];
-    *reinterpret_cast<dgemm::floatx4 *>(to + at + 4) = v[1];
+    for (int u = 0; u < 4; ++u) raw[u] = *reinterpret_cast<const uintx2 *>(from + at + 1024 * u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      dgemm::floatx4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = IO::load((uint16_t)(raw[u][i / 2] >> (16 * (i % 2))));
+      *reinterpret_cast<dgemm::floatx4 *>(to + at + 1024 * u) = v;
+    }
   } else {
-    for (int i = 0; i < 8; ++i)
-      if (at + i < n) to[at + i] = IO::load(from[at + i]);
+    for (int u = 0; u < 4; ++u)
+      for (int i = 0; i < 4; ++i)
+        if (at + 1024 * u + i < n) to[at + 1024 * u + i] = IO::load(from[at + 1024 * u + i]);
   }
 }
 
@@ -1310,7 +1338,8 @@ int simple_logprobs_bwd_smoothed(const float *lm, const float *am, const int64_t
 }
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
                   long n_lm, long n_am, hipStream_t stream) {
-  const unsigned lm_blocks = (unsigned)((n_lm + 2047) / 2048), am_blocks = (unsigned)((n_am + 2047) / 2048);
+  const unsigned lm_blocks = (unsigned)((n_lm + kWidenBlock - 1) / kWidenBlock);
+  const unsigned am_blocks = (unsigned)((n_am + kWidenBlock - 1) / kWidenBlock);
   if (lm_blocks + am_blocks == 0) return;
   hipLaunchKernelGGL((dtype == FRNNT_F16 ? widen_kernel<HalfIO> : widen_kernel<Bf16IO>),
                      dim3(lm_blocks + am_blocks), dim3(256), 0, stream,
