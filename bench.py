@@ -451,9 +451,9 @@ def _bench_lattice(args, w, dev):
     # gradient kernel: reads the rows inside the windows, writes every row (zeros outside);
     # normalizer kernel: reads the rows inside the windows
     lines = [
-        _hbm_line(table, "row_grad_regs_kernel" if esize == 4 else "row_grad_narrow_kernel",
+        _hbm_line(table, "row_grad_kernel",
                   in_bytes + nbytes, t_b, padded_bytes=2 * nbytes),
-        _hbm_line(table, "row_norm_regs_kernel" if esize == 4 else "row_norm_narrow_kernel",
+        _hbm_line(table, "row_norm_kernel",
                   in_bytes, t_f, padded_bytes=nbytes,
                   note="launch time includes the small assemble_kernel of the same entry point"),
     ]
@@ -583,14 +583,10 @@ def main():
         t_bwd = _event_time_ms(rec_bwd, args.kernel_reps)
         # The two gradient products (lm.grad, am.grad) through the backward entry point of
         # the logprobs: it also launches the small prep kernel, which the same call without
-        # outputs runs alone; the difference of the two event timings is the product kernel(s).
+        # outputs runs alone; the difference of the two event timings is the product kernel, which
+        # holds both products' tiles in one launch.
         t_prep = _event_time_ms(lambda: grads(False, False), args.kernel_reps)
-        one_launch = float(B) * (S + 1) * T * C < 1e9  # the library's rule for a single launch
-        if one_launch:
-            t_grads = {"both": _event_time_ms(lambda: grads(True, True), args.kernel_reps) - t_prep}
-        else:
-            t_grads = {"lm": _event_time_ms(lambda: grads(True, False), args.kernel_reps) - t_prep,
-                       "am": _event_time_ms(lambda: grads(False, True), args.kernel_reps) - t_prep}
+        t_grads = {"both": _event_time_ms(lambda: grads(True, True), args.kernel_reps) - t_prep}
     stages = {"logprobs_fwd_ms": t_logp, "mi_forward_ms": t_fwd, "mi_backward_ms": t_bwd,
               "bwd_prep_ms": t_prep}
     stages.update({"bwd_grad_%s_ms" % k: v for k, v in t_grads.items()})
@@ -602,24 +598,15 @@ def main():
     Sb, Tb = _windows(w.boundary)
     gemm_flops = 2.0 * C * ((Sb + 1) * Tb).sum().item()
     gemm_padded = 2.0 * B * (S + 1) * T * C
-    rows96 = (S + 1 + 95) // 96 * 96 < (S + 1 + 127) // 128 * 128
-    fwd_name = "simple_fwd_panel_kernel<%s>" % ("96, 16" if rows96 else "128, 16")
-    lm_shape = "96, 32" if rows96 else "128, 16"     # the lm.grad kernel on its own
-    both_shape = "96, 16" if rows96 else "128, 16"   # inside the common launch
     # each gradient product is one GEMM of the forward's size (the one-hot product that
-    # scatters px_grad into am.grad is not counted)
-    if "both" in t_grads:
-        lines = [_mfma_line(table, "simple_bwd_am_lm_kernel<%s>" % both_shape, 2 * gemm_flops,
-                            2 * gemm_padded, t_grads["both"])]
-    else:
-        lines = [_mfma_line(table, "simple_bwd_am_panel_kernel", gemm_flops, gemm_padded,
-                            t_grads["am"]),
-                 _mfma_line(table, "simple_bwd_lm_slab_kernel<%s>" % lm_shape, gemm_flops,
-                            gemm_padded, t_grads["lm"])]
+    # scatters px_grad into am.grad is not counted); it runs as six bfloat16 products of
+    # operands cut in three, and is priced here as the float32 product that it stands for
+    lines = [_mfma_line(table, "simple_bwd_am_lm_kernel", 2 * gemm_flops, 2 * gemm_padded,
+                        t_grads["both"])]
     steps_chain = int((Sb + Tb).max().item())
     lines += [
         # the same kernel finds the row maxima on the way and assembles px / py at the end
-        _mfma_line(table, fwd_name, gemm_flops, gemm_padded, t_logp),
+        _mfma_line(table, "simple_fwd_panel_kernel", gemm_flops, gemm_padded, t_logp),
         # the recursion kernels are bound by their dependent chain (S_b + T_b steps), not by
         # bytes: cycles per step at 2.4 GHz are given beside the bandwidth figure
         _hbm_line(table, "mi_forward_kernel", _recursion_bytes(w.boundary, S, T, B, False), t_fwd,

@@ -1067,12 +1067,11 @@ void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
                      dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad, window, B, S, T, C, ldd,
                      term, rnnt_type, (int)lm_blocks, shift, out_type, smooth);
 }
-// Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand along
-// the vocabulary half as
-// often as 64 (am.grad at B 16, T 400, C 5000: 92 against 97 us; lm.grad 60 against 65), which is
-// what counts once the chip is full; they lose where the padding of the last tile outweighs
-// that (up to 64 rows: 24 against 18 us at B 21, S 47, T 333, C 503) or where fewer of them than fill
-// the chip remain (B 3, S 250, T 1335, C 198: 71 against 55 us).
+// Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand
+// along the vocabulary half as often as 64 (am.grad at B 16, T 400, C 5000: 92 against 97 us;
+// lm.grad 60 against 65), which is what counts once the chip is full; they lose where the padding
+// of the last tile outweighs that (up to 64 rows: 24 against 18 us at B 21, S 47, T 333, C 503) or
+// where fewer of them than fill the chip remain (B 3, S 250, T 1335, C 198: 71 against 55 us).
 bool wide_tile(long columns_of_tiles, int rows) {
   const long wide = (rows + 127) / 128, narrow = (rows + 63) / 64;
   return narrow > 1 && 14 * wide <= 8 * narrow && columns_of_tiles * wide >= kMinWideTiles;

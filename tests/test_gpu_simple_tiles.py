@@ -1,7 +1,7 @@
-"""rnnt_loss_simple where the kernels' choice of tiles and
-their splits into chunks, can go wrong: sizes on either side of a tile of lattice rows, frames and
-vocabulary entries, sums over few and many chunks, batches small and large, 2-byte inputs, long
-lists of equal symbols.  Oracle: the CPU restatement on the same values in float32."""
+"""rnnt_loss_simple where the kernels' choice of tiles and their splits into chunks can go wrong:
+sizes on either side of a tile of lattice rows, frames and vocabulary entries, sums over few and
+many chunks, batches small and large, 2-byte inputs, long lists of equal symbols.  Oracle: the CPU
+restatement on the same values in float32."""
 import pytest
 import torch
 
