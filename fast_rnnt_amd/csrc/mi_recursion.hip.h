@@ -1287,16 +1287,32 @@ size_t lds_bytes(int nsweep, int T, int buffers, size_t elem) {
                            (size_t)buffers * (2 * kTileElems + kTileSteps)) * elem;
 }
 
+// Dynamic LDS of a workgroup that has a band to itself: one sweep wave's share, and a second seam row.
+constexpr int kApartBuffers = 3;
+size_t apart_lds_bytes(int T) {
+  return lds_bytes(1, T, kApartBuffers, sizeof(float)) +
+         (size_t)((T + 1 + kSeamSlack + 3) & ~3) * sizeof(float);
+}
+
 // Whether every band of 64 rows gets a workgroup of its own.  It costs a fixed time -- the marks, and
 // the way of a seam from one workgroup to the next -- and saves some of each of the sweep's steps;
 // both measured (microseconds, nanoseconds), for 2, 3 and 4 bands.
 // (B 12, S 220, T 1500: 134 + 164 -> 72 + 80 us; B 3, S 250, T 1335: 120 + 149 -> 67 + 74;
 // B 10, S 137, T 817: 51 + 60 -> 43 + 48.)
+// Both seam rows must fit into LDS (T up to 12 988; the other launch goes to 30 636).  Two workgroups
+// share a compute unit while their LDS allows it (T up to 3 004).  Beyond, a band that finds no unit
+// of its own starts when an earlier one is done: two bands, which one workgroup sweeps almost as fast
+// as two, then stay together (B 136, S 100, T 6000: 595 + 599 apart, 407 + 555 together; B 136, S 70,
+// T 5000: 443 + 438, 281 + 318); three and four are still better off apart (B 128, S 250, T 5000:
+// 674 + 831 apart, 763 + 1125 together; B 96, S 180, T 6000: 656 + 696, 681 + 862).
 template <typename R>
 bool bands_apart(int B, int S, int T, bool backward) {
   const int bands = (S + kWave) / kWave;
   if (sizeof(R) != 4 || bands < 2 || bands > kMaxSweep || T < 1) return false;
-  if ((long)((B + 7) / 8 * 8) * bands > 512) return false;  // two workgroups per compute unit
+  const size_t per_cu = kLdsBudget / apart_lds_bytes(T);
+  if (per_cu == 0) return false;
+  const long workgroups = (long)((B + 7) / 8 * 8) * bands;
+  if (workgroups > (bands == 2 && per_cu == 1 ? 256 : 512)) return false;
   constexpr double kCost[2][3] = {{6, 7, 10}, {11, 16, 20}}, kSaved[2][3] = {{6.7, 7, 39}, {13, 28, 60}};
   return 1e-3 * kSaved[backward][bands - 2] * (S + T) > kCost[backward][bands - 2];
 }
@@ -1335,10 +1351,9 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
                  static_cast<hipStream_t>(stream));
     if (apart) {
       const int pitch = (B + 7) / 8 * 8;  // (an utterance's bands on one XCD)
-      const size_t lds = lds_bytes(1, T, kFewBuffers, sizeof(R)) +
-                         (size_t)((T + 1 + kSeamSlack + 3) & ~3) * sizeof(R);  // (a second seam row)
-      auto kernel = modified ? mi_forward_kernel<R, true, 1, kFew, kFewBuffers, true>
-                             : mi_forward_kernel<R, false, 1, kFew, kFewBuffers, true>;
+      const size_t lds = apart_lds_bytes(T);
+      auto kernel = modified ? mi_forward_kernel<R, true, 1, kFew, kApartBuffers, true>
+                             : mi_forward_kernel<R, false, 1, kFew, kApartBuffers, true>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_forward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kFew) * kWave), lds,
@@ -1395,10 +1410,9 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
       if (!marked)
         mark_seams(boundary, nullptr, px_grad, B, S, T, modified, static_cast<hipStream_t>(stream));
       const int pitch = (B + 7) / 8 * 8;
-      const size_t lds = lds_bytes(1, T, kFewBuffers, sizeof(R)) +
-                         (size_t)((T + 1 + kSeamSlack + 3) & ~3) * sizeof(R);  // (a second seam row)
-      auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kFewBuffers, true>
-                             : mi_backward_kernel<R, false, 1, kFew, kFewBuffers, true>;
+      const size_t lds = apart_lds_bytes(T);
+      auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kApartBuffers, true>
+                             : mi_backward_kernel<R, false, 1, kFew, kApartBuffers, true>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_backward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kFew) * kWave), lds,

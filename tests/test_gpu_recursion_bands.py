@@ -44,3 +44,24 @@ def test_bands_in_workgroups_of_their_own(gpu_device, S, T, modified):
     gx, gy = oracle.mi_backward(px, py, bnd, p_cpu, torch.ones(n))
     for a, b in ((got[2], gx), (got[3], gy)):
         assert not torch.isnan(a).any() and bool((a - b).norm() <= 2e-3 * b.norm().clamp(min=1))
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("S,T", [(64, 12988), (65, 12989), (100, 13480), (255, 14000), (70, 30000)])
+def test_long_utterances_take_the_launch_that_fits(gpu_device, S, T, modified):
+    """The LDS of a workgroup grows with T, twice as fast where a band has one to itself: such a
+    launch fits up to T = 12 988, the others up to 30 636."""
+    g = torch.Generator().manual_seed(S + T)
+    T1 = T if modified else T + 1
+    px = -4 + torch.randn(1, S, T1, generator=g)
+    py = -0.1 * torch.rand(1, S + 1, T, generator=g)
+    print(f"S={S} T={T} modified={modified}", flush=True)
+    p = torch.zeros(1, S + 1, T + 1, device=gpu_device)
+    x, y = px.to(gpu_device), py.to(gpu_device)
+    score = _fast_rnnt.mutual_information_forward(x, y, None, p)
+    gx, gy = _fast_rnnt.mutual_information_backward(x, y, None, p, torch.ones(1, device=gpu_device))
+    want = oracle.mi_forward(px, py, None, torch.zeros(1, S + 1, T + 1))
+    assert abs(score.item() - want.item()) <= 1e-5 * abs(want.item())
+    # every path passes every frame once; each of the S + T steps of a path rounds once
+    frames = gy.double().sum(1) + (gx.double().sum(1) if modified else 0)
+    assert bool(((frames - 1).abs() <= (S + T) * 2.0 ** -24).all()), (frames - 1).abs().max().item()
