@@ -1269,29 +1269,26 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
 
 constexpr size_t kLdsBudget = 156 * 1024;
 
+// Dynamic LDS of a launch: per sweep wave a seam row and 2 x buffers tiles.
+size_t lds_bytes(int nsweep, int T, int buffers, size_t elem) {
+  return (size_t)nsweep *
+         ((size_t)((T + 1 + kSeamSlack + 3) & ~3) + (size_t)buffers * 2 * kTileElems) * elem;
+}
+
 // Sweep waves per workgroup: one per 64 rows, as many as LDS allows.
-int pick_sweep_waves(int S, int T, size_t elem, int arrays) {
+int pick_sweep_waves(int S, int T, size_t elem) {
   int n = (S + 1 + kWave - 1) / kWave;
   n = n < 1 ? 1 : (n > kMaxSweep ? kMaxSweep : n);
-  auto bytes = [&](int k) {
-    return (size_t)k * ((size_t)((T + 1 + kSeamSlack + 3) & ~3) + (size_t)arrays * 2 * kTileElems) * elem;
-  };
-  while (n > 1 && bytes(n) > kLdsBudget) --n;
+  while (n > 1 && lds_bytes(n, T, 2, elem) > kLdsBudget) --n;
   return n;
 }
 
-// Dynamic LDS of a launch: per sweep wave a seam row, 2 x buffers tiles and (backward) what the row
-// above hands to each buffer's steps.
-size_t lds_bytes(int nsweep, int T, int buffers, size_t elem) {
-  return (size_t)nsweep * ((size_t)((T + 1 + kSeamSlack + 3) & ~3) +
-                           (size_t)buffers * (2 * kTileElems + kTileSteps)) * elem;
-}
-
-// Dynamic LDS of a workgroup that has a band to itself: one sweep wave's share, and a second seam row.
+// Dynamic LDS of a workgroup that has a band to itself: one sweep wave's share, a second seam row and
+// (backward) what the row above hands to each buffer's steps.
 constexpr int kApartBuffers = 3;
 size_t apart_lds_bytes(int T) {
   return lds_bytes(1, T, kApartBuffers, sizeof(float)) +
-         (size_t)((T + 1 + kSeamSlack + 3) & ~3) * sizeof(float);
+         (size_t)(((T + 1 + kSeamSlack + 3) & ~3) + kApartBuffers * kTileSteps) * sizeof(float);
 }
 
 // Whether every band of 64 rows gets a workgroup of its own.  It costs a fixed time -- the marks, and
@@ -1299,7 +1296,7 @@ size_t apart_lds_bytes(int T) {
 // both measured (microseconds, nanoseconds), for 2, 3 and 4 bands.
 // (B 12, S 220, T 1500: 134 + 164 -> 72 + 80 us; B 3, S 250, T 1335: 120 + 149 -> 67 + 74;
 // B 10, S 137, T 817: 51 + 60 -> 43 + 48.)
-// Both seam rows must fit into LDS (T up to 12 988; the other launch goes to 30 636).  Two workgroups
+// Both seam rows must fit into LDS (T up to 12 988; the other launch goes to 30 700).  Two workgroups
 // share a compute unit while their LDS allows it (T up to 3 004).  Beyond, a band that finds no unit
 // of its own starts when an earlier one is done: two bands, which one workgroup sweeps almost as fast
 // as two, then stay together (B 136, S 100, T 6000: 595 + 599 apart, 407 + 555 together; B 136, S 70,
@@ -1333,7 +1330,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   if (!px || !py || !p || !ans) return fail(FRNNT_EINVAL, "mi_forward: null pointer");
   if ((size_t)(S + 1) * (T + 1) * sizeof(R) >= ((size_t)1 << 30))
     return fail(FRNNT_ELIMIT, "mi_forward: one utterance's lattice exceeds 1 GiB");
-  const int n = pick_sweep_waves(S, T, sizeof(R), 2);
+  const int n = pick_sweep_waves(S, T, sizeof(R));
   if (lds_bytes(n, T, 2, sizeof(R)) > kLdsBudget)
     return fail(FRNNT_ELIMIT, "mi_forward: T=%d needs %zu bytes of LDS", T, lds_bytes(n, T, 2, sizeof(R)));
   // With at most two sweep waves there is room, for floats, for a third tile buffer, which
@@ -1393,7 +1390,7 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
     return fail(FRNNT_EINVAL, "mi_backward: null pointer");
   if ((size_t)(S + 1) * (T + 1) * sizeof(R) >= ((size_t)1 << 30))
     return fail(FRNNT_ELIMIT, "mi_backward: one utterance's lattice exceeds 1 GiB");
-  const int n = pick_sweep_waves(S, T, sizeof(R), 2);
+  const int n = pick_sweep_waves(S, T, sizeof(R));
   if (lds_bytes(n, T, 2, sizeof(R)) > kLdsBudget)
     return fail(FRNNT_ELIMIT, "mi_backward: T=%d needs %zu bytes of LDS", T, lds_bytes(n, T, 2, sizeof(R)));
   // With at most two sweep waves there is room for more staging waves per sweep wave and,

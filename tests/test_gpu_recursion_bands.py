@@ -46,21 +46,28 @@ def test_bands_in_workgroups_of_their_own(gpu_device, S, T, modified):
         assert not torch.isnan(a).any() and bool((a - b).norm() <= 2e-3 * b.norm().clamp(min=1))
 
 
+LONG = [(64, 12988), (65, 12989), (100, 13480), (255, 14000), (70, 30700), (250, 686), (192, 748),
+        (255, 749), (150, 4074), (100, 10730)]
+
+
 @pytest.mark.parametrize("modified", [False, True])
-@pytest.mark.parametrize("S,T", [(64, 12988), (65, 12989), (100, 13480), (255, 14000), (70, 30000)])
-def test_long_utterances_take_the_launch_that_fits(gpu_device, S, T, modified):
-    """The LDS of a workgroup grows with T, twice as fast where a band has one to itself: such a
-    launch fits up to T = 12 988, the others up to 30 636."""
+@pytest.mark.parametrize("S,T,dtype", [(*size, torch.float32) for size in LONG] +
+                         [(100, 700, torch.float64), (100, 749, torch.float64),
+                          (40, 10732, torch.float64)])
+def test_every_length_finds_a_launch_that_fits(gpu_device, S, T, dtype, modified):
+    """The LDS of a workgroup grows with T.  float32: a band has a workgroup to itself up to
+    T = 12 988; a workgroup holds four sweep waves up to T = 748, three up to 4 076, two up to
+    10 732, one up to 30 700.  float64: two up to 748, one up to 10 732."""
     g = torch.Generator().manual_seed(S + T)
     T1 = T if modified else T + 1
-    px = -4 + torch.randn(1, S, T1, generator=g)
-    py = -0.1 * torch.rand(1, S + 1, T, generator=g)
-    print(f"S={S} T={T} modified={modified}", flush=True)
-    p = torch.zeros(1, S + 1, T + 1, device=gpu_device)
+    px = -4 + torch.randn(1, S, T1, generator=g, dtype=dtype)
+    py = -0.1 * torch.rand(1, S + 1, T, generator=g, dtype=dtype)
+    print(f"S={S} T={T} {dtype} modified={modified}", flush=True)
+    p = torch.zeros(1, S + 1, T + 1, device=gpu_device, dtype=dtype)
     x, y = px.to(gpu_device), py.to(gpu_device)
     score = _fast_rnnt.mutual_information_forward(x, y, None, p)
-    gx, gy = _fast_rnnt.mutual_information_backward(x, y, None, p, torch.ones(1, device=gpu_device))
-    want = oracle.mi_forward(px, py, None, torch.zeros(1, S + 1, T + 1))
+    gx, gy = _fast_rnnt.mutual_information_backward(x, y, None, p, torch.ones_like(score))
+    want = oracle.mi_forward(px, py, None, torch.zeros(1, S + 1, T + 1, dtype=dtype))
     assert abs(score.item() - want.item()) <= 1e-5 * abs(want.item())
     # every path passes every frame once; each of the S + T steps of a path rounds once
     frames = gy.double().sum(1) + (gx.double().sum(1) if modified else 0)
