@@ -372,13 +372,29 @@ __device__ __forceinline__ bool send_seam(double *, int, int, const double *, co
   return false;
 }
 
+// A word that any of an utterance's workgroups may make NaN (a wait of theirs ran out) and that the
+// last one gives its value: the value replaces what the word held before the launch and nothing
+// else, the NaN replaces anything.  Whichever comes first, the NaN stays.
+__device__ __forceinline__ void store_nan(float *word) {
+  __hip_atomic_store(reinterpret_cast<int *>(word),
+                     __float_as_int(std::numeric_limits<float>::quiet_NaN()), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_once(float *word, int before, float value) {
+  __hip_atomic_compare_exchange_strong(reinterpret_cast<int *>(word), &before,
+                                       __float_as_int(value), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The marks of an utterance's seam rows: in p (which may be NULL) where rows s0 + 63, s0 + 127, ...
-// of the window feed the next one, in px_grad (which may be NULL) where the reversed rows do.
-// A block per utterance and seam.
+// of the window feed the next one, in px_grad (which may be NULL) where the reversed rows do; and,
+// with p, the utterance's score (see store_once).  A block per utterance and seam.
 __global__ void __launch_bounds__(256)
     mark_seams_kernel(const int64_t *__restrict__ boundary, float *__restrict__ p,
-                      float *__restrict__ px_grad, int S, int T, int modified) {
+                      float *__restrict__ ans, float *__restrict__ px_grad, int S, int T,
+                      int modified) {
   const int b = blockIdx.x, last = (int)blockIdx.y * kWave + kWave - 1;  // (row, or reversed row)
+  if (p && blockIdx.y == 0 && threadIdx.x == 0) ans[b] = __int_as_float(kSeamMark);
   const Window win = load_window(boundary, b, S, T);
   if (!win.ok || last + 1 > win.ns) return;
   const float mark = __int_as_float(kSeamMark);
@@ -463,7 +479,10 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   auto give_up = [&]() {
     if (lane == 0) {
       publish(&cnt.failed, 1);
-      ans[b] = std::numeric_limits<R>::quiet_NaN();
+      if constexpr (kApart)
+        store_nan(&ans[b]);
+      else
+        ans[b] = std::numeric_limits<R>::quiet_NaN();
     }
   };
 
@@ -750,7 +769,10 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       if (!one_tile(m, std::true_type{})) return;
     for (int m = plain; m < g.ntiles; ++m)
       if (!one_tile(m, std::false_type{})) return;
-    if (lane == fin_lane) {
+    if (kApart && lane == fin_lane) {
+      // (one that gave up here or in another band's workgroup has stored, or will store, its NaN)
+      if constexpr (kApart) store_once(&ans[b], kSeamMark, fin);
+    } else if (lane == fin_lane) {
       ans[b] = peek(&cnt.failed) ? std::numeric_limits<R>::quiet_NaN() : fin;
       // A staging wave may give up between that look and the store, and its NaN must not be
       // covered by the score: once the store has left, look again.  A wave that gives up
@@ -869,13 +891,23 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   // A wave whose bounded wait ran out leaves NaN where the window starts -- in px_grad,
   // in py_grad and, when it is written back, in ans_grad -- so that the utterance's
   // gradients cannot pass for a result; every staging wave repeats that when it is done
-  // and finds the mark, so no later store of a good value covers it up.
+  // and finds the mark, so no later store of a good value covers it up.  (apart: and where the
+  // band's first row starts, because another workgroup, which does not see the mark, may store
+  // the window's start later; nobody else stores the band's rows.)
   auto poison = [&]() {
     if (lane != 0) return;
     const R nan = std::numeric_limits<R>::quiet_NaN();
-    if (NS > 0) put1(gx_rsrc, (win.s0 * T1 + win.t0) * (int)sizeof(R), nan);
+    if (NS > 0 && NT >= shift) put1(gx_rsrc, (win.s0 * T1 + win.t0) * (int)sizeof(R), nan);
     if (NT > 0) put1(gy_rsrc, (win.s0 * T + win.t0) * (int)sizeof(R), nan);
-    if (overwrite_ans_grad && ans_grad) ans_grad[b] = nan;
+    if constexpr (kApart) {
+      const int i = NS - part * kWave;  // the band's first row
+      if (i > 0 && NT >= shift)
+        put1(gx_rsrc, ((win.s0 + i - 1) * T1 + win.t0) * (int)sizeof(R), nan);
+      if (NT > 0) put1(gy_rsrc, ((win.s0 + i) * T + win.t0) * (int)sizeof(R), nan);
+      if (overwrite_ans_grad && ans_grad) store_nan(&ans_grad[b]);
+    } else {
+      if (overwrite_ans_grad && ans_grad) ans_grad[b] = nan;
+    }
   };
   auto give_up = [&]() {
     if (lane == 0) publish(&cnt.failed, 1);
@@ -1261,8 +1293,14 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       done = has_down ? sweep_tiles(std::false_type{}, std::true_type{})
                       : sweep_tiles(std::false_type{}, std::false_type{});
     if (!done) return;
-    if (lane == fin_lane && overwrite_ans_grad && ans_grad)
-      ans_grad[b] = peek(&cnt.failed) ? std::numeric_limits<R>::quiet_NaN() : g_origin;
+    if (lane == fin_lane && overwrite_ans_grad && ans_grad) {
+      if constexpr (kApart) {
+        // (a NaN found as the seed is the caller's or another workgroup's: it stays either way)
+        if (seed == seed) store_once(&ans_grad[b], __float_as_int(seed), g_origin);
+      } else {
+        ans_grad[b] = peek(&cnt.failed) ? std::numeric_limits<R>::quiet_NaN() : g_origin;
+      }
+    }
     tile_base += g.ntiles;
   }
 }
@@ -1313,12 +1351,11 @@ bool bands_apart(int B, int S, int T, bool backward) {
   constexpr double kCost[2][3] = {{6, 7, 10}, {11, 16, 20}}, kSaved[2][3] = {{6.7, 7, 39}, {13, 28, 60}};
   return 1e-3 * kSaved[backward][bands - 2] * (S + T) > kCost[backward][bands - 2];
 }
-inline void mark_seams(const int64_t *boundary, float *p, float *px_grad, int B, int S, int T,
-                       int modified, hipStream_t stream) {
+inline void mark_seams(const int64_t *boundary, float *p, float *ans, float *px_grad, int B, int S,
+                       int T, int modified, hipStream_t stream) {
   hipLaunchKernelGGL(mark_seams_kernel, dim3(B, (S + kWave) / kWave - 1), dim3(256), 0, stream,
-                     boundary, p, px_grad, S, T, modified);
+                     boundary, p, ans, px_grad, S, T, modified);
 }
-inline void mark_seams(const int64_t *, double *, double *, int, int, int, int, hipStream_t) {}
 
 // `px_grad`: if given, its seams are marked as well (for a backward_impl that follows and is told so).
 template <typename R>
@@ -1344,7 +1381,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   if constexpr (sizeof(R) == 4) {
     const bool apart = bands_apart<R>(B, S, T, false), later = px_grad && bands_apart<R>(B, S, T, true);
     if (apart || later)
-      mark_seams(boundary, apart ? p : nullptr, later ? px_grad : nullptr, B, S, T, modified,
+      mark_seams(boundary, apart ? p : nullptr, ans, later ? px_grad : nullptr, B, S, T, modified,
                  static_cast<hipStream_t>(stream));
     if (apart) {
       const int pitch = (B + 7) / 8 * 8;  // (an utterance's bands on one XCD)
@@ -1405,7 +1442,8 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   if constexpr (kFloat) {
     if (bands_apart<R>(B, S, T, true)) {
       if (!marked)
-        mark_seams(boundary, nullptr, px_grad, B, S, T, modified, static_cast<hipStream_t>(stream));
+        mark_seams(boundary, nullptr, nullptr, px_grad, B, S, T, modified,
+                   static_cast<hipStream_t>(stream));
       const int pitch = (B + 7) / 8 * 8;
       const size_t lds = apart_lds_bytes(T);
       auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kApartBuffers, true>

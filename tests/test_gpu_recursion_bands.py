@@ -5,7 +5,7 @@ each: the results must be the same bits.  Oracle: the CPU restatement in float32
 import pytest
 import torch
 
-from fast_rnnt_amd import _fast_rnnt
+from fast_rnnt_amd import _fast_rnnt, _lib
 from oracle import recursion as oracle
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +72,48 @@ def test_every_length_finds_a_launch_that_fits(gpu_device, S, T, dtype, modified
     # every path passes every frame once; each of the S + T steps of a path rounds once
     frames = gy.double().sum(1) + (gx.double().sum(1) if modified else 0)
     assert bool(((frames - 1).abs() <= (S + T) * 2.0 ** -24).all()), (frames - 1).abs().max().item()
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("S,T", [(100, 900), (250, 700)])
+def test_a_wait_that_runs_out_in_any_band_shows_as_nan(gpu_device, S, T, modified):
+    """Whichever band's waits run out, the utterance's score is NaN, and so is a gradient of it and
+    what reaches its start, unless every cell is what it is without a bound."""
+    B, T1 = 8, T if modified else T + 1
+    g = torch.Generator().manual_seed(S + T)
+    px = (-1 + torch.randn(B, S, T1, generator=g)).to(gpu_device)
+    py = (-1 + torch.randn(B, S + 1, T, generator=g)).to(gpu_device)
+
+    def forward():
+        p = torch.full((B, S + 1, T + 1), 12345.0, device=gpu_device)
+        return _fast_rnnt.mutual_information_forward(px, py, None, p), p
+
+    def backward():
+        seed = torch.ones(B, device=gpu_device)
+        return (*_fast_rnnt.mutual_information_backward(px, py, None, p, seed), seed)
+
+    score, p = forward()
+    gx, gy, seed = backward()
+    lib = _lib.load()
+    gave_up = 0
+    for polls in (1, 2, 5, 20, 60, 150, 400, 1000, 1 << 22):
+        print(f"S={S} T={T} modified={modified} polls={polls}", flush=True)
+        lib.frnnt_set_spin_limit(polls)
+        try:
+            score1, p1 = forward()
+            gx1, gy1, seed1 = backward()
+            torch.cuda.synchronize()
+        finally:
+            lib.frnnt_set_spin_limit(0)
+        for b in range(B):
+            failed = bool(torch.isnan(score1[b]))
+            gave_up += failed
+            assert failed or (torch.equal(score1[b], score[b]) and torch.equal(p1[b], p[b]))
+            nan = bool(torch.isnan(gx1[b]).any()), bool(torch.isnan(gy1[b]).any())
+            if not any(nan) and not torch.isnan(seed1[b]):
+                assert torch.equal(gx1[b], gx[b]) and torch.equal(gy1[b], gy[b])
+                assert torch.equal(seed1[b], seed[b])
+            else:
+                assert all(nan) and bool(torch.isnan(seed1[b]))
+        assert polls > 1 or gave_up == B
+        assert polls < 1 << 22 or torch.equal(score1, score)
