@@ -996,9 +996,53 @@ Tensor gather_rows(const Tensor &lm, const Tensor &rng) {
   return out;
 }
 
+// the adjoint of gather_rows: [B][T][R][C] -> [B][rows][C]
+Tensor scatter_rows(const Tensor &grad, const Tensor &rng, int64_t rows) {
+  const Tensor g = grad.contiguous();
+  const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2), C = g.size(3);
+  Tensor out = at::empty({B, rows, C}, g.options());
+  check_rc(frnnt_pruning_bwd(dtype_code(g.scalar_type()), nullptr, g.data_ptr(), iptr(rng), nullptr,
+                             out.data_ptr(), (int)B, (int)rows - 1, (int)T, (int)R, (int)C,
+                             stream_of(g)),
+           "frnnt_pruning_bwd");
+  return out;
+}
+
+// gather_rows and its adjoint as autograd nodes, each the other's derivative: both can be
+// differentiated as often as the caller likes (create_graph=True).
+struct GatherRowsFn : public torch::autograd::Function<GatherRowsFn> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &ranges);
+  static variable_list backward(AutogradContext *ctx, variable_list grads);
+};
+struct ScatterRowsFn : public torch::autograd::Function<ScatterRowsFn> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &grad, const Tensor &rng, int64_t rows) {
+    DeviceGuard guard(grad.device());
+    ctx->save_for_backward({rng});
+    return scatter_rows(grad, rng, rows);
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    return {GatherRowsFn::apply(grads[0], ctx->get_saved_variables()[0]), Tensor(), Tensor()};
+  }
+};
+Tensor GatherRowsFn::forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &ranges) {
+  DeviceGuard guard(lm_.device());
+  const Tensor lm = lm_.contiguous(), rng = ranges.contiguous();
+  ctx->save_for_backward({rng});
+  ctx->saved_data["rows"] = lm.size(1);
+  return gather_rows(lm, rng);
+}
+variable_list GatherRowsFn::backward(AutogradContext *ctx, variable_list grads) {
+  const Tensor rng = ctx->get_saved_variables()[0];
+  const int64_t rows = ctx->saved_data["rows"].toInt();
+  if (at::GradMode::is_enabled()) return {ScatterRowsFn::apply(grads[0], rng, rows), Tensor()};
+  DeviceGuard guard(grads[0].device());
+  return {scatter_rows(grads[0], rng, rows), Tensor()};
+}
+
 // do_rnnt_pruning as one autograd node (rnnt_loss.py:780-818): am_pruned is a view of am, lm_pruned
 // a gathered copy; backward = frnnt_pruning_bwd, which reads a gradient that both share -- the
-// joiner that follows adds the two -- once.
+// joiner that follows adds the two -- once.  A backward that is to be differentiated itself takes
+// the two adjoints as nodes of their own.
 struct PruningFn : public torch::autograd::Function<PruningFn> {
   static variable_list forward(AutogradContext *ctx, const Tensor &am, const Tensor &lm_,
                                const Tensor &ranges) {
@@ -1019,6 +1063,11 @@ struct PruningFn : public torch::autograd::Function<PruningFn> {
     const Tensor &any = grads[0].defined() ? grads[0] : grads[1];
     if (!any.defined()) return out;
     const int64_t C = any.size(3);
+    if (at::GradMode::is_enabled()) {
+      if (grads[0].defined()) out[0] = grads[0].sum(2);
+      if (grads[1].defined()) out[1] = ScatterRowsFn::apply(grads[1], rng, S1);
+      return out;
+    }
     DeviceGuard guard(any.device());
     const Tensor ga = grads[0].defined() ? grads[0].contiguous() : Tensor();
     // (one tensor stays one, also where a copy of it has to be made)
@@ -1036,30 +1085,6 @@ struct PruningFn : public torch::autograd::Function<PruningFn> {
   }
 };
 
-// lm alone
-struct GatherRowsFn : public torch::autograd::Function<GatherRowsFn> {
-  static Tensor forward(AutogradContext *ctx, const Tensor &lm_, const Tensor &ranges) {
-    DeviceGuard guard(lm_.device());
-    const Tensor lm = lm_.contiguous(), rng = ranges.contiguous();
-    ctx->save_for_backward({rng});
-    ctx->saved_data["rows"] = lm.size(1);
-    return gather_rows(lm, rng);
-  }
-  static variable_list backward(AutogradContext *ctx, variable_list grads) {
-    const Tensor rng = ctx->get_saved_variables()[0];
-    const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2), C = grads[0].size(3),
-                  S1 = ctx->saved_data["rows"].toInt();
-    DeviceGuard guard(grads[0].device());
-    const Tensor g = grads[0].contiguous();
-    Tensor lm_grad = at::empty({B, S1, C}, g.options());
-    check_rc(frnnt_pruning_bwd(dtype_code(g.scalar_type()), nullptr, g.data_ptr(), iptr(rng),
-                               nullptr, lm_grad.data_ptr(), (int)B, (int)S1 - 1, (int)T, (int)R,
-                               (int)C, stream_of(g)),
-             "frnnt_pruning_bwd");
-    return {lm_grad, Tensor()};
-  }
-};
-
 std::tuple<Tensor, Tensor> pruning(const Tensor &am, const Tensor &lm, const Tensor &ranges) {
   TORCH_CHECK(lm.is_cuda(), "fast_rnnt_amd runs on GPU tensors only (no CPU path): lm");
   TORCH_CHECK(lm.scalar_type() == at::kFloat || lm.scalar_type() == at::kDouble ||
@@ -1072,8 +1097,10 @@ std::tuple<Tensor, Tensor> pruning(const Tensor &am, const Tensor &lm, const Ten
   TORCH_CHECK(am.device() == lm.device() && ranges.device() == lm.device() &&
                   am.scalar_type() == lm.scalar_type() && ranges.scalar_type() == at::kLong,
               "am and lm must share a device and a type, ranges be int64 on that device");
-  const bool grad_mode = at::GradMode::is_enabled();
-  if (grad_mode && am.requires_grad() && lm.requires_grad() && am.size(2) == lm.size(2)) {
+  // (a tangent of am passes through the view, which the node does not know; with one kept position
+  // am_pruned may be written to, which is not allowed for a view that a node of two outputs returns)
+  if (at::GradMode::is_enabled() && am.requires_grad() && lm.requires_grad() &&
+      am.size(2) == lm.size(2) && ranges.size(2) > 1 && !am._fw_grad(/*level=*/0).defined()) {
     const variable_list out = PruningFn::apply(am, lm, ranges);
     return {out[0], out[1]};
   }

@@ -1,0 +1,55 @@
+"""Where an autograd node stands in for torch operations: what passes through them -- a second
+derivative, a tangent, a write to a view -- passes through it as well."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwd
+
+import fast_rnnt_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def _pruning_inputs(device, R=3, dtype=torch.float64):
+    g = torch.Generator().manual_seed(7)
+    B, T, S, C = 2, 6, 5, 4
+    am = torch.randn(B, T, C, generator=g, dtype=dtype).to(device).requires_grad_(True)
+    lm = torch.randn(B, S + 1, C, generator=g, dtype=dtype).to(device).requires_grad_(True)
+    begin = torch.tensor([[0, 0, 1, 2, 2, 3], [0, 1, 1, 1, 3, 3]])
+    return am, lm, (begin.unsqueeze(2) + torch.arange(R)).to(device)
+
+
+@pytest.mark.parametrize("R", [1, 3])
+def test_second_derivatives_of_the_pruning(gpu_device, R):
+    am, lm, ranges = _pruning_inputs(gpu_device, R)
+    prune = fast_rnnt_amd.do_rnnt_pruning
+    assert torch.autograd.gradgradcheck(lambda a, l: prune(a, l, ranges), (am, lm))
+    assert torch.autograd.gradgradcheck(lambda a: prune(a, lm, ranges)[0], (am,))
+    assert torch.autograd.gradgradcheck(lambda l: prune(am.detach(), l, ranges)[1], (lm,))
+    # a gradient penalty, against the same with torch's own operations
+    rows = ranges.reshape(2, -1, 1).expand(2, 6 * R, 4)
+    want, got = [], []
+    for out, kept in ((want, (am.unsqueeze(2).expand(2, 6, R, 4),
+                              torch.gather(lm, 1, rows).reshape(2, 6, R, 4))),
+                      (got, prune(am, lm, ranges))):
+        grads = torch.autograd.grad(torch.tanh(kept[0] + kept[1]).sum(), (am, lm), create_graph=True)
+        out.extend(torch.autograd.grad(sum(x.square().sum() for x in grads), (am, lm)))
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-12, atol=1e-12)
+
+
+def test_a_tangent_of_am_passes_through_the_pruning(gpu_device):
+    am, lm, ranges = _pruning_inputs(gpu_device)
+    tangent = torch.randn_like(am)
+    with fwd.dual_level():
+        am_pruned, lm_pruned = fast_rnnt_amd.do_rnnt_pruning(fwd.make_dual(am, tangent), lm, ranges)
+        got = fwd.unpack_dual(am_pruned).tangent
+        assert torch.equal(got, tangent.unsqueeze(2).expand(am_pruned.shape))
+        assert lm_pruned.requires_grad and am_pruned.requires_grad
+
+
+def test_one_kept_position_may_be_written_to(gpu_device):
+    am, lm, ranges = _pruning_inputs(gpu_device, R=1)
+    am_pruned, lm_pruned = fast_rnnt_amd.do_rnnt_pruning(am * 1, lm, ranges)
+    am_pruned.mul_(2)
+    (am_pruned + lm_pruned).sum().backward()
+    assert torch.equal(am.grad, torch.full_like(am, 2.0))
