@@ -404,10 +404,15 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &gx = saved[0], &gy = saved[1];
+    Tensor gx = saved[0], gy = saved[1];
     const int64_t B = gx.size(0), S = gx.size(1), T1 = gx.size(2), T = gy.size(2);
     DeviceGuard guard(gx.device());
     const Tensor g = grads[0].contiguous();
+    if (at::GradMode::is_enabled() && g.requires_grad()) {
+      // (differentiated itself, e.g. with respect to weights of the scores: an operation on record)
+      const Tensor f = g.view({B, 1, 1});
+      return {gx.mul_(f), gy.mul_(f), Tensor(), Tensor(), Tensor()};
+    }
     auto run = [&](auto r) {
       using R = decltype(r);
       return abi_mi_scale_grads(ptr<R>(gx), ptr<R>(gy), ptr<R>(g), 1, 1.0, (int)B, (int)S, (int)T,

@@ -53,3 +53,21 @@ def test_one_kept_position_may_be_written_to(gpu_device):
     am_pruned.mul_(2)
     (am_pruned + lm_pruned).sum().backward()
     assert torch.equal(am.grad, torch.full_like(am, 2.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_gradients_of_the_recursion_keep_the_history_of_the_scores_gradient(gpu_device, dtype):
+    g = torch.Generator().manual_seed(3)
+    B, S, T = 3, 4, 6
+    px = torch.randn(B, S, T + 1, generator=g, dtype=dtype).to(gpu_device).requires_grad_(True)
+    py = torch.randn(B, S + 1, T, generator=g, dtype=dtype).to(gpu_device).requires_grad_(True)
+    weights = torch.tensor([1.0, 2.0, -0.5], dtype=dtype, device=gpu_device, requires_grad=True)
+    scores, occupation = fast_rnnt_amd.mutual_information_recursion(px, py, return_grad=True)
+    occ_x, occ_y = (x.clone() for x in occupation)
+    gx, gy = torch.autograd.grad((weights * scores).sum(), (px, py), create_graph=True)
+    for got, occ, handed_out in ((gx, occ_x, occupation[0]), (gy, occ_y, occupation[1])):
+        assert torch.equal(handed_out.detach(), got.detach())  # (scaled in place)
+        assert torch.equal(got.detach(), occ * weights.detach().reshape(B, 1, 1))
+    (gx.sum() + gy.square().sum()).backward()
+    want = occ_x.sum((1, 2)) + 2 * weights.detach() * occ_y.square().sum((1, 2))
+    assert torch.allclose(weights.grad, want, rtol=1e-5, atol=1e-6)
