@@ -16,7 +16,7 @@ row (default ``[0, 0, S, T]``)::
 with out-of-window terms taken as -inf; the result is ``p[b, s_end, t_end]``.
 """
 import weakref
-from typing import Optional, Sequence, Tuple, Union
+from typing import List, Optional, Sequence, Tuple, Union
 
 import torch
 from torch import Tensor
@@ -94,6 +94,45 @@ def check_boundaries(device=None) -> None:
     calls so far has found bad on the device (see :func:`set_boundary_checks`)."""
     index = torch.cuda.current_device() if device is None else torch.device(device).index
     _lib.ops().check_boundaries(int(index))
+
+
+class MutualInformationRecursionFunction(torch.autograd.Function):
+    """The reference's autograd wrapper under its own name
+    (fast_rnnt/python/fast_rnnt/mutual_information.py:24-181), for code that calls ``.apply``;
+    :func:`mutual_information_recursion` itself goes through a compiled node of the same behaviour.
+
+    ``forward`` runs the forward operator and, when gradients may be needed, immediately the
+    backward operator with a gradient of ones, whose results also go into the caller's list
+    ``pxy_grads`` of two; ``backward`` only scales them, in place.
+    """
+
+    @staticmethod
+    def forward(ctx, px: Tensor, py: Tensor, pxy_grads: List[Optional[Tensor]],
+                boundary: Optional[Tensor] = None, return_grad: bool = False) -> Tensor:
+        (B, S, T1) = px.shape
+        T = py.shape[-1]
+        assert T1 in [T, T + 1]
+        assert py.shape == (B, S + 1, T)
+        if boundary is not None:
+            assert boundary.shape == (B, 4)
+        assert len(pxy_grads) == 2
+        p = torch.empty(B, S + 1, T + 1, device=px.device, dtype=px.dtype)
+        scores = _fast_rnnt.mutual_information_forward(px, py, boundary, p)
+        grads = [None, None]
+        if return_grad or px.requires_grad or py.requires_grad:
+            grads = _fast_rnnt.mutual_information_backward(px, py, boundary, p,
+                                                           torch.ones_like(scores))
+            ctx.save_for_backward(*grads)
+        pxy_grads[:] = grads
+        return scores
+
+    @staticmethod
+    def backward(ctx, ans_grad: Tensor) -> Tuple[Tensor, Tensor, None, None, None]:
+        px_grad, py_grad = ctx.saved_tensors
+        scale = ans_grad.reshape(-1, 1, 1)
+        px_grad *= scale
+        py_grad *= scale
+        return px_grad, py_grad, None, None, None
 
 
 def mutual_information_recursion(

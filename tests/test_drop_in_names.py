@@ -39,6 +39,14 @@ def test_submodules_are_the_implementation():
     assert rnnt_loss_pruned is fast_rnnt_amd.rnnt_loss_pruned
 
 
+def test_autograd_wrapper_keeps_its_name():
+    # mutual_information.py:24, reachable in its submodule
+    from fast_rnnt.mutual_information import MutualInformationRecursionFunction as wrapper
+    assert issubclass(wrapper, torch.autograd.Function)
+    assert list(inspect.signature(wrapper.forward).parameters) == \
+        ["ctx", "px", "py", "pxy_grads", "boundary", "return_grad"]
+
+
 def test_operator_module_signatures():
     # python/csrc/mutual_information.cu:27-67: keyword names are part of the interface
     assert list(inspect.signature(_fast_rnnt.mutual_information_forward).parameters) == \

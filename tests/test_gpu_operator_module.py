@@ -180,3 +180,30 @@ def test_other_losses_report_bad_rows_too(gpu_device):
     with pytest.raises(AssertionError, match="boundary row 1"):
         fast_rnnt_amd.check_boundaries()
     assert torch.isnan(loss[1]) and torch.isfinite(loss[[0, 2]]).all()
+
+
+@pytest.mark.parametrize("return_grad", [False, True])
+def test_autograd_wrapper_equals_the_compiled_node(gpu_device, return_grad):
+    from fast_rnnt_amd.mutual_information import MutualInformationRecursionFunction
+    B, S, T = 3, 9, 14
+    px, py = _lattice(5, B, S, T)
+    boundary = torch.tensor([[0, 0, S, T], [1, 2, 7, 11], [0, 0, 4, T]]).to(gpu_device)
+    weights = torch.tensor([1.0, -2.0, 0.5], device=gpu_device)
+    results = []
+    for direct in (True, False):
+        x, y = (v.to(gpu_device).requires_grad_(True) for v in (px, py))
+        grads = [None, None]
+        if direct:
+            scores = MutualInformationRecursionFunction.apply(x, y, grads, boundary, return_grad)
+        else:
+            scores, grads = fast_rnnt_amd.mutual_information_recursion(x, y, boundary, True)
+        occupation = [v.clone() for v in grads]
+        (weights * scores).sum().backward()
+        results.append([scores.detach(), *occupation, *grads, x.grad, y.grad])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        grads = [None, None]
+        MutualInformationRecursionFunction.apply(px.to(gpu_device), py.to(gpu_device), grads,
+                                                 boundary, return_grad)
+    assert all((v is not None) == return_grad for v in grads)
