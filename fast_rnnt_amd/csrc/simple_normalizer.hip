@@ -178,9 +178,10 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   // (rnnt_loss.py:174-178); a maximum is known only after the whole row has been seen, so
   // each wave works with a SHIFT per row instead: the largest value of the row it had
   // seen when the shift was last set.  A value more than kMargin above the shift (always
-  // the case for the first finite value of a row) makes the wave raise its shifts and
+  // the case for the first finite value of a row) makes the wave raise the row's shift and
   // scale its partial sums to match; anything closer stays representable, e^(2 kMargin)
-  // per product.  The running maxima are kept beside the shifts, and when the waves
+  // per product.  Only rows that exceed their margin are touched: which rows share a tile
+  // with them has no say in how a row rounds.  The running maxima are kept beside the shifts, and when the waves
   // meet their partial sums are brought to the true maxima, exp(shift - max) <= 1.
   constexpr float kMargin = 30.f;
   floatx4 slab[kLoads];
@@ -234,14 +235,22 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
     v = fmaxf(v, __shfl_xor(v, 1, kWave));
     return fmaxf(v, __shfl_xor(v, 2, kWave));
   };
+  // a row is above its margin exactly when its maximum is
+  auto above_margin = [&](float top, float shift2_) {
+    return __builtin_fmaf(top, kLog2e, shift2_) > kMargin * kLog2e;
+  };
   // (the sums are brought along; -across_row(seen) is the new shift)
   auto raise_shifts = [&](auto live) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       if (j >= 2 * live && j < kLmLoads) continue;
-      const float now = fminf(shift2[j], -across_row(seen[j]) * kLog2e);
-      const float f = __builtin_amdgcn_exp2f(now - shift2[j]);  // exp(old shift - new shift)
-      shift2[j] = now;
+      const float top = across_row(seen[j]);
+      float f = 1.f;
+      if (above_margin(top, shift2[j])) {
+        const float now = fminf(shift2[j], -top * kLog2e);
+        f = __builtin_amdgcn_exp2f(now - shift2[j]);  // exp(old shift - new shift)
+        shift2[j] = now;
+      }
       if (lane % 4 == 0) factor[wave][sub + 16 * j] = f;
     }
     __builtin_amdgcn_wave_barrier();
@@ -265,9 +274,9 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       if (j >= 2 * live && j < kLmLoads) continue;
-      // two three-input maxima; a row is above its margin exactly when its maximum is
+      // two three-input maxima
       seen[j] = max3_raw(max3_raw(slab[j][0], slab[j][1], slab[j][2]), slab[j][3], seen[j]);
-      above |= __builtin_fmaf(seen[j], kLog2e, shift2[j]) > kMargin * kLog2e;
+      above |= above_margin(seen[j], shift2[j]);
     }
     return above;
   };

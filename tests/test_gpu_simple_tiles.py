@@ -47,3 +47,36 @@ def test_simple_loss_at_the_edges_of_tiles(gpu_device, B, S, T, C):
             assert x.grad.dtype == dtype
             off = (x.grad.float().cpu() - y.grad).abs()
             assert bool((off <= 2e-4 + ulp * y.grad.abs()).all()), off.max().item()
+
+
+# (S, T, C, batch sizes at which launch_normalizer_f32 takes tiles of 32, 64, 96 or 128 rows)
+HEIGHTS = [(95, 128, 500, {1: 32, 26: 64, 51: 96}), (120, 200, 600, {1: 32, 11: 64, 22: 128})]
+
+
+@pytest.mark.parametrize("S,T,C,batches", HEIGHTS)
+def test_normalizers_are_the_same_bits_in_tiles_of_any_height(gpu_device, S, T, C, batches):
+    # some rows have values far above what their first entries suggest, so that their shifts are
+    # raised on the way; their neighbours in a tile, which differ with its height, must not notice
+    g = torch.Generator().manual_seed(S)
+    most = max(batches)
+    lm, am = torch.randn(most, S + 1, C, generator=g), torch.randn(most, T, C, generator=g)
+    for x in (lm, am):
+        for b, r in torch.nonzero(torch.rand(x.shape[:2], generator=g) < 0.05).tolist():
+            x[b, r, torch.randint(C // 3, C, (3,), generator=g)] += 40.0
+    symbols = torch.randint(0, C, (most, S), generator=g)
+    lm, am, symbols = lm.to(gpu_device), am.to(gpu_device), symbols.to(gpu_device)
+    first = None
+    for B in batches:
+        print(f"S={S} T={T} C={C} B={B}", flush=True)
+        px, py = fast_rnnt_amd.get_rnnt_logprobs(lm[:B], am[:B], symbols[:B], 0)
+        if first is None:
+            first = px[0].clone(), py[0].clone()
+        assert torch.equal(px[0], first[0]) and torch.equal(py[0], first[1])
+    # (the last column is closed)
+    px, py = px[0, :, :T].double().cpu(), py[0].double().cpu()
+    joint = lm[0].double().cpu().unsqueeze(1) + am[0].double().cpu().unsqueeze(0)  # [S+1][T][C]
+    norm = torch.logsumexp(joint, dim=2)
+    want_y = joint[:, :, 0] - norm
+    want_x = joint[:S].gather(2, symbols[0].cpu().reshape(S, 1, 1).expand(S, T, 1)).squeeze(2) - norm[:S]
+    for got, want in ((px, want_x), (py, want_y)):
+        assert bool(((got - want).abs() <= 2e-6 * want.abs().clamp(min=1) + 2e-5).all())
