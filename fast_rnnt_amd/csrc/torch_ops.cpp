@@ -813,14 +813,16 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
     ctx->set_materialize_grads(false);
     DeviceGuard guard(logits.device());
     const auto opts = logits.options().dtype(c10::CppTypeToScalarType<R>::value);
-    // internal buffers in one allocation: norm | px | py | xr | yr | p | scores
+    // internal buffers in one allocation: px | py | xr | yr | p | scores | norm, unless a backward
+    // will read it, which keeps norm alone
     Carver carve;
-    const int64_t o_nr = carve.take(B * T * K), o_px = carve.take(B * S * T1),
-                  o_py = carve.take(B * (S + 1) * T), o_xr = carve.take(B * T * K),
-                  o_yr = carve.take(B * T * K), o_p = carve.take(B * (S + 1) * (T + 1)),
-                  o_sc = carve.take(B);
-    Tensor work = at::empty({carve.total}, opts);
-    R *w = work.data_ptr<R>();
+    const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(B * (S + 1) * T),
+                  o_xr = carve.take(B * T * K), o_yr = carve.take(B * T * K),
+                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B),
+                  o_nr = carve.take(need_grad ? 0 : B * T * K);
+    const Tensor work = at::empty({carve.total}, opts);
+    const Tensor norm = need_grad ? at::empty({B * T * K}, opts) : Tensor();
+    R *w = work.data_ptr<R>(), *nr = need_grad ? ptr<R>(norm) : w + o_nr;
     Tensor gx, gy;
     if (want_grads || need_grad) {
       gx = at::empty({B, S, T1}, opts);
@@ -828,15 +830,15 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
     }
     Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
     check_rc(abi_lattice_loss_fwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
-                                  iptr(bnd), w + o_px, w + o_py, w + o_nr, w + o_xr, w + o_yr,
-                                  w + o_p, w + o_sc, ptr<R>(gx), ptr<R>(gy), ptr<R>(loss), (int)B,
+                                  iptr(bnd), w + o_px, w + o_py, nr, w + o_xr, w + o_yr, w + o_p,
+                                  w + o_sc, ptr<R>(gx), ptr<R>(gy), ptr<R>(loss), (int)B,
                                   (int)S, (int)T, (int)K, (int)C, (int)term, (int)kind,
                                   delay_penalty > 0.0 ? delay_penalty : 0.0, (int)reduction,
                                   (int)checks, status_for(logits, bnd), stream_of(logits)),
              "frnnt_lattice_loss_fwd");
     if (need_grad) {
       // (absent tensors are not saved: saved tensors must be defined)
-      variable_list save{logits, sym, work, gx, gy};
+      variable_list save{logits, sym, norm, gx, gy};
       if (rng.defined()) save.push_back(rng);
       if (bnd.defined()) save.push_back(bnd);
       ctx->save_for_backward(std::move(save));
@@ -862,7 +864,7 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
   template <typename R>
   static Tensor run_backward(AutogradContext *ctx, const variable_list &saved,
                              const Tensor &g_loss) {
-    const Tensor &logits = saved[0], &sym = saved[1], &work = saved[2];
+    const Tensor &logits = saved[0], &sym = saved[1], &norm = saved[2];
     Tensor gx = saved[3], gy = saved[4];
     const std::vector<int64_t> meta = ctx->saved_data["meta"].toIntVector();
     const int64_t kind = meta[1], reduction = meta[2];
@@ -882,7 +884,7 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
                "frnnt_mi_scale_grads");
     Tensor grad = at::empty(logits.sizes(), logits.options());
     check_rc(abi_lattice_loss_bwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
-                                  iptr(bnd), work.data_ptr<R>(),
+                                  iptr(bnd), ptr<R>(norm),
                                   handed_out ? (const R *)nullptr : ptr<R>(g), stride, scale,
                                   ptr<R>(gx), ptr<R>(gy), grad.data_ptr(), (int)B, (int)S, (int)T,
                                   (int)K, (int)C, (int)meta[0], (int)kind, stream),

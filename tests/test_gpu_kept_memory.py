@@ -1,0 +1,32 @@
+"""What a loss on logits keeps between its forward and its backward: the normalizers and the
+occupation gradients, not the lattices that only the forward needs."""
+import pytest
+import torch
+
+import fast_rnnt_amd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("path", ["joint", "pruned"])
+def test_memory_kept_for_the_backward(gpu_device, path):
+    B, T, S, C, R = 4, 200, 40, 30, 5
+    g = torch.Generator().manual_seed(0)
+    K = S + 1 if path == "joint" else R
+    logits = torch.randn(B, T, K, C, generator=g).to(gpu_device).requires_grad_(True)
+    symbols = torch.randint(1, C, (B, S), generator=g).to(gpu_device)
+    begin = (torch.arange(T) * (S + 2 - R) // T).reshape(1, T, 1).expand(B, T, 1)
+    ranges = (begin + torch.arange(R)).to(gpu_device)
+
+    def loss():
+        if path == "joint":
+            return fast_rnnt_amd.rnnt_loss(logits, symbols, 0, reduction="sum")
+        return fast_rnnt_amd.rnnt_loss_pruned(logits, symbols, ranges, 0, reduction="sum")
+
+    loss().backward()
+    before = torch.cuda.memory_allocated()
+    kept = loss()
+    norm, px_grad, py_grad = B * T * K, B * S * (T + 1), B * (S + 1) * T
+    # (the allocator hands out multiples of 512 bytes)
+    assert torch.cuda.memory_allocated() - before <= 4 * (norm + px_grad + py_grad) + 4 * 512
+    kept.backward()
