@@ -381,6 +381,7 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
     const Tensor px = px_.contiguous(), py = py_.contiguous();
     const Tensor bnd = boundary.defined() ? boundary.contiguous() : Tensor();
     const int64_t B = px.size(0), S = px.size(1), T1 = px.size(2), T = py.size(2);
+    ctx->set_materialize_grads(false);
     DeviceGuard guard(px.device());
     const auto opts = px.options();
     Tensor p = at::empty({B, S + 1, T + 1}, opts), scores = at::empty({B}, opts);
@@ -403,6 +404,7 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    if (!grads[0].defined()) return variable_list(5);
     const auto saved = ctx->get_saved_variables();
     Tensor gx = saved[0], gy = saved[1];
     const int64_t B = gx.size(0), S = gx.size(1), T1 = gx.size(2), T = gy.size(2);

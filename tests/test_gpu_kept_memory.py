@@ -30,3 +30,18 @@ def test_memory_kept_for_the_backward(gpu_device, path):
     # (the allocator hands out multiples of 512 bytes)
     assert torch.cuda.memory_allocated() - before <= 4 * (norm + px_grad + py_grad) + 4 * 512
     kept.backward()
+
+
+def test_backward_of_the_recursion_allocates_no_lattices(gpu_device):
+    B, S, T = 4, 60, 300
+    g = torch.Generator().manual_seed(1)
+    px = torch.randn(B, S, T + 1, generator=g).to(gpu_device).requires_grad_(True)
+    py = torch.randn(B, S + 1, T, generator=g).to(gpu_device).requires_grad_(True)
+    scores, occupation = fast_rnnt_amd.mutual_information_recursion(px, py, return_grad=True)
+    total = scores.sum()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    grads = torch.autograd.grad(total, (px, py))
+    assert torch.cuda.max_memory_allocated() - before < occupation[0].numel() * 4
+    assert all(torch.equal(a, b) for a, b in zip(grads, occupation))
