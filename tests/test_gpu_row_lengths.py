@@ -48,3 +48,43 @@ def test_loss_on_logits_of_any_row_length(gpu_device, dtype, C):
         (3.0 * got).backward()
         off = (gpu.grad.float().cpu() - cpu.grad).abs()
         assert bool((off <= 1e-4 + ULP[dtype] * cpu.grad.abs()).all()), off.max().item()
+
+
+# vocabularies (in 16-byte pieces) on either side of every split of a row
+PIECES = [1, 15, 16, 17, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 512, 513, 640, 641,
+          896, 897, 1280, 1281]
+
+
+@pytest.mark.parametrize("sfx,dtype", [("f32", torch.float32), ("f16", torch.float16),
+                                       ("bf16", torch.bfloat16)])
+def test_gradients_of_aligned_rows_are_the_bits_of_any_others(gpu_device, sfx, dtype):
+    # the same rows through the kernel for rows that begin and end on 16 bytes, the one for any
+    # alignment (logits and gradients one element off) and the one without pieces (one of them off)
+    from fast_rnnt_amd import _lib
+    B, S, T, R = 2, 5, 6, 3
+    g = torch.Generator().manual_seed(9)
+    T1 = T + 1
+    symbols = torch.randint(0, 4, (B, S), generator=g).to(gpu_device)
+    boundary = torch.tensor([[0, 0, S, T], [0, 1, S - 1, T - 1]]).to(gpu_device)
+    ranges = (torch.tensor([0, 0, 1, 2, 3, 3]).reshape(1, T, 1) + torch.arange(R)).expand(B, T, R)
+    ranges = ranges.contiguous().to(gpu_device)
+    gx = torch.rand(B, S, T1, generator=g).to(gpu_device)
+    gy = torch.rand(B, S + 1, T, generator=g).to(gpu_device)
+    for pieces in PIECES:
+        C = pieces * (16 // dtype.itemsize)
+        n = B * T * R * C
+        values = (2 * torch.randn(n, generator=g)).to(dtype).to(gpu_device)
+        norm = torch.logsumexp(values.reshape(B * T * R, C).float(), 1)
+        results = []
+        for in_off, out_off in ((0, 0), (1, 1), (1, 0)):
+            print(f"{dtype} C={C} offsets {in_off} {out_off}", flush=True)
+            logits = torch.zeros(n + 8, dtype=dtype, device=gpu_device)
+            logits[in_off:in_off + n] = values
+            out = torch.full((n + 8,), 7.0, dtype=dtype, device=gpu_device)
+            _lib.call("frnnt_lattice_logprobs_bwd_" + sfx, logits[in_off:].data_ptr(),
+                      symbols.data_ptr(), ranges.data_ptr(), boundary.data_ptr(), norm.data_ptr(),
+                      gx.data_ptr(), gy.data_ptr(), out[out_off:].data_ptr(), B, S, T, R, C, 3, 0, 1,
+                      _lib.stream_of(out))
+            assert bool((out[:out_off] == 7).all()) and bool((out[out_off + n:] == 7).all())
+            results.append(out[out_off:out_off + n])
+        assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
