@@ -1094,9 +1094,11 @@ void launch_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
                     const SmoothTerms &smooth, hipStream_t stream) {
   const long columns = (long)B * ((C + kProdC - 1) / kProdC);
   // Where lm, am and their gradients together outgrow the last-level cache (256 MB) the gradients
-  // are streamed past it, which leaves it to lm and am: these are read by both products.  (Whole
-  // pass of the loss, B 16, S 120, T 400, C 5000, 334 MB: 300 -> 295 us; B 64, S 120, T 600,
-  // C 500, 185 MB: 266 -> 267.)
+  // are streamed past it, which leaves it to lm and am: these are read by both products.  Whole pass
+  // of the loss, with the hint against without: C 5000, S 120, T 400: B 14, 278 MB: 291 / 299 us;
+  // B 24, 476 MB: 452 / 476; B 64, S 120, T 600, C 1000, 352 MB: 424 / 444; C 500, B 128, 352 MB:
+  // 545 / 547; B 8, S 200, T 1000, C 5000, 366 MB: 558 / 589.  Below, either way: B 10, C 5000,
+  // 198 MB: 267 / 263; B 32, S 60, T 300, C 2500, 220 MB: 188 / 188; B 45, C 1000, 247 MB: 320 / 327.
   if (out_type == FRNNT_F32 && 8L * B * (S + 1 + T) * C > (256L << 20)) out_type = kStreamed;
   const bool wide_l = wide_tile(columns, S + 1), wide_a = wide_tile(columns, T);
   auto launch = wide_l ? wide_a ? launch_bwd_t<128, 128, kSmooth> : launch_bwd_t<128, 64, kSmooth>

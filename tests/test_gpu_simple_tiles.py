@@ -80,3 +80,22 @@ def test_normalizers_are_the_same_bits_in_tiles_of_any_height(gpu_device, S, T, 
     want_x = joint[:S].gather(2, symbols[0].cpu().reshape(S, 1, 1).expand(S, T, 1)).squeeze(2) - norm[:S]
     for got, want in ((px, want_x), (py, want_y)):
         assert bool(((got - want).abs() <= 2e-6 * want.abs().clamp(min=1) + 2e-5).all())
+
+
+def test_gradients_that_are_streamed_past_the_cache(gpu_device):
+    # lm, am and their gradients take 278 MB together, more than the last-level cache: the gradients
+    # are stored with another hint than those of the two halves of the batch
+    B, S, T, C = 14, 120, 400, 5000
+    g = torch.Generator(device=gpu_device).manual_seed(2)
+    lm = torch.randn(B, S + 1, C, generator=g, device=gpu_device)
+    am = torch.randn(B, T, C, generator=g, device=gpu_device)
+    symbols = torch.randint(1, C, (B, S), generator=g, device=gpu_device)
+
+    def grads(rows):
+        leaves = [x[rows].clone().requires_grad_(True) for x in (lm, am)]
+        fast_rnnt_amd.rnnt_loss_simple(*leaves, symbols[rows], 0, reduction="sum").backward()
+        return [x.grad for x in leaves]
+
+    whole, halves = grads(slice(0, B)), [grads(slice(0, 7)), grads(slice(7, B))]
+    for i in range(2):
+        assert torch.equal(whole[i], torch.cat([h[i] for h in halves]))
