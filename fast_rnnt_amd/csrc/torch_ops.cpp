@@ -1053,15 +1053,16 @@ variable_list GatherRowsFn::backward(AutogradContext *ctx, variable_list grads) 
 // joiner that follows adds the two -- once.  A backward that is to be differentiated itself takes
 // the two adjoints as nodes of their own.
 struct PruningFn : public torch::autograd::Function<PruningFn> {
-  static variable_list forward(AutogradContext *ctx, const Tensor &am, const Tensor &lm_,
+  static variable_list forward(AutogradContext *ctx, const Tensor &, const Tensor &lm_,
                                const Tensor &ranges) {
     DeviceGuard guard(lm_.device());
     const Tensor lm = lm_.contiguous(), rng = ranges.contiguous();
-    const int64_t B = rng.size(0), T = rng.size(1), R = rng.size(2), C = lm.size(2);
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({rng});
     ctx->saved_data["rows"] = lm.size(1);
-    return {am.unsqueeze(2).expand({B, T, R, C}), gather_rows(lm, rng)};
+    const Tensor rows = gather_rows(lm, rng);
+    // (the first output stands for am_pruned: its sizes and type, not its values -- see pruning)
+    return {rows.detach(), rows};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
@@ -1106,15 +1107,18 @@ std::tuple<Tensor, Tensor> pruning(const Tensor &am, const Tensor &lm, const Ten
   TORCH_CHECK(am.device() == lm.device() && ranges.device() == lm.device() &&
                   am.scalar_type() == lm.scalar_type() && ranges.scalar_type() == at::kLong,
               "am and lm must share a device and a type, ranges be int64 on that device");
-  // (a tangent of am passes through the view, which the node does not know; with one kept position
-  // am_pruned may be written to, which is not allowed for a view that a node of two outputs returns)
-  if (at::GradMode::is_enabled() && am.requires_grad() && lm.requires_grad() &&
-      am.size(2) == lm.size(2) && ranges.size(2) > 1 && !am._fw_grad(/*level=*/0).defined()) {
-    const variable_list out = PruningFn::apply(am, lm, ranges);
-    return {out[0], out[1]};
-  }
-  return {am.unsqueeze(2).expand({am.size(0), am.size(1), ranges.size(2), lm.size(2)}),
-          GatherRowsFn::apply(lm, ranges)};
+  const Tensor am_pruned =
+      am.unsqueeze(2).expand({am.size(0), am.size(1), ranges.size(2), lm.size(2)});
+  // (a tangent of am passes through the view and would be refused by the node)
+  if (!at::GradMode::is_enabled() || !am.requires_grad() || !lm.requires_grad() ||
+      am.size(2) != lm.size(2) || am._fw_grad(/*level=*/0).defined())
+    return {am_pruned, GatherRowsFn::apply(lm, ranges)};
+  // The view stays the plain one, which autograd follows when am or the view itself is written to
+  // (a view that a node returns is refused then); only its gradient goes to the node.
+  const variable_list out = PruningFn::apply(am, lm, ranges);
+  torch::autograd::impl::set_gradient_edge(
+      am_pruned, {out[0].grad_fn(), static_cast<uint32_t>(out[0].output_nr())});
+  return {am_pruned, out[1]};
 }
 
 void set_deferred_checks(bool on) { g_deferred = on; }

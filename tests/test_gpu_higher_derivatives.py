@@ -55,6 +55,43 @@ def test_one_kept_position_may_be_written_to(gpu_device):
     assert torch.equal(am.grad, torch.full_like(am, 2.0))
 
 
+@pytest.mark.parametrize("R", [1, 3])
+def test_am_may_be_written_to_after_the_pruning(gpu_device, R):
+    am, lm, ranges = _pruning_inputs(gpu_device, R)
+    weights = torch.randn(2, 6, R, 4, dtype=am.dtype, device=gpu_device)
+    # a parameter that is updated in between
+    am_pruned, lm_pruned = fast_rnnt_amd.do_rnnt_pruning(am, lm, ranges)
+    with torch.no_grad():
+        am.add_(1)
+    assert torch.equal(am_pruned, am.unsqueeze(2).expand(2, 6, R, 4))
+    (weights * (am_pruned + lm_pruned)).sum().backward()
+    assert torch.allclose(am.grad, weights.sum(2), rtol=1e-12, atol=1e-12)
+    # an activation that is changed on record: what am_pruned shows of it is differentiated too
+    results = []
+    for prune in (True, False):
+        x, y = am.detach().clone().requires_grad_(True), lm.detach().clone().requires_grad_(True)
+        hidden = x * 3
+        if prune:
+            kept = fast_rnnt_amd.do_rnnt_pruning(hidden, y, ranges)
+        else:
+            rows = ranges.reshape(2, -1, 1).expand(2, 6 * R, 4)
+            kept = (hidden.unsqueeze(2).expand(2, 6, R, 4),
+                    torch.gather(y, 1, rows).reshape(2, 6, R, 4))
+        hidden.mul_(2)
+        kept[1].add_(kept[0])  # a joiner that adds in place
+        (weights * torch.tanh(kept[1])).sum().backward()
+        results.append((x.grad, y.grad))
+    for a, b in zip(*results):
+        assert torch.allclose(a, b, rtol=1e-12, atol=1e-12)
+    # a tensor that a later operation has kept: refused, as with torch's own view
+    hidden = am * 1
+    am_pruned, lm_pruned = fast_rnnt_amd.do_rnnt_pruning(hidden, lm, ranges)
+    out = (am_pruned * lm_pruned).sum()
+    hidden.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_gradients_of_the_recursion_keep_the_history_of_the_scores_gradient(gpu_device, dtype):
     g = torch.Generator().manual_seed(3)
