@@ -289,6 +289,14 @@ bool with_cuda() { return true; }
 // with the reduction's sign and 1/B folded in.
 constexpr int kRedNone = 0, kRedMean = 1;
 
+// The occupation gradients of a node that has scaled them in place: a second backward through it
+// (retain_graph=True) finds its saved tensors changed and raises, as after torch's own "*=" in
+// mutual_information.py:179-180, instead of scaling them twice.
+void count_as_changed(const Tensor &gx, const Tensor &gy) {
+  gx.unsafeGetTensorImpl()->bump_version();
+  gy.unsafeGetTensorImpl()->bump_version();
+}
+
 // element offsets of consecutive buffers, each 16-byte aligned for 4- and 8-byte elements
 struct Carver {
   int64_t total = 0;
@@ -363,6 +371,7 @@ struct RecursionLossFn : public torch::autograd::Function<RecursionLossFn> {
       rc = abi_mi_scale_grads(ptr<double>(gx), ptr<double>(gy), ptr<double>(g), stride, scale,
                               (int)B, (int)S, (int)T, (int)(T1 == T), stream_of(gx));
     check_rc(rc, "frnnt_mi_scale_grads");
+    count_as_changed(gx, gy);
     out[0] = gx;
     out[1] = gy;
     return out;
@@ -421,9 +430,7 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
                                 (int)(T1 == T), stream_of(gx));
     };
     check_rc(gx.scalar_type() == at::kFloat ? run(float()) : run(double()), "frnnt_mi_scale_grads");
-    // (a second backward through the node finds them changed, as it would after torch's own "*=")
-    gx.unsafeGetTensorImpl()->bump_version();
-    gy.unsafeGetTensorImpl()->bump_version();
+    count_as_changed(gx, gy);
     return {gx, gy, Tensor(), Tensor(), Tensor()};
   }
 };
@@ -600,6 +607,7 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
                  meta[3] ? out[0].data_ptr() : nullptr, meta[4] ? out[1].data_ptr() : nullptr,
                  (int)B, (int)S, (int)T, (int)C, (int)meta[0], (int)meta[1], stream_of(am)),
              "frnnt_additive_loss_bwd");
+    count_as_changed(gx, gy);
     return out;
   }
 };
@@ -717,6 +725,7 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
                  ptr<float>(scratch), ptr<float>(out[0]), ptr<float>(out[1]), (int)B, (int)S, (int)T,
                  (int)C, (int)meta[0], (int)meta[1], scales[0], scales[1], stream_of(am)),
              "frnnt_smoothed_loss_bwd");
+    count_as_changed(gx, gy);
     return out;
   }
 };
@@ -880,10 +889,12 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
     const double scale = reduction == kRedMean ? -1.0 / (double)B : -1.0;
     void *stream = stream_of(logits);
     const bool handed_out = meta[5] != 0;
-    if (handed_out)
+    if (handed_out) {
       check_rc(abi_mi_scale_grads(ptr<R>(gx), ptr<R>(gy), ptr<R>(g), stride, scale, (int)B, (int)S,
                                   (int)T, (int)(kind != 0), stream),
                "frnnt_mi_scale_grads");
+      count_as_changed(gx, gy);
+    }
     Tensor grad = at::empty(logits.sizes(), logits.options());
     check_rc(abi_lattice_loss_bwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
                                   iptr(bnd), ptr<R>(norm),

@@ -108,3 +108,28 @@ def test_gradients_of_the_recursion_keep_the_history_of_the_scores_gradient(gpu_
     (gx.sum() + gy.square().sum()).backward()
     want = occ_x.sum((1, 2)) + 2 * weights.detach() * occ_y.square().sum((1, 2))
     assert torch.allclose(weights.grad, want, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("return_grad", [False, True])
+@pytest.mark.parametrize("path", ["simple", "smoothed", "smoothed_constrained", "joint"])
+def test_a_second_backward_is_right_or_refused(gpu_device, path, return_grad):
+    g = torch.Generator().manual_seed(4)
+    B, S, T, C = 2, 4, 7, 5
+    symbols = torch.randint(1, C, (B, S), generator=g).to(gpu_device)
+    if path == "joint":
+        leaves = [torch.randn(B, T, S + 1, C, generator=g)]
+    else:
+        leaves = [torch.randn(B, S + 1, C, generator=g), torch.randn(B, T, C, generator=g)]
+    leaves = [x.to(gpu_device).requires_grad_(True) for x in leaves]
+    kind = "constrained" if path == "smoothed_constrained" else "regular"
+    loss_fn = {"simple": fast_rnnt_amd.rnnt_loss_simple, "joint": fast_rnnt_amd.rnnt_loss,
+               "smoothed": fast_rnnt_amd.rnnt_loss_smoothed,
+               "smoothed_constrained": fast_rnnt_amd.rnnt_loss_smoothed}[path]
+    loss = loss_fn(*leaves, symbols, 0, rnnt_type=kind, reduction="mean", return_grad=return_grad)
+    loss = loss[0] if return_grad else loss
+    first = torch.autograd.grad(loss, leaves, retain_graph=True)
+    if path == "joint" and not return_grad:  # (nothing is scaled in place)
+        assert all(torch.equal(a, b) for a, b in zip(first, torch.autograd.grad(loss, leaves)))
+    else:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(loss, leaves)
