@@ -65,9 +65,9 @@ constexpr int kSeamSlack = kSeamPadLeft + kSeamPad;
 constexpr int kFwdStagers = 3;         // staging waves per sweep wave
 constexpr int kBwdStagers = 3;
 // With at most two sweep waves a workgroup has room for more staging waves per sweep wave.
-// The backward kernel's evaluate d1 / d2 and are what its sweep waves wait for (c2 shape:
-// 17.2 us with 6, 16.9 with 7: 16 waves, the most a workgroup holds); the forward kernel's
-// only copy (18.45 us with 2, 18.05 with 3, 17.9 with 4).
+// The backward kernel's evaluate d1 / d2 and are what its sweep waves wait for (B 32, S 80, T 250,
+// when a launch took 17 us: 17.2 us with 6, 16.9 with 7: 16 waves, the most a workgroup holds); the
+// forward kernel's only copy (then 18.45 us with 2, 18.05 with 3, 17.9 with 4).
 constexpr int kFwdStagersFew = 4;
 constexpr int kBwdStagersFew = 7;
 constexpr int kSpinLimit = 1 << 22;   // polls before a wait gives up (seconds, not microseconds)
@@ -324,8 +324,10 @@ __device__ __forceinline__ PlainTiles plain_tiles(const Band &g, int fin_step, b
 // holds it puts it into LDS as soon as a tile is done, a courier wave stores it, and one of the next
 // band's workgroup polls it, value by value: the row has been filled with a mark beforehand
 // (mark_seams_kernel), a signalling NaN, which no arithmetic instruction ever returns.  The
-// values are stored and loaded with agent scope, past the XCDs' own L2.  Producers have the
-// lower block numbers, so they are running or done before a consumer starts.
+// values are stored and loaded with agent scope, past the XCDs' own L2.  The workgroups of a
+// launch need not all be resident: an utterance's bands run on one XCD, producers have the lower
+// block numbers, and an XCD starts its workgroups in their order, so that a producer is running or
+// done before its consumer starts.
 constexpr int kSeamMark = 0x7fa5a5a5;
 // What a courier wave of a band does: takes the seam's `total` values from memory -- value c at
 // from + c * stride -- to the seam row in LDS as they arrive, and counts them in.  A wave of its
@@ -696,11 +698,10 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     // the counter is read one tile ahead of its use, so that the LDS round trip is off the
     // chain; a stale value only costs a re-read
     int seen_loaded = 0;
-    // One tile, specialised at compile time on whether the wave feeds a seam (kDown), and on
-    // kPlain: a tile whose 32 steps all exist and do not hold the answer's step.  A single
-    // wave pays for every instruction it issues, scalar tests and branches included, so
-    // plain tiles run without the tests; and every kind of tile has a loop of its own (see
-    // sweep_tiles): with all kinds in one loop body the compiler's code for the steps
+    // One tile, specialised at compile time on kPlain: a tile whose 32 steps all exist and do
+    // not hold the answer's step.  A single wave pays for every instruction it issues, scalar
+    // tests and branches included, so plain tiles run without the tests; and either kind of tile
+    // has a loop of its own (below): with both in one loop body the compiler's code for the steps
     // themselves took twice as long.
     auto one_tile = [&](int m, auto plain_c) __attribute__((always_inline)) -> bool {
       constexpr bool kPlain = decltype(plain_c)::value;
@@ -1156,7 +1157,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     int seen_ready = 0;
     R seen_seam = 0;
     int seen_loaded = 0;
-    // one tile; the compile-time flags and the loops are those of the forward kernel
+    // one tile, specialised at compile time on whether the wave takes from a seam (kUp) and feeds
+    // one (kDown), and on kPlain, with a loop for each kind, for the forward kernel's reasons
     auto one_tile = [&](int m, auto up_c, auto down_c, auto plain_c) __attribute__((always_inline)) -> bool {
       constexpr bool kUp = decltype(up_c)::value;
       constexpr bool kDown = decltype(down_c)::value;
@@ -1191,7 +1193,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
           const int need = kPlain ? e0 + kChunk - shift : min(e0 + kChunk - shift, cols);
           handed = seen_seam;
           if ((kPlain || need > 0) && __builtin_amdgcn_readfirstlane(seen_ready) < up_base + need) {
-            // (a wait that has run out is not tried again, see the forward kernel)
+            // (a wait that has run out is not tried again: the tile is finished on whatever the
+            // seam holds, and the wave gives up afterwards)
             if (!failed && !wait_for(&cnt.ready[prev], up_base + need, spin_limit)) failed = true;
             const int col = e0 + lane - shift;
             handed = (lane < kChunk && col >= 0 && col <= NT) ? up_seam[col] : (R)0;

@@ -824,34 +824,40 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
     ctx->set_materialize_grads(false);
     DeviceGuard guard(logits.device());
     const auto opts = logits.options().dtype(c10::CppTypeToScalarType<R>::value);
-    // internal buffers in one allocation: px | py | xr | yr | p | scores | norm, unless a backward
-    // will read it, which keeps norm alone
+    const int64_t n_px = B * S * T1, n_py = B * (S + 1) * T;
+    // what the backward reads besides its inputs, in one allocation: norm | px_grad | py_grad, the
+    // latter two unless they are handed out
+    Carver keep;
+    const int64_t o_nr = keep.take(B * T * K), o_gx = keep.take(want_grads ? 0 : n_px),
+                  o_gy = keep.take(want_grads ? 0 : n_py);
+    const Tensor kept = need_grad ? at::empty({keep.total}, opts) : Tensor();
+    // what it does not: px | py | xr | yr | p | scores (and norm, without a backward)
     Carver carve;
-    const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(B * (S + 1) * T),
-                  o_xr = carve.take(B * T * K), o_yr = carve.take(B * T * K),
-                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B),
-                  o_nr = carve.take(need_grad ? 0 : B * T * K);
+    const int64_t o_px = carve.take(n_px), o_py = carve.take(n_py), o_xr = carve.take(B * T * K),
+                  o_yr = carve.take(B * T * K), o_p = carve.take(B * (S + 1) * (T + 1)),
+                  o_sc = carve.take(B), o_unkept = carve.take(need_grad ? 0 : B * T * K);
     const Tensor work = at::empty({carve.total}, opts);
-    const Tensor norm = need_grad ? at::empty({B * T * K}, opts) : Tensor();
-    R *w = work.data_ptr<R>(), *nr = need_grad ? ptr<R>(norm) : w + o_nr;
+    R *w = work.data_ptr<R>(), *k = ptr<R>(kept);
     Tensor gx, gy;
-    if (want_grads || need_grad) {
+    if (want_grads) {
       gx = at::empty({B, S, T1}, opts);
       gy = at::empty({B, S + 1, T}, opts);
     }
+    R *p_gx = want_grads ? ptr<R>(gx) : need_grad ? k + o_gx : nullptr;
+    R *p_gy = want_grads ? ptr<R>(gy) : need_grad ? k + o_gy : nullptr;
     Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
     check_rc(abi_lattice_loss_fwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
-                                  iptr(bnd), w + o_px, w + o_py, nr, w + o_xr, w + o_yr, w + o_p,
-                                  w + o_sc, ptr<R>(gx), ptr<R>(gy), ptr<R>(loss), (int)B,
-                                  (int)S, (int)T, (int)K, (int)C, (int)term, (int)kind,
+                                  iptr(bnd), w + o_px, w + o_py, need_grad ? k + o_nr : w + o_unkept,
+                                  w + o_xr, w + o_yr, w + o_p, w + o_sc, p_gx, p_gy, ptr<R>(loss),
+                                  (int)B, (int)S, (int)T, (int)K, (int)C, (int)term, (int)kind,
                                   delay_penalty > 0.0 ? delay_penalty : 0.0, (int)reduction,
                                   (int)checks, status_for(logits, bnd), stream_of(logits)),
              "frnnt_lattice_loss_fwd");
     if (need_grad) {
       // (absent tensors are not saved: saved tensors must be defined)
-      variable_list save{logits, sym, norm, gx, gy};
-      if (rng.defined()) save.push_back(rng);
-      if (bnd.defined()) save.push_back(bnd);
+      variable_list save{logits, sym, kept};
+      for (const Tensor &t : {rng, bnd, gx, gy})
+        if (t.defined()) save.push_back(t);
       ctx->save_for_backward(std::move(save));
       ctx->saved_data["meta"] =
           std::vector<int64_t>{term, kind, reduction, rng.defined(), bnd.defined(), want_grads};
@@ -875,12 +881,12 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
   template <typename R>
   static Tensor run_backward(AutogradContext *ctx, const variable_list &saved,
                              const Tensor &g_loss) {
-    const Tensor &logits = saved[0], &sym = saved[1], &norm = saved[2];
-    Tensor gx = saved[3], gy = saved[4];
+    const Tensor &logits = saved[0], &sym = saved[1], &kept = saved[2];
     const std::vector<int64_t> meta = ctx->saved_data["meta"].toIntVector();
     const int64_t kind = meta[1], reduction = meta[2];
-    const Tensor rng = meta[3] ? saved[5] : Tensor();
-    const Tensor bnd = meta[4] ? saved[5 + meta[3]] : Tensor();
+    const Tensor rng = meta[3] ? saved[3] : Tensor();
+    const Tensor bnd = meta[4] ? saved[3 + meta[3]] : Tensor();
+    const bool handed_out = meta[5] != 0;
     const int64_t B = logits.size(0), T = logits.size(1), K = logits.size(2), C = logits.size(3),
                   S = sym.size(1);
     DeviceGuard guard(logits.device());
@@ -888,18 +894,24 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
     const int stride = reduction == kRedNone ? 1 : 0;
     const double scale = reduction == kRedMean ? -1.0 / (double)B : -1.0;
     void *stream = stream_of(logits);
-    const bool handed_out = meta[5] != 0;
+    // (the forward's layout)
+    Carver keep;
+    const int64_t o_nr = keep.take(B * T * K),
+                  o_gx = keep.take(handed_out ? 0 : B * S * (kind == 0 ? T + 1 : T)),
+                  o_gy = keep.take(handed_out ? 0 : B * (S + 1) * T);
+    R *k = ptr<R>(kept), *gx = k + o_gx, *gy = k + o_gy;
     if (handed_out) {
-      check_rc(abi_mi_scale_grads(ptr<R>(gx), ptr<R>(gy), ptr<R>(g), stride, scale, (int)B, (int)S,
-                                  (int)T, (int)(kind != 0), stream),
+      const Tensor &t_gx = saved[3 + meta[3] + meta[4]], &t_gy = saved[4 + meta[3] + meta[4]];
+      gx = ptr<R>(t_gx), gy = ptr<R>(t_gy);
+      check_rc(abi_mi_scale_grads(gx, gy, ptr<R>(g), stride, scale, (int)B, (int)S, (int)T,
+                                  (int)(kind != 0), stream),
                "frnnt_mi_scale_grads");
-      count_as_changed(gx, gy);
+      count_as_changed(t_gx, t_gy);
     }
     Tensor grad = at::empty(logits.sizes(), logits.options());
     check_rc(abi_lattice_loss_bwd(logits.scalar_type(), logits.data_ptr(), iptr(sym), iptr(rng),
-                                  iptr(bnd), ptr<R>(norm),
-                                  handed_out ? (const R *)nullptr : ptr<R>(g), stride, scale,
-                                  ptr<R>(gx), ptr<R>(gy), grad.data_ptr(), (int)B, (int)S, (int)T,
+                                  iptr(bnd), k + o_nr, handed_out ? (const R *)nullptr : ptr<R>(g),
+                                  stride, scale, gx, gy, grad.data_ptr(), (int)B, (int)S, (int)T,
                                   (int)K, (int)C, (int)meta[0], (int)kind, stream),
              "frnnt_lattice_loss_bwd");
     return grad;

@@ -1,7 +1,7 @@
-"""The row kernels of the losses on logits (csrc/lattice_logprobs.hip) where their split of a row
-over lanes and 16-byte pieces can go wrong: vocabularies on either side of every split (a quarter,
-a half, a whole wave per row, 2 ... 20 pieces per lane, rows in chunks), rows that share a
-piece with their neighbours, logits that begin off a 16-byte boundary.  Oracle: the CPU
+"""The row kernels of the losses on logits (csrc/lattice_logprobs.hip, lattice_gradient.hip) where
+their split of a row over lanes and 16-byte pieces can go wrong: vocabularies on either side of every
+split (a quarter, a half, a whole wave per row, 2 ... 20 pieces per lane, rows in chunks), rows that
+share a piece with their neighbours, logits that begin off a 16-byte boundary.  Oracle: the CPU
 restatement on the same values in float32."""
 import pytest
 import torch
