@@ -455,7 +455,8 @@ def _bench_lattice(args, w, dev):
                   in_bytes + nbytes, t_b, padded_bytes=2 * nbytes),
         _hbm_line(table, "row_norm_kernel",
                   in_bytes, t_f, padded_bytes=nbytes,
-                  note="launch time includes the small assemble_kernel of the same entry point"),
+                  **({} if ranges is None else {"note": "launch time includes the small "
+                                                "assemble_kernel of the same entry point"})),
     ]
     lines.sort(key=lambda r: -r["avg_launch_us"])
     eager = _rate(args.steps, elapsed)
