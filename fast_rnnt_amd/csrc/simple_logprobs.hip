@@ -75,28 +75,49 @@ inline int part_shift_for(int B, int c_tiles) {
   while ((B << shift) < 64 && (8 << shift) <= c_tiles) ++shift;
   return shift;
 }
-inline unsigned placed_grid(int c_tiles, int other_tiles, int B, int part_shift) {
-  const long units = (long)B << part_shift;
-  const int c_per = (c_tiles + (1 << part_shift) - 1) >> part_shift;
-  return (unsigned)(dgemm::kXcds * ((units + dgemm::kXcds - 1) / dgemm::kXcds) * c_per * other_tiles);
-}
-// (utterance, tile, window) of workgroup `id` of a grid of placed_grid() workgroups; a tile is
-// other * c_tiles + (its index along the vocabulary)
-__device__ __forceinline__ bool place_block(int id, int c_tiles, int other_tiles, int part_shift,
-                                            int B, const float *row_x, const int64_t *window, int S,
-                                            int T, int &b, int &tile, Limits &lim) {
+// n / d for n < 2^32, the reciprocal made on the host (the round-up method of Granlund and
+// Montgomery): a multiplication and three more scalar instructions instead of the compiler's thirty.
+struct Divisor {
+  unsigned d, reciprocal, shift1, shift2;
+  explicit Divisor(unsigned d_) : d(d_) {
+    unsigned l = 0;
+    while (l < 32 && (1ull << l) < d) ++l;
+    reciprocal = (unsigned)((((1ull << l) - d) << 32) / d + 1);
+    shift1 = l < 1 ? l : 1, shift2 = l < 1 ? 0 : l - 1;
+  }
+  __device__ __forceinline__ unsigned divide(unsigned n) const {
+    const unsigned t = __umulhi(reciprocal, n);
+    return (t + ((n - t) >> shift1)) >> shift2;
+  }
+};
+// One product's share of the grid: its tiles of c_per stretches of the vocabulary, rows of tiles
+// outermost, for the units of one XCD one after the other.
+struct Placement {
+  Divisor c_per, unit_tiles;
+  int c_tiles, part_shift;
+  unsigned blocks;
+  Placement(int c_tiles_, int row_tiles, int B, int part_shift_)
+      : c_per((c_tiles_ + (1 << part_shift_) - 1) >> part_shift_),
+        unit_tiles(row_tiles > 0 ? c_per.d * row_tiles : 1), c_tiles(c_tiles_), part_shift(part_shift_) {
+    const long units = (long)B << part_shift;
+    blocks = row_tiles > 0
+                 ? (unsigned)(dgemm::kXcds * ((units + dgemm::kXcds - 1) / dgemm::kXcds) * unit_tiles.d)
+                 : 0;
+  }
+};
+// (utterance, row of tiles, tile along the vocabulary) of workgroup `id`
+__device__ __forceinline__ bool place_block(unsigned id, const Placement &at, int B,
+                                            const float *row_x, int S, int &b, int &row_idx,
+                                            int &c_idx) {
   using dgemm::kXcds;
-  const int c_per = (c_tiles + (1 << part_shift) - 1) >> part_shift;
-  const int unit_tiles = c_per * other_tiles;
-  const int xcd = id % kXcds, slot = id / kXcds, round = slot / unit_tiles;
-  const int within = slot - round * unit_tiles;
+  const unsigned xcd = id % kXcds, slot = id / kXcds, round = at.unit_tiles.divide(slot);
+  const unsigned within = slot - round * at.unit_tiles.d;
   const int unit = round * kXcds + ((round & 1) ? kXcds - 1 - xcd : xcd);
-  const int rank = unit >> part_shift, part = unit & ((1 << part_shift) - 1);
-  const int other = within / c_per, c_idx = part * c_per + (within - other * c_per);
-  if (rank >= B || c_idx >= c_tiles) return false;
-  tile = other * c_tiles + c_idx;
+  const int rank = unit >> at.part_shift, part = unit & ((1 << at.part_shift) - 1);
+  row_idx = at.c_per.divide(within);
+  c_idx = part * at.c_per.d + (within - row_idx * at.c_per.d);
+  if (rank >= B || c_idx >= at.c_tiles) return false;
   b = *reinterpret_cast<const int *>(row_x + (long)rank * (S + 1) + S);
-  lim = limits_of(window, b, S, T);
   return true;
 }
 
@@ -322,7 +343,7 @@ __global__ void __launch_bounds__(256)
         }
         gx[u] = ok && t != t_mask ? gx[u] * joint : (R)0;
         gy[u] = ok ? gy[u] * joint : (R)0;
-        if (t < T) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
+        if (t < ldd) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
         sx += gx[u];
         sy += gy[u];
       }
@@ -474,74 +495,61 @@ __global__ void __launch_bounds__(256)
 // ---- float32 gradient products on the bfloat16 matrix cores ----------------------------------
 //   lm.grad[s,c] = exp(lm[s,c] - max[s]) * sum_t D[s,t] exp(am[t,c] - max[t]) + one-hots
 //   am.grad[t,c] = exp(am[t,c] - max[t]) * sum_s D[s,t] exp(lm[s,c] - max[s]) + one-hots
-// A workgroup of four waves takes kM rows (lattice rows of lm.grad, frames of am.grad) x kC
-// vocabulary entries, a wave kM / 2 x kC / 2 of them as 32 x 32 accumulators.  k (frames, lattice
-// rows) runs in chunks of 32: the 256 threads fetch a chunk of both operands, apply exp to
-// the one that needs it, split the values into bfloat16 parts (Split8) and write them to LDS as
-// [k-step][row or entry][part][16 k]; after a barrier every wave reads its operands from there.
-// Where an operand lies k-major in memory (am and lm always, D for am.grad) a thread takes eight
-// consecutive k of one column -- loads that are contiguous over the lanes -- and has its
-// 16-byte piece of the operand without any transposition.
-// Four workgroups share a compute unit (37 KB of LDS, 128 registers each): while one waits for
-// memory, at a barrier or for its epilogue the others convert or multiply; one alone takes 1 us per
-// chunk, a full compute unit 1.6 us for four.  What bounds them then is no unit alone but that their
-// phases hardly overlap: of a compute unit's cycles (counters, B 16, S 120, T 400, C 5000) the VALU
-// issues in 55 % (about 26 cycles per 64 operand elements for exp and split), LDS moves data in 40 %,
-// a third of them bank conflicts, and the matrix cores work in 28 %.
-// Measured (both products): B 32, S 80, T 250, C 500: 29 us with the float32 matrix instruction,
-// 24 here; B 64, S 120, T 600, C 500: 119 and 79; B 16, S 120, T 400, C 5000: 202 and 134.
+// A workgroup of four waves takes kM rows (lattice rows of lm.grad, frames of am.grad) x 64
+// vocabulary entries, a wave 32 rows x 64 or 32 of them as 32 x 32 accumulators.  k (frames, lattice
+// rows) runs in chunks of 32.  D belongs to one wave's rows: it goes from memory straight
+// into the lanes that multiply it and is split into bfloat16 parts (split_pair) there.  The
+// operand along the vocabulary is shared: a thread fetches eight consecutive k of one entry, loads
+// that are contiguous over the lanes, takes exp, splits, and has its 16-byte piece of the operand
+// without any transposition; the pieces lie in LDS as [octet of k][part][entry], where consecutive
+// lanes write and read consecutive pieces.  Two such images alternate: a chunk is staged while the
+// one before it is multiplied, one barrier per chunk.
+// What bounds it: instructions issued.  Of 250 000 cycles per SIMD (counters, B 16, S 120, T 400,
+// C 5000, the matrix cores busy for 71 000) almost every group of four issues one.  Taking 12
+// million of 21 million scalar instructions out (offsets made once instead of per load, reciprocals
+// instead of divisions, a list that ends with its last hit) took 116 to 108 us, while the same kernel
+// without any loads of D takes 104, with fewer and wider tiles (128 entries: 110), with its L2
+// requests down by 15 % (eight waves, 128 entries: 130) or with its reads of HBM down by a third
+// (the tiles of both products that read the same entries side by side: 119) gains nothing.
+// Measured (both products; B 32, S 80, T 250, C 500 / B 64, S 120, T 600, C 500 / B 16, S 120, T 400,
+// C 5000): 23.5 / 83 / 124 us when both operands went through one LDS image, 20 / 72.5 / 108 now.
 constexpr int kProdThreads = 256;
-constexpr int kProdC = 64;         // vocabulary entries of a tile
-constexpr int kProdPerCu = 4;      // workgroups that share a compute unit
+constexpr int kProdC = 64;      // vocabulary entries of a tile
+constexpr int kProdK = 32;      // k per chunk: two k-steps
+constexpr int kProdPerCu = 4;   // workgroups that share a compute unit
 constexpr long kMinWideTiles = 256;
-constexpr int kProdK = 32;       // k per chunk: two k-steps
-constexpr int kProdRowBytes = 96;
-template <int kM, int kC>
+constexpr int kPartBytes = 16 * kProdC;            // one part of an octet of k
+constexpr int kImageBytes = 4 * 3 * kPartBytes;    // a chunk of the operand along the vocabulary
+template <int kM>
 struct ProdShape {
-  static constexpr int kRows = kM + kC;                         // rows of a k-step in LDS: m, then c
-  static constexpr int kStepBytes = kRows * kProdRowBytes;
-  static constexpr size_t kLdsBytes = 2 * kStepBytes;  // (holds the listed gx rows as well)
-  // (four workgroups share 160 KB: with the bodies' own arrays, 6 floats per row)
-  static_assert(kLdsBytes + 6 * 4 * kM <= 40 << 10, "LDS per CU");
-  static constexpr int kMTiles = kM / 64, kCTiles = kC / 64;    // 32-row and -column tiles per wave
-  static constexpr int kMColumns = kM / 64, kColumns = kC / 64; // columns per thread of a k-major fetch
+  static constexpr int kWavesM = kM / 32, kWavesC = 4 / kWavesM;
+  static constexpr int kWaveC = kProdC / kWavesC, kTiles = kWaveC / 32;  // 32-column tiles of a wave
+  static constexpr int kMColumns = kM / 64;  // frames per thread of a sum over lattice rows
 };
 typedef int intx4 __attribute__((ext_vector_type(4)));
-// Byte offset of k-octet `octet` (0 .. 3) of row `row` within a chunk's LDS image; the parts lie 32
-// bytes apart.  Rows whose bit 3 is set have the halves of a part swapped: the 16-byte accesses of
-// 16 consecutive rows then fall on all 64 banks (rows are 24 words apart).
-template <int kM, int kC>
-__device__ __forceinline__ int octet_at(int row, int octet) {
-  return (octet >> 1) * ProdShape<kM, kC>::kStepBytes + row * kProdRowBytes +
-         16 * ((octet & 1) ^ ((row >> 3) & 1));
-}
-__device__ __forceinline__ void write_octet(char *to, const float (&e)[8]) {
-  uintx4 hi, mid, lo;
+// k-octet `octet` (0 .. 3) of entry `c` in a chunk's LDS image
+__device__ __forceinline__ int octet_at(int c, int octet) { return octet * 3 * kPartBytes + c * 16; }
+__device__ __forceinline__ void split_octet(const float (&e)[8], uintx4 &hi, uintx4 &mid, uintx4 &lo) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     unsigned h, m, l;
     split_pair(e[2 * q], e[2 * q + 1], h, m, l);
     hi[q] = h, mid[q] = m, lo[q] = l;
   }
+}
+__device__ __forceinline__ void write_octet(char *to, const float (&e)[8]) {
+  uintx4 hi, mid, lo;
+  split_octet(e, hi, mid, lo);
   *reinterpret_cast<uintx4 *>(to) = hi;
-  *reinterpret_cast<uintx4 *>(to + 32) = mid;
-  *reinterpret_cast<uintx4 *>(to + 64) = lo;
+  *reinterpret_cast<uintx4 *>(to + kPartBytes) = mid;
+  *reinterpret_cast<uintx4 *>(to + 2 * kPartBytes) = lo;
 }
 __device__ __forceinline__ Split8 read_octet(const char *at) {
   Split8 o;
   o.hi = *reinterpret_cast<const bf16x8 *>(at);
-  o.mid = *reinterpret_cast<const bf16x8 *>(at + 32);
-  o.lo = *reinterpret_cast<const bf16x8 *>(at + 64);
+  o.mid = *reinterpret_cast<const bf16x8 *>(at + kPartBytes);
+  o.lo = *reinterpret_cast<const bf16x8 *>(at + 2 * kPartBytes);
   return o;
-}
-// eight k of one column of a k-major matrix (rows `ld` floats apart): `off` is the byte offset of
-// the column in row k0, rows from `k_end` on read as 0
-__device__ __forceinline__ void fetch_octet(float (&into)[8], __amdgpu_buffer_rsrc_t rs, int off,
-                                            int k0, int k_end, int ld) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    into[i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-        rs, k0 + i < k_end ? off : kNowhere, (k0 + i) * ld * 4, 0));
 }
 // (the gradients that a product writes are FRNNT_F32, FRNNT_F16 or FRNNT_BF16, or kStreamed:
 // float32 with the non-temporal hint)
@@ -574,57 +582,123 @@ __device__ __forceinline__ void with_store(int type, F f) {
                                             there ? 2 * at : kNowhere, 2 * uniform, 0);
     });
 }
-// the products of a chunk: the first `m_tiles` of this wave's 32-row tiles
-template <int kM, int kC>
-__device__ __forceinline__ void multiply_chunk(const char *lds, int wave_m, int wave_n, int half,
-                                               int r32, int m_tiles,
-                                               dgemm::floatx16 (&acc)[ProdShape<kM, kC>::kMTiles]
-                                                                     [ProdShape<kM, kC>::kCTiles]) {
-  constexpr int kMTiles = ProdShape<kM, kC>::kMTiles;
+// acc[n] += D (rows of this wave's 32) times exp(x - max) (its 32-column tiles) over k < k_lim.
+// kFrames: the rows are frames and k the lattice rows (am.grad), else the other way round.  `x` holds
+// the rows of the operand along the vocabulary, one per k; `live`: this wave's rows count.  `early()` is
+// called once the first chunk is staged, `late()` before the end, to request what follows.
+template <int kM, bool kFrames, typename Early, typename Late>
+__device__ __forceinline__ void accumulate_products(
+    char *lds, __amdgpu_buffer_rsrc_t d_rs, int row, int ldd, __amdgpu_buffer_rsrc_t x_rs,
+    const float *x_max, int c_tile, int C, int k_lim, bool live, int wave, int lane,
+    dgemm::floatx16 (&acc)[ProdShape<kM>::kTiles], Early early, Late late) {
+  using Shape = ProdShape<kM>;
+  const int half = lane >> 5, r32 = lane & 31;
+  const int c_wave = Shape::kWaveC * (wave / Shape::kWavesM);
+  // D: a lane's operand is eight consecutive k of its row, straight from memory.  It is 0 wherever a
+  // row or a frame does not count, and up to the end of its rows of ldd; nothing is read past them.
+  float d[2][8];
+  const int d_off = kFrames ? (8 * half * ldd + row) * 4 : (row * ldd + 8 * half) * 4;
+  auto fetch_d = [&](int g, int k0) {
+    if constexpr (kFrames) {
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    Split8 m_op[kMTiles];
+      for (int i = 0; i < 8; ++i)
+        d[g][i] = get_float(d_rs, true, d_off + k0 * ldd * 4, (16 * g + i) * ldd * 4);
+    } else {
 #pragma unroll
-    for (int j = 0; j < kMTiles; ++j)
-      m_op[j] = read_octet(lds + octet_at<kM, kC>(kM / 2 * wave_m + 32 * j + r32, 2 * g + half));
+      for (int j = 0; j < 2; ++j) {
+        const int k = 16 * g + 4 * j;
+        const intx4 raw = __builtin_amdgcn_raw_buffer_load_b128(
+            d_rs, 8 * half + k < ldd - k0 ? d_off + 4 * (k0 + k) : kNowhere, 0, 0);
 #pragma unroll
-    for (int n = 0; n < ProdShape<kM, kC>::kCTiles; ++n) {
-      const Split8 c_op = read_octet(
-          lds + octet_at<kM, kC>(kM + (kC / 2) * wave_n + 32 * n + r32, 2 * g + half));
-#pragma unroll
-      for (int j = 0; j < kMTiles; ++j)
-        if (m_tiles > j) acc[j][n] = multiply_add(m_op[j], c_op, acc[j][n]);
+        for (int i = 0; i < 4; ++i) d[g][4 * j + i] = __int_as_float(raw[i]);
+      }
     }
+  };
+  // the operand along the vocabulary: eight consecutive k of one entry per thread.  The
+  // resource ends with row k_lim - 1: what follows reads as 0 with a shift of 0, a factor of 1.
+  float x[8], shift;  // (lane i: the shift of k i)
+  const int x_off = (8 * wave * C + c_tile + lane) * 4;
+  auto fetch_x = [&](int k0) {
+    const int k = k0 + 8 * wave + (lane & 7);
+    const float mx = x_max[min(k, k_lim - 1)];
+    shift = k < k_lim ? -mx * kLog2e : 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = get_float(x_rs, true, x_off + k0 * C * 4, i * C * 4);
+  };
+  auto stage_x = [&](char *image) {
+    float e[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) e[i] = exp_shifted(x[i], read_lane(shift, i));
+    write_octet(image + octet_at(lane, wave), e);
+  };
+  auto multiply = [&](int g, const char *image) {
+    uintx4 hi, mid, lo;
+    split_octet(d[g], hi, mid, lo);
+    Split8 d_op;
+    __builtin_memcpy(&d_op.hi, &hi, 16);
+    __builtin_memcpy(&d_op.mid, &mid, 16);
+    __builtin_memcpy(&d_op.lo, &lo, 16);
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
+      acc[n] = multiply_add(
+          d_op, read_octet(image + octet_at(c_wave + 32 * n + r32, 2 * g + half)), acc[n]);
+  };
+  if (k_lim <= 0) {
+    early();
+    late();
+    lds_barrier();
+    return;
   }
+  fetch_x(0);
+  fetch_d(0, 0);
+  fetch_d(1, 0);
+  early();
+  stage_x(lds);
+  fetch_x(kProdK);
+  lds_barrier();
+  int image = 0, k0 = 0;
+  for (; k0 + kProdK < k_lim; k0 += kProdK) {
+    const char *from = lds + image;
+    image ^= kImageBytes;
+    stage_x(lds + image);
+    fetch_x(k0 + 2 * kProdK);
+    if (live) {
+      multiply(0, from);
+      fetch_d(0, k0 + kProdK);
+      multiply(1, from);
+      fetch_d(1, k0 + kProdK);
+    }
+    lds_barrier();
+  }
+  if (live) {
+    multiply(0, lds + image);
+    multiply(1, lds + image);
+  }
+  late();
 }
 
-template <int kM, int kC, bool kSmooth>
+template <int kM, bool kSmooth>
 __device__ __forceinline__ void simple_bwd_lm_body(
-    int block_id, const float *__restrict__ lm, const float *__restrict__ am,
+    int b, int row_idx, int c_idx, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const float *__restrict__ lm_max,
     const float *__restrict__ am_max, const float *__restrict__ dmat,
     const float *__restrict__ row_x, const float *__restrict__ row_y,
-    void *__restrict__ lm_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
-    int ldd, int term, int part_shift, int out_type) {
-  using Shape = ProdShape<kM, kC>;
+    void *__restrict__ lm_grad, const int64_t *__restrict__ window, int S, int T, int C, int ldd,
+    int term, int out_type) {
+  using Shape = ProdShape<kM>;
   using namespace dgemm;
   extern __shared__ __align__(16) char prod_lds[];
   __shared__ float row_mx[kM], row_rx[kM], row_ry[kM];
   __shared__ int row_sym[kM];
   const int S1 = S + 1;
-  const int c_tiles = (C + kC - 1) / kC, s_tiles = (S1 + kM - 1) / kM;
-  int b, tile;
-  Limits lim;
-  if (!place_block(block_id, c_tiles, s_tiles, part_shift, B, row_x, window, S, T, b, tile, lim))
-    return;
-  const int s_tile = (tile / c_tiles) * kM, c_tile = (tile % c_tiles) * kC;
+  const Limits lim = limits_of(window, b, S, T);
+  const int s_tile = row_idx * kM, c_tile = c_idx * kProdC;
   const float *lmb = lm + (long)b * S1 * C;
   const float *amb = am + (long)b * T * C;
   const float *amx = am_max + (long)b * T;
   const float *db = dmat + (long)b * S1 * ldd;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave >> 1, wave_n = wave & 1;
   const int half = lane >> 5, r32 = lane & 31;
   // With a window, D vanishes at frames >= t_end and on rows > s_end: the sum over frames
   // stops at t_end (the row maxima of later frames may not even be defined) and rows past s_end
@@ -632,153 +706,112 @@ __device__ __forceinline__ void simple_bwd_lm_body(
   const int t_lim = __builtin_amdgcn_readfirstlane(lim.t_end);
   const int s_lim = __builtin_amdgcn_readfirstlane(min(S1, lim.s_end + 1));
   // The loads go through buffer resources that cover D[b] and am[b]: one instruction each, no
-  // branch; a row past the last one lies past the resource and reads as 0.  Frames at and past
-  // t_lim must give products of 0: there D is replaced by 0 and am reads as 0, whose
-  // exponential is finite.  Vocabulary columns at and past C belong to the next row: they only
-  // feed output columns that are never written.
-  const __amdgpu_buffer_rsrc_t d_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(db), 0, S1 * ldd * 4, 0x00020000);
-  const __amdgpu_buffer_rsrc_t am_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(amb), 0, T * C * 4, 0x00020000);
-  // D lies k-contiguous: eight lanes per row; a thread takes rows sub + 32 j at k-offset kq
-  const int sub = tid / 8, kq = 4 * (tid % 8);
-  const int d_off = ((s_tile + sub) * ldd + kq) * 4;
-  const int am_off = (c_tile + lane) * 4;
-  struct {
-    floatx4 d[kM / 32];
-    float a[Shape::kColumns][8], shift2[8];
-  } stage;
-  auto fetch = [&](int k0) {
+  // branch; rows past the last one read as 0 or as other rows of D and only feed rows that are never
+  // written.  Vocabulary columns at and past C belong to the next row: they only feed output
+  // columns that are never written.
+  const __amdgpu_buffer_rsrc_t d_rs = buffer_of(db, S1 * ldd * 4);
+  const __amdgpu_buffer_rsrc_t am_rs = buffer_of(amb, t_lim * C * 4);
+  const int m_wave = 32 * (wave % Shape::kWavesM);
+  floatx16 acc[Shape::kTiles];
 #pragma unroll
-    for (int j = 0; j < kM / 32; ++j) {
-      const intx4 raw = __builtin_amdgcn_raw_buffer_load_b128(d_rs, d_off, (32 * j * ldd + k0) * 4, 0);
-      stage.d[j] = floatx4{__int_as_float(raw[0]), __int_as_float(raw[1]), __int_as_float(raw[2]),
-                        __int_as_float(raw[3])};
-    }
-    if (k0 + kProdK > t_lim) {  // (uniform) the chunk that holds the last frame
+  for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
-      for (int j = 0; j < kM / 32; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (k0 + kq + i >= t_lim) stage.d[j][i] = 0.f;
-    }
-#pragma unroll
-    for (int n = 0; n < Shape::kColumns; ++n)
-      fetch_octet(stage.a[n], am_rs, am_off + 256 * n, k0 + 8 * wave, t_lim, C);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int t = k0 + 8 * wave + i;
-      const float mx = amx[min(t, t_lim - 1)];
-      stage.shift2[i] = t < t_lim ? -mx * kLog2e : 0.f;
-    }
-  };
-  if (t_lim > 0) fetch(0);
-  if (tid < kM) {
-    const int s = s_tile + tid, at = 4 * s;
-    const long first = (long)b * S1;
-    const float mx = get_float(buffer_of(lm_max + first, S1 * 4), s < s_lim, at);
-    const float rx = get_float(buffer_of(row_x + first, S1 * 4), s < S, at);
-    const float ry = get_float(buffer_of(row_y + first, S1 * 4), s < S1, at);
-    row_sym[tid] = get_symbol(symbols_of(symbols + (long)b * S, S), s < S, s, C);
-    row_mx[tid] = mx, row_rx[tid] = rx, row_ry[tid] = ry;
-  }
-  const int m_tiles = min(Shape::kMTiles, (s_lim - s_tile - kM / 2 * wave_m + 31) / 32);  // (may be <= 0)
-  floatx16 acc[Shape::kMTiles][Shape::kCTiles];
-#pragma unroll
-  for (int j = 0; j < Shape::kMTiles; ++j)
-#pragma unroll
-    for (int n = 0; n < Shape::kCTiles; ++n)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[j][n][v] = 0.f;
-  auto consume = [&](int k0) {
-#pragma unroll
-    for (int j = 0; j < kM / 32; ++j) {
-      unsigned h0, h1, m0, m1, l0, l1;
-      split_pair(stage.d[j][0], stage.d[j][1], h0, m0, l0);
-      split_pair(stage.d[j][2], stage.d[j][3], h1, m1, l1);
-      char *to = prod_lds + octet_at<kM, kC>(sub + 32 * j, kq / 8) + 2 * (kq % 8);
-      *reinterpret_cast<uintx2 *>(to) = uintx2{h0, h1};
-      *reinterpret_cast<uintx2 *>(to + 32) = uintx2{m0, m1};
-      *reinterpret_cast<uintx2 *>(to + 64) = uintx2{l0, l1};
-    }
-#pragma unroll
-    for (int n = 0; n < Shape::kColumns; ++n) {
-      float e[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) e[i] = exp_shifted(stage.a[n][i], stage.shift2[i]);
-      write_octet(prod_lds + octet_at<kM, kC>(kM + lane + 64 * n, wave), e);
-    }
-    if (k0 + kProdK < t_lim) fetch(k0 + kProdK);
-    lds_barrier();
-    multiply_chunk<kM, kC>(prod_lds, wave_m, wave_n, half, r32, m_tiles, acc);
-    lds_barrier();  // the operands have been read
-  };
-  for (int k0 = 0; k0 < t_lim; k0 += kProdK) consume(k0);
-  if (t_lim <= 0) lds_barrier();
-
-  // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
-  // (the exponentials' arguments of all tiles are requested together)
+    for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
   const __amdgpu_buffer_rsrc_t lm_rs = buffer_of(lmb, S1 * C * 4);
   const __amdgpu_buffer_rsrc_t out_rs = out_buffer(lm_grad, (long)b * S1 * C, S1 * C, out_type);
-  const int m0 = kM / 2 * wave_m + 4 * half, c0 = c_tile + (kC / 2) * wave_n + r32;
-  auto row_of = [&](int j, int v) { return m0 + 32 * j + 8 * (v / 4) + v % 4; };
+  const int m0 = m_wave + 4 * half, c0 = c_tile + Shape::kWaveC * (wave / Shape::kWavesM) + r32;
+  auto row_of = [&](int v) { return m0 + 8 * (v / 4) + v % 4; };
   const int first = (s_tile + m0) * C + c0;  // (element)
-  auto below = [&](int j, int v) { return (32 * j + 8 * (v / 4) + v % 4) * C; };  // (uniform)
-  float in[Shape::kMTiles][Shape::kCTiles][16];
+  auto below = [&](int v) { return (8 * (v / 4) + v % 4) * C; };  // (uniform)
+  float in[Shape::kTiles][16];
+  accumulate_products<kM, false>(
+      prod_lds, d_rs, s_tile + m_wave + r32, ldd, am_rs, amx, c_tile, C, t_lim, s_tile + m_wave < s_lim,
+      wave, lane, acc,
+      [&] {
+        if (tid < kM) {
+          const int s = s_tile + tid, at = 4 * s;
+          const long first_row = (long)b * S1;
+          const float mx = get_float(buffer_of(lm_max + first_row, S1 * 4), s < s_lim, at);
+          const float rx = get_float(buffer_of(row_x + first_row, S1 * 4), s < S, at);
+          const float ry = get_float(buffer_of(row_y + first_row, S1 * 4), s < S1, at);
+          row_sym[tid] = get_symbol(symbols_of(symbols + (long)b * S, S), s < S, s, C);
+          row_mx[tid] = mx, row_rx[tid] = rx, row_ry[tid] = ry;
+        }
+      },
+      [&] {
 #pragma unroll
-  for (int j = 0; j < Shape::kMTiles; ++j)
+        for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
-    for (int n = 0; n < Shape::kCTiles; ++n)
+          for (int v = 0; v < 16; ++v)
+            in[n][v] = get_float(lm_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(v));
+      });
+
+  // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
+#pragma unroll
+  for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[n][v] *= __expf(in[n][v] - row_mx[row_of(v)]);
+  const bool symbols_here = __any((unsigned)(row_sym[m_wave + r32] - c_tile) < (unsigned)kProdC);
+  if (symbols_here || (unsigned)(term - c_tile) < (unsigned)kProdC) {  // (uniform)
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        // (selects: branches around elements of a vector register make the compiler move all of it)
+        const int m = row_of(v), c = c0 + 32 * n;
+        const float rx = c == row_sym[m] ? row_rx[m] : 0.f, ry = c == term ? row_ry[m] : 0.f;
+        acc[n][v] = (acc[n][v] + rx) + ry;
+      }
+  }
+  if (s_tile + m_wave + 32 > s_lim) {  // (uniform)
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
       for (int v = 0; v < 16; ++v)
-        in[j][n][v] = get_float(lm_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(j, v));
+        acc[n][v] = s_tile + row_of(v) < s_lim ? acc[n][v] : 0.f;
+  }
+  if (kSmooth) {
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[n][v] += get_float(out_rs, c0 + 32 * n < C, 4 * (first + 32 * n), 4 * below(v));
+  }
   with_store(out_type, [&](auto store) {
 #pragma unroll
-    for (int j = 0; j < Shape::kMTiles; ++j)
+    for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
-      for (int n = 0; n < Shape::kCTiles; ++n)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = row_of(j, v), s = s_tile + m, c = c0 + 32 * n;
-          float g = __expf(in[j][n][v] - row_mx[m]) * acc[j][n][v];
-          if (c == row_sym[m]) g += row_rx[m];
-          if (c == term) g += row_ry[m];
-          if (!(s < s_lim)) g = 0.f;
-          if (kSmooth) g += get_float(out_rs, c < C, 4 * (first + 32 * n), 4 * below(j, v));
-          store(out_rs, c < C, first + 32 * n, below(j, v), g);
-        }
+      for (int v = 0; v < 16; ++v)
+        store(out_rs, c0 + 32 * n < C, first + 32 * n, below(v), acc[n][v]);
   });
 }
 
 // The per-symbol term of am.grad,  sum_s [c = sym[b,s]] gx[b,s,t],  is a second product, gx^T times
 // a one-hot matrix made in registers from the symbols, on the float32 matrix instruction: it is
 // exact (products by 0 or 1) and has a fixed summation order.  The lattice rows whose symbol lies
-// in the workgroup's vocabulary range are listed in order; their gx rows go to LDS, some at a
-// time, and are multiplied two rows at a time onto the finished dense results.
-template <int kM, int kC, bool kSmooth>
+// in the workgroup's vocabulary range are listed in order, sixteen at a time, and multiplied two
+// rows at a time onto the finished dense results; the first sixteen are requested before the dense
+// products and wait in registers.
+constexpr int kListed = 16;
+template <int kM, bool kSmooth>
 __device__ __forceinline__ void simple_bwd_am_body(
-    int block_id, const float *__restrict__ lm, const float *__restrict__ am,
+    int b, int row_idx, int c_idx, const float *__restrict__ lm, const float *__restrict__ am,
     const int64_t *__restrict__ symbols, const int64_t *__restrict__ boundary,
     const float *__restrict__ lm_max, const float *__restrict__ am_max,
     const float *__restrict__ dmat, const float *__restrict__ gpx,
     const float *__restrict__ gpy, const float *__restrict__ row_x,
-    void *__restrict__ am_grad, const int64_t *__restrict__ window, int B, int S, int T, int C,
-    int ldd, int term, int rnnt_type, int part_shift, int out_type, const SmoothTerms &smooth) {
-  using Shape = ProdShape<kM, kC>;
+    void *__restrict__ am_grad, const int64_t *__restrict__ window, int S, int T, int C, int ldd,
+    int term, int rnnt_type, int out_type, const SmoothTerms &smooth) {
+  using Shape = ProdShape<kM>;
   using namespace dgemm;
   extern __shared__ __align__(16) char prod_lds[];
   __shared__ float frame_mx[kM], frame_y[kM], frame_w[kSmooth ? kM : 1];
   const int S1 = S + 1;
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
-  const int c_tiles = (C + kC - 1) / kC, t_tiles = (T + kM - 1) / kM;
-  int b, tile;
-  Limits lim;
-  if (!place_block(block_id, c_tiles, t_tiles, part_shift, B, row_x, window, S, T, b, tile, lim))
-    return;
-  const int t_tile = (tile / c_tiles) * kM, c_tile = (tile % c_tiles) * kC;
+  const Limits lim = limits_of(window, b, S, T);
+  const int t_tile = row_idx * kM, c_tile = c_idx * kProdC;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave >> 1, wave_n = wave & 1;
   const int half = lane >> 5, r32 = lane & 31;
   const float *lmb = lm + (long)b * S1 * C;
   const float *amb = am + (long)b * T * C;
@@ -795,104 +828,106 @@ __device__ __forceinline__ void simple_bwd_am_body(
   const bool live = t_tile < t_lim;
   const __amdgpu_buffer_rsrc_t am_rs = buffer_of(amb, T * C * 4);
   const __amdgpu_buffer_rsrc_t out_rs = out_buffer(am_grad, (long)b * T * C, T * C, out_type);
-  const int m0 = kM / 2 * wave_m + 4 * half, c_lo = c_tile + (kC / 2) * wave_n, c0 = c_lo + r32;
-  auto row_of = [&](int j, int v) { return m0 + 32 * j + 8 * (v / 4) + v % 4; };
+  const int m_wave = 32 * (wave % Shape::kWavesM);
+  const int m0 = m_wave + 4 * half, c_lo = c_tile + Shape::kWaveC * (wave / Shape::kWavesM),
+            c0 = c_lo + r32;
+  auto row_of = [&](int v) { return m0 + 8 * (v / 4) + v % 4; };
   const int first = (t_tile + m0) * C + c0;  // (element)
-  auto below = [&](int j, int v) { return (32 * j + 8 * (v / 4) + v % 4) * C; };  // (uniform)
-  floatx16 acc[Shape::kMTiles][Shape::kCTiles];
+  auto below = [&](int v) { return (8 * (v / 4) + v % 4) * C; };  // (uniform)
+  floatx16 acc[Shape::kTiles];
 #pragma unroll
-  for (int j = 0; j < Shape::kMTiles; ++j)
+  for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
-    for (int n = 0; n < Shape::kCTiles; ++n)
+    for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
+  float in[Shape::kTiles][16];
+  const __amdgpu_buffer_rsrc_t gx_rs = buffer_of(gxb, S * T1 * 4);
+  // ---- the listed rows, from 128 symbols at a time: two masks of those in this tile
+  const int s_count = live ? min(k_lim, S) : 0;
+  int sym[2];
+  unsigned long long hits[2];
+  int column[kListed];        // (uniform) entry of the tile, -1 for none
+  float value[kListed / 2];   // of rows 2 i + half at this lane's frame
+  auto find_hits = [&](int s0) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[j][n][v] = 0.f;
-  if (live) {
-    // (resources as in the kernel above; frames at and past T of D's rows only feed outputs that
-    // are never written, lattice rows that do not count read as 0)
-    const __amdgpu_buffer_rsrc_t d_rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(db), 0, S1 * ldd * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t lm_rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(lmb), 0, S1 * C * 4, 0x00020000);
-    const int d_off = (t_tile + lane) * 4, lm_off = (c_tile + lane) * 4;
-    struct {
-      float d[Shape::kMColumns][8], l[Shape::kColumns][8], shift2[8];
-    } stage;
-    auto fetch = [&](int k0) {
-#pragma unroll
-      for (int n = 0; n < Shape::kMColumns; ++n)
-        fetch_octet(stage.d[n], d_rs, d_off + 256 * n, k0 + 8 * wave, k_lim, ldd);
-#pragma unroll
-      for (int n = 0; n < Shape::kColumns; ++n)
-        fetch_octet(stage.l[n], lm_rs, lm_off + 256 * n, k0 + 8 * wave, k_lim, C);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int k = k0 + 8 * wave + i;
-        const float mx = lmx[min(k, k_lim - 1)];
-        stage.shift2[i] = k < k_lim ? -mx * kLog2e : 0.f;
-      }
-    };
-    if (k_lim > 0) fetch(0);
-    if (tid < kM) {
-      const int t = t_tile + tid;
-      const float mx = get_float(buffer_of(am_max + (long)b * T, T * 4), t < t_lim, 4 * t);
-      frame_mx[tid] = mx;
-      if (kSmooth) {
-        const float g = get_float(buffer_of(smooth.am_g + (long)b * T, T * 4), t < t_lim, 4 * t);
-        const float z = get_float(buffer_of(smooth.am_z + (long)b * T, T * 4), t < t_lim, 4 * t);
-        frame_w[tid] = t < t_lim ? -smooth.am_scale * g / z : 0.f;
-      }
+    for (int u = 0; u < 2; ++u) {
+      const int s = s0 + 64 * u + lane;
+      sym[u] = get_symbol(sym_rs, s < s_count, s, C) - c_tile;
     }
-    const int m_tiles = min(Shape::kMTiles, (t_lim - t_tile - kM / 2 * wave_m + 31) / 32);  // (may be <= 0)
-    auto consume = [&](int k0) {
 #pragma unroll
-      for (int n = 0; n < Shape::kMColumns; ++n)
-        write_octet(prod_lds + octet_at<kM, kC>(lane + 64 * n, wave), stage.d[n]);
+    for (int u = 0; u < 2; ++u)
+      hits[u] = __ballot(s0 + 64 * u + lane < s_count && (unsigned)sym[u] < (unsigned)kProdC);
+  };
+  auto fetch_listed = [&](int s0) {
+    const int t = t_tile + m_wave + r32;
+    const bool there = t < T && t != t_mask;
 #pragma unroll
-      for (int n = 0; n < Shape::kColumns; ++n) {
-        float e[8];
+    for (int i = 0; i < kListed / 2; ++i) column[2 * i] = -1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) e[i] = exp_shifted(stage.l[n][i], stage.shift2[i]);
-        write_octet(prod_lds + octet_at<kM, kC>(kM + lane + 64 * n, wave), e);
+    for (int i = 0; i < kListed / 2; ++i) {
+      if (!(hits[0] | hits[1])) break;  // (uniform)
+      int row[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool low = hits[0] != 0, any = (hits[0] | hits[1]) != 0;
+        unsigned long long &mask = low ? hits[0] : hits[1];
+        const int at = any ? __builtin_ctzll(mask) : 0;
+        row[u] = any ? s0 + at + (low ? 0 : kWave) : -1;
+        column[2 * i + u] = any ? __builtin_amdgcn_readlane(low ? sym[0] : sym[1], at) : -1;
+        mask &= mask - 1;
       }
-      if (k0 + kProdK < k_lim) fetch(k0 + kProdK);
-      lds_barrier();
-      multiply_chunk<kM, kC>(prod_lds, wave_m, wave_n, half, r32, m_tiles, acc);
-      lds_barrier();  // the operands have been read
-    };
-    for (int k0 = 0; k0 < k_lim; k0 += kProdK) consume(k0);
-  }
+      const int mine = half ? row[1] : row[0];
+      value[i] = get_float(gx_rs, there && mine >= 0, (mine * T1 + t) * 4);
+    }
+  };
+  if (live)
+    accumulate_products<kM, true>(
+        prod_lds, buffer_of(db, S1 * ldd * 4), t_tile + m_wave + r32, ldd, buffer_of(lmb, k_lim * C * 4),
+        lmx, c_tile, C, k_lim, t_tile + m_wave < t_lim, wave, lane, acc,
+        [&] {
+          if (tid < kM) {
+            const int t = t_tile + tid;
+            const float mx = get_float(buffer_of(am_max + (long)b * T, T * 4), t < t_lim, 4 * t);
+            frame_mx[tid] = mx;
+            if (kSmooth) {
+              const float g = get_float(buffer_of(smooth.am_g + (long)b * T, T * 4), t < t_lim, 4 * t);
+              const float z = get_float(buffer_of(smooth.am_z + (long)b * T, T * 4), t < t_lim, 4 * t);
+              frame_w[tid] = t < t_lim ? -smooth.am_scale * g / z : 0.f;
+            }
+          }
+          find_hits(0);
+          fetch_listed(0);
+        },
+        [&] {
+#pragma unroll
+          for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+              in[n][v] = get_float(am_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(v));
+        });
 
   // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
   if (live) {
-    // the exponentials' arguments of all tiles are requested together
-    float in[Shape::kMTiles][Shape::kCTiles][16];
-#pragma unroll
-    for (int j = 0; j < Shape::kMTiles; ++j)
-#pragma unroll
-      for (int n = 0; n < Shape::kCTiles; ++n)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          in[j][n][v] = get_float(am_rs, c0 + 32 * n < C, 4 * first + 128 * n, 4 * below(j, v));
     // The termination symbol's term, sum_s gy[s,t], in the workgroups that hold its column: every
     // wave sums a quarter of the lattice rows.
     const __amdgpu_buffer_rsrc_t gx_rs = buffer_of(gxb, S * T1 * 4);
-    if ((unsigned)(term - c_tile) < (unsigned)kC) {  // (uniform)
+    if ((unsigned)(term - c_tile) < (unsigned)kProdC) {  // (uniform)
       const __amdgpu_buffer_rsrc_t gy_rs = buffer_of(gpy + (long)b * S1 * T, S1 * T * 4);
+      lds_barrier();  // the operands have been read
       float *part = reinterpret_cast<float *>(prod_lds);
       float sum[Shape::kMColumns] = {};
-      constexpr int kAhead = 8;
+      constexpr int kRowsAhead = 8;
       auto add_rows = [&](__amdgpu_buffer_rsrc_t rs, int rows, int pitch) {
-        for (int s0 = wave; s0 < rows; s0 += 4 * kAhead) {
-          float y[kAhead][Shape::kMColumns];
+        for (int s0 = wave; s0 < rows; s0 += 4 * kRowsAhead) {
+          float y[kRowsAhead][Shape::kMColumns];
 #pragma unroll
-          for (int u = 0; u < kAhead; ++u)
+          for (int u = 0; u < kRowsAhead; ++u)
 #pragma unroll
             for (int w = 0; w < Shape::kMColumns; ++w) {
               const int s = s0 + 4 * u, t = t_tile + lane + 64 * w;
               y[u][w] = get_float(rs, s < rows && t >= lim.t_begin && t < t_lim, 4 * t, s * pitch * 4);
             }
 #pragma unroll
-          for (int u = 0; u < kAhead; ++u)
+          for (int u = 0; u < kRowsAhead; ++u)
 #pragma unroll
             for (int w = 0; w < Shape::kMColumns; ++w) sum[w] += y[u][w];
         }
@@ -908,110 +943,57 @@ __device__ __forceinline__ void simple_bwd_am_body(
                        (kSmooth ? smooth.symbol_scale : 1.f);
       lds_barrier();
     }
-    constexpr int kHotPitch = kM + 4;
-    constexpr int kHotRows = kM == 128 ? 64 : 32;  // rows of the list in LDS at a time
-    static_assert(Shape::kLdsBytes >= kHotRows * (kHotPitch + 1) * 4, "room for the listed rows");
-    float *hot = reinterpret_cast<float *>(prod_lds);
-    int *hot_sym = reinterpret_cast<int *>(hot + kHotRows * kHotPitch);
-    const int s_count = min(k_lim, S);
-    auto multiply_hot = [&](int listed) {
-      lds_barrier();  // the listed rows are in LDS
-      for (int i = 0; i < listed; i += 2) {
-        const int row = i + half;
-        const int sym = row < listed ? hot_sym[row] : -1;
-        // (wave-uniform) does one of the two fall into this wave's columns
-        if (!__any((unsigned)(sym - c_lo) < (unsigned)(kC / 2))) continue;
-        float value[Shape::kMTiles];
-#pragma unroll
-        for (int j = 0; j < Shape::kMTiles; ++j)
-          value[j] = row < listed ? hot[row * kHotPitch + kM / 2 * wave_m + 32 * j + r32] : 0.f;
-#pragma unroll
-        for (int n = 0; n < Shape::kCTiles; ++n) {
-          const float one = sym == c0 + 32 * n ? (kSmooth ? smooth.symbol_scale : 1.f) : 0.f;
-          if (!__any(one != 0.f)) continue;
-#pragma unroll
-          for (int j = 0; j < Shape::kMTiles; ++j)
-            acc[j][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(value[j], one, acc[j][n], 0, 0, 0);
-        }
-      }
-      lds_barrier();  // ... and have been read
-    };
-    float unigram[Shape::kCTiles];
+    float unigram[Shape::kTiles];
     if (kSmooth)
 #pragma unroll
-      for (int n = 0; n < Shape::kCTiles; ++n)
+      for (int n = 0; n < Shape::kTiles; ++n)
         unigram[n] = get_float(buffer_of(smooth.unigram, C * 4), c0 + 32 * n < C, 4 * (c0 + 32 * n));
-    auto finish_dense = [&]() {
 #pragma unroll
-      for (int j = 0; j < Shape::kMTiles; ++j)
+    for (int n = 0; n < Shape::kTiles; ++n) {
 #pragma unroll
-        for (int n = 0; n < Shape::kCTiles; ++n)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int m = row_of(j, v);
-            if (kSmooth) acc[j][n][v] += frame_w[m] * unigram[n];
-            acc[j][n][v] *= __expf(in[j][n][v] - frame_mx[m]);
-            if (c0 + 32 * n == term)
-              acc[j][n][v] += frame_y[m];
-          }
-    };
-    int listed = 0;
-    bool dense_done = false;
-    for (int s0 = 0; s0 < s_count; s0 += kWave) {
-      const int sym = get_symbol(sym_rs, s0 + lane < s_count, s0 + lane, C);
-      unsigned long long hits = __ballot((unsigned)(sym - c_tile) < (unsigned)kC);
-      while (hits) {  // (uniform over the workgroup)
-        // the next sixteen rows of the list, four per wave: kM frames each (nothing for the masked
-        // frame and past T), requested together
-        int row[4];
-        const int old = listed;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          if (u % 4 == 0) row[u / 4] = -1;
-          const int at = hits ? __builtin_ctzll(hits) : -1;
-          if (u % 4 == wave) row[u / 4] = at;
-          listed += hits ? 1 : 0;
-          hits &= hits - 1;
-        }
-        float value[4][Shape::kMColumns];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int w = 0; w < Shape::kMColumns; ++w) {
-            const int t = t_tile + lane + 64 * w;
-            value[u][w] = get_float(gx_rs, row[u] >= 0 && t < T && t != t_mask,
-                                    ((s0 + row[u]) * T1 + t) * 4);
-          }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (row[u] < 0) continue;  // (wave-uniform)
-          const int slot = old + 4 * u + wave;
-#pragma unroll
-          for (int w = 0; w < Shape::kMColumns; ++w) hot[slot * kHotPitch + lane + 64 * w] = value[u][w];
-          const int its = __builtin_amdgcn_readlane(sym, row[u]);
-          if (lane == 0) hot_sym[slot] = its;
-        }
-        if (listed > kHotRows - 16) {
-          if (!dense_done) finish_dense();
-          dense_done = true;
-          multiply_hot(listed);
-          listed = 0;
-        }
+      for (int v = 0; v < 16; ++v) {
+        const int m = row_of(v);
+        if (kSmooth) acc[n][v] += frame_w[m] * unigram[n];
+        acc[n][v] *= __expf(in[n][v] - frame_mx[m]);
+        if (c0 + 32 * n == term) acc[n][v] += frame_y[m];
       }
     }
-    if (!dense_done) finish_dense();
-    if (listed > 0) multiply_hot(listed);
+    auto add_listed = [&] {
+#pragma unroll
+      for (int i = 0; i < kListed / 2; ++i) {
+        if (column[2 * i] < 0) break;  // (uniform)
+        const int mine = half ? column[2 * i + 1] : column[2 * i];
+#pragma unroll
+        for (int n = 0; n < Shape::kTiles; ++n) {
+          const int at = Shape::kWaveC * (wave / Shape::kWavesM) + 32 * n;
+          if ((unsigned)(column[2 * i] - at) >= 32u && (unsigned)(column[2 * i + 1] - at) >= 32u) continue;
+          const float one = mine == at + r32 ? (kSmooth ? smooth.symbol_scale : 1.f) : 0.f;
+          acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(value[i], one, acc[n], 0, 0, 0);
+        }
+      }
+    };
+    add_listed();
+    for (int s0 = 0; s0 < s_count; s0 += 2 * kWave) {
+      if (s0 > 0) find_hits(s0);
+      while (hits[0] | hits[1]) {  // (uniform)
+        fetch_listed(s0);
+        add_listed();
+      }
+    }
+  }
+  if (t_tile + m_wave + 32 > t_lim) {  // (uniform)
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[n][v] = t_tile + row_of(v) < t_lim ? acc[n][v] : 0.f;
   }
   with_store(out_type, [&](auto store) {
 #pragma unroll
-    for (int j = 0; j < Shape::kMTiles; ++j)
+    for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
-      for (int n = 0; n < Shape::kCTiles; ++n)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int t = t_tile + row_of(j, v);
-          store(out_rs, c0 + 32 * n < C, first + 32 * n, below(j, v), t < t_lim ? acc[j][n][v] : 0.f);
-        }
+      for (int v = 0; v < 16; ++v)
+        store(out_rs, c0 + 32 * n < C, first + 32 * n, below(v), acc[n][v]);
   });
 }
 
@@ -1050,15 +1032,19 @@ __global__ void __launch_bounds__(kProdThreads, kProdPerCu)
                             const float *__restrict__ row_y, void *__restrict__ lm_grad,
                             void *__restrict__ am_grad, const int64_t *__restrict__ window, int B,
                             int S, int T, int C, int ldd, int term, int rnnt_type,
-                            int lm_blocks, int part_shift, int out_type, SmoothTerms smooth) {
-  if ((int)blockIdx.x < lm_blocks)
-    simple_bwd_lm_body<kMl, kProdC, kSmooth>((int)blockIdx.x, lm, am, symbols, lm_max, am_max, dmat, row_x,
-                                    row_y, lm_grad, window, B, S, T, C, ldd, term, part_shift,
-                                    out_type);
-  else
-    simple_bwd_am_body<kMa, kProdC, kSmooth>((int)blockIdx.x - lm_blocks, lm, am, symbols, boundary, lm_max,
-                                    am_max, dmat, gpx, gpy, row_x, am_grad, window, B, S, T, C,
-                                    ldd, term, rnnt_type, part_shift, out_type, smooth);
+                            Placement lm_at, Placement am_at, int out_type, SmoothTerms smooth) {
+  int b, row_idx, c_idx;
+  if (blockIdx.x < lm_at.blocks) {
+    if (!place_block(blockIdx.x, lm_at, B, row_x, S, b, row_idx, c_idx)) return;
+    simple_bwd_lm_body<kMl, kSmooth>(b, row_idx, c_idx, lm, am, symbols, lm_max, am_max, dmat,
+                                         row_x, row_y, lm_grad, window, S, T, C, ldd, term,
+                                         out_type);
+  } else {
+    if (!place_block(blockIdx.x - lm_at.blocks, am_at, B, row_x, S, b, row_idx, c_idx)) return;
+    simple_bwd_am_body<kMa, kSmooth>(b, row_idx, c_idx, lm, am, symbols, boundary, lm_max, am_max,
+                                         dmat, gpx, gpy, row_x, am_grad, window, S, T, C, ldd, term,
+                                         rnnt_type, out_type, smooth);
+  }
 }
 template <int kMl, int kMa, bool kSmooth>
 void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
@@ -1067,22 +1053,25 @@ void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
                   const float *row_y, void *lm_grad, void *am_grad, const int64_t *window, int B,
                   int S, int T, int C, int ldd, int term, int rnnt_type, int out_type,
                   const SmoothTerms &smooth, hipStream_t stream) {
-  constexpr size_t lds = ProdShape<(kMl > kMa ? kMl : kMa), kProdC>::kLdsBytes;
   const int c_tiles = (C + kProdC - 1) / kProdC, shift = part_shift_for(B, c_tiles);
-  const unsigned am_blocks =
-      am_grad && T > 0 ? placed_grid(c_tiles, (T + kMa - 1) / kMa, B, shift) : 0;
-  const unsigned lm_blocks = lm_grad ? placed_grid(c_tiles, (S + kMl) / kMl, B, shift) : 0;
-  if (am_blocks + lm_blocks == 0) return;
-  hipLaunchKernelGGL((simple_bwd_am_lm_kernel<kMl, kMa, kSmooth>), dim3(am_blocks + lm_blocks),
-                     dim3(kProdThreads), lds, stream, lm, am, symbols, boundary, lm_max, am_max,
+  const Placement lm_at(c_tiles, lm_grad ? (S + kMl) / kMl : 0, B, shift);
+  const Placement am_at(c_tiles, am_grad && T > 0 ? (T + kMa - 1) / kMa : 0, B, shift);
+  if (lm_at.blocks + am_at.blocks == 0) return;
+  hipLaunchKernelGGL((simple_bwd_am_lm_kernel<kMl, kMa, kSmooth>), dim3(lm_at.blocks + am_at.blocks),
+                     dim3(kProdThreads), 2 * kImageBytes, stream, lm, am, symbols, boundary, lm_max, am_max,
                      dmat, gpx, gpy, row_x, row_y, lm_grad, am_grad, window, B, S, T, C, ldd,
-                     term, rnnt_type, (int)lm_blocks, shift, out_type, smooth);
+                     term, rnnt_type, lm_at, am_at, out_type, smooth);
 }
 // Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand
 // along the vocabulary half as often as 64 (am.grad at B 16, T 400, C 5000: 92 against 97 us;
 // lm.grad 60 against 65), which is what counts once the chip is full; they lose where the padding
 // of the last tile outweighs that (up to 64 rows: 24 against 18 us at B 21, S 47, T 333, C 503) or
 // where fewer of them than fill the chip remain (B 3, S 250, T 1335, C 198: 71 against 55 us).
+// Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand
+// along the vocabulary half as often as 64 (both products at B 64, S 120, T 600, C 500: 74 against 90
+// us; B 16, S 120, T 400, C 5000: 108 against 132), which is what counts once the chip is full; they
+// lose where the padding of the last tile outweighs that (lm.grad's up to 64 rows: 20 against 17 us at
+// B 21, S 47, T 333, C 503) or where fewer of them than fill the chip remain.
 bool wide_tile(long columns_of_tiles, int rows) {
   const long wide = (rows + 127) / 128, narrow = (rows + 63) / 64;
   return narrow > 1 && 14 * wide <= 8 * narrow && columns_of_tiles * wide >= kMinWideTiles;
@@ -1094,7 +1083,6 @@ void launch_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
                     const float *row_y, void *lm_grad, void *am_grad, const int64_t *window, int B,
                     int S, int T, int C, int ldd, int term, int rnnt_type, int out_type,
                     const SmoothTerms &smooth, hipStream_t stream) {
-  const long columns = (long)B * ((C + kProdC - 1) / kProdC);
   // Where lm, am and their gradients together outgrow the last-level cache (256 MB) the gradients
   // are streamed past it, which leaves it to lm and am: these are read by both products.  Whole pass
   // of the loss, with the hint against without: C 5000, S 120, T 400: B 14, 278 MB: 291 / 299 us;
@@ -1102,6 +1090,7 @@ void launch_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
   // 545 / 547; B 8, S 200, T 1000, C 5000, 366 MB: 558 / 589.  Below, either way: B 10, C 5000,
   // 198 MB: 267 / 263; B 32, S 60, T 300, C 2500, 220 MB: 188 / 188; B 45, C 1000, 247 MB: 320 / 327.
   if (out_type == FRNNT_F32 && 8L * B * (S + 1 + T) * C > (256L << 20)) out_type = kStreamed;
+  const long columns = (long)B * ((C + kProdC - 1) / kProdC);
   const bool wide_l = wide_tile(columns, S + 1), wide_a = wide_tile(columns, T);
   auto launch = wide_l ? wide_a ? launch_bwd_t<128, 128, kSmooth> : launch_bwd_t<128, 64, kSmooth>
                        : wide_a ? launch_bwd_t<64, 128, kSmooth> : launch_bwd_t<64, 64, kSmooth>;

@@ -58,13 +58,27 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {  // v_cvt_pk_b
   __builtin_memcpy(&w, &h, 4);
   return w;
 }
+// c minus the low (`high`: the high) half of w: v_dot2c_f32_bf16 with a unit vector, one instruction
+// for the unpacking and the subtraction.  The difference of a float32 and its bfloat16 rounding is
+// exact, and so are both products: the same bits as unpacking and subtracting (16 million values,
+// 2^-119 to 2^20), in 7 instead of 11 instructions per split pair.  (Not finite: a NaN or an
+// infinity also makes the other value of its pair NaN; the two belong to the same sums.)
+__device__ __forceinline__ float minus_half(float c, unsigned w, bool high) {
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  unsigned unit = high ? 0xbf800000u : 0x0000bf80u;
+  asm("" : "+s"(unit));  // (the compiler's inline constant -1.0 is not this word)
+  b2 values, units;
+  __builtin_memcpy(&values, &w, 4);
+  __builtin_memcpy(&units, &unit, 4);
+  return __builtin_amdgcn_fdot2_f32_bf16(values, units, c, false);
+}
 // the three parts of a pair of floats, each part's two values in one word
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &hi, unsigned &mid,
                                            unsigned &lo) {
   hi = pack_bf16(a, b);
-  const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xffff0000u);
+  const float ra = minus_half(a, hi, false), rb = minus_half(b, hi, true);
   mid = pack_bf16(ra, rb);
-  lo = pack_bf16(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
+  lo = pack_bf16(minus_half(ra, mid, false), minus_half(rb, mid, true));
 }
 struct Split8 {  // eight consecutive k of one row: a lane's operand of a 32 x 32 x 16 product
   bf16x8 hi, mid, lo;

@@ -49,6 +49,34 @@ def test_simple_loss_at_the_edges_of_tiles(gpu_device, B, S, T, C):
             assert bool((off <= 2e-4 + ulp * y.grad.abs()).all()), off.max().item()
 
 
+# (S, T, C, s_end, t_end): sums over k that end before, at and after a chunk of 32 and a k-step of 16,
+# rows of D whose length is no multiple of 4, lists of 16, 17, 128 and more equal symbols
+CHUNKS = [(16, 33, 70, 15, 31), (17, 34, 70, 16, 32), (40, 61, 65, 31, 33), (33, 255, 64, 32, 47),
+          (70, 98, 130, 63, 64), (140, 257, 66, 128, 65), (145, 150, 64, 145, 150)]
+
+
+@pytest.mark.parametrize("S,T,C,s_end,t_end", CHUNKS)
+def test_gradient_products_read_nothing_outside_a_window(gpu_device, S, T, C, s_end, t_end):
+    g = torch.Generator().manual_seed(S + T)
+    lm, am = torch.randn(2, S + 1, C, generator=g), torch.randn(2, T, C, generator=g)
+    symbols = torch.full((2, S), C // 2)
+    boundary = torch.tensor([[0, 0, s_end, t_end], [0, 0, s_end - 1, t_end - 1]])
+    cpu = [x.clone().requires_grad_(True) for x in (lm, am)]
+    O.loss_simple(*cpu, symbols, 0, boundary=boundary, reduction="sum").backward()
+    for b in range(2):  # rows and frames outside the windows must not be looked at
+        lm[b, boundary[b, 2] + 1:] = float("nan")
+        am[b, boundary[b, 3]:] = float("nan")
+    gpu = [x.to(gpu_device).requires_grad_(True) for x in (lm, am)]
+    loss = fast_rnnt_amd.rnnt_loss_simple(*gpu, symbols.to(gpu_device), 0,
+                                          boundary=boundary.to(gpu_device), reduction="sum")
+    # (what the scratch of the backward holds before it runs)
+    del_me = [torch.full((n,), float("nan"), device=gpu_device) for n in (1 << 10, 1 << 14, 1 << 18)]
+    del del_me
+    loss.backward()
+    for x, y in zip(gpu, cpu):
+        assert bool(((x.grad.cpu() - y.grad).abs() <= 2e-4 + 1e-4 * y.grad.abs()).all())
+
+
 # (S, T, C, batch sizes at which launch_normalizer_f32 takes tiles of 32, 64, 96 or 128 rows)
 HEIGHTS = [(95, 128, 500, {1: 32, 26: 64, 51: 96}), (120, 200, 600, {1: 32, 11: 64, 22: 128})]
 
