@@ -27,20 +27,30 @@ namespace {
 // of 102 at B 64, S 120, T 600, C 500, but rounds differently: single occupation probabilities
 // moved by up to 8e-3.)
 //
-// What bounds it: 32 matrix cycles per k and 32 x 32 cells (fp32 MFMA) plus what the wave issues
-// for its operands (maximum, exp, LDS: about 14 cycles per 64 elements) -- on this part the two
-// add up, also across the waves of a SIMD -- and the prologue and epilogue of a workgroup, which
-// another one on the compute unit has to hide: with 32 or 64 lattice rows two share it, with 96 or
-// 128, which convert less per cell, one fills it (launch_normalizer_f32 chooses; 96 or 128 rows
-// always -> the choice: B 64, S 120, T 600, C 500: 102 -> 74 us; B 8, S 100, T 400, C 5000:
-// 105 -> 64; B 2, S 53, T 343, C 4627: 56 -> 33; B 32, S 80, T 250, C 500: 18.6 -> 17.2).
+// What bounds it: what its waves issue.  On this part the float32 matrix instruction, the VALU and the
+// LDS accesses of a SIMD's waves add up (a slab of 32 x 32 cells takes a wave 512 cycles of the
+// first, about 250 for maxima, conversions and a quarter-rate exp2, 100 for LDS, and 300 besides), so
+// what counts is that every SIMD of the chip has its share of that, and that another workgroup's loop
+// covers a workgroup's prologue and epilogue (4.5 and 5 us).  Hence small tiles -- taller ones convert
+// less per cell, but of 16 utterances' tiles of 128 rows a third of the compute units got none --
+// dealt out evenly (find_tile), and eight waves of one share each or four of two
+// (launch_normalizer_f32).  Measured within training steps on three batches in turn, against tiles of
+// 32 to 128 rows with a workgroup per tile whether it counted or not: B 64, S 120, T 600, C 500: 96 ->
+// 89 us; B 32, S 80, T 250, C 500: 20.4 and 20.6; B 16, S 120, T 400, C 5000: 127 -> 122; B 10, S 137,
+// T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64 sizes, B 1 .. 128,
+// C 50 .. 5000: 5.6 %, the worst of them B 8, S 100, T 400, C 5000: 73 -> 81.  Tiles of 64, 96 and
+// 128 rows dealt out the same way were the fastest at 12 of the 64, mostly by 1 to 5 %, and a choice
+// among all of them, which cannot know how ragged a batch is, gained nothing over this one.
 constexpr int kNormK = 16;      // k per slab
-constexpr int kNormWaves = 8;   // of a workgroup
+constexpr int kNormShares = 8;  // of k
+constexpr int kNormS = 32;      // lattice rows of a tile
 constexpr int kNormT = 32;      // frames of a tile
-template <int kS>
+constexpr int kComputeUnits = 256;
+template <int kWaves_>
 struct NormShape {
-  static constexpr int kWaves = kNormWaves, kThreads = kWaves * kWave;
-  static constexpr int kRows = kS + kNormT;      // rows of a slab: lm rows, then am rows
+  static constexpr int kWaves = kWaves_, kThreads = kWaves * kWave;
+  static constexpr int kTurns = kNormShares / kWaves;  // shares of a wave, one after the other
+  static constexpr int kRows = kNormS + kNormT;  // rows of a slab: lm rows, then am rows
   static constexpr int kLoads = kRows / 16;      // 16-byte loads per lane and slab
   // Row pitch in LDS: 20 floats.  Rows start 16-byte aligned, so a lane's four values of a row go
   // in as one 16-byte write, and a lane reads its row's eight k of a slab half as two 16-byte reads:
@@ -49,36 +59,94 @@ struct NormShape {
   static constexpr int kSlab = kRows * kPitch;   // floats
   // the partial sums of the waves meet in the slabs' space
   static constexpr int kSumPitch = kNormT + 4;
-  static constexpr int kSums = kWaves * kS * kSumPitch;
+  static constexpr int kSums = kWaves * kNormS * kSumPitch;
   static constexpr size_t kLdsBytes = std::max(kWaves * kSlab, kSums) * 4;
-  static constexpr int kItems =  // 16-byte outputs per thread
-      (kS * kNormT / 4 + kThreads - 1) / kThreads;
-  static constexpr size_t kFixedBytes = ((kWaves + 1) * kRows + 3 * kS + kNormT) * 4;  // (below)
-  static constexpr int kPerCu = kS <= 64 ? 2 : 1;  // workgroups
-  static_assert(kS % 32 == 0 && kS <= 128, "shape");
+  static constexpr size_t kFixedBytes = ((kNormShares + 1) * kRows + 3 * kNormS + kNormT) * 4;  // (below)
+  static constexpr int kPerCu = 16 / kWaves;     // workgroups
   static_assert(kPerCu * (kLdsBytes + kFixedBytes) <= 160 << 10, "LDS per CU");
 };
 
-// Which tile a workgroup takes.  A unit of placement is an utterance or, for batches of fewer than
-// eight, a part of its frames (the parts share lm, the small operand): unit u runs on XCD u % 8,
-// whose L2 then holds its operands.
+// Which tile a workgroup takes.  Only tiles that hold a row <= s_end and a frame <= t_end count.  They
+// are numbered utterance by utterance, the row tiles of a stretch of frames side by side, and dealt
+// out in eight equal runs, one per XCD: every compute unit gets its share, and an utterance's operands
+// lie in the L2 of one XCD or two.  (The grid has room for all tiles; the workgroups that are too
+// many come last and end at once.  With utterance b on XCD b % 8 and a workgroup per tile whether it
+// counts or not, ragged batches left the fullest XCD 15 to 50 % above the average, and workgroups
+// that had nothing to do left holes between those that had.)  Every wave finds its tile itself, a lane
+// per utterance.
 struct NormPlan {
-  int t_tiles, s_tiles, part_shift;
+  int t_tiles, s_tiles;
+  bool all;  // number all tiles: nothing to look up
 };
 struct NormTile {
   int b, s_idx, t_idx;
+  Limits lim;
 };
-__device__ __forceinline__ bool place_tile(int id, const NormPlan &plan, int B, NormTile &o) {
+// Batches of few tiles, counting or not, number them all (launch_normalizer_f32): a tile is then known
+// without a look at the window, whose words arrive beside the first operands.
+__device__ __forceinline__ bool number_tile(int id, const NormPlan &plan, int B, NormTile &o) {
   using dgemm::kXcds;
-  const int t_per = (plan.t_tiles + (1 << plan.part_shift) - 1) >> plan.part_shift;
-  const int unit_tiles = t_per * plan.s_tiles;
-  const int xcd = id % kXcds, slot = id / kXcds, round = slot / unit_tiles;
-  const int within = slot - round * unit_tiles;
-  const int unit = round * kXcds + xcd;
-  o.b = unit >> plan.part_shift;
-  o.s_idx = within / t_per;
-  o.t_idx = (unit & ((1 << plan.part_shift) - 1)) * t_per + (within - o.s_idx * t_per);
-  return o.b < B && o.t_idx < plan.t_tiles;
+  const int of_utterance = plan.s_tiles * plan.t_tiles, total = B * of_utterance;
+  const int per_xcd = (total + kXcds - 1) / kXcds, in_run = id / kXcds;
+  const int n = id % kXcds * per_xcd + in_run;
+  if (in_run >= per_xcd || n >= total) return false;
+  o.b = n / of_utterance;
+  const int within = n - o.b * of_utterance;
+  o.t_idx = within / plan.s_tiles, o.s_idx = within - o.t_idx * plan.s_tiles;
+  return true;
+}
+// inclusive sum over the lanes up to this one
+__device__ __forceinline__ int sum_up_to_lane(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+// row tiles of an utterance that count
+__device__ __forceinline__ int row_tiles(const Limits &lim) {
+  return lim.s_end / kNormS + 1;
+}
+__device__ __forceinline__ bool find_tile(int id, const NormPlan &plan, const int64_t *window, int B,
+                                          int S, int T, int lane, NormTile &o) {
+  using dgemm::kXcds;
+  struct {
+    Limits lim;
+    int tiles;
+  } mine;
+  auto look_up = [&](int b) {
+    mine.lim = limits_of(window, min(b, B - 1), S, T);
+    mine.tiles = b < B ? row_tiles(mine.lim) * min(plan.t_tiles, mine.lim.t_end / kNormT + 1) : 0;
+  };
+  look_up(lane);
+  int sum = sum_up_to_lane(mine.tiles), total = __builtin_amdgcn_readlane(sum, kWave - 1);
+  for (int b0 = kWave; b0 < B; b0 += kWave) {
+    look_up(b0 + lane);
+    total += __builtin_amdgcn_readlane(sum_up_to_lane(mine.tiles), kWave - 1);
+  }
+  const int per_xcd = (total + kXcds - 1) / kXcds, in_run = id / kXcds;
+  int n = id % kXcds * per_xcd + in_run;
+  if (in_run >= per_xcd || n >= total) return false;
+  if (B > kWave) {
+    look_up(lane);
+    sum = sum_up_to_lane(mine.tiles);
+  }
+  int b0 = 0;
+  for (int upto; n >= (upto = __builtin_amdgcn_readlane(sum, kWave - 1)); n -= upto) {
+    b0 += kWave;
+    look_up(b0 + lane);
+    sum = sum_up_to_lane(mine.tiles);
+  }
+  const int at = __builtin_popcountll(__ballot(sum <= n));  // the first lane whose sum exceeds n
+  n -= __builtin_amdgcn_readlane(sum - mine.tiles, at);
+  o.b = b0 + at;
+  o.lim.s_end = __builtin_amdgcn_readlane(mine.lim.s_end, at);
+  o.lim.t_end = __builtin_amdgcn_readlane(mine.lim.t_end, at);
+  const int s_tiles = row_tiles(o.lim);
+  o.t_idx = n / s_tiles, o.s_idx = n - o.t_idx * s_tiles;
+  return true;
 }
 
 struct NormArgs {
@@ -89,45 +157,34 @@ struct NormArgs {
   int B, S, T, C, term, rnnt_type;
 };
 
-// f(a constant), the constant being min(max(n, 1), kMost)
-template <int kMost, typename F>
-__device__ __forceinline__ void with_tiles(int n, F &f) {
-  if constexpr (kMost > 1) {
-    if (n < kMost) return with_tiles<kMost - 1>(n, f);
-  }
-  f(std::integral_constant<int, kMost>{});
-}
-
-template <int kS>
-__global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
+template <int kWaves>
+__global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>::kPerCu)
     simple_fwd_panel_kernel(NormArgs A, NormPlan plan) {
-  using Shape = NormShape<kS>;
-  constexpr int kT = kNormT, kWaves = kNormWaves;
+  using Shape = NormShape<kWaves>;
+  constexpr int kS = kNormS, kT = kNormT, kShares = kNormShares, kTurns = Shape::kTurns;
   constexpr int kRows = Shape::kRows, kLoads = Shape::kLoads, kLmLoads = kS / 16;
-  constexpr int kThreads = Shape::kThreads, kItems = Shape::kItems, kPitch = Shape::kPitch;
+  constexpr int kThreads = Shape::kThreads, kPitch = Shape::kPitch;
   using namespace dgemm;
   extern __shared__ __align__(16) float norm_lds[];
-  __shared__ float factor[kWaves][kRows];      // scale factors for a wave's partial sums
+  __shared__ float factor[kShares][kRows];      // scale factors for a wave's partial sums
   __shared__ float row_term[kS], row_sym[kS];  // lm[s,term], lm[s,sym[s]]
   __shared__ float slab_max[kRows];            // row maxima
   __shared__ int row_symbol[kS];
   __shared__ float col_term[kT];  // am[t,term]
   const int S = A.S, T = A.T, C = A.C, S1 = S + 1;
   NormTile tile;
-  if (!place_tile((int)blockIdx.x, plan, A.B, tile)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (plan.all ? !number_tile((int)blockIdx.x, plan, A.B, tile)
+               : !find_tile((int)blockIdx.x, plan, A.window, A.B, S, T, lane, tile))
+    return;
   const int b = tile.b, s_tile = tile.s_idx * kS, t_tile = tile.t_idx * kT;
   const int T1 = A.rnnt_type == kRegular ? T + 1 : T;
   // With a window only rows <= s_end and frames <= t_end are looked at afterwards (frame
-  // t_end itself only for the -inf that closes the regular lattice): a tile past t_end has
-  // nothing to do -- except the tiles of frame 0, which also store the row maxima of lm
-  // and the lattice's last column -- and 32-row tiles past s_end are not computed.
-  // (The window's words are looked at only after the first slab has been requested, so that
-  // the two round trips to memory overlap; a tile that turns out to have nothing to do has
-  // then requested a slab in vain, range-checked like all the others.)
+  // t_end itself only for the -inf that closes the regular lattice): other tiles are not
+  // computed, nor 32-row tiles past s_end.
   const float *lmb = A.lm + (long)b * S1 * C;
   const float *amb = A.am + (long)b * T * C;
   const int64_t *symb = A.symbols + (long)b * S;
-  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, r32 = lane & 31;
   const float ninf = -__builtin_huge_valf();
@@ -152,10 +209,9 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   const int lm_off = ((s_tile + sub) * C + kq) * 4, am_off = ((t_tile + sub) * C + kq) * 4;  // bytes
   const int step = 16 * C * 4;
   typedef int intx4 __attribute__((ext_vector_type(4)));
-  auto fetch = [&](auto live, floatx4 (&into)[kLoads], int k0) {
+  auto fetch = [&](floatx4 (&into)[kLoads], int k0) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      if (j >= 2 * live && j < kLmLoads) continue;
       // (the wave-uniform part of the offset rides in a scalar register)
       const intx4 raw = j < kLmLoads
                             ? __builtin_amdgcn_raw_buffer_load_b128(lm_rs, lm_off, j * step + k0 * 4, 0)
@@ -185,10 +241,13 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   // meet their partial sums are brought to the true maxima, exp(shift - max) <= 1.
   constexpr float kMargin = 30.f;
   floatx4 slab[kLoads];
-  if (wave < chunks) fetch(std::integral_constant<int, kS / 32>{}, slab, wave * kNormK);
-  const Limits lim = limits_of(A.window, b, S, T);
-  if (t_tile > lim.t_end && t_tile > 0) return;
-  const int live_rows = min(S1, lim.s_end + 1) - s_tile;  // rows that count
+  if (wave < chunks) fetch(slab, wave * kNormK);
+  if (plan.all) {
+    tile.lim = limits_of(A.window, b, S, T);
+    if (t_tile > 0 && t_tile > tile.lim.t_end) return;
+    if (tile.s_idx >= row_tiles(tile.lim)) return;
+  }
+  const int live_rows = min(S1, tile.lim.s_end + 1) - s_tile;  // rows that count
 
   // ---- epilogue inputs, requested behind the first slab so that their latency hides under the
   // loop: the per-row / per-column terms
@@ -199,37 +258,35 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   const float frame_value =
       get_float(am_rs, tid >= 128 && t_tile + tid - 128 < T, (my_frame + A.term) * 4);
   const float my_term = tid < kS ? row_value : frame_value;
-  // ... and am[b, t, sym[b, s]] of this thread's outputs: 16-byte pieces (row item / 8, frames
-  // 4 (item % 8) ..)
-  float am_sym[kItems][4];
-  auto item_row = [&](int j) { return (tid + kThreads * j) / (kT / 4); };
-  const int out_t = 4 * (tid % (kT / 4));
-#pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const int m = item_row(j), sr = s_tile + m;
-    const int y = get_symbol(sym_rs, m < kS && sr < S && m < live_rows, sr, C);
+  // ... and am[b, t, sym[b, s]] of this thread's outputs: a 16-byte piece (row tid / 8, frames
+  // 4 (tid % 8) ..) each for the first 256
+  float am_sym[4];
+  const int out_m = tid / (kT / 4), out_s = s_tile + out_m, out_t = 4 * (tid % (kT / 4));
+  {
+    const int y = get_symbol(sym_rs, out_m < kS && out_s < S && out_m < live_rows, out_s, C);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tr = t_tile + out_t + i;
-      am_sym[j][i] = get_float(am_rs, y >= 0 && tr < T, (tr * C + y) * 4);
+      am_sym[i] = get_float(am_rs, y >= 0 && tr < T, (tr * C + y) * 4);
     }
   }
 
-  float seen[kLoads];     // largest value this lane has met in the row
+  float seen[kTurns][kLoads];     // largest value this lane has met in the row, per share
   // -shift * log2(e), see exp_shifted; the lanes of a row agree on it.  kUnset while the
   // row has shown nothing finite: it sends -inf to exp2(-inf) = 0 and anything finite
   // above the margin.
-  float shift2[kLoads];
+  float shift2[kTurns][kLoads];
   constexpr float kUnset = 3.0e38f;
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) seen[j] = ninf, shift2[j] = kUnset;
-  const int live_tiles = max(1, min(kS / 32, (live_rows + 31) / 32));
+  for (int q = 0; q < kTurns; ++q)
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) seen[q][j] = ninf, shift2[q][j] = kUnset;
   float *mine = norm_lds + wave * Shape::kSlab;
-  floatx16 acc[kS / 32];
+  floatx16 acc[kTurns];
 #pragma unroll
-  for (int j = 0; j < kS / 32; ++j)
+  for (int q = 0; q < kTurns; ++q)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[j][v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[q][v] = 0.f;
 
   auto across_row = [&](float v) {  // maximum over the four lanes that share a row
     v = fmaxf(v, __shfl_xor(v, 1, kWave));
@@ -240,99 +297,91 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
     return __builtin_fmaf(top, kLog2e, shift2_) > kMargin * kLog2e;
   };
   // (the sums are brought along; -across_row(seen) is the new shift)
-  auto raise_shifts = [&](auto live) {
+  auto raise_shifts = [&](auto q) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      if (j >= 2 * live && j < kLmLoads) continue;
-      const float top = across_row(seen[j]);
+      const float top = across_row(seen[q][j]);
       float f = 1.f;
-      if (above_margin(top, shift2[j])) {
-        const float now = fminf(shift2[j], -top * kLog2e);
-        f = __builtin_amdgcn_exp2f(now - shift2[j]);  // exp(old shift - new shift)
-        shift2[j] = now;
+      if (above_margin(top, shift2[q][j])) {
+        const float now = fminf(shift2[q][j], -top * kLog2e);
+        f = __builtin_amdgcn_exp2f(now - shift2[q][j]);  // exp(old shift - new shift)
+        shift2[q][j] = now;
       }
       if (lane % 4 == 0) factor[wave][sub + 16 * j] = f;
     }
     __builtin_amdgcn_wave_barrier();
     const float ft = factor[wave][kS + r32];
 #pragma unroll
-    for (int j = 0; j < live; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        acc[j][v] *= factor[wave][32 * j + 8 * (v / 4) + 4 * half + (v % 4)] * ft;
+    for (int v = 0; v < 16; ++v) acc[q][v] *= factor[wave][8 * (v / 4) + 4 * half + (v % 4)] * ft;
     __builtin_amdgcn_wave_barrier();
   };
   // where this lane's values of a slab row go, and where its operands lie
   float *put = mine + sub * kPitch + kq;
   const float *get = mine + r32 * kPitch + 8 * half;
-  // This wave's share of k, with `live` 32-row tiles that hold lattice rows which count (a
-  // constant: the code of a slab is one straight line, whose rows' chains of dependent
-  // instructions the compiler interleaves -- with a test per row group a slab took 2.5 times as
-  // long).
-  auto look = [&](auto live) {  // maxima; true if a row exceeds its margin
+  // a share of k
+  auto look = [&](auto q) {  // maxima; true if a row exceeds its margin
     bool above = false;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      if (j >= 2 * live && j < kLmLoads) continue;
       // two three-input maxima
-      seen[j] = max3_raw(max3_raw(slab[j][0], slab[j][1], slab[j][2]), slab[j][3], seen[j]);
-      above |= above_margin(seen[j], shift2[j]);
+      seen[q][j] = max3_raw(max3_raw(slab[j][0], slab[j][1], slab[j][2]), slab[j][3], seen[q][j]);
+      above |= above_margin(seen[q][j], shift2[q][j]);
     }
     return above;
   };
-  auto walk = [&](auto live) {
-    int chunk = wave;
+  auto walk_share = [&](auto q) {
+    const int share = wave + kWaves * q;
+    int chunk = share;
     if (chunk < chunks) {  // the first slab sets the shifts: there are no sums to bring along yet
-      (void)look(live);
+      (void)look(q);
 #pragma unroll
       for (int j = 0; j < kLoads; ++j)
-        if (j < 2 * live || j >= kLmLoads)
-          shift2[j] = fminf(shift2[j], -across_row(seen[j]) * kLog2e);
+        shift2[q][j] = fminf(shift2[q][j], -across_row(seen[q][j]) * kLog2e);
     }
-    for (; chunk < chunks; chunk += kWaves) {
+    for (; chunk < chunks; chunk += kShares) {
       // exp(x - shift) to LDS, the request for the slab that takes these registers next, then
       // the products
-      if (__any(look(live))) raise_shifts(live);
+      if (__any(look(q))) raise_shifts(q);
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
-        if (j >= 2 * live && j < kLmLoads) continue;
         floatx4 e;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) e[i] = exp_shifted(slab[j][i], shift2[j]);
+        for (int i = 0; i < 4; ++i) e[i] = exp_shifted(slab[j][i], shift2[q][j]);
         *reinterpret_cast<floatx4 *>(put + j * 16 * kPitch) = e;
       }
-      if (chunk + kWaves < chunks) fetch(live, slab, (chunk + kWaves) * kNormK);
+      int next = chunk + kShares;
+      if (q + 1 < kTurns && next >= chunks) next = share + kWaves;  // (the next share's first)
+      if (next < chunks) fetch(slab, next * kNormK);
       // MFMA i of the slab multiplies k = i (lanes 0..31) and k = i + 8 (lanes 32..63): a lane takes
       // its row's share of the slab with 16-byte reads
-      floatx4 t_op[2], s_op[kS / 32][2];
+      floatx4 t_op[2], s_op[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         t_op[h] = *reinterpret_cast<const floatx4 *>(get + kS * kPitch + 4 * h);
-#pragma unroll
-        for (int j = 0; j < live; ++j)
-          s_op[j][h] = *reinterpret_cast<const floatx4 *>(get + 32 * j * kPitch + 4 * h);
+        s_op[h] = *reinterpret_cast<const floatx4 *>(get + 4 * h);
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < live; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(s_op[j][h][i], t_op[h][i], acc[j], 0, 0, 0);
+          acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(s_op[h][i], t_op[h][i], acc[q], 0, 0, 0);
     }
   };
-  with_tiles<kS / 32>(live_tiles, walk);
+  walk_share(std::integral_constant<int, 0>{});
+  if constexpr (kTurns > 1) walk_share(std::integral_constant<int, 1>{});
 
   // ---- the waves meet: maxima first (each wave's in what was its slab: the row maxima over its
   // share of k, then its final shifts) ...
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) {
-    const float top = across_row(seen[j]);
-    if (lane % 4 == 0) {
-      mine[sub + 16 * j] = top;
-      mine[kRows + sub + 16 * j] = shift2[j];
+  for (int q = 0; q < kTurns; ++q)
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const float top = across_row(seen[q][j]);
+      if (lane % 4 == 0) {
+        mine[2 * kRows * q + sub + 16 * j] = top;
+        mine[2 * kRows * q + kRows + sub + 16 * j] = shift2[q][j];
+      }
     }
-  }
   if (tid < kS) {
     row_term[tid] = my_term;
     row_sym[tid] = my_symval;
@@ -344,14 +393,16 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   float *lm_max = A.lm_max + (long)b * S1, *am_max = A.am_max + (long)b * T;
   if (tid < kRows) {
     const int row = tid;
-    auto met_by = [&](int w, int i) { return norm_lds[w * Shape::kSlab + i]; };
+    auto met_by = [&](int share, int i) {
+      return norm_lds[share % kWaves * Shape::kSlab + share / kWaves * 2 * kRows + i];
+    };
     float r = met_by(0, row);
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) r = fmaxf(r, met_by(w, row));
+    for (int w = 1; w < kShares; ++w) r = fmaxf(r, met_by(w, row));
     // saved for the backward pass; rows that do not exist get a harmless shift
     bool exists;
     if (row < kS) {
-      exists = s_tile + row < S1 && row < 32 * live_tiles;
+      exists = s_tile + row < S1;
       if (s_tile + row < S1 && t_tile == 0) lm_max[s_tile + row] = exists ? r : 0.f;
     } else {
       exists = t_tile + row - kS < T;
@@ -361,47 +412,48 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
     // what brings a wave's partial sums from its shift to the maximum (a wave that met
     // nothing finite in the row holds zeros there)
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w)
+    for (int w = 0; w < kShares; ++w)
       factor[w][row] = exists ? __builtin_amdgcn_exp2f(-__builtin_fmaf(r, kLog2e, met_by(w, kRows + row))) : 1.f;
   }
   __syncthreads();
-  // ... then the partial sums: [wave][kS][kSumPitch] in the slab space
+  // ... then the partial sums: [wave][kS][kSumPitch] in the slab space, a share of every wave at a time
   constexpr int kSumPitch = Shape::kSumPitch;
   const int t_mask = (A.rnnt_type == kRegular && A.boundary) ? (int)A.boundary[4 * b + 3] : -1;
   float *pxb = A.px + (long)b * S * T1;
   float *pyb = A.py + (long)b * S1 * T;
   float *nrb = A.norm_raw ? A.norm_raw + (long)b * S1 * T : nullptr;
-  {
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < kTurns; ++q) {
+    if (q > 0) __syncthreads();
     float *part = norm_lds + wave * kS * kSumPitch;
-    const float ft = factor[wave][kS + r32];
+    const float *my_factor = factor[wave + kWaves * q];
+    const float ft = my_factor[kS + r32];
 #pragma unroll
-    for (int j = 0; j < kS / 32; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = 32 * j + 8 * (v / 4) + 4 * half + (v % 4);
-        part[m * kSumPitch + r32] = acc[j][v] * (factor[wave][m] * ft);
-      }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const int m = item_row(j), sr = s_tile + m, tr = t_tile + out_t;
-    if (m >= kS || sr >= S1 || m >= live_rows) continue;
-    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const floatx4 one =
-          *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + m) * kSumPitch + out_t);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sum[i] += one[i];
+    for (int v = 0; v < 16; ++v) {
+      const int m = 8 * (v / 4) + 4 * half + (v % 4);
+      part[m * kSumPitch + r32] = acc[q][v] * (my_factor[m] * ft);
     }
+    __syncthreads();
+    if (out_m < kS) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const floatx4 one =
+            *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + out_m) * kSumPitch + out_t);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] += one[i];
+      }
+    }
+  }
+  if (out_m < kS && out_s < S1 && out_m < live_rows) {
+    const int m = out_m, sr = out_s, tr = t_tile + out_t;
     floatx4 raw, yv, xv;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       raw[i] = logf(sum[i] + 1.17549435e-38f);
       const float norm = raw[i] + slab_max[m] + slab_max[kS + out_t + i];
       yv[i] = (col_term[out_t + i] + row_term[m]) - norm;
-      xv[i] = (am_sym[j][i] + row_sym[m]) - norm;
+      xv[i] = (am_sym[i] + row_sym[m]) - norm;
       if (row_symbol[m] < 0) xv[i] = std::numeric_limits<float>::quiet_NaN();  // out-of-vocabulary
       if (tr + i == t_mask) xv[i] = ninf;
       xv[i] = A.delay.at(xv[i], A.boundary, b, tr + i, T);
@@ -425,45 +477,21 @@ __global__ void __launch_bounds__(kNormWaves *kWave, 2 * NormShape<kS>::kPerCu)
   // the extra column of the regular lattice: nothing can be emitted after the last frame
   if (A.rnnt_type == kRegular && t_tile == 0 && tid < kS && s_tile + tid < S)
     pxb[(s_tile + tid) * T1 + T] = ninf;
-}
-
-template <int kS>
-void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, hipStream_t stream) {
-  auto kernel = simple_fwd_panel_kernel<kS>;
-  constexpr size_t lds = NormShape<kS>::kLdsBytes;
-  if (!allow_lds(reinterpret_cast<const void *>(kernel), lds)) return;
-  const int t_per = (plan.t_tiles + (1 << plan.part_shift) - 1) >> plan.part_shift;
-  const long units = (long)args.B << plan.part_shift;
-  const unsigned grid = (unsigned)(dgemm::kXcds * ((units + dgemm::kXcds - 1) / dgemm::kXcds) *
-                                   t_per * plan.s_tiles);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS>::kThreads), lds, stream, args, plan);
-}
-
-// The lattice rows of a workgroup's tile: what a model of the kernel's time says is fastest.  A
-// workgroup takes a fixed time and one per round of its eight waves over k, both growing with the
-// rows that count; two of 32 or 64 rows share a compute unit, where their loops take 1.76 times as
-// long as one's, and their fixed parts overlap only once there is more than one round of
-// workgroups.  The constants (microseconds) are fitted to 36 sizes, B 1 .. 128, C 50 .. 5000, that
-// were timed with every row count; over these the choice is 0.4 % (geometric mean) from the best.
-int rows_of_tile(int B, int S, int T, int C) {
-  const int S1 = S + 1, t_tiles = (T + kNormT - 1) / kNormT;
-  const int rounds_of_k = (C + kNormWaves * kNormK - 1) / (kNormWaves * kNormK);
-  int best = 0;
-  double best_us = 0;
-  for (int rows : {32, 64, 96, 128}) {
-    const int s_tiles = (S1 + rows - 1) / rows;
-    const double live = 32.0 * ((S1 + 31) / 32) / s_tiles;  // rows of a tile that count
-    const double fixed = 3.4 + 0.072 * live, loop = rounds_of_k * (0.35 + 0.0172 * live);
-    // workgroups per compute unit (a ragged batch leaves about 0.85 of the tiles to compute)
-    const double per_cu = 0.85 * B * s_tiles * (double)t_tiles / 256;
-    double us;
-    if (rows > 64) us = std::max(1.0, std::ceil(per_cu)) * (fixed + loop);
-    else if (per_cu <= 1) us = fixed + loop;
-    else if (per_cu <= 2) us = 1.58 * fixed + 1.76 * loop;
-    else us = std::ceil(per_cu / 2) * (fixed + 1.76 * loop);
-    if (best == 0 || us < best_us) best = rows, best_us = us;
+  // (and what the row tiles that do not count would have left)
+  if (t_tile == 0 && tile.s_idx == row_tiles(tile.lim) - 1) {
+    for (int s = s_tile + kS + tid; s < S1; s += kThreads) {
+      lm_max[s] = 0.f;
+      if (A.rnnt_type == kRegular && s < S) pxb[s * T1 + T] = ninf;
+    }
   }
-  return best;
+}
+
+template <int kWaves>
+void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, unsigned grid, hipStream_t stream) {
+  auto kernel = simple_fwd_panel_kernel<kWaves>;
+  constexpr size_t lds = NormShape<kWaves>::kLdsBytes;
+  if (!allow_lds(reinterpret_cast<const void *>(kernel), lds)) return;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kWaves>::kThreads), lds, stream, args, plan);
 }
 }  // namespace
 
@@ -472,20 +500,26 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
                            int rnnt_type, hipStream_t stream) {
-  const int rows = rows_of_tile(B, S, T, C);
   const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
                       Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
   NormPlan plan;
   plan.t_tiles = T > 0 ? (T + kNormT - 1) / kNormT : 1;
-  plan.s_tiles = (S + 1 + rows - 1) / rows;
-  plan.part_shift = 0;
-  while (((long)B << plan.part_shift) < dgemm::kXcds && (2 << plan.part_shift) <= plan.t_tiles)
-    ++plan.part_shift;
-  switch (rows) {
-    case 32: launch_fwd_panel<32>(args, plan, stream); break;
-    case 64: launch_fwd_panel<64>(args, plan, stream); break;
-    case 96: launch_fwd_panel<96>(args, plan, stream); break;
-    default: launch_fwd_panel<128>(args, plan, stream);
-  }
+  plan.s_tiles = (S + kNormS) / kNormS;
+  const long tiles = (long)B * plan.t_tiles * plan.s_tiles;
+  const int rounds = (C + kNormShares * kNormK - 1) / (kNormShares * kNormK);
+  // a compute unit for each, or two to a unit that soon end: the look-up would cost more than it gains
+  // (B 70, S 13, T 149, C 80: 9.3 us with it, 8.0 without)
+  plan.all = tiles <= (rounds <= 2 ? 2 : 1) * kComputeUnits || !window;
+  const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
+  // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
+  // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
+  // a compute unit has several workgroups in turn and their loops are short (B 64, S 120, T 600,
+  // C 500: 89 against 98 us; B 13, S 125, T 451, C 60: 12.1 against 14.7; B 10, S 137, T 817, C 500: 26.2
+  // against 28.5), the latter elsewhere (B 23, S 41, T 444, C 444: 15.5 against 16.4; B 98, S 65,
+  // T 209, C 722: 55.7 against 57.3; B 4, S 15, T 47, C 4482: 32 against 42).
+  if (tiles > 3 * kComputeUnits && rounds <= 5)
+    launch_fwd_panel<4>(args, plan, grid, stream);
+  else
+    launch_fwd_panel<8>(args, plan, grid, stream);
 }
 }  // namespace frnnt

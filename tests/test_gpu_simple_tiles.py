@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import fast_rnnt_amd
+from fast_rnnt_amd import _lib
 from oracle import losses as O
 
 pytestmark = pytest.mark.gpu
@@ -47,6 +48,48 @@ def test_simple_loss_at_the_edges_of_tiles(gpu_device, B, S, T, C):
             assert x.grad.dtype == dtype
             off = (x.grad.float().cpu() - y.grad).abs()
             assert bool((off <= 2e-4 + ulp * y.grad.abs()).all()), off.max().item()
+
+
+# (B, S, T, C): fewer and more tiles than compute units, one, two and more waves' lanes of utterances,
+# short and long loops (launch_normalizer_f32 takes eight or four waves)
+WINDOWED = [(3, 40, 70, 33), (9, 200, 300, 700), (64, 63, 65, 90), (65, 31, 200, 40),
+            (130, 64, 129, 20), (300, 5, 33, 9), (40, 33, 256, 1100)]
+
+
+@pytest.mark.parametrize("B,S,T,C", WINDOWED)
+def test_tiles_of_windows_are_the_tiles_of_the_whole_lattice(gpu_device, B, S, T, C):
+    # the tiles that count are found from the windows of the whole batch; each must be there, and hold
+    # the bits that the whole lattice has there
+    g = torch.Generator().manual_seed(B + S)
+    edges_s = torch.tensor([0, 1, 30, 31, 32, 62, 63, 64, S - 1, S]).clamp(max=S)
+    edges_t = torch.tensor([0, 1, 31, 32, 33, 64, T - 1, T]).clamp(max=T)
+    s_end = edges_s[torch.randint(len(edges_s), (B,), generator=g)]
+    t_end = edges_t[torch.randint(len(edges_t), (B,), generator=g)]
+    s_end[B // 2], t_end[B // 2] = S, T
+    boundary = torch.stack([torch.zeros_like(s_end)] * 2 + [s_end, t_end], 1).to(gpu_device)
+    lm = torch.randn(B, S + 1, C, generator=g).to(gpu_device)
+    am = torch.randn(B, T, C, generator=g).to(gpu_device)
+    symbols = torch.randint(0, C, (B, S), generator=g).to(gpu_device)
+
+    def run(window_only):
+        shapes = [(B, S, T + 1), (B, S + 1, T), (B, S + 1), (B, T), (B, S + 1, T)]
+        out = [torch.full(n, float("nan"), device=gpu_device) for n in shapes]
+        _lib.call("frnnt_simple_logprobs_fwd_f32", lm.data_ptr(), am.data_ptr(), symbols.data_ptr(),
+                  boundary.data_ptr(), *(x.data_ptr() for x in out), B, S, T, C, 0, 0, window_only,
+                  _lib.stream_of(am))
+        return out
+
+    whole, windowed = run(0), run(1)
+    s = torch.arange(S + 1, device=gpu_device).view(1, -1, 1)
+    t = torch.arange(T + 1, device=gpu_device).view(1, 1, -1)
+    rows, frames = s <= boundary[:, 2].view(-1, 1, 1), t < boundary[:, 3].view(-1, 1, 1)
+    last = t <= boundary[:, 3].view(-1, 1, 1)  # (the -inf that closes the lattice)
+    px_there = (rows[:, :S] & last) | (t == T)
+    there = [px_there, rows & frames[:, :, :T], rows[:, :, 0], frames[:, 0, :T],
+             rows & frames[:, :, :T]]
+    for got, want, here in zip(windowed, whole, there):
+        assert not torch.isnan(want).any()
+        assert torch.equal(got[here], want[here])
 
 
 # (S, T, C, s_end, t_end): sums over k that end before, at and after a chunk of 32 and a k-step of 16,
