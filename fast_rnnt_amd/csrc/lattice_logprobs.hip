@@ -104,7 +104,6 @@ __device__ __forceinline__ float row_entry(const intx4 (&raw)[kVecs], int off, i
 template <typename P, int kLanes, int kVecs, bool kLoop, bool kStream>
 __global__ void __launch_bounds__(256)
     row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out) {
-  constexpr int kAux = kStream ? 2 : 0;
   constexpr int kRows = kWave / kLanes;
   const int b = block_batch();
   if (b >= L.B) return;
@@ -122,15 +121,23 @@ __global__ void __launch_bounds__(256)
       pieces_of<P, kLanes>(base, reinterpret_cast<uintptr_t>(logits + row.index * L.C), L.C);
   const float ninf = -__builtin_huge_valf();
   float m = ninf, sum = 0, shift = 0;
+  // (wave-uniform) the rows that the backward will look at first stay in the cache
+  const bool past_cache =
+      kStream && ((long)L.B * L.T * L.Rr - first) * L.C * (long)sizeof(typename P::Elem) > kKeptBytes;
   intx4 raw[kVecs];
   for (int p0 = 0; p0 < (kLoop ? q.pieces : 1); p0 += kLanes * kVecs) {
+    auto load_pieces = [&](auto aux) {
 #pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-      const int p = p0 + lane + kLanes * i;
-      const bool wanted = (kRows == 1 || row.live) && p < q.pieces;
-      raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, wanted ? q.at + 16 * p : kOutOfRange, 0,
-                                                     kAux);
-    }
+      for (int i = 0; i < kVecs; ++i) {
+        const int p = p0 + lane + kLanes * i;
+        const bool wanted = (kRows == 1 || row.live) && p < q.pieces;
+        raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, wanted ? q.at + 16 * p : kOutOfRange, 0, aux);
+      }
+    };
+    if (kStream && past_cache)
+      load_pieces(std::integral_constant<int, 2>{});
+    else
+      load_pieces(std::integral_constant<int, 0>{});
     // entries that are not the row's become -inf (whole pieces of a whole wave need no test)
 #pragma unroll
     for (int i = 0; i < kVecs; ++i) {

@@ -181,8 +181,7 @@ inline dim3 batch_grid(long blocks, int B) {
 // before the first is used, through a raw buffer resource over the wave's rows: a piece that is
 // not wanted gets an offset outside it, reads as 0 and moves no data -- no branch stands between
 // the loads.  kLoop: rows of more pieces than registers, in chunks of kLanes * kVecs.
-// kStream: logits that the last-level cache cannot hold until the backward pass are read
-// with the non-temporal hint.
+// kStream: see kStreamBytes.
 template <typename P, int kLanes>
 struct RowPieces {
   int off;      // elements of the first piece that lie before the row
@@ -213,10 +212,19 @@ __device__ __forceinline__ long wave_bytes(int C) {
   return ((long)(kWave / kLanes) * C * (long)sizeof(typename P::Elem) + 31) & ~15L;
 }
 
-// Logits beyond this many bytes do not stay in the last-level cache between the forward
-// and the backward pass: they are streamed (non-temporal hint), which leaves the cache to
-// what is used again.  Below it the hint costs (a 80 MB gradient pass: 23.8 -> 26.6 us).
-constexpr long kStreamBytes = 192L << 20;
+// Logits beyond this many bytes are streamed (non-temporal hint): the gradient as it is read and
+// written, which leaves the last-level cache (256 MB) to the logits of the next forward pass and
+// of this one, and, of the forward, the rows further than kKeptBytes from the end.  The backward starts
+// from the end, where it finds in the cache what the forward read last.  Forward + backward, five rows a
+// frame, B 20, T 500, against 192 MiB, a forward streamed throughout and a backward from the
+// first row on: C 560, 112 MB: 29.4 + 32.4 -> 27.1 + 31.3 us; C 900: 39.2 + 51.8 -> 30.4 + 49.4; C 1300:
+// 34.9 + 81.6 -> 37.6 + 69.2; the whole lattice, B 8, S 60, T 200, C 1000, 390 MB: 53 + 115 -> 55 + 95;
+// bfloat16, B 16, T 400, C 5000, 320 MB: 46 + 100 -> 49 + 89; 1.6 GB (B 32, S 60, T 200, C 1000): 195 +
+// 482 -> 200 + 471.  Below the line the hint costs (80 MB: 20.1 + 24.0 -> 21.2 + 25.4).
+constexpr long kStreamBytes = 96L << 20;
+// (1.5 times the cache: of a ragged batch a fifth to a third is never read.  B 8, S 60, T 200, C 1000:
+// backward 121 us with 128 MiB, 116 with 192, 108 with 256, 100 with 320, 95 with 384.)
+constexpr long kKeptBytes = 384L << 20;
 
 // Whether every row begins and ends on 16 bytes.
 template <typename P>

@@ -88,3 +88,25 @@ def test_gradients_of_aligned_rows_are_the_bits_of_any_others(gpu_device, sfx, d
             assert bool((out[:out_off] == 7).all()) and bool((out[out_off + n:] == 7).all())
             results.append(out[out_off:out_off + n])
         assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
+@pytest.mark.parametrize("B,C", [(3, 750), (12, 751)])
+def test_streamed_logits_give_the_bits_of_their_utterances(gpu_device, B, C):
+    # 110 and 440 MB: past the size from which logits are streamed, and past the one from which the
+    # forward streams the rows that lie far from the end; an utterance alone takes neither path
+    T, S = 200, 60
+    g = torch.Generator(device=gpu_device).manual_seed(C)
+    logits = torch.randn(B, T, S + 1, C, generator=g, device=gpu_device)
+    symbols = torch.randint(1, C, (B, S), generator=g, device=gpu_device)
+    ends = torch.tensor([[0, 0, S - 5 * (b % 3), T - 17 * (b % 4)] for b in range(B)], device=gpu_device)
+
+    def run(rows):
+        leaf = logits[rows].clone().requires_grad_(True)
+        loss = fast_rnnt_amd.rnnt_loss(leaf, symbols[rows], 0, boundary=ends[rows], reduction="none")
+        loss.sum().backward()
+        return loss.detach(), leaf.grad
+
+    loss, grad = run(slice(0, B))
+    for b in range(B):
+        one_loss, one_grad = run(slice(b, b + 1))
+        assert torch.equal(loss[b:b + 1], one_loss) and torch.equal(grad[b:b + 1], one_grad)
