@@ -7,11 +7,12 @@
 // per logits row (b, t, j), which forms norm = logsumexp and the two picked log-probs
 //   x = logits[b,t,j,sym(b, ranges[b,t,j])] - norm   (sym(b, S) = termination symbol)
 //   y = logits[b,t,j,term] - norm.
-// Without ranges (and without the constrained step) every cell of px / py comes from one row,
-// which writes it.  Otherwise the picks go to xr / yr and a second, small kernel lays them
-// out: row j of frame t lands at lattice row (j + ranges[b,t,0]) mod (S+1), everything
-// else is -inf, plus the -inf columns of the regular lattice and the constrained
-// "px += py[:, 1:]" step.  (The backward: lattice_gradient.hip.)
+// Without the constrained step every cell of px / py comes from one row, which writes it: row j of
+// frame t lands at lattice row (j + ranges[b,t,0]) mod (S+1).  The cells around the rows' --
+// everything else is -inf, and the -inf columns of the regular lattice -- are written by
+// workgroups of their own in the same launch.  The constrained "px += py[:, 1:]" step needs two rows
+// in one cell: there (and in float64) the picks go to xr / yr and a second, small kernel lays
+// them out.  (The backward: lattice_gradient.hip.)
 #include "lattice_rows.hip.h"
 
 namespace frnnt {
@@ -101,15 +102,51 @@ __device__ __forceinline__ float row_entry(const intx4 (&raw)[kVecs], int off, i
   return P::at(intx4{word, word, word, word}, e % kPerWord);
 }
 
+// The cells of px / py that no row of the logits is placed at: tiles of 64 columns x 32 lattice rows
+// like assemble_kernel's, lanes along t, the first `blocks` of an utterance's workgroups.  They write
+// nothing that a row writes, but for the -inf of closed columns, so that neither waits for the
+// other.  (With a launch of its own after the rows', which laid out what they had left in xr / yr,
+// B 32, S 80, T 250, C 500, five rows a frame, took 20.2 + 5.7 us, now 24.0; B 8, S 200, T 1200, C 400,
+// eight rows: 38.4 + 13.2, now 42.3.)
+constexpr int kAssembleRows = 32;
+struct Surround {
+  unsigned blocks;
+  int t_tiles;
+  __device__ __forceinline__ void fill(const Lattice &L, int b, unsigned block, float *px,
+                                       float *py) const {
+    const bool regular = L.rnnt_type == kRegular;
+    const int T1 = regular ? L.T + 1 : L.T, S1 = L.S + 1;
+    const int t = (int)(block % t_tiles) * 64 + (threadIdx.x & 63);
+    const int s0 = (int)(block / t_tiles) * kAssembleRows + (threadIdx.x >> 6);
+    if (L.window) {
+      const int64_t *w = L.window + 4 * b;
+      if ((t & ~63) > w[3] || (t | 63) < w[1] || (s0 & ~3) > w[2] || (s0 & ~3) + kAssembleRows <= w[0])
+        return;
+    }
+    const int r0 = placed_at(L.ranges[((long)b * L.T + min(t, L.T - 1)) * L.Rr], 0, L.S);
+    const bool closed = regular && L.boundary && L.boundary[4 * b + 3] == t;
+    float *px_b = px + (long)b * L.S * T1, *py_b = py + (long)b * S1 * L.T;
+#pragma unroll
+    for (int k = 0; k < kAssembleRows / 4; ++k) {
+      const int s = s0 + 4 * k, rel = s - r0 < 0 ? s - r0 + S1 : s - r0;
+      const bool placed = rel < L.Rr && t < L.T;
+      if (s < L.S && t < T1 && (!placed || closed)) px_b[(long)s * T1 + t] = Num<float>::neg_inf();
+      if (s < S1 && t < L.T && !placed) py_b[(long)s * L.T + t] = Num<float>::neg_inf();
+    }
+  }
+};
+
 template <typename P, int kLanes, int kVecs, bool kLoop, bool kStream>
 __global__ void __launch_bounds__(256)
-    row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out) {
+    row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out,
+                    Surround around) {
   constexpr int kRows = kWave / kLanes;
   const int b = block_batch();
   if (b >= L.B) return;
+  if (blockIdx.x < around.blocks) return around.fill(L, b, blockIdx.x, out.px, out.py);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register
   const int lane = threadIdx.x & (kLanes - 1);
-  const unsigned r0 = (blockIdx.x * 4 + wave) * kRows;
+  const unsigned r0 = ((blockIdx.x - around.blocks) * 4 + wave) * kRows;
   const unsigned r = kRows == 1 ? r0 : r0 + (threadIdx.x & 63) / kLanes;
   const Row row = locate(L, b, r);
   if (!row.live && lane == 0) out.skip(L, row);
@@ -199,21 +236,31 @@ __global__ void __launch_bounds__(256)
               at_term - lse);
 }
 
+// (rows in 16-byte pieces; else the plain kernel takes them)
+template <typename P>
+bool rows_in_pieces(int C) {
+  return !std::is_same<P, DoublePiece>::value && (long)C * (long)sizeof(typename P::Elem) < (1L << 26);
+}
 template <typename P, typename R>
 void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Picks<R> &out,
                      hipStream_t stream) {
   const long rows = (long)L.T * L.Rr;
   if constexpr (!std::is_same<P, DoublePiece>::value) {
-    if ((long)L.C * (long)sizeof(typename P::Elem) < (1L << 26)) {
+    if (rows_in_pieces<P>(L.C)) {
+      Surround around{0, 1};
+      if (L.ranges && out.direct) {
+        around.t_tiles = (L.T + (L.rnnt_type == kRegular ? 1 : 0) + 63) / 64;
+        around.blocks = (unsigned)around.t_tiles * ((L.S + kAssembleRows) / kAssembleRows);
+      }
       const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) > kStreamBytes;
       with_row_split<P>(logits, L.C, [&](auto lanes, auto vecs, auto loop) {
-        const dim3 grid = batch_grid((rows + 256 / lanes - 1) / (256 / lanes), L.B);
+        const dim3 grid = batch_grid(around.blocks + (rows + 256 / lanes - 1) / (256 / lanes), L.B);
         if (big && lanes == 64)
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, lanes == 64>), grid, dim3(256),
-                             0, stream, logits, L, out);
+                             0, stream, logits, L, out, around);
         else
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, false>), grid, dim3(256), 0,
-                             stream, logits, L, out);
+                             stream, logits, L, out, around);
       });
       return;
     }
@@ -225,7 +272,6 @@ void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Pic
 // px / py of a tile of 64 columns x 32 lattice rows: lanes along t (coalesced stores), a frame's
 // first range entry read once per lane, four waves with eight rows each.  Tiles that the
 // recursion cannot reach are left alone when the caller allows it.
-constexpr int kAssembleRows = 32;
 template <typename R>
 __global__ void __launch_bounds__(256)
     assemble_kernel(const R *__restrict__ xr, const R *__restrict__ yr, Lattice L,
@@ -309,7 +355,7 @@ int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
   const Lattice L{symbols, ranges, boundary, window_only ? boundary : nullptr, B, S, T, Rr, C,
                   term, rnnt_type};
   const Delay<R> delay{(R)delay_penalty};
-  const bool direct = !ranges && rnnt_type != kConstrained;
+  const bool direct = rnnt_type != kConstrained && (!ranges || rows_in_pieces<P>(C));
   if (T > 0)
     launch_row_norm<P, R>(static_cast<const typename P::Elem *>(logits_), L,
                           Picks<R>{norm, xr, yr, px, py, delay, direct}, stream);

@@ -804,3 +804,33 @@ def test_c3_pruned_full_size(gpu_device):
     assert _close(ggx, wgx, bound) and _close(ggy, wgy, bound)
     # am.grad / lm.grad add such cells up over lattice rows / frames
     assert _close(da.grad, a.grad, 2 * bound, 1e-3) and _close(dl.grad, l.grad, 2 * bound, 1e-3)
+
+
+# (B, S, T, R, C): lattices on either side of the tiles that fill the cells around the rows (64 columns
+# x 32 lattice rows), few and many rows of them, rows that share a wave and rows of their own
+@pytest.mark.parametrize("kind", ["regular", "modified"])
+@pytest.mark.parametrize("B,S,T,R,C", [(1, 1, 1, 1, 5), (2, 31, 63, 32, 40), (3, 32, 64, 5, 70),
+                                       (2, 33, 65, 3, 300), (2, 64, 130, 8, 33), (1, 95, 128, 2, 600)])
+def test_every_cell_of_the_pruned_lattice_is_written(gpu_device, kind, B, S, T, R, C):
+    g = torch.Generator().manual_seed(S + T)
+    logits = torch.randn(B, T, R, C, generator=g)
+    symbols = torch.randint(0, C, (B, S), generator=g)
+    # (also ranges that begin near the end and wrap around, which the roll places at the front)
+    begin = torch.randint(0, S + 1, (B, T), generator=g)
+    ranges = (begin.unsqueeze(2) + torch.arange(R)) % (S + 1)
+    ends = torch.tensor([[0, 0, S, T]] + [[0, 0, max(1, S - 7), max(S - 7, T - 9, 1)]] * (B - 1))
+    for boundary in (None, ends):
+        want = O.lattice_logprobs_pruned(logits, symbols, ranges, 0, boundary=boundary, rnnt_type=kind)
+        # the allocator hands out what was freed last: a cell that nothing writes would be seen as NaN
+        poison = [torch.full(w.shape, float("nan"), device=gpu_device) for w in want]
+        del poison
+        got = fast_rnnt_amd.get_rnnt_logprobs_pruned(
+            logits.to(gpu_device), symbols.to(gpu_device), ranges.to(gpu_device), 0,
+            boundary=None if boundary is None else boundary.to(gpu_device), rnnt_type=kind)
+        # a cell is the difference of a logit and a log-sum, both below 16 here: 2^-21 for the roundings
+        # to such values, and as much again per side for the log and the sum of the exponentials
+        for x, y in zip(got, want):
+            x = x.cpu()
+            assert torch.equal(torch.isinf(x), torch.isinf(y))
+            there = ~torch.isinf(y)
+            assert bool(((x - y)[there].abs() <= 2 ** -19).all())
