@@ -70,6 +70,11 @@ constexpr int kBwdStagers = 3;
 // forward kernel's only copy (then 18.45 us with 2, 18.05 with 3, 17.9 with 4).
 constexpr int kFwdStagersFew = 4;
 constexpr int kBwdStagersFew = 7;
+// How many tiles ahead of the one it stages a forward staging wave requests inputs (see the loop below).
+// (Doubles have no registers for a second set.  Backward the second set costs more than it gives: the
+// code there has no scalar registers left, B 64, S 120, T 600: 37 -> 41 us.)
+template <typename R>
+constexpr int kFetchAhead = sizeof(R) == 4 ? 2 : 1;
 constexpr int kSpinLimit = 1 << 22;   // polls before a wait gives up (seconds, not microseconds)
 struct Window {
   int s0, t0, ns, nt;  // origin and extent (ns = s_end - s_begin, ...)
@@ -514,26 +519,27 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     const int half = lane >> 5, q = lane & 31;
     // rows of a tile this wave stages: r(u) = 2*l + half + 2*kStagers*u
     constexpr int kRows = (kWave + 2 * kStagers - 1) / (2 * kStagers);
+    constexpr int kAhead = kFetchAhead<R>;
     struct Staged {
       R x[kRows], y[kRows];
     };
-    // Global fetches of tile m+1 are issued (into registers) as soon as tile m is staged,
-    // before this wave waits for the next LDS buffer, so their latency overlaps the
-    // sweep.  The loads are range-checked and otherwise unconditional: what a lane reads
-    // for cells outside the window is either replaced at staging time (row 0, column 0:
-    // the -inf that closes the lattice) or never reaches a cell of the window (columns
-    // before a row's start or beyond its end only feed cells at least as far out).
+    // Global fetches (into registers) are issued kAhead tiles before they are staged, so that their
+    // latency overlaps the sweep.  The loads are range-checked and otherwise unconditional: what a lane
+    // reads for cells outside the window is either replaced at staging time (row 0, column 0: the -inf
+    // that closes the lattice) or never reaches a cell of the window (columns before a row's start or
+    // beyond its end only feed cells at least as far out).
     const __amdgpu_buffer_rsrc_t px_rsrc = buffer_of(const_cast<R *>(pxb), (size_t)S * T1);
     const __amdgpu_buffer_rsrc_t py_rsrc = buffer_of(const_cast<R *>(pyb), (size_t)(S + 1) * T);
-    const __amdgpu_buffer_rsrc_t p_rsrc = buffer_of(pb, (size_t)(S + 1) * TP);
+    // (what is stored: the rows of the window, so that a row beyond them is outside the resource)
+    const __amdgpu_buffer_rsrc_t p_rsrc = buffer_of(pb + (size_t)win.s0 * TP, (size_t)(NS + 1) * TP);
     constexpr int kStep = 2 * kStagers;
     constexpr int kSize = (int)sizeof(R);
     const int r_first = 2 * l + half;
     auto fetch = [&](Staged &in, const Band &g, int m) {
       const int s_first = win.s0 + g.row0 + r_first;
       const int j_first = m * kTileSteps + q - r_first;
-      const int x0 = ((s_first - 1) * T1 + win.t0 + j_first - shift) * kSize;
-      const int y0 = (s_first * T + win.t0 + j_first - 1) * kSize;
+      const int x0 = m < g.ntiles ? ((s_first - 1) * T1 + win.t0 + j_first - shift) * kSize : kDropped;
+      const int y0 = m < g.ntiles ? (s_first * T + win.t0 + j_first - 1) * kSize : kDropped;
 #pragma unroll
       for (int u = 0; u < kRows; ++u) {
         // kStep rows further up: as many rows down in memory, as many columns left
@@ -543,12 +549,18 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     };
     // p of tile pm of the band that starts at row0, left by the sweep wave in buffer `buf`:
     // element (row r, step q) is the cell (row0 + r, 32 pm + q - r) of the window.  Taking
-    // it out of the buffer and storing it are two steps: a wave's wait for a load also
-    // waits for every store it has issued before, so the stores of a tile go out after
+    // it out of the buffer and storing it are two steps: the stores of a tile go out after
     // the buffer has been refilled and handed back to the sweep wave, not before.
     struct Drained {
       R v[kRows];
       int row0, pm;
+    };
+    constexpr int kNowhere = -(1 << 20);  // (a tile with no cell in the window)
+    // As many stores as a tile's, all dropped: outside the resources that the loads come from, which
+    // keeps the compiler from moving them before the loads.
+    auto store_nothing = [&]() {
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) put1(u & 1 ? py_rsrc : px_rsrc, kDropped + u * kSize, (R)0);
     };
     auto take = [&](Drained &d, int row0, int pm, int buf) {
       const R *ps = base + buf * kTileElems + r_first * kTilePitch + q;
@@ -574,51 +586,57 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     auto store = [&](const Drained &d) {
       const int i0 = d.row0 + r_first;
       const int j0 = d.pm * kTileSteps + q - r_first;
-      const int o0 = ((win.s0 + i0) * TP + win.t0 + j0) * kSize;
+      const int o0 = (i0 * TP + win.t0 + j0) * kSize;
 #pragma unroll
       for (int u = 0; u < kRows; ++u) {
-        if (r_first + kStep * u >= kWave) continue;
-        const int i = i0 + kStep * u, j = j0 - kStep * u;
-        const bool ok = i <= NS && (unsigned)j <= (unsigned)NT;
+        const bool ok = (unsigned)(j0 - kStep * u) <= (unsigned)NT && r_first + kStep * u < kWave;
         put1(p_rsrc, ok ? o0 + u * (kStep * (TP - 1) * kSize) : kDropped, d.v[u]);
       }
     };
-    // which tile each buffer holds: its band's first row and its number in the band
-    int held_row0[kBuffers], held_m[kBuffers];
+    // The tile that a buffer held before tile m of the band that starts at row0.  Bands that
+    // another one follows have whole_tiles tiles, two at least, so that it lies two bands back at most.
+    const int whole_tiles = (NT + kWave + kTileSteps - 1) / kTileSteps;
+    auto take_buffer = [&](Drained &d, int row0, int m, int buf) {
+      int pm = m - kBuffers;
 #pragma unroll
-    for (int k = 0; k < kBuffers; ++k) held_row0[k] = held_m[k] = 0;
-    auto take_buffer = [&](Drained &d, int buf) {
-      int row0 = held_row0[0], pm = held_m[0];
-#pragma unroll
-      for (int k = 1; k < kBuffers; ++k) {
-        row0 = buf == k ? held_row0[k] : row0;
-        pm = buf == k ? held_m[k] : pm;
+      for (int k = 0; k < 2; ++k) {
+        row0 = pm < 0 ? row0 - band_rows : row0;
+        pm = pm < 0 ? pm + whole_tiles : pm;
       }
       take(d, row0, pm, buf);
     };
     int tile_base = 0, buf = 0;  // buf = tile number modulo kBuffers
+    int end_row0 = 0, end_tiles = 0;
     for (int band = part; band * band_rows <= last_row; ++band) {
       const Band g = band_of(band, w, nsweep, NS, NT);
       if (g.row0 > NS) break;
-      Staged cur;
-      fetch(cur, g, 0);
-      for (int m = 0; m < g.ntiles; ++m) {
+      // A wave's memory accesses are counted off in their order, so that a wait for a load is also one
+      // for every access issued before it, and for those issued after it that the compiler cannot count
+      // on.  With one tile requested at a time, behind the stores of the tile before, a tile's staging
+      // took the latency of both, longer than the sweep needs for a tile.  Here two tiles' inputs are on
+      // their way, in two sets of registers, and on every path exactly one tile's loads and one tile's
+      // stores follow each other -- dropped ones where there is nothing to fetch or to store, and a wait
+      // that ran out ends the loop only after both halves -- so that the wait for a tile's inputs leaves
+      // the later loads and stores on their way.  (B 64, S 120, T 600: 37.4 -> 32.2 us, 29.4 with no
+      // stores at all; B 12, S 220, T 1500: 68.0 -> 65.7; B 32, S 80, T 250: 17.0 -> 16.2.)
+      Staged ahead[kAhead];
+      Drained out = {};
+      out.pm = kNowhere;
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        fetch(ahead[k], g, k);
+        store_nothing();
+      }
+      auto stage = [&](const Staged &cur, int m) __attribute__((always_inline)) -> bool {
         const int gt = tile_base + m;
-        Drained out;
-        const bool refill = gt >= kBuffers;
-        if (refill) {
+        if (gt >= kBuffers) {
           // the buffer still holds p of tile gt - kBuffers
           if (!wait_for(&cnt.written[w], gt - kBuffers + 1, spin_limit)) {
             give_up();
-            return;
+            return false;
           }
-          take_buffer(out, buf);
+          take_buffer(out, g.row0, m, buf);
           hand_on(out);
-        }
-#pragma unroll
-        for (int k = 0; k < kBuffers; ++k) {
-          held_row0[k] = buf == k ? g.row0 : held_row0[k];
-          held_m[k] = buf == k ? m : held_m[k];
         }
         // The row above the band belongs to another sweep wave: what it feeds into the band's first
         // row is added to that row's x here (the sweep would add it with the same rounding), so
@@ -631,11 +649,14 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
           const int before = kApart ? 0 : (w > 0 ? band : band - 1) * cols;
           if (need > 0 && !wait_for(&cnt.ready[prev], before + need, spin_limit)) {
             give_up();
-            return;
+            return false;
           }
           seam_value = ninf;
           if (there) seam_value = up_seam[col];
         }
+        // (the wait for this tile's inputs, on every path through what follows)
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) asm volatile("" ::"v"(cur.x[u]), "v"(cur.y[u]));
         R *xdst = base + buf * kTileElems + r_first * kTilePitch + q;
         R *ydst = xdst + kBuffers * kTileElems;
         // only the first tiles hold a column 0 (local step = row), and only the first
@@ -659,12 +680,26 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
         }
         // every lane's LDS writes precede the release by lane 0 of the same wave
         if (lane == 0) count_in(&cnt.loaded[w * kBuffers + buf]);
-        if (refill) store(out);
-        // the next tile's inputs, fetched while this wave waits for its buffer
-        if (m + 1 < g.ntiles) fetch(cur, g, m + 1);
         buf = buf + 1 == kBuffers ? 0 : buf + 1;
+        return true;
+      };
+      bool failed = false;
+      for (int m = 0; m < g.ntiles; m += kAhead) {
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+          if (m + k < g.ntiles && !failed)
+            failed = !stage(ahead[k], m + k);
+          else
+            out.pm = kNowhere;
+          fetch(ahead[k], g, m + k + kAhead);
+          asm volatile("" ::: "memory");
+          store(out);
+        }
+        if (failed) return;
       }
       tile_base += g.ntiles;
+      end_row0 = g.row0;
+      end_tiles = g.ntiles;
     }
     // the tiles still in the buffers
     const int first_left = max(tile_base - kBuffers, 0);
@@ -675,7 +710,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
         return;
       }
       Drained out;
-      take_buffer(out, buf);
+      take_buffer(out, end_row0, gt - tile_base + end_tiles + kBuffers, buf);
       hand_on(out);
       store(out);
       buf = buf + 1 == kBuffers ? 0 : buf + 1;

@@ -159,6 +159,21 @@ def test_taller_than_one_workgroup(gpu_device):
     _compare(px32, py32, None, torch.ones(B), gpu_device, "tall32")
 
 
+@pytest.mark.parametrize("S", [64, 255, 256, 575, 577])
+def test_few_tiles_in_many_bands(gpu_device, S):
+    # A buffer is emptied of a tile that lies one or two bands of 64 rows back when a band has fewer
+    # tiles than there are buffers or inputs on their way: bands of two (T 1), three (T 2, 32) and
+    # four tiles (T 33), the last band with as few as one.
+    g = torch.Generator().manual_seed(S)
+    for T in (1, 2, 32, 33):
+        px = -0.7 + 0.3 * torch.randn(3, S, T + 1, generator=g)
+        py = -0.7 + 0.3 * torch.randn(3, S + 1, T, generator=g)
+        bnd = torch.tensor([[0, 0, S, T], [S // 3, 0, S, T], [1, T // 2, S - S // 4, T]], dtype=torch.int64)
+        for b in range(3):
+            px[b, :, bnd[b, 3]] = -math.inf
+        _compare(px, py, bnd, torch.ones(3), gpu_device, f"bands{S}x{T}")
+
+
 def test_long_utterance_two_tile_buffers(gpu_device):
     # T beyond what three LDS tile buffers per sweep wave leave room for (about 6100 frames
     # with two sweep waves): the float kernels fall back to two buffers and fewer staging
