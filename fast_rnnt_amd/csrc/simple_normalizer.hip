@@ -507,9 +507,14 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
   plan.s_tiles = (S + kNormS) / kNormS;
   const long tiles = (long)B * plan.t_tiles * plan.s_tiles;
   const int rounds = (C + kNormShares * kNormK - 1) / (kNormShares * kNormK);
-  // a compute unit for each, or two to a unit that soon end: the look-up would cost more than it gains
-  // (B 70, S 13, T 149, C 80: 9.3 us with it, 8.0 without)
-  plan.all = tiles <= (rounds <= 2 ? 2 : 1) * kComputeUnits || !window;
+  // A compute unit for each tile, or two to a unit that soon end or belong to lattices of a single row of
+  // tiles, of which only the frames are ragged: the look-up would cost more than it gains.  (B 70, S 13,
+  // T 149, C 80: 9.3 us with it, 8.0 without; one row of 384 to 500 tiles, B 96, S 14, T 114, C 854: 20.2 and
+  // 19.2; B 128, S 10, T 100, C 500: 16.1 and 14.6; B 110, S 28, T 128, C 640: 18.7 and 17.4.  Two rows of
+  // them, B 25, S 50, T 258, C 1400: 26.7 and 37.8; one row of more than two to a unit, B 80, S 12, T 250,
+  // C 1500: 45 and 53; B 128, S 20, T 300, C 500: 30.5 and 34.5.)
+  const bool two = rounds <= 2 || plan.s_tiles == 1;
+  plan.all = tiles <= (two ? 2 : 1) * kComputeUnits || !window;
   const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
   // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
   // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
