@@ -38,19 +38,18 @@ namespace {
 // 32 to 128 rows with a workgroup per tile whether it counted or not: B 64, S 120, T 600, C 500: 96 ->
 // 89 us; B 32, S 80, T 250, C 500: 20.4 and 20.6; B 16, S 120, T 400, C 5000: 127 -> 122; B 10, S 137,
 // T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64 sizes, B 1 .. 128,
-// C 50 .. 5000: 5.6 %, the worst of them B 8, S 100, T 400, C 5000: 73 -> 81.  Tiles of 64, 96 and
-// 128 rows dealt out the same way were the fastest at 12 of the 64, mostly by 1 to 5 %, and a choice
-// among all of them, which cannot know how ragged a batch is, gained nothing over this one.
+// C 50 .. 5000: 5.6 %.  Tiles of 64, 96 and 128 rows dealt out the same way were the fastest at 12 of the
+// 64, mostly by 1 to 5 %, and a choice among all of them, which cannot know how ragged a batch is, gained
+// nothing; 64 rows are left where they have a compute unit each (launch_normalizer_f32).
 constexpr int kNormK = 16;      // k per slab
 constexpr int kNormShares = 8;  // of k
-constexpr int kNormS = 32;      // lattice rows of a tile
 constexpr int kNormT = 32;      // frames of a tile
 constexpr int kComputeUnits = 256;
-template <int kWaves_>
+template <int kS, int kWaves_>
 struct NormShape {
   static constexpr int kWaves = kWaves_, kThreads = kWaves * kWave;
   static constexpr int kTurns = kNormShares / kWaves;  // shares of a wave, one after the other
-  static constexpr int kRows = kNormS + kNormT;  // rows of a slab: lm rows, then am rows
+  static constexpr int kRows = kS + kNormT;      // rows of a slab: lm rows, then am rows
   static constexpr int kLoads = kRows / 16;      // 16-byte loads per lane and slab
   // Row pitch in LDS: 20 floats.  Rows start 16-byte aligned, so a lane's four values of a row go
   // in as one 16-byte write, and a lane reads its row's eight k of a slab half as two 16-byte reads:
@@ -59,10 +58,13 @@ struct NormShape {
   static constexpr int kSlab = kRows * kPitch;   // floats
   // the partial sums of the waves meet in the slabs' space
   static constexpr int kSumPitch = kNormT + 4;
-  static constexpr int kSums = kWaves * kNormS * kSumPitch;
+  static constexpr int kSums = kWaves * kS * kSumPitch;
   static constexpr size_t kLdsBytes = std::max(kWaves * kSlab, kSums) * 4;
-  static constexpr size_t kFixedBytes = ((kNormShares + 1) * kRows + 3 * kNormS + kNormT) * 4;  // (below)
-  static constexpr int kPerCu = 16 / kWaves;     // workgroups
+  static constexpr int kItems =  // 16-byte outputs per thread
+      (kS * kNormT / 4 + kThreads - 1) / kThreads;
+  static constexpr size_t kFixedBytes = ((kNormShares + 1) * kRows + 3 * kS + kNormT) * 4;  // (below)
+  static constexpr int kPerCu = kS <= 64 ? 16 / kWaves : 1;  // workgroups
+  static_assert(kS % 32 == 0 && kS <= 128, "shape");
   static_assert(kPerCu * (kLdsBytes + kFixedBytes) <= 160 << 10, "LDS per CU");
 };
 
@@ -106,9 +108,11 @@ __device__ __forceinline__ int sum_up_to_lane(int v) {
   return v;
 }
 // row tiles of an utterance that count
+template <int kS>
 __device__ __forceinline__ int row_tiles(const Limits &lim) {
-  return lim.s_end / kNormS + 1;
+  return lim.s_end / kS + 1;
 }
+template <int kS>
 __device__ __forceinline__ bool find_tile(int id, const NormPlan &plan, const int64_t *window, int B,
                                           int S, int T, int lane, NormTile &o) {
   using dgemm::kXcds;
@@ -118,7 +122,7 @@ __device__ __forceinline__ bool find_tile(int id, const NormPlan &plan, const in
   } mine;
   auto look_up = [&](int b) {
     mine.lim = limits_of(window, min(b, B - 1), S, T);
-    mine.tiles = b < B ? row_tiles(mine.lim) * min(plan.t_tiles, mine.lim.t_end / kNormT + 1) : 0;
+    mine.tiles = b < B ? row_tiles<kS>(mine.lim) * min(plan.t_tiles, mine.lim.t_end / kNormT + 1) : 0;
   };
   look_up(lane);
   int sum = sum_up_to_lane(mine.tiles), total = __builtin_amdgcn_readlane(sum, kWave - 1);
@@ -144,7 +148,7 @@ __device__ __forceinline__ bool find_tile(int id, const NormPlan &plan, const in
   o.b = b0 + at;
   o.lim.s_end = __builtin_amdgcn_readlane(mine.lim.s_end, at);
   o.lim.t_end = __builtin_amdgcn_readlane(mine.lim.t_end, at);
-  const int s_tiles = row_tiles(o.lim);
+  const int s_tiles = row_tiles<kS>(o.lim);
   o.t_idx = n / s_tiles, o.s_idx = n - o.t_idx * s_tiles;
   return true;
 }
@@ -157,13 +161,22 @@ struct NormArgs {
   int B, S, T, C, term, rnnt_type;
 };
 
-template <int kWaves>
-__global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>::kPerCu)
+// f(a constant), the constant being min(max(n, 1), kMost)
+template <int kMost, typename F>
+__device__ __forceinline__ void with_tiles(int n, F &f) {
+  if constexpr (kMost > 1) {
+    if (n < kMost) return with_tiles<kMost - 1>(n, f);
+  }
+  f(std::integral_constant<int, kMost>{});
+}
+
+template <int kS, int kWaves>
+__global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / kWaves : 1))
     simple_fwd_panel_kernel(NormArgs A, NormPlan plan) {
-  using Shape = NormShape<kWaves>;
-  constexpr int kS = kNormS, kT = kNormT, kShares = kNormShares, kTurns = Shape::kTurns;
+  using Shape = NormShape<kS, kWaves>;
+  constexpr int kT = kNormT, kShares = kNormShares, kTurns = Shape::kTurns;
   constexpr int kRows = Shape::kRows, kLoads = Shape::kLoads, kLmLoads = kS / 16;
-  constexpr int kThreads = Shape::kThreads, kPitch = Shape::kPitch;
+  constexpr int kThreads = Shape::kThreads, kItems = Shape::kItems, kPitch = Shape::kPitch;
   using namespace dgemm;
   extern __shared__ __align__(16) float norm_lds[];
   __shared__ float factor[kShares][kRows];      // scale factors for a wave's partial sums
@@ -175,7 +188,7 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   NormTile tile;
   const int tid = threadIdx.x, lane = tid & 63;
   if (plan.all ? !number_tile((int)blockIdx.x, plan, A.B, tile)
-               : !find_tile((int)blockIdx.x, plan, A.window, A.B, S, T, lane, tile))
+               : !find_tile<kS>((int)blockIdx.x, plan, A.window, A.B, S, T, lane, tile))
     return;
   const int b = tile.b, s_tile = tile.s_idx * kS, t_tile = tile.t_idx * kT;
   const int T1 = A.rnnt_type == kRegular ? T + 1 : T;
@@ -209,9 +222,10 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   const int lm_off = ((s_tile + sub) * C + kq) * 4, am_off = ((t_tile + sub) * C + kq) * 4;  // bytes
   const int step = 16 * C * 4;
   typedef int intx4 __attribute__((ext_vector_type(4)));
-  auto fetch = [&](floatx4 (&into)[kLoads], int k0) {
+  auto fetch = [&](auto live, floatx4 (&into)[kLoads], int k0) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
+      if (j >= 2 * live && j < kLmLoads) continue;
       // (the wave-uniform part of the offset rides in a scalar register)
       const intx4 raw = j < kLmLoads
                             ? __builtin_amdgcn_raw_buffer_load_b128(lm_rs, lm_off, j * step + k0 * 4, 0)
@@ -241,11 +255,11 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   // meet their partial sums are brought to the true maxima, exp(shift - max) <= 1.
   constexpr float kMargin = 30.f;
   floatx4 slab[kLoads];
-  if (wave < chunks) fetch(slab, wave * kNormK);
+  if (wave < chunks) fetch(std::integral_constant<int, kS / 32>{}, slab, wave * kNormK);
   if (plan.all) {
     tile.lim = limits_of(A.window, b, S, T);
     if (t_tile > 0 && t_tile > tile.lim.t_end) return;
-    if (tile.s_idx >= row_tiles(tile.lim)) return;
+    if (tile.s_idx >= row_tiles<kS>(tile.lim)) return;
   }
   const int live_rows = min(S1, tile.lim.s_end + 1) - s_tile;  // rows that count
 
@@ -258,16 +272,19 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   const float frame_value =
       get_float(am_rs, tid >= 128 && t_tile + tid - 128 < T, (my_frame + A.term) * 4);
   const float my_term = tid < kS ? row_value : frame_value;
-  // ... and am[b, t, sym[b, s]] of this thread's outputs: a 16-byte piece (row tid / 8, frames
-  // 4 (tid % 8) ..) each for the first 256
-  float am_sym[4];
-  const int out_m = tid / (kT / 4), out_s = s_tile + out_m, out_t = 4 * (tid % (kT / 4));
-  {
-    const int y = get_symbol(sym_rs, out_m < kS && out_s < S && out_m < live_rows, out_s, C);
+  // ... and am[b, t, sym[b, s]] of this thread's outputs: 16-byte pieces (row item / 8, frames
+  // 4 (item % 8) ..)
+  float am_sym[kItems][4];
+  auto item_row = [&](int j) { return (tid + kThreads * j) / (kT / 4); };
+  const int out_t = 4 * (tid % (kT / 4));
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const int m = item_row(j), sr = s_tile + m;
+    const int y = get_symbol(sym_rs, m < kS && sr < S && m < live_rows, sr, C);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tr = t_tile + out_t + i;
-      am_sym[i] = get_float(am_rs, y >= 0 && tr < T, (tr * C + y) * 4);
+      am_sym[j][i] = get_float(am_rs, y >= 0 && tr < T, (tr * C + y) * 4);
     }
   }
 
@@ -281,12 +298,15 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   for (int q = 0; q < kTurns; ++q)
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) seen[q][j] = ninf, shift2[q][j] = kUnset;
+  const int live_tiles = min(kS / 32, (live_rows + 31) / 32);
   float *mine = norm_lds + wave * Shape::kSlab;
-  floatx16 acc[kTurns];
+  floatx16 acc[kTurns][kS / 32];
 #pragma unroll
   for (int q = 0; q < kTurns; ++q)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[q][v] = 0.f;
+    for (int j = 0; j < kS / 32; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[q][j][v] = 0.f;
 
   auto across_row = [&](float v) {  // maximum over the four lanes that share a row
     v = fmaxf(v, __shfl_xor(v, 1, kWave));
@@ -297,9 +317,10 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
     return __builtin_fmaf(top, kLog2e, shift2_) > kMargin * kLog2e;
   };
   // (the sums are brought along; -across_row(seen) is the new shift)
-  auto raise_shifts = [&](auto q) {
+  auto raise_shifts = [&](auto live, auto q) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
+      if (j >= 2 * live && j < kLmLoads) continue;
       const float top = across_row(seen[q][j]);
       float f = 1.f;
       if (above_margin(top, shift2[q][j])) {
@@ -312,38 +333,47 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
     __builtin_amdgcn_wave_barrier();
     const float ft = factor[wave][kS + r32];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[q][v] *= factor[wave][8 * (v / 4) + 4 * half + (v % 4)] * ft;
+    for (int j = 0; j < live; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[q][j][v] *= factor[wave][32 * j + 8 * (v / 4) + 4 * half + (v % 4)] * ft;
     __builtin_amdgcn_wave_barrier();
   };
   // where this lane's values of a slab row go, and where its operands lie
   float *put = mine + sub * kPitch + kq;
   const float *get = mine + r32 * kPitch + 8 * half;
-  // a share of k
-  auto look = [&](auto q) {  // maxima; true if a row exceeds its margin
+  // This wave's share of k, with `live` 32-row tiles that hold lattice rows which count (a
+  // constant: the code of a slab is one straight line, whose rows' chains of dependent
+  // instructions the compiler interleaves -- with a test per row group a slab took 2.5 times as
+  // long).
+  auto look = [&](auto live, auto q) {  // maxima; true if a row exceeds its margin
     bool above = false;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
+      if (j >= 2 * live && j < kLmLoads) continue;
       // two three-input maxima
       seen[q][j] = max3_raw(max3_raw(slab[j][0], slab[j][1], slab[j][2]), slab[j][3], seen[q][j]);
       above |= above_margin(seen[q][j], shift2[q][j]);
     }
     return above;
   };
-  auto walk_share = [&](auto q) {
+  auto walk_share = [&](auto live, auto q) {
     const int share = wave + kWaves * q;
     int chunk = share;
     if (chunk < chunks) {  // the first slab sets the shifts: there are no sums to bring along yet
-      (void)look(q);
+      (void)look(live, q);
 #pragma unroll
       for (int j = 0; j < kLoads; ++j)
-        shift2[q][j] = fminf(shift2[q][j], -across_row(seen[q][j]) * kLog2e);
+        if (j < 2 * live || j >= kLmLoads)
+          shift2[q][j] = fminf(shift2[q][j], -across_row(seen[q][j]) * kLog2e);
     }
     for (; chunk < chunks; chunk += kShares) {
       // exp(x - shift) to LDS, the request for the slab that takes these registers next, then
       // the products
-      if (__any(look(q))) raise_shifts(q);
+      if (__any(look(live, q))) raise_shifts(live, q);
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
+        if (j >= 2 * live && j < kLmLoads) continue;
         floatx4 e;
 #pragma unroll
         for (int i = 0; i < 4; ++i) e[i] = exp_shifted(slab[j][i], shift2[q][j]);
@@ -351,24 +381,32 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
       }
       int next = chunk + kShares;
       if (q + 1 < kTurns && next >= chunks) next = share + kWaves;  // (the next share's first)
-      if (next < chunks) fetch(slab, next * kNormK);
+      if (next < chunks) fetch(live, slab, next * kNormK);
       // MFMA i of the slab multiplies k = i (lanes 0..31) and k = i + 8 (lanes 32..63): a lane takes
       // its row's share of the slab with 16-byte reads
-      floatx4 t_op[2], s_op[2];
+      floatx4 t_op[2], s_op[kS / 32][2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         t_op[h] = *reinterpret_cast<const floatx4 *>(get + kS * kPitch + 4 * h);
-        s_op[h] = *reinterpret_cast<const floatx4 *>(get + 4 * h);
+#pragma unroll
+        for (int j = 0; j < live; ++j)
+          s_op[j][h] = *reinterpret_cast<const floatx4 *>(get + 32 * j * kPitch + 4 * h);
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(s_op[h][i], t_op[h][i], acc[q], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < live; ++j)
+            acc[q][j] =
+                __builtin_amdgcn_mfma_f32_32x32x2f32(s_op[j][h][i], t_op[h][i], acc[q][j], 0, 0, 0);
     }
   };
-  walk_share(std::integral_constant<int, 0>{});
-  if constexpr (kTurns > 1) walk_share(std::integral_constant<int, 1>{});
+  auto walk = [&](auto live) {
+    walk_share(live, std::integral_constant<int, 0>{});
+    if constexpr (kTurns > 1) walk_share(live, std::integral_constant<int, 1>{});
+  };
+  with_tiles<kS / 32>(live_tiles, walk);
 
   // ---- the waves meet: maxima first (each wave's in what was its slab: the row maxima over its
   // share of k, then its final shifts) ...
@@ -402,7 +440,7 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
     // saved for the backward pass; rows that do not exist get a harmless shift
     bool exists;
     if (row < kS) {
-      exists = s_tile + row < S1;
+      exists = s_tile + row < S1 && row < 32 * live_tiles;
       if (s_tile + row < S1 && t_tile == 0) lm_max[s_tile + row] = exists ? r : 0.f;
     } else {
       exists = t_tile + row - kS < T;
@@ -422,7 +460,9 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   float *pxb = A.px + (long)b * S * T1;
   float *pyb = A.py + (long)b * S1 * T;
   float *nrb = A.norm_raw ? A.norm_raw + (long)b * S1 * T : nullptr;
-  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+  floatx4 sums[kItems];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) sums[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int q = 0; q < kTurns; ++q) {
     if (q > 0) __syncthreads();
@@ -430,30 +470,38 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
     const float *my_factor = factor[wave + kWaves * q];
     const float ft = my_factor[kS + r32];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = 8 * (v / 4) + 4 * half + (v % 4);
-      part[m * kSumPitch + r32] = acc[q][v] * (my_factor[m] * ft);
-    }
+    for (int j = 0; j < kS / 32; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = 32 * j + 8 * (v / 4) + 4 * half + (v % 4);
+        part[m * kSumPitch + r32] = acc[q][j][v] * (my_factor[m] * ft);
+      }
     __syncthreads();
-    if (out_m < kS) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const int m = item_row(j);
+      if (m >= kS) continue;
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) {
         const floatx4 one =
-            *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + out_m) * kSumPitch + out_t);
+            *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + m) * kSumPitch + out_t);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sum[i] += one[i];
+        for (int i = 0; i < 4; ++i) sums[j][i] += one[i];
       }
     }
   }
-  if (out_m < kS && out_s < S1 && out_m < live_rows) {
-    const int m = out_m, sr = out_s, tr = t_tile + out_t;
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const int m = item_row(j), sr = s_tile + m, tr = t_tile + out_t;
+    if (m >= kS || sr >= S1 || m >= live_rows) continue;
+    const floatx4 sum = sums[j];
     floatx4 raw, yv, xv;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       raw[i] = logf(sum[i] + 1.17549435e-38f);
       const float norm = raw[i] + slab_max[m] + slab_max[kS + out_t + i];
       yv[i] = (col_term[out_t + i] + row_term[m]) - norm;
-      xv[i] = (am_sym[i] + row_sym[m]) - norm;
+      xv[i] = (am_sym[j][i] + row_sym[m]) - norm;
       if (row_symbol[m] < 0) xv[i] = std::numeric_limits<float>::quiet_NaN();  // out-of-vocabulary
       if (tr + i == t_mask) xv[i] = ninf;
       xv[i] = A.delay.at(xv[i], A.boundary, b, tr + i, T);
@@ -478,7 +526,7 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   if (A.rnnt_type == kRegular && t_tile == 0 && tid < kS && s_tile + tid < S)
     pxb[(s_tile + tid) * T1 + T] = ninf;
   // (and what the row tiles that do not count would have left)
-  if (t_tile == 0 && tile.s_idx == row_tiles(tile.lim) - 1) {
+  if (t_tile == 0 && tile.s_idx == row_tiles<kS>(tile.lim) - 1) {
     for (int s = s_tile + kS + tid; s < S1; s += kThreads) {
       lm_max[s] = 0.f;
       if (A.rnnt_type == kRegular && s < S) pxb[s * T1 + T] = ninf;
@@ -486,12 +534,14 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * NormShape<kWaves>:
   }
 }
 
-template <int kWaves>
-void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, unsigned grid, hipStream_t stream) {
-  auto kernel = simple_fwd_panel_kernel<kWaves>;
-  constexpr size_t lds = NormShape<kWaves>::kLdsBytes;
+template <int kS, int kWaves>
+void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, hipStream_t stream) {
+  auto kernel = simple_fwd_panel_kernel<kS, kWaves>;
+  constexpr size_t lds = NormShape<kS, kWaves>::kLdsBytes;
   if (!allow_lds(reinterpret_cast<const void *>(kernel), lds)) return;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kWaves>::kThreads), lds, stream, args, plan);
+  const long tiles = (long)args.B * plan.t_tiles * plan.s_tiles;
+  const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS, kWaves>::kThreads), lds, stream, args, plan);
 }
 }  // namespace
 
@@ -504,7 +554,7 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                       Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
   NormPlan plan;
   plan.t_tiles = T > 0 ? (T + kNormT - 1) / kNormT : 1;
-  plan.s_tiles = (S + kNormS) / kNormS;
+  plan.s_tiles = (S + 32) / 32;
   const long tiles = (long)B * plan.t_tiles * plan.s_tiles;
   const int rounds = (C + kNormShares * kNormK - 1) / (kNormShares * kNormK);
   // A compute unit for each tile, or two to a unit that soon end or belong to lattices of a single row of
@@ -515,7 +565,18 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
   // C 1500: 45 and 53; B 128, S 20, T 300, C 500: 30.5 and 34.5.)
   const bool two = rounds <= 2 || plan.s_tiles == 1;
   plan.all = tiles <= (two ? 2 : 1) * kComputeUnits || !window;
-  const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
+  // Where tiles of 64 rows have a compute unit each and those of 32 would leave a third of the units and
+  // more with two (of a ragged batch some 0.7 of the tiles count, hence the 1.6), the taller ones are
+  // faster: B 60, S 50, T 110, C 2500 (480 of 32 rows, 240 of 64): 41.3 us against 49.5; B 8, S 100,
+  // T 400, C 5000 (416): 68.3 against 69.3; B 21, S 47, T 333, C 503 (462): 14.8 against 15.5; B 64, S 40,
+  // T 100, C 800 (512): 18.3 against 19.3.  Below, B 40, S 60, T 100, C 600 (320): 15.8 against 12.2; B 40, S 33,
+  // T 150, C 400 (400): 12.2 against 10.3.
+  const int tall = (S + 64) / 64;
+  if (!plan.all && 5 * tiles > 8 * kComputeUnits && (long)B * plan.t_tiles * tall <= kComputeUnits) {
+    plan.s_tiles = tall;
+    plan.all = true;
+    return launch_fwd_panel<64, 8>(args, plan, stream);
+  }
   // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
   // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
   // a compute unit has several workgroups in turn and their loops are short (B 64, S 120, T 600,
@@ -523,8 +584,8 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
   // against 28.5), the latter elsewhere (B 23, S 41, T 444, C 444: 15.5 against 16.4; B 98, S 65,
   // T 209, C 722: 55.7 against 57.3; B 4, S 15, T 47, C 4482: 32 against 42).
   if (tiles > 3 * kComputeUnits && rounds <= 5)
-    launch_fwd_panel<4>(args, plan, grid, stream);
+    launch_fwd_panel<32, 4>(args, plan, stream);
   else
-    launch_fwd_panel<8>(args, plan, grid, stream);
+    launch_fwd_panel<32, 8>(args, plan, stream);
 }
 }  // namespace frnnt
