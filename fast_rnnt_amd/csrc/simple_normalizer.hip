@@ -40,7 +40,7 @@ namespace {
 // T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64 sizes, B 1 .. 128,
 // C 50 .. 5000: 5.6 %.  Tiles of 64, 96 and 128 rows dealt out the same way were the fastest at 12 of the
 // 64, mostly by 1 to 5 %, and a choice among all of them, which cannot know how ragged a batch is, gained
-// nothing; 64 rows are left where they have a compute unit each (launch_normalizer_f32).
+// nothing; 64 and 96 rows are left where they have a compute unit each (launch_normalizer_f32).
 constexpr int kNormK = 16;      // k per slab
 constexpr int kNormShares = 8;  // of k
 constexpr int kNormT = 32;      // frames of a tile
@@ -565,17 +565,25 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
   // C 1500: 45 and 53; B 128, S 20, T 300, C 500: 30.5 and 34.5.)
   const bool two = rounds <= 2 || plan.s_tiles == 1;
   plan.all = tiles <= (two ? 2 : 1) * kComputeUnits || !window;
-  // Where tiles of 64 rows have a compute unit each and those of 32 would leave a third of the units and
-  // more with two (of a ragged batch some 0.7 of the tiles count, hence the 1.6), the taller ones are
-  // faster: B 60, S 50, T 110, C 2500 (480 of 32 rows, 240 of 64): 41.3 us against 49.5; B 8, S 100,
-  // T 400, C 5000 (416): 68.3 against 69.3; B 21, S 47, T 333, C 503 (462): 14.8 against 15.5; B 64, S 40,
-  // T 100, C 800 (512): 18.3 against 19.3.  Below, B 40, S 60, T 100, C 600 (320): 15.8 against 12.2; B 40, S 33,
-  // T 150, C 400 (400): 12.2 against 10.3.
-  const int tall = (S + 64) / 64;
-  if (!plan.all && 5 * tiles > 8 * kComputeUnits && (long)B * plan.t_tiles * tall <= kComputeUnits) {
-    plan.s_tiles = tall;
+  // Where tiles of 64 or 96 rows all but fill the compute units, one to each, those of 32 would leave many
+  // units with one more than the rest, and the taller ones are faster: 64 rows, B 60, S 50, T 110, C 2500
+  // (240 tiles): 41.3 us against 49.5; B 8, S 100, T 400, C 5000 (208): 68.3 against 69.3; B 21, S 47, T 333,
+  // C 503 (231): 14.8 against 15.5; B 64, S 40, T 100, C 800 (256): 18.3 against 19.3; 96 rows, B 32, S 80,
+  // T 250 (256), C 500: 19.5 against 20.1, C 2500: 54.7 against 58.5; B 14, S 95, T 570, C 2000 (252): 46.6
+  // against 49.1; B 64, S 85, T 110, C 150 (256): 12.9 against 15.0.  With fewer of them (of a ragged
+  // batch some 0.7 of the small tiles count, and they come to one each as well) the small ones are: 64 rows,
+  // B 40, S 60, T 100, C 600 (160): 15.8 against 12.2; B 40, S 33, T 150, C 400 (200): 12.2 against 10.3;
+  // 96 rows, B 30, S 70, T 250, C 500 (240): 18.9 against 16.2; B 23, S 73, T 202, C 4093 (161): 78 against 75.
+  auto fills = [&](int rows) {
+    const long taller = (long)B * plan.t_tiles * ((S + rows) / rows);
+    return taller <= kComputeUnits && 20 * taller > (rows == 64 ? 16 : 19) * kComputeUnits;
+  };
+  const int rows = plan.all ? 32 : fills(64) ? 64 : fills(96) ? 96 : 32;
+  if (rows > 32) {
+    plan.s_tiles = (S + rows) / rows;
     plan.all = true;
-    return launch_fwd_panel<64, 8>(args, plan, stream);
+    if (rows == 64) return launch_fwd_panel<64, 8>(args, plan, stream);
+    return launch_fwd_panel<96, 8>(args, plan, stream);
   }
   // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
   // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where

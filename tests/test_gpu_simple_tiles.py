@@ -54,7 +54,8 @@ def test_simple_loss_at_the_edges_of_tiles(gpu_device, B, S, T, C):
 # short and long loops (launch_normalizer_f32 takes eight or four waves), one row of 384 and 650 tiles
 WINDOWED = [(3, 40, 70, 33), (9, 200, 300, 700), (64, 63, 65, 90), (65, 31, 200, 40),
             (130, 64, 129, 20), (300, 5, 33, 9), (40, 33, 256, 1100),
-            (96, 14, 114, 300), (130, 31, 150, 300), (30, 40, 250, 300), (15, 63, 450, 400)]
+            (96, 14, 114, 300), (130, 31, 150, 300), (30, 40, 250, 300), (15, 63, 450, 400),
+            (16, 90, 500, 300)]
 
 
 @pytest.mark.parametrize("B,S,T,C", WINDOWED)
