@@ -455,8 +455,8 @@ def _bench_lattice(args, w, dev):
                   in_bytes + nbytes, t_b, padded_bytes=2 * nbytes),
         _hbm_line(table, "row_norm_kernel",
                   in_bytes, t_f, padded_bytes=nbytes,
-                  **({} if ranges is None else {"note": "launch time includes the small "
-                                                "assemble_kernel of the same entry point"})),
+                  **({} if ranges is None else {"note": "the launch also fills the cells of the "
+                                                "lattice around the rows"})),
     ]
     lines.sort(key=lambda r: -r["avg_launch_us"])
     eager = _rate(args.steps, elapsed)
