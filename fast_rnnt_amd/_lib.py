@@ -37,6 +37,7 @@ _SIGNATURES = {
     "frnnt_mi_backward_f64": ([_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "frnnt_simple_logprobs_fwd_f32": ([_P] * 9 + [_I] * 7 + [_P], _I),
     "frnnt_simple_logprobs_fwd_f64": ([_P] * 9 + [_I] * 7 + [_P], _I),
+    "frnnt_simple_logprobs_tile": ([_I] * 5 + [ctypes.POINTER(_I)], _I),
     "frnnt_simple_logprobs_bwd_f32": ([_P] * 8 + [_I, _D] + [_P] * 8 + [_I] * 7 + [_P], _I),
     "frnnt_simple_logprobs_bwd_f64": ([_P] * 8 + [_I, _D] + [_P] * 8 + [_I] * 7 + [_P], _I),
     "frnnt_simple_logprobs_bwd_noalloc_f32": ([_P] * 8 + [_I, _D] + [_P] * 4 + [_I] * 7 + [_P], _I),

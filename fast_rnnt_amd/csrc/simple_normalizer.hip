@@ -34,13 +34,14 @@ namespace {
 // covers a workgroup's prologue and epilogue (4.5 and 5 us).  Hence small tiles -- taller ones convert
 // less per cell, but of 16 utterances' tiles of 128 rows a third of the compute units got none --
 // dealt out evenly (find_tile), and eight waves of one share each or four of two
-// (launch_normalizer_f32).  Measured within training steps on three batches in turn, against tiles of
+// (choose_tile).  Measured within training steps on three batches in turn, against tiles of
 // 32 to 128 rows with a workgroup per tile whether it counted or not: B 64, S 120, T 600, C 500: 96 ->
 // 89 us; B 32, S 80, T 250, C 500: 20.4 and 20.6; B 16, S 120, T 400, C 5000: 127 -> 122; B 10, S 137,
 // T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64 sizes, B 1 .. 128,
 // C 50 .. 5000: 5.6 %.  Tiles of 64, 96 and 128 rows dealt out the same way were the fastest at 12 of the
 // 64, mostly by 1 to 5 %, and a choice among all of them, which cannot know how ragged a batch is, gained
-// nothing; 64 and 96 rows are left where they have a compute unit each (launch_normalizer_f32).
+// nothing; 64 and 96 rows are left where they have a compute unit each and, where no window makes a batch
+// ragged, by the number of tiles of each height (choose_tile).
 constexpr int kNormK = 16;      // k per slab
 constexpr int kNormShares = 8;  // of k
 constexpr int kNormT = 32;      // frames of a tile
@@ -84,8 +85,8 @@ struct NormTile {
   int b, s_idx, t_idx;
   Limits lim;
 };
-// Batches of few tiles, counting or not, number them all (launch_normalizer_f32): a tile is then known
-// without a look at the window, whose words arrive beside the first operands.
+// Batches of few tiles, counting or not, number them all (choose_tile), and so do those without windows:
+// a tile is then known without a look at the window, whose words arrive beside the first operands.
 __device__ __forceinline__ bool number_tile(int id, const NormPlan &plan, int B, NormTile &o) {
   using dgemm::kXcds;
   const int of_utterance = plan.s_tiles * plan.t_tiles, total = B * of_utterance;
@@ -543,28 +544,52 @@ void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, hipStream_t st
   const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS, kWaves>::kThreads), lds, stream, args, plan);
 }
-}  // namespace
 
-void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symbols,
-                           const int64_t *boundary, float *lm_max, float *am_max, float *px,
-                           float *py, float *norm_raw, const int64_t *window,
-                           double delay_penalty, int B, int S, int T, int C, int term,
-                           int rnnt_type, hipStream_t stream) {
-  const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
-                      Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
-  NormPlan plan;
-  plan.t_tiles = T > 0 ? (T + kNormT - 1) / kNormT : 1;
-  plan.s_tiles = (S + 32) / 32;
-  const long tiles = (long)B * plan.t_tiles * plan.s_tiles;
+struct NormChoice {
+  int rows, waves;  // of a tile
+  bool all;         // its numbering: see number_tile
+};
+// The tile that a call takes.  `windowed`: what lies outside an utterance's window does not count.
+NormChoice choose_tile(int B, int S, int T, int C, bool windowed) {
+  const long t_tiles = T > 0 ? (T + kNormT - 1) / kNormT : 1;
+  const int s_tiles = (S + 32) / 32;
+  const long tiles = B * t_tiles * s_tiles;
   const int rounds = (C + kNormShares * kNormK - 1) / (kNormShares * kNormK);
+  auto taller = [&](int rows) { return B * t_tiles * ((S + rows) / rows); };
+  // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
+  // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
+  // a compute unit has several workgroups in turn and their loops are short (B 64, S 120, T 600,
+  // C 500: 89 against 98 us; B 13, S 125, T 451, C 60: 12.1 against 14.7; B 10, S 137, T 817, C 500: 26.2
+  // against 28.5), the latter elsewhere (B 23, S 41, T 444, C 444: 15.5 against 16.4; B 98, S 65,
+  // T 209, C 722: 55.7 against 57.3; B 4, S 15, T 47, C 4482: 32 against 42).
+  const int waves = tiles > 3 * kComputeUnits && rounds <= 5 ? 4 : 8;
+  if (!windowed) {
+    // Every tile counts and none is looked up.  The compute units take them in turn, so that a launch
+    // lasts as long as the fullest unit: its tiles times what one takes, 1 : 1.8 : 2.35 for 32, 64 and 96
+    // rows (C 5000: 35, 64 and 81 us).  32 rows against taller ones: 64 rows, B 16, S 120, T 400, C 5000:
+    // 142 us against 129; B 64, S 40, T 200, C 1000: 44 against 39; B 5, S 224, T 743, C 2536: 77 against 70; 96
+    // rows, B 32, S 80, T 250, C 500: 24.6 against 20.4, C 2500: 82 against 61; B 2, S 250, T 1320, C 4606: 103
+    // against 87.  Prologue and epilogue of a tall tile show where loops are short (64 rows, B 128, S 60, T 250,
+    // C 100: 23.1 against 23.7), and those of 96 rows, which have a unit to themselves, wherever
+    // they come in turn (B 70, S 78, T 565, C 461: 83 against 95).  Three tiles of 32 to a unit are all there at
+    // once with four waves, not with eight (B 47, S 53, T 243, C 1246: 45 against 53; B 45, S 33, T 240,
+    // C 892: 29.7 against 34.0; B 15, S 58, T 568, C 120: 12.8 against 14.7).  Over 256 sizes, B 1 .. 128, C 50 ..
+    // 5000, the choice is 0.2 % (geometric mean) from the best, 32 rows by the rule above 1.8 %.
+    auto of_a_unit = [&](int rows) { return (taller(rows) + kComputeUnits - 1) / kComputeUnits; };
+    NormChoice best{32, of_a_unit(32) == 3 ? 4 : waves, true};
+    double least = (double)of_a_unit(32);
+    if (rounds >= 4 && 1.8 * of_a_unit(64) < least) least = 1.8 * of_a_unit(64), best = {64, 8, true};
+    if ((rounds >= 4 || best.waves == 8) && of_a_unit(96) == 1 && 2.35 < least) best = {96, 8, true};
+    return best;
+  }
   // A compute unit for each tile, or two to a unit that soon end or belong to lattices of a single row of
   // tiles, of which only the frames are ragged: the look-up would cost more than it gains.  (B 70, S 13,
   // T 149, C 80: 9.3 us with it, 8.0 without; one row of 384 to 500 tiles, B 96, S 14, T 114, C 854: 20.2 and
   // 19.2; B 128, S 10, T 100, C 500: 16.1 and 14.6; B 110, S 28, T 128, C 640: 18.7 and 17.4.  Two rows of
   // them, B 25, S 50, T 258, C 1400: 26.7 and 37.8; one row of more than two to a unit, B 80, S 12, T 250,
   // C 1500: 45 and 53; B 128, S 20, T 300, C 500: 30.5 and 34.5.)
-  const bool two = rounds <= 2 || plan.s_tiles == 1;
-  plan.all = tiles <= (two ? 2 : 1) * kComputeUnits || !window;
+  const bool two = rounds <= 2 || s_tiles == 1;
+  if (tiles <= (two ? 2 : 1) * kComputeUnits) return {32, waves, true};
   // Where tiles of 64 or 96 rows all but fill the compute units, one to each, those of 32 would leave many
   // units with one more than the rest, and the taller ones are faster: 64 rows, B 60, S 50, T 110, C 2500
   // (240 tiles): 41.3 us against 49.5; B 8, S 100, T 400, C 5000 (208): 68.3 against 69.3; B 21, S 47, T 333,
@@ -575,25 +600,38 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
   // B 40, S 60, T 100, C 600 (160): 15.8 against 12.2; B 40, S 33, T 150, C 400 (200): 12.2 against 10.3;
   // 96 rows, B 30, S 70, T 250, C 500 (240): 18.9 against 16.2; B 23, S 73, T 202, C 4093 (161): 78 against 75.
   auto fills = [&](int rows) {
-    const long taller = (long)B * plan.t_tiles * ((S + rows) / rows);
-    return taller <= kComputeUnits && 20 * taller > (rows == 64 ? 16 : 19) * kComputeUnits;
+    return taller(rows) <= kComputeUnits && 20 * taller(rows) > (rows == 64 ? 16 : 19) * kComputeUnits;
   };
-  const int rows = plan.all ? 32 : fills(64) ? 64 : fills(96) ? 96 : 32;
-  if (rows > 32) {
-    plan.s_tiles = (S + rows) / rows;
-    plan.all = true;
-    if (rows == 64) return launch_fwd_panel<64, 8>(args, plan, stream);
-    return launch_fwd_panel<96, 8>(args, plan, stream);
-  }
-  // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
-  // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
-  // a compute unit has several workgroups in turn and their loops are short (B 64, S 120, T 600,
-  // C 500: 89 against 98 us; B 13, S 125, T 451, C 60: 12.1 against 14.7; B 10, S 137, T 817, C 500: 26.2
-  // against 28.5), the latter elsewhere (B 23, S 41, T 444, C 444: 15.5 against 16.4; B 98, S 65,
-  // T 209, C 722: 55.7 against 57.3; B 4, S 15, T 47, C 4482: 32 against 42).
-  if (tiles > 3 * kComputeUnits && rounds <= 5)
+  if (fills(64)) return {64, 8, true};
+  if (fills(96)) return {96, 8, true};
+  return {32, waves, false};
+}
+}  // namespace
+
+void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symbols,
+                           const int64_t *boundary, float *lm_max, float *am_max, float *px,
+                           float *py, float *norm_raw, const int64_t *window,
+                           double delay_penalty, int B, int S, int T, int C, int term,
+                           int rnnt_type, hipStream_t stream) {
+  const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
+                      Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
+  const NormChoice choice = choose_tile(B, S, T, C, window != nullptr);
+  const NormPlan plan{T > 0 ? (T + kNormT - 1) / kNormT : 1, (S + choice.rows) / choice.rows, choice.all};
+  if (choice.rows == 96)
+    launch_fwd_panel<96, 8>(args, plan, stream);
+  else if (choice.rows == 64)
+    launch_fwd_panel<64, 8>(args, plan, stream);
+  else if (choice.waves == 4)
     launch_fwd_panel<32, 4>(args, plan, stream);
   else
     launch_fwd_panel<32, 8>(args, plan, stream);
 }
 }  // namespace frnnt
+
+extern "C" int frnnt_simple_logprobs_tile(int B, int S, int T, int C, int window_only, int *waves) {
+  using namespace frnnt;
+  if (B < 1 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_tile: bad size");
+  const NormChoice choice = choose_tile(B, S, T, C, window_only != 0);
+  if (waves) *waves = choice.waves;
+  return choice.rows;
+}

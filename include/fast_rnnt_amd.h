@@ -159,6 +159,12 @@ int frnnt_simple_logprobs_fwd_f64(const double *lm, const double *am, const int6
                                   double *am_max, double *norm_raw, int B, int S, int T, int C,
                                   int termination_symbol, int rnnt_type, int window_only,
                                   void *stream);
+/*
+ * The lattice rows of a tile of that product's float32 kernel at this size (32, 64 or 96), and
+ * the waves that share one (may be NULL).  px, py and the normalizers are the same bits in every
+ * form; `window_only` with a boundary, as above.  Host only.
+ */
+int frnnt_simple_logprobs_tile(int B, int S, int T, int C, int window_only, int *waves);
 
 /*
  * Backward of the above: what autograd derives for rnnt_loss.py:174-225, as one

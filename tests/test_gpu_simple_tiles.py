@@ -2,6 +2,8 @@
 sizes on either side of a tile of lattice rows, frames and vocabulary entries, sums over few and
 many chunks, batches small and large, 2-byte inputs, long lists of equal symbols.  Oracle: the CPU
 restatement on the same values in float32."""
+import ctypes
+
 import pytest
 import torch
 
@@ -50,8 +52,19 @@ def test_simple_loss_at_the_edges_of_tiles(gpu_device, B, S, T, C):
             assert bool((off <= 2e-4 + ulp * y.grad.abs()).all()), off.max().item()
 
 
+def logprobs(lm, am, symbols, boundary, window_only):
+    """px, py, lm_max, am_max and norm_raw of the regular lattice; NaN where nothing was written."""
+    (B, S1, C), T = lm.shape, am.shape[1]
+    shapes = [(B, S1 - 1, T + 1), (B, S1, T), (B, S1), (B, T), (B, S1, T)]
+    out = [torch.full(n, float("nan"), device=lm.device) for n in shapes]
+    _lib.call("frnnt_simple_logprobs_fwd_f32", lm.data_ptr(), am.data_ptr(), symbols.data_ptr(),
+              _lib.ptr(boundary), *(x.data_ptr() for x in out), B, S1 - 1, T, C, 0, 0, window_only,
+              _lib.stream_of(am))
+    return out
+
+
 # (B, S, T, C): fewer and more tiles than compute units, one, two and more waves' lanes of utterances,
-# short and long loops (launch_normalizer_f32 takes eight or four waves), one row of 384 and 650 tiles
+# short and long loops (the product takes eight or four waves), one row of 384 and 650 tiles
 WINDOWED = [(3, 40, 70, 33), (9, 200, 300, 700), (64, 63, 65, 90), (65, 31, 200, 40),
             (130, 64, 129, 20), (300, 5, 33, 9), (40, 33, 256, 1100),
             (96, 14, 114, 300), (130, 31, 150, 300), (30, 40, 250, 300), (15, 63, 450, 400),
@@ -73,15 +86,7 @@ def test_tiles_of_windows_are_the_tiles_of_the_whole_lattice(gpu_device, B, S, T
     am = torch.randn(B, T, C, generator=g).to(gpu_device)
     symbols = torch.randint(0, C, (B, S), generator=g).to(gpu_device)
 
-    def run(window_only):
-        shapes = [(B, S, T + 1), (B, S + 1, T), (B, S + 1), (B, T), (B, S + 1, T)]
-        out = [torch.full(n, float("nan"), device=gpu_device) for n in shapes]
-        _lib.call("frnnt_simple_logprobs_fwd_f32", lm.data_ptr(), am.data_ptr(), symbols.data_ptr(),
-                  boundary.data_ptr(), *(x.data_ptr() for x in out), B, S, T, C, 0, 0, window_only,
-                  _lib.stream_of(am))
-        return out
-
-    whole, windowed = run(0), run(1)
+    whole, windowed = (logprobs(lm, am, symbols, boundary, w) for w in (0, 1))
     s = torch.arange(S + 1, device=gpu_device).view(1, -1, 1)
     t = torch.arange(T + 1, device=gpu_device).view(1, 1, -1)
     rows, frames = s <= boundary[:, 2].view(-1, 1, 1), t < boundary[:, 3].view(-1, 1, 1)
@@ -122,8 +127,11 @@ def test_gradient_products_read_nothing_outside_a_window(gpu_device, S, T, C, s_
         assert bool(((x.grad.cpu() - y.grad).abs() <= 2e-4 + 1e-4 * y.grad.abs()).all())
 
 
-# (S, T, C, batch sizes at which launch_normalizer_f32 takes tiles of 32, 64, 96 or 128 rows)
-HEIGHTS = [(95, 128, 500, {1: 32, 26: 64, 51: 96}), (120, 200, 600, {1: 32, 11: 64, 22: 128})]
+# (S, T, C, [(B, whether with windows, rows of a tile, waves that share it)]): every form of the product
+HEIGHTS = [(95, 128, 500, [(1, 0, 32, 8), (26, 0, 64, 8), (51, 0, 96, 8), (70, 0, 32, 4),
+                           (26, 1, 64, 8), (40, 1, 32, 8), (64, 1, 96, 8), (70, 1, 32, 4)]),
+           (120, 200, 600, [(1, 0, 32, 8), (11, 0, 64, 8), (22, 0, 32, 4), (37, 0, 32, 4),
+                            (16, 1, 64, 8), (20, 1, 32, 8), (37, 1, 32, 4)])]
 
 
 @pytest.mark.parametrize("S,T,C,batches", HEIGHTS)
@@ -131,22 +139,30 @@ def test_normalizers_are_the_same_bits_in_tiles_of_any_height(gpu_device, S, T, 
     # some rows have values far above what their first entries suggest, so that their shifts are
     # raised on the way; their neighbours in a tile, which differ with its height, must not notice
     g = torch.Generator().manual_seed(S)
-    most = max(batches)
+    most = max(B for B, *_ in batches)
     lm, am = torch.randn(most, S + 1, C, generator=g), torch.randn(most, T, C, generator=g)
     for x in (lm, am):
         for b, r in torch.nonzero(torch.rand(x.shape[:2], generator=g) < 0.05).tolist():
             x[b, r, torch.randint(C // 3, C, (3,), generator=g)] += 40.0
     symbols = torch.randint(0, C, (most, S), generator=g)
+    # (the first utterance is whole, the others' windows end anywhere)
+    s_end, t_end = torch.randint(1, S + 1, (most,), generator=g), torch.randint(1, T + 1, (most,), generator=g)
+    s_end[0], t_end[0] = S, T
+    boundary = torch.stack([torch.zeros_like(s_end)] * 2 + [s_end, t_end], 1).to(gpu_device)
     lm, am, symbols = lm.to(gpu_device), am.to(gpu_device), symbols.to(gpu_device)
     first = None
-    for B in batches:
-        print(f"S={S} T={T} C={C} B={B}", flush=True)
-        px, py = fast_rnnt_amd.get_rnnt_logprobs(lm[:B], am[:B], symbols[:B], 0)
+    for B, windowed, rows, waves in batches:
+        print(f"S={S} T={T} C={C} B={B} windows={windowed}", flush=True)
+        got_waves = ctypes.c_int()
+        assert _lib.load().frnnt_simple_logprobs_tile(B, S, T, C, windowed, ctypes.byref(got_waves)) == rows
+        assert got_waves.value == waves
+        out = logprobs(lm[:B], am[:B], symbols[:B], boundary[:B] if windowed else None, windowed)
         if first is None:
-            first = px[0].clone(), py[0].clone()
-        assert torch.equal(px[0], first[0]) and torch.equal(py[0], first[1])
+            first = [x[0].clone() for x in out]
+        for got, want in zip(out, first):
+            assert torch.equal(got[0], want)
     # (the last column is closed)
-    px, py = px[0, :, :T].double().cpu(), py[0].double().cpu()
+    px, py = first[0][:, :T].double().cpu(), first[1].double().cpu()
     joint = lm[0].double().cpu().unsqueeze(1) + am[0].double().cpu().unsqueeze(0)  # [S+1][T][C]
     norm = torch.logsumexp(joint, dim=2)
     want_y = joint[:, :, 0] - norm
