@@ -64,11 +64,12 @@ def logprobs(lm, am, symbols, boundary, window_only):
 
 
 # (B, S, T, C): fewer and more tiles than compute units, one, two and more waves' lanes of utterances,
-# short and long loops (the product takes eight or four waves), one row of 384 and 650 tiles
+# short and long loops (the product takes eight or four waves, and the four have one, two, four and
+# five slabs of a share), one row of 384 and 650 tiles
 WINDOWED = [(3, 40, 70, 33), (9, 200, 300, 700), (64, 63, 65, 90), (65, 31, 200, 40),
             (130, 64, 129, 20), (300, 5, 33, 9), (40, 33, 256, 1100),
             (96, 14, 114, 300), (130, 31, 150, 300), (30, 40, 250, 300), (15, 63, 450, 400),
-            (16, 90, 500, 300)]
+            (16, 90, 500, 300), (30, 130, 280, 500), (28, 127, 250, 640)]
 
 
 @pytest.mark.parametrize("B,S,T,C", WINDOWED)
