@@ -139,7 +139,7 @@ struct Surround {
 template <typename P, int kLanes, int kVecs, bool kLoop, bool kStream>
 __global__ void __launch_bounds__(256)
     row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out,
-                    Surround around) {
+                    Surround around, long kept) {
   constexpr int kRows = kWave / kLanes;
   const int b = block_batch();
   if (b >= L.B) return;
@@ -158,9 +158,9 @@ __global__ void __launch_bounds__(256)
       pieces_of<P, kLanes>(base, reinterpret_cast<uintptr_t>(logits + row.index * L.C), L.C);
   const float ninf = -__builtin_huge_valf();
   float m = ninf, sum = 0, shift = 0;
-  // (wave-uniform) the rows that the backward will look at first stay in the cache
+  // (wave-uniform) the rows that the backward will look at first, `kept` bytes, stay in the cache
   const bool past_cache =
-      kStream && ((long)L.B * L.T * L.Rr - first) * L.C * (long)sizeof(typename P::Elem) > kKeptBytes;
+      kStream && ((long)L.B * L.T * L.Rr - first) * L.C * (long)sizeof(typename P::Elem) > kept;
   intx4 raw[kVecs];
   for (int p0 = 0; p0 < (kLoop ? q.pieces : 1); p0 += kLanes * kVecs) {
     auto load_pieces = [&](auto aux) {
@@ -243,7 +243,7 @@ bool rows_in_pieces(int C) {
 }
 template <typename P, typename R>
 void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Picks<R> &out,
-                     hipStream_t stream) {
+                     bool read_again, hipStream_t stream) {
   const long rows = (long)L.T * L.Rr;
   if constexpr (!std::is_same<P, DoublePiece>::value) {
     if (rows_in_pieces<P>(L.C)) {
@@ -252,15 +252,17 @@ void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Pic
         around.t_tiles = (L.T + (L.rnnt_type == kRegular ? 1 : 0) + 63) / 64;
         around.blocks = (unsigned)around.t_tiles * ((L.S + kAssembleRows) / kAssembleRows);
       }
-      const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) > kStreamBytes;
+      const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) >
+                       (read_again ? kStreamBytes : kReadOnceBytes);
+      const long kept = read_again ? kKeptBytes : 0;
       with_row_split<P>(logits, L.C, [&](auto lanes, auto vecs, auto loop) {
         const dim3 grid = batch_grid(around.blocks + (rows + 256 / lanes - 1) / (256 / lanes), L.B);
         if (big && lanes == 64)
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, lanes == 64>), grid, dim3(256),
-                             0, stream, logits, L, out, around);
+                             0, stream, logits, L, out, around, kept);
         else
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, false>), grid, dim3(256), 0,
-                             stream, logits, L, out, around);
+                             stream, logits, L, out, around, kept);
       });
       return;
     }
@@ -338,7 +340,7 @@ template <typename P, typename R>
 int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
              const int64_t *boundary, R *px, R *py, R *norm, R *xr, R *yr, int B, int S, int T,
              int Rr, int C, int term, int rnnt_type, int window_only, double delay_penalty,
-             void *stream_) {
+             bool read_again, void *stream_) {
   if (B < 0 || S < 0 || T < 0 || Rr < 1 || C < 1)
     return fail(FRNNT_EINVAL, "lattice_logprobs_fwd: bad size");
   if (Rr > S + 1) return fail(FRNNT_EINVAL, "lattice_logprobs_fwd: more range rows than S + 1");
@@ -358,7 +360,7 @@ int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
   const bool direct = rnnt_type != kConstrained && (!ranges || rows_in_pieces<P>(C));
   if (T > 0)
     launch_row_norm<P, R>(static_cast<const typename P::Elem *>(logits_), L,
-                          Picks<R>{norm, xr, yr, px, py, delay, direct}, stream);
+                          Picks<R>{norm, xr, yr, px, py, delay, direct}, read_again, stream);
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
   if (T == 0 && T1 > 0) {
     // no frames: nothing but the closed column
@@ -379,7 +381,8 @@ int loss_fwd_impl(Tail tail, const void *logits, const int64_t *symbols, const i
                   int rnnt_type, double delay_penalty, int reduction, int checks, int32_t *status,
                   void *stream) {
   const int rc = fwd_impl<P, R>(logits, symbols, ranges, boundary, px, py, norm, xr, yr, B, S, T,
-                                Rr, C, term, rnnt_type, boundary != nullptr, delay_penalty, stream);
+                                Rr, C, term, rnnt_type, boundary != nullptr, delay_penalty,
+                                px_grad != nullptr, stream);
   if (rc != FRNNT_OK) return rc;
   return tail(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, rnnt_type != kRegular,
               reduction, checks, status, stream);
@@ -397,7 +400,7 @@ extern "C" {
       int termination_symbol, int rnnt_type, int window_only, void *stream) {                    \
     return frnnt::fwd_impl<frnnt::P, R>(logits, symbols, ranges, boundary, px, py, norm, xr, yr,  \
                                         B, S, T, Rr, C, termination_symbol, rnnt_type,            \
-                                        window_only, 0.0, stream);                               \
+                                        window_only, 0.0, true, stream);                         \
   }                                                                                              \
   int frnnt_lattice_loss_fwd_##sfx(                                                              \
       const io *logits, const int64_t *symbols, const int64_t *ranges, const int64_t *boundary,   \

@@ -107,6 +107,9 @@ def test_streamed_logits_give_the_bits_of_their_utterances(gpu_device, B, C):
         return loss.detach(), leaf.grad
 
     loss, grad = run(slice(0, B))
+    with torch.no_grad():  # (the forward that no backward follows has a line of its own)
+        alone = fast_rnnt_amd.rnnt_loss(logits, symbols, 0, boundary=ends, reduction="none")
+    assert torch.equal(alone, loss)
     for b in range(B):
         one_loss, one_grad = run(slice(b, b + 1))
         assert torch.equal(loss[b:b + 1], one_loss) and torch.equal(grad[b:b + 1], one_grad)
