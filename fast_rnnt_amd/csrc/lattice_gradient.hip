@@ -83,12 +83,11 @@ __global__ void __launch_bounds__(256)
                     typename P::Elem *__restrict__ glogits) {
   constexpr int kAux = kStream ? 2 : 0;
   constexpr int kRows = kWave / kLanes;
-  // (from the last row to the first: the forward has left what it read last in the cache)
-  const int b = L.B - 1 - block_batch();
-  if (b < 0) return;
+  const int b = block_batch();
+  if (b >= L.B) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register
   const int lane = threadIdx.x & (kLanes - 1);
-  const unsigned r0 = ((gridDim.x - 1 - blockIdx.x) * 4 + wave) * kRows;
+  const unsigned r0 = (blockIdx.x * 4 + wave) * kRows;
   const unsigned r = kRows == 1 ? r0 : r0 + (threadIdx.x & 63) / kLanes;
   const Row row = locate(L, b, r);
   const bool inside = row.t < L.T;

@@ -139,14 +139,16 @@ struct Surround {
 template <typename P, int kLanes, int kVecs, bool kLoop, bool kStream>
 __global__ void __launch_bounds__(256)
     row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out,
-                    Surround around, long kept) {
+                    Surround around) {
+  constexpr int kAux = kStream ? 2 : 0;
   constexpr int kRows = kWave / kLanes;
-  const int b = block_batch();
-  if (b >= L.B) return;
+  // (from the last row to the first: the caller has left what it wrote last in the cache)
+  const int b = L.B - 1 - block_batch();
+  if (b < 0) return;
   if (blockIdx.x < around.blocks) return around.fill(L, b, blockIdx.x, out.px, out.py);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register
   const int lane = threadIdx.x & (kLanes - 1);
-  const unsigned r0 = ((blockIdx.x - around.blocks) * 4 + wave) * kRows;
+  const unsigned r0 = ((gridDim.x - 1 - blockIdx.x) * 4 + wave) * kRows;
   const unsigned r = kRows == 1 ? r0 : r0 + (threadIdx.x & 63) / kLanes;
   const Row row = locate(L, b, r);
   if (!row.live && lane == 0) out.skip(L, row);
@@ -158,23 +160,14 @@ __global__ void __launch_bounds__(256)
       pieces_of<P, kLanes>(base, reinterpret_cast<uintptr_t>(logits + row.index * L.C), L.C);
   const float ninf = -__builtin_huge_valf();
   float m = ninf, sum = 0, shift = 0;
-  // (wave-uniform) the rows that the backward will look at first, `kept` bytes, stay in the cache
-  const bool past_cache =
-      kStream && ((long)L.B * L.T * L.Rr - first) * L.C * (long)sizeof(typename P::Elem) > kept;
   intx4 raw[kVecs];
   for (int p0 = 0; p0 < (kLoop ? q.pieces : 1); p0 += kLanes * kVecs) {
-    auto load_pieces = [&](auto aux) {
 #pragma unroll
-      for (int i = 0; i < kVecs; ++i) {
-        const int p = p0 + lane + kLanes * i;
-        const bool wanted = (kRows == 1 || row.live) && p < q.pieces;
-        raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, wanted ? q.at + 16 * p : kOutOfRange, 0, aux);
-      }
-    };
-    if (kStream && past_cache)
-      load_pieces(std::integral_constant<int, 2>{});
-    else
-      load_pieces(std::integral_constant<int, 0>{});
+    for (int i = 0; i < kVecs; ++i) {
+      const int p = p0 + lane + kLanes * i;
+      const bool wanted = (kRows == 1 || row.live) && p < q.pieces;
+      raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, wanted ? q.at + 16 * p : kOutOfRange, 0, kAux);
+    }
     // entries that are not the row's become -inf (whole pieces of a whole wave need no test)
 #pragma unroll
     for (int i = 0; i < kVecs; ++i) {
@@ -253,16 +246,15 @@ void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Pic
         around.blocks = (unsigned)around.t_tiles * ((L.S + kAssembleRows) / kAssembleRows);
       }
       const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) >
-                       (read_again ? kStreamBytes : kReadOnceBytes);
-      const long kept = read_again ? kKeptBytes : 0;
+                       (read_again ? 2 * kCacheBytes : kCacheBytes);
       with_row_split<P>(logits, L.C, [&](auto lanes, auto vecs, auto loop) {
         const dim3 grid = batch_grid(around.blocks + (rows + 256 / lanes - 1) / (256 / lanes), L.B);
         if (big && lanes == 64)
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, lanes == 64>), grid, dim3(256),
-                             0, stream, logits, L, out, around, kept);
+                             0, stream, logits, L, out, around);
         else
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, false>), grid, dim3(256), 0,
-                             stream, logits, L, out, around, kept);
+                             stream, logits, L, out, around);
       });
       return;
     }

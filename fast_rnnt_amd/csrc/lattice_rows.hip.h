@@ -181,7 +181,7 @@ inline dim3 batch_grid(long blocks, int B) {
 // before the first is used, through a raw buffer resource over the wave's rows: a piece that is
 // not wanted gets an offset outside it, reads as 0 and moves no data -- no branch stands between
 // the loads.  kLoop: rows of more pieces than registers, in chunks of kLanes * kVecs.
-// kStream: see kStreamBytes.
+// kStream: see kCacheBytes and kStreamBytes.
 template <typename P, int kLanes>
 struct RowPieces {
   int off;      // elements of the first piece that lie before the row
@@ -212,25 +212,32 @@ __device__ __forceinline__ long wave_bytes(int C) {
   return ((long)(kWave / kLanes) * C * (long)sizeof(typename P::Elem) + 31) & ~15L;
 }
 
-// Logits beyond this many bytes are streamed (non-temporal hint): the gradient as it is read and
-// written, which leaves the last-level cache (256 MB) to the logits of the next forward pass and
-// of this one, and, of the forward, the rows further than kKeptBytes from the end.  The backward starts
-// from the end, where it finds in the cache what the forward read last.  Forward + backward, five rows a
-// frame, B 20, T 500, against 192 MiB, a forward streamed throughout and a backward from the
-// first row on: C 560, 112 MB: 29.4 + 32.4 -> 27.1 + 31.3 us; C 900: 39.2 + 51.8 -> 30.4 + 49.4; C 1300:
-// 34.9 + 81.6 -> 37.6 + 69.2; the whole lattice, B 8, S 60, T 200, C 1000, 390 MB: 53 + 115 -> 55 + 95;
-// bfloat16, B 16, T 400, C 5000, 320 MB: 46 + 100 -> 49 + 89; 1.6 GB (B 32, S 60, T 200, C 1000): 195 +
-// 482 -> 200 + 471.  Below the line the hint costs (80 MB: 20.1 + 24.0 -> 21.2 + 25.4).
+// ---- the last-level cache (256 MB) ---------------------------------------------------------------
+// A joiner writes the logits from the first row to the last and leaves the last ones in the cache; its
+// backward reads the gradient from the first row on.  So the forward pass goes from the last row to the
+// first, and finds what the joiner has left, and the backward from the first to the last, and finds what
+// the forward has left.  (With a forward from the first row on, which pushes out what it has yet to come
+// to, and a backward from the last, behind a linear layer that writes the logits: B 8, S 60, T 200, C 1000,
+// 372 MiB: 71 + 97 us, now 58 + 103; bfloat16, B 16, T 400, five rows a frame, C 5000, 305 MiB: 69 + 92,
+// now 54 + 99; float32, B 20, T 500, C 1500, 286 MiB: 50 + 79, now 45 + 84.  On logits that lie in memory
+// untouched the two are worth the same to 2 %: 53 + 95 and 52 + 98 at 372 MiB.)
+//
+// Logits of more than two caches that the backward will read, or of more than one that it will not, are
+// read with the non-temporal hint: too little of them would still be there when it is wanted, and read
+// past the cache they leave it to what the joiner wrote last.  Without the hint and with it, behind that
+// layer: forward and backward, pruned bfloat16, 763 MiB: 411 and 362 us, 534 MiB: 281 and 254, 458 MiB:
+// 233 and 219; the whole lattice, 605 MiB: 286 and 272, 512 MiB: 224 and 228, 465 MiB: 202 and 210, 372
+// MiB: 162 and 169; a forward alone, 372 MiB: 60 and 53, 305 MiB: 51 and 49, 298 MiB: 43 and 42, 248 MiB:
+// 38 and 38, 208 MiB: 38.6 and 39.5, 183 MiB: 32 and 36.
+constexpr long kCacheBytes = 256L << 20;
+// The gradient is read and written with that hint from this many bytes of logits on, which leaves the
+// cache to what the joiner's backward reads beside it.  Forward, backward, and the linear layer and its
+// gradients around them, without the hint and with it: bfloat16, 104 MiB: 465 and 462 us; 122 MiB: 488 and
+// 479; 153 MiB: 616 and 607; 183 MiB: 614 and 599; float32, 107 to 210 MiB: 0.1 to 0.3 % less with it at
+// six sizes, 0.3 % more at a seventh; float16, 122 MiB: 857 and 865.  The gradient pass itself is 13 %
+// slower to 3 % faster with it below 200 MiB and faster above (372 MiB: 113 and 103).  Below the line
+// the hint costs (80 MiB: 851 and 855).
 constexpr long kStreamBytes = 96L << 20;
-// (1.5 times the cache: of a ragged batch a fifth to a third is never read.  B 8, S 60, T 200, C 1000:
-// backward 121 us with 128 MiB, 116 with 192, 108 with 256, 100 with 320, 95 with 384.)
-constexpr long kKeptBytes = 384L << 20;
-// A forward pass that no backward follows reads logits larger than the cache with the hint, all of them:
-// what the caller wrote last is found in the cache while the rest passes it by.  Behind the linear layer that
-// writes the logits, without the hint and with it: B 8, S 60, T 200, C 1000, 372 MiB: 73 and 54 us; bfloat16,
-// B 16, T 400, five rows a frame, C 5000, 305 MiB: 71 and 51; float32, B 20, T 500, five rows, C 1300, 248 MiB:
-// 37.3 and 36.6; C 900, 172 MiB: 30.3 and 31.4; bfloat16, C 3400, 208 MiB: 38.1 and 39.3.
-constexpr long kReadOnceBytes = 256L << 20;
 
 // Whether every row begins and ends on 16 bytes.
 template <typename P>

@@ -90,10 +90,10 @@ def test_gradients_of_aligned_rows_are_the_bits_of_any_others(gpu_device, sfx, d
         assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
 
 
-@pytest.mark.parametrize("B,C", [(3, 750), (12, 751)])
+@pytest.mark.parametrize("B,C", [(3, 750), (12, 751), (16, 752)])
 def test_streamed_logits_give_the_bits_of_their_utterances(gpu_device, B, C):
-    # 110 and 440 MB: past the size from which logits are streamed, and past the one from which the
-    # forward streams the rows that lie far from the end; an utterance alone takes neither path
+    # 105, 419 and 560 MiB: past the sizes from which the gradient, a forward pass alone and a forward pass
+    # before a backward are streamed; an utterance alone takes none of these paths
     T, S = 200, 60
     g = torch.Generator(device=gpu_device).manual_seed(C)
     logits = torch.randn(B, T, S + 1, C, generator=g, device=gpu_device)
