@@ -1078,11 +1078,6 @@ void launch_bwd_t(const float *lm, const float *am, const int64_t *symbols,
                      term, rnnt_type, lm_at, am_at, out_type, smooth);
 }
 // Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand
-// along the vocabulary half as often as 64 (am.grad at B 16, T 400, C 5000: 92 against 97 us;
-// lm.grad 60 against 65), which is what counts once the chip is full; they lose where the padding
-// of the last tile outweighs that (up to 64 rows: 24 against 18 us at B 21, S 47, T 333, C 503) or
-// where fewer of them than fill the chip remain (B 3, S 250, T 1335, C 198: 71 against 55 us).
-// Rows of a workgroup's tile, each product's by its own.  128 rows read and convert the operand
 // along the vocabulary half as often as 64 (both products at B 64, S 120, T 600, C 500: 74 against 90
 // us; B 16, S 120, T 400, C 5000: 108 against 132), which is what counts once the chip is full; they
 // lose where the padding of the last tile outweighs that (lm.grad's up to 64 rows: 20 against 17 us at

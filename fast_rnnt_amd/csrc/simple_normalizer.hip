@@ -32,16 +32,16 @@ namespace {
 // first, about 250 for maxima, conversions and a quarter-rate exp2, 100 for LDS, and 300 besides), so
 // what counts is that every SIMD of the chip has its share of that, and that another workgroup's loop
 // covers a workgroup's prologue and epilogue (4.5 and 5 us).  Hence small tiles -- taller ones convert
-// less per cell, but of 16 utterances' tiles of 128 rows a third of the compute units got none --
-// dealt out evenly (find_tile), and eight waves of one share each or four of two
-// (choose_tile).  Measured within training steps on three batches in turn, against tiles of
-// 32 to 128 rows with a workgroup per tile whether it counted or not: B 64, S 120, T 600, C 500: 96 ->
-// 89 us; B 32, S 80, T 250, C 500: 20.4 and 20.6; B 16, S 120, T 400, C 5000: 127 -> 122; B 10, S 137,
-// T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64 sizes, B 1 .. 128,
-// C 50 .. 5000: 5.6 %.  Tiles of 64, 96 and 128 rows dealt out the same way were the fastest at 12 of the
+// less per cell, but leave compute units without any -- dealt out evenly (find_tile), and eight waves of
+// one share each or four of two (choose_tile).  Measured within training steps on three batches in turn,
+// against tiles chosen among 32 to 128 rows, a workgroup per tile whether it counted or not: B 64, S 120,
+// T 600, C 500: 96 -> 89 us; B 32, S 80, T 250, C 500: 20.4 and 20.6; B 16, S 120, T 400, C 5000: 127 ->
+// 122; B 10, S 137, T 817, C 500: 47 -> 26; B 5, S 224, T 743, C 2536: 131 -> 64; geometric mean over 64
+// sizes, B 1 .. 128, C 50 .. 5000: 5.6 %.  Taller tiles dealt out the same way were the fastest at 12 of the
 // 64, mostly by 1 to 5 %, and a choice among all of them, which cannot know how ragged a batch is, gained
 // nothing; 64 and 96 rows are left where they have a compute unit each and, where no window makes a batch
-// ragged, by the number of tiles of each height (choose_tile).
+// ragged, by the number of tiles of each height.  (128 rows there: 123 us instead of 129 at B 16, S 120,
+// T 400, C 5000, and 68 instead of 70 at B 5, S 224, T 743, C 2536, the fastest at these two of 256 sizes.)
 constexpr int kNormK = 16;      // k per slab
 constexpr int kNormShares = 8;  // of k
 constexpr int kNormT = 32;      // frames of a tile
@@ -65,7 +65,7 @@ struct NormShape {
       (kS * kNormT / 4 + kThreads - 1) / kThreads;
   static constexpr size_t kFixedBytes = ((kNormShares + 1) * kRows + 3 * kS + kNormT) * 4;  // (below)
   static constexpr int kPerCu = kS <= 64 ? 16 / kWaves : 1;  // workgroups
-  static_assert(kS % 32 == 0 && kS <= 128, "shape");
+  static_assert(kS % 32 == 0 && kS <= 96, "shape");
   static_assert(kPerCu * (kLdsBytes + kFixedBytes) <= 160 << 10, "LDS per CU");
 };
 
