@@ -98,7 +98,7 @@ def _rate(steps, elapsed):
 
 
 def _measured_traffic(workload):
-    """{kernel name: HBM bytes per launch} from the committed counter summary of this
+    """{kernel name: bytes per launch behind the L2s} from the committed counter summary of this
     workload: the table rows `kernel  FETCH_SIZE  WRITE_SIZE  fetch MB  write MB  total MB`."""
     path = os.path.join(ROOT, "profiles", TRAFFIC_FILES.get(workload, ""))
     table = {}
