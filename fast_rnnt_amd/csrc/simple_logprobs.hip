@@ -283,7 +283,7 @@ constexpr int kProdK = 32;  // k per chunk of the float32 gradient products: two
 // 256-thread workgroups.  The first ceil(B*(S+1)/4) of them give each wave one
 // lattice row (b, s): D[b,s,:] and the two row sums.  With `score_grad` the wave first scales
 // its row of the occupation gradients in place (scale_by_batch_kernel's work, for lattices whose
-// rows do not read each other's: one pass over them less).  `joint`: what they count for here
+// rows do not read each other's: one pass over them less).  `joint`: what they count for in D
 // (1, less in the smoothed loss).  Loads are issued in batches of
 // four before anything is stored, so a row costs one memory round trip, not one per 64 frames.
 // Bound by memory; cells outside the windows, a third of a ragged batch, are neither read nor written
@@ -357,9 +357,9 @@ __global__ void __launch_bounds__(256)
           gx_row.put(t >= scaled_lo && t < scaled_hi, t, gx[u]);
           gy_row.put(t >= scaled_lo && t < scaled_hi, t, gy[u]);
         }
-        gx[u] = ok && t != t_mask ? gx[u] * joint : (R)0;
-        gy[u] = ok ? gy[u] * joint : (R)0;
-        if (t < d_hi) d_row[t] = -(gx[u] + gy[u]) * fast_exp<R>(-nr[u]);
+        gx[u] = ok && t != t_mask ? gx[u] : (R)0;
+        gy[u] = ok ? gy[u] : (R)0;
+        if (t < d_hi) d_row[t] = -(gx[u] * joint + gy[u] * joint) * fast_exp<R>(-nr[u]);
         sx += gx[u];
         sy += gy[u];
       }
@@ -699,11 +699,12 @@ __device__ __forceinline__ void simple_bwd_lm_body(
     const float *__restrict__ am_max, const float *__restrict__ dmat,
     const float *__restrict__ row_x, const float *__restrict__ row_y,
     void *__restrict__ lm_grad, const int64_t *__restrict__ window, int S, int T, int C, int ldd,
-    int term, int out_type) {
+    int term, int out_type, const SmoothTerms &smooth) {
   using Shape = ProdShape<kM>;
   using namespace dgemm;
   extern __shared__ __align__(16) char prod_lds[];
   __shared__ float row_mx[kM], row_rx[kM], row_ry[kM];
+  __shared__ float row_w[kSmooth ? kM : 1], row_inv[kSmooth ? kM : 1];  // (times exp(lm - max): lm-only terms)
   __shared__ int row_sym[kM];
   const int S1 = S + 1;
   const Limits lim = limits_of(window, b, S, T);
@@ -746,11 +747,23 @@ __device__ __forceinline__ void simple_bwd_lm_body(
         if (tid < kM) {
           const int s = s_tile + tid, at = 4 * s;
           const long first_row = (long)b * S1;
-          const float mx = get_float(buffer_of(lm_max + first_row, S1 * 4), s < s_lim, at);
+          float mx = get_float(buffer_of((kSmooth ? smooth.lm_max : lm_max) + first_row, S1 * 4),
+                               s < (kSmooth ? S1 : s_lim), at);
           const float rx = get_float(buffer_of(row_x + first_row, S1 * 4), s < S, at);
           const float ry = get_float(buffer_of(row_y + first_row, S1 * 4), s < S1, at);
+          if (kSmooth) {
+            const float sum = get_float(buffer_of(smooth.lm_sum + first_row, S1 * 4), s < S1, at);
+            const float dot = smooth.am_scale != 0.f
+                                  ? get_float(buffer_of(smooth.lm_dot + first_row, S1 * 4), s < S1, at)
+                                  : 0.f;
+            if (smooth.am_scale == 0.f) mx += *smooth.unigram;
+            const float inv = 1.f / sum;
+            row_w[tid] = (-dot * smooth.per_row - smooth.lm_scale * (rx + ry)) * inv;
+            row_inv[tid] = smooth.per_row * inv;
+          }
+          const float times = kSmooth ? smooth.joint + smooth.lm_scale : 1.f;
           row_sym[tid] = get_symbol(symbols_of(symbols + (long)b * S, S), s < S, s, C);
-          row_mx[tid] = mx, row_rx[tid] = rx, row_ry[tid] = ry;
+          row_mx[tid] = mx, row_rx[tid] = rx * times, row_ry[tid] = ry * times;
         }
       },
       [&] {
@@ -762,6 +775,30 @@ __device__ __forceinline__ void simple_bwd_lm_body(
       });
 
   // ---- results: a lane holds column r32 of rows 8 (v / 4) + 4 half + v % 4 of its tiles (row_of)
+  auto zero_past_end = [&] {
+    if (s_tile + m_wave + 32 > s_lim) {  // (uniform)
+#pragma unroll
+      for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[n][v] = s_tile + row_of(v) < s_lim ? acc[n][v] : 0.f;
+    }
+  };
+  if (kSmooth) {
+    zero_past_end();  // (the lm-only model's rows all count)
+#pragma unroll
+    for (int n = 0; n < Shape::kTiles; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[n][v] += row_w[row_of(v)];
+    if (smooth.am_scale != 0.f) {  // (uniform)
+#pragma unroll
+      for (int n = 0; n < Shape::kTiles; ++n) {
+        const float gu = get_float(buffer_of(smooth.g_unigram, C * 4), c0 + 32 * n < C, 4 * (c0 + 32 * n));
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[n][v] += gu * row_inv[row_of(v)];
+      }
+    }
+  }
 #pragma unroll
   for (int n = 0; n < Shape::kTiles; ++n)
 #pragma unroll
@@ -778,20 +815,7 @@ __device__ __forceinline__ void simple_bwd_lm_body(
         acc[n][v] = (acc[n][v] + rx) + ry;
       }
   }
-  if (s_tile + m_wave + 32 > s_lim) {  // (uniform)
-#pragma unroll
-    for (int n = 0; n < Shape::kTiles; ++n)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        acc[n][v] = s_tile + row_of(v) < s_lim ? acc[n][v] : 0.f;
-  }
-  if (kSmooth) {
-#pragma unroll
-    for (int n = 0; n < Shape::kTiles; ++n)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        acc[n][v] += get_float(out_rs, c0 + 32 * n < C, 4 * (first + 32 * n), 4 * below(v));
-  }
+  if (!kSmooth) zero_past_end();
   with_store(out_type, [&](auto store) {
 #pragma unroll
     for (int n = 0; n < Shape::kTiles; ++n)
@@ -902,8 +926,8 @@ __device__ __forceinline__ void simple_bwd_am_body(
           if (tid < kM) {
             const int t = t_tile + tid;
             const float mx = get_float(buffer_of(am_max + (long)b * T, T * 4), t < t_lim, 4 * t);
-            frame_mx[tid] = mx;
-            if (kSmooth) {
+            frame_mx[tid] = kSmooth && smooth.am_scale == 0.f ? mx + *smooth.unigram : mx;
+            if (kSmooth && smooth.am_scale != 0.f) {
               const float g = get_float(buffer_of(smooth.am_g + (long)b * T, T * 4), t < t_lim, 4 * t);
               const float z = get_float(buffer_of(smooth.am_z + (long)b * T, T * 4), t < t_lim, 4 * t);
               frame_w[tid] = t < t_lim ? -smooth.am_scale * g / z : 0.f;
@@ -959,7 +983,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
       lds_barrier();
     }
     float unigram[Shape::kTiles];
-    if (kSmooth)
+    if (kSmooth && smooth.am_scale != 0.f)
 #pragma unroll
       for (int n = 0; n < Shape::kTiles; ++n)
         unigram[n] = get_float(buffer_of(smooth.unigram, C * 4), c0 + 32 * n < C, 4 * (c0 + 32 * n));
@@ -968,7 +992,7 @@ __device__ __forceinline__ void simple_bwd_am_body(
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int m = row_of(v);
-        if (kSmooth) acc[n][v] += frame_w[m] * unigram[n];
+        if (kSmooth && smooth.am_scale != 0.f) acc[n][v] += frame_w[m] * unigram[n];
         acc[n][v] *= __expf(in[n][v] - frame_mx[m]);
         if (c0 + 32 * n == term) acc[n][v] += frame_y[m];
       }
@@ -1016,14 +1040,14 @@ __device__ __forceinline__ void simple_bwd_am_body(
 void launch_fwd_gemm(const float *lm, const float *am, const int64_t *symbols,
                      const int64_t *boundary, float *lm_max, float *am_max, float *px,
                      float *py, float *norm_raw, const int64_t *window, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
-                     hipStream_t stream) {
+                     const SmoothMix *mix, hipStream_t stream) {
   launch_normalizer_f32(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw, window,
-                        delay_penalty, B, S, T, C, term, rnnt_type, stream);
+                        delay_penalty, B, S, T, C, term, rnnt_type, mix, stream);
 }
 void launch_fwd_gemm(const double *lm, const double *am, const int64_t *symbols,
                      const int64_t *boundary, const double *lm_max, const double *am_max,
                      double *px, double *py, double *norm_raw, const int64_t *, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
-                     hipStream_t stream) {
+                     const SmoothMix *, hipStream_t stream) {
   // (the double kernels compute the whole lattice whether or not a window is given)
   const int t_tiles = T > 0 ? (T + kTileN - 1) / kTileN : 1;
   const dim3 grid(t_tiles, (S + 1 + kTileM - 1) / kTileM, B);
@@ -1053,7 +1077,7 @@ __global__ void __launch_bounds__(kProdThreads, kProdPerCu)
     if (!place_block(blockIdx.x, lm_at, B, row_x, S, b, row_idx, c_idx)) return;
     simple_bwd_lm_body<kMl, kSmooth>(b, row_idx, c_idx, lm, am, symbols, lm_max, am_max, dmat,
                                          row_x, row_y, lm_grad, window, S, T, C, ldd, term,
-                                         out_type);
+                                         out_type, smooth);
   } else {
     if (!place_block(blockIdx.x - lm_at.blocks, am_at, B, row_x, S, b, row_idx, c_idx)) return;
     simple_bwd_am_body<kMa, kSmooth>(b, row_idx, c_idx, lm, am, symbols, boundary, lm_max, am_max,
@@ -1159,7 +1183,8 @@ void launch_scale(R *px_grad, R *py_grad, const R *score_grad, int score_grad_st
 template <typename R>
 int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary, R *px,
              R *py, R *lm_max, R *am_max, R *norm_raw, double delay_penalty, int B,
-             int S, int T, int C, int term, int rnnt_type, int window_only, void *stream_) {
+             int S, int T, int C, int term, int rnnt_type, int window_only, void *stream_,
+             const SmoothMix *mix = nullptr) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_fwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2)
     return fail(FRNNT_EINVAL, "simple_logprobs_fwd: rnnt_type must be 0, 1 or 2");
@@ -1184,7 +1209,7 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   const bool constrained = rnnt_type == kConstrained;
   launch_fwd_gemm(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw,
                   window_only ? boundary : nullptr, constrained ? 0.0 : delay_penalty, B,
-                  S, T, C, term, rnnt_type, stream);
+                  S, T, C, term, rnnt_type, mix, stream);
   if (constrained && S > 0 && T > 0) {
     const long total = (long)B * S * T;
     hipLaunchKernelGGL(add_next_row_kernel<R>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
@@ -1199,7 +1224,7 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
              int score_grad_stride, double score_grad_scale, R *px_grad, R *py_grad, R *dmat,
              R *row_x, R *row_y, R *col_y, void *lm_grad, void *am_grad, int B, int S, int T, int C,
              int term, int rnnt_type, int window_only, int out_type, void *stream_,
-             const SmoothTerms *smooth = nullptr) {
+             const SmoothTerms *smooth = nullptr, const std::function<void()> *between = nullptr) {
   constexpr bool is_float = std::is_same<R, float>::value;
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_bwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2 || term < 0 || term >= C)
@@ -1234,6 +1259,7 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
                      px_grad, py_grad, norm_raw, boundary, window, score_grad, score_grad_stride,
                      (R)score_grad_scale, smooth ? (R)smooth->joint : (R)1, dmat, row_x, row_y, col_y, B,
                      S, T, ldd, rnnt_type);
+  if (between) (*between)();
   launch_bwd(lm, am, symbols, boundary, lm_max, am_max, dmat, px_grad, py_grad, row_x, row_y, col_y,
              lm_grad, am_grad, window, B, S, T, C, ldd, term, rnnt_type, out_type, smooth, stream);
   return check_launch("simple_logprobs_bwd");
@@ -1329,9 +1355,9 @@ float *own_scratch_address() {
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
                         float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
-                        void *stream) {
+                        void *stream, const SmoothMix *mix) {
   return fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                         delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream);
+                         delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream, mix);
 }
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
@@ -1345,12 +1371,13 @@ int simple_logprobs_bwd_smoothed(const float *lm, const float *am, const int64_t
                                  const float *norm_raw, const float *score_grad,
                                  int score_grad_stride, double score_grad_scale, float *px_grad,
                                  float *py_grad, float *dmat, float *row_x, float *row_y,
-                                 const SmoothTerms &smooth, float *lm_grad, float *am_grad, int B,
-                                 int S, int T, int C, int term, int rnnt_type, void *stream) {
+                                 const SmoothTerms &smooth, const std::function<void()> &between,
+                                 float *lm_grad, float *am_grad, int B, int S, int T, int C, int term,
+                                 int rnnt_type, void *stream) {
   return bwd_impl<float>(lm, am, symbols, boundary, lm_max, am_max, norm_raw, score_grad,
                          score_grad_stride, score_grad_scale, px_grad, py_grad, dmat, row_x, row_y,
                          nullptr, lm_grad, am_grad, B, S, T, C, term, rnnt_type, boundary != nullptr,
-                         FRNNT_F32, stream, &smooth);
+                         FRNNT_F32, stream, &smooth, &between);
 }
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
                   long n_lm, long n_am, hipStream_t stream) {

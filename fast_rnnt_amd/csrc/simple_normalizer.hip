@@ -162,6 +162,9 @@ struct NormArgs {
   int B, S, T, C, term, rnnt_type;
 };
 
+// A joint model on its own
+struct NoMix {};
+
 // f(a constant), the constant being min(max(n, 1), kMost)
 template <int kMost, typename F>
 __device__ __forceinline__ void with_tiles(int n, F &f) {
@@ -171,9 +174,13 @@ __device__ __forceinline__ void with_tiles(int n, F &f) {
   f(std::integral_constant<int, kMost>{});
 }
 
-template <int kS, int kWaves>
+// With a Mix (the smoothed loss) px and py leave interpolated with the lm-only and the am-only model:
+// am[t,sym[s]] and what depends on a row or a frame alone are here already, and a launch of its own for
+// the interpolation would read and write every cell again (B 32, S 80, T 250, C 500: 12.8 us).
+template <int kS, int kWaves, typename Mix>
 __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / kWaves : 1))
-    simple_fwd_panel_kernel(NormArgs A, NormPlan plan) {
+    simple_fwd_panel_kernel(NormArgs A, NormPlan plan, Mix mix) {
+  constexpr bool kMix = !std::is_same_v<Mix, NoMix>;
   using Shape = NormShape<kS, kWaves>;
   constexpr int kT = kNormT, kShares = kNormShares, kTurns = Shape::kTurns;
   constexpr int kRows = Shape::kRows, kLoads = Shape::kLoads, kLmLoads = kS / 16;
@@ -185,6 +192,9 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   __shared__ float slab_max[kRows];            // row maxima
   __shared__ int row_symbol[kS];
   __shared__ float col_term[kT];  // am[t,term]
+  // lm-only terms of a row (px, py), log-unigram of its symbol; am-only term (py) and normalizer of a frame
+  constexpr int kMixRows = kMix ? kS : 1, kMixFrames = kMix ? kT : 1;
+  __shared__ float mix_x[kMixRows], mix_y[kMixRows], mix_u[kMixRows], mix_n[kMixFrames], mix_t[kMixFrames];
   const int S = A.S, T = A.T, C = A.C, S1 = S + 1;
   NormTile tile;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -273,6 +283,26 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   const float frame_value =
       get_float(am_rs, tid >= 128 && t_tile + tid - 128 < T, (my_frame + A.term) * 4);
   const float my_term = tid < kS ? row_value : frame_value;
+  // (of a row: maximum and sum of the lm-only model, unigram of its symbol; of a frame: maximum and sum
+  // of the am-only model, unigram of the termination symbol)
+  float mix_max = 0.f, mix_sum = 1.f, mix_unigram = 1.f;
+  if constexpr (kMix) {
+    const bool is_row = tid < kS, has_frame = tid >= 128 && t_tile + tid - 128 < T;
+    const long rows = (long)b * S1, frames = (long)b * T;
+    const int at = 4 * (is_row ? s_tile + tid : t_tile + tid - 128);
+    mix_max = get_float(buffer_of(mix.lm_max + rows, S1 * 4), has_row, at);
+    mix_sum = get_float(buffer_of(mix.lm_sum + rows, S1 * 4), has_row, at);
+    if (mix.k_am != 0.f) {  // (uniform)
+      const float am_max = get_float(buffer_of(mix.am_max + frames, T * 4), has_frame, at);
+      const float am_z = get_float(buffer_of(mix.am_z + frames, T * 4), has_frame, at);
+      mix_unigram = get_float(buffer_of(mix.unigram, C * 4), true, 4 * (is_row ? max(my_sym, 0) : A.term));
+      mix_max = is_row ? mix_max : am_max, mix_sum = is_row ? mix_sum : am_z;
+    } else if (!is_row) {
+      for (int i = lane; i < mix.n_checks; i += 4 * kWave)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mix_max += mix.checks[min(i + kWave * u, mix.n_checks - 1)];
+    }
+  }
   // ... and am[b, t, sym[b, s]] of this thread's outputs: 16-byte pieces (row item / 8, frames
   // 4 (item % 8) ..)
   float am_sym[kItems][4];
@@ -421,12 +451,26 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
         mine[2 * kRows * q + kRows + sub + 16 * j] = shift2[q][j];
       }
     }
+  // (all of wave 2, whose first lanes own the frames)
+  const float check = kMix && __any(mix_max != mix_max) ? std::numeric_limits<float>::quiet_NaN() : 0.f;
   if (tid < kS) {
     row_term[tid] = my_term;
     row_sym[tid] = my_symval;
     row_symbol[tid] = my_sym;
+    if constexpr (kMix) {
+      const float ln = logf(mix_sum) + mix_max;
+      mix_x[tid] = my_symval - ln;
+      mix_y[tid] = my_term - ln;
+      mix_u[tid] = logf(mix_unigram);
+    }
   } else if (tid >= 128 && tid < 128 + kT) {
     col_term[tid - 128] = my_term;
+    if constexpr (kMix) {
+      if (mix.k_am == 0.f && tid == 128 && b == 0 && t_tile == 0 && s_tile == 0) *mix.check = check;
+      const float an = logf(mix_sum) + mix_max;
+      mix_n[tid - 128] = mix.k_am != 0.f ? an : check;
+      mix_t[tid - 128] = mix.k_am != 0.f ? ((my_term + logf(mix_unigram)) - an) * mix.k_am : check;
+    }
   }
   __syncthreads();
   float *lm_max = A.lm_max + (long)b * S1, *am_max = A.am_max + (long)b * T;
@@ -503,6 +547,13 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
       const float norm = raw[i] + slab_max[m] + slab_max[kS + out_t + i];
       yv[i] = (col_term[out_t + i] + row_term[m]) - norm;
       xv[i] = (am_sym[j][i] + row_sym[m]) - norm;
+      if constexpr (kMix) {
+        // (left to right, as rnnt_loss.py:1338-1362)
+        float am_only = mix_n[out_t + i];
+        if (mix.k_am != 0.f) am_only = ((am_sym[j][i] + mix_u[m]) - am_only) * mix.k_am;  // (uniform)
+        yv[i] = yv[i] * mix.k_joint + mix_y[m] * mix.k_lm + mix_t[out_t + i];
+        xv[i] = xv[i] * mix.k_joint + mix_x[m] * mix.k_lm + am_only;
+      }
       if (row_symbol[m] < 0) xv[i] = std::numeric_limits<float>::quiet_NaN();  // out-of-vocabulary
       if (tr + i == t_mask) xv[i] = ninf;
       xv[i] = A.delay.at(xv[i], A.boundary, b, tr + i, T);
@@ -535,14 +586,15 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   }
 }
 
-template <int kS, int kWaves>
-void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, hipStream_t stream) {
-  auto kernel = simple_fwd_panel_kernel<kS, kWaves>;
+template <int kS, int kWaves, typename Mix>
+void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, const Mix &mix, hipStream_t stream) {
+  auto kernel = simple_fwd_panel_kernel<kS, kWaves, Mix>;
   constexpr size_t lds = NormShape<kS, kWaves>::kLdsBytes;
   if (!allow_lds(reinterpret_cast<const void *>(kernel), lds)) return;
   const long tiles = (long)args.B * plan.t_tiles * plan.s_tiles;
   const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS, kWaves>::kThreads), lds, stream, args, plan);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS, kWaves>::kThreads), lds, stream, args, plan,
+                     mix);
 }
 
 struct NormChoice {
@@ -612,19 +664,25 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                            const int64_t *boundary, float *lm_max, float *am_max, float *px,
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
-                           int rnnt_type, hipStream_t stream) {
+                           int rnnt_type, const SmoothMix *mix, hipStream_t stream) {
   const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
                       Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
   const NormChoice choice = choose_tile(B, S, T, C, window != nullptr);
   const NormPlan plan{T > 0 ? (T + kNormT - 1) / kNormT : 1, (S + choice.rows) / choice.rows, choice.all};
-  if (choice.rows == 96)
-    launch_fwd_panel<96, 8>(args, plan, stream);
-  else if (choice.rows == 64)
-    launch_fwd_panel<64, 8>(args, plan, stream);
-  else if (choice.waves == 4)
-    launch_fwd_panel<32, 4>(args, plan, stream);
+  auto launch = [&](const auto &m) {
+    if (choice.rows == 96)
+      launch_fwd_panel<96, 8>(args, plan, m, stream);
+    else if (choice.rows == 64)
+      launch_fwd_panel<64, 8>(args, plan, m, stream);
+    else if (choice.waves == 4)
+      launch_fwd_panel<32, 4>(args, plan, m, stream);
+    else
+      launch_fwd_panel<32, 8>(args, plan, m, stream);
+  };
+  if (mix)
+    launch(*mix);
   else
-    launch_fwd_panel<32, 8>(args, plan, stream);
+    launch(NoMix{});
 }
 }  // namespace frnnt
 

@@ -2,6 +2,8 @@
 // files: simple_normalizer.hip (the forward's normalizer product, compiled with a scheduling
 // strategy of its own) and simple_logprobs.hip (everything else).
 #pragma once
+#include <functional>
+
 #include "xcd_grid.hip.h"
 
 namespace frnnt {
@@ -130,40 +132,56 @@ __device__ __forceinline__ void lds_barrier() {
 
 }  // namespace
 
+// What the smoothed loss mixes into px and py where they are formed: px = joint k_joint + lm_only k_lm +
+// am_only k_am (py likewise), with the row statistics of the two models, max and sum of exp(x - max).
+// k_am = 0: no am-only model; its three arrays are not read, but px and py still take the sum of
+// `checks`, 0 or a NaN (the unigram of the am-only model is a mean over the whole batch, so that one bad
+// row of lm reaches every utterance), which is also left in `check` for the backward.
+struct SmoothMix {
+  const float *lm_max, *lm_sum, *am_max, *am_z, *unigram, *checks;
+  float *check;
+  float k_joint, k_lm, k_am;
+  int n_checks;
+};
 // The float32 normalizer product with px / py in its epilogue (simple_normalizer.hip).
 void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symbols,
                            const int64_t *boundary, float *lm_max, float *am_max, float *px,
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
-                           int rnnt_type, hipStream_t stream);
+                           int rnnt_type, const SmoothMix *mix, hipStream_t stream);
 
 // frnnt_simple_logprobs_fwd with the delay penalty (simple_logprobs.hip).
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
                         float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
-                        void *stream);
+                        void *stream, const SmoothMix *mix = nullptr);
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
                         double *am_max, double *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
                         void *stream);
-// What the smoothed loss adds to the gradient products (smoothed_logprobs.hip): lm_grad already holds
-// its own part of lm's gradient, and
-//   am.grad[t,c] -= exp(am[t,c] - max[t]) * am_scale * am_g[t] / am_z[t] * unigram[c],
-// the per-symbol and termination terms of am are taken times symbol_scale, and everything that
-// belongs to the joint model times `joint`.
+// What the smoothed loss adds to the gradient products (smoothed_logprobs.hip): to lm's gradient
+//   exp(lm[s,c] - lm_max[s]) / lm_sum[s] * ((g_unigram[c] - lm_dot[s]) / N - lm_scale (rx + ry))
+//   + lm_scale (rx [c = sym] + ry [c = term]),
+// rx and ry the row sums of px_grad and py_grad, and to am's
+//   -exp(am[t,c] - max[t]) * am_scale * am_g[t] / am_z[t] * unigram[c];
+// the joint model's terms count `joint` times and the per-symbol and termination terms of am symbol_scale
+// times.  am_scale = 0: no am-only model; am_g, am_z, lm_dot and g_unigram are not read, and unigram is the
+// check that the forward left (SmoothMix).
 struct SmoothTerms {
-  const float *am_g, *am_z, *unigram;
-  float am_scale, symbol_scale, joint;
+  const float *am_g, *am_z, *unigram, *lm_max, *lm_sum, *lm_dot, *g_unigram;
+  float am_scale, symbol_scale, joint, lm_scale, per_row;  // (1 / N)
 };
 // The backward of the joint model within the smoothed loss: simple_logprobs_bwd with these terms.
-// px_grad and py_grad are scaled in place by score_grad (may be NULL).
+// px_grad and py_grad are scaled in place by score_grad (may be NULL); `between` is called when row_x and
+// row_y (sums of the scaled gradients) are on their way and the products are not.
 int simple_logprobs_bwd_smoothed(const float *lm, const float *am, const int64_t *symbols,
                                  const int64_t *boundary, const float *lm_max, const float *am_max,
                                  const float *norm_raw, const float *score_grad,
                                  int score_grad_stride, double score_grad_scale, float *px_grad,
                                  float *py_grad, float *dmat, float *row_x, float *row_y,
-                                 const SmoothTerms &smooth, float *lm_grad, float *am_grad, int B,
-                                 int S, int T, int C, int term, int rnnt_type, void *stream);
+                                 const SmoothTerms &smooth, const std::function<void()> &between,
+                                 float *lm_grad, float *am_grad, int B, int S, int T, int C, int term,
+                                 int rnnt_type, void *stream);
 // 2-byte lm and am (`dtype`: FRNNT_F16 or FRNNT_BF16) as float32, in one launch.
 void widen_inputs(int dtype, const void *lm, const void *am, float *lm_wide, float *am_wide,
                   long n_lm, long n_am, hipStream_t stream);

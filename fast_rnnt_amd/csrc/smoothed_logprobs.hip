@@ -186,8 +186,95 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// one thread per px / py element, t fastest.  delay, ends: the delay penalty and the boundary rows
-// that it is counted from (the fused loss; rnnt_loss.py:1470-1479)
+// ---- row statistics of the fused loss --------------------------------------------------------
+// Maximum of one row and the sum of exp(x - maximum), times weight[c] if there are weights, by one wave:
+// eight values per lane in flight, and rows of up to 512 entries stay in registers between the two passes
+// (bound by memory latency: a loop of one load at a time took 8.6 us over the am rows of B 32, T 250,
+// C 500, and 16 over those of B 16, T 400, C 1000; now 6.2 and 10.4).
+template <bool kWeighted>
+__device__ __forceinline__ void row_stats(const float *__restrict__ x, const float *__restrict__ weight,
+                                          int C, int lane, float &max, float &sum) {
+  constexpr int kAhead = 8, kStep = kAhead * kWave;
+  float v[kAhead], w[kAhead];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int c = min(c0 + u * kWave + lane, C - 1);
+      v[u] = x[c];
+      if (kWeighted) w[u] = weight[c];
+    }
+  };
+  max = -__builtin_huge_valf();
+  int c0 = 0;
+  for (; c0 < C; c0 += kStep) {
+    fetch(c0);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) max = fmaxf(max, v[u]);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) max = fmaxf(max, __shfl_xor(max, off, kWave));
+  sum = 0.f;
+  for (c0 = 0; c0 < C; c0 += kStep) {
+    if (C > kStep) fetch(c0);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const float e = __expf(v[u] - max);  // (a NaN among them: the sum is one)
+      if (c0 + u * kWave + lane < C) sum += kWeighted ? e * w[u] : e;
+    }
+  }
+  sum = wave_total(sum);
+}
+// A wave per lm row: its statistics.  Then, with an am-only model, the block's part of the unigram (the sum
+// of its rows' softmax, as weighted_column_partial_kernel forms it: one launch and a read of lm from memory
+// less, 5.3 + 6.7 -> 6.2 us at B 32, S 80, C 500), without one its check: 0, or a NaN where a row has no
+// softmax (4.4 us).
+template <bool kUnigram>
+__global__ void __launch_bounds__(kRowsPerBlock *kWave)
+    lm_models_kernel(const float *__restrict__ lm, float *__restrict__ row_max,
+                     float *__restrict__ row_sum, float *__restrict__ partial, long rows, int C) {
+  __shared__ float max_of[kRowsPerBlock], weight_of[kRowsPerBlock];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row0 = (long)blockIdx.x * kRowsPerBlock, row = row0 + wave;
+  float max = 0.f, sum = 1.f;
+  if (row < rows) row_stats<false>(lm + row * C, nullptr, C, lane, max, sum);
+  if (lane == 0) {
+    if (row < rows) row_max[row] = max, row_sum[row] = sum;
+    max_of[wave] = max;
+    weight_of[wave] = kUnigram ? 1.f / sum : sum * 0.f;
+  }
+  __syncthreads();
+  if (!kUnigram) {
+    if (threadIdx.x == 0) {
+      float check = 0.f;
+#pragma unroll
+      for (int k = 0; k < kRowsPerBlock; ++k) check += weight_of[k];
+      partial[blockIdx.x] = check;
+    }
+    return;
+  }
+  for (int c = threadIdx.x; c < C; c += kRowsPerBlock * kWave) {
+    float v[kRowsPerBlock], acc = 0.f;
+#pragma unroll
+    for (int k = 0; k < kRowsPerBlock; ++k) v[k] = lm[min(row0 + k, rows - 1) * C + c];
+#pragma unroll
+    for (int k = 0; k < kRowsPerBlock; ++k)
+      if (row0 + k < rows) acc += __expf(v[k] - max_of[k]) * weight_of[k];
+    partial[(long)blockIdx.x * C + c] = acc;
+  }
+}
+// a wave per am row: maximum and z = sum_c exp(x - max) unigram[c]
+__global__ void __launch_bounds__(256)
+    am_model_kernel(const float *__restrict__ am, const float *__restrict__ unigram,
+                    float *__restrict__ row_max, float *__restrict__ row_z, long rows, int C) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row = (long)blockIdx.x * 4 + wave;
+  if (row >= rows) return;
+  float max, z;
+  row_stats<true>(am + row * C, unigram, C, lane, max, z);
+  if (lane == 0) row_max[row] = max, row_z[row] = z;
+}
+
+// one thread per px / py element, t fastest
 template <typename R>
 __global__ void __launch_bounds__(256)
     smoothed_combine_kernel(const R *__restrict__ lm, const R *__restrict__ am,
@@ -197,8 +284,7 @@ __global__ void __launch_bounds__(256)
                             const R *__restrict__ lm_sum, const R *__restrict__ am_max,
                             const R *__restrict__ am_z, const R *__restrict__ unigram,
                             R *__restrict__ px, R *__restrict__ py, int B, int S, int T, int C,
-                            int term, int regular, R k_joint, R k_lm, R k_am, Delay<R> delay,
-                            const int64_t *__restrict__ ends) {
+                            int term, int regular, R k_joint, R k_lm, R k_am) {
   const int T1 = regular ? T + 1 : T;
   const int S1 = S + 1;
   const long n_px = (long)B * S * T1, n_py = (long)B * S1 * T;
@@ -223,7 +309,7 @@ __global__ void __launch_bounds__(256)
     // nothing can be emitted after an utterance's last frame (fix_for_boundary,
     // rnnt_loss.py:45-63, applied by the reference after the interpolation)
     if (boundary && regular && boundary[4 * b + 3] == t) v = Num<R>::neg_inf();
-    px[idx] = delay.at(v, ends, b, t, T);
+    px[idx] = v;
   } else if (idx < n_px + n_py) {
     const long j = idx - n_px;
     const int t = (int)(j % T);
@@ -260,8 +346,7 @@ __global__ void __launch_bounds__(256)
                                  const R *__restrict__ lm_sum, const R *__restrict__ am_max,
                                  const R *__restrict__ am_z, const R *__restrict__ unigram,
                                  R *__restrict__ px, R *__restrict__ py, int S, int T, int C,
-                                 int term, int regular, R k_joint, R k_lm, R k_am, Delay<R> delay,
-                                 const int64_t *__restrict__ ends) {
+                                 int term, int regular, R k_joint, R k_lm, R k_am) {
   extern __shared__ __align__(16) unsigned char combine_lds[];
   const int S1 = S + 1, T1 = regular ? T + 1 : T, pitch = S1 | 1;
   R *am_s = reinterpret_cast<R *>(combine_lds);  // [32][pitch]: am[t][sym[s]], column S: am[t][term]
@@ -313,7 +398,7 @@ __global__ void __launch_bounds__(256)
     // nothing can be emitted after an utterance's last frame (fix_for_boundary,
     // rnnt_loss.py:45-63, applied by the reference after the interpolation)
     if (t == t_mask) v = ninf;
-    pxb[(long)s * T1 + t] = delay.at(v, ends, b, t, T);
+    pxb[(long)s * T1 + t] = v;
   }
   const R *pyjb = pyj + (long)b * S1 * T;
   R *pyb = py + (long)b * S1 * T;
@@ -330,17 +415,16 @@ __global__ void __launch_bounds__(256)
 // Row sums rx, ry (one wave per lattice row; rx over all T1 columns) and column sums
 // cy = sum_s gy, G = sum_s (gx + gy) over the frames (64 frames per block, waves split
 // the rows, eight of a wave's requested together); also the gradients of the joint inputs,
-// k * (gx, gy), where gxj and gyj are given.
+// k * (gx, gy).
 // t_masks (optional): per utterance the frame whose px the forward kernel set to -inf for
 // the regular lattice; like the reference's scatter_ there (rnnt_loss.py:45-63) that cuts
 // the gradient, whatever the recursion left in px_grad at those cells (1 when no path
-// exists at all, 0 otherwise).  score_grad (optional): gpx and gpy are taken times
-// scale * score_grad[b * stride].
+// exists at all, 0 otherwise).
 template <typename R>
 __global__ void __launch_bounds__(256)
     smoothed_bwd_sums_kernel(const R *__restrict__ gpx, const R *__restrict__ gpy,
-                             const int64_t *__restrict__ boundary, const R *__restrict__ score_grad,
-                             int stride, R scale, R *__restrict__ gxj, R *__restrict__ gyj,
+                             const int64_t *__restrict__ boundary, R *__restrict__ gxj,
+                             R *__restrict__ gyj,
                              R *__restrict__ row_x, R *__restrict__ row_y, R *__restrict__ col_y,
                              R *__restrict__ col_g, int B, int S, int T, int T1, R k_joint) {
   __shared__ R part[2][4][kWave];
@@ -353,20 +437,19 @@ __global__ void __launch_bounds__(256)
     if (row >= n_rows) return;
     const int b = (int)(row / S1), s = (int)(row % S1);
     const int t_mask = boundary ? (int)boundary[4 * b + 3] : -1;
-    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
     R sx = 0, sy = 0;
     if (s < S) {
       const long o = ((long)b * S + s) * T1;
       for (int t = lane; t < T1; t += kWave) {
-        const R v = t == t_mask ? (R)0 : gpx[o + t] * g;
-        if (gxj) gxj[o + t] = v * k_joint;
+        const R v = t == t_mask ? (R)0 : gpx[o + t];
+        gxj[o + t] = v * k_joint;
         sx += v;
       }
     }
     const long o = row * T;
     for (int t = lane; t < T; t += kWave) {
-      const R v = gpy[o + t] * g;
-      if (gyj) gyj[o + t] = v * k_joint;
+      const R v = gpy[o + t];
+      gyj[o + t] = v * k_joint;
       sy += v;
     }
     sx = wave_total(sx);
@@ -381,7 +464,6 @@ __global__ void __launch_bounds__(256)
     const int b = (int)(cb / tiles), t = (int)(cb % tiles) * kWave + lane;
     const bool ok = t < T;
     const bool masked = boundary && boundary[4 * b + 3] == t;
-    const R g = score_grad ? scale * score_grad[(long)b * stride] : (R)1;
     R ax = 0, ay = 0;
     constexpr int kAhead = 8;
     for (int s0 = wave; s0 < S1; s0 += 4 * kAhead) {
@@ -395,8 +477,8 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
         const int s = s0 + 4 * u;
-        if (s < S1) ay += y[u] * g;
-        if (s < S && !masked) ax += x[u] * g;
+        if (s < S1) ay += y[u];
+        if (s < S && !masked) ax += x[u];
       }
     }
     part[0][wave][lane] = ax;
@@ -409,6 +491,71 @@ __global__ void __launch_bounds__(256)
       col_g[(long)b * T + t] = x + y;
     }
   }
+}
+
+// G[b,t] = sum_s (gx + gy) of the scaled gradients, for the fused loss: 64 frames per block, eight waves
+// of which take every eighth lattice row of the window, eight of them requested together (B 32, S 80,
+// T 250: 4.1 us; 6.0 with the row sums, which the preparation of the products forms anyway, beside them).
+constexpr int kFrameSumWaves = 8;
+__global__ void __launch_bounds__(kFrameSumWaves *kWave)
+    frame_sums_kernel(const float *__restrict__ gpx, const float *__restrict__ gpy,
+                      const int64_t *__restrict__ boundary, const float *__restrict__ score_grad,
+                      int stride, float scale, float *__restrict__ col_g, int S, int T, int T1) {
+  __shared__ float part[kFrameSumWaves][kWave];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y, t = (int)blockIdx.x * kWave + lane, S1 = S + 1;
+  const Limits lim = limits_of(boundary, b, S, T);
+  const bool in = t >= lim.t_begin && t < lim.t_end;
+  const bool masked = T1 > T && boundary && boundary[4 * b + 3] == t;
+  const __amdgpu_buffer_rsrc_t gx_rs = buffer_of(gpx + (long)b * S * T1, S * T1 * 4);
+  const __amdgpu_buffer_rsrc_t gy_rs = buffer_of(gpy + (long)b * S1 * T, S1 * T * 4);
+  constexpr int kAhead = 8;
+  float sum = 0.f;
+  for (int s0 = lim.s_begin + wave; s0 <= lim.s_end; s0 += kFrameSumWaves * kAhead) {
+    float x[kAhead], y[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int s = s0 + kFrameSumWaves * u;  // (row S of px lies past the resource)
+      x[u] = get_float(gx_rs, in && !masked && s <= lim.s_end, 4 * t, s * T1 * 4);
+      y[u] = get_float(gy_rs, in && s <= lim.s_end, 4 * t, s * T * 4);
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) sum += x[u] + y[u];
+  }
+  part[wave][lane] = sum;
+  __syncthreads();
+  if (wave == 0 && t < T) {
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kFrameSumWaves; ++w) total += part[w][lane];
+    col_g[(long)b * T + t] = total * (scale * score_grad[(long)b * stride]);
+  }
+}
+// sum_c softmax(lm)[row][c] gU[c], a wave per row
+__global__ void __launch_bounds__(256)
+    lm_dot_kernel(const float *__restrict__ lm, const float *__restrict__ lm_max,
+                  const float *__restrict__ lm_sum, const float *__restrict__ g_unigram,
+                  float *__restrict__ dot_out, long rows, int C) {
+  constexpr int kAhead = 8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row = (long)blockIdx.x * 4 + wave;
+  if (row >= rows) return;
+  const float *x = lm + row * C;
+  const float m = lm_max[row], inv = 1.f / lm_sum[row];
+  float dot = 0.f;
+  for (int c0 = 0; c0 < C; c0 += kAhead * kWave) {
+    float v[kAhead], g[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int c = min(c0 + u * kWave + lane, C - 1);
+      v[u] = x[c], g[u] = g_unigram[c];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (c0 + u * kWave + lane < C) dot += __expf(v[u] - m) * inv * g[u];
+  }
+  dot = wave_total(dot);
+  if (lane == 0) dot_out[row] = dot;
 }
 
 // gU[c] = a (sum_{(b,s): sym=c} rx + [c=term] sum ry) / U[c] - a sum of the partials,
@@ -628,7 +775,7 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
              const R *pxj, const R *pyj, R *px,
              R *py, R *lm_max, R *lm_sum, R *am_max, R *am_z, R *unigram, R *partial, int B, int S,
              int T, int C, int term, int regular, double lm_only_scale, double am_only_scale,
-             void *stream_, double delay_penalty = 0.0, const int64_t *ends = nullptr) {
+             void *stream_) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "smoothed_logprobs_fwd: bad size");
   if (term < 0 || term >= C)
     return fail(FRNNT_EINVAL, "smoothed_logprobs_fwd: termination symbol outside [0, C)");
@@ -661,12 +808,11 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
                        dim3((unsigned)((T1 + kCombineFrames - 1) / kCombineFrames), (unsigned)B),
                        dim3(256), tile_lds, stream, lm, am, symbols, boundary, pxj, pyj, lm_max,
                        lm_sum, am_max, am_z, unigram, px, py, S, T, C, term, regular, k_joint, k_lm,
-                       k_am, Delay<R>{(R)delay_penalty}, ends);
+                       k_am);
   else if (total > 0)
     hipLaunchKernelGGL(smoothed_combine_kernel<R>, dim3((unsigned)((total + 255) / 256)),
                        dim3(256), 0, stream, lm, am, symbols, boundary, pxj, pyj, lm_max, lm_sum, am_max,
-                       am_z, unigram, px, py, B, S, T, C, term, regular, k_joint, k_lm, k_am,
-                       Delay<R>{(R)delay_penalty}, ends);
+                       am_z, unigram, px, py, B, S, T, C, term, regular, k_joint, k_lm, k_am);
   return check_launch("smoothed_logprobs_fwd");
 }
 
@@ -693,7 +839,7 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   const int64_t *t_masks = regular ? boundary : nullptr;
   const long sums_blocks = (n_lm + 3) / 4 + (long)B * ((T + kWave - 1) / kWave);
   hipLaunchKernelGGL(smoothed_bwd_sums_kernel<R>, dim3((unsigned)sums_blocks), dim3(256), 0, stream,
-                     px_grad, py_grad, t_masks, (const R *)nullptr, 0, (R)1, pxj_grad, pyj_grad, row_x,
+                     px_grad, py_grad, t_masks, pxj_grad, pyj_grad, row_x,
                      row_y, col_y, col_g, B, S, T, T1, k_joint);
   const int blocks = (int)((n_am + kRowsPerBlock - 1) / kRowsPerBlock);
   if (n_am > 0)
@@ -732,6 +878,11 @@ struct Kept {
   float *lm_max, *s_lm_max, *lm_sum, *am_max, *s_am_max, *am_z, *unigram, *norm_raw;
   size_t floats;
 };
+// Whether a scale asks for an am-only model.  The reference takes 1e-20 in place of 0 (rnnt_loss.py:1346-1351)
+// to keep 0 * -inf out of px: such a model's terms are below 1e-16, next to log-probabilities and
+// gradients of which a unit in the last place is more than that wherever they count, and neither its
+// statistics nor its gradients are formed.
+bool has_am_model(double am_only_scale) { return fabs(am_only_scale) > 1e-19; }
 Kept keep_of(float *base, long B, long S, long T, long C) {
   size_t at = 0;
   auto take = [&](size_t n) {
@@ -818,16 +969,30 @@ int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t 
   if (rnnt_type != kRegular && rnnt_type != kModified)
     return fail(FRNNT_EINVAL, "smoothed_loss_fwd: rnnt_type must be 0 or 1");
   if (B > 0 && !kept) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: null pointer");
+  if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: bad size");
+  if (B > 0 && (!lm || !partial || (!am && T > 0))) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: null pointer");
   const int regular = rnnt_type == kRegular;
   const Kept k = keep_of(kept, B, S, T, C);
-  int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px_joint, py_joint, k.lm_max, k.am_max,
-                               k.norm_raw, 0.0, B, S, T, C, termination_symbol, rnnt_type,
-                               boundary != nullptr, stream);
-  if (rc != FRNNT_OK) return rc;
-  rc = fwd_impl<float>(lm, am, symbols, boundary, px_joint, py_joint, px, py, k.s_lm_max, k.lm_sum,
-                       k.s_am_max, k.am_z, k.unigram, partial, B, S, T, C, termination_symbol,
-                       regular, lm_only_scale, am_only_scale, stream,
-                       delay_penalty > 0.0 ? delay_penalty : 0.0, boundary);
+  hipStream_t on = static_cast<hipStream_t>(stream);
+  const bool am_model = has_am_model(am_only_scale);
+  const long n_lm = (long)B * (S + 1), n_am = (long)B * T;
+  const int blocks = (int)((n_lm + kRowsPerBlock - 1) / kRowsPerBlock);
+  if (B > 0)
+    hipLaunchKernelGGL((am_model ? lm_models_kernel<true> : lm_models_kernel<false>), dim3(blocks),
+                       dim3(kRowsPerBlock * kWave), 0, on, lm, k.s_lm_max, k.lm_sum, partial, n_lm, C);
+  if (B > 0 && am_model) {
+    hipLaunchKernelGGL(unigram_final_kernel<float>, dim3((C + kColsPerBlock - 1) / kColsPerBlock),
+                       dim3(kUnigramThreads), 0, on, partial, k.unigram, blocks, n_lm, C);
+    if (n_am > 0)
+      hipLaunchKernelGGL(am_model_kernel, dim3((unsigned)((n_am + 3) / 4)), dim3(256), 0, on, am,
+                         k.unigram, k.s_am_max, k.am_z, n_am, C);
+  }
+  const SmoothMix mix{k.s_lm_max, k.lm_sum, k.s_am_max, k.am_z, k.unigram, partial, k.unigram,
+                      (float)(1.0 - lm_only_scale - am_only_scale), (float)lm_only_scale,
+                      am_model ? (float)am_only_scale : 0.f, blocks};
+  const int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, k.lm_max, k.am_max, k.norm_raw,
+                                     delay_penalty > 0.0 ? delay_penalty : 0.0, B, S, T, C,
+                                     termination_symbol, rnnt_type, boundary != nullptr, stream, &mix);
   if (rc != FRNNT_OK) return rc;
   return frnnt_mi_loss_fwd_f32(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, !regular,
                                reduction, checks, status, stream);
@@ -854,36 +1019,40 @@ int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t 
   const long n_lm = (long)B * (S + 1), n_am = (long)B * T;
   const float k_lm = (float)lm_only_scale, k_am = (float)am_only_scale;
   const float k_joint = (float)(1.0 - lm_only_scale - am_only_scale);
-  // scratch: the sums of the unscaled gradients first, the joint model's buffers after them
   size_t at = 0;
   auto take = [&](size_t n) {
     float *q = scratch + at;
     at += (n + 3) & ~(size_t)3;
     return q;
   };
-  float *row_x = take(n_lm), *row_y = take(n_lm), *col_y = take(n_am), *col_g = take(n_am);
-  float *g_unigram = take(C), *partial = take((n_am + 15) / 16 * C);
-  float *dmat = take(n_lm * ((T + 3) & ~3)), *joint_x = take(n_lm), *joint_y = take(n_lm);
-  hipLaunchKernelGGL(smoothed_bwd_sums_kernel<float>,
-                     dim3((unsigned)((n_lm + 3) / 4 + (long)B * ((T + kWave - 1) / kWave))), dim3(256), 0,
-                     stream, px_grad, py_grad, regular ? boundary : nullptr, score_grad,
-                     score_grad_stride, (float)score_grad_scale, nullptr, nullptr, row_x, row_y,
-                     col_y, col_g, B, S, T, T1, k_joint);
+  float *row_x = take(n_lm), *row_y = take(n_lm), *dot = take(n_lm), *col_g = take(n_am);
+  float *g_unigram = take(C), *partial = take((n_am + 15) / 16 * C), *dmat = take(n_lm * ((T + 3) & ~3));
+  const bool am_model = has_am_model(am_only_scale);
   const int blocks = (int)((n_am + kRowsPerBlock - 1) / kRowsPerBlock);
-  if (n_am > 0)
-    hipLaunchKernelGGL(weighted_column_partial_kernel<float>, dim3(blocks), dim3(256), 0, stream, am,
-                       k.s_am_max, col_g, k.am_z, partial, n_am, C);
-  hipLaunchKernelGGL(unigram_grad_kernel<float>, dim3((C + kColsPerBlock - 1) / kColsPerBlock),
-                     dim3(kUnigramThreads), 0, stream, partial, symbols, row_x, row_y, k.unigram,
-                     g_unigram, n_am > 0 ? blocks : 0, B, S, C, termination_symbol, k_am);
-  hipLaunchKernelGGL(smoothed_bwd_lm_kernel<float>, dim3((unsigned)((n_lm + 3) / 4)), dim3(256), 0,
-                     stream, lm, symbols, k.s_lm_max, k.lm_sum, row_x, row_y, g_unigram, lm_grad, n_lm,
-                     S, C, termination_symbol, k_lm, (float)(1.0 / (double)n_lm));
-  const SmoothTerms smooth{col_g, k.am_z, k.unigram, k_am, k_joint + k_am, k_joint};
+  // (of the gradients as they are: the preparation scales them in place)
+  if (am_model && n_am > 0)
+    hipLaunchKernelGGL(frame_sums_kernel, dim3((T + kWave - 1) / kWave, B),
+                       dim3(kFrameSumWaves * kWave), 0, stream, px_grad, py_grad, boundary, score_grad,
+                       score_grad_stride, (float)score_grad_scale, col_g, S, T, T1);
+  const SmoothTerms smooth{col_g,     k.am_z, k.unigram,
+                           k.s_lm_max, k.lm_sum, dot,
+                           g_unigram, am_model ? k_am : 0.f, k_joint + k_am,
+                           k_joint,   k_lm,   (float)(1.0 / (double)n_lm)};
+  const auto am_model_terms = [&] {
+    if (!am_model) return;
+    if (n_am > 0)
+      hipLaunchKernelGGL(weighted_column_partial_kernel<float>, dim3(blocks), dim3(256), 0, stream, am,
+                         k.s_am_max, col_g, k.am_z, partial, n_am, C);
+    hipLaunchKernelGGL(unigram_grad_kernel<float>, dim3((C + kColsPerBlock - 1) / kColsPerBlock),
+                       dim3(kUnigramThreads), 0, stream, partial, symbols, row_x, row_y, k.unigram,
+                       g_unigram, n_am > 0 ? blocks : 0, B, S, C, termination_symbol, k_am);
+    hipLaunchKernelGGL(lm_dot_kernel, dim3((unsigned)((n_lm + 3) / 4)), dim3(256), 0, stream, lm,
+                       k.s_lm_max, k.lm_sum, g_unigram, dot, n_lm, C);
+  };
   return simple_logprobs_bwd_smoothed(lm, am, symbols, boundary, k.lm_max, k.am_max, k.norm_raw,
                                       score_grad, score_grad_stride, score_grad_scale, px_grad,
-                                      py_grad, dmat, joint_x, joint_y, smooth, lm_grad, am_grad, B, S,
-                                      T, C, termination_symbol, rnnt_type, stream_);
+                                      py_grad, dmat, row_x, row_y, smooth, am_model_terms, lm_grad,
+                                      am_grad, B, S, T, C, termination_symbol, rnnt_type, stream_);
 }
 
 }  // extern "C"

@@ -669,7 +669,7 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
     Tensor kept = at::empty({frnnt_smoothed_loss_kept((int)B, (int)S, (int)T, (int)C)}, opts);
     const int64_t n_px = B * S * T1, n_py = B * (S + 1) * T;
     Carver carve;
-    const int64_t o_jx = carve.take(n_px), o_jy = carve.take(n_py), o_px = carve.take(n_px),
+    const int64_t o_px = carve.take(n_px),
                   o_py = carve.take(n_py), o_p = carve.take(B * (S + 1) * (T + 1)),
                   o_sc = carve.take(B), o_part = carve.take((B * (S + 1) + 15) / 16 * C);
     const Tensor work = at::empty({carve.total}, opts);
@@ -681,7 +681,7 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
     }
     Tensor loss = reduction == kRedNone ? at::empty({B}, opts) : at::empty({}, opts);
     check_rc(frnnt_smoothed_loss_fwd_f32(
-                 ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), w + o_jx, w + o_jy, w + o_px,
+                 ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), nullptr, nullptr, w + o_px,
                  w + o_py, ptr<float>(kept), w + o_part, w + o_p, w + o_sc, ptr<float>(gx),
                  ptr<float>(gy), ptr<float>(loss), (int)B, (int)S, (int)T, (int)C, (int)term,
                  (int)kind, lm_scale, am_scale, delay_penalty, (int)reduction, (int)checks,

@@ -281,16 +281,18 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
 
 /*
  * rnnt_loss_smoothed (rnnt_loss.py:1372-1494) in float32 for the regular and the modified lattice
- * (rnnt_type 0, 1): _fwd chains frnnt_simple_logprobs_fwd (window_only when a boundary is
- * given), frnnt_smoothed_logprobs_fwd, the delay penalty and frnnt_mi_loss_fwd; _bwd scales px_grad
+ * (rnnt_type 0, 1): _fwd forms the statistics of the two unigram models, then px and py,
+ * interpolated and with the delay penalty, as frnnt_simple_logprobs_fwd does (window_only when a boundary
+ * is given), and chains frnnt_mi_loss_fwd; an am_only_scale below 1e-19 (the reference's 1e-20 for 0)
+ * means no am-only model.  _bwd scales px_grad
  * and py_grad in place as frnnt_simple_logprobs_bwd does (score_grad is required) and forms the
- * whole lm_grad and am_grad: the am-only model's terms inside the joint model's gradient
- * product, the lm-only model's beneath it.
+ * whole lm_grad and am_grad: the terms of both unigram models inside the joint model's gradient
+ * products.
  *   kept: frnnt_smoothed_loss_kept() floats, written by _fwd for _bwd
- *   px_joint, py_joint, px, py, p, scores: as in those entry points, not needed afterwards
+ *   px, py, p, scores: as in those entry points, not needed afterwards; px_joint, py_joint: not used
  *   partial [ceil(B*(S+1)/16)][C]: scratch
  *   scratch of _bwd: B (S+1) (4 + T rounded up to 4) + 2 B T + C + ceil(B*T/16) C floats, each
- *     of its nine parts rounded up to 4 (40 more are enough for that)
+ *     of its seven parts rounded up to 4 (40 more are enough for that)
  */
 int64_t frnnt_smoothed_loss_kept(int B, int S, int T, int C);
 int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t *symbols,
