@@ -203,6 +203,14 @@ int mi_backward_and_loss(const float *px, const int64_t *boundary, const float *
 int mi_backward_and_loss(const double *px, const int64_t *boundary, const double *p,
                          double *px_grad, double *py_grad, const double *scores, double *loss,
                          int B, int S, int T, int modified, int reduction, void *stream);
+// The same pair where nobody wants p: `shares`, of p's size, is scratch between the two.
+// Host side, mi_shares_forward.hip and mi_shares_backward.hip.
+int mi_forward_shares(const float *px, const float *py, const int64_t *boundary, float *shares,
+                      float *scores, int B, int S, int T, int modified, int checks, int32_t *status,
+                      float *px_grad, float *py_grad, void *stream);
+int mi_backward_shares(const int64_t *boundary, const float *shares, float *px_grad, float *py_grad,
+                       const float *scores, float *loss, int B, int S, int T, int modified,
+                       int reduction, void *stream);
 
 // ((T_b - 1) / 2 - t) * delay_penalty, what rnnt_loss.py:309-324 adds to px, rounded as there.
 template <typename R>

@@ -75,6 +75,22 @@ constexpr int kBwdStagersFew = 7;
 // code there has no scalar registers left, B 64, S 120, T 600: 37 -> 41 us.)
 template <typename R>
 constexpr int kFetchAhead = sizeof(R) == 4 ? 2 : 1;
+// The kernels that pass shares (kShares) deal a sweep wave's tiles out to two groups of its staging waves in
+// turn.  A wave's time per tile is mostly latency -- the look at the counter, the way through LDS, its own
+// count -- and hardly shrinks with its rows: 2 000 - 2 600 cycles with five rows a lane (backward) and 2 800
+// with eight (forward), where a sweep wave needs 1 200 and 2 400 for a tile.  All waves on every tile,
+// forward: B 64, S 120, T 600 39.5 us instead of 34.6; backward, B 12, S 220, T 1500: 69 instead of 50.
+// With as much time for a tile, inputs requested one tile ahead of a wave's next are enough; two sets of
+// registers cost more in code to fetch at the start (1 000 - 2 400 cycles) than they give.
+template <int kStagers, bool kShares>
+constexpr int kStagerGroups = kShares && kStagers % 2 == 0 ? 2 : 1;
+
+// Staging waves per sweep wave there, with at most two sweep waves, and waves of a backward workgroup that do what
+// is on nobody's way: the zeros around the window and the loss.  (By the staging waves, between two tiles, they
+// held up the sweep for 2 600 - 12 700 cycles.)
+constexpr int kSharesStagers = 6;
+template <int kSweepCap, bool kShares>
+constexpr int kHelpers = kShares && kSweepCap <= 2 ? 2 : 0;
 constexpr int kSpinLimit = 1 << 22;   // polls before a wait gives up (seconds, not microseconds)
 struct Window {
   int s0, t0, ns, nt;  // origin and extent (ns = s_end - s_begin, ...)
@@ -269,6 +285,14 @@ __device__ __forceinline__ void push_half(R *dst, const R (&src)[kChunk]) {
   }
 }
 
+// Two values to neighbouring elements, in one LDS write (the address is a multiple of two elements).
+template <typename R>
+__device__ __forceinline__ void push_two(R *dst, R a, R b) {
+  typedef R Pair __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<Pair *>(dst) = Pair{a, b};
+}
+static_assert(kTilePitch >= kTileSteps + 2 && kTilePitch % 2 == 0, "no room in front of a tile's rows");
+
 // Keeps the registers of a half chunk that has just been written to LDS from being given
 // to the next results at once (see push_half): called four steps later, it makes them
 // count as still in use until then.  Emits no instruction.
@@ -283,9 +307,12 @@ struct Counters {
   int failed;                             // set by a wave whose bounded wait ran out
   int ready[kMaxSweep];                   // seam columns published by sweep wave w
   int written[kMaxSweep];                 // tiles whose results sweep wave w has left in LDS
+  // (forward, kShares) per sweep wave and tile buffer, as in `loaded`: how many times a staging wave has taken a
+  // tile's results out of it
+  int taken[16];
   // per sweep wave w and tile buffer k (index w * buffers + k): how many times a staging
-  // wave has finished staging a tile into that buffer, all of w's staging waves and all
-  // tiles together -- the buffer's n-th tile is complete at n * stagers.  One counter for
+  // wave has finished staging a tile into that buffer, all of the waves that stage it and all
+  // tiles together -- the buffer's n-th tile is complete at n * those.  One counter for
   // all staging waves: a sweep wave pays for every test it makes.
   int loaded[16];
 };
@@ -381,6 +408,20 @@ __device__ __forceinline__ bool send_seam(double *, int, int, const double *, co
   return false;
 }
 
+// The word of the share d1 of a cell that passes nothing on, in LDS: the largest finite number, which all
+// that is not finite (mutual_information_cpu.cu:203-206: such a cell has no shares) or negative (no cell
+// of the window's) becomes.  And the bit of Counters::loaded for a buffer that has held such a cell.
+constexpr unsigned kNoShares = 0x7f7fffff;
+constexpr int kNoSharesHere = 1 << 30;
+// Where p of lattice row s, the last of a band, passes to the next band if p itself is not stored: T + 1
+// elements from row s of py_grad on, which nothing else uses before the backward kernel writes all of
+// it.  (The element past the row's end is the first of the row after it, which exists and is no band's
+// last.)
+template <typename R>
+__device__ __forceinline__ R *mail_row(R *py_grad, int b, int s, int S, int T) {
+  return py_grad + ((size_t)b * (S + 1) + s) * T;
+}
+
 // A word that any of an utterance's workgroups may make NaN (a wait of theirs ran out) and that the
 // last one gives its value: the value replaces what the word held before the launch and nothing
 // else, the NaN replaces anything.  Whichever comes first, the NaN stays.
@@ -395,20 +436,23 @@ __device__ __forceinline__ void store_once(float *word, int before, float value)
                                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The marks of an utterance's seam rows: in p (which may be NULL) where rows s0 + 63, s0 + 127, ...
-// of the window feed the next one, in px_grad (which may be NULL) where the reversed rows do; and,
-// with p, the utterance's score (see store_once).  A block per utterance and seam.
+// The marks of an utterance's seam rows: in p or, with `mail`, in the rows that stand for p's (mail_row;
+// both may be NULL) where rows s0 + 63, s0 + 127, ... of the window feed the next one, in px_grad (which
+// may be NULL) where the reversed rows do; and, with p or mail, the utterance's score (see store_once).
+// A block per utterance and seam.
 __global__ void __launch_bounds__(256)
-    mark_seams_kernel(const int64_t *__restrict__ boundary, float *__restrict__ p,
+    mark_seams_kernel(const int64_t *__restrict__ boundary, float *__restrict__ p, float *__restrict__ mail,
                       float *__restrict__ ans, float *__restrict__ px_grad, int S, int T,
                       int modified) {
   const int b = blockIdx.x, last = (int)blockIdx.y * kWave + kWave - 1;  // (row, or reversed row)
-  if (p && blockIdx.y == 0 && threadIdx.x == 0) ans[b] = __int_as_float(kSeamMark);
+  if ((p || mail) && blockIdx.y == 0 && threadIdx.x == 0) ans[b] = __int_as_float(kSeamMark);
   const Window win = load_window(boundary, b, S, T);
   if (!win.ok || last + 1 > win.ns) return;
   const float mark = __int_as_float(kSeamMark);
-  if (p) {
-    int *row = reinterpret_cast<int *>(p + ((size_t)b * (S + 1) + win.s0 + last) * (T + 1) + win.t0);
+  if (p || mail) {
+    int *row = reinterpret_cast<int *>((mail ? mail_row(mail, b, win.s0 + last, S, T)
+                                             : p + ((size_t)b * (S + 1) + win.s0 + last) * (T + 1)) +
+                                       win.t0);
     for (int j = threadIdx.x; j <= win.nt; j += 256) row[j] = __float_as_int(mark);
   }
   if (px_grad) {
@@ -423,16 +467,18 @@ __global__ void __launch_bounds__(256)
 // y = py feeding it from the left; -inf where that edge does not exist, and
 // y = 0 at the origin cell so that the chain produces p = 0 there.
 // A sweep wave only runs the chain: it takes a tile's x / y from an LDS buffer and
-// leaves the tile's p in the place of x (16 bytes per LDS write); the staging waves
+// leaves the tile's p in the place of y (16 bytes per LDS write); the staging waves
 // carry p to memory, each for the rows it stages, before they refill the buffer.
 // kSweepCap: most sweep waves the launch may use; it only sets the register budget.
 // kApart: a workgroup per band; `pitch` workgroups per band, one per utterance (of B).
-template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart>
+// kShares: what a cell hands down of its gradient, d1 = exp(term1 - p), is stored in the place of p (see
+// the backward kernel); the seams of workgroups apart then go through `mail` (see mail_row).
+template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart, bool kShares>
 __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)) * kWave)
     mi_forward_kernel(const R *__restrict__ px, const R *__restrict__ py,
                       const int64_t *__restrict__ boundary, R *__restrict__ p,
                       R *__restrict__ ans, int S, int T, int spin_limit, int checks,
-                      int *__restrict__ status, int B, int pitch) {
+                      int *__restrict__ status, int B, int pitch, R *mail) {
   // (lattices of one band -- a cap of one sweep wave -- have no seams)
   constexpr bool kSeams = kApart || kSweepCap > 1;
   extern __shared__ __align__(16) unsigned char dyn_lds[];
@@ -495,31 +541,37 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     }
   };
 
+  // (apart) where p of the window's row i passes from one workgroup to the next
+  auto seam_row = [&](int i) -> R * {
+    return kShares ? mail_row(mail, b, win.s0 + i, S, T) + win.t0 : pb + (size_t)(win.s0 + i) * TP + win.t0;
+  };
   if (kApart && wave >= 1 + kStagers) {
     // ------------------------------- courier waves -------------------------------
     if (wave == 1 + kStagers) {
       const int next = (part + 1) * kWave;
-      if (next <= NS && !send_seam(pb + (size_t)(win.s0 + next - 1) * TP + win.t0, 1, cols,
-                                   seam + seam_pitch, &cnt.ready[1], lane, spin_limit))
+      if (next <= NS && !send_seam(seam_row(next - 1), 1, cols, seam + seam_pitch, &cnt.ready[1], lane,
+                                   spin_limit))
         give_up();
       return;
     }
-    if (part > 0 && !bring_seam(pb + (size_t)(win.s0 + part * kWave - 1) * TP + win.t0, 1, cols, seam,
-                                &cnt.ready[0], lane, spin_limit))
+    if (part > 0 &&
+        !bring_seam(seam_row(part * kWave - 1), 1, cols, seam, &cnt.ready[0], lane, spin_limit))
       give_up();
     return;
   }
   if (wave >= nsweep) {
     // ------------------------------ staging wave -------------------------------
-    const int w = (wave - nsweep) / kStagers, l = (wave - nsweep) % kStagers;
+    constexpr int kGroups = kStagerGroups<kStagers, kShares>, kPer = kStagers / kGroups;
+    const int w = (wave - nsweep) / kStagers, l = (wave - nsweep) % kPer;
+    const int group = (wave - nsweep) % kStagers / kPer;  // which of the tiles m = group, group + kGroups, ...
     const int prev = (w + nsweep - 1) % nsweep;
     const R *up_seam = seam + (size_t)prev * seam_pitch;
     R *my_seam = seam + (size_t)(kApart ? 1 : w) * seam_pitch;
     R *base = tiles + (size_t)w * 2 * kBuffers * kTileElems;
     const int half = lane >> 5, q = lane & 31;
-    // rows of a tile this wave stages: r(u) = 2*l + half + 2*kStagers*u
-    constexpr int kRows = (kWave + 2 * kStagers - 1) / (2 * kStagers);
-    constexpr int kAhead = kFetchAhead<R>;
+    // rows of a tile this wave stages: r(u) = 2*l + half + 2*kPer*u
+    constexpr int kRows = (kWave + 2 * kPer - 1) / (2 * kPer);
+    constexpr int kAhead = kShares ? 1 : kFetchAhead<R>;
     struct Staged {
       R x[kRows], y[kRows];
     };
@@ -532,7 +584,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     const __amdgpu_buffer_rsrc_t py_rsrc = buffer_of(const_cast<R *>(pyb), (size_t)(S + 1) * T);
     // (what is stored: the rows of the window, so that a row beyond them is outside the resource)
     const __amdgpu_buffer_rsrc_t p_rsrc = buffer_of(pb + (size_t)win.s0 * TP, (size_t)(NS + 1) * TP);
-    constexpr int kStep = 2 * kStagers;
+    constexpr int kStep = 2 * kPer;
     constexpr int kSize = (int)sizeof(R);
     const int r_first = 2 * l + half;
     auto fetch = [&](Staged &in, const Band &g, int m) {
@@ -551,8 +603,11 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     // element (row r, step q) is the cell (row0 + r, 32 pm + q - r) of the window.  Taking
     // it out of the buffer and storing it are two steps: the stores of a tile go out after
     // the buffer has been refilled and handed back to the sweep wave, not before.
+    // (kShares: and what the cell below had and the edge between the two, for the share of the cell's
+    // gradient that goes down.  That cell's p is one step back (modified: two) in the row below; the
+    // last steps of the tile before lie in front of each row, where the sweep wave has left them.)
     struct Drained {
-      R v[kRows];
+      R v[kRows], below[kShares ? kRows : 1], x[kShares ? kRows : 1];
       int row0, pm;
     };
     constexpr int kNowhere = -(1 << 20);  // (a tile with no cell in the window)
@@ -563,34 +618,67 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       for (int u = 0; u < kRows; ++u) put1(u & 1 ? py_rsrc : px_rsrc, kDropped + u * kSize, (R)0);
     };
     auto take = [&](Drained &d, int row0, int pm, int buf) {
-      const R *ps = base + buf * kTileElems + r_first * kTilePitch + q;
+      const R *xs = base + buf * kTileElems + r_first * kTilePitch + q;
+      const R *ps = xs + kBuffers * kTileElems;
       d.row0 = row0;
       d.pm = pm;
 #pragma unroll
       for (int u = 0; u < kRows; ++u) {
         if (r_first + kStep * u >= kWave) continue;
         d.v[u] = ps[u * kStep * kTilePitch];
+        if constexpr (kShares) {
+          d.below[u] = ps[(u * kStep - 1) * kTilePitch - 1 - shift];  // (row 0: not a cell's, replaced below)
+          d.x[u] = xs[u * kStep * kTilePitch];
+        }
       }
     };
     // The tile's last row, for the sweep wave below (one staging wave holds it): to the seam row, as
     // soon as the tile is done.
-    constexpr int kLastL = (kWave / 2 - 1) % kStagers, kLastU = (kWave / 2 - 1) / kStagers;
-    auto hand_on = [&](const Drained &d) {
-      if (!kSeams || l != kLastL || d.row0 + kWave > NS) return;  // (wave-uniform)
+    constexpr int kLastL = (kWave / 2 - 1) % kPer, kLastU = (kWave / 2 - 1) / kPer;
+    auto hand_on = [&](const Drained &d) -> bool {
+      if (!kSeams || l != kLastL || d.row0 + kWave > NS) return true;  // (wave-uniform)
       const int col = d.pm * kTileSteps + q - (kWave - 1);
       if (half == 1 && (unsigned)col <= (unsigned)NT) my_seam[col] = d.v[kLastU];
       const int done = max(0, min(d.pm * kTileSteps + kTileSteps - (kWave - 1), cols));
       const int before = kApart ? 0 : (d.row0 / kWave - w) / nsweep * cols;
-      if (lane == 0) publish_lds_writes(&cnt.ready[kApart ? 1 : w], before + done);
+      int *ready = &cnt.ready[kApart ? 1 : w];
+      // The tile before may be the other group's, which counts its columns in first.  (A tile without
+      // columns counts nothing: that could come after, and would take back, what a later tile has counted.)
+      if (kGroups > 1) {
+        const int already = max(0, min(d.pm * kTileSteps - (kWave - 1), cols));
+        if (done == already) return true;
+        if (!wait_for(ready, before + already, spin_limit)) return false;
+      }
+      if (lane == 0) publish_lds_writes(ready, before + done);
+      return true;
     };
     auto store = [&](const Drained &d) {
       const int i0 = d.row0 + r_first;
       const int j0 = d.pm * kTileSteps + q - r_first;
       const int o0 = (i0 * TP + win.t0 + j0) * kSize;
+      R out[kRows];
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        out[u] = d.v[u];
+        if constexpr (kShares) {
+          // mutual_information_cpu.cu:196-212.  A band's first row has what comes from below in its x.
+          const R below = u == 0 && r_first == 0 ? (R)0 : d.below[u];
+          R total = d.v[u];
+          if (total - total != 0) total = 0;
+          out[u] = Num<R>::exp_(below + d.x[u] - total);
+        }
+      }
+      if constexpr (kShares) {
+        // column 0 hands everything down (:219-226), in the modified lattice nothing
+        if (d.pm * kTileSteps < kWave)
+#pragma unroll
+          for (int u = 0; u < kRows; ++u)
+            if (j0 == kStep * u) out[u] = kModified ? (R)0 : (R)1;
+      }
 #pragma unroll
       for (int u = 0; u < kRows; ++u) {
         const bool ok = (unsigned)(j0 - kStep * u) <= (unsigned)NT && r_first + kStep * u < kWave;
-        put1(p_rsrc, ok ? o0 + u * (kStep * (TP - 1) * kSize) : kDropped, d.v[u]);
+        put1(p_rsrc, ok ? o0 + u * (kStep * (TP - 1) * kSize) : kDropped, out[u]);
       }
     };
     // The tile that a buffer held before tile m of the band that starts at row0.  Bands that
@@ -605,7 +693,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       }
       take(d, row0, pm, buf);
     };
-    int tile_base = 0, buf = 0;  // buf = tile number modulo kBuffers
+    int tile_base = 0;
     int end_row0 = 0, end_tiles = 0;
     for (int band = part; band * band_rows <= last_row; ++band) {
       const Band g = band_of(band, w, nsweep, NS, NT);
@@ -624,11 +712,11 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       out.pm = kNowhere;
 #pragma unroll
       for (int k = 0; k < kAhead; ++k) {
-        fetch(ahead[k], g, k);
+        fetch(ahead[k], g, group + k * kGroups);
         store_nothing();
       }
       auto stage = [&](const Staged &cur, int m) __attribute__((always_inline)) -> bool {
-        const int gt = tile_base + m;
+        const int gt = tile_base + m, buf = gt % kBuffers;
         if (gt >= kBuffers) {
           // the buffer still holds p of tile gt - kBuffers
           if (!wait_for(&cnt.written[w], gt - kBuffers + 1, spin_limit)) {
@@ -636,7 +724,13 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
             return false;
           }
           take_buffer(out, g.row0, m, buf);
-          hand_on(out);
+          // (kShares: the row below a staging wave's is another one's, who must not refill it before)
+          if (kShares && lane == 0) count_in(&cnt.taken[w * kBuffers + buf]);
+          if (!hand_on(out) ||
+              (kShares && !wait_for(&cnt.taken[w * kBuffers + buf], kPer * (gt / kBuffers), spin_limit))) {
+            give_up();
+            return false;
+          }
         }
         // The row above the band belongs to another sweep wave: what it feeds into the band's first
         // row is added to that row's x here (the sweep would add it with the same rounding), so
@@ -680,18 +774,17 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
         }
         // every lane's LDS writes precede the release by lane 0 of the same wave
         if (lane == 0) count_in(&cnt.loaded[w * kBuffers + buf]);
-        buf = buf + 1 == kBuffers ? 0 : buf + 1;
         return true;
       };
       bool failed = false;
-      for (int m = 0; m < g.ntiles; m += kAhead) {
+      for (int m = group; m < g.ntiles; m += kAhead * kGroups) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
-          if (m + k < g.ntiles && !failed)
-            failed = !stage(ahead[k], m + k);
+          if (m + k * kGroups < g.ntiles && !failed)
+            failed = !stage(ahead[k], m + k * kGroups);
           else
             out.pm = kNowhere;
-          fetch(ahead[k], g, m + k + kAhead);
+          fetch(ahead[k], g, m + (k + kAhead) * kGroups);
           asm volatile("" ::: "memory");
           store(out);
         }
@@ -703,17 +796,19 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     }
     // the tiles still in the buffers
     const int first_left = max(tile_base - kBuffers, 0);
-    buf = first_left % kBuffers;
     for (int gt = first_left; gt < tile_base; ++gt) {
+      if (gt % kGroups != group) continue;
+      Drained out;
       if (!wait_for(&cnt.written[w], gt + 1, spin_limit)) {
         give_up();
         return;
       }
-      Drained out;
-      take_buffer(out, end_row0, gt - tile_base + end_tiles + kBuffers, buf);
-      hand_on(out);
+      take_buffer(out, end_row0, gt - tile_base + end_tiles + kBuffers, gt % kBuffers);
+      if (!hand_on(out)) {
+        give_up();
+        return;
+      }
       store(out);
-      buf = buf + 1 == kBuffers ? 0 : buf + 1;
     }
     return;
   }
@@ -743,16 +838,20 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     auto one_tile = [&](int m, auto plain_c) __attribute__((always_inline)) -> bool {
       constexpr bool kPlain = decltype(plain_c)::value;
       const int gt = tile_base + m;
-      if (__builtin_amdgcn_readfirstlane(seen_loaded) < kStagers * (rounds + 1) &&
-          !wait_for(&cnt.loaded[w * kBuffers + buf], kStagers * (rounds + 1), spin_limit)) {
+      constexpr int kPer = kStagers / kStagerGroups<kStagers, kShares>;
+      if (__builtin_amdgcn_readfirstlane(seen_loaded) < kPer * (rounds + 1) &&
+          !wait_for(&cnt.loaded[w * kBuffers + buf], kPer * (rounds + 1), spin_limit)) {
         give_up();
         return false;
       }
       // this lane's 32 steps of inputs go to registers in one burst
       R xq[kTileSteps], yq[kTileSteps];
-      R *x_row = base + buf * kTileElems + lane * kTilePitch;  // x in, p out
+      const R *x_row = base + buf * kTileElems + lane * kTilePitch;
+      R *y_row = base + (kBuffers + buf) * kTileElems + lane * kTilePitch;  // y in, p out
       pull_row(xq, x_row);
-      pull_row(yq, x_row + kBuffers * kTileElems);
+      pull_row(yq, y_row);
+      // the two steps before the tile's, in the two unused elements in front of the lane's row
+      if constexpr (kShares) push_two(y_row - 2, own2, own);
       buf = buf + 1 == kBuffers ? 0 : buf + 1;
       rounds += buf == 0;
 
@@ -774,8 +873,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
           own2 = own;
           own = v;
           if (k == kChunk / 2 - 1) {
-            // the chunk's p takes the place of its x in the tile: first half
-            push_half<0>(x_row + c4 * kChunk, vals);
+            // the chunk's p takes the place of its y in the tile: first half
+            push_half<0>(y_row + c4 * kChunk, vals);
             still_in_use(last, kChunk / 2);
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -789,7 +888,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
               if (k == kf) fin = vals[k];
           }
         }
-        push_half<1>(x_row + c4 * kChunk, vals);
+        push_half<1>(y_row + c4 * kChunk, vals);
 #pragma unroll
         for (int k = kChunk / 2; k < kChunk; ++k) last[k] = vals[k];
       };
@@ -837,8 +936,15 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
 // tile's d1 / d2 from (a lane's 32 steps, 16 bytes per write), and the staging waves
 // carry them to memory, each for the rows it stages, before they refill the buffer.
 // kApart, pitch: as in the forward kernel.
-template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart>
-__global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)) * kWave)
+// kShares: the forward kernel has left d1 in `p`, borders and all.  The staging waves then only copy it to
+// LDS, a third of the loads and no exp; the sweep wave takes d2 = 1 - d1 itself, off the chain, and leaves
+// the cells' gradients, one value per cell in LDS instead of two; and the staging waves split those as they
+// carry them to memory.  Same operations, same bits.  The forward kernel's staging waves, of which the
+// sweep needs less, do the exp.  Both kernels, from p and px -> with shares: B 12, S 220, T 1500 143 -> 119 us;
+// B 64, S 120, T 600 70.2 -> 61.3; B 32, S 80, T 250 33.8 -> 32.1; B 8, S 60, T 200 25.7 -> 23.5.
+template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart, bool kShares>
+__global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0) +
+                                   kHelpers<kSweepCap, kShares>) * kWave)
     mi_backward_kernel(const R *__restrict__ px, const int64_t *__restrict__ boundary,
                        const R *__restrict__ p, R *ans_grad, R *__restrict__ px_grad,
                        R *__restrict__ py_grad, int S, int T, int overwrite_ans_grad,
@@ -849,7 +955,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
 
   const int b = kApart ? blockIdx.x % pitch : blockIdx.x, part = kApart ? blockIdx.x / pitch : 0;
   if (kApart && b >= B) return;
-  const int nsweep = blockDim.x / (kWave * (1 + kStagers));
+  constexpr int kHelp = kHelpers<kSweepCap, kShares>;
+  const int nsweep = (blockDim.x / kWave - (kApart ? 2 : 0) - kHelp) / (1 + kStagers);
   const int nwaves = blockDim.x / kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // in a scalar register
   const int lane = threadIdx.x % kWave;
@@ -863,47 +970,51 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   const __amdgpu_buffer_rsrc_t gx_rsrc = buffer_of(gxb, (size_t)S * T1);
   const __amdgpu_buffer_rsrc_t gy_rsrc = buffer_of(gyb, (size_t)(S + 1) * T);
 
-  // Exact zeros everywhere the sweep does not write, one wave per row.  The staging
-  // waves do this once they are two tiles ahead of their sweep wave, off the critical
-  // path (a barrier after these stores would have to wait until they have all reached
-  // memory).
-  // elements [begin, end) of the row that starts at element `row` of the resource;
-  // begin and end are wave-uniform
-  auto zero_range = [&](__amdgpu_buffer_rsrc_t rs, int row, int begin, int end) {
-    const int len = end - begin;
-    if (len <= 0) return;
+  // Exact zeros everywhere the sweep does not write, by wave `part` of `parts`, off the critical path (a
+  // barrier after these stores would have to wait until they have all reached memory).  An array's
+  // window leaves a run before it, one after it and, all of one length, those between its rows: four rows'
+  // to an instruction, 16 lanes each (row by row, with a run's ends tested for each, two waves took
+  // longer than the sweep: 24 000 cycles at S 80, T 250, a third of it outside).
+  auto zero_run = [&](__amdgpu_buffer_rsrc_t rs, int begin, int end, int first, int lanes) {
+    // elements [begin, end), by lanes `first` .. of `lanes` that step through it together; overlapping the
+    // last four, so that all stores are whole
     const R z = 0;
-    if (len < 4) {
-      put1(rs, lane < len ? (row + begin + lane) * (int)sizeof(R) : kDropped, z);
+    if (end - begin < 4) {
+      put1(rs, first < end - begin ? (begin + first) * (int)sizeof(R) : kDropped, z);
       return;
     }
-    for (int t0 = begin; t0 + 4 <= end; t0 += 4 * kWave) {
-      const int t = t0 + 4 * lane;
-      put4(rs, t + 4 <= end ? (row + t) * (int)sizeof(R) : kDropped, z, z, z, z);
+    for (int t = begin + 4 * first; t - 4 * first < end; t += 4 * lanes)
+      put4(rs, t < end ? min(t, end - 4) * (int)sizeof(R) : kDropped, z, z, z, z);
+  };
+  // rows [r_lo, r_hi) and columns [lo, hi) of the array's rows x width are the sweep's
+  auto zero_around = [&](__amdgpu_buffer_rsrc_t rs, int rows, int width, int r_lo, int r_hi, int lo, int hi,
+                         int part, int parts) {
+    if (r_hi <= r_lo) {
+      zero_run(rs, 0, rows * width, part * kWave + lane, parts * kWave);
+      return;
     }
-    // what is left of the last group, as one group that ends with the range
-    if (len & 3) put4(rs, lane == 0 ? (row + end - 4) * (int)sizeof(R) : kDropped, z, z, z, z);
+    zero_run(rs, 0, r_lo * width + lo, part * kWave + lane, parts * kWave);
+    zero_run(rs, (r_hi - 1) * width + hi, rows * width, part * kWave + lane, parts * kWave);
+    const int gap = width - hi + lo, q = lane & 15;
+    if (gap <= 0) return;
+    for (int r = r_lo + 4 * part; r < r_hi - 1; r += 4 * parts) {
+      const int row = r + (lane >> 4), begin = row * width + hi;
+      const bool there = row < r_hi - 1;
+      if (gap < 4) {
+        put1(rs, there && q < gap ? (begin + q) * (int)sizeof(R) : kDropped, (R)0);
+      } else {
+        for (int t = 4 * q; t - 4 * q < gap; t += 64)
+          put4(rs, there && t < gap ? (begin + min(t, gap - 4)) * (int)sizeof(R) : kDropped, (R)0, (R)0, (R)0,
+               (R)0);
+      }
+    }
   };
   auto zero_outside = [&](int part, int parts) {
     if (!boundary) return;
-    const int s_lo = win.s0, s_hi = win.s0 + win.ns;
-    const int t_lo = win.t0, t_hi = win.t0 + win.nt;
-    for (int s = part; s <= S; s += parts) {
-      if (s < S) {
-        if (win.ok && s >= s_lo && s < s_hi) {
-          zero_range(gx_rsrc, s * T1, 0, t_lo);
-          zero_range(gx_rsrc, s * T1, t_hi - shift + 1, T1);
-        } else {
-          zero_range(gx_rsrc, s * T1, 0, T1);
-        }
-      }
-      if (win.ok && s >= s_lo && s <= s_hi) {
-        zero_range(gy_rsrc, s * T, 0, t_lo);
-        zero_range(gy_rsrc, s * T, t_hi, T);
-      } else {
-        zero_range(gy_rsrc, s * T, 0, T);
-      }
-    }
+    const int s_hi = win.ok ? win.s0 + win.ns : 0, s_lo = win.ok ? win.s0 : 0;
+    const int t_hi = win.t0 + win.nt;
+    zero_around(gx_rsrc, S, T1, s_lo, s_hi, win.t0, t_hi - shift + 1, part, parts);
+    zero_around(gy_rsrc, S + 1, T, s_lo, win.ok ? s_hi + 1 : 0, win.t0, t_hi, part, parts);
   };
   if (kApart && part > 0 && (!win.ok || part * kWave > win.ns)) return;
   if (!win.ok) {
@@ -952,6 +1063,13 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     poison();
   };
 
+  if (kHelp > 0 && wave >= nwaves - kHelp) {
+    // -------------------------------- helpers ------------------------------------
+    const int parts = kApart ? (NS + kWave) / kWave : 1;  // (the bands' workgroups)
+    zero_outside(part * kHelp + nwaves - 1 - wave, parts * kHelp);
+    if (loss && b == 0 && part == 0 && wave == nwaves - 1) reduce_scores(scores, loss, B, reduction, lane);
+    return;
+  }
   if (kApart && wave >= 1 + kStagers) {
     // ------------------------------- courier waves -------------------------------
     if (wave == 1 + kStagers) {
@@ -968,13 +1086,15 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   }
   if (wave >= nsweep) {
     // ------------------------------ staging wave -------------------------------
-    const int w = (wave - nsweep) / kStagers, l = (wave - nsweep) % kStagers;
+    constexpr int kGroups = kStagerGroups<kStagers, kShares>, kPer = kStagers / kGroups;
+    const int w = (wave - nsweep) / kStagers, l = (wave - nsweep) % kPer;
+    const int group = (wave - nsweep) % kStagers / kPer;  // as in the forward kernel
     R *base = tiles + (size_t)w * 2 * kBuffers * kTileElems;
     const int half = lane >> 5, q = lane & 31;
-    // rows of a tile this wave stages: r(u) = 2*l + half + 2*kStagers*u
-    constexpr int kRows = (kWave + 2 * kStagers - 1) / (2 * kStagers);
+    // rows of a tile this wave stages: r(u) = 2*l + half + 2*kPer*u
+    constexpr int kRows = (kWave + 2 * kPer - 1) / (2 * kPer);
     struct Staged {
-      R here[kRows], below[kRows], x[kRows];
+      R here[kRows], below[kRows], x[kRows];  // (kShares: here = d1, and nothing else)
     };
     // Global fetches of tile m+1 are issued (into registers) as soon as tile m is staged,
     // before this wave waits for the next LDS buffer, so their latency overlaps the
@@ -982,7 +1102,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     // what was read for cells outside the window.
     const __amdgpu_buffer_rsrc_t p_rsrc = buffer_of(const_cast<R *>(pb), (size_t)(S + 1) * TP);
     const __amdgpu_buffer_rsrc_t px_rsrc = buffer_of(const_cast<R *>(pxb), (size_t)S * T1);
-    constexpr int kStep = 2 * kStagers;
+    constexpr int kStep = 2 * kPer;
     constexpr int kSize = (int)sizeof(R);
     const int r_first = 2 * l + half;
     auto fetch = [&](Staged &in, const Band &g, int m) {
@@ -1026,15 +1146,32 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
         d.vy[u] = gys[u * kStep * kTilePitch];
       }
     };
+    // (kShares) what a tile holds are d1 and the cells' gradients, 0 where d1 is kNoShares; the + 0 makes a
+    // -0 of that 0
+    auto split = [&](Drained &d) {
+      if constexpr (kShares)
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) {
+          const R d1 = d.vx[u], cell = d.vy[u];
+          d.vx[u] = d1 * cell;
+          d.vy[u] = __builtin_fmaf((R)1 - d1, cell, (R)0);
+        }
+    };
     // (apart) The gradients that the tile's last row hands down go to the outgoing seam as soon as
     // the tile is done: the workgroup of the next band waits for them.
-    constexpr int kLastL = (kWave / 2 - 1) % kStagers, kLastU = (kWave / 2 - 1) / kStagers;
-    auto hand_on = [&](const Drained &d) {
-      if (!kApart || l != kLastL || d.row0 + kWave > NS) return;  // (wave-uniform)
+    constexpr int kLastL = (kWave / 2 - 1) % kPer, kLastU = (kWave / 2 - 1) / kPer;
+    auto hand_on = [&](const Drained &d) -> bool {
+      if (!kApart || l != kLastL || d.row0 + kWave > NS) return true;  // (wave-uniform)
       const int col = d.pm * kTileSteps + q - (kWave - 1);
-      if (half == 1 && (unsigned)col <= (unsigned)NT) seam[seam_pitch + col] = d.vx[kLastU];
+      if (half == 1 && (unsigned)col <= (unsigned)NT) seam[seam_pitch + col] = kShares ? d.vx[kLastU] * d.vy[kLastU] : d.vx[kLastU];
       const int done = max(0, min(d.pm * kTileSteps + kTileSteps - (kWave - 1), cols));
+      if (kGroups > 1) {  // as in the forward kernel
+        const int already = max(0, min(d.pm * kTileSteps - (kWave - 1), cols));
+        if (done == already) return true;
+        if (!wait_for(&cnt.ready[1], already, spin_limit)) return false;
+      }
       if (lane == 0) publish_lds_writes(&cnt.ready[1], done);
+      return true;
     };
     auto store = [&](const Drained &d) {
       constexpr int kMinX = kModified ? 1 : 0;
@@ -1069,7 +1206,139 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     };
     int tile_base = 0, buf = 0;  // buf = tile number modulo kBuffers
     bool zeroed = false;
-    for (int band = part; band * band_rows <= last_row; ++band) {
+    if constexpr (kShares) {
+      // As in the forward kernel: several tiles' d1 are on their way, each in a set of registers, and one
+      // tile's loads and one tile's stores follow each other on every path.
+      auto request = [&](Staged &in, const Band &g, int m) {
+        const int s_first = win.s0 + NS - (g.row0 + r_first);
+        const int j_first = NT - (m * kTileSteps + q - r_first);
+        const int at = m < g.ntiles ? (s_first * TP + win.t0 + j_first) * kSize : kDropped;
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) in.here[u] = get1(p_rsrc, at - u * (kStep * (TP - 1) * kSize), R());
+      };
+      constexpr int kAhead = kGroups > 1 ? 1 : kFetchAhead<R>;
+      constexpr int kNowhere = -(1 << 20);  // (a tile with no cell in the window)
+      // the tile that a buffer held before tile m of the band that starts at row0
+      const int whole_tiles = (NT + kWave + kTileSteps - 1) / kTileSteps;
+      auto take_before = [&](Drained &d, int row0, int m, int buf) {
+        int pm = m - kBuffers;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          row0 = pm < 0 ? row0 - band_rows : row0;
+          pm = pm < 0 ? pm + whole_tiles : pm;
+        }
+        take(d, row0, pm, buf);
+      };
+      int end_row0 = 0, end_tiles = 0;
+      for (int band = part; band * band_rows <= last_row; ++band) {
+        const Band g = band_of(band, w, nsweep, NS, NT);
+        if (g.row0 > NS) break;
+        Staged ahead[kAhead];
+        Drained out = {};
+        out.pm = kNowhere;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+          request(ahead[k], g, group + k * kGroups);
+#pragma unroll
+          for (int u = 0; u < 2 * kRows; ++u) put1(p_rsrc, kDropped + u * kSize, (R)0);
+        }
+        auto stage = [&](const Staged &cur, int m) __attribute__((always_inline)) -> bool {
+          const int gt = tile_base + m, buf = gt % kBuffers;
+          if (gt >= kBuffers) {
+            // the buffer still holds the gradients of tile gt - kBuffers
+            if (!wait_for(&cnt.written[w], gt - kBuffers + 1, spin_limit)) return false;
+            take_before(out, g.row0, m, buf);
+            if (!hand_on(out)) return false;
+          }
+          if (kApart && l == 0 && g.row0 > 0) {  // (wave-uniform) the row above is another workgroup's
+            const int col = m * kTileSteps + q - shift;
+            const int need = min((m + 1) * kTileSteps - shift, cols - shift);
+            if (need > 0 && !wait_for(&cnt.ready[0], need, spin_limit)) return false;
+            R v = 0;
+            if (half == 0 && col >= 0 && col < cols - shift) v = seam[col];
+            if (half == 0) handed_down[buf * kTileSteps + q] = v;
+          }
+          // (the wait for this tile's inputs, on every path through what follows)
+#pragma unroll
+          for (int u = 0; u < kRows; ++u) asm volatile("" ::"v"(cur.here[u]));
+          R *dst = base + buf * kTileElems + r_first * kTilePitch + q;
+          // (cells outside the window: any finite value)
+          unsigned most = 0;
+#pragma unroll
+          for (int u = 0; u < kRows; ++u) {
+            if (r_first + kStep * u >= kWave) continue;
+            const unsigned d1 = min(__float_as_uint(cur.here[u]), kNoShares);
+            most = max(most, d1);
+            dst[u * kStep * kTilePitch] = __uint_as_float(d1);
+          }
+          // cells of the window that pass nothing on, if there are any: the sweep then looks at each cell
+          if (__ballot(most == kNoShares)) {
+            bool there = false;
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+              const int r = r_first + kStep * u;
+              there = there || (r < kWave && g.row0 + r <= NS && __float_as_uint(cur.here[u]) >= kNoShares &&
+                                (unsigned)(m * kTileSteps + q - r) <= (unsigned)NT);
+            }
+            if (__ballot(there) && lane == 0)
+              __hip_atomic_fetch_or(&cnt.loaded[w * kBuffers + buf], kNoSharesHere, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+          // every lane's LDS writes precede the release by lane 0 of the same wave
+          if (lane == 0) count_in(&cnt.loaded[w * kBuffers + buf]);
+          return true;
+        };
+        bool failed = false;
+        for (int m = group; m < g.ntiles; m += kAhead * kGroups) {
+#pragma unroll
+          for (int k = 0; k < kAhead; ++k) {
+            if (m + k * kGroups < g.ntiles && !failed)
+              failed = !stage(ahead[k], m + k * kGroups);
+            else
+              out.pm = kNowhere;
+            request(ahead[k], g, m + (k + kAhead) * kGroups);
+            asm volatile("" ::: "memory");
+            split(out);
+            store(out);
+          }
+          if (failed) {
+            give_up();
+            return;
+          }
+          if (kHelp == 0 && !zeroed && m + kAhead * kGroups >= kBuffers) {
+            // the sweep wave is that many tiles behind now: time for the zeros around the window
+            if (part == 0) zero_outside(wave - nsweep, nsweep * kStagers);
+            zeroed = true;
+          }
+        }
+        tile_base += g.ntiles;
+        end_row0 = g.row0;
+        end_tiles = g.ntiles;
+      }
+      // the tiles still in the buffers
+      for (int gt = max(tile_base - kBuffers, 0); gt < tile_base; ++gt) {
+        if (gt % kGroups != group) continue;
+        Drained out;
+        if (!wait_for(&cnt.written[w], gt + 1, spin_limit)) {
+          give_up();
+          return;
+        }
+        take_before(out, end_row0, gt - tile_base + end_tiles + kBuffers, gt % kBuffers);
+        if (!hand_on(out)) {
+          give_up();
+          return;
+        }
+        split(out);
+        store(out);
+      }
+      if (kHelp == 0) {
+        if (!zeroed && part == 0) zero_outside(wave - nsweep, nsweep * kStagers);
+        if (loss && b == 0 && part == 0 && wave == nsweep) reduce_scores(scores, loss, B, reduction, lane);
+      }
+      if (peek(&cnt.failed)) poison();
+      return;
+    }
+    for (int band = part; band * band_rows <= last_row && !kShares; ++band) {
       const Band g = band_of(band, w, nsweep, NS, NT);
       if (g.row0 > NS) break;
       Staged cur;
@@ -1194,6 +1463,28 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     int seen_ready = 0;
     R seen_seam = 0;
     int seen_loaded = 0;
+    // waits until the tile is staged; kShares: and notes whether any so far held a cell that passes nothing
+    // on, which only the tiles that are not plain look for
+    bool some_keep = false;
+    auto staged = [&]() __attribute__((always_inline)) -> bool {
+      constexpr int kMask = kShares ? kNoSharesHere - 1 : -1;
+      constexpr int kPer = kStagers / kStagerGroups<kStagers, kShares>;
+      int *loaded = &cnt.loaded[w * kBuffers + buf];
+      int seen = __builtin_amdgcn_readfirstlane(seen_loaded);
+      for (int spins = 0; (seen & kMask) < kPer * (rounds + 1);) {
+        seen = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(loaded, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+        if ((seen & kMask) >= kPer * (rounds + 1)) break;
+        __builtin_amdgcn_s_sleep(1);
+        if (++spins > spin_limit) {
+          give_up();
+          return false;
+        }
+      }
+      some_keep = kShares && (seen & kNoSharesHere) != 0;
+      seen_loaded = seen;  // (asked again where a loop of plain tiles ends before its time)
+      return true;
+    };
     // one tile, specialised at compile time on whether the wave takes from a seam (kUp) and feeds
     // one (kDown), and on kPlain, with a loop for each kind, for the forward kernel's reasons
     auto one_tile = [&](int m, auto up_c, auto down_c, auto plain_c) __attribute__((always_inline)) -> bool {
@@ -1201,21 +1492,17 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       constexpr bool kDown = decltype(down_c)::value;
       constexpr bool kPlain = decltype(plain_c)::value;
       const int gt = tile_base + m;
-      if (__builtin_amdgcn_readfirstlane(seen_loaded) < kStagers * (rounds + 1) &&
-          !wait_for(&cnt.loaded[w * kBuffers + buf], kStagers * (rounds + 1), spin_limit)) {
-        give_up();
-        return false;
-      }
-      R d1q[kTileSteps], d2q[kTileSteps];
+      R d1q[kTileSteps], d2q[kShares ? 1 : kTileSteps];
       const R *handed_at = handed_down + buf * kTileSteps;
       R arrived[kChunk];  // (apart) what lane 0 receives in the chunk's steps
       if constexpr (kApart && kUp) pull_chunk(arrived, handed_at);
       R *gx_row = base + buf * kTileElems + lane * kTilePitch;               // d1 in, gx out
       R *gy_row = base + (kBuffers + buf) * kTileElems + lane * kTilePitch;  // d2 in, gy out
+      // (kShares: d1 in and left there; cells out)
       buf = buf + 1 == kBuffers ? 0 : buf + 1;
       rounds += buf == 0;
       pull_row(d1q, gx_row);
-      pull_row(d2q, gy_row);
+      if constexpr (!kShares) pull_row(d2q, gy_row);
 
       bool failed = false;
       auto chunk = [&](int c4, int e0) __attribute__((always_inline)) {
@@ -1265,15 +1552,16 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
           }
           // cells outside the window carry d1 = d2 = 0, so nothing leaks in or out
           cell[k] = from_above + to_left;
+          if constexpr (kShares && !kPlain) cell[k] = d1q[kk] == __uint_as_float(kNoShares) ? (R)0 : cell[k];
           down[k] = d1q[kk] * cell[k];
-          left[k] = d2q[kk] * cell[k];
+          left[k] = (kShares ? (R)1 - d1q[kk] : d2q[kShares ? 0 : kk]) * cell[k];
           to_below2 = to_below;
           to_below = down[k];
           to_left = left[k];
           if (k == kChunk / 2 - 1) {
             // the chunk's gradients take the place of its d1 / d2 in the tile: first half
-            push_half<0>(gx_row + c4 * kChunk, down);
-            push_half<0>(gy_row + c4 * kChunk, left);
+            if constexpr (!kShares) push_half<0>(gx_row + c4 * kChunk, down);
+            push_half<0>(gy_row + c4 * kChunk, kShares ? cell : left);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -1294,8 +1582,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
             publish_lds_writes(&cnt.ready[w], my_base + done);
           }
         }
-        push_half<1>(gx_row + c4 * kChunk, down);
-        push_half<1>(gy_row + c4 * kChunk, left);
+        if constexpr (!kShares) push_half<1>(gx_row + c4 * kChunk, down);
+        push_half<1>(gy_row + c4 * kChunk, kShares ? cell : left);
         if constexpr (kApart && kUp) {
           if (c4 + 1 < kTileSteps / kChunk)
 #pragma unroll
@@ -1317,12 +1605,16 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     };
     auto sweep_tiles = [&](auto up_c, auto down_c) __attribute__((always_inline)) -> bool {
       const PlainTiles plain = plain_tiles(g, fin_step, !kApart && decltype(up_c)::value, shift, NT);
-      for (int m = 0; m < plain.lo; ++m)
-        if (!one_tile(m, up_c, down_c, std::false_type{})) return false;
-      for (int m = plain.lo; m < plain.hi; ++m)
+      int m = 0;
+      for (; m < plain.lo; ++m)
+        if (!staged() || !one_tile(m, up_c, down_c, std::false_type{})) return false;
+      for (; m < plain.hi; ++m) {
+        if (!staged()) return false;
+        if (kShares && some_keep) break;
         if (!one_tile(m, up_c, down_c, std::true_type{})) return false;
-      for (int m = plain.hi; m < g.ntiles; ++m)
-        if (!one_tile(m, up_c, down_c, std::false_type{})) return false;
+      }
+      for (; m < g.ntiles; ++m)
+        if (!staged() || !one_tile(m, up_c, down_c, std::false_type{})) return false;
       return true;
     };
     bool done;
@@ -1391,17 +1683,19 @@ bool bands_apart(int B, int S, int T, bool backward) {
   constexpr double kCost[2][3] = {{6, 7, 10}, {11, 16, 20}}, kSaved[2][3] = {{6.7, 7, 39}, {13, 28, 60}};
   return 1e-3 * kSaved[backward][bands - 2] * (S + T) > kCost[backward][bands - 2];
 }
-inline void mark_seams(const int64_t *boundary, float *p, float *ans, float *px_grad, int B, int S,
-                       int T, int modified, hipStream_t stream) {
+inline void mark_seams(const int64_t *boundary, float *p, float *mail, float *ans, float *px_grad, int B,
+                       int S, int T, int modified, hipStream_t stream) {
   hipLaunchKernelGGL(mark_seams_kernel, dim3(B, (S + kWave) / kWave - 1), dim3(256), 0, stream,
-                     boundary, p, ans, px_grad, S, T, modified);
+                     boundary, p, mail, ans, px_grad, S, T, modified);
 }
 
 // `px_grad`: if given, its seams are marked as well (for a backward_impl that follows and is told so).
-template <typename R>
+// kShares (float only): p is filled for a backward_impl with kShares; py_grad is its py_grad.
+template <typename R, bool kShares = false>
 int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans, int B, int S,
                  int T, int modified, void *stream, int checks = 0, int *status = nullptr,
-                 R *px_grad = nullptr) {
+                 R *px_grad = nullptr, R *py_grad = nullptr) {
+  static_assert(!kShares || sizeof(R) == 4, "shares are float's");
   if (B < 0 || S < 0 || T < 0) return fail(FRNNT_EINVAL, "mi_forward: negative size");
   if (B == 0) return FRNNT_OK;
   if (!px || !py || !p || !ans) return fail(FRNNT_EINVAL, "mi_forward: null pointer");
@@ -1417,43 +1711,45 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   const bool few = n <= 2 && lds_bytes(n, T, kFewBuffers, sizeof(R)) <= kLdsBudget;
   // (doubles keep two staging waves per sweep wave: with more waves in the workgroup a sweep
   // wave's two tile rows of doubles no longer fit its share of the registers)
-  constexpr int kMany = sizeof(R) == 4 ? kFwdStagers : 2, kFew = sizeof(R) == 4 ? kFwdStagersFew : 2;
+  constexpr int kMany = sizeof(R) == 4 ? kFwdStagers : 2;
+  constexpr int kFew = kShares ? kSharesStagers : sizeof(R) == 4 ? kFwdStagersFew : 2;
   if constexpr (sizeof(R) == 4) {
     const bool apart = bands_apart<R>(B, S, T, false), later = px_grad && bands_apart<R>(B, S, T, true);
     if (apart || later)
-      mark_seams(boundary, apart ? p : nullptr, ans, later ? px_grad : nullptr, B, S, T, modified,
-                 static_cast<hipStream_t>(stream));
+      mark_seams(boundary, apart && !kShares ? p : nullptr, apart && kShares ? py_grad : nullptr, ans,
+                 later ? px_grad : nullptr, B, S, T, modified, static_cast<hipStream_t>(stream));
     if (apart) {
       const int pitch = (B + 7) / 8 * 8;  // (an utterance's bands on one XCD)
       const size_t lds = apart_lds_bytes(T);
-      auto kernel = modified ? mi_forward_kernel<R, true, 1, kFew, kApartBuffers, true>
-                             : mi_forward_kernel<R, false, 1, kFew, kApartBuffers, true>;
+      auto kernel = modified ? mi_forward_kernel<R, true, 1, kFew, kApartBuffers, true, kShares>
+                             : mi_forward_kernel<R, false, 1, kFew, kApartBuffers, true, kShares>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_forward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kFew) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T,
-                         mi_spin_limit, checks, status, B, pitch);
+                         mi_spin_limit, checks, status, B, pitch, py_grad);
       return check_launch("mi_forward");
     }
   }
   const int stagers = few ? kFew : kMany;
   const size_t lds = lds_bytes(n, T, few ? kFewBuffers : 2, sizeof(R));
   const bool one_band = few && S + 1 <= kWave;
-  auto kernel = one_band ? (modified ? mi_forward_kernel<R, true, 1, kFew, kFewBuffers, false>
-                                     : mi_forward_kernel<R, false, 1, kFew, kFewBuffers, false>)
-              : few      ? (modified ? mi_forward_kernel<R, true, 2, kFew, kFewBuffers, false>
-                                     : mi_forward_kernel<R, false, 2, kFew, kFewBuffers, false>)
-                         : (modified ? mi_forward_kernel<R, true, kMaxSweep, kMany, 2, false>
-                                     : mi_forward_kernel<R, false, kMaxSweep, kMany, 2, false>);
+  auto kernel = one_band ? (modified ? mi_forward_kernel<R, true, 1, kFew, kFewBuffers, false, kShares>
+                                     : mi_forward_kernel<R, false, 1, kFew, kFewBuffers, false, kShares>)
+              : few      ? (modified ? mi_forward_kernel<R, true, 2, kFew, kFewBuffers, false, kShares>
+                                     : mi_forward_kernel<R, false, 2, kFew, kFewBuffers, false, kShares>)
+                         : (modified ? mi_forward_kernel<R, true, kMaxSweep, kMany, 2, false, kShares>
+                                     : mi_forward_kernel<R, false, kMaxSweep, kMany, 2, false, kShares>);
   if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
     return check_launch("mi_forward: hipFuncSetAttribute");
   hipLaunchKernelGGL(kernel, dim3(B), dim3(n * (1 + stagers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T, mi_spin_limit,
-                     checks, status, B, B);
+                     checks, status, B, B, py_grad);
   return check_launch("mi_forward");
 }
 
-template <typename R>
+// kShares: p is what a forward_impl with kShares has left; px is not read.
+template <typename R, bool kShares = false>
 int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p, R *ans_grad,
                   R *px_grad, R *py_grad, int B, int S, int T, int modified,
                   int overwrite_ans_grad, void *stream, const R *scores = nullptr,
@@ -1463,7 +1759,7 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
     return fail(FRNNT_EINVAL, "mi_backward: loss without scores, or bad reduction");
   if (B < 0 || S < 0 || T < 0) return fail(FRNNT_EINVAL, "mi_backward: negative size");
   if (B == 0) return FRNNT_OK;
-  if (!px || !p || !px_grad || !py_grad)
+  if ((!px && !kShares) || !p || !px_grad || !py_grad)
     return fail(FRNNT_EINVAL, "mi_backward: null pointer");
   if ((size_t)(S + 1) * (T + 1) * sizeof(R) >= ((size_t)1 << 30))
     return fail(FRNNT_ELIMIT, "mi_backward: one utterance's lattice exceeds 1 GiB");
@@ -1475,22 +1771,23 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   // of one to empty and refill a buffer.  (A workgroup of 16 waves leaves each 128
   // registers, too few for a sweep wave's two tile rows of doubles.)
   constexpr bool kFloat = sizeof(R) == 4;
-  constexpr int kFew = kFloat ? kBwdStagersFew : kBwdStagers;
+  constexpr int kFew = kShares ? kSharesStagers : kFloat ? kBwdStagersFew : kBwdStagers;
   constexpr int kFewBuffers = kFloat ? 3 : 2;
   static_assert(kMaxSweep * 2 <= 16 && 2 * kFewBuffers <= 16, "Counters::loaded is too short");
   const bool few = n <= 2 && lds_bytes(n, T, kFewBuffers, sizeof(R)) <= kLdsBudget;
   if constexpr (kFloat) {
     if (bands_apart<R>(B, S, T, true)) {
       if (!marked)
-        mark_seams(boundary, nullptr, nullptr, px_grad, B, S, T, modified,
+        mark_seams(boundary, nullptr, nullptr, nullptr, px_grad, B, S, T, modified,
                    static_cast<hipStream_t>(stream));
       const int pitch = (B + 7) / 8 * 8;
       const size_t lds = apart_lds_bytes(T);
-      auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kApartBuffers, true>
-                             : mi_backward_kernel<R, false, 1, kFew, kApartBuffers, true>;
+      auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kApartBuffers, true, kShares>
+                             : mi_backward_kernel<R, false, 1, kFew, kApartBuffers, true, kShares>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_backward: hipFuncSetAttribute");
-      hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kFew) * kWave), lds,
+      hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)),
+                         dim3((3 + kFew + kHelpers<1, kShares>) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
                          py_grad, S, T, overwrite_ans_grad, scores, loss, B, reduction, mi_spin_limit,
                          pitch);
@@ -1499,13 +1796,14 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   }
   const int stagers = few ? kFew : kBwdStagers;
   const size_t lds = lds_bytes(n, T, few ? kFewBuffers : 2, sizeof(R));
-  auto kernel = few ? (modified ? mi_backward_kernel<R, true, 2, kFew, kFewBuffers, false>
-                                : mi_backward_kernel<R, false, 2, kFew, kFewBuffers, false>)
-                    : (modified ? mi_backward_kernel<R, true, kMaxSweep, kBwdStagers, 2, false>
-                                : mi_backward_kernel<R, false, kMaxSweep, kBwdStagers, 2, false>);
+  auto kernel = few ? (modified ? mi_backward_kernel<R, true, 2, kFew, kFewBuffers, false, kShares>
+                                : mi_backward_kernel<R, false, 2, kFew, kFewBuffers, false, kShares>)
+                    : (modified ? mi_backward_kernel<R, true, kMaxSweep, kBwdStagers, 2, false, kShares>
+                                : mi_backward_kernel<R, false, kMaxSweep, kBwdStagers, 2, false, kShares>);
   if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
     return check_launch("mi_backward: hipFuncSetAttribute");
-  hipLaunchKernelGGL(kernel, dim3(B), dim3(n * (1 + stagers) * kWave), lds,
+  const int helpers = few ? kHelpers<2, kShares> : kHelpers<kMaxSweep, kShares>;
+  hipLaunchKernelGGL(kernel, dim3(B), dim3((n * (1 + stagers) + helpers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
                      py_grad, S, T, overwrite_ans_grad, scores, loss, B, reduction, mi_spin_limit, B);
   return check_launch("mi_backward");

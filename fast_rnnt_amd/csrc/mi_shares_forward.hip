@@ -1,0 +1,15 @@
+// The lattice recursion's forward kernel in float32 for callers that want the scores and the occupation
+// gradients and not the table of p: it leaves in p's place what the backward kernel needs (kShares in
+// mi_recursion.hip.h; mi_shares_backward.hip).
+#include "mi_recursion.hip.h"
+
+namespace frnnt {
+
+int mi_forward_shares(const float *px, const float *py, const int64_t *boundary, float *shares,
+                      float *scores, int B, int S, int T, int modified, int checks, int32_t *status,
+                      float *px_grad, float *py_grad, void *stream) {
+  return forward_impl<float, true>(px, py, boundary, shares, scores, B, S, T, modified, stream, checks,
+                                   status, px_grad, py_grad);
+}
+
+}  // namespace frnnt

@@ -3,6 +3,8 @@
 // gradient of ones (the occupation probabilities), and the reduction of the scores.
 // It only chains the entry points of the other files on one stream; what it saves
 // is host time, which matters once a whole call takes ~100 us on the GPU.
+#include <type_traits>
+
 #include "simple_shared.hip.h"
 
 namespace frnnt {
@@ -17,6 +19,19 @@ int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
                 void *stream) {
   if ((px_grad == nullptr) != (py_grad == nullptr))
     return fail(FRNNT_EINVAL, "mi_loss_fwd: px_grad and py_grad go together");
+  const bool p_wanted = (checks & FRNNT_SCRATCH_P) == 0;
+  checks &= ~FRNNT_SCRATCH_P;
+  if constexpr (std::is_same<R, float>::value) {
+    if (px_grad && !p_wanted) {
+      int rc = mi_forward_shares(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad,
+                                 py_grad, stream);
+      if (rc != FRNNT_OK) return rc;
+      rc = mi_backward_shares(boundary, p, px_grad, py_grad, scores, loss, B, S, T, modified, reduction,
+                              stream);
+      if (rc != FRNNT_OK || B > 0) return rc;
+      return loss ? reduce(scores, loss, B, reduction, stream) : rc;
+    }
+  }
   int rc = mi_forward(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad, stream);
   if (rc != FRNNT_OK) return rc;
   if (px_grad) {

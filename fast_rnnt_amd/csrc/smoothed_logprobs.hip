@@ -995,7 +995,7 @@ int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t 
                                      termination_symbol, rnnt_type, boundary != nullptr, stream, &mix);
   if (rc != FRNNT_OK) return rc;
   return frnnt_mi_loss_fwd_f32(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, !regular,
-                               reduction, checks, status, stream);
+                               reduction, checks | FRNNT_SCRATCH_P, status, stream);
 }
 int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t *symbols,
                                 const int64_t *boundary, const float *kept, const float *score_grad,

@@ -74,7 +74,8 @@ FRNNT_BOTH(mi_loss_fwd,
            (const double *px, const double *py, const int64_t *bnd, double *p, double *sc,
             double *gx, double *gy, double *loss, int B, int S, int T, int modified, int red,
             int checks, int32_t *status, void *st),
-           (px, py, bnd, p, sc, gx, gy, loss, B, S, T, modified, red, checks, status, st))
+           (px, py, bnd, p, sc, gx, gy, loss, B, S, T, modified, red, checks | FRNNT_SCRATCH_P, status,
+            st))
 FRNNT_BOTH(mi_scale_grads,
            (float *gx, float *gy, const float *g, int gstride, double gscale, int B, int S, int T,
             int modified, void *st),
@@ -547,7 +548,7 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
                  need_grad ? k + o_nr * item : nullptr, w + o_p * item, w + o_sc * item,
                  gx.defined() ? gx.data_ptr() : nullptr, gy.defined() ? gy.data_ptr() : nullptr,
                  loss.data_ptr(), (int)B, (int)S, (int)T, (int)C,
-                 (int)term, (int)kind, delay_penalty, (int)reduction, (int)checks,
+                 (int)term, (int)kind, delay_penalty, (int)reduction, (int)checks | FRNNT_SCRATCH_P,
                  status_for(am, bnd), stream_of(am)),
              "frnnt_additive_loss_fwd");
     if (need_grad) {
@@ -851,7 +852,8 @@ struct LatticeLossFn : public torch::autograd::Function<LatticeLossFn> {
                                   w + o_xr, w + o_yr, w + o_p, w + o_sc, p_gx, p_gy, ptr<R>(loss),
                                   (int)B, (int)S, (int)T, (int)K, (int)C, (int)term, (int)kind,
                                   delay_penalty > 0.0 ? delay_penalty : 0.0, (int)reduction,
-                                  (int)checks, status_for(logits, bnd), stream_of(logits)),
+                                  (int)checks | FRNNT_SCRATCH_P, status_for(logits, bnd),
+                                  stream_of(logits)),
              "frnnt_lattice_loss_fwd");
     if (need_grad) {
       // (absent tensors are not saved: saved tensors must be defined)

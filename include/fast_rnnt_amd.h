@@ -289,7 +289,7 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
  * whole lm_grad and am_grad: the terms of both unigram models inside the joint model's gradient
  * products.
  *   kept: frnnt_smoothed_loss_kept() floats, written by _fwd for _bwd
- *   px, py, p, scores: as in those entry points, not needed afterwards; px_joint, py_joint: not used
+ *   px, py, p, scores: as in those entry points, not needed afterwards (p is scratch); px_joint, py_joint: not used
  *   partial [ceil(B*(S+1)/16)][C]: scratch
  *   scratch of _bwd: B (S+1) (4 + T rounded up to 4) + 2 B T + C + ceil(B*T/16) C floats, each
  *     of its seven parts rounded up to 4 (40 more are enough for that)
@@ -367,8 +367,11 @@ int frnnt_additive_loss_bwd(int dtype, const void *lm, const void *am, const int
  * with a gradient of ones (mutual_information.py:159-168), then -- when loss is given --
  * frnnt_loss_reduce (the backward kernel reduces the scores on its way: no extra launch).
  * p [B][S+1][T+1] and scores [B] are outputs as well; checks / status (may be 0 / NULL) as
- * in frnnt_mi_forward_checked.
+ * in frnnt_mi_forward_checked.  FRNNT_SCRATCH_P among the checks, here and in the losses that chain this
+ * entry point: the caller does not want p, whose buffer is then scratch (the float32 kernels pass the
+ * shares of the cells' gradients from the forward to the backward there; the same results, faster).
  */
+#define FRNNT_SCRATCH_P 0x100
 int frnnt_mi_loss_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *p,
                           float *scores, float *px_grad, float *py_grad, float *loss, int B, int S,
                           int T, int modified, int reduction, int checks, int32_t *status,

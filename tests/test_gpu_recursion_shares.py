@@ -1,0 +1,123 @@
+"""The recursion of the losses, which leaves the shares of the cells' gradients in the place of p, against
+the two entry points that go through p: the same operations, so the same bits."""
+import math
+
+import pytest
+import torch
+
+import fast_rnnt_amd as F
+from fast_rnnt_amd import _fast_rnnt, _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(B, S, T, modified, seed):
+    g = torch.Generator().manual_seed(seed)
+    T1 = T if modified else T + 1
+    px = -2.0 + 1.5 * torch.randn(B, S, T1, generator=g)
+    py = -1.0 + torch.randn(B, S + 1, T, generator=g)
+    if not modified:
+        px[:, :, T] = -math.inf
+    return px, py, g
+
+
+def _window(B, S, T, g):
+    rows = []
+    for _ in range(B):
+        s0 = int(torch.randint(0, S // 3 + 1, (), generator=g))
+        t0 = int(torch.randint(0, T // 3 + 1, (), generator=g))
+        rows.append([s0, t0, int(torch.randint(s0, S + 1, (), generator=g)),
+                     int(torch.randint(t0, T + 1, (), generator=g))])
+    rows[0] = [0, 0, S, T]
+    return torch.tensor(rows)
+
+
+def _compare(px, py, boundary):
+    px, py = px.cuda(), py.cuda()
+    boundary = None if boundary is None else boundary.cuda()
+    B, S, T = px.shape[0], px.shape[1], py.shape[2]
+    p = torch.empty(B, S + 1, T + 1, device="cuda")
+    want = _fast_rnnt.mutual_information_forward(px, py, boundary, p)
+    want_x, want_y = _fast_rnnt.mutual_information_backward(px, py, boundary, p,
+                                                            torch.ones(B, device="cuda"))
+    got, (got_x, got_y) = F.mutual_information_recursion(px, py, boundary, return_grad=True)
+    for a, b in ((got, want), (got_x, want_x), (got_y, want_y)):
+        assert torch.allclose(a, b, rtol=0, atol=0, equal_nan=True)
+    return want_x, want_y
+
+
+# one step to a tile's remainder either way, one row to a band's, one to four bands in a workgroup or
+# apart, more than four
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("B,S,T", [
+    (2, 1, 1), (5, 7, 31), (4, 30, 33), (3, 62, 64), (3, 63, 65), (3, 64, 95), (2, 65, 160),
+    (9, 127, 130), (2, 128, 191), (2, 200, 257), (3, 255, 1100), (2, 300, 310), (130, 66, 300), (2, 70, 900),
+])
+def test_same_bits_as_through_p(B, S, T, modified):
+    px, py, g = _inputs(B, S, T, modified, 17 * S + T)
+    _compare(px, py, None)
+    _compare(px, py, _window(B, S, T, g))
+
+
+# cells whose share is not finite pass nothing on; cells that cannot be reached hand everything left
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("S,T", [(20, 40), (63, 150), (64, 150), (150, 200), (130, 1300)])
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+def test_cells_that_are_not_finite(S, T, modified, value):
+    px, py, g = _inputs(6, S, T, modified, S + T)
+    for b in range(1, 6):  # 1, 4, 16, ... cells of px, or of px and py; utterance 0 stays as it is
+        for x in (px, py)[:1 + b % 2]:
+            flat = x[b].reshape(-1)
+            flat[torch.randint(0, flat.numel(), (4 ** (b - 1),), generator=g)] = value
+    _compare(px, py, None)
+    _compare(px, py, _window(6, S, T, g))
+
+
+@pytest.mark.parametrize("modified", [False, True])
+def test_lattice_without_a_path(modified):
+    px, py, _ = _inputs(3, 90, 120, modified, 3)
+    px[1, 40] = -math.inf  # no way from row 40 to row 41
+    py[2] = -math.inf
+    px[2] = -math.inf
+    _compare(px, py, None)
+
+
+# memory that the scratch is made of may hold anything: cells around the windows must not be felt
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("value", [math.nan, math.inf, -3.0, 3e38])
+def test_what_the_scratch_held_before(modified, value):
+    px, py, g = _inputs(8, 100, 140, modified, 9)
+    boundary = _window(8, 100, 140, g)
+    free = torch.full((4, 8, 101, 141), value, device="cuda")
+    del free
+    want_x, want_y = _compare(px, py, boundary)
+    assert torch.isfinite(want_x).all() and torch.isfinite(want_y).all()
+
+
+@pytest.mark.parametrize("B,S,T", [(6, 40, 150), (6, 80, 250), (8, 100, 900), (8, 250, 700)])
+def test_a_wait_that_runs_out_shows_as_nan(B, S, T):
+    """With the bound of the kernels' waits set from the host: an utterance's score is NaN, or its gradients
+    hold one, unless everything is what it is without a bound."""
+    px, py, _ = _inputs(B, S, T, False, S)
+    px, py = px.cuda(), py.cuda()
+    score, (gx, gy) = F.mutual_information_recursion(px, py, None, return_grad=True)
+    lib = _lib.load()
+    gave_up = 0
+    for polls in (1, 3, 10, 40, 150, 600, 1 << 22):
+        print(f"S={S} T={T} polls={polls}", flush=True)
+        lib.frnnt_set_spin_limit(polls)
+        try:
+            score1, (gx1, gy1) = F.mutual_information_recursion(px, py, None, return_grad=True)
+            torch.cuda.synchronize()
+        finally:
+            lib.frnnt_set_spin_limit(0)
+        for b in range(B):
+            failed = bool(torch.isnan(score1[b]))
+            gave_up += failed
+            if failed:
+                continue
+            assert torch.equal(score1[b], score[b])
+            nan = bool(torch.isnan(gx1[b]).any()), bool(torch.isnan(gy1[b]).any())
+            assert all(nan) or (torch.equal(gx1[b], gx[b]) and torch.equal(gy1[b], gy[b]))
+        assert polls > 1 or gave_up == B
+        assert polls < 1 << 22 or (torch.equal(score1, score) and torch.equal(gx1, gx))
