@@ -167,33 +167,50 @@ __device__ __forceinline__ double from_lane_above(double v) {
 
 // loss = -scores, -mean(scores) or -sum(scores) (rnnt_loss.py:330-340) by ONE wave: every
 // lane sums a contiguous slice, then a fixed butterfly over the lanes.
-template <typename R>
-__device__ __forceinline__ void reduce_scores(const R *__restrict__ scores, R *__restrict__ loss,
-                                              int B, int reduction, int lane) {
+// score(b): utterance b's.
+template <typename R, typename Score>
+__device__ __forceinline__ void reduce_scores(Score score, R *__restrict__ loss, int B, int reduction,
+                                              int lane) {
   if (reduction == 0) {
-    for (int b = lane; b < B; b += kWave) loss[b] = -scores[b];
+    for (int b = lane; b < B; b += kWave) loss[b] = -score(b);
     return;
   }
   const int per = (B + kWave - 1) / kWave;
   R acc = 0;
   for (int k = 0; k < per; ++k) {
     const int b = lane * per + k;
-    if (b < B) acc += scores[b];
+    if (b < B) acc += score(b);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
   if (lane == 0) loss[0] = reduction == 1 ? -(acc / (R)B) : -acc;
 }
+template <typename R>
+__device__ __forceinline__ void reduce_scores(const R *__restrict__ scores, R *__restrict__ loss,
+                                              int B, int reduction, int lane) {
+  reduce_scores([&](int b) { return scores[b]; }, loss, B, reduction, lane);
+}
+
+// The loss that a forward kernel of the recursion is to form of the scores: `arrived` is 0 and *out NaN when
+// it starts (not needed without a reduction).  formed: whether it does; where an utterance's bands have
+// workgroups of their own, or without `arrived`, it does not.
+template <typename R>
+struct LossOf {
+  R *out;
+  int reduction;
+  int *arrived;
+  bool formed;
+};
 
 // The recursion's forward for a caller that goes on to mi_backward_and_loss with `px_grad` (NULL: it
 // does not): what that kernel wants to find there is prepared along with what this one wants.
 // Host side, mi_recursion.hip.
 int mi_forward(const float *px, const float *py, const int64_t *boundary, float *p, float *scores,
                int B, int S, int T, int modified, int checks, int32_t *status, float *px_grad,
-               void *stream);
+               LossOf<float> *loss, void *stream);
 int mi_forward(const double *px, const double *py, const int64_t *boundary, double *p,
                double *scores, int B, int S, int T, int modified, int checks, int32_t *status,
-               double *px_grad, void *stream);
+               double *px_grad, LossOf<double> *loss, void *stream);
 // The backward with a gradient of ones, after such a forward, which, on its way, also reduces the
 // forward's scores to the loss (a staging wave of the first workgroup does it once its
 // tiles are done): saves the launch of a reduction kernel.
@@ -211,6 +228,14 @@ int mi_forward_shares(const float *px, const float *py, const int64_t *boundary,
 int mi_backward_shares(const int64_t *boundary, const float *shares, float *px_grad, float *py_grad,
                        const float *scores, float *loss, int B, int S, int T, int modified,
                        int reduction, void *stream);
+
+// frnnt_mi_loss_fwd; `arrived` as in LossOf (may be NULL).  Host side, simple_loss.hip.
+int mi_loss(const float *px, const float *py, const int64_t *boundary, float *p, float *scores,
+            float *px_grad, float *py_grad, float *loss, int B, int S, int T, int modified, int reduction,
+            int checks, int32_t *status, int *arrived, void *stream);
+int mi_loss(const double *px, const double *py, const int64_t *boundary, double *p, double *scores,
+            double *px_grad, double *py_grad, double *loss, int B, int S, int T, int modified,
+            int reduction, int checks, int32_t *status, int *arrived, void *stream);
 
 // ((T_b - 1) / 2 - t) * delay_penalty, what rnnt_loss.py:309-324 adds to px, rounded as there.
 template <typename R>

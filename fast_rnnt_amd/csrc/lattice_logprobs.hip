@@ -24,6 +24,14 @@ struct Picks {
   R *norm, *xr, *yr, *px, *py;
   Delay<R> delay;
   bool direct;
+  int *arrived;  // (may be NULL) to be 0, and *loss NaN, when the recursion starts (LossOf)
+  R *loss;
+  __device__ __forceinline__ void start() const {
+    if (arrived && (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0) {
+      *arrived = 0;
+      *loss = std::numeric_limits<R>::quiet_NaN();
+    }
+  }
   // the cell (s, t_end) of the regular lattice, and its last column: no symbol is emitted there
   // (rnnt_loss.py:45-63)
   __device__ __forceinline__ void close(const Lattice &L, int b, int s, int t) const {
@@ -142,6 +150,7 @@ __global__ void __launch_bounds__(256)
                     Surround around) {
   constexpr int kAux = kStream ? 2 : 0;
   constexpr int kRows = kWave / kLanes;
+  out.start();
   // (from the last row to the first: the caller has left what it wrote last in the cache)
   const int b = L.B - 1 - block_batch();
   if (b < 0) return;
@@ -332,7 +341,7 @@ template <typename P, typename R>
 int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
              const int64_t *boundary, R *px, R *py, R *norm, R *xr, R *yr, int B, int S, int T,
              int Rr, int C, int term, int rnnt_type, int window_only, double delay_penalty,
-             bool read_again, void *stream_) {
+             bool read_again, int *arrived, R *loss, void *stream_) {
   if (B < 0 || S < 0 || T < 0 || Rr < 1 || C < 1)
     return fail(FRNNT_EINVAL, "lattice_logprobs_fwd: bad size");
   if (Rr > S + 1) return fail(FRNNT_EINVAL, "lattice_logprobs_fwd: more range rows than S + 1");
@@ -352,7 +361,7 @@ int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
   const bool direct = rnnt_type != kConstrained && (!ranges || rows_in_pieces<P>(C));
   if (T > 0)
     launch_row_norm<P, R>(static_cast<const typename P::Elem *>(logits_), L,
-                          Picks<R>{norm, xr, yr, px, py, delay, direct}, read_again, stream);
+                          Picks<R>{norm, xr, yr, px, py, delay, direct, arrived, loss}, read_again, stream);
   const int T1 = rnnt_type == kRegular ? T + 1 : T;
   if (T == 0 && T1 > 0) {
     // no frames: nothing but the closed column
@@ -366,18 +375,23 @@ int fwd_impl(const void *logits_, const int64_t *symbols, const int64_t *ranges,
 }
 
 // A whole loss on logits up to its scores' gradient: px / py, then what every loss shares.
-template <typename P, typename R, typename Tail>
-int loss_fwd_impl(Tail tail, const void *logits, const int64_t *symbols, const int64_t *ranges,
+template <typename P, typename R>
+int loss_fwd_impl(const void *logits, const int64_t *symbols, const int64_t *ranges,
                   const int64_t *boundary, R *px, R *py, R *norm, R *xr, R *yr, R *p, R *scores,
                   R *px_grad, R *py_grad, R *loss, int B, int S, int T, int Rr, int C, int term,
                   int rnnt_type, double delay_penalty, int reduction, int checks, int32_t *status,
                   void *stream) {
+  // the recursion's forward can form the loss if it finds a counter cleared; the rows' picks leave xr to it
+  // where they go to px and py themselves
+  const bool counted = std::is_same<R, float>::value && rnnt_type != kConstrained && T > 0 && loss &&
+                       rows_in_pieces<P>(C);
+  int *arrived = counted ? reinterpret_cast<int *>(xr) : nullptr;
   const int rc = fwd_impl<P, R>(logits, symbols, ranges, boundary, px, py, norm, xr, yr, B, S, T,
                                 Rr, C, term, rnnt_type, boundary != nullptr, delay_penalty,
-                                px_grad != nullptr, stream);
+                                px_grad != nullptr, arrived, loss, stream);
   if (rc != FRNNT_OK) return rc;
-  return tail(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, rnnt_type != kRegular,
-              reduction, checks, status, stream);
+  return mi_loss(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, rnnt_type != kRegular,
+                 reduction, checks, status, arrived, stream);
 }
 
 }  // namespace
@@ -385,14 +399,14 @@ int loss_fwd_impl(Tail tail, const void *logits, const int64_t *symbols, const i
 
 extern "C" {
 
-#define FRNNT_LATTICE_ENTRY(sfx, io, P, R, tail)                                                 \
+#define FRNNT_LATTICE_ENTRY(sfx, io, P, R)                                                       \
   int frnnt_lattice_logprobs_fwd_##sfx(                                                          \
       const io *logits, const int64_t *symbols, const int64_t *ranges, const int64_t *boundary,   \
       R *px, R *py, R *norm, R *xr, R *yr, int B, int S, int T, int Rr, int C,                    \
       int termination_symbol, int rnnt_type, int window_only, void *stream) {                    \
     return frnnt::fwd_impl<frnnt::P, R>(logits, symbols, ranges, boundary, px, py, norm, xr, yr,  \
                                         B, S, T, Rr, C, termination_symbol, rnnt_type,            \
-                                        window_only, 0.0, true, stream);                         \
+                                        window_only, 0.0, true, nullptr, nullptr, stream);                         \
   }                                                                                              \
   int frnnt_lattice_loss_fwd_##sfx(                                                              \
       const io *logits, const int64_t *symbols, const int64_t *ranges, const int64_t *boundary,   \
@@ -400,14 +414,14 @@ extern "C" {
       int B, int S, int T, int Rr, int C, int termination_symbol, int rnnt_type,                 \
       double delay_penalty, int reduction, int checks, int32_t *status, void *stream) {          \
     return frnnt::loss_fwd_impl<frnnt::P, R>(                                                    \
-        tail, logits, symbols, ranges, boundary, px, py, norm, xr, yr, p, scores, px_grad,       \
+        logits, symbols, ranges, boundary, px, py, norm, xr, yr, p, scores, px_grad,             \
         py_grad, loss, B, S, T, Rr, C, termination_symbol, rnnt_type, delay_penalty, reduction,  \
         checks, status, stream);                                                                 \
   }
-FRNNT_LATTICE_ENTRY(f32, float, FloatPiece, float, frnnt_mi_loss_fwd_f32)
-FRNNT_LATTICE_ENTRY(f64, double, DoublePiece, double, frnnt_mi_loss_fwd_f64)
-FRNNT_LATTICE_ENTRY(f16, void, HalfPiece, float, frnnt_mi_loss_fwd_f32)
-FRNNT_LATTICE_ENTRY(bf16, void, Bf16Piece, float, frnnt_mi_loss_fwd_f32)
+FRNNT_LATTICE_ENTRY(f32, float, FloatPiece, float)
+FRNNT_LATTICE_ENTRY(f64, double, DoublePiece, double)
+FRNNT_LATTICE_ENTRY(f16, void, HalfPiece, float)
+FRNNT_LATTICE_ENTRY(bf16, void, Bf16Piece, float)
 #undef FRNNT_LATTICE_ENTRY
 
 }  // extern "C"

@@ -7,9 +7,9 @@ int mi_spin_limit = kSpinLimit;
 
 int mi_forward(const float *px, const float *py, const int64_t *boundary, float *p, float *scores,
                int B, int S, int T, int modified, int checks, int32_t *status, float *px_grad,
-               void *stream) {
+               LossOf<float> *loss, void *stream) {
   return forward_impl<float>(px, py, boundary, p, scores, B, S, T, modified, stream, checks, status,
-                             px_grad);
+                             px_grad, nullptr, loss);
 }
 int mi_backward_and_loss(const float *px, const int64_t *boundary, const float *p, float *px_grad,
                          float *py_grad, const float *scores, float *loss, int B, int S, int T,

@@ -5,9 +5,9 @@ namespace frnnt {
 
 int mi_forward(const double *px, const double *py, const int64_t *boundary, double *p, double *scores,
                int B, int S, int T, int modified, int checks, int32_t *status, double *px_grad,
-               void *stream) {
+               LossOf<double> *loss, void *stream) {
   return forward_impl<double>(px, py, boundary, p, scores, B, S, T, modified, stream, checks, status,
-                             px_grad);
+                             px_grad, nullptr, loss);
 }
 int mi_backward_and_loss(const double *px, const int64_t *boundary, const double *p, double *px_grad,
                          double *py_grad, const double *scores, double *loss, int B, int S, int T,

@@ -16,7 +16,7 @@ template <typename R, typename Reduce>
 int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
                 const int64_t *boundary, R *p, R *scores, R *px_grad, R *py_grad, R *loss, int B,
                 int S, int T, int modified, int reduction, int checks, int32_t *status,
-                void *stream) {
+                int *arrived, void *stream) {
   if ((px_grad == nullptr) != (py_grad == nullptr))
     return fail(FRNNT_EINVAL, "mi_loss_fwd: px_grad and py_grad go together");
   const bool p_wanted = (checks & FRNNT_SCRATCH_P) == 0;
@@ -32,8 +32,10 @@ int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
       return loss ? reduce(scores, loss, B, reduction, stream) : rc;
     }
   }
-  int rc = mi_forward(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad, stream);
-  if (rc != FRNNT_OK) return rc;
+  LossOf<R> formed{loss, reduction, arrived, false};
+  int rc = mi_forward(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad,
+                      px_grad ? nullptr : &formed, stream);
+  if (rc != FRNNT_OK || formed.formed) return rc;
   if (px_grad) {
     // with a loss to form, the backward kernel reduces the scores on its way
     rc = mi_backward_and_loss(px, boundary, p, px_grad, py_grad, scores, loss, B, S, T, modified,
@@ -60,10 +62,24 @@ int simple_loss_fwd(Reduce reduce,
                                      boundary != nullptr, stream);
   if (rc != FRNNT_OK) return rc;
   return mi_loss_fwd<R>(reduce, px, py, boundary, p, scores, px_grad, py_grad,
-                        loss, B, S, T, rnnt_type != kRegular, reduction, checks, status, stream);
+                        loss, B, S, T, rnnt_type != kRegular, reduction, checks, status, nullptr, stream);
 }
 
 }  // namespace
+
+int mi_loss(const float *px, const float *py, const int64_t *boundary, float *p, float *scores,
+            float *px_grad, float *py_grad, float *loss, int B, int S, int T, int modified, int reduction,
+            int checks, int32_t *status, int *arrived, void *stream) {
+  return mi_loss_fwd<float>(frnnt_loss_reduce_f32, px, py, boundary, p, scores, px_grad, py_grad, loss, B,
+                            S, T, modified, reduction, checks, status, arrived, stream);
+}
+int mi_loss(const double *px, const double *py, const int64_t *boundary, double *p, double *scores,
+            double *px_grad, double *py_grad, double *loss, int B, int S, int T, int modified,
+            int reduction, int checks, int32_t *status, int *arrived, void *stream) {
+  return mi_loss_fwd<double>(frnnt_loss_reduce_f64, px, py, boundary, p, scores, px_grad, py_grad, loss,
+                             B, S, T, modified, reduction, checks, status, arrived, stream);
+}
+
 }  // namespace frnnt
 
 extern "C" {
@@ -72,17 +88,15 @@ int frnnt_mi_loss_fwd_f32(const float *px, const float *py, const int64_t *bound
                           float *scores, float *px_grad, float *py_grad, float *loss, int B, int S,
                           int T, int modified, int reduction, int checks, int32_t *status,
                           void *stream) {
-  return frnnt::mi_loss_fwd<float>(frnnt_loss_reduce_f32, px, py, boundary, p, scores, px_grad,
-                                   py_grad, loss, B, S, T, modified, reduction, checks, status,
-                                   stream);
+  return frnnt::mi_loss(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, modified, reduction,
+                        checks, status, nullptr, stream);
 }
 int frnnt_mi_loss_fwd_f64(const double *px, const double *py, const int64_t *boundary, double *p,
                           double *scores, double *px_grad, double *py_grad, double *loss, int B,
                           int S, int T, int modified, int reduction, int checks, int32_t *status,
                           void *stream) {
-  return frnnt::mi_loss_fwd<double>(frnnt_loss_reduce_f64, px, py, boundary, p, scores, px_grad,
-                                    py_grad, loss, B, S, T, modified, reduction, checks, status,
-                                    stream);
+  return frnnt::mi_loss(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, modified, reduction,
+                        checks, status, nullptr, stream);
 }
 
 int frnnt_simple_loss_fwd_f32(const float *lm, const float *am, const int64_t *symbols,
