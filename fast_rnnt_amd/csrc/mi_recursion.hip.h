@@ -986,7 +986,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
                                    kHelpers<kSweepCap, kShares>) * kWave)
     mi_backward_kernel(const R *__restrict__ px, const int64_t *__restrict__ boundary,
                        const R *__restrict__ p, R *ans_grad, R *__restrict__ px_grad,
-                       R *__restrict__ py_grad, int S, int T, int overwrite_ans_grad,
+                       R *__restrict__ py_grad, int S, int T, int seed_stride, int overwrite_ans_grad,
                        const R *__restrict__ scores, R *__restrict__ loss, int B, int reduction,
                        int spin_limit, int pitch) {
   extern __shared__ __align__(16) unsigned char dyn_lds[];
@@ -1009,7 +1009,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   const __amdgpu_buffer_rsrc_t gx_rsrc = buffer_of(gxb, (size_t)S * T1);
   const __amdgpu_buffer_rsrc_t gy_rsrc = buffer_of(gyb, (size_t)(S + 1) * T);
 
-  // Exact zeros everywhere the sweep does not write, by wave `part` of `parts`, off the critical path (a
+  const R seed = ans_grad ? ans_grad[(size_t)b * seed_stride] : (R)1;
+  // Exact zeros everywhere the sweep does not write (0 times the seed: NaN if that is not finite), by wave `part` of `parts`, off the critical path (a
   // barrier after these stores would have to wait until they have all reached memory).  An array's
   // window leaves a run before it, one after it and, all of one length, those between its rows: four rows'
   // to an instruction, 16 lanes each (row by row, with a run's ends tested for each, two waves took
@@ -1017,7 +1018,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   auto zero_run = [&](__amdgpu_buffer_rsrc_t rs, int begin, int end, int first, int lanes) {
     // elements [begin, end), by lanes `first` .. of `lanes` that step through it together; overlapping the
     // last four, so that all stores are whole
-    const R z = 0;
+    const R z = seed - seed;
     if (end - begin < 4) {
       put1(rs, first < end - begin ? (begin + first) * (int)sizeof(R) : kDropped, z);
       return;
@@ -1040,11 +1041,11 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       const int row = r + (lane >> 4), begin = row * width + hi;
       const bool there = row < r_hi - 1;
       if (gap < 4) {
-        put1(rs, there && q < gap ? (begin + q) * (int)sizeof(R) : kDropped, (R)0);
+        put1(rs, there && q < gap ? (begin + q) * (int)sizeof(R) : kDropped, seed - seed);
       } else {
         for (int t = 4 * q; t - 4 * q < gap; t += 64)
-          put4(rs, there && t < gap ? (begin + min(t, gap - 4)) * (int)sizeof(R) : kDropped, (R)0, (R)0, (R)0,
-               (R)0);
+          put4(rs, there && t < gap ? (begin + min(t, gap - 4)) * (int)sizeof(R) : kDropped, seed - seed,
+               seed - seed, seed - seed, seed - seed);
       }
     }
   };
@@ -1480,7 +1481,6 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   R *my_seam = seam + (size_t)w * seam_pitch + kSeamPadLeft;
   const R *up_seam = seam + (size_t)prev * seam_pitch + kSeamPadLeft;
   R *base = tiles + (size_t)w * 2 * kBuffers * kTileElems;
-  const R seed = ans_grad ? ans_grad[b] : (R)1;
   int tile_base = 0, buf = 0, rounds = 0;  // tile number modulo kBuffers, and divided by it
   for (int band = part; band * band_rows <= last_row; ++band) {
     const Band g = band_of(band, w, nsweep, NS, NT);
@@ -1494,7 +1494,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     const int fin_step = (fin_lane < kWave) ? NT + fin_lane : -1;
 
     // the seed enters as "handed left" into the first cell of the reversed sweep
-    R to_below = 0, to_below2 = 0, to_left = (r == 0) ? seed : (R)0;
+    // (a seed that is not finite makes cells that it does not reach NaN as well)
+    R to_below = seed - seed, to_below2 = seed - seed, to_left = (r == 0) ? seed : seed - seed;
     R g_origin = 0;
     const R *seam_at = up_seam + (lane - shift);  // seam_at[e]: what lane 0 needs at step e + lane
     // rows below this wave's: someone reads the seam
@@ -1797,7 +1798,7 @@ template <typename R, bool kShares = false>
 int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p, R *ans_grad,
                   R *px_grad, R *py_grad, int B, int S, int T, int modified,
                   int overwrite_ans_grad, void *stream, const R *scores = nullptr,
-                  R *loss = nullptr, int reduction = 0, bool marked = false) {
+                  R *loss = nullptr, int reduction = 0, bool marked = false, int seed_stride = 1) {
   (void)py;  // the d2 = 1 - d1 split needs only p and px
   if (loss && (!scores || reduction < 0 || reduction > 2))
     return fail(FRNNT_EINVAL, "mi_backward: loss without scores, or bad reduction");
@@ -1833,8 +1834,8 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)),
                          dim3((3 + kFew + kHelpers<1, kShares>) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
-                         py_grad, S, T, overwrite_ans_grad, scores, loss, B, reduction, mi_spin_limit,
-                         pitch);
+                         py_grad, S, T, seed_stride, overwrite_ans_grad, scores, loss, B, reduction,
+                         mi_spin_limit, pitch);
       return check_launch("mi_backward");
     }
   }
@@ -1849,7 +1850,8 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   const int helpers = few ? kHelpers<2, kShares> : kHelpers<kMaxSweep, kShares>;
   hipLaunchKernelGGL(kernel, dim3(B), dim3((n * (1 + stagers) + helpers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
-                     py_grad, S, T, overwrite_ans_grad, scores, loss, B, reduction, mi_spin_limit, B);
+                     py_grad, S, T, seed_stride, overwrite_ans_grad, scores, loss, B, reduction,
+                     mi_spin_limit, B);
   return check_launch("mi_backward");
 }
 

@@ -12,3 +12,14 @@ int mi_backward_shares(const int64_t *boundary, const float *shares, float *px_g
 }
 
 }  // namespace frnnt
+
+extern "C" int frnnt_mi_shares_bwd_f32(const int64_t *boundary, const float *shares,
+                                       const float *score_grad, int score_grad_stride, float *px_grad,
+                                       float *py_grad, int B, int S, int T, int modified, void *stream) {
+  if (score_grad_stride != 0 && score_grad_stride != 1)
+    return frnnt::fail(FRNNT_EINVAL, "mi_shares_bwd: score_grad_stride must be 0 or 1");
+  return frnnt::backward_impl<float, true>(nullptr, nullptr, boundary, shares,
+                                           const_cast<float *>(score_grad), px_grad, py_grad, B, S, T,
+                                           modified, 0, stream, nullptr, nullptr, 0, true,
+                                           score_grad_stride);
+}

@@ -130,6 +130,20 @@ int frnnt_mi_backward_f64(const double *px, const double *py, const int64_t *bou
                           int overwrite_ans_grad, void *stream);
 
 /*
+ * The two as a pair for callers that do not want p (float32; no counterpart in the reference): _fwd leaves
+ * the scores and, in `shares` [B][S+1][T+1], what _bwd needs; arguments otherwise as above.  px_grad
+ * and py_grad are _bwd's outputs; both calls get the same buffers, which nothing else may write to in
+ * between (_fwd prepares them).  _bwd takes utterance b's gradient of its score from
+ * score_grad[b * score_grad_stride] (stride 0 or 1; NULL: 1).
+ */
+int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *shares,
+                            float *scores, float *px_grad, float *py_grad, int B, int S, int T,
+                            int modified, int checks, int32_t *status, void *stream);
+int frnnt_mi_shares_bwd_f32(const int64_t *boundary, const float *shares, const float *score_grad,
+                            int score_grad_stride, float *px_grad, float *py_grad, int B, int S, int T,
+                            int modified, void *stream);
+
+/*
  * px / py of the simple (additive-joiner) RNN-T loss.  Replaces the tensor
  * algebra of get_rnnt_logprobs (fast_rnnt/python/fast_rnnt/rnnt_loss.py:66-227):
  * row maxima, the exp(lm) exp(am)^T contraction (fp32 / fp64 MFMA with the

@@ -121,3 +121,55 @@ def test_a_wait_that_runs_out_shows_as_nan(B, S, T):
             assert all(nan) or (torch.equal(gx1[b], gx[b]) and torch.equal(gy1[b], gy[b]))
         assert polls > 1 or gave_up == B
         assert polls < 1 << 22 or (torch.equal(score1, score) and torch.equal(gx1, gx))
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("B,S,T", [(4, 9, 20), (5, 70, 100), (4, 130, 1200)])
+def test_gradients_formed_in_the_backward(B, S, T, modified):
+    """Without return_grad the occupation gradients are formed in the backward, from the gradient of the
+    scores: against those that are formed in the forward and scaled.  A factor that is a power of two
+    commutes with every rounding but those of subnormal numbers, by 2^-149 per step of a path; another
+    one rounds once per step at most, S + T of them."""
+    px, py, g = _inputs(B, S, T, modified, S)
+    px, py, boundary = px.cuda(), py.cuda(), _window(B, S, T, g).cuda()
+    powers = torch.tensor([-1.0, 0.25, 2.0, 0.0, -4.0])[:B].cuda()
+    anything = torch.randn(B, generator=g).cuda()
+
+    def grads(factor, return_grad):
+        x, y = px.clone().requires_grad_(), py.clone().requires_grad_()
+        out = F.mutual_information_recursion(x, y, boundary, return_grad=return_grad)
+        (out[0] if return_grad else out).backward(factor)
+        return x.grad, y.grad
+
+    for factor in (powers, anything, powers[1:2].expand(B)):
+        want, got = grads(factor, True), grads(factor, False)
+        for w, h in zip(want, got):
+            if factor is anything:
+                assert torch.allclose(h, w, rtol=2 * (S + T) * 2.0 ** -24, atol=1e-37)
+            else:
+                assert torch.allclose(h, w, rtol=0, atol=4 * (S + T) * 2.0 ** -149)
+    for value in (float("nan"), float("inf")):
+        factor = anything.clone()
+        factor[1] = value
+        for w, h in zip(grads(factor, True), grads(factor, False)):
+            assert not torch.isfinite(h[1]).any() and not torch.isfinite(w[1]).any()
+            assert torch.isfinite(h[0]).all()
+
+    x, y = px.clone().requires_grad_(), py.clone().requires_grad_()
+    total = -F.mutual_information_recursion(x, y, boundary).sum()
+    total.backward(retain_graph=True)
+    with pytest.raises(RuntimeError):  # scaled in place, as after the reference's "*="
+        total.backward()
+
+
+def test_gradient_of_a_gradient_formed_in_the_backward():
+    px, py, _ = _inputs(3, 12, 30, False, 5)
+    px, py = px.cuda(), py.cuda()
+    _, (occ_x, _) = F.mutual_information_recursion(px, py, None, return_grad=True)
+    x, y = px.clone().requires_grad_(), py.clone().requires_grad_()
+    weight = torch.tensor([0.5, 1.0, 2.0], device="cuda", requires_grad=True)
+    loss = (weight * F.mutual_information_recursion(x, y)).sum()
+    (gx,) = torch.autograd.grad(loss, x, create_graph=True)
+    assert torch.equal(gx.detach(), occ_x * weight.detach().reshape(-1, 1, 1))
+    (gw,) = torch.autograd.grad(gx.sum(), weight)
+    assert torch.allclose(gw, occ_x.sum(dim=(1, 2)), rtol=1e-5)
