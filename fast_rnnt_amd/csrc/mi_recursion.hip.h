@@ -85,10 +85,17 @@ constexpr int kFetchAhead = sizeof(R) == 4 ? 2 : 1;
 template <int kStagers, bool kShares>
 constexpr int kStagerGroups = kShares && kStagers % 2 == 0 ? 2 : 1;
 
-// Staging waves per sweep wave there, with at most two sweep waves, and waves of a backward workgroup that do what
+// Staging waves per sweep wave there, with two sweep waves, and waves of a backward workgroup that do what
 // is on nobody's way: the zeros around the window and the loss.  (By the staging waves, between two tiles, they
 // held up the sweep for 2 600 - 12 700 cycles.)
 constexpr int kSharesStagers = 6;
+// The same with one sweep wave, where there is room for more: a wave has fewer rows, and so less code to
+// fetch at the start.  6 -> 8, forward and backward, B 8, S 60, T 200: 13.3 + 9.8 -> 12.8 + 9.0 us; B 46, S 47,
+// T 204: 12.0 + 10.6 -> 11.8 + 9.5; B 15, S 33, T 153: 11.3 + 8.6 -> 10.6 + 7.6 (10: 12.6 + 8.8, 12.2 + 9.3,
+// 10.8 + 7.8); in the backward kernel with bands apart, where a wave also hands on the seam, B 12, S 220,
+// T 1500: 50.4 with 6, 49.2 with 8, 46.3 with 10.
+constexpr int kSharesStagersOne = 8;
+constexpr int kSharesStagersApart = 10;
 template <int kSweepCap, bool kShares>
 constexpr int kHelpers = kShares && kSweepCap <= 2 ? 2 : 0;
 constexpr int kSpinLimit = 1 << 22;   // polls before a wait gives up (seconds, not microseconds)
@@ -1658,7 +1665,9 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       return true;
     };
     bool done;
-    if (has_up)
+    if constexpr (!kApart && kSweepCap == 1)  // (lattices of one band)
+      done = sweep_tiles(std::false_type{}, std::false_type{});
+    else if (has_up)
       done = has_down ? sweep_tiles(std::true_type{}, std::true_type{})
                       : sweep_tiles(std::true_type{}, std::false_type{});
     else
@@ -1757,6 +1766,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   // wave's two tile rows of doubles no longer fit its share of the registers)
   constexpr int kMany = sizeof(R) == 4 ? kFwdStagers : 2;
   constexpr int kFew = kShares ? kSharesStagers : sizeof(R) == 4 ? kFwdStagersFew : 2;
+  constexpr int kOne = kShares ? kSharesStagersOne : kFew;  // with one sweep wave
   if constexpr (sizeof(R) == 4) {
     const bool apart = bands_apart<R>(B, S, T, false), later = px_grad && bands_apart<R>(B, S, T, true);
     if (apart || later)
@@ -1765,21 +1775,21 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
     if (apart) {
       const int pitch = (B + 7) / 8 * 8;  // (an utterance's bands on one XCD)
       const size_t lds = apart_lds_bytes(T);
-      auto kernel = modified ? mi_forward_kernel<R, true, 1, kFew, kApartBuffers, true, kShares>
-                             : mi_forward_kernel<R, false, 1, kFew, kApartBuffers, true, kShares>;
+      auto kernel = modified ? mi_forward_kernel<R, true, 1, kOne, kApartBuffers, true, kShares>
+                             : mi_forward_kernel<R, false, 1, kOne, kApartBuffers, true, kShares>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_forward: hipFuncSetAttribute");
-      hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kFew) * kWave), lds,
+      hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kOne) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T,
                          mi_spin_limit, checks, status, B, pitch, py_grad, nullptr, 0, nullptr);
       return check_launch("mi_forward");
     }
   }
-  const int stagers = few ? kFew : kMany;
-  const size_t lds = lds_bytes(n, T, few ? kFewBuffers : 2, sizeof(R));
   const bool one_band = few && S + 1 <= kWave;
-  auto kernel = one_band ? (modified ? mi_forward_kernel<R, true, 1, kFew, kFewBuffers, false, kShares>
-                                     : mi_forward_kernel<R, false, 1, kFew, kFewBuffers, false, kShares>)
+  const int stagers = one_band ? kOne : few ? kFew : kMany;
+  const size_t lds = lds_bytes(n, T, few ? kFewBuffers : 2, sizeof(R));
+  auto kernel = one_band ? (modified ? mi_forward_kernel<R, true, 1, kOne, kFewBuffers, false, kShares>
+                                     : mi_forward_kernel<R, false, 1, kOne, kFewBuffers, false, kShares>)
               : few      ? (modified ? mi_forward_kernel<R, true, 2, kFew, kFewBuffers, false, kShares>
                                      : mi_forward_kernel<R, false, 2, kFew, kFewBuffers, false, kShares>)
                          : (modified ? mi_forward_kernel<R, true, kMaxSweep, kMany, 2, false, kShares>
@@ -1817,6 +1827,8 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   // registers, too few for a sweep wave's two tile rows of doubles.)
   constexpr bool kFloat = sizeof(R) == 4;
   constexpr int kFew = kShares ? kSharesStagers : kFloat ? kBwdStagersFew : kBwdStagers;
+  constexpr int kOne = kShares ? kSharesStagersOne : kFew;  // with one sweep wave
+  constexpr int kAlone = kShares ? kSharesStagersApart : kFew;  // bands apart
   constexpr int kFewBuffers = kFloat ? 3 : 2;
   static_assert(kMaxSweep * 2 <= 16 && 2 * kFewBuffers <= 16, "Counters::loaded is too short");
   const bool few = n <= 2 && lds_bytes(n, T, kFewBuffers, sizeof(R)) <= kLdsBudget;
@@ -1827,21 +1839,25 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
                    static_cast<hipStream_t>(stream));
       const int pitch = (B + 7) / 8 * 8;
       const size_t lds = apart_lds_bytes(T);
-      auto kernel = modified ? mi_backward_kernel<R, true, 1, kFew, kApartBuffers, true, kShares>
-                             : mi_backward_kernel<R, false, 1, kFew, kApartBuffers, true, kShares>;
+      auto kernel = modified ? mi_backward_kernel<R, true, 1, kAlone, kApartBuffers, true, kShares>
+                             : mi_backward_kernel<R, false, 1, kAlone, kApartBuffers, true, kShares>;
       if (!allow_lds(reinterpret_cast<const void *>(kernel), lds))
         return check_launch("mi_backward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)),
-                         dim3((3 + kFew + kHelpers<1, kShares>) * kWave), lds,
+                         dim3((3 + kAlone + kHelpers<1, kShares>) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
                          py_grad, S, T, seed_stride, overwrite_ans_grad, scores, loss, B, reduction,
                          mi_spin_limit, pitch);
       return check_launch("mi_backward");
     }
   }
-  const int stagers = few ? kFew : kBwdStagers;
+  const bool one_band = kShares && few && S + 1 <= kWave;
+  const int stagers = one_band ? kOne : few ? kFew : kBwdStagers;
   const size_t lds = lds_bytes(n, T, few ? kFewBuffers : 2, sizeof(R));
-  auto kernel = few ? (modified ? mi_backward_kernel<R, true, 2, kFew, kFewBuffers, false, kShares>
+  constexpr int kOneCap = kShares ? 1 : 2;  // (without shares: the kernel for two)
+  auto kernel = one_band ? (modified ? mi_backward_kernel<R, true, kOneCap, kOne, kFewBuffers, false, kShares>
+                                     : mi_backward_kernel<R, false, kOneCap, kOne, kFewBuffers, false, kShares>)
+              : few ? (modified ? mi_backward_kernel<R, true, 2, kFew, kFewBuffers, false, kShares>
                                 : mi_backward_kernel<R, false, 2, kFew, kFewBuffers, false, kShares>)
                     : (modified ? mi_backward_kernel<R, true, kMaxSweep, kBwdStagers, 2, false, kShares>
                                 : mi_backward_kernel<R, false, kMaxSweep, kBwdStagers, 2, false, kShares>);
