@@ -52,6 +52,7 @@ _SIGNATURES = {
     "frnnt_simple_loss_fwd_f64": ([_P] * 14 + [_I] * 8 + [_P, _P], _I),
     "frnnt_additive_loss_fwd": ([_I] + [_P] * 16 + [_I] * 6 + [_D, _I, _I, _P, _P], _I),
     "frnnt_additive_loss_bwd": ([_I] + [_P] * 8 + [_I, _D] + [_P] * 8 + [_I] * 6 + [_P], _I),
+    "frnnt_loss_scratch": ([_I] * 5, ctypes.c_int64),
     "frnnt_mi_shares_fwd_f32": ([_P] * 7 + [_I] * 5 + [_P, _P], _I),
     "frnnt_mi_shares_bwd_f32": ([_P] * 3 + [_I] + [_P] * 2 + [_I] * 4 + [_P], _I),
     "frnnt_mi_loss_fwd_f32": ([_P] * 8 + [_I] * 6 + [_P, _P], _I),

@@ -1040,14 +1040,14 @@ __device__ __forceinline__ void simple_bwd_am_body(
 void launch_fwd_gemm(const float *lm, const float *am, const int64_t *symbols,
                      const int64_t *boundary, float *lm_max, float *am_max, float *px,
                      float *py, float *norm_raw, const int64_t *window, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
-                     const SmoothMix *mix, hipStream_t stream) {
+                     const SmoothMix *mix, float *workspace, hipStream_t stream) {
   launch_normalizer_f32(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw, window,
-                        delay_penalty, B, S, T, C, term, rnnt_type, mix, stream);
+                        delay_penalty, B, S, T, C, term, rnnt_type, mix, workspace, stream);
 }
 void launch_fwd_gemm(const double *lm, const double *am, const int64_t *symbols,
                      const int64_t *boundary, const double *lm_max, const double *am_max,
                      double *px, double *py, double *norm_raw, const int64_t *, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type,
-                     const SmoothMix *, hipStream_t stream) {
+                     const SmoothMix *, float *, hipStream_t stream) {
   // (the double kernels compute the whole lattice whether or not a window is given)
   const int t_tiles = T > 0 ? (T + kTileN - 1) / kTileN : 1;
   const dim3 grid(t_tiles, (S + 1 + kTileM - 1) / kTileM, B);
@@ -1184,7 +1184,7 @@ template <typename R>
 int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *boundary, R *px,
              R *py, R *lm_max, R *am_max, R *norm_raw, double delay_penalty, int B,
              int S, int T, int C, int term, int rnnt_type, int window_only, void *stream_,
-             const SmoothMix *mix = nullptr) {
+             const SmoothMix *mix = nullptr, float *workspace = nullptr) {
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_fwd: bad size");
   if (rnnt_type < 0 || rnnt_type > 2)
     return fail(FRNNT_EINVAL, "simple_logprobs_fwd: rnnt_type must be 0, 1 or 2");
@@ -1209,7 +1209,7 @@ int fwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
   const bool constrained = rnnt_type == kConstrained;
   launch_fwd_gemm(lm, am, symbols, boundary, lm_max, am_max, px, py, norm_raw,
                   window_only ? boundary : nullptr, constrained ? 0.0 : delay_penalty, B,
-                  S, T, C, term, rnnt_type, mix, stream);
+                  S, T, C, term, rnnt_type, mix, workspace, stream);
   if (constrained && S > 0 && T > 0) {
     const long total = (long)B * S * T;
     hipLaunchKernelGGL(add_next_row_kernel<R>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
@@ -1355,9 +1355,9 @@ float *own_scratch_address() {
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
                         float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
-                        void *stream, const SmoothMix *mix) {
+                        void *stream, const SmoothMix *mix, float *workspace) {
   return fwd_impl<float>(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                         delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream, mix);
+                         delay_penalty, B, S, T, C, term, rnnt_type, window_only, stream, mix, workspace);
 }
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
@@ -1459,6 +1459,13 @@ int frnnt_simple_logprobs_bwd_noalloc_f32(const float *lm, const float *am, cons
                                 score_grad_stride, score_grad_scale, px_grad, py_grad, dmat, row_x,
                                 row_y, col_y, lm_grad, am_grad, B, S, T, C, termination_symbol,
                                 rnnt_type, window_only, FRNNT_F32, stream);
+}
+
+int64_t frnnt_loss_scratch(int B, int S, int T, int C, int has_boundary) {
+  if (B < 1 || S < 0 || T < 0 || C < 1) return 0;
+  const long lattice = (long)B * (S + 1) * (T + 1);
+  const long work = frnnt::normalizer_workspace(B, S, T, C, has_boundary != 0);
+  return lattice > work ? lattice : work;
 }
 
 int frnnt_simple_logprobs_fwd_f32(const float *lm, const float *am, const int64_t *symbols,

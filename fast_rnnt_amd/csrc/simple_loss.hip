@@ -20,7 +20,7 @@ int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
   if ((px_grad == nullptr) != (py_grad == nullptr))
     return fail(FRNNT_EINVAL, "mi_loss_fwd: px_grad and py_grad go together");
   const bool p_wanted = (checks & FRNNT_SCRATCH_P) == 0;
-  checks &= ~FRNNT_SCRATCH_P;
+  checks &= ~(FRNNT_SCRATCH_P | FRNNT_LARGE_SCRATCH);
   if constexpr (std::is_same<R, float>::value) {
     if (px_grad && !p_wanted) {
       int rc = mi_forward_shares(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad,
@@ -57,9 +57,14 @@ int simple_loss_fwd(Reduce reduce,
     return fail(FRNNT_EINVAL, "simple_loss_fwd: px_grad and py_grad go together");
   // px / py only feed the recursion below, with the same boundary: what lies outside an
   // utterance's window need not be computed
-  const int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw,
-                                     delay_penalty, B, S, T, C, term, rnnt_type,
-                                     boundary != nullptr, stream);
+  int rc;
+  if constexpr (std::is_same<R, float>::value)
+    rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, delay_penalty, B,
+                             S, T, C, term, rnnt_type, boundary != nullptr, stream, nullptr,
+                             checks & FRNNT_LARGE_SCRATCH ? p : nullptr);
+  else
+    rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, lm_max, am_max, norm_raw, delay_penalty, B,
+                             S, T, C, term, rnnt_type, boundary != nullptr, stream);
   if (rc != FRNNT_OK) return rc;
   return mi_loss_fwd<R>(reduce, px, py, boundary, p, scores, px_grad, py_grad,
                         loss, B, S, T, rnnt_type != kRegular, reduction, checks, status, nullptr, stream);

@@ -2,6 +2,7 @@
 // log(P + tiny) written from its accumulators (rnnt_loss.py:66-227; the formulas are at the
 // top of simple_logprobs.hip).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 
 #include "common.hip.h"
@@ -46,10 +47,10 @@ constexpr int kNormK = 16;      // k per slab
 constexpr int kNormShares = 8;  // of k
 constexpr int kNormT = 32;      // frames of a tile
 constexpr int kComputeUnits = 256;
-template <int kS, int kWaves_>
+template <int kS, int kWaves_, int kParts_>
 struct NormShape {
-  static constexpr int kWaves = kWaves_, kThreads = kWaves * kWave;
-  static constexpr int kTurns = kNormShares / kWaves;  // shares of a wave, one after the other
+  static constexpr int kWaves = kWaves_, kParts = kParts_, kThreads = kWaves * kWave;
+  static constexpr int kTurns = kNormShares / kParts / kWaves;  // shares of a wave, one after the other
   static constexpr int kRows = kS + kNormT;      // rows of a slab: lm rows, then am rows
   static constexpr int kLoads = kRows / 16;      // 16-byte loads per lane and slab
   // Row pitch in LDS: 20 floats.  Rows start 16-byte aligned, so a lane's four values of a row go
@@ -59,7 +60,9 @@ struct NormShape {
   static constexpr int kSlab = kRows * kPitch;   // floats
   // the partial sums of the waves meet in the slabs' space
   static constexpr int kSumPitch = kNormT + 4;
-  static constexpr int kSums = kWaves * kS * kSumPitch;
+  static constexpr int kSums = kParts > 1 ? 0 : kWaves * kS * kSumPitch;
+  // of a tile, in the workspace: every share's partial sums, then its row maxima and final shifts
+  static constexpr int kPartial = kS * kNormT + 2 * kRows;
   static constexpr size_t kLdsBytes = std::max(kWaves * kSlab, kSums) * 4;
   static constexpr int kItems =  // 16-byte outputs per thread
       (kS * kNormT / 4 + kThreads - 1) / kThreads;
@@ -160,6 +163,9 @@ struct NormArgs {
   float *lm_max, *am_max, *px, *py, *norm_raw;
   Delay<float> delay;
   int B, S, T, C, term, rnnt_type;
+  unsigned long long *met;    // (tiles in parts) a word per tile, holding anything
+  float *partial;             // kNormShares * kPartial floats per tile
+  unsigned long long ticket;  // an even number that no other call has had
 };
 
 // A joint model on its own
@@ -177,11 +183,14 @@ __device__ __forceinline__ void with_tiles(int n, F &f) {
 // With a Mix (the smoothed loss) px and py leave interpolated with the lm-only and the am-only model:
 // am[t,sym[s]] and what depends on a row or a frame alone are here already, and a launch of its own for
 // the interpolation would read and write every cell again (B 32, S 80, T 250, C 500: 12.8 us).
-template <int kS, int kWaves, typename Mix>
-__global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / kWaves : 1))
+//
+// kParts = 2: two workgroups share a tile, four of k's shares each.  They leave their partial sums in a
+// workspace; the one that comes second brings all together, in the one order that there is.
+template <int kS, int kWaves, int kParts, typename Mix>
+__global__ void __launch_bounds__(kWaves *kWave, (kWaves / 4 * NormShape<kS, kWaves, kParts>::kPerCu))
     simple_fwd_panel_kernel(NormArgs A, NormPlan plan, Mix mix) {
   constexpr bool kMix = !std::is_same_v<Mix, NoMix>;
-  using Shape = NormShape<kS, kWaves>;
+  using Shape = NormShape<kS, kWaves, kParts>;
   constexpr int kT = kNormT, kShares = kNormShares, kTurns = Shape::kTurns;
   constexpr int kRows = Shape::kRows, kLoads = Shape::kLoads, kLmLoads = kS / 16;
   constexpr int kThreads = Shape::kThreads, kItems = Shape::kItems, kPitch = Shape::kPitch;
@@ -198,8 +207,11 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   const int S = A.S, T = A.T, C = A.C, S1 = S + 1;
   NormTile tile;
   const int tid = threadIdx.x, lane = tid & 63;
-  if (plan.all ? !number_tile((int)blockIdx.x, plan, A.B, tile)
-               : !find_tile<kS>((int)blockIdx.x, plan, A.window, A.B, S, T, lane, tile))
+  // (a tile's parts on one XCD, one after the other)
+  const int part = kParts > 1 ? (int)blockIdx.x / kXcds % kParts : 0;
+  const int id = kParts > 1 ? (int)blockIdx.x / (kXcds * kParts) * kXcds + (int)blockIdx.x % kXcds : (int)blockIdx.x;
+  if (plan.all ? !number_tile(id, plan, A.B, tile)
+               : !find_tile<kS>(id, plan, A.window, A.B, S, T, lane, tile))
     return;
   const int b = tile.b, s_tile = tile.s_idx * kS, t_tile = tile.t_idx * kT;
   const int T1 = A.rnnt_type == kRegular ? T + 1 : T;
@@ -266,7 +278,8 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   // meet their partial sums are brought to the true maxima, exp(shift - max) <= 1.
   constexpr float kMargin = 30.f;
   floatx4 slab[kLoads];
-  if (wave < chunks) fetch(std::integral_constant<int, kS / 32>{}, slab, wave * kNormK);
+  const int first_share = part * kWaves + wave;
+  if (first_share < chunks) fetch(std::integral_constant<int, kS / 32>{}, slab, first_share * kNormK);
   if (plan.all) {
     tile.lim = limits_of(A.window, b, S, T);
     if (t_tile > 0 && t_tile > tile.lim.t_end) return;
@@ -389,7 +402,7 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
     return above;
   };
   auto walk_share = [&](auto live, auto q) {
-    const int share = wave + kWaves * q;
+    const int share = first_share + kWaves * q;
     int chunk = share;
     if (chunk < chunks) {  // the first slab sets the shifts: there are no sums to bring along yet
       (void)look(live, q);
@@ -441,16 +454,57 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
 
   // ---- the waves meet: maxima first (each wave's in what was its slab: the row maxima over its
   // share of k, then its final shifts) ...
+  // (tiles in parts) Both parts' sums go through the workspace, past the XCDs' own L2: a share's cells, then
+  // what follows; a part that finds the other's ticket in the tile's word comes second.  (What the word held
+  // before is no ticket of this call: a call's ticket is its own, and a replay of a recorded call finds the 0
+  // that the second part leaves.)
+  const long tile_id = ((long)b * plan.t_tiles + tile.t_idx) * plan.s_tiles + tile.s_idx;
+  float *const met = kParts > 1 ? A.partial + tile_id * (kNormShares * Shape::kPartial) : nullptr;
+  const __amdgpu_buffer_rsrc_t met_rs = buffer_of(met, kNormShares * Shape::kPartial * 4);
+  constexpr int kAgent = 16;  // sc1: device scope
+  if constexpr (kParts > 1) {
+    const int at = first_share * Shape::kPartial;
 #pragma unroll
-  for (int q = 0; q < kTurns; ++q)
+    for (int j = 0; j < kS / 32; ++j) {
+      if (j >= live_tiles) break;  // (uniform)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        __builtin_amdgcn_raw_buffer_store_b32(
+            __float_as_int(acc[0][j][v]), met_rs,
+            4 * (at + (32 * j + 8 * (v / 4) + 4 * half + (v % 4)) * kT + r32), 0, kAgent);
+    }
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      const float top = across_row(seen[q][j]);
-      if (lane % 4 == 0) {
-        mine[2 * kRows * q + sub + 16 * j] = top;
-        mine[2 * kRows * q + kRows + sub + 16 * j] = shift2[q][j];
-      }
+      const float top = across_row(seen[0][j]);
+      const int to = lane % 4 == 0 ? 4 * (at + kS * kT + sub + 16 * j) : kNowhere;
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(top), met_rs, to, 0, kAgent);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(shift2[0][j]), met_rs, to, 4 * kRows, kAgent);
     }
+    __shared__ int second;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): they have arrived
+    asm volatile("" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      unsigned long long *word = A.met + tile_id;
+      second = __hip_atomic_exchange(word, A.ticket + part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               A.ticket + (1 - part);
+      if (second) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!second) return;
+  } else {
+#pragma unroll
+    for (int q = 0; q < kTurns; ++q)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const float top = across_row(seen[q][j]);
+        if (lane % 4 == 0) {
+          mine[2 * kRows * q + sub + 16 * j] = top;
+          mine[2 * kRows * q + kRows + sub + 16 * j] = shift2[q][j];
+        }
+      }
+  }
   // (all of wave 2, whose first lanes own the frames)
   const float check = kMix && __any(mix_max != mix_max) ? std::numeric_limits<float>::quiet_NaN() : 0.f;
   if (tid < kS) {
@@ -476,12 +530,21 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   float *lm_max = A.lm_max + (long)b * S1, *am_max = A.am_max + (long)b * T;
   if (tid < kRows) {
     const int row = tid;
-    auto met_by = [&](int share, int i) {
-      return norm_lds[share % kWaves * Shape::kSlab + share / kWaves * 2 * kRows + i];
-    };
-    float r = met_by(0, row);
+    float tops[kShares], shifts[kShares];
 #pragma unroll
-    for (int w = 1; w < kShares; ++w) r = fmaxf(r, met_by(w, row));
+    for (int w = 0; w < kShares; ++w) {
+      if constexpr (kParts > 1) {
+        const int at = 4 * (w * Shape::kPartial + kS * kT + row);
+        tops[w] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(met_rs, at, 0, kAgent));
+        shifts[w] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(met_rs, at, 4 * kRows, kAgent));
+      } else {
+        const float *met_by = norm_lds + w % kWaves * Shape::kSlab + w / kWaves * 2 * kRows + row;
+        tops[w] = met_by[0], shifts[w] = met_by[kRows];
+      }
+    }
+    float r = tops[0];
+#pragma unroll
+    for (int w = 1; w < kShares; ++w) r = fmaxf(r, tops[w]);
     // saved for the backward pass; rows that do not exist get a harmless shift
     bool exists;
     if (row < kS) {
@@ -496,7 +559,7 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
     // nothing finite in the row holds zeros there)
 #pragma unroll
     for (int w = 0; w < kShares; ++w)
-      factor[w][row] = exists ? __builtin_amdgcn_exp2f(-__builtin_fmaf(r, kLog2e, met_by(w, kRows + row))) : 1.f;
+      factor[w][row] = exists ? __builtin_amdgcn_exp2f(-__builtin_fmaf(r, kLog2e, shifts[w])) : 1.f;
   }
   __syncthreads();
   // ... then the partial sums: [wave][kS][kSumPitch] in the slab space, a share of every wave at a time
@@ -508,30 +571,48 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   floatx4 sums[kItems];
 #pragma unroll
   for (int j = 0; j < kItems; ++j) sums[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int q = 0; q < kTurns; ++q) {
-    if (q > 0) __syncthreads();
-    float *part = norm_lds + wave * kS * kSumPitch;
-    const float *my_factor = factor[wave + kWaves * q];
-    const float ft = my_factor[kS + r32];
-#pragma unroll
-    for (int j = 0; j < kS / 32; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = 32 * j + 8 * (v / 4) + 4 * half + (v % 4);
-        part[m * kSumPitch + r32] = acc[q][j][v] * (my_factor[m] * ft);
-      }
-    __syncthreads();
+  if constexpr (kParts > 1) {
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
       const int m = item_row(j);
       if (m >= kS) continue;
+      intx4 one[kShares];
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const floatx4 one =
-            *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + m) * kSumPitch + out_t);
+      for (int w = 0; w < kShares; ++w)
+        one[w] = __builtin_amdgcn_raw_buffer_load_b128(met_rs, 4 * (m * kT + out_t), 4 * w * Shape::kPartial,
+                                                       kAgent);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[j][i] += one[i];
+      for (int w = 0; w < kShares; ++w)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          sums[j][i] += __int_as_float(one[w][i]) * (factor[w][m] * factor[w][kS + out_t + i]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < kTurns; ++q) {
+      if (q > 0) __syncthreads();
+      float *part = norm_lds + wave * kS * kSumPitch;
+      const float *my_factor = factor[wave + kWaves * q];
+      const float ft = my_factor[kS + r32];
+#pragma unroll
+      for (int j = 0; j < kS / 32; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = 32 * j + 8 * (v / 4) + 4 * half + (v % 4);
+          part[m * kSumPitch + r32] = acc[q][j][v] * (my_factor[m] * ft);
+        }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kItems; ++j) {
+        const int m = item_row(j);
+        if (m >= kS) continue;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          const floatx4 one =
+              *reinterpret_cast<const floatx4 *>(norm_lds + (w * kS + m) * kSumPitch + out_t);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sums[j][i] += one[i];
+        }
       }
     }
   }
@@ -586,28 +667,45 @@ __global__ void __launch_bounds__(kWaves *kWave, kWaves / 4 * (kS <= 64 ? 16 / k
   }
 }
 
-template <int kS, int kWaves, typename Mix>
-void launch_fwd_panel(const NormArgs &args, const NormPlan &plan, const Mix &mix, hipStream_t stream) {
-  auto kernel = simple_fwd_panel_kernel<kS, kWaves, Mix>;
-  constexpr size_t lds = NormShape<kS, kWaves>::kLdsBytes;
+template <int kS, int kWaves, int kParts, typename Mix>
+void launch_fwd_panel(NormArgs args, const NormPlan &plan, const Mix &mix, float *workspace, hipStream_t stream) {
+  using Shape = NormShape<kS, kWaves, kParts>;
+  auto kernel = simple_fwd_panel_kernel<kS, kWaves, kParts, Mix>;
+  constexpr size_t lds = Shape::kLdsBytes;
   if (!allow_lds(reinterpret_cast<const void *>(kernel), lds)) return;
   const long tiles = (long)args.B * plan.t_tiles * plan.s_tiles;
-  const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NormShape<kS, kWaves>::kThreads), lds, stream, args, plan,
-                     mix);
+  const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds * kParts);
+  if (kParts > 1) {
+    // The memory may hold anything, also small whole numbers: above a count of the calls, a ticket has the bits
+    // of a signalling NaN that no arithmetic forms.
+    static std::atomic<unsigned long long> calls{0};
+    args.ticket = 0xffa5c3ull << 40 | (2 * calls.fetch_add(1, std::memory_order_relaxed) & ((1ull << 40) - 1));
+    args.met = reinterpret_cast<unsigned long long *>(workspace);
+    args.partial = workspace + (2 * tiles + 3) / 4 * 4;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Shape::kThreads), lds, stream, args, plan, mix);
 }
 
 struct NormChoice {
   int rows, waves;  // of a tile
   bool all;         // its numbering: see number_tile
+  int parts = 1;    // workgroups that share it
 };
 // The tile that a call takes.  `windowed`: what lies outside an utterance's window does not count.
-NormChoice choose_tile(int B, int S, int T, int C, bool windowed) {
+NormChoice choose_tile(int B, int S, int T, int C, bool windowed, bool workspace) {
   const long t_tiles = T > 0 ? (T + kNormT - 1) / kNormT : 1;
   const int s_tiles = (S + 32) / 32;
   const long tiles = B * t_tiles * s_tiles;
   const int rounds = (C + kNormShares * kNormK - 1) / (kNormShares * kNormK);
   auto taller = [&](int rows) { return B * t_tiles * ((S + rows) / rows); };
+  // Batches that leave half of the compute units without a tile, and loops of some length: two workgroups
+  // share a tile, which moves half of its waves to an idle unit (B 2, S 44, T 287, C 5194, 36 tiles: 35.7 -> 27.9
+  // us; B 4, S 28, T 186, C 3806, 24: 28.1 -> 21.9; B 2, S 114, T 463, C 3713, 120: 29.7 -> 24.1; B 8, S 15, T 84,
+  // C 1961, 24: 17.4 -> 15.1; B 1, S 90, T 299, C 838, 30: 11.6 -> 10.1).  With shorter loops, or as many tiles as
+  // there are units, the way through the workspace costs more than it gives (B 49, S 8, T 51, C 654, 98
+  // tiles: 9.8 -> 11.3; B 49, S 17, T 130, C 1219, 245: 16.3 -> 17.3; B 53, S 24, T 116, C 2485, 212: 23.4 -> 27.1;
+  // B 6, S 152, T 415, C 2803, 390: 42.9 -> 51.2).
+  if (workspace && 2 * tiles <= kComputeUnits && rounds >= 7) return {32, 4, true, 2};
   // Four waves of two shares let four workgroups share a compute unit, whose prologues and epilogues
   // hide under each other's loops; eight of one share end a workgroup sooner.  The former pay where
   // a compute unit has several workgroups in turn and their loops are short (B 64, S 120, T 600,
@@ -664,32 +762,41 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                            const int64_t *boundary, float *lm_max, float *am_max, float *px,
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
-                           int rnnt_type, const SmoothMix *mix, hipStream_t stream) {
+                           int rnnt_type, const SmoothMix *mix, float *workspace, hipStream_t stream) {
   const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
-                      Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type};
-  const NormChoice choice = choose_tile(B, S, T, C, window != nullptr);
+                      Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type, nullptr, nullptr, 0};
+  const NormChoice choice = choose_tile(B, S, T, C, window != nullptr, workspace != nullptr);
   const NormPlan plan{T > 0 ? (T + kNormT - 1) / kNormT : 1, (S + choice.rows) / choice.rows, choice.all};
   auto launch = [&](const auto &m) {
-    if (choice.rows == 96)
-      launch_fwd_panel<96, 8>(args, plan, m, stream);
+    if (choice.parts > 1)
+      launch_fwd_panel<32, 4, 2>(args, plan, m, workspace, stream);
+    else if (choice.rows == 96)
+      launch_fwd_panel<96, 8, 1>(args, plan, m, nullptr, stream);
     else if (choice.rows == 64)
-      launch_fwd_panel<64, 8>(args, plan, m, stream);
+      launch_fwd_panel<64, 8, 1>(args, plan, m, nullptr, stream);
     else if (choice.waves == 4)
-      launch_fwd_panel<32, 4>(args, plan, m, stream);
+      launch_fwd_panel<32, 4, 1>(args, plan, m, nullptr, stream);
     else
-      launch_fwd_panel<32, 8>(args, plan, m, stream);
+      launch_fwd_panel<32, 8, 1>(args, plan, m, nullptr, stream);
   };
   if (mix)
     launch(*mix);
   else
     launch(NoMix{});
 }
+long normalizer_workspace(int B, int S, int T, int C, bool windowed) {
+  const NormChoice choice = choose_tile(B, S, T, C, windowed, true);
+  if (choice.parts == 1) return 0;
+  const long tiles = (long)B * (T > 0 ? (T + kNormT - 1) / kNormT : 1) * ((S + choice.rows) / choice.rows);
+  return (2 * tiles + 3) / 4 * 4 +
+         tiles * kNormShares * ((long)choice.rows * kNormT + 2 * (choice.rows + kNormT));
+}
 }  // namespace frnnt
 
 extern "C" int frnnt_simple_logprobs_tile(int B, int S, int T, int C, int window_only, int *waves) {
   using namespace frnnt;
   if (B < 1 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "simple_logprobs_tile: bad size");
-  const NormChoice choice = choose_tile(B, S, T, C, window_only != 0);
+  const NormChoice choice = choose_tile(B, S, T, C, window_only != 0, false);
   if (waves) *waves = choice.waves;
   return choice.rows;
 }

@@ -148,13 +148,15 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                            const int64_t *boundary, float *lm_max, float *am_max, float *px,
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
-                           int rnnt_type, const SmoothMix *mix, hipStream_t stream);
+                           int rnnt_type, const SmoothMix *mix, float *workspace, hipStream_t stream);
+// Floats of the workspace that it takes at this size, 0 if it needs none; without one it does without.
+long normalizer_workspace(int B, int S, int T, int C, bool windowed);
 
 // frnnt_simple_logprobs_fwd with the delay penalty (simple_logprobs.hip).
 int simple_logprobs_fwd(const float *lm, const float *am, const int64_t *symbols,
                         const int64_t *boundary, float *px, float *py, float *lm_max,
                         float *am_max, float *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,
-                        void *stream, const SmoothMix *mix = nullptr);
+                        void *stream, const SmoothMix *mix = nullptr, float *workspace = nullptr);
 int simple_logprobs_fwd(const double *lm, const double *am, const int64_t *symbols,
                         const int64_t *boundary, double *px, double *py, double *lm_max,
                         double *am_max, double *norm_raw, double delay_penalty, int B, int S, int T, int C, int term, int rnnt_type, int window_only,

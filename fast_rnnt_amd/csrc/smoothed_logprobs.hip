@@ -992,7 +992,8 @@ int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t 
                       am_model ? (float)am_only_scale : 0.f, blocks};
   const int rc = simple_logprobs_fwd(lm, am, symbols, boundary, px, py, k.lm_max, k.am_max, k.norm_raw,
                                      delay_penalty > 0.0 ? delay_penalty : 0.0, B, S, T, C,
-                                     termination_symbol, rnnt_type, boundary != nullptr, stream, &mix);
+                                     termination_symbol, rnnt_type, boundary != nullptr, stream, &mix,
+                                     checks & FRNNT_LARGE_SCRATCH ? p : nullptr);
   if (rc != FRNNT_OK) return rc;
   return frnnt_mi_loss_fwd_f32(px, py, boundary, p, scores, px_grad, py_grad, loss, B, S, T, !regular,
                                reduction, checks | FRNNT_SCRATCH_P, status, stream);

@@ -558,8 +558,10 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
     Tensor kept = at::empty({keep.total}, opts);
     // what it does not: px | py | p | scores
     Carver carve;
-    const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(n_py),
-                  o_p = carve.take(B * (S + 1) * (T + 1)), o_sc = carve.take(B);
+    const int64_t n_p = dtype == FRNNT_F64 ? B * (S + 1) * (T + 1)
+                                           : frnnt_loss_scratch((int)B, (int)S, (int)T, (int)C, bnd.defined());
+    const int64_t o_px = carve.take(B * S * T1), o_py = carve.take(n_py), o_p = carve.take(n_p),
+                  o_sc = carve.take(B);
     const Tensor work = at::empty({carve.total}, opts);
     char *k = static_cast<char *>(kept.data_ptr()), *w = static_cast<char *>(work.data_ptr());
     Tensor gx, gy;
@@ -575,7 +577,8 @@ struct SimpleLossFn : public torch::autograd::Function<SimpleLossFn> {
                  need_grad ? k + o_nr * item : nullptr, w + o_p * item, w + o_sc * item,
                  gx.defined() ? gx.data_ptr() : nullptr, gy.defined() ? gy.data_ptr() : nullptr,
                  loss.data_ptr(), (int)B, (int)S, (int)T, (int)C,
-                 (int)term, (int)kind, delay_penalty, (int)reduction, (int)checks | FRNNT_SCRATCH_P,
+                 (int)term, (int)kind, delay_penalty, (int)reduction,
+                 (int)checks | FRNNT_SCRATCH_P | FRNNT_LARGE_SCRATCH,
                  status_for(am, bnd), stream_of(am)),
              "frnnt_additive_loss_fwd");
     if (need_grad) {
@@ -698,7 +701,8 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
     const int64_t n_px = B * S * T1, n_py = B * (S + 1) * T;
     Carver carve;
     const int64_t o_px = carve.take(n_px),
-                  o_py = carve.take(n_py), o_p = carve.take(B * (S + 1) * (T + 1)),
+                  o_py = carve.take(n_py),
+                  o_p = carve.take(frnnt_loss_scratch((int)B, (int)S, (int)T, (int)C, bnd.defined())),
                   o_sc = carve.take(B), o_part = carve.take((B * (S + 1) + 15) / 16 * C);
     const Tensor work = at::empty({carve.total}, opts);
     float *w = work.data_ptr<float>();
@@ -712,8 +716,8 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
                  ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), nullptr, nullptr, w + o_px,
                  w + o_py, ptr<float>(kept), w + o_part, w + o_p, w + o_sc, ptr<float>(gx),
                  ptr<float>(gy), ptr<float>(loss), (int)B, (int)S, (int)T, (int)C, (int)term,
-                 (int)kind, lm_scale, am_scale, delay_penalty, (int)reduction, (int)checks,
-                 status_for(am, bnd), stream_of(am)),
+                 (int)kind, lm_scale, am_scale, delay_penalty, (int)reduction,
+                 (int)checks | FRNNT_LARGE_SCRATCH, status_for(am, bnd), stream_of(am)),
              "frnnt_smoothed_loss_fwd");
     if (need_grad) {
       variable_list save{lm, am, sym, kept, gx, gy};

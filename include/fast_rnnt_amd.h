@@ -386,6 +386,12 @@ int frnnt_additive_loss_bwd(int dtype, const void *lm, const void *am, const int
  * shares of the cells' gradients from the forward to the backward there; the same results, faster).
  */
 #define FRNNT_SCRATCH_P 0x100
+/*
+ * Beside it, in the additive losses: that buffer has frnnt_loss_scratch() floats (the lattice's and more),
+ * with which their float32 product can share a tile among workgroups.  The same results.
+ */
+#define FRNNT_LARGE_SCRATCH 0x400
+int64_t frnnt_loss_scratch(int B, int S, int T, int C, int has_boundary);
 int frnnt_mi_loss_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *p,
                           float *scores, float *px_grad, float *py_grad, float *loss, int B, int S,
                           int T, int modified, int reduction, int checks, int32_t *status,
