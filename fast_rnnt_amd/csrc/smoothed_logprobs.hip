@@ -493,14 +493,16 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// G[b,t] = sum_s (gx + gy) of the scaled gradients, for the fused loss: 64 frames per block, eight waves
+// G[b,t] = sum_s (x_weight gx + gy) of the scaled gradients, for the fused loss (x_weight 2: the constrained
+// lattice, where the py of a row went into the px of the row above as well): 64 frames per block, eight waves
 // of which take every eighth lattice row of the window, eight of them requested together (B 32, S 80,
 // T 250: 4.1 us; 6.0 with the row sums, which the preparation of the products forms anyway, beside them).
 constexpr int kFrameSumWaves = 8;
 __global__ void __launch_bounds__(kFrameSumWaves *kWave)
     frame_sums_kernel(const float *__restrict__ gpx, const float *__restrict__ gpy,
                       const int64_t *__restrict__ boundary, const float *__restrict__ score_grad,
-                      int stride, float scale, float *__restrict__ col_g, int S, int T, int T1) {
+                      int stride, float scale, float x_weight, float *__restrict__ col_g, int S, int T,
+                      int T1) {
   __shared__ float part[kFrameSumWaves][kWave];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.y, t = (int)blockIdx.x * kWave + lane, S1 = S + 1;
@@ -520,7 +522,7 @@ __global__ void __launch_bounds__(kFrameSumWaves *kWave)
       y[u] = get_float(gy_rs, in && s <= lim.s_end, 4 * t, s * T * 4);
     }
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) sum += x[u] + y[u];
+    for (int u = 0; u < kAhead; ++u) sum += x_weight * x[u] + y[u];
   }
   part[wave][lane] = sum;
   __syncthreads();
@@ -966,8 +968,8 @@ int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t 
                                 double lm_only_scale, double am_only_scale, double delay_penalty,
                                 int reduction, int checks, int32_t *status, void *stream) {
   using namespace frnnt;
-  if (rnnt_type != kRegular && rnnt_type != kModified)
-    return fail(FRNNT_EINVAL, "smoothed_loss_fwd: rnnt_type must be 0 or 1");
+  if (rnnt_type < kRegular || rnnt_type > kConstrained)
+    return fail(FRNNT_EINVAL, "smoothed_loss_fwd: rnnt_type must be 0, 1 or 2");
   if (B > 0 && !kept) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: null pointer");
   if (B < 0 || S < 0 || T < 0 || C < 1) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: bad size");
   if (B > 0 && (!lm || !partial || (!am && T > 0))) return fail(FRNNT_EINVAL, "smoothed_loss_fwd: null pointer");
@@ -1006,7 +1008,7 @@ int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t 
                                 double lm_only_scale, double am_only_scale, void *stream_) {
   using namespace frnnt;
   if (B < 0 || S < 0 || T < 0 || C < 1 || termination_symbol < 0 || termination_symbol >= C ||
-      (rnnt_type != kRegular && rnnt_type != kModified) ||
+      rnnt_type < kRegular || rnnt_type > kConstrained ||
       (score_grad_stride != 0 && score_grad_stride != 1))
     return fail(FRNNT_EINVAL, "smoothed_loss_bwd: bad size or type");
   if (B == 0) return FRNNT_OK;
@@ -1034,7 +1036,8 @@ int frnnt_smoothed_loss_bwd_f32(const float *lm, const float *am, const int64_t 
   if (am_model && n_am > 0)
     hipLaunchKernelGGL(frame_sums_kernel, dim3((T + kWave - 1) / kWave, B),
                        dim3(kFrameSumWaves * kWave), 0, stream, px_grad, py_grad, boundary, score_grad,
-                       score_grad_stride, (float)score_grad_scale, col_g, S, T, T1);
+                       score_grad_stride, (float)score_grad_scale, rnnt_type == kConstrained ? 2.f : 1.f, col_g,
+                       S, T, T1);
   const SmoothTerms smooth{col_g,     k.am_z, k.unigram,
                            k.s_lm_max, k.lm_sum, dot,
                            g_unigram, am_model ? k_am : 0.f, k_joint + k_am,

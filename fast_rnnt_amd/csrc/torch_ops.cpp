@@ -680,7 +680,7 @@ LossResult simple_loss(const Tensor &lm, const Tensor &am, const Tensor &symbols
                                        need_am));
 }
 
-// ---- rnnt_loss_smoothed behind one autograd node (float32; regular and modified lattices) -----
+// ---- rnnt_loss_smoothed behind one autograd node (float32) -----------------------------------
 // forward = frnnt_smoothed_loss_fwd, backward = frnnt_smoothed_loss_bwd: the joint model's node
 // above with the lm-only and am-only models' terms folded into its kernels.
 struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
@@ -770,7 +770,7 @@ LossResult smoothed_loss(const Tensor &lm, const Tensor &am, const Tensor &symbo
   require_float_gpu(am, "am");
   TORCH_CHECK(am.scalar_type() == at::kFloat, "smoothed_loss takes float32 tensors");
   check_additive(lm, am, symbols, or_undefined(boundary_));
-  TORCH_CHECK(rnnt_type == 0 || rnnt_type == 1, "rnnt_type must be 0 or 1");
+  TORCH_CHECK(rnnt_type >= 0 && rnnt_type <= 2, "rnnt_type must be 0, 1 or 2");
   TORCH_CHECK(reduction >= 0 && reduction <= 2, "reduction must be 0 (none), 1 (mean) or 2 (sum)");
   const bool need_grad = at::GradMode::is_enabled() && (lm.requires_grad() || am.requires_grad());
   return as_result(SmoothedLossFn::apply(lm, am, symbols, boundary_, termination_symbol, rnnt_type,

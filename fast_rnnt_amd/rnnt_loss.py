@@ -725,7 +725,7 @@ def rnnt_loss_smoothed(
     delay_penalty: float = 0.0, reduction: Optional[str] = "mean", return_grad: bool = False,
 ) -> Union[Tuple[Tensor, Tuple[Tensor, Tensor]], Tensor]:
     """rnnt_loss_simple with lm-only / am-only smoothing (rnnt_loss.py:1372-1494)."""
-    if rnnt_type != "constrained" and am.dtype in (torch.float32, *_NARROW):
+    if am.dtype in (torch.float32, *_NARROW):
         # one autograd node of the operator module
         checks = _device_checks(rnnt_type, boundary)
         _check_smoothed(lm, am, symbols, boundary, rnnt_type, checks)

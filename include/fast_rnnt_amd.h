@@ -294,8 +294,7 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
                                     double am_only_scale, void *stream);
 
 /*
- * rnnt_loss_smoothed (rnnt_loss.py:1372-1494) in float32 for the regular and the modified lattice
- * (rnnt_type 0, 1): _fwd forms the statistics of the two unigram models, then px and py,
+ * rnnt_loss_smoothed (rnnt_loss.py:1372-1494) in float32: _fwd forms the statistics of the two unigram models, then px and py,
  * interpolated and with the delay penalty, as frnnt_simple_logprobs_fwd does (window_only when a boundary
  * is given), and chains frnnt_mi_loss_fwd; an am_only_scale below 1e-19 (the reference's 1e-20 for 0)
  * means no am-only model.  _bwd scales px_grad
