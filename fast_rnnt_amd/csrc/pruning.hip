@@ -9,8 +9,8 @@
 // T_b - 1 by max(S_b - R + 1, 0), then make the starts non-decreasing, starting
 // at 0, with steps smaller than r (r = R for the regular lattice, 2 otherwise)
 // by two suffix-minimum passes.  Two kernels: one lane per frame for the window
-// starts (left in ranges[b][t][0]), then one wave per utterance for the two passes,
-// with the starts in LDS and the suffix minima as a chunked wave scan.
+// starts (left in ranges[b][t][0]), then one workgroup per utterance for the two passes,
+// with the starts in LDS and the suffix minima as a chunked scan.
 //
 // prune_gather (rnnt_loss.py:780-818): lm_pruned[b,t,j,:] = lm[b, ranges[b,t,j], :]
 // and its adjoint, a deterministic segmented sum (one block per lm row).
@@ -21,31 +21,22 @@
 namespace frnnt {
 namespace {
 
-// suffix minimum of v[0..n) in place; v in LDS, one wave
-__device__ __forceinline__ void suffix_min_inplace(int *v, int n, int lane) {
-  const int per = (n + kWave - 1) / kWave;
-  const int lo = lane * per, hi = min(n, lo + per);
-  int local = INT_MAX;
-  for (int k = hi - 1; k >= lo; --k) local = min(local, v[k]);
-  // minimum over all chunks to the right of this lane's chunk
-  int right = INT_MAX;
-  {
-    int acc = local;  // inclusive suffix scan over lanes
+constexpr int kMonotoneThreads = 256, kMonotoneWaves = kMonotoneThreads / kWave;
+// the minimum over the threads above this one; `totals` (kMonotoneWaves ints of LDS) is its own
+__device__ __forceinline__ int min_of_threads_above(int v, int *totals, int wave, int lane) {
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int o = __shfl_down(acc, off, kWave);
-      if (lane + off < kWave) acc = min(acc, o);
-    }
-    const int next = __shfl_down(acc, 1, kWave);
-    right = (lane + 1 < kWave) ? next : INT_MAX;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int o = __shfl_down(v, off, kWave);
+    if (lane + off < kWave) v = min(v, o);
   }
+  if (lane == 0) totals[wave] = v;
+  const int next = __shfl_down(v, 1, kWave);
+  int above = lane + 1 < kWave ? next : INT_MAX;
   __syncthreads();
-  int run = right;
-  for (int k = hi - 1; k >= lo; --k) {
-    run = min(run, v[k]);
-    v[k] = run;
-  }
-  __syncthreads();
+#pragma unroll
+  for (int w = 1; w < kMonotoneWaves; ++w)
+    if (w > wave) above = min(above, totals[w]);
+  return above;
 }
 
 // The sum of the s_range values of one window, in the order in which the reference's
@@ -130,12 +121,14 @@ __global__ void __launch_bounds__(kWave)
 
 // The same with the columns of py_grad and px_grad of 32 frames staged in LDS first: every
 // load of the tile is in flight at once (the kernel above walks the rows with a few loads
-// in flight), and eight groups of 32 threads share the candidate starts, each scanning a
-// contiguous eighth; the first group then takes the others' winners in order under the same
-// rule, which is the sequential scan's result.  Bound by the latency of its loads and of the
-// scan; tiles of 32 frames fill the chip at the batches of training where 64 left half of it
-// idle (B 32, S 80, T 250: 14.5 -> 9.6 us).
-constexpr int kStartFrames = 32, kStartGroups = 8;
+// in flight), and sixteen groups of 32 threads share the candidate starts, each scanning a
+// contiguous sixteenth, four candidates side by side; the first group then takes the others' winners in
+// order under the same rule, which is the sequential scan's result.  Bound by the latency of its loads and of
+// the scan: tiles of 32 frames fill the chip at the batches of training where 64 left half of it
+// idle (B 32, S 80, T 250: 14.5 -> 9.6 us), and sixteen groups with four candidates side by side wait less than
+// eight with one, whose window is a chain of LDS reads (that size: 9.2 -> 6.4 us; B 6, S 250, T 1357: 19.2 ->
+// 12.3, 1.3 TB/s).
+constexpr int kStartFrames = 32, kStartGroups = 16, kStartAhead = 4;
 template <typename R>
 __global__ void __launch_bounds__(kStartFrames *kStartGroups)
     prune_starts_tile_kernel(const R *__restrict__ px_grad, const R *__restrict__ py_grad,
@@ -154,6 +147,7 @@ __global__ void __launch_bounds__(kStartFrames *kStartGroups)
   const int t_read = ok ? t : T - 1;
   const R *gx = px_grad + (long)b * S * T1 + t_read;
   const R *gy = py_grad + (long)b * (S + 1) * T + t_read;
+  const int64_t Sb = boundary[4 * b + 2], Tb = boundary[4 * b + 3];
   for (int s0 = group; s0 <= S; s0 += 8 * kStartGroups) {
     R v[8], x[8];
 #pragma unroll
@@ -179,37 +173,87 @@ __global__ void __launch_bounds__(kStartFrames *kStartGroups)
       best_score = score;
     }
   };
-  for (int s = lo; s < hi; ++s) {
-    const R sum = window_sum<R>(Rr, [&](int j) { return ty[(s + j) * kStartFrames + frame]; });
-    const R below = s >= 1 ? tx[(s - 1) * kStartFrames + frame] : (R)0;
-    consider(s, sum - below);
+  if (Rr <= 16) {  // (window_sum's plain order)
+    const R *lower = S > 0 ? tx : ty;  // (no row of px_grad at all)
+    for (int s0 = lo; s0 < hi; s0 += kStartAhead) {
+      R sum[kStartAhead], below[kStartAhead];
+#pragma unroll
+      for (int u = 0; u < kStartAhead; ++u) {
+        sum[u] = ty[min(s0 + u, S) * kStartFrames + frame];
+        below[u] = lower[min(max(s0 + u - 1, 0), max(S - 1, 0)) * kStartFrames + frame];
+      }
+      for (int j = 1; j < Rr; ++j) {
+        R v[kStartAhead];
+#pragma unroll
+        for (int u = 0; u < kStartAhead; ++u) v[u] = ty[min(s0 + u + j, S) * kStartFrames + frame];
+#pragma unroll
+        for (int u = 0; u < kStartAhead; ++u) sum[u] = sum[u] + v[u];
+      }
+#pragma unroll
+      for (int u = 0; u < kStartAhead; ++u)
+        if (s0 + u < hi) consider(s0 + u, sum[u] - (s0 + u >= 1 ? below[u] : (R)0));
+    }
+  } else {
+    for (int s = lo; s < hi; ++s) {
+      const R sum = window_sum<R>(Rr, [&](int j) { return ty[(s + j) * kStartFrames + frame]; });
+      const R below = s >= 1 ? tx[(s - 1) * kStartFrames + frame] : (R)0;
+      consider(s, sum - below);
+    }
   }
   seg_best[group][frame] = best;
   seg_score[group][frame] = best_score;
   __syncthreads();
   if (group != 0 || !ok) return;
+  int others[kStartGroups];
+  R scores[kStartGroups];
+#pragma unroll
+  for (int w = 1; w < kStartGroups; ++w) others[w] = seg_best[w][frame], scores[w] = seg_score[w][frame];
+#pragma unroll
   for (int w = 1; w < kStartGroups; ++w)
-    if (seg_best[w][frame] >= 0) consider(seg_best[w][frame], seg_score[w][frame]);
-  const int64_t Sb = boundary[4 * b + 2], Tb = boundary[4 * b + 3];
+    if (others[w] >= 0) consider(others[w], scores[w]);
   int64_t tail = Sb - Rr + 1;
   if (tail < 0) tail = 0;
   ranges[((long)b * T + t) * Rr] = ((int64_t)t < Tb - 1) ? (int64_t)best : tail;
 }
 
-// Step 2, one wave per utterance: the starts are made non-decreasing with bounded
-// steps by two suffix-minimum passes and expanded to the R entries of each frame.
-__global__ void __launch_bounds__(kWave)
+// Step 2, a workgroup per utterance: the starts are made non-decreasing with bounded
+// steps by two suffix-minimum passes and expanded to the R entries of each frame.  A thread owns a run of
+// frames in both passes.  Bound by latency: a wave per utterance, whose loads went one after the other, took 4.8
+// us at B 32, T 250 (4.2 now) and 16.1 at B 6, T 1357 (6.9).
+__global__ void __launch_bounds__(kMonotoneThreads)
     prune_monotone_kernel(int64_t *__restrict__ ranges, int T, int r, int Rr) {
   extern __shared__ int start[];  // [T]
-  const int b = blockIdx.x, lane = threadIdx.x;
+  __shared__ int totals[2][kMonotoneWaves];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int64_t *rb = ranges + (long)b * T * Rr;
-  for (int t = lane; t < T; t += kWave) start[t] = (int)rb[(long)t * Rr];
+  for (int t0 = tid; t0 < T; t0 += 4 * kMonotoneThreads) {
+    int v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = (int)rb[(long)min(t0 + u * kMonotoneThreads, T - 1) * Rr];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (t0 + u * kMonotoneThreads < T) start[t0 + u * kMonotoneThreads] = v[u];
+  }
   __syncthreads();
-  suffix_min_inplace(start, T, lane);
-  for (int t = lane; t < T; t += kWave) start[t] = (r - 1) * t - start[t];
+  const int per = (T + kMonotoneThreads - 1) / kMonotoneThreads, lo = tid * per, hi = min(T, lo + per);
+  int least = INT_MAX;
+  for (int k = hi - 1; k >= lo; --k) least = min(least, start[k]);
+  int run = min_of_threads_above(least, totals[0], wave, lane);
+  least = INT_MAX;
+  for (int k = hi - 1; k >= lo; --k) {
+    run = min(run, start[k]);
+    const int y = (r - 1) * k - run;
+    start[k] = y;
+    least = min(least, y);
+  }
+  run = min_of_threads_above(least, totals[1], wave, lane);
+  for (int k = hi - 1; k >= lo; --k) {
+    run = min(run, start[k]);
+    start[k] = run;
+  }
   __syncthreads();
-  suffix_min_inplace(start, T, lane);
-  for (int t = lane; t < T; t += kWave) {
+  for (int t = tid; t < T; t += kMonotoneThreads) {
     const int y = max(start[t], 0);
     const int64_t s0 = (int64_t)(r - 1) * t - y;
     int64_t *out = rb + (long)t * Rr;
@@ -684,7 +728,7 @@ int ranges_impl(const R *px_grad, const R *py_grad, const int64_t *boundary, int
     hipLaunchKernelGGL(prune_starts_kernel<R>, dim3((T + kWave - 1) / kWave, B), dim3(kWave), 0,
                        static_cast<hipStream_t>(stream), px_grad, py_grad, boundary, ranges, S, T,
                        T1, s_range);
-  hipLaunchKernelGGL(prune_monotone_kernel, dim3(B), dim3(kWave), lds,
+  hipLaunchKernelGGL(prune_monotone_kernel, dim3(B), dim3(kMonotoneThreads), lds,
                      static_cast<hipStream_t>(stream), ranges, T, modified ? 2 : s_range, s_range);
   return check_launch("prune_ranges");
 }
