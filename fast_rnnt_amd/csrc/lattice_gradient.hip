@@ -156,6 +156,123 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// For short rows, kIter of them per lane group, in steps of four a wave: what a row's gradient needs besides the row,
+// a chain of dependent loads, is fetched for all rows of a wave at once, a lane per row, beside the pieces, which are
+// all requested first.
+// Bound by the latency of the loads of the waves that fit: float16, C 302, five rows a frame, B 34, T 1028: 81 -> 61
+// us; float32, B 32, T 500, C 256: 32.4 -> 26.0 (5.5 TB/s); B 64, T 300, C 128: 23.2 -> 18.3; bfloat16, B 128, T 200,
+// C 80: 18.4 -> 14.1; B 32, T 250, C 500: 22.8 -> 21.7.  Rows of two pieces a lane have enough in flight without
+// (float32, C 500: 143.8 -> 152.3 at B 100, T 500; bfloat16, C 1000: 26.2 -> 31.7), and few rows do not fill the chip
+// (bfloat16, B 8, T 100, C 500: 5.6 -> 7.0; float32, B 16, T 150, C 60: 4.9 -> 5.2).
+template <int kLanes, int kAt>
+__device__ __forceinline__ void of_rows(float x, float (&v)[kLanes / 16]) {
+  // (in lane kAt of the quarters)
+  if constexpr (kLanes == 64)
+    to_rows<64>(x, v, kAt);
+  else
+    to_rows<kLanes>(__int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x150 + kAt, 0xf, 0xf, true)), v);
+}
+template <typename P, int kLanes, int kVecs, int kIter, bool kStream, bool kAligned>
+__global__ void __launch_bounds__(256)
+    row_grad_rows_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Grads<float> in,
+                         typename P::Elem *__restrict__ glogits) {
+  constexpr int kAux = kStream ? 2 : 0;
+  constexpr int kRows = kWave / kLanes, kN = kRows * kIter, kSteps = 4 / kRows;
+  static_assert(kN % 4 == 0 && kN <= 8, "of_rows");
+  const int b = block_batch();
+  if (b >= L.B) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register
+  const int at = threadIdx.x & 63, lane = at & (kLanes - 1);
+  const unsigned r0 = (blockIdx.x * 4 + wave) * kN, rows = (unsigned)(L.T * L.Rr);
+  if (r0 >= rows) return;
+  // this lane's row: of the fours, number at % 16
+  const bool mine = at % 16 < kN / 4;
+  Row row = placed_in_frame(L, b, r0 + (mine ? 4 * (at % 16) + row_of_quarter(at / 16) : 0));
+  // (a row whose range begins outside the window is read all the same)
+  const unsigned long long there = __ballot(mine && row.live);
+  const long first = (long)b * L.T * L.Rr + r0;
+  const uintptr_t base = wave_base<P, kLanes>(logits, first, L.C);
+  const uintptr_t gbase = wave_base<P, kLanes>(glogits, first, L.C);
+  const long bytes = ((long)kN * L.C * (long)sizeof(typename P::Elem) + 31) & ~15L;
+  const __amdgpu_buffer_rsrc_t in_rs = resource(base, bytes), out_rs = resource(gbase, bytes);
+  intx4 raw[kIter][kVecs];
+  RowPieces<P, kLanes> q[kIter];
+  auto number = [&](int n) {
+    return kRows * n + (kRows == 4 ? row_of_quarter(at / 16) : kRows == 2 ? at / 32 : 0);
+  };
+  auto bit_of = [&](unsigned long long mask, int nth) {
+    return (int)(mask >> (16 * row_of_quarter(nth % 4) + nth / 4) & 1);
+  };
+#pragma unroll
+  for (int n = 0; n < kIter; ++n) {
+    const int nth = number(n);
+    q[n] = pieces_of<P, kLanes>(base, reinterpret_cast<uintptr_t>(logits + (first + nth) * L.C), L.C);
+    if (kAligned) q[n].off = 0, q[n].whole = q[n].pieces = L.C / P::kPer;
+    const int wanted = bit_of(there, nth);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      const int p = lane + kLanes * i;
+      raw[n][i] = __builtin_amdgcn_raw_buffer_load_b128(
+          in_rs, wanted & (int)(p < q[n].pieces) ? q[n].at + 16 * p : kOutOfRange, 0, kAux);
+    }
+  }
+  place(L, row);
+  RowScalars<float> mine_k{0.f, 0.f, 0.f, -1};
+  float my_w = 0.f;  // (exact zeros for a row that does not count: its pieces are 0 as well)
+  if (mine && row.live) {
+    mine_k = in.of(L, row);
+    my_w = -(mine_k.gx + mine_k.gy);
+  }
+  const unsigned long long live = __ballot(mine && row.live);
+  auto four = [&](auto which) {
+    constexpr int kAt = which;
+    float gx[kSteps], gy[kSteps], lse[kSteps], w[kSteps], sym[kSteps];
+    of_rows<kLanes, kAt>(mine_k.gx, gx);
+    of_rows<kLanes, kAt>(mine_k.gy, gy);
+    of_rows<kLanes, kAt>(mine_k.lse, lse);
+    of_rows<kLanes, kAt>(my_w, w);
+    of_rows<kLanes, kAt>(__int_as_float(mine_k.sym), sym);
+#pragma unroll
+    for (int m = 0; m < kSteps; ++m) {
+      const int n = kAt * kSteps + m, nth = number(n);
+      const bool inside = r0 + nth < rows;
+      const bool counts = bit_of(live, nth) != 0;
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i) {
+        const int first_piece = kLanes * i, p = first_piece + lane, c = p * P::kPer - q[n].off;
+        const intx4 x = counts ? raw[n][i] : intx4{0, 0, 0, 0};
+        float v[P::kPer];
+#pragma unroll
+        for (int e = 0; e < P::kPer; ++e) {
+          v[e] = __expf(P::at(x, e) - lse[m]) * w[m];
+          if (c + e == __float_as_int(sym[m])) v[e] += gx[m];
+          if (c + e == L.term) v[e] += gy[m];
+        }
+        const intx4 o = P::pack(v);
+        const bool whole = inside && p < q[n].whole && (p > 0 || q[n].off == 0);
+        __builtin_amdgcn_raw_buffer_store_b128(o, out_rs, whole ? q[n].at + 16 * p : kOutOfRange, 0, kAux);
+        // pieces shared with a neighbouring row, if this vector holds any
+        const bool ragged = (first_piece == 0 && q[n].off != 0) ||
+                            (q[n].pieces > q[n].whole && (unsigned)(q[n].whole - first_piece) < kLanes);
+        if (!kAligned && (kRows > 1 || ragged)) {
+#pragma unroll
+          for (int e = 0; e < P::kPer; ++e) {
+            const bool own = inside && !whole && (unsigned)(c + e) < (unsigned)L.C;
+            const int to = own ? q[n].at + 16 * p + e * (int)sizeof(typename P::Elem) : kOutOfRange;
+            if (sizeof(typename P::Elem) == 4)
+              __builtin_amdgcn_raw_buffer_store_b32(o[e & 3], out_rs, to, 0, kAux);
+            else
+              __builtin_amdgcn_raw_buffer_store_b16((short)((unsigned)o[e >> 1] >> (16 * (e & 1))), out_rs, to, 0,
+                                                    kAux);
+          }
+        }
+      }
+    }
+  };
+  four(std::integral_constant<int, 0>{});
+  if constexpr (kN > 4) four(std::integral_constant<int, 1>{});
+}
+
 template <typename P, typename R>
 void launch_row_grad(const typename P::Elem *logits, const Lattice &L, const Grads<R> &in,
                      typename P::Elem *glogits, hipStream_t stream) {
@@ -165,6 +282,23 @@ void launch_row_grad(const typename P::Elem *logits, const Lattice &L, const Gra
         ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(glogits)) & 15) == 0) {
       const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) > kStreamBytes;
       with_row_split<P>(logits, L.C, [&](auto lanes, auto vecs, auto loop) {
+        if constexpr (vecs == 1 && !loop) {
+          constexpr int kIter = lanes == 16 ? 2 : 4, kRowsOfBlock = kIter * 256 / lanes;
+          if (several_rows(rows * L.B, kRowsOfBlock)) {
+            auto launch = [&](auto stream_hint, auto aligned) {
+              hipLaunchKernelGGL((row_grad_rows_kernel<P, lanes, vecs, kIter, stream_hint, aligned>),
+                                 batch_grid((rows + kRowsOfBlock - 1) / kRowsOfBlock, L.B), dim3(256), 0, stream,
+                                 logits, L, in, glogits);
+            };
+            constexpr std::integral_constant<bool, lanes == 64> hint;
+            if (big)
+              rows_aligned<P>(logits, L.C) ? launch(hint, std::true_type{}) : launch(hint, std::false_type{});
+            else
+              rows_aligned<P>(logits, L.C) ? launch(std::false_type{}, std::true_type{})
+                                           : launch(std::false_type{}, std::false_type{});
+            return;
+          }
+        }
         const dim3 grid = batch_grid((rows + 256 / lanes - 1) / (256 / lanes), L.B);
         auto launch = [&](auto stream_hint, auto aligned) {
           hipLaunchKernelGGL((row_grad_kernel<P, lanes, vecs, loop, stream_hint, aligned>), grid,

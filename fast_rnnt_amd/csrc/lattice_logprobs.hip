@@ -144,6 +144,45 @@ struct Surround {
   }
 };
 
+// What of a row's pieces (the vectors from piece p0 on) is a neighbour's becomes -inf (whole pieces of a whole
+// wave need no test; kAligned: no piece is shared); the largest entry of a lane's pieces, without the NaNs, which
+// come back through the sum.
+template <typename P, int kLanes, int kVecs, bool kAligned = false>
+__device__ __forceinline__ float largest_of_lane(intx4 (&raw)[kVecs], const RowPieces<P, kLanes> &q, int p0,
+                                                 int lane, int C) {
+#pragma unroll
+  for (int i = 0; i < kVecs; ++i) {
+    const int first_piece = p0 + kLanes * i;
+    if (kLanes == kWave && first_piece + kLanes <= q.whole && (first_piece > 0 || q.off == 0)) continue;
+    if (kAligned) {
+      intx4 none = {};
+#pragma unroll
+      for (int e = 0; e < P::kPer; ++e) P::drop(none, e);
+      raw[i] = first_piece + lane < q.pieces ? raw[i] : none;
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < P::kPer; ++e)
+      if ((unsigned)((first_piece + lane) * P::kPer + e - q.off) >= (unsigned)C) P::drop(raw[i], e);
+  }
+  float here = -__builtin_huge_valf();
+#pragma unroll
+  for (int i = 0; i < kVecs; ++i)
+#pragma unroll
+    for (int e = 0; e < P::kPer; e += 2)
+      here = max3_raw(P::at(raw[i], e), P::at(raw[i], e + 1), here);
+  // (the pieces stay packed: unpacked twice rather than kept as floats)
+#pragma unroll
+  for (int i = 0; i < kVecs; ++i)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      int word = raw[i][w];
+      asm("" : "+v"(word));
+      raw[i][w] = word;
+    }
+  return here;
+}
+
 template <typename P, int kLanes, int kVecs, bool kLoop, bool kStream>
 __global__ void __launch_bounds__(256)
     row_norm_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out,
@@ -177,32 +216,8 @@ __global__ void __launch_bounds__(256)
       const bool wanted = (kRows == 1 || row.live) && p < q.pieces;
       raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, wanted ? q.at + 16 * p : kOutOfRange, 0, kAux);
     }
-    // entries that are not the row's become -inf (whole pieces of a whole wave need no test)
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-      const int first_piece = p0 + kLanes * i;
-      if (kRows == 1 && first_piece + kLanes <= q.whole && (first_piece > 0 || q.off == 0)) continue;
-#pragma unroll
-      for (int e = 0; e < P::kPer; ++e)
-        if ((unsigned)((first_piece + lane) * P::kPer + e - q.off) >= (unsigned)L.C)
-          P::drop(raw[i], e);
-    }
-    float here = ninf;
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i)
-#pragma unroll
-      for (int e = 0; e < P::kPer; e += 2)
-        here = max3_raw(P::at(raw[i], e), P::at(raw[i], e + 1), here);
-    // (the pieces stay packed: unpacked twice rather than kept as floats)
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i)
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        int word = raw[i][w];
-        asm("" : "+v"(word));
-        raw[i][w] = word;
-      }
-    here = group_max(here, kLanes);
+    const float here = over_group(largest_of_lane<P, kLanes>(raw, q, p0, lane, L.C), kLanes,
+                                  [](float a, float b) { return max3_raw(a, b, b); });
     if (kLoop) {
       // (a NaN is ignored by the maximum and comes back through the sum)
       const float to = here > m ? here : m;
@@ -238,6 +253,113 @@ __global__ void __launch_bounds__(256)
               at_term - lse);
 }
 
+// ---- several short rows per wave ------------------------------------------------------------------
+// Four rows are reduced together: where the halves and quarters of a wave would be joined for each of them, two
+// rows' change places, and a quarter of the wave ends with each row.  The order in which a row's lanes are joined
+// is over_group's.
+template <int kLanes, typename F>
+__device__ __forceinline__ float over_four_rows(const float (&v)[kLanes / 16], F f) {
+  auto halves = [&](float a, float b) {
+    const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return f(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
+  };
+  auto quarters = [&](float a, float b) {
+    const auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return f(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
+  };
+  if constexpr (kLanes == 64) return over_group(quarters(halves(v[0], v[1]), halves(v[2], v[3])), 16, f);
+  if constexpr (kLanes == 32) return over_group(quarters(v[0], v[1]), 16, f);
+  if constexpr (kLanes == 16) return over_group(v[0], 16, f);
+}
+// For short rows: a lane group takes kIter rows, in steps of four a wave.  A row's chain of dependent loads -- its
+// range, its symbol, that entry -- is walked for all rows of a wave at once, a lane per row, beside the pieces,
+// which are all requested first, and that lane writes its row's results.
+// Bound by the latency of the loads of the waves that fit, and by issue: a wave per row is 604 bytes in flight at
+// float16, C 302, five rows a frame, B 34, T 1028, S 148: 83 -> 49 us (1.7 TB/s of what counts); bfloat16, B 128,
+// T 200, C 80: 18.4 -> 13.0; float32, B 100, T 500, C 500: 126 -> 86 (4.7 TB/s); B 32, T 500, C 256: 38 -> 23.7;
+// B 32, T 250, C 500: 23.6 -> 22.2, C 700: 24.0 -> 22.2; B 8, T 200, C 500: 7.2 -> 6.6.  Where rows are longer, a row is enough
+// in flight for a wave (float32, C 1000: 26.7 -> 29.9; bfloat16: 25.9 -> 26.7), and few rows do not
+// fill the chip (B 4, T 100, C 500: 4.3 -> 4.8; bfloat16, B 8, T 100: 5.1 -> 5.7).
+template <typename P, int kLanes, int kVecs, int kIter, bool kStream, bool kAligned>
+__global__ void __launch_bounds__(256)
+    row_norm_rows_kernel(const typename P::Elem *__restrict__ logits, Lattice L, Picks<float> out,
+                         Surround around) {
+  constexpr int kAux = kStream ? 2 : 0;
+  constexpr int kRows = kWave / kLanes, kN = kRows * kIter, kSteps = 4 / kRows;
+  static_assert(kN % 4 == 0 && kN <= kWave, "a lane per row");
+  out.start();
+  const int b = L.B - 1 - block_batch();
+  if (b < 0) return;
+  if (blockIdx.x < around.blocks) return around.fill(L, b, blockIdx.x, out.px, out.py);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register
+  const int at = threadIdx.x & 63, lane = at & (kLanes - 1);
+  const unsigned r0 = ((gridDim.x - 1 - blockIdx.x) * 4 + wave) * kN;
+  if (r0 >= (unsigned)(L.T * L.Rr)) return;
+  // this lane's row: of the fours, number at % 16
+  const bool mine = at % 16 < kN / 4;
+  Row row = placed_in_frame(L, b, r0 + (mine ? 4 * (at % 16) + row_of_quarter(at / 16) : 0));
+  // (a row whose range begins outside the window is read all the same)
+  const unsigned long long there = __ballot(mine && row.live);
+  if (there == 0 && !__any(mine && row.t < L.T)) return;
+  const long first = (long)b * L.T * L.Rr + r0;
+  const uintptr_t base = wave_base<P, kLanes>(logits, first, L.C);
+  const __amdgpu_buffer_rsrc_t rs =
+      resource(base, ((long)kN * L.C * (long)sizeof(typename P::Elem) + 31) & ~15L);
+  intx4 raw[kIter][kVecs];
+  RowPieces<P, kLanes> q[kIter];
+#pragma unroll
+  for (int n = 0; n < kIter; ++n) {
+    const int group = kRows == 4 ? row_of_quarter(at / 16) : kRows == 2 ? at / 32 : 0;
+    const int nth = kRows * n + group;
+    q[n] = pieces_of<P, kLanes>(base, reinterpret_cast<uintptr_t>(logits + (first + nth) * L.C), L.C);
+    if (kAligned) q[n].off = 0, q[n].whole = q[n].pieces = L.C / P::kPer;
+    const bool wanted = there >> (16 * row_of_quarter(nth % 4) + nth / 4) & 1;
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      const int p = lane + kLanes * i;
+      raw[n][i] = __builtin_amdgcn_raw_buffer_load_b128(
+          rs, (int)wanted & (int)(p < q[n].pieces) ? q[n].at + 16 * p : kOutOfRange, 0, kAux);
+    }
+  }
+  place(L, row);
+  const bool live = mine && row.live;
+  if (mine && !row.live) out.skip(L, row);
+  const int sym = live ? row_symbol(L, row) : -1;
+  float at_sym = 0, at_term = 0;
+  if (live) {
+    const typename P::Elem *x = logits + row.index * L.C;
+    at_term = P::load(x[L.term]);
+    if (sym >= 0) at_sym = P::load(x[sym]);
+  }
+  float my_sum = 0, my_shift = 0;
+#pragma unroll
+  for (int n0 = 0; n0 < kIter; n0 += kSteps) {
+    float v[kSteps];
+#pragma unroll
+    for (int n = 0; n < kSteps; ++n)
+      v[n] = largest_of_lane<P, kLanes, kVecs, kAligned>(raw[n0 + n], q[n0 + n], 0, lane, L.C);
+    const float m = over_four_rows<kLanes>(v, [](float a, float b) { return max3_raw(a, b, b); });
+    const float shift = (m - m == 0) ? m : 0.f;  // torch.logsumexp: infinite max -> shift by 0
+    float shifts[kSteps];
+    to_rows<kLanes>(shift, shifts);
+#pragma unroll
+    for (int n = 0; n < kSteps; ++n) {
+      v[n] = 0;
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i)
+#pragma unroll
+        for (int e = 0; e < P::kPer; ++e) v[n] += __expf(P::at(raw[n0 + n][i], e) - shifts[n]);
+    }
+    const float sum = over_four_rows<kLanes>(v, [](float a, float b) { return a + b; });
+    const bool here = at % 16 == n0 / kSteps;
+    my_sum = here ? sum : my_sum;
+    my_shift = here ? shift : my_shift;
+  }
+  const float lse = logf(my_sum) + my_shift;
+  if (live)
+    out.write(L, row, lse, sym >= 0 ? at_sym - lse : std::numeric_limits<float>::quiet_NaN(), at_term - lse);
+}
+
 // (rows in 16-byte pieces; else the plain kernel takes them)
 template <typename P>
 bool rows_in_pieces(int C) {
@@ -257,6 +379,24 @@ void launch_row_norm(const typename P::Elem *logits, const Lattice &L, const Pic
       const bool big = rows * L.B * L.C * (long)sizeof(typename P::Elem) >
                        (read_again ? 2 * kCacheBytes : kCacheBytes);
       with_row_split<P>(logits, L.C, [&](auto lanes, auto vecs, auto loop) {
+        if constexpr (vecs <= (P::kPer == 4 ? 3 : 1) && !loop) {
+          constexpr int kIter = lanes == 64 && vecs == 1 && P::kPer == 4 ? 8 : 4;
+          constexpr int kRowsOfBlock = kIter * 256 / lanes;
+          if (several_rows(rows * L.B, kRowsOfBlock)) {
+            auto launch = [&](auto stream_hint, auto aligned) {
+              hipLaunchKernelGGL((row_norm_rows_kernel<P, lanes, vecs, kIter, stream_hint, aligned>),
+                                 batch_grid(around.blocks + (rows + kRowsOfBlock - 1) / kRowsOfBlock, L.B),
+                                 dim3(256), 0, stream, logits, L, out, around);
+            };
+            constexpr std::integral_constant<bool, lanes == 64> hint;
+            if (big)
+              rows_aligned<P>(logits, L.C) ? launch(hint, std::true_type{}) : launch(hint, std::false_type{});
+            else
+              rows_aligned<P>(logits, L.C) ? launch(std::false_type{}, std::true_type{})
+                                           : launch(std::false_type{}, std::false_type{});
+            return;
+          }
+        }
         const dim3 grid = batch_grid(around.blocks + (rows + 256 / lanes - 1) / (256 / lanes), L.B);
         if (big && lanes == 64)
           hipLaunchKernelGGL((row_norm_kernel<P, lanes, vecs, loop, lanes == 64>), grid, dim3(256),

@@ -73,16 +73,41 @@ struct AccumOf<DoublePiece> {
   typedef double type;
 };
 
-template <typename R>
-__device__ __forceinline__ R group_max(R v, int lanes) {
+// Sums and maxima over the kLanes lanes of a group, in every one of them.  In float32 through the vector unit's own
+// lane exchanges, one instruction a step (a shuffle goes through the LDS unit and waits for it): the other half of
+// the wave, the other row of 16 lanes, then rotations within the row, whose partners are those of an exchange with
+// lane ^ 8, 4, 2, 1, since what has been combined already repeats.
+template <int kControl>
+__device__ __forceinline__ float rotated_in_row(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kControl, 0xf, 0xf, true));
+}
+template <typename F>
+__device__ __forceinline__ float over_group(float v, int lanes, F f) {
+  auto joined = [&](auto pair) { return f(__uint_as_float(pair[0]), __uint_as_float(pair[1])); };
+  if (lanes > 32)
+    v = joined(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  if (lanes > 16)
+    v = joined(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  v = f(v, rotated_in_row<0x128>(v));
+  v = f(v, rotated_in_row<0x124>(v));
+  v = f(v, rotated_in_row<0x122>(v));
+  return f(v, rotated_in_row<0x121>(v));
+}
+// (NaN if any is)
+__device__ __forceinline__ float group_max(float v, int lanes) {
+  return over_group(v, lanes, [](float a, float b) { return b > a || b != b ? b : a; });
+}
+__device__ __forceinline__ float group_sum(float v, int lanes) {
+  return over_group(v, lanes, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ double group_max(double v, int lanes) {
   for (int off = lanes / 2; off > 0; off >>= 1) {
-    const R o = __shfl_xor(v, off, 64);
+    const double o = __shfl_xor(v, off, 64);
     v = (o > v || o != o) ? o : v;
   }
   return v;
 }
-template <typename R>
-__device__ __forceinline__ R group_sum(R v, int lanes) {
+__device__ __forceinline__ double group_sum(double v, int lanes) {
   for (int off = lanes / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
@@ -139,7 +164,10 @@ __device__ __forceinline__ int placed_at(int64_t r0, int j, int S) {
 // window [s_begin, s_end] x [t_begin, t_end) is never looked at by the recursion, which hands
 // it a gradient of exact zeros: callers that go on to it with the same boundary (the loss
 // functions) let the kernels skip such rows -- about a third of a ragged batch.
-__device__ __forceinline__ Row locate(const Lattice &L, int b, unsigned r) {
+//
+// In two steps: what is known without the ranges -- `live` as far as the frame and, where there are none, the
+// lattice row decide -- and the rest.
+__device__ __forceinline__ Row placed_in_frame(const Lattice &L, int b, unsigned r) {
   Row o;
   o.b = b;
   o.t = (int)(r / (unsigned)L.Rr);
@@ -147,13 +175,23 @@ __device__ __forceinline__ Row locate(const Lattice &L, int b, unsigned r) {
   o.s = o.j;
   o.index = (long)b * L.T * L.Rr + r;
   o.live = o.t < L.T;
-  if (o.live) {
-    if (L.ranges) o.s = placed_at(L.ranges[o.index - o.j], o.j, L.S);
-    if (L.window) {
-      const int64_t *w = L.window + 4 * b;
-      o.live = o.t >= w[1] && o.t < w[3] && o.s >= w[0] && o.s <= w[2];
-    }
+  if (o.live && L.window) {
+    const int64_t *w = L.window + 4 * b;
+    o.live = o.t >= w[1] && o.t < w[3] && (L.ranges || (o.s >= w[0] && o.s <= w[2]));
   }
+  return o;
+}
+__device__ __forceinline__ void place(const Lattice &L, Row &o) {
+  if (!L.ranges || o.t >= L.T) return;
+  o.s = placed_at(L.ranges[o.index - o.j], o.j, L.S);
+  if (o.live && L.window) {
+    const int64_t *w = L.window + 4 * o.b;
+    o.live = o.s >= w[0] && o.s <= w[2];
+  }
+}
+__device__ __forceinline__ Row locate(const Lattice &L, int b, unsigned r) {
+  Row o = placed_in_frame(L, b, r);
+  place(L, o);
   return o;
 }
 
@@ -244,6 +282,29 @@ template <typename P>
 bool rows_aligned(const void *logits, int C) {
   return C % P::kPer == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
 }
+
+// Several short rows of a wave, in fours: quarter `seg` of the wave (16 lanes) has the results or the parameters of
+// row row_of_quarter(seg) of the four, `to_rows` brings them to the lanes that hold a row's pieces: of a whole wave
+// each (v[0 .. 3]), of a half (rows 0 and 1, then 2 and 3), or its own quarter.
+__device__ __forceinline__ constexpr int row_of_quarter(int seg) { return (seg & 1) * 2 + seg / 2; }
+template <int kLanes>
+__device__ __forceinline__ void to_rows(float of_quarters, float (&v)[kLanes / 16], int at = 0) {
+  if constexpr (kLanes == 64) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      v[n] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(of_quarters), 16 * row_of_quarter(n) + at));
+  } else if constexpr (kLanes == 32) {
+    const unsigned w = __float_as_uint(of_quarters);
+    const auto pair = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    v[0] = __uint_as_float(pair[0]), v[1] = __uint_as_float(pair[1]);
+  } else {
+    v[0] = of_quarters;
+  }
+}
+
+// Whether a launch with several rows per lane group has enough workgroups (of rows_of_block rows) to be worth it:
+// each is a longer chain, which shows where they do not all but fill the chip (figures at the kernels).
+inline bool several_rows(long rows, int rows_of_block) { return rows >= 384L * rows_of_block; }
 
 // Calls f(lanes, vecs, loop) with the split of a row's pieces as compile-time constants: the
 // fewest pieces per lane that hold the row, so that little is computed on padding; chunks of
