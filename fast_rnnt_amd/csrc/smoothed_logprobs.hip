@@ -564,8 +564,11 @@ __global__ void __launch_bounds__(256)
 // the partials being sum_rows G[row] exp(am - max) / z[row].  Same layout as
 // unigram_final_kernel.  The (b, s) pairs pass through LDS in chunks -- symbol and
 // row_x, fetched once by the whole block -- and every group scans a contiguous share
-// of each chunk.
-constexpr int kPairChunk = 2048;
+// of each chunk.  Bound by the LDS unit, which answers a group's reads one wave
+// after the other, and by the requests of a chunk, which go out together: with a pair a read, chunks of half the size
+// and a request at a time B 107, S 78, T 217, C 142 took 22.5 us, now 14.7; B 15, S 87, T 544, C 406: 7.2, now 6.5.
+constexpr int kPairChunk = 4096, kPairsAhead = kPairChunk / kUnigramThreads;
+static_assert(kPairChunk / kRowGroups % 4 == 0, "the groups' shares end with the chunk");
 
 template <typename R>
 __global__ void __launch_bounds__(kUnigramThreads)
@@ -574,8 +577,8 @@ __global__ void __launch_bounds__(kUnigramThreads)
                         const R *__restrict__ unigram, R *__restrict__ g_unigram, int blocks,
                         int B, int S, int C, int term, R k_am) {
   __shared__ R meet[kRowGroups][kColsPerBlock];
-  __shared__ int pair_sym[kPairChunk];
-  __shared__ R pair_x[kPairChunk];
+  __shared__ __align__(16) int pair_sym[kPairChunk];
+  __shared__ __align__(16) R pair_x[kPairChunk];
   const int col = threadIdx.x % kColsPerBlock, grp = threadIdx.x / kColsPerBlock;
   const int c = blockIdx.x * kColsPerBlock + col;
   const int S1 = S + 1, n = B * S1;
@@ -583,17 +586,35 @@ __global__ void __launch_bounds__(kUnigramThreads)
   for (int row0 = 0; row0 < n; row0 += kPairChunk) {
     const int count = min(kPairChunk, n - row0);
     __syncthreads();
-    for (int i = threadIdx.x; i < count; i += kUnigramThreads) {
-      const int row = row0 + i, b = row / S1, s = row - b * S1;
-      const int64_t y = s < S ? symbols[(long)b * S + s] : -1;
-      pair_sym[i] = (y >= 0 && y < C) ? (int)y : -1;
-      pair_x[i] = row_x[row];
+    int64_t y[kPairsAhead];
+    R x[kPairsAhead];
+#pragma unroll
+    for (int u = 0; u < kPairsAhead; ++u) {
+      // (a row that is not there, and one without a symbol, reads another's)
+      const int row = row0 + min((int)threadIdx.x + u * kUnigramThreads, count - 1), b = row / S1;
+      const int s = row - b * S1;
+      y[u] = S > 0 ? symbols[(long)b * S + min(s, S - 1)] : -1;
+      if (s == S) y[u] = -1;
+      x[u] = row_x[row];
+    }
+#pragma unroll
+    for (int u = 0; u < kPairsAhead; ++u) {
+      const int i = threadIdx.x + u * kUnigramThreads;
+      pair_sym[i] = i < count && y[u] >= 0 && y[u] < C ? (int)y[u] : -1;
+      pair_x[i] = x[u];
     }
     __syncthreads();
-    const int share = (count + kRowGroups - 1) / kRowGroups;
-    const int first = grp * share, last = min(first + share, count);
-    for (int i = first; i < last; ++i)
-      if (pair_sym[i] == c) direct += pair_x[i];
+    // (four pairs a read; what follows the last pair names no symbol)
+    const int share = ((count + kRowGroups - 1) / kRowGroups + 3) / 4 * 4;
+    for (int i = grp * share; i < (grp + 1) * share; i += 4) {
+      const auto sym = *reinterpret_cast<const int4 *>(pair_sym + i);
+      const R *v = pair_x + i;
+      const R v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+      direct = sym.x == c ? direct + v0 : direct;
+      direct = sym.y == c ? direct + v1 : direct;
+      direct = sym.z == c ? direct + v2 : direct;
+      direct = sym.w == c ? direct + v3 : direct;
+    }
   }
   // the termination symbol's column also takes the sum of row_y over all rows: the whole
   // block adds it up (every thread a strided share, eight loads in flight, then a fixed
