@@ -1721,7 +1721,13 @@ size_t apart_lds_bytes(int T) {
 // as two, then stay together (B 136, S 100, T 6000: 595 + 599 apart, 407 + 555 together; B 136, S 70,
 // T 5000: 443 + 438, 281 + 318); three and four are still better off apart (B 128, S 250, T 5000:
 // 674 + 831 apart, 763 + 1125 together; B 96, S 180, T 6000: 656 + 696, 681 + 862).
-template <typename R>
+//
+// The kernels that pass shares have faster steps apart (kSharesStagersApart).  Three bands then pay for any length
+// while each has a compute unit: forward and backward with the marks, together and apart, B 8, S 130, T 140: 41.5 and
+// 37.9 us; S 160, T 300: 58.5 and 48.2; T 600: 85 and 64; B 64, S 190, T 200: 56.5 and 49.0.  (With more
+// of them than units the rule is that of the other kernels: B 100, S 130, T 600: 88 and 92; B 168, S 160, T 300: 67 and 74.  Two bands
+// gain from where they did: B 24, S 80, T 600: 55.7 and 56.3; T 900: 72.5 and 71.1.)
+template <typename R, bool kShares>
 bool bands_apart(int B, int S, int T, bool backward) {
   const int bands = (S + kWave) / kWave;
   if (sizeof(R) != 4 || bands < 2 || bands > kMaxSweep || T < 1) return false;
@@ -1729,6 +1735,7 @@ bool bands_apart(int B, int S, int T, bool backward) {
   if (per_cu == 0) return false;
   const long workgroups = (long)((B + 7) / 8 * 8) * bands;
   if (workgroups > (bands == 2 && per_cu == 1 ? 256 : 512)) return false;
+  if (kShares && bands == 3 && workgroups <= 256) return true;
   constexpr double kCost[2][3] = {{6, 7, 10}, {11, 16, 20}}, kSaved[2][3] = {{6.7, 7, 39}, {13, 28, 60}};
   return 1e-3 * kSaved[backward][bands - 2] * (S + T) > kCost[backward][bands - 2];
 }
@@ -1768,7 +1775,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   constexpr int kFew = kShares ? kSharesStagers : sizeof(R) == 4 ? kFwdStagersFew : 2;
   constexpr int kOne = kShares ? kSharesStagersOne : kFew;  // with one sweep wave
   if constexpr (sizeof(R) == 4) {
-    const bool apart = bands_apart<R>(B, S, T, false), later = px_grad && bands_apart<R>(B, S, T, true);
+    const bool apart = bands_apart<R, kShares>(B, S, T, false), later = px_grad && bands_apart<R, kShares>(B, S, T, true);
     if (apart || later)
       mark_seams(boundary, apart && !kShares ? p : nullptr, apart && kShares ? py_grad : nullptr, ans,
                  later ? px_grad : nullptr, B, S, T, modified, static_cast<hipStream_t>(stream));
@@ -1833,7 +1840,7 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   static_assert(kMaxSweep * 2 <= 16 && 2 * kFewBuffers <= 16, "Counters::loaded is too short");
   const bool few = n <= 2 && lds_bytes(n, T, kFewBuffers, sizeof(R)) <= kLdsBudget;
   if constexpr (kFloat) {
-    if (bands_apart<R>(B, S, T, true)) {
+    if (bands_apart<R, kShares>(B, S, T, true)) {
       if (!marked)
         mark_seams(boundary, nullptr, nullptr, nullptr, px_grad, B, S, T, modified,
                    static_cast<hipStream_t>(stream));
