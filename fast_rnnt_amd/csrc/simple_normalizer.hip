@@ -763,6 +763,7 @@ void launch_normalizer_f32(const float *lm, const float *am, const int64_t *symb
                            float *py, float *norm_raw, const int64_t *window,
                            double delay_penalty, int B, int S, int T, int C, int term,
                            int rnnt_type, const SmoothMix *mix, float *workspace, hipStream_t stream) {
+  if (reinterpret_cast<uintptr_t>(workspace) & 15) workspace = nullptr;  // (words of 8 bytes, pieces of 16)
   const NormArgs args{lm, am, symbols, boundary, window, lm_max, am_max, px, py, norm_raw,
                       Delay<float>{(float)delay_penalty}, B, S, T, C, term, rnnt_type, nullptr, nullptr, 0};
   const NormChoice choice = choose_tile(B, S, T, C, window != nullptr, workspace != nullptr);
