@@ -222,6 +222,7 @@ int mi_backward_and_loss(const double *px, const int64_t *boundary, const double
                          int B, int S, int T, int modified, int reduction, void *stream);
 // The same pair where nobody wants p: `shares`, of p's size, is scratch between the two.
 // Host side, mi_shares_forward.hip and mi_shares_backward.hip.
+bool mi_shares_pay(int B, int S, int T);
 int mi_forward_shares(const float *px, const float *py, const int64_t *boundary, float *shares,
                       float *scores, int B, int S, int T, int modified, int checks, int32_t *status,
                       float *px_grad, float *py_grad, void *stream);

@@ -5,6 +5,20 @@
 
 namespace frnnt {
 
+// Whether a loss is faster with shares than with p (both kernels and the marks, p against shares).  With one sweep
+// wave in the workgroup, always (S 40, B 32: T 100: 16.0 and 15.4 us; T 500: 39.5 and 35.1).  With two the forward
+// kernel's staging waves, who have more to do, are what short lattices wait for, and the backward makes up for it from
+// some 200 frames on (S 90, B 32, T 100: 22.9 and 24.3; T 200: 30.0 and 30.5; T 350: 41.2 and 40.5; S 120, B 100, T 500:
+// 57.0 and 51.6); with three and four, which have three staging waves each, later (B 100, S 160, T 260: 53.2 and 60.1; T
+// 450: 77.1 and 76.2; B 168, S 190, T 350: 93.2 and 90.1; T 900: 230 and 185).  Bands apart have the marks to make up
+// for (B 4, S 130, T 100: 33.5 and 34.4; T 140: 36.8 and 35.0).
+bool mi_shares_pay(int B, int S, int T) {
+  if (S < kWave) return true;
+  if (S < 2 * kWave) return T >= 200;
+  const bool apart = bands_apart<float, true>(B, S, T, false) && bands_apart<float, true>(B, S, T, true);
+  return T >= (apart ? 120 : 400);
+}
+
 int mi_forward_shares(const float *px, const float *py, const int64_t *boundary, float *shares,
                       float *scores, int B, int S, int T, int modified, int checks, int32_t *status,
                       float *px_grad, float *py_grad, void *stream) {

@@ -22,7 +22,7 @@ int mi_loss_fwd(Reduce reduce, const R *px, const R *py,
   const bool p_wanted = (checks & FRNNT_SCRATCH_P) == 0;
   checks &= ~(FRNNT_SCRATCH_P | FRNNT_LARGE_SCRATCH);
   if constexpr (std::is_same<R, float>::value) {
-    if (px_grad && !p_wanted) {
+    if (px_grad && !p_wanted && mi_shares_pay(B, S, T)) {
       int rc = mi_forward_shares(px, py, boundary, p, scores, B, S, T, modified, checks, status, px_grad,
                                  py_grad, stream);
       if (rc != FRNNT_OK) return rc;
