@@ -14,7 +14,8 @@
 // each kind of tile in a loop of its own.  *Staging waves* of the same workgroup fetch
 // px/py (forward) or p/px (backward) with coalesced, range-checked row loads, turn
 // them into diagonal ("sheared") 64-row x 32-step tiles in LDS and -- for the
-// backward sweep -- also evaluate the exp() of the gradient split; the sweep wave
+// backward sweep -- also evaluate the exp() of the gradient split (the forward kernel's do,
+// where nobody wants p: kShares); the sweep wave
 // pulls a tile into registers with 16-byte LDS reads and leaves the tile's results
 // in the same LDS buffer with 16-byte writes.  The staging waves carry the results
 // to memory as coalesced row segments through range-checked buffer stores (a cell
