@@ -1018,7 +1018,10 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   const __amdgpu_buffer_rsrc_t gy_rsrc = buffer_of(gyb, (size_t)(S + 1) * T);
 
   const R seed = ans_grad ? ans_grad[(size_t)b * seed_stride] : (R)1;
-  // Exact zeros everywhere the sweep does not write (0 times the seed: NaN if that is not finite), by wave `part` of `parts`, off the critical path (a
+  // What a cell without a gradient holds.  mi_backward takes a seed as it is: 0.  The pair that passes shares stands for
+  // gradients of ones that are scaled afterwards, all of them: 0 times the seed, NaN if that is not finite.
+  const R nothing = kShares ? seed - seed : (R)0;
+  // That everywhere the sweep does not write, by wave `part` of `parts`, off the critical path (a
   // barrier after these stores would have to wait until they have all reached memory).  An array's
   // window leaves a run before it, one after it and, all of one length, those between its rows: four rows'
   // to an instruction, 16 lanes each (row by row, with a run's ends tested for each, two waves took
@@ -1026,7 +1029,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   auto zero_run = [&](__amdgpu_buffer_rsrc_t rs, int begin, int end, int first, int lanes) {
     // elements [begin, end), by lanes `first` .. of `lanes` that step through it together; overlapping the
     // last four, so that all stores are whole
-    const R z = seed - seed;
+    const R z = nothing;
     if (end - begin < 4) {
       put1(rs, first < end - begin ? (begin + first) * (int)sizeof(R) : kDropped, z);
       return;
@@ -1049,11 +1052,11 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       const int row = r + (lane >> 4), begin = row * width + hi;
       const bool there = row < r_hi - 1;
       if (gap < 4) {
-        put1(rs, there && q < gap ? (begin + q) * (int)sizeof(R) : kDropped, seed - seed);
+        put1(rs, there && q < gap ? (begin + q) * (int)sizeof(R) : kDropped, nothing);
       } else {
         for (int t = 4 * q; t - 4 * q < gap; t += 64)
-          put4(rs, there && t < gap ? (begin + min(t, gap - 4)) * (int)sizeof(R) : kDropped, seed - seed,
-               seed - seed, seed - seed, seed - seed);
+          put4(rs, there && t < gap ? (begin + min(t, gap - 4)) * (int)sizeof(R) : kDropped, nothing,
+               nothing, nothing, nothing);
       }
     }
   };
@@ -1502,8 +1505,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     const int fin_step = (fin_lane < kWave) ? NT + fin_lane : -1;
 
     // the seed enters as "handed left" into the first cell of the reversed sweep
-    // (a seed that is not finite makes cells that it does not reach NaN as well)
-    R to_below = seed - seed, to_below2 = seed - seed, to_left = (r == 0) ? seed : seed - seed;
+    // (shares: a seed that is not finite makes cells that it does not reach NaN as well)
+    R to_below = nothing, to_below2 = nothing, to_left = (r == 0) ? seed : nothing;
     R g_origin = 0;
     const R *seam_at = up_seam + (lane - shift);  // seam_at[e]: what lane 0 needs at step e + lane
     // rows below this wave's: someone reads the seam
