@@ -20,6 +20,6 @@ extern "C" int frnnt_mi_shares_bwd_f32(const int64_t *boundary, const float *sha
     return frnnt::fail(FRNNT_EINVAL, "mi_shares_bwd: score_grad_stride must be 0 or 1");
   return frnnt::backward_impl<float, true>(nullptr, nullptr, boundary, shares,
                                            const_cast<float *>(score_grad), px_grad, py_grad, B, S, T,
-                                           modified, 0, stream, nullptr, nullptr, 0, true,
+                                           modified, 0, stream, nullptr, nullptr, 0, false,
                                            score_grad_stride);
 }

@@ -32,7 +32,8 @@ extern "C" int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const i
                                        float *shares, float *scores, float *px_grad, float *py_grad, int B,
                                        int S, int T, int modified, int checks, int32_t *status,
                                        void *stream) {
-  if (B > 0 && (!px_grad || !py_grad)) return frnnt::fail(FRNNT_EINVAL, "mi_shares_fwd: null pointer");
+  (void)px_grad;  // (marked by the call that writes it)
+  if (B > 0 && !py_grad) return frnnt::fail(FRNNT_EINVAL, "mi_shares_fwd: null pointer");
   return frnnt::mi_forward_shares(px, py, boundary, shares, scores, B, S, T, modified, checks, status,
-                                  px_grad, py_grad, stream);
+                                  nullptr, py_grad, stream);
 }

@@ -132,9 +132,9 @@ int frnnt_mi_backward_f64(const double *px, const double *py, const int64_t *bou
 /*
  * The two as a pair for callers that do not want p (float32; no counterpart in the reference): _fwd leaves
  * the scores and, in `shares` [B][S+1][T+1], what _bwd needs; arguments otherwise as above.  px_grad
- * and py_grad are _bwd's outputs; both calls get the same buffers, which nothing else may write to in
- * between (_fwd prepares them).  _bwd takes utterance b's gradient of its score from
- * score_grad[b * score_grad_stride] (stride 0 or 1; NULL: 1).
+ * and py_grad are _bwd's outputs.  _fwd takes py_grad as scratch (any B (S+1) T floats) and leaves px_grad alone (may
+ * be NULL).  _bwd takes utterance b's gradient of its score from score_grad[b * score_grad_stride] (stride 0 or 1;
+ * NULL: 1); it may be called again on the same shares.
  */
 int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *shares,
                             float *scores, float *px_grad, float *py_grad, int B, int S, int T,

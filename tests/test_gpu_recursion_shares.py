@@ -94,6 +94,40 @@ def test_what_the_scratch_held_before(modified, value):
     assert torch.isfinite(want_x).all() and torch.isfinite(want_y).all()
 
 
+# one band, two together, two, three and four apart
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("B,S,T", [(5, 20, 33), (5, 100, 90), (4, 100, 1300), (4, 150, 200), (3, 250, 700)])
+def test_backward_again_on_the_same_shares(B, S, T, modified):
+    """With another gradient of the scores, into buffers that hold anything, those of the first call among them: what
+    a first call on shares of their own forms."""
+    px, py, g = _inputs(B, S, T, modified, S)
+    px, py, boundary = px.cuda(), py.cuda(), _window(B, S, T, g).cuda()
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+
+    def forward():
+        shares, scores = torch.empty(B, S + 1, T + 1, device="cuda"), torch.empty(B, device="cuda")
+        scratch = torch.empty_like(px), torch.empty_like(py)
+        assert lib.frnnt_mi_shares_fwd_f32(
+            px.data_ptr(), py.data_ptr(), boundary.data_ptr(), shares.data_ptr(), scores.data_ptr(),
+            scratch[0].data_ptr(), scratch[1].data_ptr(), B, S, T, int(modified), 0, None, stream) == 0
+        return shares
+
+    def backward(shares, seeds, grads):
+        assert lib.frnnt_mi_shares_bwd_f32(boundary.data_ptr(), shares.data_ptr(), seeds.data_ptr(), 1,
+                                           grads[0].data_ptr(), grads[1].data_ptr(), B, S, T, int(modified),
+                                           stream) == 0
+        return [x.clone() for x in grads]
+
+    one, two = torch.linspace(1, 3, B, device="cuda"), torch.linspace(-2, 0.5, B, device="cuda")
+    shares, grads = forward(), [torch.full_like(px, 7.0), torch.full_like(py, 7.0)]
+    first, second, third = (backward(shares, seeds, grads) for seeds in (one, two, one))
+    want = backward(forward(), two, [torch.zeros_like(px), torch.zeros_like(py)])
+    occ = F.mutual_information_recursion(px, py, boundary, return_grad=True)[1]
+    for a, b, c, w, o in zip(first, second, third, want, occ):
+        assert torch.equal(a, c) and torch.equal(b, w)
+        assert torch.allclose(b, o * two.reshape(-1, 1, 1), rtol=2 * (S + T) * 2.0 ** -24, atol=1e-37)
+
+
 @pytest.mark.parametrize("B,S,T", [(6, 40, 150), (6, 80, 250), (8, 100, 900), (8, 250, 700)])
 def test_a_wait_that_runs_out_shows_as_nan(B, S, T):
     """With the bound of the kernels' waits set from the host: an utterance's score is NaN, or its gradients
