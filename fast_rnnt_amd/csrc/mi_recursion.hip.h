@@ -374,12 +374,13 @@ constexpr int kSeamMark = 0x7fa5a5a5;
 // What a courier wave of a band does: takes the seam's `total` values from memory -- value c at
 // from + c * stride -- to the seam row in LDS as they arrive, and counts them in.  A wave of its
 // own: a staging wave's waits are for everything it has requested and stored, in order.
-__device__ __forceinline__ bool bring_seam(const float *from, int stride, int total, float *seam,
-                                           int *ready, int lane, int limit) {
+// `again`: marks what it has taken, for the next launch that finds its seam there.
+__device__ __forceinline__ bool bring_seam(float *from, int stride, int total, float *seam,
+                                           int *ready, int lane, int limit, bool again) {
   for (int done = 0, spins = 0; done < total;) {
     int bits = kSeamMark;
     if (done + lane < total)
-      bits = __hip_atomic_load(reinterpret_cast<const int *>(from + (long)(done + lane) * stride),
+      bits = __hip_atomic_load(reinterpret_cast<int *>(from + (long)(done + lane) * stride),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long missing = __ballot(bits == kSeamMark);
     const int n = missing ? __builtin_ctzll(missing) : kWave;
@@ -389,6 +390,9 @@ __device__ __forceinline__ bool bring_seam(const float *from, int stride, int to
       continue;
     }
     if (lane < n) seam[done + lane] = __int_as_float(bits);
+    if (again && lane < n)
+      __hip_atomic_store(reinterpret_cast<int *>(from + (long)(done + lane) * stride), kSeamMark,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     done += n;
     spins = 0;
     if (lane == 0) publish_lds_writes(ready, done);
@@ -409,7 +413,7 @@ __device__ __forceinline__ bool send_seam(float *to, int stride, int total, cons
   }
   return true;
 }
-__device__ __forceinline__ bool bring_seam(const double *, int, int, double *, int *, int, int) {
+__device__ __forceinline__ bool bring_seam(double *, int, int, double *, int *, int, int, bool) {
   return false;
 }
 __device__ __forceinline__ bool send_seam(double *, int, int, const double *, const int *, int, int) {
@@ -430,6 +434,13 @@ __device__ __forceinline__ R *mail_row(R *py_grad, int b, int s, int S, int T) {
   return py_grad + ((size_t)b * (S + 1) + s) * T;
 }
 
+// Or, with a post, where the seam behind band `band` passes in either direction: a row of its own, T + 1 elements for
+// each band but the last.  Marked once, by the forward's call; who has read a value leaves a mark again.
+template <typename R>
+__device__ __forceinline__ R *post_row(R *post, int b, int band, int S, int T) {
+  return post + ((size_t)b * (S / kWave) + band) * (T + 1);
+}
+
 // A word that any of an utterance's workgroups may make NaN (a wait of theirs ran out) and that the
 // last one gives its value: the value replaces what the word held before the launch and nothing
 // else, the NaN replaces anything.  Whichever comes first, the NaN stays.
@@ -444,23 +455,24 @@ __device__ __forceinline__ void store_once(float *word, int before, float value)
                                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The marks of an utterance's seam rows: in p or, with `mail`, in the rows that stand for p's (mail_row;
-// both may be NULL) where rows s0 + 63, s0 + 127, ... of the window feed the next one, in px_grad (which
-// may be NULL) where the reversed rows do; and, with p or mail, the utterance's score (see store_once).
+// The marks of an utterance's seam rows: in p or, with `mail`, in the rows that stand for p's (mail_row or, if it is
+// a post, post_row; both may be NULL) where rows s0 + 63, s0 + 127, ... of the window feed the next one, in px_grad
+// (which may be NULL) where the reversed rows do; and, with p or mail, the utterance's score (see store_once).
 // A block per utterance and seam.
 __global__ void __launch_bounds__(256)
     mark_seams_kernel(const int64_t *__restrict__ boundary, float *__restrict__ p, float *__restrict__ mail,
                       float *__restrict__ ans, float *__restrict__ px_grad, int S, int T,
-                      int modified) {
+                      int modified, int posted) {
   const int b = blockIdx.x, last = (int)blockIdx.y * kWave + kWave - 1;  // (row, or reversed row)
   if ((p || mail) && blockIdx.y == 0 && threadIdx.x == 0) ans[b] = __int_as_float(kSeamMark);
   const Window win = load_window(boundary, b, S, T);
   if (!win.ok || last + 1 > win.ns) return;
   const float mark = __int_as_float(kSeamMark);
   if (p || mail) {
-    int *row = reinterpret_cast<int *>((mail ? mail_row(mail, b, win.s0 + last, S, T)
-                                             : p + ((size_t)b * (S + 1) + win.s0 + last) * (T + 1)) +
-                                       win.t0);
+    int *row = reinterpret_cast<int *>(
+        posted ? post_row(mail, b, blockIdx.y, S, T)
+               : (mail ? mail_row(mail, b, win.s0 + last, S, T) : p + ((size_t)b * (S + 1) + win.s0 + last) * (T + 1)) +
+                     win.t0);
     for (int j = threadIdx.x; j <= win.nt; j += 256) row[j] = __float_as_int(mark);
   }
   if (px_grad) {
@@ -480,14 +492,14 @@ __global__ void __launch_bounds__(256)
 // kSweepCap: most sweep waves the launch may use; it only sets the register budget.
 // kApart: a workgroup per band; `pitch` workgroups per band, one per utterance (of B).
 // kShares: what a cell hands down of its gradient, d1 = exp(term1 - p), is stored in the place of p (see
-// the backward kernel); the seams of workgroups apart then go through `mail` (see mail_row).
+// the backward kernel); the seams of workgroups apart then go through `mail` (see mail_row; posted: post_row).
 template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart, bool kShares>
 __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)) * kWave)
     mi_forward_kernel(const R *__restrict__ px, const R *__restrict__ py,
                       const int64_t *__restrict__ boundary, R *__restrict__ p,
                       R *__restrict__ ans, int S, int T, int spin_limit, int checks,
-                      int *__restrict__ status, int B, int pitch, R *mail, R *loss, int reduction,
-                      int *arrived) {
+                      int *__restrict__ status, int B, int pitch, R *mail, int posted, R *loss,
+                      int reduction, int *arrived) {
   // (lattices of one band -- a cap of one sweep wave -- have no seams)
   constexpr bool kSeams = kApart || kSweepCap > 1;
   extern __shared__ __align__(16) unsigned char dyn_lds[];
@@ -585,7 +597,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
 
   // (apart) where p of the window's row i passes from one workgroup to the next
   auto seam_row = [&](int i) -> R * {
-    return kShares ? mail_row(mail, b, win.s0 + i, S, T) + win.t0 : pb + (size_t)(win.s0 + i) * TP + win.t0;
+    if (kShares && posted) return post_row(mail, b, i / kWave, S, T);
+    return (kShares ? mail_row(mail, b, win.s0 + i, S, T) : pb + (size_t)(win.s0 + i) * TP) + win.t0;
   };
   if (kApart && wave >= 1 + kStagers) {
     // ------------------------------- courier waves -------------------------------
@@ -597,7 +610,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
       return;
     }
     if (part > 0 &&
-        !bring_seam(seam_row(part * kWave - 1), 1, cols, seam, &cnt.ready[0], lane, spin_limit))
+        !bring_seam(seam_row(part * kWave - 1), 1, cols, seam, &cnt.ready[0], lane, spin_limit, kShares && posted))
       give_up();
     return;
   }
@@ -996,7 +1009,7 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
                        const R *__restrict__ p, R *ans_grad, R *__restrict__ px_grad,
                        R *__restrict__ py_grad, int S, int T, int seed_stride, int overwrite_ans_grad,
                        const R *__restrict__ scores, R *__restrict__ loss, int B, int reduction,
-                       int spin_limit, int pitch) {
+                       int spin_limit, int pitch, R *post) {
   extern __shared__ __align__(16) unsigned char dyn_lds[];
   __shared__ Counters cnt;
 
@@ -1123,15 +1136,21 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
   }
   if (kApart && wave >= 1 + kStagers) {
     // ------------------------------- courier waves -------------------------------
+    // where the gradients that band `of` hands down pass: through its last row of px_grad, from the end, or the post
+    const bool posted = kShares && post != nullptr;
+    const int stride = posted ? 1 : -1;
+    auto seam_row = [&](int of) -> R * {
+      if (posted) return post_row(post, b, of, S, T);
+      return gxb + (size_t)(win.s0 + NS - (of + 1) * kWave) * T1 + win.t0 + NT - shift;
+    };
     if (wave == 1 + kStagers) {
-      const int next = (part + 1) * kWave;
-      if (next <= NS && !send_seam(gxb + (size_t)(win.s0 + NS - next) * T1 + win.t0 + NT - shift, -1,
-                                   cols - shift, seam + seam_pitch, &cnt.ready[1], lane, spin_limit))
+      if ((part + 1) * kWave <= NS && !send_seam(seam_row(part), stride, cols - shift, seam + seam_pitch,
+                                                 &cnt.ready[1], lane, spin_limit))
         give_up();
       return;
     }
-    if (part > 0 && !bring_seam(gxb + (size_t)(win.s0 + NS - part * kWave) * T1 + win.t0 + NT - shift, -1,
-                                cols - shift, seam, &cnt.ready[0], lane, spin_limit))
+    if (part > 0 && !bring_seam(seam_row(part - 1), stride, cols - shift, seam, &cnt.ready[0], lane, spin_limit,
+                                posted))
       give_up();
     return;
   }
@@ -1744,18 +1763,24 @@ bool bands_apart(int B, int S, int T, bool backward) {
   return 1e-3 * kSaved[backward][bands - 2] * (S + T) > kCost[backward][bands - 2];
 }
 inline void mark_seams(const int64_t *boundary, float *p, float *mail, float *ans, float *px_grad, int B,
-                       int S, int T, int modified, hipStream_t stream) {
+                       int S, int T, int modified, bool posted, hipStream_t stream) {
   hipLaunchKernelGGL(mark_seams_kernel, dim3(B, (S + kWave) / kWave - 1), dim3(256), 0, stream,
-                     boundary, p, mail, ans, px_grad, S, T, modified);
+                     boundary, p, mail, ans, px_grad, S, T, modified, (int)posted);
+}
+// What a caller's buffer holds behind the shares: the post, if there is a seam to pass.
+inline int64_t shares_floats(int B, int S, int T) { return (int64_t)B * (S + 1) * (T + 1); }
+inline int64_t post_floats(int B, int S, int T) {
+  const bool seams = bands_apart<float, true>(B, S, T, false) || bands_apart<float, true>(B, S, T, true);
+  return seams ? (int64_t)B * (S / kWave) * (T + 1) : 0;
 }
 
 // `px_grad`: if given, its seams are marked as well (for a backward_impl that follows and is told so).
-// kShares (float only): p is filled for a backward_impl with kShares; py_grad is its py_grad.
+// kShares (float only): p is filled for a backward_impl with kShares; py_grad is its py_grad or, posted, the post of both.
 // `loss`: if it can, the kernel forms the loss (see count_for_loss) and sets loss->formed.
 template <typename R, bool kShares = false>
 int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans, int B, int S,
                  int T, int modified, void *stream, int checks = 0, int *status = nullptr,
-                 R *px_grad = nullptr, R *py_grad = nullptr, LossOf<R> *loss = nullptr) {
+                 R *px_grad = nullptr, R *py_grad = nullptr, LossOf<R> *loss = nullptr, bool posted = false) {
   static_assert(!kShares || sizeof(R) == 4, "shares are float's");
   R *loss_out = loss && loss->out && (loss->reduction == 0 || loss->arrived) ? loss->out : nullptr;
   const int reduction = loss ? loss->reduction : 0;
@@ -1779,10 +1804,11 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
   constexpr int kFew = kShares ? kSharesStagers : sizeof(R) == 4 ? kFwdStagersFew : 2;
   constexpr int kOne = kShares ? kSharesStagersOne : kFew;  // with one sweep wave
   if constexpr (sizeof(R) == 4) {
-    const bool apart = bands_apart<R, kShares>(B, S, T, false), later = px_grad && bands_apart<R, kShares>(B, S, T, true);
+    const bool apart = bands_apart<R, kShares>(B, S, T, false);
+    const bool later = (px_grad || posted) && bands_apart<R, kShares>(B, S, T, true);
     if (apart || later)
-      mark_seams(boundary, apart && !kShares ? p : nullptr, apart && kShares ? py_grad : nullptr, ans,
-                 later ? px_grad : nullptr, B, S, T, modified, static_cast<hipStream_t>(stream));
+      mark_seams(boundary, apart && !kShares ? p : nullptr, (apart && kShares) || posted ? py_grad : nullptr, ans,
+                 later ? px_grad : nullptr, B, S, T, modified, posted, static_cast<hipStream_t>(stream));
     if (apart) {
       const int pitch = (B + 7) / 8 * 8;  // (an utterance's bands on one XCD)
       const size_t lds = apart_lds_bytes(T);
@@ -1792,7 +1818,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
         return check_launch("mi_forward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kOne) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T,
-                         mi_spin_limit, checks, status, B, pitch, py_grad, nullptr, 0, nullptr);
+                         mi_spin_limit, checks, status, B, pitch, py_grad, (int)posted, nullptr, 0, nullptr);
       return check_launch("mi_forward");
     }
   }
@@ -1809,17 +1835,18 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
     return check_launch("mi_forward: hipFuncSetAttribute");
   hipLaunchKernelGGL(kernel, dim3(B), dim3(n * (1 + stagers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T, mi_spin_limit,
-                     checks, status, B, B, py_grad, loss_out, reduction, arrived);
+                     checks, status, B, B, py_grad, (int)posted, loss_out, reduction, arrived);
   if (loss) loss->formed = loss_out != nullptr;
   return check_launch("mi_forward");
 }
 
-// kShares: p is what a forward_impl with kShares has left; px is not read.
+// kShares: p is what a forward_impl with kShares has left; px is not read.  post: that of such a forward_impl.
 template <typename R, bool kShares = false>
 int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p, R *ans_grad,
                   R *px_grad, R *py_grad, int B, int S, int T, int modified,
                   int overwrite_ans_grad, void *stream, const R *scores = nullptr,
-                  R *loss = nullptr, int reduction = 0, bool marked = false, int seed_stride = 1) {
+                  R *loss = nullptr, int reduction = 0, bool marked = false, int seed_stride = 1,
+                  R *post = nullptr) {
   (void)py;  // the d2 = 1 - d1 split needs only p and px
   if (loss && (!scores || reduction < 0 || reduction > 2))
     return fail(FRNNT_EINVAL, "mi_backward: loss without scores, or bad reduction");
@@ -1845,8 +1872,8 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   const bool few = n <= 2 && lds_bytes(n, T, kFewBuffers, sizeof(R)) <= kLdsBudget;
   if constexpr (kFloat) {
     if (bands_apart<R, kShares>(B, S, T, true)) {
-      if (!marked)
-        mark_seams(boundary, nullptr, nullptr, nullptr, px_grad, B, S, T, modified,
+      if (!marked && !post)
+        mark_seams(boundary, nullptr, nullptr, nullptr, px_grad, B, S, T, modified, false,
                    static_cast<hipStream_t>(stream));
       const int pitch = (B + 7) / 8 * 8;
       const size_t lds = apart_lds_bytes(T);
@@ -1858,7 +1885,7 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
                          dim3((3 + kAlone + kHelpers<1, kShares>) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
                          py_grad, S, T, seed_stride, overwrite_ans_grad, scores, loss, B, reduction,
-                         mi_spin_limit, pitch);
+                         mi_spin_limit, pitch, post);
       return check_launch("mi_backward");
     }
   }
@@ -1878,7 +1905,7 @@ int backward_impl(const R *px, const R *py, const int64_t *boundary, const R *p,
   hipLaunchKernelGGL(kernel, dim3(B), dim3((n * (1 + stagers) + helpers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, boundary, p, ans_grad, px_grad,
                      py_grad, S, T, seed_stride, overwrite_ans_grad, scores, loss, B, reduction,
-                     mi_spin_limit, B);
+                     mi_spin_limit, B, post);
   return check_launch("mi_backward");
 }
 

@@ -37,3 +37,16 @@ extern "C" int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const i
   return frnnt::mi_forward_shares(px, py, boundary, shares, scores, B, S, T, modified, checks, status,
                                   nullptr, py_grad, stream);
 }
+
+extern "C" int64_t frnnt_mi_kept_size(int B, int S, int T) {
+  if (B < 1 || S < 0 || T < 0) return 0;
+  return frnnt::shares_floats(B, S, T) + frnnt::post_floats(B, S, T);
+}
+extern "C" int frnnt_mi_kept_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *kept,
+                                     float *scores, int B, int S, int T, int modified, int checks,
+                                     int32_t *status, void *stream) {
+  using namespace frnnt;
+  float *post = kept && B > 0 && S >= 0 && T >= 0 ? kept + shares_floats(B, S, T) : nullptr;
+  return forward_impl<float, true>(px, py, boundary, kept, scores, B, S, T, modified, stream, checks, status,
+                                   nullptr, post, nullptr, true);
+}

@@ -384,7 +384,7 @@ struct RecursionLossFn : public torch::autograd::Function<RecursionLossFn> {
 // in-place scaling in the backward.  Unless they are handed out nobody else holds them by then, so
 // that px.grad and py.grad take them over without a copy; and in float32 they are formed then, from
 // the gradient of the scores, instead of in the forward and scaled afterwards (a pass over both:
-// 12 us of 144 at B 12, S 220, T 1500).
+// 12 us of 144 at B 12, S 220, T 1500).  Kept until then are the shares, one lattice, instead of two.
 struct RecursionFn : public torch::autograd::Function<RecursionFn> {
   static variable_list forward(AutogradContext *ctx, const Tensor &px_, const Tensor &py_,
                                const std::optional<Tensor> &boundary_, bool want_grads,
@@ -396,22 +396,23 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
     ctx->set_materialize_grads(false);
     DeviceGuard guard(px.device());
     const auto opts = px.options();
-    Tensor p = at::empty({B, S + 1, T + 1}, opts), scores = at::empty({B}, opts);
-    Tensor gx, gy;
+    Tensor scores = at::empty({B}, opts);
+    if (need_grad && !want_grads && px.scalar_type() == at::kFloat) {
+      const Tensor kept = at::empty({frnnt_mi_kept_size((int)B, (int)S, (int)T)}, opts);
+      check_rc(frnnt_mi_kept_fwd_f32(ptr<float>(px), ptr<float>(py), iptr(bnd), ptr<float>(kept),
+                                     ptr<float>(scores), (int)B, (int)S, (int)T, (int)(T1 == T), 0,
+                                     status_for(px, bnd), stream_of(px)),
+               "frnnt_mi_kept_fwd");
+      variable_list save{kept};
+      if (bnd.defined()) save.push_back(bnd);
+      ctx->save_for_backward(std::move(save));
+      ctx->saved_data["sizes"] = std::vector<int64_t>{B, S, T1, T};
+      return {scores};
+    }
+    Tensor p = at::empty({B, S + 1, T + 1}, opts), gx, gy;
     if (want_grads || need_grad) {
       gx = at::empty({B, S, T1}, opts);
       gy = at::empty({B, S + 1, T}, opts);
-    }
-    if (need_grad && !want_grads && px.scalar_type() == at::kFloat) {
-      check_rc(frnnt_mi_shares_fwd_f32(ptr<float>(px), ptr<float>(py), iptr(bnd), ptr<float>(p),
-                                       ptr<float>(scores), ptr<float>(gx), ptr<float>(gy), (int)B,
-                                       (int)S, (int)T, (int)(T1 == T), 0, status_for(px, bnd),
-                                       stream_of(px)),
-               "frnnt_mi_shares_fwd");
-      variable_list save{gx, gy, p};
-      if (bnd.defined()) save.push_back(bnd);
-      ctx->save_for_backward(std::move(save));
-      return {scores};
     }
     auto run = [&](auto r) {
       using R = decltype(r);
@@ -429,23 +430,31 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     if (!grads[0].defined()) return variable_list(5);
     const auto saved = ctx->get_saved_variables();
-    Tensor gx = saved[0], gy = saved[1];
+    const auto sizes = ctx->saved_data.find("sizes");
+    const bool of_shares = sizes != ctx->saved_data.end();
+    DeviceGuard guard(saved[0].device());
+    Tensor gx, gy;
+    if (of_shares) {
+      const auto n = sizes->second.toIntVector();
+      gx = at::empty({n[0], n[1], n[2]}, saved[0].options());
+      gy = at::empty({n[0], n[1] + 1, n[3]}, saved[0].options());
+    } else {
+      gx = saved[0];
+      gy = saved[1];
+    }
     const int64_t B = gx.size(0), S = gx.size(1), T1 = gx.size(2), T = gy.size(2);
-    DeviceGuard guard(gx.device());
     const bool one_for_all = B > 1 && grads[0].stride(0) == 0;  // (e.g. of a sum)
     const Tensor g = one_for_all ? grads[0] : grads[0].contiguous();
     const bool on_record = at::GradMode::is_enabled() && g.requires_grad();
-    if (saved.size() > 2) {
-      const Tensor bnd = saved.size() > 3 ? saved[3] : Tensor();
-      check_rc(frnnt_mi_shares_bwd_f32(iptr(bnd), ptr<float>(saved[2]),
-                                       on_record ? nullptr : ptr<float>(g), one_for_all ? 0 : 1,
-                                       ptr<float>(gx), ptr<float>(gy), (int)B, (int)S, (int)T,
-                                       (int)(T1 == T), stream_of(gx)),
-               "frnnt_mi_shares_bwd");
-      if (!on_record) {
-        count_as_changed(gx, gy);
-        return {gx, gy, Tensor(), Tensor(), Tensor()};
-      }
+    if (of_shares) {
+      const Tensor bnd = saved.size() > 1 ? saved[1] : Tensor();
+      check_rc(frnnt_mi_kept_bwd_f32(iptr(bnd), ptr<float>(saved[0]), on_record ? nullptr : ptr<float>(g),
+                                     one_for_all ? 0 : 1, ptr<float>(gx), ptr<float>(gy), (int)B, (int)S,
+                                     (int)T, (int)(T1 == T), stream_of(gx)),
+               "frnnt_mi_kept_bwd");
+      // (a second backward is refused as where the gradients are scaled in place)
+      saved[0].unsafeGetTensorImpl()->bump_version();
+      if (!on_record) return {gx, gy, Tensor(), Tensor(), Tensor()};
     }
     if (on_record) {
       // (differentiated itself, e.g. with respect to weights of the scores: an operation on record)

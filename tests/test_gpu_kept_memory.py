@@ -45,3 +45,19 @@ def test_backward_of_the_recursion_allocates_no_lattices(gpu_device):
     grads = torch.autograd.grad(total, (px, py))
     assert torch.cuda.max_memory_allocated() - before < occupation[0].numel() * 4
     assert all(torch.equal(a, b) for a, b in zip(grads, occupation))
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("B,S,T", [(4, 60, 300), (4, 200, 900)])
+def test_memory_that_the_recursion_keeps(gpu_device, B, S, T, modified):
+    """One lattice -- not the gradients, which are formed in the backward."""
+    g = torch.Generator().manual_seed(2)
+    px = torch.randn(B, S, T if modified else T + 1, generator=g).to(gpu_device).requires_grad_(True)
+    py = torch.randn(B, S + 1, T, generator=g).to(gpu_device).requires_grad_(True)
+    boundary = torch.tensor([[0, 0, S, T]] * B).to(gpu_device)
+    fast_rnnt_amd.mutual_information_recursion(px, py, boundary).sum().backward()
+    before = torch.cuda.memory_allocated()
+    scores = fast_rnnt_amd.mutual_information_recursion(px, py, boundary)
+    # (the scores; the shares, with a row for each seam between bands of 64 rows; in multiples of 512 bytes)
+    assert torch.cuda.memory_allocated() - before <= 4 * B * (S + 1 + S // 64) * (T + 1) + 2 * 512
+    scores.sum().backward()

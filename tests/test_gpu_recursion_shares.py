@@ -95,27 +95,31 @@ def test_what_the_scratch_held_before(modified, value):
 
 
 # one band, two together, two, three and four apart
+@pytest.mark.parametrize("kept", [False, True])
 @pytest.mark.parametrize("modified", [False, True])
 @pytest.mark.parametrize("B,S,T", [(5, 20, 33), (5, 100, 90), (4, 100, 1300), (4, 150, 200), (3, 250, 700)])
-def test_backward_again_on_the_same_shares(B, S, T, modified):
+def test_backward_again_on_the_same_shares(B, S, T, modified, kept):
     """With another gradient of the scores, into buffers that hold anything, those of the first call among them: what
-    a first call on shares of their own forms."""
+    a first call on shares of their own forms.  With and without the room behind the shares."""
     px, py, g = _inputs(B, S, T, modified, S)
     px, py, boundary = px.cuda(), py.cuda(), _window(B, S, T, g).cuda()
     lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    room = lib.frnnt_mi_kept_size(B, S, T)
+    assert room >= B * (S + 1) * (T + 1)
 
     def forward():
-        shares, scores = torch.empty(B, S + 1, T + 1, device="cuda"), torch.empty(B, device="cuda")
-        scratch = torch.empty_like(px), torch.empty_like(py)
-        assert lib.frnnt_mi_shares_fwd_f32(
-            px.data_ptr(), py.data_ptr(), boundary.data_ptr(), shares.data_ptr(), scores.data_ptr(),
-            scratch[0].data_ptr(), scratch[1].data_ptr(), B, S, T, int(modified), 0, None, stream) == 0
+        shares = torch.full((room if kept else B * (S + 1) * (T + 1),), 7.0, device="cuda")
+        scores, scratch = torch.empty(B, device="cuda"), torch.empty_like(py)
+        ins, rest = [x.data_ptr() for x in (px, py, boundary, shares, scores)], (B, S, T, int(modified), 0, None, stream)
+        rc = (lib.frnnt_mi_kept_fwd_f32(*ins, *rest) if kept else
+              lib.frnnt_mi_shares_fwd_f32(*ins, None, scratch.data_ptr(), *rest))
+        assert rc == 0
         return shares
 
     def backward(shares, seeds, grads):
-        assert lib.frnnt_mi_shares_bwd_f32(boundary.data_ptr(), shares.data_ptr(), seeds.data_ptr(), 1,
-                                           grads[0].data_ptr(), grads[1].data_ptr(), B, S, T, int(modified),
-                                           stream) == 0
+        call = lib.frnnt_mi_kept_bwd_f32 if kept else lib.frnnt_mi_shares_bwd_f32
+        assert call(boundary.data_ptr(), shares.data_ptr(), seeds.data_ptr(), 1, grads[0].data_ptr(),
+                    grads[1].data_ptr(), B, S, T, int(modified), stream) == 0
         return [x.clone() for x in grads]
 
     one, two = torch.linspace(1, 3, B, device="cuda"), torch.linspace(-2, 0.5, B, device="cuda")
@@ -207,3 +211,30 @@ def test_gradient_of_a_gradient_formed_in_the_backward():
     assert torch.equal(gx.detach(), occ_x * weight.detach().reshape(-1, 1, 1))
     (gw,) = torch.autograd.grad(gx.sum(), weight)
     assert torch.allclose(gw, occ_x.sum(dim=(1, 2)), rtol=1e-5)
+
+
+@pytest.mark.parametrize("B,S,T", [(5, 100, 90), (4, 150, 300)])
+def test_recursion_and_its_backward_in_a_graph(B, S, T):
+    """Replays on other inputs, with eager calls between them: each finds the room between the workgroups as it
+    was."""
+    px, py, g = _inputs(B, S, T, False, S)
+    px, py, boundary = px.cuda().requires_grad_(), py.cuda().requires_grad_(), _window(B, S, T, g).cuda()
+    seeds = torch.linspace(0.5, 2, B, device="cuda")
+
+    def step():
+        scores = F.mutual_information_recursion(px, py, boundary)
+        return scores, *torch.autograd.grad(scores, (px, py), seeds)
+
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for n in range(3):
+        with torch.no_grad():
+            px.add_(0.25)
+        want = step()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, want):
+            assert torch.equal(a, b)
