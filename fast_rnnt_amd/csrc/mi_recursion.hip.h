@@ -493,13 +493,14 @@ __global__ void __launch_bounds__(256)
 // kApart: a workgroup per band; `pitch` workgroups per band, one per utterance (of B).
 // kShares: what a cell hands down of its gradient, d1 = exp(term1 - p), is stored in the place of p (see
 // the backward kernel); the seams of workgroups apart then go through `mail` (see mail_row; posted: post_row).
+// rows (may be NULL): takes a copy of the boundary.
 template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart, bool kShares>
 __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)) * kWave)
     mi_forward_kernel(const R *__restrict__ px, const R *__restrict__ py,
                       const int64_t *__restrict__ boundary, R *__restrict__ p,
                       R *__restrict__ ans, int S, int T, int spin_limit, int checks,
-                      int *__restrict__ status, int B, int pitch, R *mail, int posted, R *loss,
-                      int reduction, int *arrived) {
+                      int *__restrict__ status, int B, int pitch, R *mail, int posted, int64_t *rows,
+                      R *loss, int reduction, int *arrived) {
   // (lattices of one band -- a cap of one sweep wave -- have no seams)
   constexpr bool kSeams = kApart || kSweepCap > 1;
   extern __shared__ __align__(16) unsigned char dyn_lds[];
@@ -525,6 +526,8 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
     if ((checks & kCheckSymbols) && win.s0 + win.ns < 1) bad = kStatusNoSymbols;
     else if ((checks & kCheckFrames) && win.t0 + win.nt < win.s0 + win.ns) bad = kStatusFewFrames;
   }
+  if (kShares && rows && boundary && part == 0 && threadIdx.x < 4)
+    rows[4 * b + threadIdx.x] = boundary[4 * b + threadIdx.x];
   // What the lane that holds the utterance's score does with it (not apart: `loss` is NULL there), and, in the
   // workgroup that comes last, the rest of its wave: the loss, for which no launch of its own is then needed (a
   // validation pass of two small kernels, B 5, S 19, T 77, C 131, float16, 14.7 -> 12.6 us).
@@ -1767,12 +1770,13 @@ inline void mark_seams(const int64_t *boundary, float *p, float *mail, float *an
   hipLaunchKernelGGL(mark_seams_kernel, dim3(B, (S + kWave) / kWave - 1), dim3(256), 0, stream,
                      boundary, p, mail, ans, px_grad, S, T, modified, (int)posted);
 }
-// What a caller's buffer holds behind the shares: the post, if there is a seam to pass.
+// What a caller's buffer holds behind the shares: the post, if there is a seam to pass, and a copy of the boundary.
 inline int64_t shares_floats(int B, int S, int T) { return (int64_t)B * (S + 1) * (T + 1); }
 inline int64_t post_floats(int B, int S, int T) {
   const bool seams = bands_apart<float, true>(B, S, T, false) || bands_apart<float, true>(B, S, T, true);
   return seams ? (int64_t)B * (S / kWave) * (T + 1) : 0;
 }
+inline int64_t rows_at(int B, int S, int T) { return (shares_floats(B, S, T) + post_floats(B, S, T) + 1) / 2 * 2; }
 
 // `px_grad`: if given, its seams are marked as well (for a backward_impl that follows and is told so).
 // kShares (float only): p is filled for a backward_impl with kShares; py_grad is its py_grad or, posted, the post of both.
@@ -1780,7 +1784,8 @@ inline int64_t post_floats(int B, int S, int T) {
 template <typename R, bool kShares = false>
 int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans, int B, int S,
                  int T, int modified, void *stream, int checks = 0, int *status = nullptr,
-                 R *px_grad = nullptr, R *py_grad = nullptr, LossOf<R> *loss = nullptr, bool posted = false) {
+                 R *px_grad = nullptr, R *py_grad = nullptr, LossOf<R> *loss = nullptr, bool posted = false,
+                 int64_t *rows = nullptr) {
   static_assert(!kShares || sizeof(R) == 4, "shares are float's");
   R *loss_out = loss && loss->out && (loss->reduction == 0 || loss->arrived) ? loss->out : nullptr;
   const int reduction = loss ? loss->reduction : 0;
@@ -1818,7 +1823,8 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
         return check_launch("mi_forward: hipFuncSetAttribute");
       hipLaunchKernelGGL(kernel, dim3(pitch * ((S + kWave) / kWave)), dim3((3 + kOne) * kWave), lds,
                          static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T,
-                         mi_spin_limit, checks, status, B, pitch, py_grad, (int)posted, nullptr, 0, nullptr);
+                         mi_spin_limit, checks, status, B, pitch, py_grad, (int)posted, rows, nullptr, 0,
+                         nullptr);
       return check_launch("mi_forward");
     }
   }
@@ -1835,7 +1841,7 @@ int forward_impl(const R *px, const R *py, const int64_t *boundary, R *p, R *ans
     return check_launch("mi_forward: hipFuncSetAttribute");
   hipLaunchKernelGGL(kernel, dim3(B), dim3(n * (1 + stagers) * kWave), lds,
                      static_cast<hipStream_t>(stream), px, py, boundary, p, ans, S, T, mi_spin_limit,
-                     checks, status, B, B, py_grad, (int)posted, loss_out, reduction, arrived);
+                     checks, status, B, B, py_grad, (int)posted, rows, loss_out, reduction, arrived);
   if (loss) loss->formed = loss_out != nullptr;
   return check_launch("mi_forward");
 }

@@ -40,13 +40,16 @@ extern "C" int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const i
 
 extern "C" int64_t frnnt_mi_kept_size(int B, int S, int T) {
   if (B < 1 || S < 0 || T < 0) return 0;
-  return frnnt::shares_floats(B, S, T) + frnnt::post_floats(B, S, T);
+  return frnnt::rows_at(B, S, T) + 8 * (int64_t)B;
 }
 extern "C" int frnnt_mi_kept_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *kept,
                                      float *scores, int B, int S, int T, int modified, int checks,
                                      int32_t *status, void *stream) {
   using namespace frnnt;
-  float *post = kept && B > 0 && S >= 0 && T >= 0 ? kept + shares_floats(B, S, T) : nullptr;
+  const bool room = kept && B > 0 && S >= 0 && T >= 0;
+  float *post = room ? kept + shares_floats(B, S, T) : nullptr;
+  int64_t *rows = room ? reinterpret_cast<int64_t *>(kept + rows_at(B, S, T)) : nullptr;
+  if (reinterpret_cast<uintptr_t>(rows) & 7) return fail(FRNNT_EINVAL, "mi_kept_fwd: kept not aligned to 8 bytes");
   return forward_impl<float, true>(px, py, boundary, kept, scores, B, S, T, modified, stream, checks, status,
-                                   nullptr, post, nullptr, true);
+                                   nullptr, post, nullptr, true, rows);
 }

@@ -384,7 +384,8 @@ struct RecursionLossFn : public torch::autograd::Function<RecursionLossFn> {
 // in-place scaling in the backward.  Unless they are handed out nobody else holds them by then, so
 // that px.grad and py.grad take them over without a copy; and in float32 they are formed then, from
 // the gradient of the scores, instead of in the forward and scaled afterwards (a pass over both:
-// 12 us of 144 at B 12, S 220, T 1500).  Kept until then are the shares, one lattice, instead of two.
+// 12 us of 144 at B 12, S 220, T 1500).  Kept until then are the shares, one lattice
+// instead of two, and a copy of the boundary: the caller may write to its own.
 struct RecursionFn : public torch::autograd::Function<RecursionFn> {
   static variable_list forward(AutogradContext *ctx, const Tensor &px_, const Tensor &py_,
                                const std::optional<Tensor> &boundary_, bool want_grads,
@@ -403,10 +404,8 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
                                      ptr<float>(scores), (int)B, (int)S, (int)T, (int)(T1 == T), 0,
                                      status_for(px, bnd), stream_of(px)),
                "frnnt_mi_kept_fwd");
-      variable_list save{kept};
-      if (bnd.defined()) save.push_back(bnd);
-      ctx->save_for_backward(std::move(save));
-      ctx->saved_data["sizes"] = std::vector<int64_t>{B, S, T1, T};
+      ctx->save_for_backward({kept});
+      ctx->saved_data["sizes"] = std::vector<int64_t>{B, S, T1, T, bnd.defined()};
       return {scores};
     }
     Tensor p = at::empty({B, S + 1, T + 1}, opts), gx, gy;
@@ -434,8 +433,10 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
     const bool of_shares = sizes != ctx->saved_data.end();
     DeviceGuard guard(saved[0].device());
     Tensor gx, gy;
+    int has_boundary = 0;
     if (of_shares) {
       const auto n = sizes->second.toIntVector();
+      has_boundary = (int)n[4];
       gx = at::empty({n[0], n[1], n[2]}, saved[0].options());
       gy = at::empty({n[0], n[1] + 1, n[3]}, saved[0].options());
     } else {
@@ -447,8 +448,7 @@ struct RecursionFn : public torch::autograd::Function<RecursionFn> {
     const Tensor g = one_for_all ? grads[0] : grads[0].contiguous();
     const bool on_record = at::GradMode::is_enabled() && g.requires_grad();
     if (of_shares) {
-      const Tensor bnd = saved.size() > 1 ? saved[1] : Tensor();
-      check_rc(frnnt_mi_kept_bwd_f32(iptr(bnd), ptr<float>(saved[0]), on_record ? nullptr : ptr<float>(g),
+      check_rc(frnnt_mi_kept_bwd_f32(ptr<float>(saved[0]), has_boundary, on_record ? nullptr : ptr<float>(g),
                                      one_for_all ? 0 : 1, ptr<float>(gx), ptr<float>(gy), (int)B, (int)S,
                                      (int)T, (int)(T1 == T), stream_of(gx)),
                "frnnt_mi_kept_bwd");

@@ -143,14 +143,15 @@ int frnnt_mi_shares_bwd_f32(const int64_t *boundary, const float *shares, const 
                             int score_grad_stride, float *px_grad, float *py_grad, int B, int S, int T,
                             int modified, void *stream);
 /*
- * The same for a caller whose buffer has frnnt_mi_kept_size() floats: what _bwd needs and, behind the shares, room in
- * which both pass on what a launch of several workgroups per utterance exchanges.  _fwd takes no scratch, and _bwd
- * has a launch less.  _bwd may be called again (it leaves `kept` as it was), but not by two streams at once.
+ * The same for a caller whose buffer has frnnt_mi_kept_size() floats, aligned to 8 bytes: all that _bwd needs, the
+ * boundary's rows among it (has_boundary: whether _fwd had one), and room in which both pass on what a launch of
+ * several workgroups per utterance exchanges.  _fwd takes no scratch, and _bwd has a launch less.  _bwd may be called
+ * again (it leaves `kept` as it was), but not by two streams at once.
  */
 int64_t frnnt_mi_kept_size(int B, int S, int T);
 int frnnt_mi_kept_fwd_f32(const float *px, const float *py, const int64_t *boundary, float *kept, float *scores,
                           int B, int S, int T, int modified, int checks, int32_t *status, void *stream);
-int frnnt_mi_kept_bwd_f32(const int64_t *boundary, float *kept, const float *score_grad, int score_grad_stride,
+int frnnt_mi_kept_bwd_f32(float *kept, int has_boundary, const float *score_grad, int score_grad_stride,
                           float *px_grad, float *py_grad, int B, int S, int T, int modified, void *stream);
 
 /*

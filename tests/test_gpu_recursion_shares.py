@@ -117,9 +117,10 @@ def test_backward_again_on_the_same_shares(B, S, T, modified, kept):
         return shares
 
     def backward(shares, seeds, grads):
-        call = lib.frnnt_mi_kept_bwd_f32 if kept else lib.frnnt_mi_shares_bwd_f32
-        assert call(boundary.data_ptr(), shares.data_ptr(), seeds.data_ptr(), 1, grads[0].data_ptr(),
-                    grads[1].data_ptr(), B, S, T, int(modified), stream) == 0
+        rest = (seeds.data_ptr(), 1, grads[0].data_ptr(), grads[1].data_ptr(), B, S, T, int(modified), stream)
+        rc = (lib.frnnt_mi_kept_bwd_f32(shares.data_ptr(), 1, *rest) if kept else
+              lib.frnnt_mi_shares_bwd_f32(boundary.data_ptr(), shares.data_ptr(), *rest))
+        assert rc == 0
         return [x.clone() for x in grads]
 
     one, two = torch.linspace(1, 3, B, device="cuda"), torch.linspace(-2, 0.5, B, device="cuda")
@@ -237,4 +238,24 @@ def test_recursion_and_its_backward_in_a_graph(B, S, T):
         graph.replay()
         torch.cuda.synchronize()
         for a, b in zip(out, want):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("B,S,T", [(1, 1, 1), (5, 20, 33), (5, 100, 90), (4, 150, 300), (3, 300, 320)])
+def test_boundary_written_to_between_forward_and_backward(B, S, T, modified):
+    """A program may fill one boundary buffer for one recursion after the other, as when the gradients were formed in
+    the forward: they are those of the rows that the scores were formed with."""
+    px, py, g = _inputs(B, S, T, modified, S)
+    px, py = px.cuda().requires_grad_(), py.cuda().requires_grad_()
+    one, two = _window(B, S, T, g).cuda(), _window(B, S, T, g).flip(0).cuda()
+    want = [torch.autograd.grad(F.mutual_information_recursion(px, py, rows.clone()).sum(), (px, py))
+            for rows in (one, two)]
+    buffer = one.clone()
+    first = F.mutual_information_recursion(px, py, buffer)
+    buffer.copy_(two)
+    second = F.mutual_information_recursion(px, py, buffer)
+    buffer.zero_()
+    for scores, grads in ((second, want[1]), (first, want[0])):
+        for a, b in zip(torch.autograd.grad(scores.sum(), (px, py)), grads):
             assert torch.equal(a, b)
