@@ -227,11 +227,15 @@ __device__ __forceinline__ void row_stats(const float *__restrict__ x, const flo
 // A wave per lm row: its statistics.  Then, with an am-only model, the block's part of the unigram (the sum
 // of its rows' softmax, as weighted_column_partial_kernel forms it: one launch and a read of lm from memory
 // less, 5.3 + 6.7 -> 6.2 us at B 32, S 80, C 500), without one its check: 0, or a NaN where a row has no
-// softmax (4.4 us).
+// softmax (4.4 us).  On the way, a copy of the boundary (in words: the buffer's alignment is the caller's) for a
+// backward whose caller may have written to its own by then.
 template <bool kUnigram>
 __global__ void __launch_bounds__(kRowsPerBlock *kWave)
     lm_models_kernel(const float *__restrict__ lm, float *__restrict__ row_max,
-                     float *__restrict__ row_sum, float *__restrict__ partial, long rows, int C) {
+                     float *__restrict__ row_sum, float *__restrict__ partial, long rows, int C,
+                     const int *__restrict__ boundary, int *__restrict__ boundary_copy, long words) {
+  const long word = (long)blockIdx.x * (kRowsPerBlock * kWave) + threadIdx.x;
+  if (boundary && word < words) boundary_copy[word] = boundary[word];
   __shared__ float max_of[kRowsPerBlock], weight_of[kRowsPerBlock];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long row0 = (long)blockIdx.x * kRowsPerBlock, row = row0 + wave;
@@ -896,9 +900,9 @@ int bwd_impl(const R *lm, const R *am, const int64_t *symbols, const int64_t *bo
 
 // ---- the whole loss in float32 -----------------------------------------------------------------
 // What its backward keeps: [S1 rows of lm] max (joint), max, sum; [T frames of am] max (joint), max,
-// z; unigram; the joint normalizers.
+// z; unigram; the joint normalizers; the boundary's rows.
 struct Kept {
-  float *lm_max, *s_lm_max, *lm_sum, *am_max, *s_am_max, *am_z, *unigram, *norm_raw;
+  float *lm_max, *s_lm_max, *lm_sum, *am_max, *s_am_max, *am_z, *unigram, *norm_raw, *rows;
   size_t floats;
 };
 // Whether a scale asks for an am-only model.  The reference takes 1e-20 in place of 0 (rnnt_loss.py:1346-1351)
@@ -917,6 +921,7 @@ Kept keep_of(float *base, long B, long S, long T, long C) {
   k.lm_max = take(B * (S + 1)), k.s_lm_max = take(B * (S + 1)), k.lm_sum = take(B * (S + 1));
   k.am_max = take(B * T), k.s_am_max = take(B * T), k.am_z = take(B * T);
   k.unigram = take(C), k.norm_raw = take(B * (S + 1) * T);
+  k.rows = take(8 * B);
   k.floats = at;
   return k;
 }
@@ -1002,7 +1007,8 @@ int frnnt_smoothed_loss_fwd_f32(const float *lm, const float *am, const int64_t 
   const int blocks = (int)((n_lm + kRowsPerBlock - 1) / kRowsPerBlock);
   if (B > 0)
     hipLaunchKernelGGL((am_model ? lm_models_kernel<true> : lm_models_kernel<false>), dim3(blocks),
-                       dim3(kRowsPerBlock * kWave), 0, on, lm, k.s_lm_max, k.lm_sum, partial, n_lm, C);
+                       dim3(kRowsPerBlock * kWave), 0, on, lm, k.s_lm_max, k.lm_sum, partial, n_lm, C,
+                       reinterpret_cast<const int *>(boundary), reinterpret_cast<int *>(k.rows), 8L * B);
   if (B > 0 && am_model) {
     hipLaunchKernelGGL(unigram_final_kernel<float>, dim3((C + kColsPerBlock - 1) / kColsPerBlock),
                        dim3(kUnigramThreads), 0, on, partial, k.unigram, blocks, n_lm, C);

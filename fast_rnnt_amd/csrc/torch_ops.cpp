@@ -729,10 +729,13 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
                  (int)checks | FRNNT_LARGE_SCRATCH, status_for(am, bnd), stream_of(am)),
              "frnnt_smoothed_loss_fwd");
     if (need_grad) {
+      // (the constrained lattice's backward reads the copy of the boundary in `kept`: its caller may write to the
+      // tensor itself, as where the backward did not need it)
       variable_list save{lm, am, sym, kept, gx, gy};
-      if (bnd.defined()) save.push_back(bnd);
+      const bool copied = kind == 2 && bnd.defined();
+      if (bnd.defined() && !copied) save.push_back(bnd);
       ctx->save_for_backward(std::move(save));
-      ctx->saved_data["meta"] = std::vector<int64_t>{term, kind, reduction};
+      ctx->saved_data["meta"] = std::vector<int64_t>{term, kind, reduction, copied};
       ctx->saved_data["scales"] = std::vector<double>{lm_scale, am_scale};
     }
     if (!gx.defined()) return {loss};
@@ -752,6 +755,8 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
     const std::vector<double> scales = ctx->saved_data["scales"].toDoubleVector();
     const int64_t reduction = meta[2];
     const int64_t B = am.size(0), T = am.size(1), C = am.size(2), S = lm.size(1) - 1;
+    const int64_t *rows =
+        meta[3] ? reinterpret_cast<const int64_t *>(ptr<float>(kept) + kept.numel() - 8 * B) : iptr(bnd);
     DeviceGuard guard(am.device());
     const Tensor g = g_loss.contiguous();
     const Tensor scratch =
@@ -760,7 +765,7 @@ struct SmoothedLossFn : public torch::autograd::Function<SmoothedLossFn> {
     out[0] = at::empty(lm.sizes(), lm.options());
     out[1] = at::empty(am.sizes(), am.options());
     check_rc(frnnt_smoothed_loss_bwd_f32(
-                 ptr<float>(lm), ptr<float>(am), iptr(sym), iptr(bnd), ptr<float>(kept),
+                 ptr<float>(lm), ptr<float>(am), iptr(sym), rows, ptr<float>(kept),
                  ptr<float>(g), reduction == kRedNone ? 1 : 0,
                  reduction == kRedMean ? -1.0 / (double)B : -1.0, ptr<float>(gx), ptr<float>(gy),
                  ptr<float>(scratch), ptr<float>(out[0]), ptr<float>(out[1]), (int)B, (int)S, (int)T,

@@ -312,7 +312,8 @@ int frnnt_smoothed_logprobs_bwd_f64(const double *lm, const double *am, const in
  * and py_grad in place as frnnt_simple_logprobs_bwd does (score_grad is required) and forms the
  * whole lm_grad and am_grad: the terms of both unigram models inside the joint model's gradient
  * products.
- *   kept: frnnt_smoothed_loss_kept() floats, written by _fwd for _bwd
+ *   kept: frnnt_smoothed_loss_kept() floats, written by _fwd for _bwd; the last 8 B are a copy of the
+ *     boundary (if there is one), which _bwd may be given for it
  *   px, py, p, scores: as in those entry points, not needed afterwards (p is scratch); px_joint, py_joint: not used
  *   partial [ceil(B*(S+1)/16)][C]: scratch
  *   scratch of _bwd: B (S+1) (4 + T rounded up to 4) + 2 B T + C + ceil(B*T/16) C floats, each

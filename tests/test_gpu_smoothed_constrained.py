@@ -43,3 +43,28 @@ def test_constrained_smoothed_loss(gpu_device, B, S, T, C):
                 off = (x.grad.cpu() - y.grad).abs()
                 # (the tolerance of the other lattices' gradients, whose bf16-split products these are)
                 assert bool((off <= 2e-4 + 1e-4 * y.grad.abs()).all()), off.max().item()
+
+
+@pytest.mark.parametrize("am_scale", [0.0, 0.1])
+def test_boundary_written_to_between_forward_and_backward(gpu_device, am_scale):
+    """The gradients are those of the rows that the loss was formed with: a program may fill one boundary buffer for one
+    batch after the other."""
+    B, S, T, C = 5, 20, 70, 33
+    g = torch.Generator().manual_seed(0)
+    lm, am = (torch.randn(B, n, C, generator=g).to(gpu_device).requires_grad_() for n in (S + 1, T))
+    symbols = torch.randint(0, C, (B, S), generator=g).to(gpu_device)
+    one, two = (torch.tensor([[0, 0, s, t]] * B).to(gpu_device) for s, t in ((S, T), (S - 7, T - 30)))
+
+    def loss(boundary):
+        return fast_rnnt_amd.rnnt_loss_smoothed(lm, am, symbols, 0, 0.25, am_scale, boundary=boundary,
+                                                rnnt_type="constrained", reduction="sum")
+
+    want = [torch.autograd.grad(loss(rows.clone()), (lm, am)) for rows in (one, two)]
+    buffer = one.clone()
+    first = loss(buffer)
+    buffer.copy_(two)
+    second = loss(buffer)
+    buffer.zero_()
+    for value, grads in ((second, want[1]), (first, want[0])):
+        for a, b in zip(torch.autograd.grad(value, (lm, am)), grads):
+            assert torch.equal(a, b)
