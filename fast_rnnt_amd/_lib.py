@@ -55,6 +55,7 @@ _SIGNATURES = {
     "frnnt_loss_scratch": ([_I] * 5, ctypes.c_int64),
     "frnnt_mi_shares_fwd_f32": ([_P] * 7 + [_I] * 5 + [_P, _P], _I),
     "frnnt_mi_shares_bwd_f32": ([_P] * 3 + [_I] + [_P] * 2 + [_I] * 4 + [_P], _I),
+    "frnnt_mi_route": ([_I] * 4, _I),
     "frnnt_mi_kept_size": ([_I] * 3, ctypes.c_int64),
     "frnnt_mi_kept_fwd_f32": ([_P] * 5 + [_I] * 5 + [_P, _P], _I),
     "frnnt_mi_kept_bwd_f32": ([_P, _I, _P, _I] + [_P] * 2 + [_I] * 4 + [_P], _I),

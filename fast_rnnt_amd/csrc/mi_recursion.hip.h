@@ -1741,8 +1741,9 @@ size_t apart_lds_bytes(int T) {
 // both measured (microseconds, nanoseconds), for 2, 3 and 4 bands.
 // (B 12, S 220, T 1500: 134 + 164 -> 72 + 80 us; B 3, S 250, T 1335: 120 + 149 -> 67 + 74;
 // B 10, S 137, T 817: 51 + 60 -> 43 + 48.)
-// Both seam rows must fit into LDS (T up to 12 988; the other launch goes to 30 700).  Two workgroups
-// share a compute unit while their LDS allows it (T up to 3 004).  Beyond, a band that finds no unit
+// Both seam rows must fit into LDS (T up to 12 988; the other launch goes to 30 700).  Two workgroups of the
+// forward kernel share a compute unit while their LDS allows it (T up to 3 004; the backward's ten waves have too
+// many registers for that).  Otherwise a band that finds no unit
 // of its own starts when an earlier one is done: two bands, which one workgroup sweeps almost as fast
 // as two, then stay together (B 136, S 100, T 6000: 595 + 599 apart, 407 + 555 together; B 136, S 70,
 // T 5000: 443 + 438, 281 + 318); three and four are still better off apart (B 128, S 250, T 5000:
@@ -1752,13 +1753,20 @@ size_t apart_lds_bytes(int T) {
 // while each has a compute unit: forward and backward with the marks, together and apart, B 8, S 130, T 140: 41.5 and
 // 37.9 us; S 160, T 300: 58.5 and 48.2; T 600: 85 and 64; B 64, S 190, T 200: 56.5 and 49.0.  (With more
 // of them than units the rule is that of the other kernels: B 100, S 130, T 600: 88 and 92; B 168, S 160, T 300: 67 and 74.  Two bands
-// gain from where they did: B 24, S 80, T 600: 55.7 and 56.3; T 900: 72.5 and 71.1.)
+// gain from where they did: B 24, S 80, T 600: 55.7 and 56.3; T 900: 72.5 and 71.1.)  Their workgroups, of eleven waves
+// with 88 registers and fifteen with 65, have a unit each whatever their LDS (a unit's registers hold 20 and 28 such
+// waves), so that two bands stay together as soon as there are more of them than units: together and
+// apart, both kernels and the marks, ragged batches of up to S 100, T 1500: B 128 159 and 138, B 160 178 and 203, B 256
+// 274 and 288; S 100, T 3000, B 160: 378 and 423; S 70, T 3000, B 200: 310 and 382.  Three and four gain apart with two
+// to a unit's place as well (S 130, T 1500, B 100: 211 and 147; S 190, T 3000, B 168: 764 and 656; S 250, T 1500, B 128:
+// 466 and 335).
 template <typename R, bool kShares>
 bool bands_apart(int B, int S, int T, bool backward) {
   const int bands = (S + kWave) / kWave;
   if (sizeof(R) != 4 || bands < 2 || bands > kMaxSweep || T < 1) return false;
-  const size_t per_cu = kLdsBudget / apart_lds_bytes(T);
+  size_t per_cu = kLdsBudget / apart_lds_bytes(T);
   if (per_cu == 0) return false;
+  if (kShares) per_cu = 1;
   const long workgroups = (long)((B + 7) / 8 * 8) * bands;
   if (workgroups > (bands == 2 && per_cu == 1 ? 256 : 512)) return false;
   if (kShares && bands == 3 && workgroups <= 256) return true;

@@ -38,6 +38,14 @@ extern "C" int frnnt_mi_shares_fwd_f32(const float *px, const float *py, const i
                                   nullptr, py_grad, stream);
 }
 
+extern "C" int frnnt_mi_route(int B, int S, int T, int shares) {
+  using namespace frnnt;
+  if (B < 1 || S < 0 || T < 0) return fail(FRNNT_EINVAL, "mi_route: bad size");
+  const bool forward = shares ? bands_apart<float, true>(B, S, T, false) : bands_apart<float, false>(B, S, T, false);
+  const bool backward = shares ? bands_apart<float, true>(B, S, T, true) : bands_apart<float, false>(B, S, T, true);
+  return (forward ? 1 : 0) | (backward ? 2 : 0) | (mi_shares_pay(B, S, T) ? 4 : 0);
+}
+
 extern "C" int64_t frnnt_mi_kept_size(int B, int S, int T) {
   if (B < 1 || S < 0 || T < 0) return 0;
   return frnnt::rows_at(B, S, T) + 8 * (int64_t)B;

@@ -155,6 +155,13 @@ int frnnt_mi_kept_bwd_f32(float *kept, int has_boundary, const float *score_grad
                           float *px_grad, float *py_grad, int B, int S, int T, int modified, void *stream);
 
 /*
+ * How a float32 recursion of this size is launched (host only, e.g. for tests): bit 0, 1: the forward's, the backward's
+ * bands of 64 rows have workgroups of their own, in the kernels that pass shares (shares != 0) or p; bit 2: a loss
+ * passes shares.
+ */
+int frnnt_mi_route(int B, int S, int T, int shares);
+
+/*
  * px / py of the simple (additive-joiner) RNN-T loss.  Replaces the tensor
  * algebra of get_rnnt_logprobs (fast_rnnt/python/fast_rnnt/rnnt_loss.py:66-227):
  * row maxima, the exp(lm) exp(am)^T contraction (fp32 / fp64 MFMA with the
