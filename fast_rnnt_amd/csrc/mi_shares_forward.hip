@@ -11,7 +11,10 @@ namespace frnnt {
 // some 200 frames on (S 90, B 32, T 100: 22.9 and 24.3; T 200: 30.0 and 30.5; T 350: 41.2 and 40.5; S 120, B 100, T 500:
 // 57.0 and 51.6); with three and four, which have three staging waves each, later (B 100, S 160, T 260: 53.2 and 60.1; T
 // 450: 77.1 and 76.2; B 168, S 190, T 350: 93.2 and 90.1; T 900: 230 and 185).  Bands apart have the marks to make up
-// for (B 4, S 130, T 100: 33.5 and 34.4; T 140: 36.8 and 35.0).
+// for (B 4, S 130, T 100: 33.5 and 34.4; T 140: 36.8 and 35.0).  More than four bands, which a workgroup takes in
+// turn, have the line of three and four together, between where large and small batches begin to gain (S 300: B 200,
+// T 400: 211 and 181; B 64, T 350: 98.9 and 98.6, T 500: 121.5 and 118.5; B 16, T 400: 95.4 and 97.8, T 600: 133.6 and
+// 129.6; B 2, T 400: 93.8 and 97.5, T 700: 139.1 and 139.2; B 16, S 500, T 400: 140 and 133).
 bool mi_shares_pay(int B, int S, int T) {
   if (S < kWave) return true;
   if (S < 2 * kWave) return T >= 200;

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["regular", "modified"])
 @pytest.mark.parametrize("B,S,T", [(3, 20, 30), (3, 63, 199), (3, 64, 199), (3, 64, 200), (2, 127, 199), (2, 127, 200),
                                    (2, 128, 119), (2, 128, 120), (2, 200, 119), (2, 200, 120), (100, 130, 399),
-                                   (100, 130, 400)])
+                                   (100, 130, 400), (2, 300, 399), (2, 300, 400)])
 def test_both_sides_of_the_lines(gpu_device, B, S, T, kind):
     g = torch.Generator().manual_seed(S + T)
     C = 7

@@ -25,5 +25,13 @@ def test_more_bands_stay_apart_with_two_to_a_unit(S, T, B):
     assert _route(B, S, T, True) & FORWARD and _route(B, S, T, True) & BACKWARD
 
 
+@pytest.mark.parametrize("B,S,T,pays", [
+    (3, 63, 1, True), (3, 64, 199, False), (3, 127, 200, True), (2, 128, 119, False), (2, 255, 120, True),
+    (100, 130, 399, False), (100, 130, 400, True), (2, 256, 399, False), (2, 300, 400, True),
+])
+def test_where_losses_pass_shares(B, S, T, pays):
+    assert bool(_route(B, S, T, True) & LOSS_SHARES) == pays
+
+
 def test_bad_sizes_are_refused():
     assert _route(0, 1, 1, False) < 0 and _route(1, -1, 1, True) < 0
