@@ -165,7 +165,7 @@ struct NormArgs {
   int B, S, T, C, term, rnnt_type;
   unsigned long long *met;    // (tiles in parts) a word per tile, holding anything
   float *partial;             // kNormShares * kPartial floats per tile
-  unsigned long long ticket;  // an even number that no other call has had
+  unsigned long long ticket;  // an even number that no other call of this process has had (next_ticket)
 };
 
 // A joint model on its own
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(kWaves *kWave, (kWaves / 4 * NormShape<kS, kWa
   // (tiles in parts) Both parts' sums go through the workspace, past the XCDs' own L2: a share's cells, then
   // what follows; a part that finds the other's ticket in the tile's word comes second.  (What the word held
   // before is no ticket of this call: a call's ticket is its own, and a replay of a recorded call finds the 0
-  // that the second part leaves.)
+  // that the second part leaves, or what the recursion, whose scratch the workspace is next, has computed since.)
   const long tile_id = ((long)b * plan.t_tiles + tile.t_idx) * plan.s_tiles + tile.s_idx;
   float *const met = kParts > 1 ? A.partial + tile_id * (kNormShares * Shape::kPartial) : nullptr;
   const __amdgpu_buffer_rsrc_t met_rs = buffer_of(met, kNormShares * Shape::kPartial * 4);
@@ -667,6 +667,13 @@ __global__ void __launch_bounds__(kWaves *kWave, (kWaves / 4 * NormShape<kS, kWa
   }
 }
 
+// A ticket for a call's shared tiles, whichever of the kernels it takes.  The memory may hold anything, also small whole
+// numbers: above a count of the calls, a ticket has the bits of a signalling NaN that no arithmetic forms.
+unsigned long long next_ticket() {
+  static std::atomic<unsigned long long> calls{0};
+  return 0xffa5c3ull << 40 | (2 * calls.fetch_add(1, std::memory_order_relaxed) & ((1ull << 40) - 1));
+}
+
 template <int kS, int kWaves, int kParts, typename Mix>
 void launch_fwd_panel(NormArgs args, const NormPlan &plan, const Mix &mix, float *workspace, hipStream_t stream) {
   using Shape = NormShape<kS, kWaves, kParts>;
@@ -676,10 +683,7 @@ void launch_fwd_panel(NormArgs args, const NormPlan &plan, const Mix &mix, float
   const long tiles = (long)args.B * plan.t_tiles * plan.s_tiles;
   const unsigned grid = (unsigned)((tiles + dgemm::kXcds - 1) / dgemm::kXcds * dgemm::kXcds * kParts);
   if (kParts > 1) {
-    // The memory may hold anything, also small whole numbers: above a count of the calls, a ticket has the bits
-    // of a signalling NaN that no arithmetic forms.
-    static std::atomic<unsigned long long> calls{0};
-    args.ticket = 0xffa5c3ull << 40 | (2 * calls.fetch_add(1, std::memory_order_relaxed) & ((1ull << 40) - 1));
+    args.ticket = next_ticket();
     args.met = reinterpret_cast<unsigned long long *>(workspace);
     args.partial = workspace + (2 * tiles + 3) / 4 * 4;
   }
