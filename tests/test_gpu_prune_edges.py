@@ -25,7 +25,6 @@ def test_ranges_at_the_edges_of_the_splits(gpu_device, S, T, dtype):
         for R in (2, 3, 8, 16, 17):
             if R > S + 1:
                 continue
-            print(f"S={S} T={T} {dtype} {kind} R={R}", flush=True)
             want = O.prune_ranges(gx, gy, bnd, R, **({"window_sum": "cascade"} if R > 16 else {}))
             got = fast_rnnt_amd.get_rnnt_prune_ranges(gx.to(gpu_device), gy.to(gpu_device), bnd.to(gpu_device), R)
             assert torch.equal(got.cpu(), want)

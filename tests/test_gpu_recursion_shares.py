@@ -32,7 +32,30 @@ def _window(B, S, T, g):
     return torch.tensor(rows)
 
 
-def _compare(px, py, boundary):
+def _pair(px, py, boundary, held, kept):
+    """Scores and gradients of ones from the kernels that pass shares, whatever a loss of this size takes; the buffer
+    between them is full of `held`, and so are the gradients'."""
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    B, S, T = px.shape[0], px.shape[1], py.shape[2]
+    sizes = B, S, T, int(px.shape[2] == T)
+    n = lib.frnnt_mi_kept_size(B, S, T) if kept else B * (S + 1) * (T + 1)
+    shares, scores = torch.full((n,), held, device="cuda"), torch.full((B,), held, device="cuda")
+    gx, gy = torch.full_like(px, held), torch.full_like(py, held)
+    ins = px.data_ptr(), py.data_ptr(), None if boundary is None else boundary.data_ptr()
+    if kept:
+        assert lib.frnnt_mi_kept_fwd_f32(*ins, shares.data_ptr(), scores.data_ptr(), *sizes, 0, None, stream) == 0
+        assert lib.frnnt_mi_kept_bwd_f32(shares.data_ptr(), int(boundary is not None), None, 0, gx.data_ptr(),
+                                         gy.data_ptr(), *sizes, stream) == 0
+    else:
+        assert lib.frnnt_mi_shares_fwd_f32(*ins, shares.data_ptr(), scores.data_ptr(), None, gy.data_ptr(), *sizes, 0,
+                                           None, stream) == 0
+        assert lib.frnnt_mi_shares_bwd_f32(ins[2], shares.data_ptr(), None, 0, gx.data_ptr(), gy.data_ptr(), *sizes,
+                                           stream) == 0
+    return scores, gx, gy
+
+
+def _compare(px, py, boundary, held=math.nan):
+    """The pair in both its forms, and whichever kernels a loss of this size takes, against the two through p."""
     px, py = px.cuda(), py.cuda()
     boundary = None if boundary is None else boundary.cuda()
     B, S, T = px.shape[0], px.shape[1], py.shape[2]
@@ -40,9 +63,10 @@ def _compare(px, py, boundary):
     want = _fast_rnnt.mutual_information_forward(px, py, boundary, p)
     want_x, want_y = _fast_rnnt.mutual_information_backward(px, py, boundary, p,
                                                             torch.ones(B, device="cuda"))
-    got, (got_x, got_y) = F.mutual_information_recursion(px, py, boundary, return_grad=True)
-    for a, b in ((got, want), (got_x, want_x), (got_y, want_y)):
-        assert torch.allclose(a, b, rtol=0, atol=0, equal_nan=True)
+    score, grads = F.mutual_information_recursion(px, py, boundary, return_grad=True)
+    for got in ((score, *grads), _pair(px, py, boundary, held, False), _pair(px, py, boundary, held, True)):
+        for a, b in zip(got, (want, want_x, want_y)):
+            assert torch.allclose(a, b, rtol=0, atol=0, equal_nan=True)
     return want_x, want_y
 
 
@@ -84,13 +108,12 @@ def test_lattice_without_a_path(modified):
 
 # memory that the scratch is made of may hold anything: cells around the windows must not be felt
 @pytest.mark.parametrize("modified", [False, True])
+@pytest.mark.parametrize("S,T", [(40, 90), (100, 140), (150, 300), (100, 1300), (300, 310)])
 @pytest.mark.parametrize("value", [math.nan, math.inf, -3.0, 3e38])
-def test_what_the_scratch_held_before(modified, value):
-    px, py, g = _inputs(8, 100, 140, modified, 9)
-    boundary = _window(8, 100, 140, g)
-    free = torch.full((4, 8, 101, 141), value, device="cuda")
-    del free
-    want_x, want_y = _compare(px, py, boundary)
+def test_what_the_scratch_held_before(S, T, modified, value):
+    px, py, g = _inputs(8, S, T, modified, 9)
+    boundary = _window(8, S, T, g)
+    want_x, want_y = _compare(px, py, boundary, value)
     assert torch.isfinite(want_x).all() and torch.isfinite(want_y).all()
 
 
@@ -143,7 +166,6 @@ def test_a_wait_that_runs_out_shows_as_nan(B, S, T):
     lib = _lib.load()
     gave_up = 0
     for polls in (1, 3, 10, 40, 150, 600, 1 << 22):
-        print(f"S={S} T={T} polls={polls}", flush=True)
         lib.frnnt_set_spin_limit(polls)
         try:
             score1, (gx1, gy1) = F.mutual_information_recursion(px, py, None, return_grad=True)
@@ -219,21 +241,21 @@ def test_recursion_and_its_backward_in_a_graph(B, S, T):
     """Replays on other inputs, with eager calls between them: each finds the room between the workgroups as it
     was."""
     px, py, g = _inputs(B, S, T, False, S)
-    px, py, boundary = px.cuda().requires_grad_(), py.cuda().requires_grad_(), _window(B, S, T, g).cuda()
+    px, py, boundary = px.cuda(), py.cuda(), _window(B, S, T, g).cuda()
     seeds = torch.linspace(0.5, 2, B, device="cuda")
 
     def step():
-        scores = F.mutual_information_recursion(px, py, boundary)
-        return scores, *torch.autograd.grad(scores, (px, py), seeds)
+        x, y = px.detach().requires_grad_(), py.detach().requires_grad_()
+        scores = F.mutual_information_recursion(x, y, boundary)
+        return scores.detach(), *torch.autograd.grad(scores, (x, y), seeds)
 
     step()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = step()
-    for n in range(3):
-        with torch.no_grad():
-            px.add_(0.25)
+    for _ in range(3):
+        px.add_(0.25)
         want = step()
         graph.replay()
         torch.cuda.synchronize()

@@ -54,7 +54,6 @@ def test_pruned_rows_hold_the_same_bits(dtype, lengths, offset):
         begin = torch.linspace(0, S + 1 - R, T, device="cuda").long().expand(B, T)
         ranges = begin.unsqueeze(2) + torch.arange(R, device="cuda")
         for kind in ("regular", "constrained"):
-            print(f"C={C} {dtype} offset={offset} {kind}", flush=True)
             few = _run(F.rnnt_loss_pruned, logits, 1, offset, sym, ranges, boundary, rnnt_type=kind)
             many = _run(F.rnnt_loss_pruned, logits, 153, offset, sym, ranges, boundary, rnnt_type=kind)
             assert all(_same(a, b) for a, b in zip(few, many))

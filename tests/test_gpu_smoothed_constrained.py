@@ -24,7 +24,6 @@ def test_constrained_smoothed_loss(gpu_device, B, S, T, C):
     weights = 1 + torch.rand(B, generator=g)
     for term, l, a, handed_out in [(0, 0.25, 0.0, True), (C - 1, 0.1, 0.2, False)]:
         for boundary in (windows, None):
-            print(f"B={B} S={S} T={T} C={C} term={term}", flush=True)
             cpu = [x.clone().requires_grad_(True) for x in (lm, am)]
             gpu = [x.to(gpu_device).requires_grad_(True) for x in (lm, am)]
             args = dict(lm_only_scale=l, am_only_scale=a, rnnt_type="constrained", delay_penalty=0.01,

@@ -1,10 +1,11 @@
-"""Three bands of 64 rows in workgroups of their own on lattices of any length, which small batches of the losses and of
-the recursion run, against one workgroup per utterance, which the same utterances run in a batch too large for that:
-the same bits.  Windows that leave bands out, are empty or start inside the lattice; one frame."""
+"""Three bands of 64 rows in workgroups of their own on lattices of any length, which small batches of the recursion and
+of the losses that pass shares run, against one workgroup per utterance, which the same utterances run in a batch too
+large for that: the same bits.  Windows that leave bands out, are empty or start inside the lattice; one frame."""
 import pytest
 import torch
 
 import fast_rnnt_amd as F
+from fast_rnnt_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -18,15 +19,20 @@ def test_three_bands_of_any_length(gpu_device, S, T, modified):
     n, T1 = len(rows), T if modified else T + 1
     px, py = -1 + torch.randn(n, S, T1, generator=g), -1 + torch.randn(n, S + 1, T, generator=g)
 
-    def run(copies):
-        print(f"S={S} T={T} modified={modified} B={n * copies}", flush=True)
+    def run(copies, apart):
+        # (the recursion always passes shares if its gradients are not handed out; a loss, and what is handed out,
+        # from some length on)
+        assert _lib.load().frnnt_mi_route(n * copies, S, T, 1) & 3 == apart
         x, y = (v.to(gpu_device).repeat(copies, 1, 1).requires_grad_() for v in (px, py))
         boundary = torch.tensor(rows).to(gpu_device).repeat(copies, 1)
-        scores, (gx, gy) = F.mutual_information_recursion(x, y, boundary, return_grad=True)
+        handed_out, (gx, gy) = F.mutual_information_recursion(x, y, boundary, return_grad=True)
+        scores = F.mutual_information_recursion(x, y, boundary)
         seeds = torch.linspace(0.5, 2, n, device=gpu_device).repeat(copies)
-        return [v[-n:].cpu() for v in (scores.detach(), gx, gy, *torch.autograd.grad(scores, (x, y), seeds))]
+        formed = torch.autograd.grad(scores, (x, y), seeds)
+        return [v[-n:].cpu() for v in (handed_out.detach(), scores.detach(), gx, gy, *formed,
+                                       *torch.autograd.grad(handed_out, (x, y), seeds))]
 
-    for a, b in zip(run(1), run(12)):
+    for a, b in zip(run(1, 3), run(12, 0)):
         assert torch.equal(torch.nan_to_num(a, nan=1e30), torch.nan_to_num(b, nan=1e30))
 
 
