@@ -1003,8 +1003,9 @@ __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0)
 // LDS, a third of the loads and no exp; the sweep wave takes d2 = 1 - d1 itself, off the chain, and leaves
 // the cells' gradients, one value per cell in LDS instead of two; and the staging waves split those as they
 // carry them to memory.  Same operations, same bits.  The forward kernel's staging waves, of which the
-// sweep needs less, do the exp.  Both kernels, from p and px -> with shares: B 12, S 220, T 1500 143 -> 119 us;
-// B 64, S 120, T 600 70.2 -> 61.3; B 32, S 80, T 250 33.8 -> 32.1; B 8, S 60, T 200 25.7 -> 23.5.
+// sweep needs less, do the exp.  Both kernels and the marks, from p and px -> with shares, full windows: B 12, S 220,
+// T 1500 139 -> 120 us; B 64, S 120, T 600 64.6 -> 58.4; B 32, S 80, T 250 33.6 -> 32.4 (17.1 + 16.5 -> 18.4 + 14.0);
+// B 8, S 60, T 200 23.7 -> 21.7.
 template <typename R, bool kModified, int kSweepCap, int kStagers, int kBuffers, bool kApart, bool kShares>
 __global__ void __launch_bounds__(((1 + kStagers) * kSweepCap + (kApart ? 2 : 0) +
                                    kHelpers<kSweepCap, kShares>) * kWave)

@@ -55,7 +55,9 @@ struct NormShape {
   static constexpr int kLoads = kRows / 16;      // 16-byte loads per lane and slab
   // Row pitch in LDS: 20 floats.  Rows start 16-byte aligned, so a lane's four values of a row go
   // in as one 16-byte write, and a lane reads its row's eight k of a slab half as two 16-byte reads:
-  // sixteen lanes' reads (rows 20 floats apart) fall on all 64 banks.
+  // sixteen lanes' reads (rows 20 floats apart) fall on all 64 banks.  Sixteen lanes' writes, four rows of 16 floats,
+  // span 76: the last row's end falls on the first one's banks (B 64, S 120, T 600, C 500: 4.0 M cycles of conflicts in
+  // 2.2 M LDS instructions, the whole kernel's).
   static constexpr int kPitch = kNormK + 4;
   static constexpr int kSlab = kRows * kPitch;   // floats
   // the partial sums of the waves meet in the slabs' space

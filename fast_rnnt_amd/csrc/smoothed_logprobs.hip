@@ -908,7 +908,8 @@ struct Kept {
 // Whether a scale asks for an am-only model.  The reference takes 1e-20 in place of 0 (rnnt_loss.py:1346-1351)
 // to keep 0 * -inf out of px: such a model's terms are below 1e-16, next to log-probabilities and
 // gradients of which a unit in the last place is more than that wherever they count, and neither its
-// statistics nor its gradients are formed.
+// statistics nor its gradients are formed.  So an entry of am that is not finite reaches its own utterance, through
+// the joint model, and not the whole batch's lm gradient, as it would through such a model's unigram.
 bool has_am_model(double am_only_scale) { return fabs(am_only_scale) > 1e-19; }
 Kept keep_of(float *base, long B, long S, long T, long C) {
   size_t at = 0;
