@@ -76,6 +76,7 @@ def _compare(px, py, boundary, held=math.nan):
 @pytest.mark.parametrize("B,S,T", [
     (2, 1, 1), (5, 7, 31), (4, 30, 33), (3, 62, 64), (3, 63, 65), (3, 64, 95), (2, 65, 160),
     (9, 127, 130), (2, 128, 191), (2, 200, 257), (3, 255, 1100), (2, 300, 310), (130, 66, 300), (2, 70, 900),
+    (4, 100, 770), (3, 200, 100),
 ])
 def test_same_bits_as_through_p(B, S, T, modified):
     px, py, g = _inputs(B, S, T, modified, 17 * S + T)
@@ -117,10 +118,11 @@ def test_what_the_scratch_held_before(S, T, modified, value):
     assert torch.isfinite(want_x).all() and torch.isfinite(want_y).all()
 
 
-# one band, two together, two, three and four apart
+# one band, two together, two, three and four apart, two apart in the backward alone, four in the forward alone
 @pytest.mark.parametrize("kept", [False, True])
 @pytest.mark.parametrize("modified", [False, True])
-@pytest.mark.parametrize("B,S,T", [(5, 20, 33), (5, 100, 90), (4, 100, 1300), (4, 150, 200), (3, 250, 700)])
+@pytest.mark.parametrize("B,S,T", [(5, 20, 33), (5, 100, 90), (4, 100, 1300), (4, 150, 200), (3, 250, 700),
+                                   (4, 100, 770), (3, 200, 100)])
 def test_backward_again_on_the_same_shares(B, S, T, modified, kept):
     """With another gradient of the scores, into buffers that hold anything, those of the first call among them: what
     a first call on shares of their own forms.  With and without the room behind the shares."""
